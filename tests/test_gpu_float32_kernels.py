@@ -46,3 +46,51 @@ def test_product_of_rows_that_begin_anywhere():
     x, w = store[1:1 + m * k].view(m, k), store[3 + m * k:3 + m * k + n * k].view(n, k)
     got = ops.gemm_f32(x, w, torch.empty((m, n), device=DEV))
     assert torch.equal(got, ops.gemm_f32(x.clone(), w.clone(), torch.empty((m, n), device=DEV)))
+
+
+@pytest.mark.parametrize("n_q, n_kv, d, dv, shared, page, window, chunk", [
+    (8, 2, 128, 128, False, 16, 0, 0), (6, 3, 20, 20, False, 8, 0, 0), (3, 1, 33, 17, False, 16, 70, 0), (16, 1, 576, 512, True, 16, 0, 0),
+    (4, 1, 256, 256, False, 32, 0, 0), (6, 1, 64, 130, False, 16, 0, 100), (2, 2, 40, 1000, False, 16, 0, 0)])
+def test_attention_of_a_token_alone_and_among_others(n_q, n_kv, d, dv, shared, page, window, chunk):
+    """Tokens at the edges of the blocks of 64 keys, alone (several waves share the keys), among a few and among enough
+    for a wave each: the same bits, against the softmax in float64."""
+    import torch
+    from kipp_amd.csrc import ops
+    rng = np.random.default_rng(d + dv)
+    length = 450
+    blocks = -(-length // page)
+    order = rng.permutation(blocks + 2)[:blocks]
+    pages = blocks + 2
+    k = rng.normal(size=(pages, n_kv, page, d)).astype(np.float32)
+    v = k if shared else rng.normal(size=(pages, n_kv, page, dv)).astype(np.float32)
+    keys = k[order].transpose(0, 2, 1, 3).reshape(-1, n_kv, d)[:length].astype(np.float64)
+    values = v[order].transpose(0, 2, 1, 3).reshape(-1, n_kv, v.shape[3])[:length, :, :dv].astype(np.float64)
+    where = [0, 1, 62, 63, 64, 127, 128, 200, 319, 320, 448, 449]
+    many = -(-8200 // (n_q // 4 or 1))
+    positions = np.array(where + [int(p) for p in rng.integers(0, length, many)], dtype=np.int32)
+    q = rng.normal(size=(len(positions), n_q * d)).astype(np.float32)
+    kd = torch.tensor(k, device=DEV)
+    vd = kd if shared else torch.tensor(v, device=DEV)
+    table = torch.tensor(order[None], dtype=torch.int32, device=DEV)
+    scale = d ** -0.5
+
+    def run(rows):
+        pos = torch.tensor(positions[rows], device=DEV)
+        return ops.paged_attention_wide(torch.tensor(q[rows], device=DEV), kd, vd, torch.empty((len(rows), n_q * dv), device=DEV), pos,
+                                        torch.zeros_like(pos), table, n_q, n_kv, d, dv, scale, window=window, chunk=chunk, sink=True).cpu().numpy()
+    every = run(np.arange(len(positions)))
+    few = run(np.arange(300))
+    assert np.array_equal(few, every[:300])
+    for i, p in enumerate(where):
+        assert np.array_equal(run(np.array([i])), every[i:i + 1]), p
+        lo = p - p % chunk if chunk else (max(0, p - window + 1) if window else 0)
+        for h in range(n_q):
+            g = h // (n_q // n_kv)
+            s = keys[lo:p + 1, g] @ q[i, h * d:(h + 1) * d].astype(np.float64) * scale
+            top = max(s.max(), 0.0)
+            e = np.exp(s - top)
+            p_ = e / (e.sum() + np.exp(-top))
+            # a score is off by d products of float32, which moves a weight by as much; then p + 1 weighted values
+            moved = 2 * d * EPS * scale * (np.abs(keys[lo:p + 1, g]) @ np.abs(q[i, h * d:(h + 1) * d])).max() + (p + 20) * EPS
+            bound = 2 * moved * (p_ @ np.abs(values[lo:p + 1, g]))
+            assert np.all(np.abs(every[i, h * dv:(h + 1) * dv] - p_ @ values[lo:p + 1, g]) <= bound + 1e-30), (p, h)
