@@ -12,9 +12,10 @@ dual form (`SSDSpec`).
                       dt = softplus(dt + dt_bias);  S <- exp(-exp(A) dt) S + dt B u^T;  y = S^T C + D u
                       delta = W_o (rms in parts of (y silu(z)) * w)
 
-The recurrences, the gates and the norms run in float32 under either precision; the state is float32.  A prompt portion
-walks its tokens in order inside one launch, a single token is a walk of one step of the same kernel, so a position's
-result does not depend on how the tokens were cut.
+The recurrences, the gates and the norms run in float32 under either precision; the state is float32.  Under float32 a
+prompt portion walks its tokens in order inside one launch, a single token is a walk of one step of the same kernel, so a
+position's result does not depend on how the tokens were cut.  Under bfloat16 a portion goes 64 tokens at a time where the
+key size allows: the same float32 sums in another order.
 """
 from __future__ import annotations
 
@@ -33,6 +34,12 @@ def _stack_rows(rt, rows):
     if pad:
         w = torch.cat([w, torch.zeros((pad, w.shape[1]), dtype=w.dtype, device=w.device)], dim=0)
     return rt.weight(w.contiguous())
+
+
+def _scan_variants(key_size, dtype):
+    """The walk, and under bfloat16 its form for prompt portions where that takes the key size."""
+    from ..csrc.ops import matrix_chunks_ok
+    return [("linear_scan", None)] + ([("linear_chunks", None)] if dtype == "bfloat16" and matrix_chunks_ok(key_size) else [])
 
 
 @register("mixer", "decay_attention")
@@ -59,7 +66,7 @@ class DecayAttention:
 
     @staticmethod
     def variants(spec, dtype):
-        return [("linear_scan", None)]
+        return _scan_variants(spec.head_dim, dtype)
 
     def load(self, tensors):
         q, k, v, g, o, norm = self.spec.names
@@ -81,7 +88,8 @@ class DecayAttention:
         hv = s.num_heads * s.v_head_dim
         proj = rt.linear(x, self.w_in)                    # float32 [n, q | k | v | gate]
         o_raw = rt.empty((n, hv), torch.float32)
-        ops.decay_scan(proj, self.decays, state, batch.q_start, batch.q_len, batch.slots, o_raw, s.num_heads, s.head_dim, s.v_head_dim, longest=batch.max_q_len)
+        ops.decay_scan(proj, self.decays, state, batch.q_start, batch.q_len, batch.slots, o_raw, s.num_heads, s.head_dim, s.v_head_dim, longest=batch.max_q_len,
+                       chunks=rt.dtype == "bfloat16")
         out = ops.scan_finish(o_raw, proj, 2 * s.num_heads * s.head_dim + hv, self.norm, s.norm_eps, "sigmoid", hv, rt.empty((n, hv), rt.act_dtype))
         return rt.linear(out, self.w_o, slabs=True, defer=True)
 
@@ -121,7 +129,7 @@ class GatedDelta:
 
     @staticmethod
     def variants(spec, dtype):
-        return [("linear_scan", None)]
+        return _scan_variants(spec.head_dim, dtype)
 
     def load(self, tensors):
         n = self._names(self.spec)
@@ -147,7 +155,8 @@ class GatedDelta:
         ops.delta_prepare(proj, self.conv, self.a_log, self.dt_bias, state, batch.seq_of_token, batch.q_start, batch.q_len, batch.slots, prep,
                           s.num_heads, s.num_kv_heads, s.head_dim, s.v_head_dim, channels + hv, channels + hv + s.num_heads, s.unit_eps)
         o_raw = rt.empty((n, hv), torch.float32)
-        ops.delta_scan(prep, state, batch.q_start, batch.q_len, batch.slots, o_raw, s.num_heads, s.num_kv_heads, s.head_dim, s.v_head_dim, longest=batch.max_q_len)
+        ops.delta_scan(prep, state, batch.q_start, batch.q_len, batch.slots, o_raw, s.num_heads, s.num_kv_heads, s.head_dim, s.v_head_dim, longest=batch.max_q_len,
+                       chunks=rt.dtype == "bfloat16")
         out = ops.scan_finish(o_raw, proj, channels, self.norm, s.norm_eps, "silu", s.v_head_dim, rt.empty((n, hv), rt.act_dtype))
         return rt.linear(out, self.w_o, slabs=True, defer=True)
 
@@ -190,7 +199,7 @@ class SSD:
 
     @staticmethod
     def variants(spec, dtype):
-        return [("linear_scan", None)]
+        return _scan_variants(spec.state_size, dtype)
 
     def load(self, tensors):
         n = self._names(self.spec)
@@ -215,7 +224,7 @@ class SSD:
                         batch.slots, prep, s.num_heads, s.groups, s.state_size, s.head_dim)
         o_raw = rt.empty((n, s.inner), torch.float32)
         ops.gated_scan(prep, state, batch.q_start, batch.q_len, batch.slots, o_raw, s.num_heads, s.groups, s.state_size, s.head_dim,
-                       longest=batch.max_q_len)
+                       longest=batch.max_q_len, chunks=rt.dtype == "bfloat16")
         out = ops.ssd_finish(o_raw, prep, 2 * s.groups * s.state_size + s.inner, proj, 0, self.skip, s.head_dim, self.norm, s.norm_eps,
                              s.inner // s.norm_groups, rt.empty((n, s.inner), rt.act_dtype))
         return rt.linear(out, self.w_o, slabs=True, defer=True)
