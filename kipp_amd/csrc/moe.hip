@@ -36,6 +36,8 @@
 #define MFMA_KC 64          // numbers of k a step brings into LDS
 #define MFMA_PITCH 72       // bfloat16 numbers from a row to the next in LDS
 #define MFMA_THREADS 256
+#define ROWS_TILE 64        // rows of a tile of the product for few rows
+#define ROWS_WAVES 8        // waves of its workgroup
 #define XCDS 8              // dies of the chip; consecutive workgroups of a launch go to them in turn
 
 enum { ACT_NONE = -1, ACT_SILU = 0, ACT_RELU = 1, ACT_GELU = 2, ACT_GELU_TANH = 3, ACT_RELU2 = 4 };
@@ -478,6 +480,99 @@ moe_expert_mfma_kernel(const bf16_t* __restrict__ x, const int32_t* __restrict__
         }
 }
 
+// Tiles of few rows (single tokens): a workgroup (16 columns, tile), its waves a share of K each, the matrix straight from memory into the
+// products' operands, 128 bytes a row and wave at a time; the waves' sums are added in order through LDS.  Bound by the read of the
+// experts' matrices: four experts' [gate; up] of 2 x 2,432 x 2,560 (100 MB) 22.9 us, twelve's 54.7 (5.5 TB/s); four experts' 2,560 x
+// 2,432 (50 MB) 11.1 us.  The kernel for whole tiles above stages 64 numbers of k a step behind two barriers with a workgroup for 128
+// columns: 80 workgroups that walk 38 steps took 44 us for those 50 MB.  One step of 64 numbers ahead for two matrices, two for one: more
+// of them in registers were slower (five: 25.4, 67.8 and 12.7 us), and so were four waves for two matrices.
+template <typename TO, bool GLU, int MT>
+__device__ __forceinline__ void expert_rows(const bf16_t* __restrict__ x, const int32_t* __restrict__ gather, const float* __restrict__ row_weight,
+                                            const bf16_t* __restrict__ w_row, TO* __restrict__ out, int row0, int rows, int n0, int n_out, int k,
+                                            int act, float (*part_s)[GLU ? 2 : 1][KIPP_WAVE][4]) {
+    constexpr int NW = GLU ? 2 : 1, STEP = 64, AHEAD = GLU || MT > 2 ? 1 : 2;
+    const int wave = threadIdx.x / KIPP_WAVE, lane = threadIdx.x & (KIPP_WAVE - 1), l16 = lane & 15, h8 = 8 * (lane >> 4);
+    const bf16_t* x_row[MT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+        const int r = row0 + min(16 * i + l16, rows - 1);           // rows beyond the last read it and are not stored
+        x_row[i] = x + (size_t)(gather != nullptr ? gather[r] : r) * k + h8;
+    }
+    const u32x4 zero = (u32x4){0u, 0u, 0u, 0u};
+    f32x4 acc[NW][MT];
+#pragma unroll
+    for (int g = 0; g < NW; ++g)
+#pragma unroll
+        for (int i = 0; i < MT; ++i) acc[g][i] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+    Frag wf[AHEAD][2][NW], xf[AHEAD][2][MT];
+    auto fetch = [&](int j, int at) {
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+            const int kk = at + 32 * half;          // k is a multiple of 32: the last step may be half a step
+#pragma unroll
+            for (int g = 0; g < NW; ++g) wf[j][half][g].u = kk < k ? *(const u32x4*)(w_row + (size_t)g * n_out * k + kk + h8) : zero;
+#pragma unroll
+            for (int i = 0; i < MT; ++i) xf[j][half][i].u = kk < k ? *(const u32x4*)(x_row[i] + kk) : zero;
+        }
+    };
+    for (int at = STEP * wave; at < k; at += STEP * ROWS_WAVES * AHEAD) {
+#pragma unroll
+        for (int j = 0; j < AHEAD; ++j) fetch(j, at + STEP * ROWS_WAVES * j);
+#pragma unroll
+        for (int j = 0; j < AHEAD; ++j)
+#pragma unroll
+            for (int half = 0; half < 2; ++half)
+#pragma unroll
+                for (int g = 0; g < NW; ++g)
+#pragma unroll
+                    for (int i = 0; i < MT; ++i)
+                        acc[g][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j][half][g].v, xf[j][half][i].v, acc[g][i], 0, 0, 0);
+    }
+    // a lane holds columns 4 (l / 16) .. + 3 of row l % 16
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+        if (i > 0) __syncthreads();
+#pragma unroll
+        for (int g = 0; g < NW; ++g) *(f32x4*)part_s[wave][g][lane] = acc[g][i];
+        __syncthreads();
+        const int c = threadIdx.x & 15, m = threadIdx.x >> 4;
+        if (m < 16 && 16 * i + m < rows && n0 + c < n_out) {
+            const int from = 16 * (c >> 2) + m;
+            float total[NW];
+#pragma unroll
+            for (int g = 0; g < NW; ++g) {
+                total[g] = 0.0f;
+#pragma unroll
+                for (int p = 0; p < ROWS_WAVES; ++p) total[g] += part_s[p][g][from][c & 3];
+            }
+            const int r = row0 + 16 * i + m;
+            float y;
+            if (GLU) {
+                const float s = row_weight != nullptr ? row_weight[r] : 1.0f;
+                y = activate(s * total[0], act) * (s * total[NW - 1]);
+            } else {
+                y = activate(total[0], act);
+            }
+            store_f(out + (size_t)r * n_out, n0 + c, y);
+        }
+    }
+}
+
+template <typename TO, bool GLU>
+__global__ void __launch_bounds__(ROWS_WAVES * KIPP_WAVE)
+moe_expert_rows_kernel(const bf16_t* __restrict__ x, const int32_t* __restrict__ gather, const float* __restrict__ row_weight,
+                       const bf16_t* __restrict__ w, const int32_t* __restrict__ tiles, TO* __restrict__ out, int n_out, int k, int act) {
+    __shared__ __attribute__((aligned(16))) float part_s[ROWS_WAVES][GLU ? 2 : 1][KIPP_WAVE][4];
+    const int32_t* tile = tiles + (size_t)blockIdx.y * 3;
+    const int rows = tile[2];
+    if (rows == 0) return;      // uniform over the workgroup
+    const int n0 = 16 * blockIdx.x, row0 = tile[1];
+    const bf16_t* w_row = w + ((size_t)tile[0] * (GLU ? 2 : 1) * n_out + min(n0 + (int)(threadIdx.x & 15), n_out - 1)) * k;
+    if (rows <= 16) expert_rows<TO, GLU, 1>(x, gather, row_weight, w_row, out, row0, rows, n0, n_out, k, act, part_s);
+    else if (rows <= 32) expert_rows<TO, GLU, 2>(x, gather, row_weight, w_row, out, row0, rows, n0, n_out, k, act, part_s);
+    else expert_rows<TO, GLU, 4>(x, gather, row_weight, w_row, out, row0, rows, n0, n_out, k, act, part_s);
+}
+
 // A logit that weighs the shared expert's result, by its sigmoid: float32 at column `column` of rows of `stride` (slabs added in
 // order); z null: none, the result as it is.
 struct SharedGate {
@@ -576,7 +671,7 @@ extern "C" int kipp_moe_route(const float* z, int parts, int stride, int32_t* ch
     if (tokens <= 0) return 0;
     if (experts <= 0 || experts > MAX_EXPERTS || top <= 0 || top > MAX_TOP || top > experts || stride < experts || parts <= 0) return -1;
     const int pairs = tokens * top;
-    if (tile_rows != TILE_ROWS && tile_rows != MFMA_ROWS) return -1;
+    if (tile_rows != TILE_ROWS && tile_rows != ROWS_TILE && tile_rows != MFMA_ROWS) return -1;
     if (max_tiles < (pairs + tile_rows - 1) / tile_rows + (experts < pairs ? experts : pairs)) return -1;
 #define KIPP_RT(REGS)                                                                                                                  \
     hipLaunchKernelGGL(moe_route_kernel<REGS>, dim3((tokens + ROUTE_WAVES - 1) / ROUTE_WAVES), dim3(ROUTE_WAVES * KIPP_WAVE), 0, stream, z, \
@@ -603,7 +698,7 @@ extern "C" int kipp_moe_route_grouped(const float* z, int parts, int stride, con
     if (group_count <= 0 || experts % group_count || group_keep <= 0 || group_keep > group_count ||
         top > group_keep * (experts / group_count)) return -1;
     const int pairs = tokens * top, real = experts - identity;
-    if (tile_rows != TILE_ROWS && tile_rows != MFMA_ROWS) return -1;
+    if (tile_rows != TILE_ROWS && tile_rows != ROWS_TILE && tile_rows != MFMA_ROWS) return -1;
     if (max_tiles < (pairs + tile_rows - 1) / tile_rows + (real < pairs ? real : pairs)) return -1;
 #define KIPP_RG(REGS)                                                                                                                     \
     hipLaunchKernelGGL(moe_route_grouped_kernel<REGS>, dim3((tokens + ROUTE_WAVES - 1) / ROUTE_WAVES), dim3(ROUTE_WAVES * KIPP_WAVE), 0, stream, \
@@ -624,6 +719,19 @@ static int launch_expert(const void* x, int x_dtype, const int32_t* gather, cons
                          hipStream_t stream) {
     if (max_tiles <= 0) return 0;
     if (n_out <= 0 || k <= 0 || act < ACT_NONE || act > ACT_RELU2) return -1;
+    if (tile_rows == ROWS_TILE) {
+        if (x_dtype != KIPP_BF16 || w_dtype != KIPP_BF16 || k % 32 || (((uintptr_t)x | (uintptr_t)w) & 15)) return -2;
+        dim3 grid((n_out + 15) / 16, max_tiles), block(ROWS_WAVES * KIPP_WAVE);
+        if (out_dtype == KIPP_BF16)
+            hipLaunchKernelGGL((moe_expert_rows_kernel<bf16_t, GLU>), grid, block, 0, stream, (const bf16_t*)x, gather, row_weight,
+                               (const bf16_t*)w, tiles, (bf16_t*)out, n_out, k, act);
+        else if (out_dtype == KIPP_F32)
+            hipLaunchKernelGGL((moe_expert_rows_kernel<float, GLU>), grid, block, 0, stream, (const bf16_t*)x, gather, row_weight,
+                               (const bf16_t*)w, tiles, (float*)out, n_out, k, act);
+        else
+            return -2;
+        return KIPP_LAUNCH_CHECK();
+    }
     if (tile_rows == MFMA_ROWS) {
         if (x_dtype != KIPP_BF16 || w_dtype != KIPP_BF16 || k % 32) return -2;
         // a lane's offsets into x and into an expert's matrix are 32 bits wide

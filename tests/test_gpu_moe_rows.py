@@ -1,0 +1,51 @@
+"""The experts' products for few rows an expert (tiles of up to 64 rows, the matrix straight from memory) beside the kernel for
+whole tiles: the same list of rows, every class of rows a tile, K that ends in half a step, columns that do not fill a fragment."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.mark.parametrize("k, n_out", [(32, 16), (96, 40), (512, 65), (1056, 130), (2432, 2560)])
+@pytest.mark.parametrize("gated", [False, True])
+def test_few_rows_beside_whole_tiles(k, n_out, gated):
+    import torch
+    from kipp_amd.csrc import ops
+    rng = np.random.default_rng(k + n_out)
+    counts = [1, 0, 16, 17, 33, 64, 65, 130, 5]
+    experts, rows = len(counts), sum(counts)
+    order = rng.permutation(rows).astype(np.int32)
+    x = torch.tensor(rng.normal(size=(rows, k)).astype(np.float32), device=DEV).bfloat16()
+    w = torch.tensor((rng.normal(size=(experts, n_out * (2 if gated else 1), k)) * k ** -0.5).astype(np.float32), device=DEV).bfloat16()
+    weight = torch.tensor(rng.uniform(0.2, 1.0, size=rows).astype(np.float32), device=DEV)
+    gather = torch.tensor(order, device=DEV)
+    starts = np.concatenate([[0], np.cumsum(counts)[:-1]])
+    # float64 of what the bfloat16 operands hold
+    xd, wd = x.double()[gather.long()], w.double()
+    ref = torch.empty((rows, n_out), dtype=torch.float64, device=DEV)
+    size = torch.empty_like(ref)
+    for e, (at, n) in enumerate(zip(starts, counts)):
+        p = xd[at:at + n] @ wd[e].T
+        a = xd[at:at + n].abs() @ wd[e].abs().T
+        if gated:
+            s = weight[at:at + n].double()[:, None]
+            g, u = s * p[:, :n_out], s * p[:, n_out:]
+            ref[at:at + n] = g * torch.sigmoid(g) * u
+            size[at:at + n] = 1.1 * s * a[:, :n_out] * u.abs() + (g * torch.sigmoid(g)).abs() * s * a[:, n_out:]     # |silu'| < 1.1
+        else:
+            ref[at:at + n], size[at:at + n] = torch.relu(p), a
+    for tile_rows in (64, 128):
+        tiles = [(e, at + j, min(tile_rows, n - j)) for e, (at, n) in enumerate(zip(starts, counts)) for j in range(0, n, tile_rows)] + [(0, 0, 0)] * 3
+        td = torch.tensor(np.array(tiles, dtype=np.int32), device=DEV)
+        for through in (gather, None):
+            xs = x if through is not None else x[gather.long()].contiguous()
+            for ty in (torch.float32, torch.bfloat16):
+                out = torch.full((rows, n_out), float("nan"), dtype=ty, device=DEV)
+                if gated:
+                    ops.moe_expert_gated(xs, through, weight, w, td, out, "silu", tile_rows=tile_rows)
+                else:
+                    ops.moe_expert(xs, through, w, td, out, "relu", tile_rows=tile_rows)
+                # sums of k exact products in float32, in any order, and one rounding of the result
+                bound = (k + 4) * 2.0 ** -24 * size + (2.0 ** -8 if ty == torch.bfloat16 else 2.0 ** -22) * ref.abs() + 1e-30
+                assert bool(((out.double() - ref).abs() <= bound).all()), (tile_rows, ty)
