@@ -21,7 +21,7 @@
 //              two fragments of 16 columns are the gate's and the up's of the same 16 inner columns
 //     combine  out[t] = sum_j weight[t][j] y[place of (t, j)], or weight[t][j] x[t] for an identity expert (+ the shared expert's
 //              result, slabs added in order, maybe times the sigmoid of a logit of its own)
-#include "common.h"
+#include "tile_walk.h"
 #include <math.h>
 
 #define ROUTE_WAVES 4
@@ -30,12 +30,19 @@
 #define TILE_ROWS 16
 #define EXPERT_COLS 256
 #define EXPERT_KC 128
-#define MFMA_ROWS 128       // rows of a tile of the matrix-core product: eight fragments of 16
-#define MFMA_COLS 128       // columns of a workgroup: four waves with two fragments each
+#define MFMA_ROWS 128       // rows of a tile of the matrix-core products for whole tiles: eight fragments of 16, or four of 32
+#define MFMA_COLS 128       // columns of a workgroup of the staged one: four waves with two fragments each
 #define MFMA_NF (MFMA_COLS / 64)
 #define MFMA_KC 64          // numbers of k a step brings into LDS
 #define MFMA_PITCH 72       // bfloat16 numbers from a row to the next in LDS
 #define MFMA_THREADS 256
+#define MANY_ROWS 256       // rows of a tile of the walking one where an expert has many
+#define WALK_FROM 48        // rows an expert (all of them) beyond which the walking one is the faster
+#define TILE_WAVES 4        // waves of its workgroup
+#ifndef TILE_STAGES
+#define TILE_STAGES 3       // steps of K that are in LDS or on their way there: two workgroups share a compute unit
+#endif
+#define MANY_STAGES 4       // one workgroup a compute unit
 #define ROWS_TILE 64        // rows of a tile of the product for few rows
 #define ROWS_WAVES 8        // waves of its workgroup
 #define XCDS 8              // dies of the chip; consecutive workgroups of a launch go to them in turn
@@ -258,12 +265,14 @@ moe_sort_kernel(const int32_t* __restrict__ chosen, int pairs, int experts, int 
     }
     __syncthreads();
     for (int e = threadIdx.x; e < experts; e += blockDim.x) {
-        const int n = count[e];
-        for (int j = 0; j * tile_rows < n; ++j) {
+        const int n = count[e], parts = (n + tile_rows - 1) / tile_rows;
+        // whole tiles: an expert's rows shared out evenly, in 32s
+        const int each = tile_rows >= MFMA_ROWS && parts > 0 ? ((n + parts - 1) / parts + 31) / 32 * 32 : tile_rows;
+        for (int j = 0; j < parts; ++j) {
             int32_t* tile = tiles + (size_t)(tile_first[e] + j) * 3;
             tile[0] = e;
-            tile[1] = first[e] + j * tile_rows;
-            tile[2] = min(tile_rows, n - j * tile_rows);
+            tile[1] = first[e] + j * each;
+            tile[2] = min(each, n - j * each);
         }
     }
     for (int i = tile_first[experts] + threadIdx.x; i < max_tiles; i += blockDim.x) {
@@ -348,16 +357,11 @@ moe_expert_kernel(const TX* __restrict__ x, const int32_t* __restrict__ gather, 
         }
 }
 
-// The same on the matrix cores: bfloat16 x and w, K a multiple of 32, tiles of up to MFMA_ROWS rows.  A 16 x 16 x 32
+// The same on the matrix cores: bfloat16 x and w, K a multiple of 32, tiles of up to MFMA_ROWS rows, a workgroup 128 columns,
+// K staged through registers and LDS 64 numbers a step.  A 16 x 16 x 32
 // product takes, from lane l, 8 numbers of row l % 16 at k = 8 (l / 16) .. + 7 of either operand, and leaves
 // C[4 (l / 16) + v][l % 16] in its register v.
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
-typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
-union Frag {
-    u32x4 u;
-    bf16x8 v;
-};
 
 template <typename TO, bool GLU>
 __global__ void __launch_bounds__(MFMA_THREADS)
@@ -478,6 +482,129 @@ moe_expert_mfma_kernel(const bf16_t* __restrict__ x, const int32_t* __restrict__
                 }
             }
         }
+}
+
+// The same for experts of many rows, tiles of up to 32 FRAGS rows.  A workgroup takes a tile's rows
+// and 256 rows of the expert's matrix (GLU: 128 of the gate's and the 128 of the up's that belong to them), a wave all of the
+// rows against 64 of them, as many products of 32 rows as the tile has.  The walk over K is the one of the products for prompt portions
+// (`tile_walk.h`), its rows of X taken through `gather`.  Bound by what a compute unit draws (a matrix of an expert meets its
+// 100 to 300 rows only) and by whole rounds of workgroups.  32 experts, matrices of 2,432 x 2,560 and back, staged kernel / this one,
+// us: 8,192 rows 251 / 214 and 230 / 201, gated 417 / 360 (256 rows a tile; 375 with 128); 5,120 rows 198 / 174, 172 / 158, 329 / 262 (306);
+// 2,048 rows 137 / 128, 125 / 119, 197 / 194 (204 with 256 rows); 1,024 rows 116 / 119, 105 / 108, 175 / 185: its lines of 64
+// bytes of a row are the slower way to read a matrix once, so the staged kernel keeps experts of up to 48 rows.
+template <typename TO, bool GLU, int FRAGS, int STAGES, int WM>
+__device__ __forceinline__ void expert_tile(const bf16_t* __restrict__ x, const int32_t* __restrict__ gather, const float* __restrict__ row_weight,
+                                            const bf16_t* __restrict__ w_e, TO* __restrict__ out, int row0, int rows, int col0, int n_out, int k,
+                                            int act, unsigned char* lds) {
+    constexpr int WAVES = TILE_WAVES, WN = 2;
+    constexpr int TM = 64 * ((WM + 1) / 2), TN = 32 * WN * WAVES;     // rows of the pieces of a step (of X: whole instructions a wave)
+    constexpr int X_PIECE = TM * BK * 2, W_PIECE = TN * BK * 2, STAGE_BYTES = X_PIECE + W_PIECE;
+    constexpr int XI = TM / INSTR_ROWS / WAVES, WI = TN / INSTR_ROWS / WAVES;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l32 = lane & 31, hh = lane >> 5;
+    int lane_row, col8;
+    dma_place(lane, lane_row, col8);
+    // a lane's rows begin at 32-bit offsets from x and from the expert's matrix (the launcher has checked that they fit)
+    uint32_t x_src[XI], w_src[WI];
+#pragma unroll
+    for (int i = 0; i < XI; ++i) {
+        const int r = row0 + min((TM / WAVES) * wave + INSTR_ROWS * i + lane_row, rows - 1);     // rows beyond the tile's read its last one and are not stored
+        x_src[i] = (uint32_t)(((size_t)(gather != nullptr ? gather[r] : r) * k + col8) * 2);
+    }
+#pragma unroll
+    for (int i = 0; i < WI; ++i) {
+        const int r = 64 * wave + INSTR_ROWS * i + lane_row;        // of the piece; a wave's 64: under GLU 32 of the gate's, then the up's
+        const int wr = GLU ? min(col0 + 32 * wave + (r & 31), n_out - 1) + (r & 32 ? n_out : 0) : min(col0 + r, n_out - 1);
+        w_src[i] = (uint32_t)(((size_t)wr * k + col8) * 2);
+    }
+    f32x16 acc[WM][WN];
+    tile_walk<WM, WN, XI, WI, STAGES, STAGE_BYTES>(lds, lane, (const unsigned char*)x, (const unsigned char*)w_e, x_src, w_src,
+                                                   wave * (X_PIECE / WAVES), X_PIECE + wave * (W_PIECE / WAVES), 0,
+                                                   X_PIECE + wave * (W_PIECE / WAVES), k / BK, acc);
+    // In accumulator tile (i, j) a lane holds column l32 and rows 8 (v / 4) + 4 hh + v % 4.  32 rows at a time go through the wave's own
+    // corner of LDS (now free) as they are; a lane then takes 8 neighbouring columns of a row, activates and stores them (the
+    // activations written out for every accumulator register were hundreds of KB of code that ran once).
+    constexpr int WCOLS = GLU ? 32 : 64, PITCH = 68, LANES_PER_ROW = WCOLS / 8, ROWS_PER_PASS = 64 / LANES_PER_ROW;
+    static_assert(32 * PITCH * 4 * WAVES <= STAGES * STAGE_BYTES, "a wave's staging fits its share of LDS");
+    __syncthreads();                                               // every wave is done reading operands
+    float* stage = (float*)lds + wave * 32 * PITCH;
+    const int c_in = (lane % LANES_PER_ROW) * 8, c = col0 + WCOLS * wave + c_in;
+#pragma unroll
+    for (int i = 0; i < WM; ++i) {
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+#pragma unroll
+            for (int j = 0; j < WN; ++j) stage[(8 * (v / 4) + 4 * hh + (v % 4)) * PITCH + 32 * j + l32] = acc[i][j][v];
+        __builtin_amdgcn_s_waitcnt(0xC07F);                        // lgkmcnt(0): what the wave wrote it reads back
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll 1
+        for (int r = lane / LANES_PER_ROW; r < 32; r += ROWS_PER_PASS) {
+            if (32 * i + r >= rows || c >= n_out) continue;
+            const float* at = stage + r * PITCH + c_in;
+            float y[8], u[8];
+#pragma unroll
+            for (int q = 0; q < 8; q += 4) {
+                *(f32x4*)(y + q) = *(const f32x4*)(at + q);
+                if (GLU) *(f32x4*)(u + q) = *(const f32x4*)(at + 32 + q);
+            }
+            const float s = GLU && row_weight != nullptr ? row_weight[row0 + 32 * i + r] : 1.0f;
+#pragma unroll
+            for (int q = 0; q < 8; ++q) y[q] = GLU ? activate(s * y[q], act) * (s * u[q]) : activate(y[q], act);
+            TO* dst = out + (size_t)(row0 + 32 * i + r) * n_out + c;
+            if (c + 8 <= n_out && (n_out & 7) == 0) {
+                if constexpr (sizeof(TO) == 4) {
+                    *(f32x4*)dst = *(const f32x4*)y;
+                    *(f32x4*)(dst + 4) = *(const f32x4*)(y + 4);
+                } else {
+                    u32x4 packed;
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) packed[q] = (uint32_t)f32_to_bf16(y[2 * q]) | ((uint32_t)f32_to_bf16(y[2 * q + 1]) << 16);
+                    *(u32x4*)dst = packed;
+                }
+            } else {
+                for (int q = 0; q < 8; ++q)
+                    if (c + q < n_out) store_f(dst, q, y[q]);
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_s_waitcnt(0xC07F);                        // the reads are done before the next 32 rows overwrite them
+    }
+}
+
+template <typename TO, bool GLU, int FRAGS, int STAGES>
+__global__ void __launch_bounds__(64 * TILE_WAVES, FRAGS <= 4 ? 2 : 1)
+moe_expert_tiles_kernel(const bf16_t* __restrict__ x, const int32_t* __restrict__ gather, const float* __restrict__ row_weight,
+                        const bf16_t* __restrict__ w, const int32_t* __restrict__ tiles, int max_tiles, int col_tiles, TO* __restrict__ out,
+                        int n_out, int k, int act) {
+    extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
+    // Used tiles come first in the list.  Workgroups id, id + 8, .. run on one die of the chip, each with an L2 of its own: a die
+    // takes a run of (tile, columns) pairs, columns fastest, so that its workgroups share rows of x and, from tile to tile of one
+    // expert, rows of w.
+    int used = 0;
+    for (int at = 0; at < max_tiles; at += KIPP_WAVE) {
+        const int i = at + (threadIdx.x & 63);
+        used += __popcll(__ballot(i < max_tiles && tiles[(size_t)i * 3 + 2] > 0));
+    }
+    const int items = used * col_tiles, per_die = (items + XCDS - 1) / XCDS;
+    const int turn = blockIdx.x / XCDS, item = (blockIdx.x % XCDS) * per_die + turn;
+    if (turn >= per_die || item >= items) return;       // uniform over the workgroup
+    const int32_t* tile = tiles + (size_t)(item / col_tiles) * 3;
+    const int expert = __builtin_amdgcn_readfirstlane(tile[0]), row0 = __builtin_amdgcn_readfirstlane(tile[1]), rows = __builtin_amdgcn_readfirstlane(tile[2]);
+    const int col0 = (item % col_tiles) * (GLU ? 32 : 64) * TILE_WAVES;
+    const bf16_t* w_e = w + (size_t)expert * (GLU ? 2 : 1) * n_out * k;
+    // a tile's products: as many of 32 rows as it has (of 64 in the larger form)
+    constexpr int GRAIN = FRAGS / 4;
+#define KIPP_ET(N)                                                                                                                     \
+    case N:                                                                                                                            \
+        expert_tile<TO, GLU, FRAGS, STAGES, N * GRAIN>(x, gather, row_weight, w_e, out, row0, rows, col0, n_out, k, act, lds);           \
+        break
+    switch ((rows + 32 * GRAIN - 1) / (32 * GRAIN)) {
+        KIPP_ET(1);
+        KIPP_ET(2);
+        KIPP_ET(3);
+        KIPP_ET(4);
+    }
+#undef KIPP_ET
 }
 
 // Tiles of few rows (single tokens): a workgroup (16 columns, tile), its waves a share of K each, the matrix straight from memory into the
@@ -671,7 +798,7 @@ extern "C" int kipp_moe_route(const float* z, int parts, int stride, int32_t* ch
     if (tokens <= 0) return 0;
     if (experts <= 0 || experts > MAX_EXPERTS || top <= 0 || top > MAX_TOP || top > experts || stride < experts || parts <= 0) return -1;
     const int pairs = tokens * top;
-    if (tile_rows != TILE_ROWS && tile_rows != ROWS_TILE && tile_rows != MFMA_ROWS) return -1;
+    if (tile_rows != TILE_ROWS && tile_rows != ROWS_TILE && tile_rows != MFMA_ROWS && tile_rows != MANY_ROWS) return -1;
     if (max_tiles < (pairs + tile_rows - 1) / tile_rows + (experts < pairs ? experts : pairs)) return -1;
 #define KIPP_RT(REGS)                                                                                                                  \
     hipLaunchKernelGGL(moe_route_kernel<REGS>, dim3((tokens + ROUTE_WAVES - 1) / ROUTE_WAVES), dim3(ROUTE_WAVES * KIPP_WAVE), 0, stream, z, \
@@ -698,7 +825,7 @@ extern "C" int kipp_moe_route_grouped(const float* z, int parts, int stride, con
     if (group_count <= 0 || experts % group_count || group_keep <= 0 || group_keep > group_count ||
         top > group_keep * (experts / group_count)) return -1;
     const int pairs = tokens * top, real = experts - identity;
-    if (tile_rows != TILE_ROWS && tile_rows != ROWS_TILE && tile_rows != MFMA_ROWS) return -1;
+    if (tile_rows != TILE_ROWS && tile_rows != ROWS_TILE && tile_rows != MFMA_ROWS && tile_rows != MANY_ROWS) return -1;
     if (max_tiles < (pairs + tile_rows - 1) / tile_rows + (real < pairs ? real : pairs)) return -1;
 #define KIPP_RG(REGS)                                                                                                                     \
     hipLaunchKernelGGL(moe_route_grouped_kernel<REGS>, dim3((tokens + ROUTE_WAVES - 1) / ROUTE_WAVES), dim3(ROUTE_WAVES * KIPP_WAVE), 0, stream, \
@@ -713,10 +840,28 @@ extern "C" int kipp_moe_route_grouped(const float* z, int parts, int stride, con
     return KIPP_LAUNCH_CHECK();
 }
 
+template <typename TO, bool GLU, int FRAGS, int STAGES>
+static int launch_tiles(const void* x, const int32_t* gather, const float* row_weight, const void* w, const int32_t* tiles, int max_tiles,
+                        void* out, int n_out, int k, int act, hipStream_t stream) {
+    constexpr int lds_bytes = STAGES * (32 * FRAGS + 64 * TILE_WAVES) * BK * 2;
+    static bool prepared = false;
+    if (!prepared) {
+        if (hipFuncSetAttribute((const void*)moe_expert_tiles_kernel<TO, GLU, FRAGS, STAGES>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                lds_bytes) != hipSuccess)
+            return -6;
+        prepared = true;
+    }
+    const int cols = (GLU ? 32 : 64) * TILE_WAVES, col_tiles = (n_out + cols - 1) / cols;
+    const int grid = (max_tiles * col_tiles + XCDS - 1) / XCDS * XCDS;
+    hipLaunchKernelGGL((moe_expert_tiles_kernel<TO, GLU, FRAGS, STAGES>), dim3(grid), dim3(64 * TILE_WAVES), lds_bytes, stream, (const bf16_t*)x,
+                       gather, row_weight, (const bf16_t*)w, tiles, max_tiles, col_tiles, (TO*)out, n_out, k, act);
+    return KIPP_LAUNCH_CHECK();
+}
+
 template <bool GLU>
 static int launch_expert(const void* x, int x_dtype, const int32_t* gather, const float* row_weight, const void* w, int w_dtype,
                          const int32_t* tiles, int max_tiles, void* out, int out_dtype, int n_out, int k, int act, int tile_rows,
-                         hipStream_t stream) {
+                         int sorted_rows, int experts, hipStream_t stream) {
     if (max_tiles <= 0) return 0;
     if (n_out <= 0 || k <= 0 || act < ACT_NONE || act > ACT_RELU2) return -1;
     if (tile_rows == ROWS_TILE) {
@@ -732,21 +877,30 @@ static int launch_expert(const void* x, int x_dtype, const int32_t* gather, cons
             return -2;
         return KIPP_LAUNCH_CHECK();
     }
-    if (tile_rows == MFMA_ROWS) {
-        if (x_dtype != KIPP_BF16 || w_dtype != KIPP_BF16 || k % 32) return -2;
+    if (tile_rows == MFMA_ROWS || tile_rows == MANY_ROWS) {
+        if (x_dtype != KIPP_BF16 || w_dtype != KIPP_BF16 || k % 32 || (((uintptr_t)x | (uintptr_t)w) & 15)) return -2;
         // a lane's offsets into x and into an expert's matrix are 32 bits wide
-        if ((long long)max_tiles * MFMA_ROWS * k >= (1ll << 31) || (long long)(GLU ? 2 : 1) * n_out * k >= (1ll << 31)) return -2;
-        const int cols = GLU ? MFMA_COLS / 2 : MFMA_COLS;
-        dim3 grid(max_tiles, (n_out + cols - 1) / cols), block(MFMA_THREADS);
+        if ((long long)max_tiles * tile_rows * k >= (1ll << 31) || (long long)(GLU ? 2 : 1) * n_out * k >= (1ll << 31)) return -2;
+        if (tile_rows == MFMA_ROWS && sorted_rows <= WALK_FROM * (long long)experts) {
+            const int cols = GLU ? MFMA_COLS / 2 : MFMA_COLS;
+            dim3 grid(max_tiles, (n_out + cols - 1) / cols), block(MFMA_THREADS);
+            if (out_dtype == KIPP_BF16)
+                hipLaunchKernelGGL((moe_expert_mfma_kernel<bf16_t, GLU>), grid, block, 0, stream, (const bf16_t*)x, gather, row_weight,
+                                   (const bf16_t*)w, tiles, (bf16_t*)out, n_out, k, act);
+            else if (out_dtype == KIPP_F32)
+                hipLaunchKernelGGL((moe_expert_mfma_kernel<float, GLU>), grid, block, 0, stream, (const bf16_t*)x, gather, row_weight,
+                                   (const bf16_t*)w, tiles, (float*)out, n_out, k, act);
+            else
+                return -2;
+            return KIPP_LAUNCH_CHECK();
+        }
         if (out_dtype == KIPP_BF16)
-            hipLaunchKernelGGL((moe_expert_mfma_kernel<bf16_t, GLU>), grid, block, 0, stream, (const bf16_t*)x, gather, row_weight,
-                               (const bf16_t*)w, tiles, (bf16_t*)out, n_out, k, act);
-        else if (out_dtype == KIPP_F32)
-            hipLaunchKernelGGL((moe_expert_mfma_kernel<float, GLU>), grid, block, 0, stream, (const bf16_t*)x, gather, row_weight,
-                               (const bf16_t*)w, tiles, (float*)out, n_out, k, act);
-        else
-            return -2;
-        return KIPP_LAUNCH_CHECK();
+            return tile_rows == MFMA_ROWS ? launch_tiles<bf16_t, GLU, 4, TILE_STAGES>(x, gather, row_weight, w, tiles, max_tiles, out, n_out, k, act, stream)
+                                          : launch_tiles<bf16_t, GLU, 8, MANY_STAGES>(x, gather, row_weight, w, tiles, max_tiles, out, n_out, k, act, stream);
+        if (out_dtype == KIPP_F32)
+            return tile_rows == MFMA_ROWS ? launch_tiles<float, GLU, 4, TILE_STAGES>(x, gather, row_weight, w, tiles, max_tiles, out, n_out, k, act, stream)
+                                          : launch_tiles<float, GLU, 8, MANY_STAGES>(x, gather, row_weight, w, tiles, max_tiles, out, n_out, k, act, stream);
+        return -2;
     }
     if (tile_rows != TILE_ROWS) return -1;
     dim3 grid(max_tiles, (n_out + EXPERT_COLS - 1) / EXPERT_COLS), block(EXPERT_COLS);
@@ -761,17 +915,21 @@ static int launch_expert(const void* x, int x_dtype, const int32_t* gather, cons
     return KIPP_LAUNCH_CHECK();
 }
 
-// `tile_rows`: the rows of the tiles that `kipp_moe_route` was asked for: 128 takes the matrix cores (bfloat16 x and w, K a multiple of 32), 16 the plain kernel.
+// `tile_rows`: the rows of the tiles that `kipp_moe_route` was asked for: 64, 128 and 256 take the matrix cores (bfloat16 x and w, K a
+// multiple of 32), 16 the plain kernel.  `sorted_rows` of `experts` experts in all: which kernel for whole tiles is the faster.
 extern "C" int kipp_moe_expert(const void* x, int x_dtype, const int32_t* gather, const void* w, int w_dtype, const int32_t* tiles,
-                               int max_tiles, void* out, int out_dtype, int n_out, int k, int act, int tile_rows, hipStream_t stream) {
-    return launch_expert<false>(x, x_dtype, gather, nullptr, w, w_dtype, tiles, max_tiles, out, out_dtype, n_out, k, act, tile_rows, stream);
+                               int max_tiles, void* out, int out_dtype, int n_out, int k, int act, int tile_rows, int sorted_rows, int experts,
+                               hipStream_t stream) {
+    return launch_expert<false>(x, x_dtype, gather, nullptr, w, w_dtype, tiles, max_tiles, out, out_dtype, n_out, k, act, tile_rows, sorted_rows,
+                                experts, stream);
 }
 
 // The same against w [experts][2 n_out][k] = [gate; up] with a weight a sorted row (or null): out = act(s gate) * (s up).
 extern "C" int kipp_moe_expert_gated(const void* x, int x_dtype, const int32_t* gather, const float* row_weight, const void* w, int w_dtype,
                                      const int32_t* tiles, int max_tiles, void* out, int out_dtype, int n_out, int k, int act,
-                                     int tile_rows, hipStream_t stream) {
-    return launch_expert<true>(x, x_dtype, gather, row_weight, w, w_dtype, tiles, max_tiles, out, out_dtype, n_out, k, act, tile_rows, stream);
+                                     int tile_rows, int sorted_rows, int experts, hipStream_t stream) {
+    return launch_expert<true>(x, x_dtype, gather, row_weight, w, w_dtype, tiles, max_tiles, out, out_dtype, n_out, k, act, tile_rows, sorted_rows,
+                               experts, stream);
 }
 
 // `x` (or null): the rows that identity experts hand on.  `gate_z` (or null): rows whose column `gate_column` holds the logit that

@@ -1023,15 +1023,25 @@ ACTIVATIONS = {"silu": 0, "relu": 1, "gelu": 2, "gelu_tanh": 3, "relu2": 4}     
 MOE_TILE_ROWS = 16
 MOE_MFMA_ROWS = 128    # rows of a tile of the experts' products on the matrix cores
 MOE_FEW_ROWS = 64      # the same in the kernel for few rows an expert, which reads the experts' matrices straight into the products
-MOE_FEW_PAIRS = 16     # pairs an expert (all of them) up to which a step takes that kernel
+MOE_MANY_ROWS = 256    # the same where an expert has many rows: its matrix is read less often, a compute unit has one workgroup
+# Pairs an expert (all of them) up to which a step takes the kernel for few rows, and from which on a gated one takes tiles of 256.
+# 32 experts, inner 2,432, width 2,560, both products, us: 256 pairs gated 251 with tiles of 64, 276 with 128; 512 pairs 314 and 281; 2,048
+# pairs 313 with tiles of 128, 326 with 256; 5,120 pairs 464 and 421; without a gate 332 and 357 there, 415 and 422 at 8,192.
+MOE_FEW_PAIRS, MOE_MANY_PAIRS = 12, 96
 
 
-def moe_tile_rows(dtype: torch.dtype, *contractions: int, pairs: Optional[int] = None, experts: int = 1) -> int:
+def moe_tile_rows(dtype: torch.dtype, *contractions: int, pairs: Optional[int] = None, experts: int = 1, gated: bool = False) -> int:
     """Rows of the tiles that the experts' products take: 128 on the matrix cores (bfloat16, every contraction a multiple of
-    32), else 16.  With `pairs`, the (token, choice) pairs of the step: 64 for few of them an expert."""
+    32), else 16.  With `pairs`, the (token, choice) pairs of the step: 64 for few of them an expert, 256 for many of a gated one."""
     if dtype != torch.bfloat16 or any(k % 32 for k in contractions):
         return MOE_TILE_ROWS
-    return MOE_FEW_ROWS if pairs is not None and pairs <= MOE_FEW_PAIRS * experts else MOE_MFMA_ROWS
+    if pairs is not None and pairs <= MOE_FEW_PAIRS * experts:
+        return MOE_FEW_ROWS
+    many = pairs is not None and gated and pairs > MOE_MANY_PAIRS * experts
+    # (a lane's offset into the rows is 32 bits wide, for as many rows as the tiles could hold)
+    if many and (-(-pairs // MOE_MANY_ROWS) + experts) * MOE_MANY_ROWS * max(contractions) < 1 << 31:
+        return MOE_MANY_ROWS
+    return MOE_MFMA_ROWS
 
 
 def moe_max_tiles(tokens: int, experts: int, top: int, tile_rows: int = 16) -> int:
@@ -1087,7 +1097,7 @@ def moe_route(z: torch.Tensor, experts: int, top: int, eps: float, chosen: torch
 def moe_expert(x: torch.Tensor, gather: Optional[torch.Tensor], w: torch.Tensor, tiles: torch.Tensor, out: torch.Tensor,
                activation: Optional[str] = None, tile_rows: int = 16) -> torch.Tensor:
     """Every tile's rows against its expert's matrix: out[row] = act(w[expert] x_row), x_row = x[gather[row]] (or x[row]);
-    `w` [experts, n_out, k], `out` [sorted rows, n_out].  `tile_rows`: what `moe_route` was given (64, 128: the matrix cores)."""
+    `w` [experts, n_out, k], `out` [sorted rows, n_out].  `tile_rows`: what `moe_route` was given (64, 128, 256: the matrix cores)."""
     _dev(x, gather, w, tiles, out)
     _i32(tiles, "tiles")
     if gather is not None:
@@ -1096,11 +1106,11 @@ def moe_expert(x: torch.Tensor, gather: Optional[torch.Tensor], w: torch.Tensor,
           "moe_expert: x [rows, k], w [experts, n_out, k] of one type, out [rows, n_out]")
     _need(out.shape[0] == (gather.numel() if gather is not None else x.shape[0]), "moe_expert: one output row a sorted row")
     _need(activation is None or activation in ACTIVATIONS, f"moe_expert: activation is one of {sorted(ACTIVATIONS)}")
-    _need(tile_rows == MOE_TILE_ROWS or (tile_rows in (MOE_FEW_ROWS, MOE_MFMA_ROWS) and x.dtype == torch.bfloat16 and w.shape[2] % 32 == 0),
-          "moe_expert: tiles of 16 rows, or of 64 or 128 for bfloat16 with K a multiple of 32")
-    fn = _fn("moe", "kipp_moe_expert", [_c_ptr, _c_int, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_int, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr])
+    _need(tile_rows == MOE_TILE_ROWS or (tile_rows in (MOE_FEW_ROWS, MOE_MFMA_ROWS, MOE_MANY_ROWS) and x.dtype == torch.bfloat16 and w.shape[2] % 32 == 0),
+          "moe_expert: tiles of 16 rows, or of 64, 128 or 256 for bfloat16 with K a multiple of 32")
+    fn = _fn("moe", "kipp_moe_expert", [_c_ptr, _c_int, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_int, _c_ptr] + [_c_int] * 7 + [_c_ptr])
     _check(fn(_ptr(x), _code(x), _ptr(gather), _ptr(w), _code(w), _ptr(tiles), tiles.shape[0], _ptr(out), _code(out), w.shape[1], w.shape[2],
-              -1 if activation is None else ACTIVATIONS[activation], int(tile_rows), _stream()), "moe_expert")
+              -1 if activation is None else ACTIVATIONS[activation], int(tile_rows), out.shape[0], w.shape[0], _stream()), "moe_expert")
     return out
 
 
@@ -1119,11 +1129,11 @@ def moe_expert_gated(x: torch.Tensor, gather: Optional[torch.Tensor], row_weight
     _need(out.shape[0] == (gather.numel() if gather is not None else x.shape[0]), "moe_expert_gated: one output row a sorted row")
     _need(row_weight is None or (row_weight.dtype == torch.float32 and row_weight.numel() == out.shape[0]), "moe_expert_gated: a float32 weight a sorted row")
     _need(activation in ACTIVATIONS, f"moe_expert_gated: activation is one of {sorted(ACTIVATIONS)}")
-    _need(tile_rows == MOE_TILE_ROWS or (tile_rows in (MOE_FEW_ROWS, MOE_MFMA_ROWS) and x.dtype == torch.bfloat16 and w.shape[2] % 32 == 0),
-          "moe_expert_gated: tiles of 16 rows, or of 64 or 128 for bfloat16 with K a multiple of 32")
-    fn = _fn("moe", "kipp_moe_expert_gated", [_c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_int, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr])
+    _need(tile_rows == MOE_TILE_ROWS or (tile_rows in (MOE_FEW_ROWS, MOE_MFMA_ROWS, MOE_MANY_ROWS) and x.dtype == torch.bfloat16 and w.shape[2] % 32 == 0),
+          "moe_expert_gated: tiles of 16 rows, or of 64, 128 or 256 for bfloat16 with K a multiple of 32")
+    fn = _fn("moe", "kipp_moe_expert_gated", [_c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_int, _c_ptr] + [_c_int] * 7 + [_c_ptr])
     _check(fn(_ptr(x), _code(x), _ptr(gather), _ptr(row_weight), _ptr(w), _code(w), _ptr(tiles), tiles.shape[0], _ptr(out), _code(out), inner, w.shape[2],
-              ACTIVATIONS[activation], int(tile_rows), _stream()), "moe_expert_gated")
+              ACTIVATIONS[activation], int(tile_rows), out.shape[0], w.shape[0], _stream()), "moe_expert_gated")
     return out
 
 

@@ -1,5 +1,6 @@
-"""The experts' products for few rows an expert (tiles of up to 64 rows, the matrix straight from memory) beside the kernel for
-whole tiles: the same list of rows, every class of rows a tile, K that ends in half a step, columns that do not fill a fragment."""
+"""The experts' products on the matrix cores, each form over the same rows: few rows an expert (tiles of up to 64, the matrix
+straight from memory), whole tiles staged through registers, whole tiles of the walk that brings both operands straight into LDS
+(up to 128 and 256 rows).  Every class of rows a tile, K of one step and of many, columns that do not fill a fragment."""
 import numpy as np
 import pytest
 
@@ -9,11 +10,12 @@ DEV = "cuda:0"
 
 @pytest.mark.parametrize("k, n_out", [(32, 16), (96, 40), (512, 65), (1056, 130), (2432, 2560)])
 @pytest.mark.parametrize("gated", [False, True])
-def test_few_rows_beside_whole_tiles(k, n_out, gated):
+@pytest.mark.parametrize("more", [1, 4])
+def test_every_form_against_float64(k, n_out, gated, more):
     import torch
     from kipp_amd.csrc import ops
     rng = np.random.default_rng(k + n_out)
-    counts = [1, 0, 16, 17, 33, 64, 65, 130, 5]
+    counts = [1, 0, 16, 17, 33, 64, 65, 130, 5] if more == 1 else [300, 97, 128, 0, 257, 31, 192, 220]
     experts, rows = len(counts), sum(counts)
     order = rng.permutation(rows).astype(np.int32)
     x = torch.tensor(rng.normal(size=(rows, k)).astype(np.float32), device=DEV).bfloat16()
@@ -35,7 +37,8 @@ def test_few_rows_beside_whole_tiles(k, n_out, gated):
             size[at:at + n] = 1.1 * s * a[:, :n_out] * u.abs() + (g * torch.sigmoid(g)).abs() * s * a[:, n_out:]     # |silu'| < 1.1
         else:
             ref[at:at + n], size[at:at + n] = torch.relu(p), a
-    for tile_rows in (64, 128):
+    assert (rows > 48 * experts) == (more > 1)          # beyond that 128 rows a tile is the walk's
+    for tile_rows in (64, 128, 256):
         tiles = [(e, at + j, min(tile_rows, n - j)) for e, (at, n) in enumerate(zip(starts, counts)) for j in range(0, n, tile_rows)] + [(0, 0, 0)] * 3
         td = torch.tensor(np.array(tiles, dtype=np.int32), device=DEV)
         for through in (gather, None):
@@ -49,3 +52,28 @@ def test_few_rows_beside_whole_tiles(k, n_out, gated):
                 # sums of k exact products in float32, in any order, and one rounding of the result
                 bound = (k + 4) * 2.0 ** -24 * size + (2.0 ** -8 if ty == torch.bfloat16 else 2.0 ** -22) * ref.abs() + 1e-30
                 assert bool(((out.double() - ref).abs() <= bound).all()), (tile_rows, ty)
+
+
+@pytest.mark.parametrize("tile_rows", [64, 128, 256])
+def test_the_sort_shares_rows_out(tile_rows):
+    """Every sorted row in one tile of its expert, tiles no larger than asked for, used ones first."""
+    import torch
+    from kipp_amd.csrc import ops
+    rng = np.random.default_rng(tile_rows)
+    tokens, experts, top = 1500, 7, 2
+    z = rng.normal(size=(tokens, experts)).astype(np.float32)
+    z[:, 0] += 1.5
+    z[:, 3] = -30.0
+    new = lambda *shape: torch.empty(shape, dtype=torch.int32, device=DEV)  # noqa: E731
+    chosen, weight, pair_token, place = new(tokens, top), torch.empty((tokens, top), device=DEV), new(tokens * top), new(tokens * top)
+    tiles = new(ops.moe_max_tiles(tokens, experts, top, tile_rows), 3)
+    ops.moe_route(torch.tensor(z, device=DEV), experts, top, 1e-20, chosen, weight, pair_token, place, tiles, tile_rows=tile_rows)
+    expert_of_row = np.empty(tokens * top, dtype=int)
+    expert_of_row[place.cpu().numpy().reshape(-1)] = chosen.cpu().numpy().reshape(-1)
+    covered = np.zeros(tokens * top, dtype=int)
+    listed = tiles.cpu().numpy()
+    assert np.all(np.diff((listed[:, 2] > 0).astype(int)) <= 0)
+    for e, first, n in listed:
+        assert 0 <= n <= tile_rows and np.all(expert_of_row[first:first + n] == e)
+        covered[first:first + n] += 1
+    assert np.all(covered == 1)
