@@ -23,6 +23,9 @@
 // D lane l holds rows 4 (l / 16) + v of column l % 16.  Scores: A = 16 keys, B = 16 query rows.  Mixing: A = 16
 // (row, key) pairs over heads, B = mix^T.  Values: A = V^T (16 value columns over 32 keys), B = p'.
 //
+// A single token has no use for a tile of 16 rows: its form is `mixed_single_scores_kernel` and `mixed_single_values_kernel` below, in which the
+// heads are the products' columns.
+//
 // Everything a workgroup does follows from device-side lengths (ctx_len, q_len), so a recorded step whose item list
 // was made for the longest context of its class still computes each sequence's own keys; an item whose run of keys
 // is empty leaves neutral statistics and zeros.
@@ -489,22 +492,282 @@ __global__ void __launch_bounds__(MX_THREADS) mixed_values_kernel(
     }
 }
 
+// ---- single tokens ------------------------------------------------------------------------------------------------
+//
+// A workgroup takes (a run of the token's keys, token), keys 64 at a time; a wave takes key/value heads in turn.
+//
+//   mixed_single_scores_kernel   scores of a key/value head's query heads (16 keys x the heads a product), scaled, biased and masked, into
+//                                memory as float32 [token][key][32 heads], and the run's (maximum, sum) of every head;
+//   mixed_single_values_kernel   merges the runs' statistics and the sink; a lane takes 8 heads of a key, makes their final weights
+//                                (two bfloat16 halves, as above) and mixes them on the matrix cores without a trip through LDS; the
+//                                mixed weights through LDS to the waves of their key/value heads, which multiply the values, asked
+//                                for before anything else.  Every run leaves float32 partial sums.
+//
+// Bound by its chains of loads (page, keys; statistics, scores), not by bytes: one token behind 1,500 keys of 8 heads (32 query
+// heads of 128 over them) takes 8.9 us for the scores, 15.0 for the values and 5.6 for the sum of the 24 runs.  The tiles of 16 rows
+// took 21.5, 41.5 and 4.9 us for it (bias, mask, exponentials and exchanges for 16 rows, at most 16 runs of 128 keys and more).
+#define SG_KEYS 64
+#define SG_PITCH 72                     // bfloat16 values from a head to the next of the mixed weights in LDS
+#define SG_PARTS (MX_THREADS / MX_HPAD)
+
+struct SingleGeometry {
+    const int32_t* rows;            // [tokens] row of the batch
+    const int32_t* positions;       // [rows of the batch]
+    const int32_t* seq_of_token;    // [rows of the batch] row of the block table
+    const int32_t* block_table;
+    int max_blocks, page, n_q, n_kv, window, keep_first, n_runs, max_tiles;
+    float scale;
+    const float *r1, *r2;           // [n_q] or null
+};
+
+struct Single {
+    int row, pos, lo, kept;                         // it sees keys 0 .. kept - 1 and lo .. pos
+    int kept_tiles, window_tile0, begin, end;       // tiles of 64 keys: 0 .. kept_tiles - 1, then window_tile0 ..; this run's indices
+    const int32_t* table;
+};
+
+__device__ __forceinline__ Single single_of(const SingleGeometry& g, int token, int run) {
+    Single t;
+    t.row = g.rows[token];
+    t.pos = g.positions[t.row];
+    t.table = g.block_table + (size_t)g.seq_of_token[t.row] * g.max_blocks;
+    t.lo = g.window > 0 ? max(0, t.pos - g.window + 1) : 0;
+    t.kept = g.window > 0 ? min(g.keep_first, t.lo) : 0;
+    t.kept_tiles = (t.kept + SG_KEYS - 1) / SG_KEYS;
+    t.window_tile0 = max(t.lo / SG_KEYS, t.kept_tiles);
+    const int total = min(g.max_tiles, t.kept_tiles + t.pos / SG_KEYS - t.window_tile0 + 1);
+    const int chunk = (total + g.n_runs - 1) / g.n_runs;
+    t.begin = min(total, run * chunk);
+    t.end = min(total, t.begin + chunk);
+    return t;
+}
+
+__device__ __forceinline__ int single_key0(const Single& t, int index) {
+    return SG_KEYS * (index < t.kept_tiles ? index : t.window_tile0 + index - t.kept_tiles);
+}
+
+// scores: float32 [tokens][max_tiles][64][32]; stats: float32 [tokens][runs][32][2].
+__global__ void __launch_bounds__(MX_THREADS) mixed_single_scores_kernel(SingleGeometry g, const bf16_t* __restrict__ q,
+                                                                         const bf16_t* __restrict__ k_cache, float* __restrict__ scores,
+                                                                         float* __restrict__ stats) {
+    const int token = blockIdx.y, run = blockIdx.x;
+    const Single t = single_of(g, token, run);
+    const int wave = threadIdx.x / KIPP_WAVE, lane = threadIdx.x & (KIPP_WAVE - 1), l16 = lane & 15, quarter = lane >> 4;
+    const int group = g.n_q / g.n_kv;
+    for (int c = wave; c < g.n_kv; c += MX_WAVES) {
+        const int h = c * group + min(l16, group - 1);      // lanes beyond the head's group compute what nobody reads
+        Frag qf[KSTEPS];
+        const bf16_t* q_at = q + ((size_t)t.row * g.n_q + h) * HEAD_DIM + 8 * quarter;
+#pragma unroll
+        for (int s = 0; s < KSTEPS; ++s) qf[s].u = *(const u32x4*)(q_at + 32 * s);
+        const float a = g.r1 != nullptr ? g.r1[h] : 0.0f, b = g.r2 != nullptr ? g.r2[h] : 0.0f;
+        float m = -INFINITY, l = 0.0f;
+        for (int index = t.begin; index < t.end; ++index) {
+            const int key0 = single_key0(t, index);
+            Frag kf[SG_KEYS / 16][KSTEPS];
+#pragma unroll
+            for (int kb = 0; kb < SG_KEYS / 16; ++kb) {
+                const int key = min(key0 + 16 * kb + l16, t.pos);       // masked below; its load stays inside the context
+                const bf16_t* k_at = k_cache + (((size_t)t.table[key / g.page] * g.n_kv + c) * g.page + key % g.page) * HEAD_DIM + 8 * quarter;
+#pragma unroll
+                for (int s = 0; s < KSTEPS; ++s) kf[kb][s].u = *(const u32x4*)(k_at + 32 * s);
+            }
+            float sc[SG_KEYS / 16][4];
+            float top = m;
+#pragma unroll
+            for (int kb = 0; kb < SG_KEYS / 16; ++kb) {
+                f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int s = 0; s < KSTEPS; ++s) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[kb][s].v, qf[s].v, acc, 0, 0, 0);
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const int j = key0 + 16 * kb + 4 * quarter + v, away = t.pos - j;
+                    sc[kb][v] = away >= 0 && (j >= t.lo || j < t.kept) ? acc[v] * g.scale - a * __logf(1.0f + b * (float)away) : -INFINITY;
+                    top = fmaxf(top, sc[kb][v]);
+                }
+            }
+            if (l16 < group) {
+                float* at = scores + (((size_t)token * g.max_tiles + index) * SG_KEYS + 4 * quarter) * MX_HPAD + h;
+#pragma unroll
+                for (int kb = 0; kb < SG_KEYS / 16; ++kb)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) at[(16 * kb + v) * MX_HPAD] = sc[kb][v];
+            }
+            if (top != -INFINITY) {
+                float sum = 0.0f;
+#pragma unroll
+                for (int kb = 0; kb < SG_KEYS / 16; ++kb)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) sum += __expf(sc[kb][v] - top);     // exp(-inf) = 0
+                l = l * __expf(m - top) + sum;
+                m = top;
+            }
+        }
+#pragma unroll
+        for (int off = 16; off <= 32; off <<= 1) {      // the four lanes that share a head
+            const float m_o = __shfl_xor(m, off, KIPP_WAVE), l_o = __shfl_xor(l, off, KIPP_WAVE);
+            const float m_new = fmaxf(m, m_o);
+            if (m_new != -INFINITY) l = l * __expf(m - m_new) + l_o * __expf(m_o - m_new);
+            m = m_new;
+        }
+        if (quarter == 0 && l16 < group) *(float2*)(stats + (((size_t)token * g.n_runs + run) * MX_HPAD + h) * 2) = make_float2(m, l);
+    }
+}
+
+// partial: float32 [runs][tokens][n_q V_DIM].
+__global__ void __launch_bounds__(MX_THREADS) mixed_single_values_kernel(SingleGeometry g, const bf16_t* __restrict__ v_cache,
+                                                                         const float* __restrict__ scores, const float* __restrict__ stats,
+                                                                         const float* __restrict__ sink, const float* __restrict__ mix,
+                                                                         float* __restrict__ partial) {
+    constexpr int BLOCKS = V_DIM / 16, KS = SG_KEYS / 32;
+    __shared__ __attribute__((aligned(16))) bf16_t p_mixed[2][MX_HPAD * SG_PITCH];
+    __shared__ float2 merged[SG_PARTS][MX_HPAD];
+    __shared__ float2 weigh[MX_HPAD];       // a head's maximum and 1 / denominator
+    const int token = blockIdx.y, run = blockIdx.x, n_tokens = gridDim.y;
+    const Single t = single_of(g, token, run);
+    const int wave = threadIdx.x / KIPP_WAVE, lane = threadIdx.x & (KIPP_WAVE - 1), l16 = lane & 15, quarter = lane >> 4;
+    const int n_q = g.n_q, group = g.n_q / g.n_kv;
+    auto load_values = [&](int c, int key0, Frag (&vf)[KS][BLOCKS]) {
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            const int key = key0 + 32 * ks + 8 * quarter;           // eight keys of one page (a page holds a multiple of 8)
+            const bf16_t* v_at = v_cache + (((size_t)t.table[min(key, t.pos) / g.page] * g.n_kv + c) * V_DIM + l16) * g.page + key % g.page;
+#pragma unroll
+            for (int mb = 0; mb < BLOCKS; ++mb) vf[ks][mb].u = *(const u32x4*)(v_at + (size_t)16 * mb * g.page);
+        }
+    };
+    Frag vf[KS][BLOCKS];
+    if (t.begin < t.end && wave < g.n_kv) load_values(wave, single_key0(t, t.begin), vf);
+
+    // the weights' numbers a head: the runs' statistics, a thread a head and every SG_PARTS-th run; the sink last
+    {
+        const int h = threadIdx.x & (MX_HPAD - 1), part = threadIdx.x / MX_HPAD;
+        float m = -INFINITY, l = 0.0f;
+        if (h < n_q)
+            for (int r0 = part; r0 < g.n_runs; r0 += 4 * SG_PARTS) {
+                float2 st[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    st[i] = r0 + i * SG_PARTS < g.n_runs ? *(const float2*)(stats + (((size_t)token * g.n_runs + r0 + i * SG_PARTS) * MX_HPAD + h) * 2)
+                                                         : make_float2(-INFINITY, 0.0f);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float m_new = fmaxf(m, st[i].x);
+                    if (m_new != -INFINITY) l = l * __expf(m - m_new) + st[i].y * __expf(st[i].x - m_new);
+                    m = m_new;
+                }
+            }
+        merged[part][h] = make_float2(m, l);
+        __syncthreads();
+        if (threadIdx.x < MX_HPAD) {
+#pragma unroll
+            for (int i = 1; i < SG_PARTS; ++i) {
+                const float2 o = merged[i][h];
+                const float m_new = fmaxf(m, o.x);
+                if (m_new != -INFINITY) l = l * __expf(m - m_new) + o.y * __expf(o.x - m_new);
+                m = m_new;
+            }
+            if (sink != nullptr && h < n_q) {
+                const float m_new = fmaxf(m, sink[h]);
+                l = (m == -INFINITY ? 0.0f : l * __expf(m - m_new)) + __expf(sink[h] - m_new);
+                m = m_new;
+            }
+            weigh[h] = make_float2(m, l > 0.0f ? 1.0f / l : 0.0f);
+        }
+        __syncthreads();
+    }
+
+    // this wave mixes 16 keys of a tile for 16 of the mixed heads; mix^T as B operand: column 16 nb + l % 16, contraction heads 8 (l / 16) ..
+    const int kb = wave & 3, nb = wave >> 2;
+    float2 of_head[8];
+    Frag mf;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const int from = 8 * quarter + j, h = 16 * nb + l16;
+        of_head[j] = weigh[from];
+        float w = 0.0f;
+        if (h < n_q && from < n_q) w = mix != nullptr ? mix[h * n_q + from] : (h == from ? 1.0f : 0.0f);
+        mf.h[j] = f32_to_bf16(w);
+    }
+    for (int c0 = 0; c0 < g.n_kv; c0 += MX_WAVES) {         // (more than eight key/value heads: the weights are made again for each eight)
+        const int c = c0 + wave;
+        f32x4 acc[BLOCKS];
+#pragma unroll
+        for (int mb = 0; mb < BLOCKS; ++mb) acc[mb] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+        for (int index = t.begin; index < t.end; ++index) {
+            const int key0 = single_key0(t, index);
+            bf16_t* pm = p_mixed[index & 1];                // the other half is read until every wave is past the barrier
+            if ((c0 > 0 || index > t.begin) && c < g.n_kv) load_values(c, key0, vf);
+            if (16 * nb < n_q) {
+                const float* at = scores + (((size_t)token * g.max_tiles + index) * SG_KEYS + 16 * kb + l16) * MX_HPAD + 8 * quarter;
+                float sc[8];
+                *(f32x4*)sc = *(const f32x4*)at;
+                *(f32x4*)(sc + 4) = *(const f32x4*)(at + 4);
+                Frag hi, lo;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    // (heads that do not exist were never written)
+                    const float p = 8 * quarter + j < n_q && sc[j] != -INFINITY ? __expf(sc[j] - of_head[j].x) * of_head[j].y : 0.0f;
+                    hi.h[j] = to_bf16(p);
+                    lo.h[j] = to_bf16(p - bf16_to_f32(hi.h[j]));
+                }
+                f32x4 d = {0.0f, 0.0f, 0.0f, 0.0f};
+                d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lo.v, mf.v, d, 0, 0, 0);
+                d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hi.v, mf.v, d, 0, 0, 0);
+                uint2 w;                                    // d[v]: key 16 kb + 4 quarter + v, head 16 nb + l16
+                w.x = (uint32_t)to_bf16(d[0]) | ((uint32_t)to_bf16(d[1]) << 16);
+                w.y = (uint32_t)to_bf16(d[2]) | ((uint32_t)to_bf16(d[3]) << 16);
+                *(uint2*)(pm + (16 * nb + l16) * SG_PITCH + 16 * kb + 4 * quarter) = w;
+            }
+            __syncthreads();
+            if (c < g.n_kv) {
+#pragma unroll
+                for (int ks = 0; ks < KS; ++ks) {
+                    const int first = key0 + 32 * ks + 8 * quarter;
+                    const bool whole = first + 7 <= t.pos && (first >= t.lo || first + 7 < t.kept);
+                    Frag pf;
+                    pf.u = *(const u32x4*)(pm + (c * group + min(l16, group - 1)) * SG_PITCH + 32 * ks + 8 * quarter);
+#pragma unroll
+                    for (int mb = 0; mb < BLOCKS; ++mb) {
+                        Frag f = vf[ks][mb];
+                        if (!whole) {           // what the token does not see weighs nothing, but its slots hold anything
+#pragma unroll
+                            for (int j = 0; j < 8; ++j)
+                                if (first + j > t.pos || (first + j < t.lo && first + j >= t.kept)) f.h[j] = 0;
+                        }
+                        acc[mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.v, pf.v, acc[mb], 0, 0, 0);
+                    }
+                }
+            }
+        }
+        // acc[mb][v]: value column 16 mb + 4 quarter + v of the head's l16-th query head
+        if (c < g.n_kv && l16 < group) {
+            float* at = partial + ((size_t)run * n_tokens + token) * ((size_t)n_q * V_DIM) + (size_t)(c * group + l16) * V_DIM + 4 * quarter;
+#pragma unroll
+            for (int mb = 0; mb < BLOCKS; ++mb) *(f32x4*)(at + 16 * mb) = acc[mb];
+        }
+        if (c0 + MX_WAVES < g.n_kv) __syncthreads();
+    }
+}
+
 // Rows whose keys were cut into runs: out = gate * (sum of the runs' partial sums, in order).  A thread takes four
-// columns of a row and asks for every run's sums before it adds the first.
+// columns of a row and asks for every run's sums before it adds the first.  `rows` (or null: every row of the batch): the
+// rows whose sums lie one after the other, all of `runs` runs; else a row's own number of them (one: it is written already).
 __global__ void __launch_bounds__(256) mixed_finish_kernel(const float* __restrict__ partial, size_t partial_stride,
-                                                           const int32_t* __restrict__ row_splits, const float* __restrict__ gate,
+                                                           const int32_t* __restrict__ row_splits, const int32_t* __restrict__ rows, int runs,
+                                                           const float* __restrict__ gate,
                                                            int gate_stride, int gate_parts, size_t gate_part_stride,
                                                            bf16_t* __restrict__ out, int width) {
-    const size_t row = blockIdx.y;
-    const int n = row_splits[row];
+    const size_t at_row = blockIdx.y, row = rows != nullptr ? rows[at_row] : at_row;
+    const int n = rows != nullptr ? runs : row_splits[row];
     const int e = 4 * (blockIdx.x * 256 + threadIdx.x);
-    if (n <= 1 || e >= width) return;
+    if ((rows == nullptr && n <= 1) || e >= width) return;
     f32x4 o = {0.0f, 0.0f, 0.0f, 0.0f};
     for (int s0 = 0; s0 < n; s0 += 8) {
         f32x4 part[8];
 #pragma unroll
         for (int s = 0; s < 8; ++s)
-            part[s] = s0 + s < n ? *(const f32x4*)(partial + (s0 + s) * partial_stride + row * width + e) : (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+            part[s] = s0 + s < n ? *(const f32x4*)(partial + (s0 + s) * partial_stride + at_row * width + e) : (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int s = 0; s < 8; ++s) o += part[s];
     }
@@ -569,8 +832,33 @@ int kipp_mixed_attention_mfma(const void* q, const void* k_cache, const void* v_
                        (const bf16_t*)k_cache, (const bf16_t*)v_cache, stats, sink, mix, gate, gate_stride, gate_parts,
                        gate_part_stride, (bf16_t*)out, partial, partial_stride);
     if (max_splits > 1)
-        hipLaunchKernelGGL(mixed_finish_kernel, dim3((n_q * V_DIM / 4 + 255) / 256, n_rows), dim3(256), 0, stream, partial, partial_stride, row_splits, gate,
-                           gate_stride, gate_parts, gate_part_stride, (bf16_t*)out, n_q * V_DIM);
+        hipLaunchKernelGGL(mixed_finish_kernel, dim3((n_q * V_DIM / 4 + 255) / 256, n_rows), dim3(256), 0, stream, partial, partial_stride, row_splits,
+                           (const int32_t*)nullptr, 0, gate, gate_stride, gate_parts, gate_part_stride, (bf16_t*)out, n_q * V_DIM);
+    return KIPP_LAUNCH_CHECK();
+}
+
+// Single tokens: rows[i] of the batch for i < n_tokens.  scores: float32 [n_tokens][max_tiles][64][32]; stats: float32
+// [n_tokens][n_runs][32][2]; partial: float32 [n_runs][n_tokens][n_q V_DIM]; out: bfloat16 [n_rows][n_q V_DIM], the rows named.
+// max_tiles: tiles of 64 keys that a token can see at most.
+int kipp_mixed_attention_single(const void* q, const void* k_cache, const void* v_cache, void* out, const float* gate, int gate_stride,
+                                int gate_parts, const int32_t* rows, int n_tokens, const int32_t* positions, const int32_t* seq_of_token,
+                                const int32_t* block_table, int max_blocks, const float* r1, const float* r2, const float* sink,
+                                const float* mix, float* scores, float* stats, float* partial, int n_runs, int max_tiles, int n_rows, int n_q,
+                                int n_kv, int d, int dv, int page, float scale, int window, int keep_first, hipStream_t stream) {
+    if (n_tokens <= 0 || n_rows <= 0) return 0;
+    if (d != HEAD_DIM || dv != V_DIM || n_kv <= 0 || n_q % n_kv || n_q > MX_HPAD || n_q / n_kv > 16) return -1;
+    if (page <= 0 || page % 16 || n_runs < 1 || max_tiles < 1) return -2;
+    SingleGeometry g;
+    g.rows = rows; g.positions = positions; g.seq_of_token = seq_of_token; g.block_table = block_table;
+    g.max_blocks = max_blocks; g.page = page; g.n_q = n_q; g.n_kv = n_kv; g.window = window; g.keep_first = keep_first;
+    g.n_runs = n_runs; g.max_tiles = max_tiles; g.scale = scale; g.r1 = r1; g.r2 = r2;
+    hipLaunchKernelGGL(mixed_single_scores_kernel, dim3(n_runs, n_tokens), dim3(MX_THREADS), 0, stream, g, (const bf16_t*)q, (const bf16_t*)k_cache,
+                       scores, stats);
+    hipLaunchKernelGGL(mixed_single_values_kernel, dim3(n_runs, n_tokens), dim3(MX_THREADS), 0, stream, g, (const bf16_t*)v_cache,
+                       (const float*)scores, (const float*)stats, sink, mix, partial);
+    hipLaunchKernelGGL(mixed_finish_kernel, dim3((n_q * V_DIM / 4 + 255) / 256, n_tokens), dim3(256), 0, stream, (const float*)partial,
+                       (size_t)n_tokens * n_q * V_DIM, (const int32_t*)nullptr, rows, n_runs, gate, gate_stride, gate_parts,
+                       (size_t)n_rows * gate_stride, (bf16_t*)out, n_q * V_DIM);
     return KIPP_LAUNCH_CHECK();
 }
 

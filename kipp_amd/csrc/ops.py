@@ -1340,6 +1340,62 @@ def mixed_attention_mfma(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.
     return out
 
 
+MIXED_SINGLE_KEYS = 64          # keys of a tile of the form for single tokens
+MIXED_SINGLE_BYTES = 512 << 20  # most bytes of scores it may keep between its two walks
+
+
+def mixed_single_plan(n_tokens: int, max_ctx: int, window: int, keep_first: int):
+    """(tiles of 64 keys a token sees at most, runs they are cut into) for single tokens in contexts of up to `max_ctx`: runs of
+    one tile until they fill the chip about four times, and at most 128 of them, whose sums a last kernel adds."""
+    keys = MIXED_SINGLE_KEYS
+    tiles = -(-max_ctx // keys)
+    if window:
+        tiles = min(tiles, -(-keep_first // keys) + -(-window // keys) + 1)
+    return max(tiles, 1), max(1, min(tiles, 128, -(-4 * COMPUTE_UNITS // max(n_tokens, 1))))
+
+
+def mixed_single_ok(n_q: int, n_kv: int, n_tokens: int, tiles: int) -> bool:
+    """Whether single tokens take their own form: up to 16 query heads a key/value head, and scores that fit the space for them."""
+    return n_q // n_kv <= 16 and n_tokens * tiles * MIXED_SINGLE_KEYS * 32 * 4 <= MIXED_SINGLE_BYTES
+
+
+def mixed_single_workspace(n_tokens: int, n_q: int, dv: int, tiles: int, runs: int, device) -> tuple:
+    """(scores, statistics, partial sums) of the form for single tokens."""
+    new = lambda *shape: torch.empty(shape, dtype=torch.float32, device=device)  # noqa: E731
+    return new(n_tokens, tiles, MIXED_SINGLE_KEYS, 32), new(n_tokens, runs, 32, 2), new(runs, n_tokens, n_q * dv)
+
+
+def mixed_attention_single(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, out: torch.Tensor, rows: torch.Tensor,
+                           positions: torch.Tensor, seq_of_token: torch.Tensor, block_table: torch.Tensor,
+                           n_q: int, n_kv: int, d: int, dv: int, scale: float, window: int, keep_first: int,
+                           r1: Optional[torch.Tensor], r2: Optional[torch.Tensor], sink: Optional[torch.Tensor],
+                           mix: Optional[torch.Tensor], workspace: tuple, gate: Optional[torch.Tensor] = None,
+                           gate_at: int = 0) -> torch.Tensor:
+    """The same attention on the matrix cores for single tokens: the rows of the batch that `rows` names, each with every key of
+    its sequence up to its own position.  `workspace` from `mixed_single_workspace`, made for contexts at least as long."""
+    scores, stats, partial = workspace
+    _dev(q, k_cache, v_cache, out, rows, positions, seq_of_token, block_table, r1, r2, sink, mix, gate, scores, stats, partial)
+    for t, name in ((rows, "rows"), (positions, "positions"), (seq_of_token, "seq_of_token"), (block_table, "block_table")):
+        _i32(t, name)
+    n, gate_parts, gate_stride = _mixed_common(q, k_cache, v_cache, out, gate, gate_at, n_q, n_kv, d, dv, r1, r2, sink, mix,
+                                               "mixed_attention_single")
+    tokens, tiles, runs = rows.numel(), scores.shape[1], stats.shape[1]
+    _need(all(t.dtype == torch.bfloat16 for t in (q, k_cache, v_cache, out)), "mixed_attention_single: bfloat16 queries, caches and output")
+    _need(mixed_attention_fast_ok(n_q, d, dv, k_cache.shape[2]) and n_q // n_kv <= 16, "mixed_attention_single: sizes refused (the other forms take them)")
+    _need(scores.shape[0] >= tokens and stats.shape[0] >= tokens and partial.shape[0] >= runs and partial.numel() >= runs * tokens * n_q * dv,
+          "mixed_attention_single: the workspace is too small")
+    _need(positions.numel() == n and seq_of_token.numel() == n and block_table.dim() == 2, "mixed_attention_single: one position and sequence a row")
+    fn = _fn("attention_mixed_mfma", "kipp_mixed_attention_single",
+             [_c_ptr] * 5 + [_c_int, _c_int, _c_ptr, _c_int] + [_c_ptr] * 3 + [_c_int] + [_c_ptr] * 7 + [_c_int] * 8 + [_c_float, _c_int, _c_int, _c_ptr],
+             mixed_attention_defines(n_q, n_kv, d, dv))
+    gate_ptr = gate.data_ptr() + 4 * gate_at if gate is not None else None
+    _check(fn(_ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(out), gate_ptr, gate_stride, gate_parts, _ptr(rows), tokens, _ptr(positions),
+              _ptr(seq_of_token), _ptr(block_table), block_table.shape[1], _ptr(r1), _ptr(r2), _ptr(sink), _ptr(mix), _ptr(scores), _ptr(stats),
+              _ptr(partial), runs, tiles, n, n_q, n_kv, d, dv, k_cache.shape[2], float(scale), int(window), int(keep_first), _stream()),
+           "mixed_attention_single")
+    return out
+
+
 PREFILL_MAX_BLOCKS = 4096   # table entries of one sequence the prefill kernel stages in LDS
 
 

@@ -112,12 +112,17 @@ class MixedHeadAttention:
         gate_at = s.q_dim + s.kv_dim + s.v_dim
         if rt.dtype == "bfloat16" and getattr(rt, "mixed_attention_fast", True) \
                 and ops.mixed_attention_fast_ok(s.num_heads, s.head_dim, s.v_head_dim, cache.page_size):
-            items, n_items, row_splits, max_splits, workspace = self._items(batch)
-            ops.mixed_attention_mfma(q, cache.k, cache.v, out, items, n_items, row_splits, max_splits,
-                                     batch.q_start, batch.q_len, batch.ctx_len, table,
-                                     s.num_heads, s.num_kv_heads, s.head_dim, s.v_head_dim, s.scale, s.window or 0,
-                                     s.keep_first, self.r1, self.r2, self.sink, self.mix, workspace,
-                                     gate=proj if s.output_gate else None, gate_at=gate_at)
+            numbers = (s.num_heads, s.num_kv_heads, s.head_dim, s.v_head_dim, s.scale, s.window or 0, s.keep_first,
+                       self.r1, self.r2, self.sink, self.mix)
+            single, tiles = self._items(batch)
+            if single is not None:
+                ops.mixed_attention_single(q, cache.k, cache.v, out, batch.decode_rows, batch.positions, batch.seq_of_token, table,
+                                           *numbers, single, gate=proj if s.output_gate else None, gate_at=gate_at)
+            if tiles is not None:
+                items, n_items, row_splits, max_splits, workspace = tiles
+                ops.mixed_attention_mfma(q, cache.k, cache.v, out, items, n_items, row_splits, max_splits,
+                                         batch.q_start, batch.q_len, batch.ctx_len, table, *numbers, workspace,
+                                         gate=proj if s.output_gate else None, gate_at=gate_at)
             return rt.linear(out, self.w_o, slabs=True, defer=True)
         if rt.dtype == "bfloat16":
             rt.generic_attention_launches += 1      # the slow kernel class: a measurement must know it ran
@@ -128,8 +133,9 @@ class MixedHeadAttention:
         return rt.linear(out, self.w_o, slabs=True, defer=True)
 
     def _items(self, batch):
-        """The item list of the matrix-core form: every entry's rows in tiles of 16, and where the tiles alone are too
-        few workgroups to fill the GPU, each tile's keys in several runs (at least 128 keys a run, at most 16 runs).
+        """What the matrix-core forms work through: the space of the one for single tokens (None: there are none, or it does not
+        take them), and the item list of the other (None: every entry brings one token): every entry's rows in tiles of 16, and where
+        the tiles alone are too few workgroups to fill the GPU, each tile's keys in several runs (at least 128 keys a run, at most 16 runs).
         Made by the first layer of a geometry and kept while the batch object lives: a recorded step keeps its own,
         made for the longest context of its class (the kernels take the true lengths from the device)."""
         s, ops = self.spec, self.rt.ops
@@ -138,8 +144,15 @@ class MixedHeadAttention:
         if work is None:
             rows_tile, keys_tile = ops.MIXED_ROWS, ops.MIXED_KEYS
             window, keep = s.window or 0, s.keep_first
+            single = None
+            if batch.n_decode:
+                seen, runs = ops.mixed_single_plan(batch.n_decode, batch.max_decode_ctx, window, keep)
+                if ops.mixed_single_ok(s.num_heads, s.num_kv_heads, batch.n_decode, seen):
+                    single = ops.mixed_single_workspace(batch.n_decode, s.num_heads, s.v_head_dim, seen, runs, self.rt.device)
             tiles = []
             for e, (n, ctx) in enumerate(zip(batch.host["q_len"], batch.host["ctx_len"])):
+                if n == 1 and single is not None:
+                    continue
                 for row0 in range(0, n, rows_tile):
                     rows = min(rows_tile, n - row0)
                     pos0 = ctx - n + row0
@@ -148,18 +161,21 @@ class MixedHeadAttention:
                     kept_tiles = (kept - 1) // keys_tile + 1 if kept > 0 else 0
                     first = max(lo // keys_tile, kept_tiles)
                     tiles.append((e, row0, rows, kept_tiles + (pos0 + rows - 1) // keys_tile - first + 1))
+            if not tiles:
+                batch.host[key] = (single, None)
+                return batch.host[key]
             want = -(-2 * ops.compute_units(self.rt.device) // len(tiles))
-            entry, row0s, split, nsplits, row_splits = [], [], [], [], []
+            entry, row0s, split, nsplits, row_splits = [], [], [], [], [1] * batch.n_tokens
             for e, row0, rows, key_tiles in tiles:
                 runs = max(1, min(16, key_tiles // 4, want))
                 entry += [e] * runs
                 row0s += [row0] * runs
                 split += list(range(runs))
                 nsplits += [runs] * runs
-                row_splits += [runs] * rows
+                at = batch.host["q_start"][e] + row0
+                row_splits[at:at + rows] = [runs] * rows
             most = max(nsplits)
             lists = batch.upload(entry, row0s, split, nsplits, row_splits)
             space = ops.mixed_attention_workspace(len(entry), batch.n_tokens, s.num_heads, s.v_head_dim, most, self.rt.device)
-            work = (tuple(lists[:4]), len(entry), lists[4], most, space)
-            batch.host[key] = work
+            work = batch.host[key] = (single, (tuple(lists[:4]), len(entry), lists[4], most, space))
         return work
