@@ -24,13 +24,14 @@
 // An output element is summed over K in the same order whatever the tile and the number of waves: cuts
 // with the same parts of K give the same bits.
 //
-// The result leaves through one of four ends:
+// The result leaves through one of five ends:
 //   slabs   float32 [parts, M, N]: K is split over `parts` workgroups (grid.z) where the tiles
 //           alone would leave compute units idle, and the consumer adds the slabs in order
 //           (the residual add, the rotary kernel: no atomics, the same bits every time);
 //   swiglu  W = [gate; up] ([2 I, K]): a wave's columns are gate rows and the up rows that belong
 //           to them, a lane holds both values of an output, and bfloat16(silu(gate) * up)
 //           [M, I] is all that is written (/root/reference/src/kipp.c:2633-2653);
+//   glu     the same with silu or relu, and maybe a bias on gate and up ahead of it;
 //   bf16    bfloat16 [M, N];
 //   relu2   bfloat16 [M, N] = bfloat16(relu(product)^2).
 // The bfloat16 ends pass through LDS so that a lane stores 16 bytes of one row.
@@ -39,12 +40,20 @@
 // eighth one) take tiles that share their rows of W, which that die's L2 then serves.
 #include "tile_walk.h"
 
-enum { END_SLABS = 0, END_SWIGLU = 1, END_BF16 = 2, END_RELU2 = 3 };
+enum { END_SLABS = 0, END_SWIGLU = 1, END_BF16 = 2, END_RELU2 = 3, END_GLU = 4 };
+constexpr bool pairs_columns(int end) { return end == END_SWIGLU || end == END_GLU; }      // W = [gate; up]
 
 // silu(g) * u with the exponential of the hardware (base 2)
 __device__ __forceinline__ float swiglu_of(float g, float u) {
     return g / (1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * g)) * u;
 }
+
+// What the end END_GLU computes of gate + its bias and up + its bias: as swiglu_of, or with relu in silu's place.  (A product of
+// 2,048 x 2,560 with 2 x 9,728 columns that ends in relu: 213 us; as slabs of float32 and an activation behind them it took 232 + 71.)
+struct Glu {
+    const float* bias;      // [2 inner]: the gate's, then the up's; or null
+    int relu;
+};
 
 // Steps of K that are in LDS or on their way there: four.  (Tiles of half the size with three steps and two
 // workgroups a compute unit, i.e. two waves a SIMD from two workgroups, were measured and are no faster: those
@@ -58,7 +67,7 @@ struct Depth {
 template <int WM, int WN, int END, int WGN = 2>
 __global__ void __launch_bounds__(64 * 2 * WGN, 1) gemm_tiles_kernel(
     const bf16_t* __restrict__ X, const bf16_t* __restrict__ W, void* __restrict__ Y, int M, int N, int K,
-    int tiles_m, int tiles_n, int parts, int inner, int col_begin, int col_end) {
+    int tiles_m, int tiles_n, int parts, int inner, int col_begin, int col_end, Glu glu) {
     constexpr int STAGES = Depth<WM, WN>::value;
     constexpr int WAVES = 2 * WGN;                                // 2 down, WGN across (2: one wave a SIMD, 4: two)
     constexpr int TM = 64 * WM, TN = 32 * WN * WGN;               // the workgroup's tile
@@ -66,7 +75,7 @@ __global__ void __launch_bounds__(64 * 2 * WGN, 1) gemm_tiles_kernel(
     constexpr int STAGE_BYTES = X_PIECE + W_PIECE;
     constexpr int XI = TM / INSTR_ROWS / WAVES, WI = TN / INSTR_ROWS / WAVES;   // DMA instructions of a wave for each piece
     static_assert(XI >= 1 && XI * INSTR_ROWS * WAVES == TM && WI * INSTR_ROWS * WAVES == TN, "the waves share the pieces evenly");
-    constexpr int OUT_N = END == END_SWIGLU ? TN / 2 : TN;        // output columns of a tile
+    constexpr int OUT_N = pairs_columns(END) ? TN / 2 : TN;        // output columns of a tile
     static_assert((WM == 2 || WM == 4) && (WN == 2 || WN == 3 || WN == 4), "wave tiles of 2 or 4 MFMA tiles down, 2 to 4 across");
     static_assert(WN != 3 || END == END_SLABS, "three tiles across only for the float32 end");
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
@@ -107,7 +116,7 @@ __global__ void __launch_bounds__(64 * 2 * WGN, 1) gemm_tiles_kernel(
     for (int i = 0; i < WI; ++i) {
         const int r = (TN / WAVES) * wave + INSTR_ROWS * i + lane_row;    // row of the piece
         int wr;
-        if (END == END_SWIGLU) {
+        if (pairs_columns(END)) {
             // the 32 WN rows of the piece that a wave multiplies are 16 WN gate rows, then the 16 WN up rows that
             // belong to them (`half`: which of the WGN waves across)
             const int half = r / (32 * WN), within = r % (32 * WN);
@@ -145,15 +154,24 @@ __global__ void __launch_bounds__(64 * 2 * WGN, 1) gemm_tiles_kernel(
     if constexpr (WN == 3) return;
     // bfloat16 ends: the wave's outputs, 32 rows at a time, go through its own corner of LDS (now free), from
     // which a lane takes 8 neighbouring columns of one row: 16 bytes a store, whole memory lines a row
-    constexpr int WCOLS = END == END_SWIGLU ? 16 * WN : 32 * WN;   // output columns of a wave
+    constexpr int WCOLS = pairs_columns(END) ? 16 * WN : 32 * WN;   // output columns of a wave
     constexpr int PITCH = WCOLS + 8;                               // bf16 elements a staged row (the pad spreads the banks)
     static_assert(32 * PITCH * 2 <= STAGES * STAGE_BYTES / WAVES, "a wave's staging fits its share of LDS");
     __syncthreads();                                               // every wave is done reading operands
     bf16_t* stage = (bf16_t*)(lds + wave * (STAGES * STAGE_BYTES / WAVES));
     bf16_t* out = (bf16_t*)Y;
-    const int out_width = END == END_SWIGLU ? inner : N;
+    const int out_width = pairs_columns(END) ? inner : N;
     const int col0 = col_begin + tn * OUT_N + wn * WCOLS;
     constexpr int LANES_PER_ROW = WCOLS / 8, ROWS_PER_PASS = 64 / LANES_PER_ROW;
+    float bias_gate[WCOLS / 32], bias_up[WCOLS / 32];
+    if (END == END_GLU) {
+#pragma unroll
+        for (int j = 0; j < WCOLS / 32; ++j) {
+            const int col = min(col0 + 32 * j + l32, col_end - 1);
+            bias_gate[j] = glu.bias != nullptr ? glu.bias[col] : 0.0f;
+            bias_up[j] = glu.bias != nullptr ? glu.bias[inner + col] : 0.0f;
+        }
+    }
 #pragma unroll
     for (int i = 0; i < WM; ++i) {
 #pragma unroll
@@ -162,6 +180,10 @@ __global__ void __launch_bounds__(64 * 2 * WGN, 1) gemm_tiles_kernel(
             for (int v = 0; v < 16; ++v) {
                 const int r = 8 * (v / 4) + 4 * hh + (v % 4);
                 float value = END == END_SWIGLU ? swiglu_of(acc[i][j][v], acc[i][(j + WN / 2) % WN][v]) : acc[i][j][v];
+                if (END == END_GLU) {
+                    const float gate = acc[i][j][v] + bias_gate[j], up = acc[i][(j + WN / 2) % WN][v] + bias_up[j];
+                    value = glu.relu ? fmaxf(gate, 0.0f) * up : swiglu_of(gate, up);
+                }
                 if (END == END_RELU2) {
                     value = fmaxf(value, 0.0f);
                     value *= value;
@@ -205,7 +227,7 @@ static const double kStep[N_SHAPES] = {0.80, 0.62, 0.47, 0.47, 0.27};    // one 
 static const double kFixed[N_SHAPES] = {13.0, 11.0, 9.0, 9.0, 6.0};      // start and end of a tile
 
 static double cut_cost(int M, int cols, int steps, int end, int shape, int parts) {
-    const int tm = 64 * kShapes[shape][0], tn = end == END_SWIGLU ? 32 * kShapes[shape][1] : 64 * kShapes[shape][1];
+    const int tm = 64 * kShapes[shape][0], tn = pairs_columns(end) ? 32 * kShapes[shape][1] : 64 * kShapes[shape][1];
     const long long tiles = (long long)((M + tm - 1) / tm) * ((cols + tn - 1) / tn);
     const long long rounds = (tiles * parts + 255) / 256;
     return rounds * (kFixed[shape] + kStep[shape] * ((steps + parts - 1) / parts)) + 1.0 * (parts - 1);
@@ -217,7 +239,7 @@ static double cut_cost(int M, int cols, int steps, int end, int shape, int parts
 // Without whole rounds, or with nothing left, one cut of the 8-wave tile.
 static int whole_rounds_then_rest(int M, int cols, int end, int rest, Cut* cuts) {
     cuts[0] = {4, 2, 1, 0, cols, 4};
-    const int tm = 256, tn = (end == END_SWIGLU ? 16 : 32) * 2 * 4;
+    const int tm = 256, tn = (pairs_columns(end) ? 16 : 32) * 2 * 4;
     const int tiles_m = (M + tm - 1) / tm;
     const long long whole = ((long long)tiles_m * (cols / tn)) / 256 * 256;
     const int first_cols = (int)(whole / tiles_m) * tn;
@@ -233,7 +255,7 @@ static int whole_rounds_then_rest(int M, int cols, int end, int rest, Cut* cuts)
 // that would hold the 256 units for another whole round, the rest of the columns is cut into smaller tiles.
 static int plan(int M, int N, int K, int end, int max_parts, Cut* cuts) {
     const int steps = K / BK;
-    const int cols = end == END_SWIGLU ? N / 2 : N;
+    const int cols = pairs_columns(end) ? N / 2 : N;
     double best = 1e30;
     int n_cuts = 1;
     for (int s = 0; s < N_SHAPES; ++s) {
@@ -246,14 +268,14 @@ static int plan(int M, int N, int K, int end, int max_parts, Cut* cuts) {
             }
         }
     }
-    if (end == END_SWIGLU && M >= 512) {
+    if (pairs_columns(end) && M >= 512) {
         // from 512 rows on the 8-wave tile is the faster one for this end, measured at 512, 1,024 and 2,048 rows of the 4B
         // shape (57 against 65 us, 115 against 114, 196 against 209); an element's sum does not depend on the tile
         return whole_rounds_then_rest(M, cols, end, 0, cuts);
     }
     if (end != END_SLABS) {
         // whole rounds of the largest tile first, the rest of the columns in smaller tiles
-        const int tn = end == END_SWIGLU ? 128 : 256;
+        const int tn = pairs_columns(end) ? 128 : 256;
         const int tiles_m = (M + 255) / 256;
         const long long whole = ((long long)tiles_m * (cols / tn)) / 256 * 256;      // tiles of whole rounds
         const int first_cols = (int)(whole / tiles_m) * tn;
@@ -273,7 +295,7 @@ static int plan(int M, int N, int K, int end, int max_parts, Cut* cuts) {
 }
 
 template <int WM, int WN, int END, int WGN = 2>
-static int launch_cut(const void* X, const void* W, void* Y, int M, int N, int K, const Cut& cut, hipStream_t stream) {
+static int launch_cut(const void* X, const void* W, void* Y, int M, int N, int K, const Cut& cut, hipStream_t stream, Glu glu) {
     constexpr int lds_bytes = Depth<WM, WN>::value * (64 * WM + 32 * WN * WGN) * BK * 2;
     static bool prepared = false;
     if (!prepared) {
@@ -282,32 +304,62 @@ static int launch_cut(const void* X, const void* W, void* Y, int M, int N, int K
             return -6;
         prepared = true;
     }
-    const int tm = 64 * WM, tn = (END == END_SWIGLU ? 16 : 32) * WN * WGN;
+    const int tm = 64 * WM, tn = (pairs_columns(END) ? 16 : 32) * WN * WGN;
     const int tiles_m = (M + tm - 1) / tm, tiles_n = (cut.col_end - cut.col_begin + tn - 1) / tn;
     const int per_die = (tiles_m * tiles_n + 7) / 8;
     hipLaunchKernelGGL((gemm_tiles_kernel<WM, WN, END, WGN>), dim3(per_die * 8, 1, cut.parts), dim3(64 * 2 * WGN), lds_bytes, stream,
                        (const bf16_t*)X, (const bf16_t*)W, Y, M, N, K, tiles_m, tiles_n, cut.parts, N / 2, cut.col_begin,
-                       cut.col_end);
+                       cut.col_end, glu);
     return KIPP_LAUNCH_CHECK();
 }
 
 template <int END>
-static int launch_end(const void* X, const void* W, void* Y, int M, int N, int K, const Cut& cut, hipStream_t stream) {
+static int launch_end(const void* X, const void* W, void* Y, int M, int N, int K, const Cut& cut, hipStream_t stream, Glu glu) {
     if (cut.wgn == 4) {
         // 8 waves, two a SIMD: the same workgroup tiles from wave tiles half as wide
-        if (cut.wm == 4 && cut.wn == 2) return launch_cut<4, 2, END, 4>(X, W, Y, M, N, K, cut, stream);
-        if (cut.wm == 2 && cut.wn == 2) return launch_cut<2, 2, END, 4>(X, W, Y, M, N, K, cut, stream);
+        if (cut.wm == 4 && cut.wn == 2) return launch_cut<4, 2, END, 4>(X, W, Y, M, N, K, cut, stream, glu);
+        if (cut.wm == 2 && cut.wn == 2) return launch_cut<2, 2, END, 4>(X, W, Y, M, N, K, cut, stream, glu);
         return -5;
     }
-    if (cut.wm == 4 && cut.wn == 4) return launch_cut<4, 4, END>(X, W, Y, M, N, K, cut, stream);
-    if (cut.wm == 4 && cut.wn == 2) return launch_cut<4, 2, END>(X, W, Y, M, N, K, cut, stream);
-    if (cut.wm == 2 && cut.wn == 4) return launch_cut<2, 4, END>(X, W, Y, M, N, K, cut, stream);
-    if (cut.wm == 2 && cut.wn == 2) return launch_cut<2, 2, END>(X, W, Y, M, N, K, cut, stream);
+    if (cut.wm == 4 && cut.wn == 4) return launch_cut<4, 4, END>(X, W, Y, M, N, K, cut, stream, glu);
+    if (cut.wm == 4 && cut.wn == 2) return launch_cut<4, 2, END>(X, W, Y, M, N, K, cut, stream, glu);
+    if (cut.wm == 2 && cut.wn == 4) return launch_cut<2, 4, END>(X, W, Y, M, N, K, cut, stream, glu);
+    if (cut.wm == 2 && cut.wn == 2) return launch_cut<2, 2, END>(X, W, Y, M, N, K, cut, stream, glu);
     if constexpr (END == END_SLABS) {
-        if (cut.wm == 4 && cut.wn == 3) return launch_cut<4, 3, END>(X, W, Y, M, N, K, cut, stream);
-        if (cut.wm == 2 && cut.wn == 3) return launch_cut<2, 3, END>(X, W, Y, M, N, K, cut, stream);
+        if (cut.wm == 4 && cut.wn == 3) return launch_cut<4, 3, END>(X, W, Y, M, N, K, cut, stream, glu);
+        if (cut.wm == 2 && cut.wn == 3) return launch_cut<2, 3, END>(X, W, Y, M, N, K, cut, stream, glu);
     }
     return -5;
+}
+
+static int launch_product(const void* X, const void* W, void* Y, int M, int N, int K, int end, int max_parts, int force, Glu glu,
+                          hipStream_t stream) {
+    if (M <= 0 || N <= 0) return 0;
+    if (K <= 0 || (K % BK) || max_parts <= 0) return -1;
+    if (pairs_columns(end) && (N & 1)) return -4;
+    // a lane's offset into an operand is 32 bits wide
+    if ((unsigned long long)M * K * 2 >= (1ull << 32) || (unsigned long long)N * K * 2 >= (1ull << 32)) return -6;
+    Cut cuts[2];
+    int n_cuts = plan(M, N, K, end, max_parts, cuts);
+    if (force) {
+        const int cols = pairs_columns(end) ? N / 2 : N;
+        n_cuts = 1;
+        const int rest_code = force / 10000;         // + 10000 r: the tile of the columns that + 2000 leaves (below)
+        force %= 10000;
+        cuts[0] = {(force / 100) % 10, (force / 10) % 10, force % 10, 0, cols, force >= 1000 ? 4 : 2};
+        if (force >= 2000 && end != END_SLABS) n_cuts = whole_rounds_then_rest(M, cols, end, rest_code, cuts);   // + 2000 (above)
+    }
+    for (int c = 0; c < n_cuts; ++c) {
+        const Cut& cut = cuts[c];
+        if (cut.parts < 1 || cut.parts > K / BK || (end != END_SLABS && cut.parts != 1)) return -2;
+        const int rc = end == END_SLABS ? launch_end<END_SLABS>(X, W, Y, M, N, K, cut, stream, glu)
+                       : end == END_SWIGLU ? launch_end<END_SWIGLU>(X, W, Y, M, N, K, cut, stream, glu)
+                       : end == END_GLU    ? launch_end<END_GLU>(X, W, Y, M, N, K, cut, stream, glu)
+                       : end == END_RELU2  ? launch_end<END_RELU2>(X, W, Y, M, N, K, cut, stream, glu)
+                                           : launch_end<END_BF16>(X, W, Y, M, N, K, cut, stream, glu);
+        if (rc != 0) return rc;
+    }
+    return 0;
 }
 
 extern "C" {
@@ -325,31 +377,15 @@ int kipp_gemm_tiles_parts(int M, int N, int K, int end, int max_parts) {
 int kipp_gemm_tiles(const void* X, const void* W, void* Y, int M, int N, int K, int end, int max_parts, int force,
                     hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;
-    if (K <= 0 || (K % BK) || max_parts <= 0) return -1;
     if (end != END_SLABS && end != END_SWIGLU && end != END_BF16 && end != END_RELU2) return -3;
-    if (end == END_SWIGLU && (N & 1)) return -4;
-    // a lane's offset into an operand is 32 bits wide
-    if ((unsigned long long)M * K * 2 >= (1ull << 32) || (unsigned long long)N * K * 2 >= (1ull << 32)) return -6;
-    Cut cuts[2];
-    int n_cuts = plan(M, N, K, end, max_parts, cuts);
-    if (force) {
-        const int cols = end == END_SWIGLU ? N / 2 : N;
-        n_cuts = 1;
-        const int rest_code = force / 10000;         // + 10000 r: the tile of the columns that + 2000 leaves (below)
-        force %= 10000;
-        cuts[0] = {(force / 100) % 10, (force / 10) % 10, force % 10, 0, cols, force >= 1000 ? 4 : 2};
-        if (force >= 2000 && end != END_SLABS) n_cuts = whole_rounds_then_rest(M, cols, end, rest_code, cuts);   // + 2000 (above)
-    }
-    for (int c = 0; c < n_cuts; ++c) {
-        const Cut& cut = cuts[c];
-        if (cut.parts < 1 || cut.parts > K / BK || (end != END_SLABS && cut.parts != 1)) return -2;
-        const int rc = end == END_SLABS ? launch_end<END_SLABS>(X, W, Y, M, N, K, cut, stream)
-                       : end == END_SWIGLU ? launch_end<END_SWIGLU>(X, W, Y, M, N, K, cut, stream)
-                       : end == END_RELU2  ? launch_end<END_RELU2>(X, W, Y, M, N, K, cut, stream)
-                                           : launch_end<END_BF16>(X, W, Y, M, N, K, cut, stream);
-        if (rc != 0) return rc;
-    }
-    return 0;
+    return launch_product(X, W, Y, M, N, K, end, max_parts, force, Glu{}, stream);
+}
+
+// Y: bfloat16 [M, N / 2] = act(gate + its bias) * (up + its bias) for W = [gate; up], act relu (`relu` 1) or silu (0); `bias`: float32 [N],
+// as W's rows, or null.  `force` as above.
+int kipp_gemm_tiles_glu(const void* X, const void* W, void* Y, int M, int N, int K, int relu, const float* bias, int force,
+                        hipStream_t stream) {
+    return launch_product(X, W, Y, M, N, K, END_GLU, 1, force, Glu{bias, relu != 0}, stream);
 }
 
 }  // extern "C"

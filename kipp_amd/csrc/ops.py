@@ -1923,7 +1923,7 @@ def gemm_rows_relu2(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, tiles: 
     return out
 
 
-TILES_END = {"slabs": 0, "swiglu": 1, "bf16": 2, "relu2": 3}
+TILES_END = {"slabs": 0, "swiglu": 1, "bf16": 2, "relu2": 3, "glu": 4}
 
 
 def gemm_tiles_ok(m: int, k: int, n: int = 1) -> bool:
@@ -1937,10 +1937,12 @@ def gemm_tiles_parts(m: int, n: int, k: int, end: str = "slabs", max_parts: int 
     return int(build.library("gemm_tiles").kipp_gemm_tiles_parts(int(m), int(n), int(k), TILES_END[end], int(max_parts)))
 
 
-def gemm_tiles(x: torch.Tensor, w: torch.Tensor, end: str = "slabs", max_parts: int = 1, force: int = 0) -> torch.Tensor:
+def gemm_tiles(x: torch.Tensor, w: torch.Tensor, end: str = "slabs", max_parts: int = 1, force: int = 0, activation: str = "silu",
+               bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """x [M, K] . w [N, K]^T on the matrix cores for many rows, bfloat16 operands, float32 accumulation.
     end "slabs": float32 [parts, M, N] whose sum over parts is the product (parts <= max_parts, chosen from the shape);
     "swiglu": w = [gate; up] of [2 I, K], the result is bfloat16 [M, I] = silu(x . gate^T) * (x . up^T);
+    "glu": the same with `activation` silu or relu and a float32 `bias` [2 I] (or none) ahead of it;
     "bf16": bfloat16 [M, N]; "relu2": bfloat16 [M, N] = relu(x . w^T)^2.  `force` = 100 wm + 10 wn + parts (+ 1000: workgroups of 8 waves, four across, wave tiles
     4 x 2 or 2 x 2; + 2000, bfloat16 ends: those for the whole rounds of 256 tiles and smaller tiles for the columns
     that are left, 8 waves on half the rows or, + 10000 r, 4 waves on 256 x 64, 128 x 128 or 128 x 64 outputs) takes
@@ -1957,11 +1959,18 @@ def gemm_tiles(x: torch.Tensor, w: torch.Tensor, end: str = "slabs", max_parts: 
         parts = force % 10 if force else lib.kipp_gemm_tiles_parts(m, n, k, code, int(max_parts))
         _need(parts >= 1, "gemm_tiles: no cut for these sizes")
         out = torch.empty((parts, m, n), dtype=torch.float32, device=x.device)
-    elif end == "swiglu":
+    elif end in ("swiglu", "glu"):
         _need(n % 2 == 0, "gemm_tiles: [gate; up] has an even number of rows")
         out = torch.empty((m, n // 2), dtype=torch.bfloat16, device=x.device)
     else:
         out = torch.empty((m, n), dtype=torch.bfloat16, device=x.device)
+    if end == "glu":
+        _dev(x, bias)
+        _need(activation in ("silu", "relu") and (bias is None or (bias.dtype == torch.float32 and bias.numel() == n and bias.is_contiguous())),
+              "gemm_tiles: silu or relu, and a float32 bias as long as [gate; up]")
+        fn = _fn("gemm_tiles", "kipp_gemm_tiles_glu", [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_int, _c_ptr])
+        _check(fn(_ptr(x), _ptr(w), _ptr(out), m, n, k, int(activation == "relu"), _ptr(bias), int(force), _stream()), "gemm_tiles")
+        return out
     fn = _fn("gemm_tiles", "kipp_gemm_tiles", [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr])
     _check(fn(_ptr(x), _ptr(w), _ptr(out), m, n, k, code, int(max_parts), int(force), _stream()), "gemm_tiles")
     return out

@@ -19,7 +19,7 @@ from .base import ParamSpec, register
 @register("feed_forward", "gated_mlp")
 class GatedMLP:
     """delta = W_down (silu(W_gate x) * (W_up x))  (/root/reference/src/kipp.c:2633-2653); with `bias_names` every
-    projection has a bias: the gate's and the up's are added in the activation's kernel, the down's rides on the delta."""
+    projection has a bias: the gate's and the up's are added ahead of the activation, the down's rides on the delta."""
 
     graph_safe = True   # forward launches kernels only: no host reads, no data-dependent launches
     takes_scaled_rows = True
@@ -64,15 +64,16 @@ class GatedMLP:
         rows, inner = x.shape[0], self.spec.intermediate_size
         act = rt.empty((rows, inner), rt.act_dtype)
         w = self.w_gate_up
-        if self.bias_gate_up is not None:
-            # biases: the gate-up product by itself, then the activation's kernel adds them ahead of the activation
-            rt.ops.activate(rt.linear(rt.rows_of(x), w, slabs=True), act, self.spec.activation, glu=True, bias=self.bias_gate_up)
-            return WeightedDelta.of(rt, rt.linear(act, self.w_down, slabs=True, defer=True), 1.0, self.bias_down)
-        if self.spec.activation != "silu":
-            # another activation: the gate-up product by itself, then the activation's own kernel (the products that
-            # end in the activation are built for silu)
-            rt.ops.activate(rt.linear(rt.rows_of(x), Weight(w.rows, None if w.pairs else w.tiles), slabs=True), act, self.spec.activation, glu=True)
-            return rt.linear(act, self.w_down, slabs=True, defer=True)
+        if self.bias_gate_up is not None or self.spec.activation != "silu":
+            x = rt.rows_of(x)
+            if w.dtype == x.dtype == torch.bfloat16 and not rt.streams(rows, x.shape[1], 2 * inner):
+                act = rt.gated(x, w, act, self.spec.activation, self.bias_gate_up)      # many rows: in the product's end
+            else:
+                # the gate-up product by itself, then the activation's kernel, which adds the biases ahead of the activation
+                rt.ops.activate(rt.linear(x, Weight(w.rows, None if w.pairs else w.tiles), slabs=True), act, self.spec.activation,
+                                glu=True, bias=self.bias_gate_up)
+            delta = rt.linear(act, self.w_down, slabs=True, defer=True)
+            return delta if self.bias_gate_up is None else WeightedDelta.of(rt, delta, 1.0, self.bias_down)
         act, major = swiglu_product(rt, x, w, act, self.w_down)
         return rt.linear(act, self.w_down, slabs=True, defer=True, x_steps_major=major)
 

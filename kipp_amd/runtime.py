@@ -347,22 +347,27 @@ class Runtime:
         # a torch without float32 results from bfloat16 products would round deltas of the residual stream
         raise RuntimeError("this torch cannot return float32 from a bfloat16 product; the library product is not used then")
 
-    def gated(self, x, w: "Weight", act: torch.Tensor) -> torch.Tensor:
-        """act [M, I] (bfloat16) = silu(x . gate^T) * (x . up^T) for many rows, w = [gate; up]: our kernel
+    def gated(self, x, w: "Weight", act: torch.Tensor, activation: str = "silu", bias=None) -> torch.Tensor:
+        """act [M, I] (bfloat16) = silu(x . gate^T) * (x . up^T) for many rows, w = [gate; up] (or with relu; `bias`: one float32
+        number a row of w, added ahead of the activation): our kernel
         computes both products and the activation in one pass; after the library's product (float32, so
         that either way rounds once, after the activation) the activation is a kernel of its own."""
         m, k = x.shape
         rows = w.rows
+        plain = activation == "silu" and bias is None
 
         def ours(force=0):
-            return self.ops.gemm_tiles(x, rows, end="swiglu", force=force)
+            if plain:
+                return self.ops.gemm_tiles(x, rows, end="swiglu", force=force)
+            return self.ops.gemm_tiles(x, rows, end="glu", force=force, activation=activation, bias=bias)
 
         def library():
-            return self.ops.swiglu(self._library_product(x, rows), act)
+            product = self._library_product(x, rows)
+            return self.ops.swiglu(product, act) if plain else self.ops.activate(product, act, activation, glu=True, bias=bias)
         if self.ops.gemm_tiles_ok(m, k, rows.shape[0]):
             ways = {"library": library, "plan": ours}
             ways.update({cut: (lambda cut=cut: ours(cut)) for cut in self.TILE_CUTS_BF16})
-            choice = self._fastest(("gated", self._rows_class(m), rows.shape[0], k), ways, ("plan",) + self.TILE_CUTS_BF16)
+            choice = self._fastest(("gated" if plain else "glu", self._rows_class(m), rows.shape[0], k), ways, ("plan",) + self.TILE_CUTS_BF16)
             if choice != "library":
                 self.tile_products += 1
                 return ours(0 if choice == "plan" else choice)
