@@ -38,11 +38,11 @@
 #define MFMA_THREADS 256
 #define MANY_ROWS 256       // rows of a tile of the walking one where an expert has many
 #define WALK_FROM 48        // rows an expert (all of them) beyond which the walking one is the faster
-#define TILE_WAVES 4        // waves of its workgroup
+#define TILE_ACROSS 4       // waves of its workgroup across the columns (one or two down)
 #ifndef TILE_STAGES
 #define TILE_STAGES 3       // steps of K that are in LDS or on their way there: two workgroups share a compute unit
 #endif
-#define MANY_STAGES 4       // one workgroup a compute unit
+#define MANY_STAGES 4       // one workgroup (two waves a SIMD) a compute unit
 #define ROWS_TILE 64        // rows of a tile of the product for few rows
 #define ROWS_WAVES 8        // waves of its workgroup
 #define XCDS 8              // dies of the chip; consecutive workgroups of a launch go to them in turn
@@ -266,8 +266,9 @@ moe_sort_kernel(const int32_t* __restrict__ chosen, int pairs, int experts, int 
     __syncthreads();
     for (int e = threadIdx.x; e < experts; e += blockDim.x) {
         const int n = count[e], parts = (n + tile_rows - 1) / tile_rows;
-        // whole tiles: an expert's rows shared out evenly, in 32s
-        const int each = tile_rows >= MFMA_ROWS && parts > 0 ? ((n + parts - 1) / parts + 31) / 32 * 32 : tile_rows;
+        // whole tiles: an expert's rows shared out evenly, in what the waves' products take
+        const int grain = tile_rows == MANY_ROWS ? 64 : 32;     // of the products that read these tiles
+        const int each = tile_rows >= MFMA_ROWS && parts > 0 ? ((n + parts - 1) / parts + grain - 1) / grain * grain : tile_rows;
         for (int j = 0; j < parts; ++j) {
             int32_t* tile = tiles + (size_t)(tile_first[e] + j) * 3;
             tile[0] = e;
@@ -484,24 +485,26 @@ moe_expert_mfma_kernel(const bf16_t* __restrict__ x, const int32_t* __restrict__
         }
 }
 
-// The same for experts of many rows, tiles of up to 32 FRAGS rows.  A workgroup takes a tile's rows
-// and 256 rows of the expert's matrix (GLU: 128 of the gate's and the 128 of the up's that belong to them), a wave all of the
-// rows against 64 of them, as many products of 32 rows as the tile has.  The walk over K is the one of the products for prompt portions
-// (`tile_walk.h`), its rows of X taken through `gather`.  Bound by what a compute unit draws (a matrix of an expert meets its
-// 100 to 300 rows only) and by whole rounds of workgroups.  32 experts, matrices of 2,432 x 2,560 and back, staged kernel / this one,
-// us: 8,192 rows 251 / 214 and 230 / 201, gated 417 / 360 (256 rows a tile; 375 with 128); 5,120 rows 198 / 174, 172 / 158, 329 / 262 (306);
-// 2,048 rows 137 / 128, 125 / 119, 197 / 194 (204 with 256 rows); 1,024 rows 116 / 119, 105 / 108, 175 / 185: its lines of 64
+// The same for experts of many rows, tiles of up to 128 DOWN rows.  A workgroup takes a tile's rows
+// and 256 rows of the expert's matrix (GLU: 128 of the gate's and the 128 of the up's that belong to them), DOWN x 4 waves, each
+// 1 / DOWN of the rows against 64 of them, as many products of 32 rows as its part has.  The walk over K is the one of the products for
+// prompt portions (`tile_walk.h`), its rows of X taken through `gather`.  Bound by what a compute unit draws (a matrix of an
+// expert meets its 100 to 300 rows only) and by whole rounds of workgroups.  32 experts, matrices of 2,432 x 2,560 and back,
+// us: staged kernel / this one with 128 rows: 8,192 rows 251 / 212 and 230 / 201, gated 417 / 363; 5,120 rows 198 / 165, 172 / 152,
+// 329 / 300; 2,048 rows 137 / 128, 125 / 119, 197 / 195; 1,024 rows 116 / 119, 105 / 108, 175 / 185: its lines of 64
 // bytes of a row are the slower way to read a matrix once, so the staged kernel keeps experts of up to 48 rows.
-template <typename TO, bool GLU, int FRAGS, int STAGES, int WM>
+// 256 rows: 8,192 rows 193, 170, gated 320; 5,120 rows 171, 153, 243; with four waves of all 256 rows, one a SIMD, instead of
+// eight: 237, 195, 365; 196, 157, 264 (whatever holds up a SIMD's one wave idles its matrix core).
+template <typename TO, bool GLU, int DOWN, int STAGES, int WM>
 __device__ __forceinline__ void expert_tile(const bf16_t* __restrict__ x, const int32_t* __restrict__ gather, const float* __restrict__ row_weight,
                                             const bf16_t* __restrict__ w_e, TO* __restrict__ out, int row0, int rows, int col0, int n_out, int k,
                                             int act, unsigned char* lds) {
-    constexpr int WAVES = TILE_WAVES, WN = 2;
-    constexpr int TM = 64 * ((WM + 1) / 2), TN = 32 * WN * WAVES;     // rows of the pieces of a step (of X: whole instructions a wave)
+    constexpr int WAVES = TILE_ACROSS * DOWN, WN = 2;
+    constexpr int TM = 64 * DOWN * ((WM + 1) / 2), TN = 32 * WN * TILE_ACROSS;     // rows of the pieces of a step (of X: whole instructions a wave)
     constexpr int X_PIECE = TM * BK * 2, W_PIECE = TN * BK * 2, STAGE_BYTES = X_PIECE + W_PIECE;
     constexpr int XI = TM / INSTR_ROWS / WAVES, WI = TN / INSTR_ROWS / WAVES;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int l32 = lane & 31, hh = lane >> 5;
+    const int l32 = lane & 31, hh = lane >> 5, across = wave % TILE_ACROSS, first = 32 * WM * (wave / TILE_ACROSS);     // this wave's columns and rows
     int lane_row, col8;
     dma_place(lane, lane_row, col8);
     // a lane's rows begin at 32-bit offsets from x and from the expert's matrix (the launcher has checked that they fit)
@@ -513,14 +516,14 @@ __device__ __forceinline__ void expert_tile(const bf16_t* __restrict__ x, const 
     }
 #pragma unroll
     for (int i = 0; i < WI; ++i) {
-        const int r = 64 * wave + INSTR_ROWS * i + lane_row;        // of the piece; a wave's 64: under GLU 32 of the gate's, then the up's
-        const int wr = GLU ? min(col0 + 32 * wave + (r & 31), n_out - 1) + (r & 32 ? n_out : 0) : min(col0 + r, n_out - 1);
+        const int r = (TN / WAVES) * wave + INSTR_ROWS * i + lane_row;      // of the piece; 64 a wave multiplies: under GLU 32 of the gate's, then the up's
+        const int wr = GLU ? min(col0 + 32 * (r / 64) + (r & 31), n_out - 1) + (r & 32 ? n_out : 0) : min(col0 + r, n_out - 1);
         w_src[i] = (uint32_t)(((size_t)wr * k + col8) * 2);
     }
     f32x16 acc[WM][WN];
     tile_walk<WM, WN, XI, WI, STAGES, STAGE_BYTES>(lds, lane, (const unsigned char*)x, (const unsigned char*)w_e, x_src, w_src,
-                                                   wave * (X_PIECE / WAVES), X_PIECE + wave * (W_PIECE / WAVES), 0,
-                                                   X_PIECE + wave * (W_PIECE / WAVES), k / BK, acc);
+                                                   wave * (X_PIECE / WAVES), X_PIECE + wave * (W_PIECE / WAVES), first * BK * 2,
+                                                   X_PIECE + across * (W_PIECE / TILE_ACROSS), k / BK, acc);
     // In accumulator tile (i, j) a lane holds column l32 and rows 8 (v / 4) + 4 hh + v % 4.  32 rows at a time go through the wave's own
     // corner of LDS (now free) as they are; a lane then takes 8 neighbouring columns of a row, activates and stores them (the
     // activations written out for every accumulator register were hundreds of KB of code that ran once).
@@ -528,7 +531,7 @@ __device__ __forceinline__ void expert_tile(const bf16_t* __restrict__ x, const 
     static_assert(32 * PITCH * 4 * WAVES <= STAGES * STAGE_BYTES, "a wave's staging fits its share of LDS");
     __syncthreads();                                               // every wave is done reading operands
     float* stage = (float*)lds + wave * 32 * PITCH;
-    const int c_in = (lane % LANES_PER_ROW) * 8, c = col0 + WCOLS * wave + c_in;
+    const int c_in = (lane % LANES_PER_ROW) * 8, c = col0 + WCOLS * across + c_in;
 #pragma unroll
     for (int i = 0; i < WM; ++i) {
 #pragma unroll
@@ -539,7 +542,7 @@ __device__ __forceinline__ void expert_tile(const bf16_t* __restrict__ x, const 
         __builtin_amdgcn_wave_barrier();
 #pragma unroll 1
         for (int r = lane / LANES_PER_ROW; r < 32; r += ROWS_PER_PASS) {
-            if (32 * i + r >= rows || c >= n_out) continue;
+            if (first + 32 * i + r >= rows || c >= n_out) continue;
             const float* at = stage + r * PITCH + c_in;
             float y[8], u[8];
 #pragma unroll
@@ -547,10 +550,10 @@ __device__ __forceinline__ void expert_tile(const bf16_t* __restrict__ x, const 
                 *(f32x4*)(y + q) = *(const f32x4*)(at + q);
                 if (GLU) *(f32x4*)(u + q) = *(const f32x4*)(at + 32 + q);
             }
-            const float s = GLU && row_weight != nullptr ? row_weight[row0 + 32 * i + r] : 1.0f;
+            const float s = GLU && row_weight != nullptr ? row_weight[row0 + first + 32 * i + r] : 1.0f;
 #pragma unroll
             for (int q = 0; q < 8; ++q) y[q] = GLU ? activate(s * y[q], act) * (s * u[q]) : activate(y[q], act);
-            TO* dst = out + (size_t)(row0 + 32 * i + r) * n_out + c;
+            TO* dst = out + (size_t)(row0 + first + 32 * i + r) * n_out + c;
             if (c + 8 <= n_out && (n_out & 7) == 0) {
                 if constexpr (sizeof(TO) == 4) {
                     *(f32x4*)dst = *(const f32x4*)y;
@@ -571,8 +574,8 @@ __device__ __forceinline__ void expert_tile(const bf16_t* __restrict__ x, const 
     }
 }
 
-template <typename TO, bool GLU, int FRAGS, int STAGES>
-__global__ void __launch_bounds__(64 * TILE_WAVES, FRAGS <= 4 ? 2 : 1)
+template <typename TO, bool GLU, int DOWN, int STAGES>
+__global__ void __launch_bounds__(64 * TILE_ACROSS * DOWN, 2)
 moe_expert_tiles_kernel(const bf16_t* __restrict__ x, const int32_t* __restrict__ gather, const float* __restrict__ row_weight,
                         const bf16_t* __restrict__ w, const int32_t* __restrict__ tiles, int max_tiles, int col_tiles, TO* __restrict__ out,
                         int n_out, int k, int act) {
@@ -590,15 +593,14 @@ moe_expert_tiles_kernel(const bf16_t* __restrict__ x, const int32_t* __restrict_
     if (turn >= per_die || item >= items) return;       // uniform over the workgroup
     const int32_t* tile = tiles + (size_t)(item / col_tiles) * 3;
     const int expert = __builtin_amdgcn_readfirstlane(tile[0]), row0 = __builtin_amdgcn_readfirstlane(tile[1]), rows = __builtin_amdgcn_readfirstlane(tile[2]);
-    const int col0 = (item % col_tiles) * (GLU ? 32 : 64) * TILE_WAVES;
+    const int col0 = (item % col_tiles) * (GLU ? 32 : 64) * TILE_ACROSS;
     const bf16_t* w_e = w + (size_t)expert * (GLU ? 2 : 1) * n_out * k;
-    // a tile's products: as many of 32 rows as it has (of 64 in the larger form)
-    constexpr int GRAIN = FRAGS / 4;
+    // a wave's products: as many of 32 rows as its part of the tile has
 #define KIPP_ET(N)                                                                                                                     \
     case N:                                                                                                                            \
-        expert_tile<TO, GLU, FRAGS, STAGES, N * GRAIN>(x, gather, row_weight, w_e, out, row0, rows, col0, n_out, k, act, lds);           \
+        expert_tile<TO, GLU, DOWN, STAGES, N>(x, gather, row_weight, w_e, out, row0, rows, col0, n_out, k, act, lds);           \
         break
-    switch ((rows + 32 * GRAIN - 1) / (32 * GRAIN)) {
+    switch ((rows + 32 * DOWN - 1) / (32 * DOWN)) {
         KIPP_ET(1);
         KIPP_ET(2);
         KIPP_ET(3);
@@ -840,20 +842,20 @@ extern "C" int kipp_moe_route_grouped(const float* z, int parts, int stride, con
     return KIPP_LAUNCH_CHECK();
 }
 
-template <typename TO, bool GLU, int FRAGS, int STAGES>
+template <typename TO, bool GLU, int DOWN, int STAGES>
 static int launch_tiles(const void* x, const int32_t* gather, const float* row_weight, const void* w, const int32_t* tiles, int max_tiles,
                         void* out, int n_out, int k, int act, hipStream_t stream) {
-    constexpr int lds_bytes = STAGES * (32 * FRAGS + 64 * TILE_WAVES) * BK * 2;
+    constexpr int lds_bytes = STAGES * (128 * DOWN + 64 * TILE_ACROSS) * BK * 2;
     static bool prepared = false;
     if (!prepared) {
-        if (hipFuncSetAttribute((const void*)moe_expert_tiles_kernel<TO, GLU, FRAGS, STAGES>, hipFuncAttributeMaxDynamicSharedMemorySize,
+        if (hipFuncSetAttribute((const void*)moe_expert_tiles_kernel<TO, GLU, DOWN, STAGES>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 lds_bytes) != hipSuccess)
             return -6;
         prepared = true;
     }
-    const int cols = (GLU ? 32 : 64) * TILE_WAVES, col_tiles = (n_out + cols - 1) / cols;
+    const int cols = (GLU ? 32 : 64) * TILE_ACROSS, col_tiles = (n_out + cols - 1) / cols;
     const int grid = (max_tiles * col_tiles + XCDS - 1) / XCDS * XCDS;
-    hipLaunchKernelGGL((moe_expert_tiles_kernel<TO, GLU, FRAGS, STAGES>), dim3(grid), dim3(64 * TILE_WAVES), lds_bytes, stream, (const bf16_t*)x,
+    hipLaunchKernelGGL((moe_expert_tiles_kernel<TO, GLU, DOWN, STAGES>), dim3(grid), dim3(64 * TILE_ACROSS * DOWN), lds_bytes, stream, (const bf16_t*)x,
                        gather, row_weight, (const bf16_t*)w, tiles, max_tiles, col_tiles, (TO*)out, n_out, k, act);
     return KIPP_LAUNCH_CHECK();
 }
@@ -895,11 +897,11 @@ static int launch_expert(const void* x, int x_dtype, const int32_t* gather, cons
             return KIPP_LAUNCH_CHECK();
         }
         if (out_dtype == KIPP_BF16)
-            return tile_rows == MFMA_ROWS ? launch_tiles<bf16_t, GLU, 4, TILE_STAGES>(x, gather, row_weight, w, tiles, max_tiles, out, n_out, k, act, stream)
-                                          : launch_tiles<bf16_t, GLU, 8, MANY_STAGES>(x, gather, row_weight, w, tiles, max_tiles, out, n_out, k, act, stream);
+            return tile_rows == MFMA_ROWS ? launch_tiles<bf16_t, GLU, 1, TILE_STAGES>(x, gather, row_weight, w, tiles, max_tiles, out, n_out, k, act, stream)
+                                          : launch_tiles<bf16_t, GLU, 2, MANY_STAGES>(x, gather, row_weight, w, tiles, max_tiles, out, n_out, k, act, stream);
         if (out_dtype == KIPP_F32)
-            return tile_rows == MFMA_ROWS ? launch_tiles<float, GLU, 4, TILE_STAGES>(x, gather, row_weight, w, tiles, max_tiles, out, n_out, k, act, stream)
-                                          : launch_tiles<float, GLU, 8, MANY_STAGES>(x, gather, row_weight, w, tiles, max_tiles, out, n_out, k, act, stream);
+            return tile_rows == MFMA_ROWS ? launch_tiles<float, GLU, 1, TILE_STAGES>(x, gather, row_weight, w, tiles, max_tiles, out, n_out, k, act, stream)
+                                          : launch_tiles<float, GLU, 2, MANY_STAGES>(x, gather, row_weight, w, tiles, max_tiles, out, n_out, k, act, stream);
         return -2;
     }
     if (tile_rows != TILE_ROWS) return -1;

@@ -1024,20 +1024,21 @@ MOE_TILE_ROWS = 16
 MOE_MFMA_ROWS = 128    # rows of a tile of the experts' products on the matrix cores
 MOE_FEW_ROWS = 64      # the same in the kernel for few rows an expert, which reads the experts' matrices straight into the products
 MOE_MANY_ROWS = 256    # the same where an expert has many rows: its matrix is read less often, a compute unit has one workgroup
-# Pairs an expert (all of them) up to which a step takes the kernel for few rows, and from which on a gated one takes tiles of 256.
-# 32 experts, inner 2,432, width 2,560, both products, us: 256 pairs gated 251 with tiles of 64, 276 with 128; 512 pairs 314 and 281; 2,048
-# pairs 313 with tiles of 128, 326 with 256; 5,120 pairs 464 and 421; without a gate 332 and 357 there, 415 and 422 at 8,192.
-MOE_FEW_PAIRS, MOE_MANY_PAIRS = 12, 96
+# Pairs an expert (all of them) up to which a step takes the kernel for few rows, and from which on a gated one, or one without a
+# gate, takes tiles of 256.  32 experts, inner 2,432, width 2,560, both products, us: 256 pairs gated 251 with tiles of 64, 276 with 128;
+# 512 pairs 314 and 281; gated with tiles of 128 / 256: 2,048 pairs 314 / 316, 3,200 341 / 343, 4,300 428 / 377, 8,192 564 / 490; without
+# a gate 6,400 340 / 362, 7,600 362 / 362, 8,192 414 / 363, 10,000 409 / 412, 12,288 511 / 458.
+MOE_FEW_PAIRS, MOE_MANY_PAIRS, MOE_MANY_PAIRS_UNGATED = 12, 96, 240
 
 
 def moe_tile_rows(dtype: torch.dtype, *contractions: int, pairs: Optional[int] = None, experts: int = 1, gated: bool = False) -> int:
     """Rows of the tiles that the experts' products take: 128 on the matrix cores (bfloat16, every contraction a multiple of
-    32), else 16.  With `pairs`, the (token, choice) pairs of the step: 64 for few of them an expert, 256 for many of a gated one."""
+    32), else 16.  With `pairs`, the (token, choice) pairs of the step: 64 for few of them an expert, 256 for many."""
     if dtype != torch.bfloat16 or any(k % 32 for k in contractions):
         return MOE_TILE_ROWS
     if pairs is not None and pairs <= MOE_FEW_PAIRS * experts:
         return MOE_FEW_ROWS
-    many = pairs is not None and gated and pairs > MOE_MANY_PAIRS * experts
+    many = pairs is not None and pairs > (MOE_MANY_PAIRS if gated else MOE_MANY_PAIRS_UNGATED) * experts
     # (a lane's offset into the rows is 32 bits wide, for as many rows as the tiles could hold)
     if many and (-(-pairs // MOE_MANY_ROWS) + experts) * MOE_MANY_ROWS * max(contractions) < 1 << 31:
         return MOE_MANY_ROWS
