@@ -34,7 +34,36 @@ __device__ __forceinline__ void rotate_pair(float& a, float& b, int pos, float f
 __device__ __forceinline__ int pair_lo(int i, int half) { return half ? i : 2 * i; }
 __device__ __forceinline__ int pair_hi(int i, int rot_dims, int half) { return half ? i + rot_dims / 2 : 2 * i + 1; }
 
-// One workgroup a token.  LDS: 16 floats for the sums.  `kv_at`: where the key/value latent's columns begin.
+// N numbers, the slabs of each added in order: all N are asked for, four slabs at a time, before the first is used.
+template <int N, typename AT>
+__device__ __forceinline__ void slab_sums(float (&total)[N], AT at, int parts, size_t part_stride) {
+    float v[N][4];
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const float* from = at(i);
+#pragma unroll
+        for (int p = 0; p < 4; ++p) v[i][p] = from[(size_t)min(p, parts - 1) * part_stride];
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        total[i] = v[i][0];
+#pragma unroll
+        for (int p = 1; p < 4; ++p) total[i] += p < parts ? v[i][p] : 0.0f;
+    }
+    for (int p = 4; p < parts; ++p)
+#pragma unroll
+        for (int i = 0; i < N; ++i) total[i] += at(i)[(size_t)p * part_stride];
+}
+__device__ __forceinline__ float slab_sum(const float* __restrict__ at, int parts, size_t part_stride) {
+    float total[1];
+    slab_sums(total, [&](int) { return at; }, parts, part_stride);
+    return total[0];
+}
+
+// One workgroup a token.  LDS: 16 floats for the sums.  `kv_at`: where the key/value latent's columns begin.  For a single token the
+// loads' latencies are the time (8 tokens of 768 + 192 + 64 columns 7.4 us; 11.6 while every sum waited for the one before it):
+// whatever the registers hold is asked for before the first sum, and read once.
+#define LP_ITEMS 2          // numbers of a latent that a thread holds (beyond: read for the sum, and again)
 template <typename TO, typename TC>
 __global__ void latent_prepare_kernel(
     const float* __restrict__ proj, int parts, size_t part_stride, int stride,
@@ -46,63 +75,65 @@ __global__ void latent_prepare_kernel(
     const int t = blockIdx.x;
     const int pos = positions[t];
     const float* src = proj + (size_t)t * stride;
-    // the query latent
-    float ss = 0.0f, scale;
-    if (q_rank > 0) {
-        for (int e = threadIdx.x; e < q_rank; e += blockDim.x) {
-            float v = 0.0f;
-            for (int p = 0; p < parts; ++p) v += src[p * part_stride + e];
-            ss = fmaf(v, v, ss);
+    const float* kv = src + kv_at;
+    const int step = blockDim.x, past = LP_ITEMS * step;
+    const int page_id = write_kv ? block_table[(size_t)seq_of_token[t] * max_blocks + pos / page] : 0;
+    float q_v[LP_ITEMS], q_w[LP_ITEMS], c_v[LP_ITEMS], c_w[LP_ITEMS];
+    slab_sums(q_v, [&](int i) { return src + min((int)threadIdx.x + i * step, max(q_rank, 1) - 1); }, parts, part_stride);
+    slab_sums(c_v, [&](int i) { return kv + min((int)threadIdx.x + i * step, rank - 1); }, parts, part_stride);
+#pragma unroll
+    for (int i = 0; i < LP_ITEMS; ++i) {
+        const int e = threadIdx.x + i * step;
+        if (e >= q_rank) q_v[i] = 0.0f;
+        if (e >= rank) c_v[i] = 0.0f;
+        q_w[i] = e < q_rank ? q_norm_w[e] : 0.0f;
+        c_w[i] = e < rank ? c_norm_w[e] : 0.0f;
+    }
+    // the shared rotated part, and the numbers of it that are not turned, one by one
+    const int pairs = rot_dims / 2;
+    if (write_kv) {
+        TC* dst = cache + ((size_t)page_id * page + pos % page) * (rank + dr) + rank;
+        for (int i = threadIdx.x; i < pairs + dr - rot_dims; i += step) {
+            const int lo = i < pairs ? pair_lo(i, half) : rot_dims + i - pairs, hi = i < pairs ? pair_hi(i, rot_dims, half) : lo;
+            float a = slab_sum(kv + rank + lo, parts, part_stride);
+            if (i < pairs) {
+                float b = slab_sum(kv + rank + hi, parts, part_stride);
+                rotate_pair(a, b, pos, freq[i], magnitude);
+                store_f(dst, hi, b);
+            }
+            store_f(dst, lo, a);
+        }
+    }
+    // a latent's numbers in registers, then those beyond
+    auto norm = [&](const float* from, int n, const float (&v)[LP_ITEMS], const float (&w)[LP_ITEMS], const float* weights, auto* to) {
+        float ss = 0.0f;
+#pragma unroll
+        for (int i = 0; i < LP_ITEMS; ++i) ss = fmaf(v[i], v[i], ss);
+        for (int e = threadIdx.x + past; e < n; e += step) {
+            const float x = slab_sum(from + e, parts, part_stride);
+            ss = fmaf(x, x, ss);
         }
         ss = block_sum(ss, scratch);
-        scale = 1.0f / sqrtf(ss / (float)q_rank + eps);
-        for (int e = threadIdx.x; e < q_rank; e += blockDim.x) {
-            float v = 0.0f;
-            for (int p = 0; p < parts; ++p) v += src[p * part_stride + e];
-            store_f(cq_out + (size_t)t * q_rank, e, v * scale * q_norm_w[e]);
+        const float scale = 1.0f / sqrtf(ss / (float)n + eps);
+#pragma unroll
+        for (int i = 0; i < LP_ITEMS; ++i) {
+            const int e = threadIdx.x + i * step;
+            if (e < n) store_f(to, e, v[i] * scale * w[i]);
         }
-    }
-    if (!write_kv) return;
-    // the key/value latent and the shared rotated part
-    src += kv_at;
-    ss = 0.0f;
-    for (int e = threadIdx.x; e < rank; e += blockDim.x) {
-        float v = 0.0f;
-        for (int p = 0; p < parts; ++p) v += src[p * part_stride + e];
-        ss = fmaf(v, v, ss);
-    }
-    ss = block_sum(ss, scratch);
-    scale = 1.0f / sqrtf(ss / (float)rank + eps);
-    const int seq = seq_of_token[t];
-    const int page_id = block_table[(size_t)seq * max_blocks + pos / page];
-    TC* dst = cache + ((size_t)page_id * page + pos % page) * (rank + dr);
-    for (int e = threadIdx.x; e < rank; e += blockDim.x) {
-        float v = 0.0f;
-        for (int p = 0; p < parts; ++p) v += src[p * part_stride + e];
-        store_f(dst, e, v * scale * c_norm_w[e]);
-    }
-    src += rank;
-    const int pairs = rot_dims / 2;         // then the numbers that are not turned, one by one
-    for (int i = threadIdx.x; i < pairs + dr - rot_dims; i += blockDim.x) {
-        const int lo = i < pairs ? pair_lo(i, half) : rot_dims + i - pairs, hi = i < pairs ? pair_hi(i, rot_dims, half) : lo;
-        float a = 0.0f, b = 0.0f;
-        for (int p = 0; p < parts; ++p) {
-            a += src[p * part_stride + lo];
-            if (i < pairs) b += src[p * part_stride + hi];
-        }
-        if (i < pairs) {
-            rotate_pair(a, b, pos, freq[i], magnitude);
-            store_f(dst, rank + hi, b);
-        }
-        store_f(dst, rank + lo, a);
-    }
+        for (int e = threadIdx.x + past; e < n; e += step) store_f(to, e, slab_sum(from + e, parts, part_stride) * scale * weights[e]);
+    };
+    if (q_rank > 0) norm(src, q_rank, q_v, q_w, q_norm_w, cq_out + (size_t)t * q_rank);
+    if (write_kv) norm(kv, rank, c_v, c_w, c_norm_w, cache + ((size_t)page_id * page + pos % page) * (rank + dr));
 }
 
 #define TILE_TOKENS 8       // tokens of a workgroup of absorb and of expand: a weight is read once for all of them
 #define TILE_COLS 64        // output columns of a workgroup (a lane a column, so that a wave reads a run of a weight row)
 #define TILE_WAVES 4        // the contraction is shared out over the waves and summed through LDS
 
-// acc[r] += sum over this wave's share of e of in_s[r][e] * w[e][c]: four weight rows asked for at a time.
+#define TILE_AHEAD 16       // weight rows asked for at a time
+// acc[r] += sum over this wave's share of e of in_s[e][r] * w[e][c].  A share is 32 to 48 rows, one after the other: for single
+// tokens their latencies are the time, and the reads of `in_s`, which is why its tokens lie side by side.  16 heads of 128 x 192, 8
+// tokens, us: absorb 8.3, expand 10.0; 12.4 and 20.7 with 4 rows at a time and a token's numbers side by side.
 template <typename TW>
 __device__ __forceinline__ void tile_product(const float* in_s, int k, const TW* w, int n, int c, bool live, float (&acc)[TILE_TOKENS]) {
     const int wave = threadIdx.x / KIPP_WAVE;
@@ -111,21 +142,23 @@ __device__ __forceinline__ void tile_product(const float* in_s, int k, const TW*
 #pragma unroll
     for (int r = 0; r < TILE_TOKENS; ++r) acc[r] = 0.0f;
     if (!live) return;
+    auto add = [&](int e, float wv) {
+        float in[TILE_TOKENS];
+#pragma unroll
+        for (int r = 0; r < TILE_TOKENS; r += 4) *(float4*)(in + r) = *(const float4*)(in_s + e * TILE_TOKENS + r);
+#pragma unroll
+        for (int r = 0; r < TILE_TOKENS; ++r) acc[r] = fmaf(in[r], wv, acc[r]);
+    };
     int e = e0;
-    for (; e + 4 <= e1; e += 4) {
-        float wv[4];
+    for (; e + TILE_AHEAD <= e1; e += TILE_AHEAD) {
+        TW wv[TILE_AHEAD];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) wv[u] = load_f(w, (size_t)(e + u) * n + c);
+        for (int u = 0; u < TILE_AHEAD; ++u) wv[u] = w[(size_t)(e + u) * n + c];
+        __builtin_amdgcn_sched_barrier(0);          // (left to itself the compiler waits for every one before it asks for the next)
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
-#pragma unroll
-            for (int r = 0; r < TILE_TOKENS; ++r) acc[r] = fmaf(in_s[r * k + e + u], wv[u], acc[r]);
+        for (int u = 0; u < TILE_AHEAD; ++u) add(e + u, load_f(wv, u));
     }
-    for (; e < e1; ++e) {
-        const float wv = load_f(w, (size_t)e * n + c);
-#pragma unroll
-        for (int r = 0; r < TILE_TOKENS; ++r) acc[r] = fmaf(in_s[r * k + e], wv, acc[r]);
-    }
+    for (; e < e1; ++e) add(e, load_f(w, (size_t)e * n + c));
 }
 
 // The waves' partial sums added in wave order; every thread of wave 0 gets its column's totals.  red: TILE_WAVES * TILE_TOKENS * TILE_COLS floats.
@@ -151,18 +184,23 @@ __global__ void __launch_bounds__(TILE_WAVES * KIPP_WAVE) latent_absorb_kernel(
     const float* __restrict__ q, int parts, size_t part_stride, const TW* __restrict__ w_uk, TO* __restrict__ out,
     const int32_t* __restrict__ positions, const float* __restrict__ freq, int rot_dims, float magnitude, int half,
     int n_tokens, int heads, int d, int dr, int rank, int q_row) {
-    extern __shared__ float lds[];
+    extern __shared__ __attribute__((aligned(16))) float lds[];
     float* q_s = lds;
     float* red = lds + TILE_TOKENS * d;
     const int t0 = blockIdx.x * TILE_TOKENS;
     const int head = blockIdx.y;
     const int rows = min(TILE_TOKENS, n_tokens - t0);
-    for (int i = threadIdx.x; i < TILE_TOKENS * d; i += blockDim.x) {
-        const int r = i / d, e = i - r * d;
-        float v = 0.0f;
-        if (r < rows)
-            for (int p = 0; p < parts; ++p) v += q[p * part_stride + (size_t)(t0 + r) * q_row + head * (d + dr) + e];
-        q_s[i] = v;
+    for (int i0 = threadIdx.x; i0 < TILE_TOKENS * d; i0 += 4 * blockDim.x) {
+        float v[4];
+        slab_sums(v, [&](int j) {
+            const int i = min(i0 + j * (int)blockDim.x, TILE_TOKENS * d - 1), r = i / d;
+            return q + (size_t)(t0 + min(r, rows - 1)) * q_row + head * (d + dr) + i - r * d;       // rows beyond the last repeat it and are not stored
+        }, parts, part_stride);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int i = i0 + j * blockDim.x, r = i / d;
+            if (i < TILE_TOKENS * d) q_s[(i - r * d) * TILE_TOKENS + r] = v[j];
+        }
     }
     __syncthreads();
     const int width = rank + dr;
@@ -183,13 +221,10 @@ __global__ void __launch_bounds__(TILE_WAVES * KIPP_WAVE) latent_absorb_kernel(
         if (r >= rows) continue;
         const size_t at = (size_t)(t0 + r) * q_row + head * (d + dr) + d;
         const int lo = pair < pairs ? pair_lo(pair, half) : rot_dims + pair - pairs, hi = pair < pairs ? pair_hi(pair, rot_dims, half) : lo;
-        float a = 0.0f, b = 0.0f;
-        for (int p = 0; p < parts; ++p) {
-            a += q[p * part_stride + at + lo];
-            if (pair < pairs) b += q[p * part_stride + at + hi];
-        }
+        float a = slab_sum(q + at + lo, parts, part_stride);
         TO* dst = out + ((size_t)(t0 + r) * heads + head) * width + rank;
         if (pair < pairs) {
+            float b = slab_sum(q + at + hi, parts, part_stride);
             rotate_pair(a, b, positions[t0 + r], freq[pair], magnitude);
             store_f(dst, hi, b);
         }
@@ -204,18 +239,33 @@ template <typename TI, typename TW, typename TO>
 __global__ void __launch_bounds__(TILE_WAVES * KIPP_WAVE) latent_expand_kernel(
     const TI* __restrict__ lat, int lat_row, const TW* __restrict__ w_uv_t, const float* __restrict__ gate, int gate_parts,
     size_t gate_part_stride, int gate_stride, int gate_each, TO* __restrict__ out, int n_tokens, int heads, int rank, int dv) {
-    extern __shared__ float lds[];
+    extern __shared__ __attribute__((aligned(16))) float lds[];
     float* l_s = lds;
     float* red = lds + TILE_TOKENS * rank;
     const int t0 = blockIdx.x * TILE_TOKENS;
     const int head = blockIdx.y;
     const int rows = min(TILE_TOKENS, n_tokens - t0);
-    for (int i = threadIdx.x; i < TILE_TOKENS * rank; i += blockDim.x) {
-        const int r = i / rank, e = i - r * rank;
-        l_s[i] = r < rows ? load_f(lat, ((size_t)(t0 + r) * heads + head) * lat_row + e) : 0.0f;
+    const int c = blockIdx.z * TILE_COLS + (threadIdx.x & (KIPP_WAVE - 1));
+    float z[TILE_TOKENS];           // the gates of the wave that will store, asked for before the product
+    if (gate != nullptr && threadIdx.x < KIPP_WAVE) {
+        slab_sums(z, [&](int r) {
+            return gate + (size_t)(t0 + min(r, rows - 1)) * gate_stride + (gate_each ? head * dv + min(c, dv - 1) : head);
+        }, gate_parts, gate_part_stride);
+    }
+    for (int i0 = threadIdx.x; i0 < TILE_TOKENS * rank; i0 += 8 * blockDim.x) {
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int i = min(i0 + j * (int)blockDim.x, TILE_TOKENS * rank - 1), r = i / rank;
+            v[j] = load_f(lat, ((size_t)(t0 + min(r, rows - 1)) * heads + head) * lat_row + i - r * rank);
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int i = i0 + j * blockDim.x, r = i / rank;
+            if (i < TILE_TOKENS * rank) l_s[(i - r * rank) * TILE_TOKENS + r] = v[j];
+        }
     }
     __syncthreads();
-    const int c = blockIdx.z * TILE_COLS + (threadIdx.x & (KIPP_WAVE - 1));
     float acc[TILE_TOKENS];
     tile_product(l_s, rank, w_uv_t + (size_t)head * rank * dv, dv, c, c < dv, acc);
     tile_reduce(red, acc);
@@ -223,12 +273,7 @@ __global__ void __launch_bounds__(TILE_WAVES * KIPP_WAVE) latent_expand_kernel(
 #pragma unroll
     for (int r = 0; r < TILE_TOKENS; ++r) {
         if (r >= rows) continue;
-        float g = 1.0f;
-        if (gate != nullptr) {
-            float z = 0.0f;
-            for (int p = 0; p < gate_parts; ++p) z += gate[p * gate_part_stride + (size_t)(t0 + r) * gate_stride + (gate_each ? head * dv + c : head)];
-            g = 1.0f / (1.0f + expf(-z));
-        }
+        const float g = gate != nullptr ? 1.0f / (1.0f + expf(-z[r])) : 1.0f;
         store_f(out + ((size_t)(t0 + r) * heads + head) * dv, c, acc[r] * g);
     }
 }
