@@ -1570,6 +1570,41 @@ def attention_decode_workspace(n_items: int, n_q: int, head_dim: int, max_contex
             torch.zeros(n_items * n_q, dtype=torch.int32, device=device))
 
 
+SHARED_KEYS, SHARED_RUNS = 64, 64       # keys of a tile of the kernel for rows that are key and value at once; runs of tiles at most
+
+
+def attention_shared_workspace(n_items: int, head_dim: int, max_context: int, window: int, device) -> tuple:
+    """(part_acc, part_ml) of `attention_shared`: single tokens in contexts of up to `max_context`, cut into runs of one tile of keys until
+    they fill the chip about twice."""
+    span = min(max_context, window) if window else max_context
+    tiles = -(-span // SHARED_KEYS) + (1 if window else 0)
+    runs = max(1, min(tiles, SHARED_RUNS, -(-2 * COMPUTE_UNITS // max(n_items, 1))))
+    return (torch.empty((n_items, runs, 16, head_dim), dtype=torch.float32, device=device),
+            torch.empty((n_items, runs, 16, 2), dtype=torch.float32, device=device))
+
+
+def attention_shared(q: torch.Tensor, cache: torch.Tensor, out: torch.Tensor, rows: torch.Tensor, positions: torch.Tensor,
+                     seq_of_token: torch.Tensor, block_table: torch.Tensor, heads: int, head_dim: int, scale: float, window: int,
+                     workspace: tuple) -> torch.Tensor:
+    """Attention of single query tokens (batch rows `rows`) whose heads all read one row a key, which is the value as well.
+    q, out: bfloat16 [tokens, heads head_dim]; cache: bfloat16 [pages, 1, page, head_dim]."""
+    part_acc, part_ml = workspace
+    _dev(q, cache, out, part_acc, part_ml, rows, positions, seq_of_token, block_table)
+    for t, name in ((rows, "rows"), (positions, "positions"), (seq_of_token, "seq_of_token"), (block_table, "block_table")):
+        _i32(t, name)
+    _attn_common(q, cache, cache, out, heads, 1, head_dim, "attention_shared")
+    items = rows.numel()
+    runs = part_ml.shape[1]
+    _need(heads <= 16 and head_dim % 16 == 0 and head_dim <= 256, "attention_shared: at most 16 heads, rows of a multiple of 16 up to 256 numbers")
+    _need(part_acc.shape == (items, runs, 16, head_dim) and part_ml.shape == (items, runs, 16, 2) and part_acc.dtype == part_ml.dtype == torch.float32,
+          "attention_shared: the workspace is of other sizes")
+    fn = _fn("attention_shared", "kipp_attention_shared", [_c_ptr] * 6 + [_c_int] + [_c_ptr] * 3 + [_c_int] * 4 + [_c_float, _c_int, _c_int, _c_ptr])
+    _check(fn(_ptr(q), _ptr(cache), _ptr(out), _ptr(part_acc), _ptr(part_ml), _ptr(rows), items, _ptr(positions), _ptr(seq_of_token),
+              _ptr(block_table), block_table.shape[1], heads, head_dim, cache.shape[2], float(scale), int(window), runs, _stream()),
+           "attention_shared")
+    return out
+
+
 def attention_prefill(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, out: torch.Tensor,
                       item_seq: torch.Tensor, item_tile: torch.Tensor, q_start: torch.Tensor, q_len: torch.Tensor,
                       positions: torch.Tensor, block_table: torch.Tensor, n_q: int, n_kv: int, head_dim: int,

@@ -56,7 +56,8 @@ def prebuilt() -> List[Spec]:
         _, cfg = parse_config(shape_config(name))
         for dtype in ("bfloat16", "float32"):
             _add(out, model_variants(cfg.model_spec(), dtype))
-    out.append(("probe", None))
+    # kernels that models take by their sizes, which the named shapes need not have
+    _add(out, [("linear_chunks", None), ("attention_shared", None), ("probe", None)])
     return out
 
 

@@ -70,7 +70,7 @@ class LatentAttention:
         out = [("latent", None), ("attention_generic", None)]
         if dtype == "bfloat16" and spec.row % 16 == 0 and spec.row <= 256 and spec.num_heads <= 16:
             out.append(("attention_prefill", {"HEAD_DIM": spec.row}))
-            out.append(("attention_decode", {"HEAD_DIM": spec.row, "GROUP": spec.num_heads}))
+            out.append(("attention_shared", None))
         return out
 
     def load(self, tensors):

@@ -267,7 +267,14 @@ def paged_attention(rt, batch, q, out, k_cache, v_cache, page_size, table, n_q, 
             rt.ops.attention_prefill(q, k_cache, v_cache, out, item_seq, item_tile, batch.q_start, batch.q_len, batch.positions,
                                      table, n_q, n_kv, d, softcap if capped else scale, span, cuts=cuts, capped=capped,
                                      chunked=bool(chunk), sink=sink)
-        if batch.n_decode:
+        if batch.n_decode and v_cache is k_cache and n_kv == 1 and not capped and not chunk and not sink:
+            # rows that are key and value at once have their own kernel, which reads them once
+            key = ("shared_workspace", batch.n_decode, batch.max_decode_ctx, d, span)
+            workspace = batch.host.get(key)
+            if workspace is None:
+                workspace = batch.host[key] = rt.ops.attention_shared_workspace(batch.n_decode, d, batch.max_decode_ctx, span, rt.device)
+            rt.ops.attention_shared(q, k_cache, out, batch.decode_rows, batch.positions, batch.seq_of_token, table, n_q, d, scale, span, workspace)
+        elif batch.n_decode:
             rt.ops.attention_decode(q, k_cache, v_cache, out, batch.decode_rows, batch.positions, batch.seq_of_token, table,
                                     n_q, n_kv, d, softcap if capped else scale, span, batch.max_decode_ctx,
                                     owner._workspace(batch) if owner is not None else decode_workspace(rt, batch, n_q, d), capped=capped,
