@@ -15,7 +15,7 @@
 //
 // `prepare` (delta rule): the short causal convolutions over q | k | v with their silu, the unit norm of every q and k head,
 // beta and g, from the input product and the slot's last taps - 1 inputs; `conv_keep` then writes the slot's new last
-// inputs.  `finish`: a root mean square over a span of columns, a weight, a gate.
+// inputs (a step of single tokens: `prepare` itself).  `finish`: a root mean square over a span of columns, a weight, a gate.
 #include "common.h"
 #include "lane_sums.h"
 #include <math.h>
@@ -239,44 +239,83 @@ extern "C" int kipp_delta_scan(const float* prep, int stride, float* state, size
                           slots, o_raw, entries, heads, heads / kv_heads, d, dv, longest, stream);
 }
 
-// One workgroup a token.  conv_w [channels][taps]; kept [slot][taps - 1][channels] at `kept_at` floats into the slot.
+// The causal filter of one channel at token t: in[j] = its input `taps - 1 - j` tokens back (column `col` of proj; ahead of the portion,
+// which begins at `first`, what the slot kept of channel c), all asked for before the first is used; returns bias + sum_j w[c][j] in[j].
+// TAPS: the taps where they are known, else 0.
+template <int TAPS>
+struct Filter {
+    static constexpr int MOST = TAPS > 0 ? TAPS : MAX_TAPS;
+    float in[MOST];
+
+    __device__ __forceinline__ float at(const float* __restrict__ proj, int stride, int col, int t, int first, const float* kept, int channels,
+                                        int c, const float* __restrict__ conv_w, int taps_, float bias) {
+        const int taps = TAPS > 0 ? TAPS : taps_;
+        float w[MOST];
+#pragma unroll
+        for (int j = 0; j < MOST; ++j) {
+            if (j >= taps) break;
+            const int at = t - (taps - 1) + j;
+            const float* from = at >= first ? proj + (size_t)at * stride + col : kept + (size_t)(taps - 1 + (at - first)) * channels + c;
+            in[j] = *from;
+            w[j] = conv_w[(size_t)c * taps + j];
+        }
+        float y = bias;
+#pragma unroll
+        for (int j = 0; j < MOST; ++j)
+            if (j < taps) y = fmaf(w[j], in[j], y);
+        return y;
+    }
+    // A single token is the whole portion: the slot's last inputs move up by one.  Only by the one thread that reads them.
+    __device__ __forceinline__ void keep(float* kept, int channels, int c, int taps_) const {
+        const int taps = TAPS > 0 ? TAPS : taps_;
+#pragma unroll
+        for (int j = 1; j < MOST; ++j)
+            if (j < taps) kept[(size_t)(j - 1) * channels + c] = in[j];
+    }
+};
+
+// A wave a head of q or k, or 64 channels of v (and, first of all, the gates); a token's waves are shared out over gridDim.y workgroups: one
+// for prompts, for single tokens as many as there are (one token, 32 heads in all, us: 12 workgroups 5.2, one 29; a prompt of 1,801 tokens 42 before the loads were asked for together, 28).
+// conv_w [channels][taps]; kept [slot][taps - 1][channels] at `kept_at` floats into the slot.  `single`: every entry brings one
+// token, whose inputs go into the slot here.
+template <int TAPS>
 __global__ void __launch_bounds__(SCAN_THREADS)
 delta_prepare_kernel(const float* __restrict__ proj, int stride, const float* __restrict__ conv_w, int taps,
-                     const float* __restrict__ a_log, const float* __restrict__ dt_bias, const float* __restrict__ state,
+                     const float* __restrict__ a_log, const float* __restrict__ dt_bias, float* state,
                      size_t state_stride, size_t kept_at, const int32_t* __restrict__ seq_of_token,
                      const int32_t* __restrict__ q_start, const int32_t* __restrict__ slots, float* __restrict__ prep,
-                     int prep_stride, int heads, int kv_heads, int d, int dv, int beta_col, int a_col, float unit_eps) {
+                     int prep_stride, int heads, int kv_heads, int d, int dv, int beta_col, int a_col, float unit_eps, int single) {
     const int t = blockIdx.x;
     const int entry = seq_of_token[t];
     const int first = q_start[entry];
-    const int channels = 2 * kv_heads * d + heads * dv;
-    const float* kept = state + (size_t)slots[entry] * state_stride + kept_at;
+    const int normed = 2 * kv_heads, channels = normed * d + heads * dv;
+    float* kept = state + (size_t)slots[entry] * state_stride + kept_at;
     float* dst = prep + (size_t)t * prep_stride;
-    for (int c = threadIdx.x; c < channels; c += SCAN_THREADS) {
-        float y = 0.0f;
-        for (int j = 0; j < taps; ++j) {
-            const int at = t - (taps - 1) + j;      // the row of the input `taps - 1 - j` tokens back
-            const float in = at >= first ? proj[(size_t)at * stride + c] : kept[(size_t)(taps - 1 + (at - first)) * channels + c];
-            y = fmaf(conv_w[(size_t)c * taps + j], in, y);
+    if (blockIdx.y == 0)
+        for (int h = threadIdx.x; h < heads; h += SCAN_THREADS) {
+            const float* row = proj + (size_t)t * stride;
+            dst[channels + h] = sigmoid_f(row[beta_col + h]);
+            dst[channels + heads + h] = expf(-expf(a_log[h]) * softplus_f(row[a_col + h] + dt_bias[h]));
         }
-        dst[c] = silu_f(y);
-    }
-    for (int h = threadIdx.x; h < heads; h += SCAN_THREADS) {
-        const float* row = proj + (size_t)t * stride;
-        dst[channels + h] = sigmoid_f(row[beta_col + h]);
-        dst[channels + heads + h] = expf(-expf(a_log[h]) * softplus_f(row[a_col + h] + dt_bias[h]));
-    }
-    __syncthreads();
-    // every q and k head over the root of its sum of squares; q also over the root of d
-    const int wave = threadIdx.x / KIPP_WAVE, lane = threadIdx.x & (KIPP_WAVE - 1);
-    for (int hh = wave; hh < 2 * kv_heads; hh += SCAN_THREADS / KIPP_WAVE) {
-        float* head = dst + (size_t)hh * d;
+    const int lane = threadIdx.x & (KIPP_WAVE - 1), waves = gridDim.y * (SCAN_THREADS / KIPP_WAVE);
+    const int units = normed + (heads * dv + KIPP_WAVE - 1) / KIPP_WAVE;
+    for (int unit = blockIdx.y * (SCAN_THREADS / KIPP_WAVE) + threadIdx.x / KIPP_WAVE; unit < units; unit += waves) {
+        const bool head = unit < normed;
+        const int c0 = head ? unit * d : normed * d + (unit - normed) * KIPP_WAVE, end = head ? c0 + d : min(c0 + KIPP_WAVE, channels);
         float ss = 0.0f;
-        for (int e = lane; e < d; e += KIPP_WAVE) ss = fmaf(head[e], head[e], ss);
+        for (int c = c0 + lane; c < end; c += KIPP_WAVE) {
+            Filter<TAPS> filter;
+            const float y = silu_f(filter.at(proj, stride, c, t, first, kept, channels, c, conv_w, taps, 0.0f));
+            if (single) filter.keep(kept, channels, c, taps);
+            dst[c] = y;
+            ss = fmaf(y, y, ss);
+        }
+        if (!head) continue;
+        // every q and k head over the root of its sum of squares; q also over the root of d (a lane takes up what it wrote)
         ss = wave_sum(ss);
         float scale = 1.0f / sqrtf(ss + unit_eps);
-        if (hh < kv_heads) scale *= 1.0f / sqrtf((float)d);
-        for (int e = lane; e < d; e += KIPP_WAVE) head[e] *= scale;
+        if (unit < kv_heads) scale *= 1.0f / sqrtf((float)d);
+        for (int c = c0 + lane; c < end; c += KIPP_WAVE) dst[c] *= scale;
     }
 }
 
@@ -310,10 +349,18 @@ extern "C" int kipp_delta_prepare(const float* proj, int stride, const float* co
     const int channels = 2 * kv_heads * d + heads * dv;
     if (taps < 1 || taps > MAX_TAPS || heads <= 0 || kv_heads <= 0 || d <= 0 || dv <= 0) return -1;
     if (stride < channels || prep_stride < channels + 2 * heads || state_stride < kept_at + (size_t)(taps - 1) * channels) return -1;
-    hipLaunchKernelGGL(delta_prepare_kernel, dim3(tokens), dim3(SCAN_THREADS), 0, stream, proj, stride, conv_w, taps, a_log, dt_bias,
-                       (const float*)state, state_stride, kept_at, seq_of_token, q_start, slots, prep, prep_stride, heads, kv_heads, d, dv,
-                       beta_col, a_col, unit_eps);
-    if (taps > 1)
+    const int waves = SCAN_THREADS / KIPP_WAVE, units = 2 * kv_heads + (heads * dv + KIPP_WAVE - 1) / KIPP_WAVE;
+    const int most = (units + waves - 1) / waves, fill = (2 * 256 + tokens - 1) / tokens;      // two workgroups a compute unit
+    const dim3 grid(tokens, most < fill ? most : fill);
+    const int single = tokens == entries;
+#define KIPP_DP(TAPS)                                                                                                                  \
+    hipLaunchKernelGGL(delta_prepare_kernel<TAPS>, grid, dim3(SCAN_THREADS), 0, stream, proj, stride, conv_w, taps, a_log, dt_bias, state,  \
+                       state_stride, kept_at, seq_of_token, q_start, slots, prep, prep_stride, heads, kv_heads, d, dv, beta_col, a_col,   \
+                       unit_eps, single)
+    if (taps == 4) KIPP_DP(4);
+    else KIPP_DP(0);
+#undef KIPP_DP
+    if (taps > 1 && !single)
         hipLaunchKernelGGL(conv_keep_kernel, dim3((channels + 255) / 256, entries), dim3(256), 0, stream, proj, stride, taps, state,
                            state_stride, kept_at, q_start, q_len, slots, channels);
     return KIPP_LAUNCH_CHECK();
@@ -334,13 +381,14 @@ extern "C" int kipp_gated_scan(const float* prep, int stride, float* state, size
 // A thread a channel, for TOKENS tokens in a row.  proj: [z: inner | x: inner | B: groups n | C: groups n | dt: heads] (inner =
 // heads p); the channels x | B | C pass a causal filter (conv_w [channels][taps] with conv_b [channels], the slot's kept inputs
 // ahead of a portion; kept [taps - 1][channels] at `kept_at` floats into the slot) and silu.  prep as `kipp_gated_scan` reads it.
-template <int TOKENS>
+// `single`: every entry brings one token, whose inputs go into the slot here.
+template <int TOKENS, int TAPS>
 __global__ void __launch_bounds__(SCAN_THREADS)
 ssd_prepare_kernel(const float* __restrict__ proj, int stride, const float* __restrict__ conv_w, const float* __restrict__ conv_b, int taps,
-                   const float* __restrict__ a_log, const float* __restrict__ dt_bias, const float* __restrict__ state,
+                   const float* __restrict__ a_log, const float* __restrict__ dt_bias, float* state,
                    size_t state_stride, size_t kept_at, const int32_t* __restrict__ seq_of_token,
                    const int32_t* __restrict__ q_start, const int32_t* __restrict__ slots, float* __restrict__ prep,
-                   int prep_stride, int tokens, int heads, int groups, int n, int p) {
+                   int prep_stride, int tokens, int heads, int groups, int n, int p, int single) {
     const int t0 = blockIdx.x * TOKENS;
     const int inner = heads * p, gn = groups * n;
     const int channels = inner + 2 * gn;
@@ -364,15 +412,12 @@ ssd_prepare_kernel(const float* __restrict__ proj, int stride, const float* __re
         if (t >= tokens) break;
         const int entry = seq_of_token[t];
         const int first = q_start[entry];
-        const float* kept = state + (size_t)slots[entry] * state_stride + kept_at;
+        float* kept = state + (size_t)slots[entry] * state_stride + kept_at;
         float* dst = prep + (size_t)t * prep_stride;
         const float z = c < inner ? proj[(size_t)t * stride + dt_at + h] : 0.0f;
-        float y = bias;
-        for (int j = 0; j < taps; ++j) {
-            const int at = t - (taps - 1) + j;      // the row of the input `taps - 1 - j` tokens back
-            const float in = at >= first ? proj[(size_t)at * stride + inner + c] : kept[(size_t)(taps - 1 + (at - first)) * channels + c];
-            y = fmaf(conv_w[(size_t)c * taps + j], in, y);
-        }
+        Filter<TAPS> filter;
+        float y = filter.at(proj, stride, inner + c, t, first, kept, channels, c, conv_w, taps, bias);
+        if (single) filter.keep(kept, channels, c, taps);
         y = silu_f(y);
         if (c < inner) {
             dst[2 * gn + c] = softplus_f(z + dtb) * y;
@@ -395,14 +440,20 @@ extern "C" int kipp_ssd_prepare(const float* proj, int stride, const float* conv
     if (stride < inner + channels + heads || prep_stride < 2 * groups * n + 2 * inner + heads ||
         state_stride < kept_at + (size_t)(taps - 1) * channels) return -1;
     const int cols = (channels + SCAN_THREADS - 1) / SCAN_THREADS;
-#define KIPP_SP(TOKENS)                                                                                                               \
-    hipLaunchKernelGGL(ssd_prepare_kernel<TOKENS>, dim3((tokens + TOKENS - 1) / TOKENS, cols), dim3(SCAN_THREADS), 0, stream, proj, stride, \
-                       conv_w, conv_b, taps, a_log, dt_bias, (const float*)state, state_stride, kept_at, seq_of_token, q_start, slots, prep, \
-                       prep_stride, tokens, heads, groups, n, p)
-    if (tokens >= 512) KIPP_SP(4);
-    else KIPP_SP(1);
+    const int single = tokens == entries;
+#define KIPP_SP(TOKENS, TAPS)                                                                                                         \
+    hipLaunchKernelGGL((ssd_prepare_kernel<TOKENS, TAPS>), dim3((tokens + TOKENS - 1) / TOKENS, cols), dim3(SCAN_THREADS), 0, stream, proj, \
+                       stride, conv_w, conv_b, taps, a_log, dt_bias, state, state_stride, kept_at, seq_of_token, q_start, slots, prep, \
+                       prep_stride, tokens, heads, groups, n, p, single)
+    if (taps == 4) {
+        if (tokens >= 512) KIPP_SP(4, 4);
+        else KIPP_SP(1, 4);
+    } else {
+        if (tokens >= 512) KIPP_SP(4, 0);
+        else KIPP_SP(1, 0);
+    }
 #undef KIPP_SP
-    if (taps > 1)
+    if (taps > 1 && !single)
         hipLaunchKernelGGL(conv_keep_kernel, dim3((channels + 255) / 256, entries), dim3(256), 0, stream, proj + inner, stride, taps, state,
                            state_stride, kept_at, q_start, q_len, slots, channels);
     return KIPP_LAUNCH_CHECK();
@@ -410,7 +461,9 @@ extern "C" int kipp_ssd_prepare(const float* proj, int stride, const float* conv
 
 // y[t][c] = (o[t][c] + skip[c / p] x[t][c]) * silu(z[t][c]); out = y * rsqrt(mean over c's span of y^2 + eps) * w[c]: the gate
 // comes before the norm.  x at column `x_at` of prep, z at column `z_at` of proj.
-template <typename TO>
+// ITEMS columns a thread (beyond: read for the sum, and again), all asked for at once: for single tokens the loads' latencies are the time
+// (a token of 5,120 columns 6.6 us; 10.9 with a column after the other).
+template <typename TO, int ITEMS>
 __global__ void __launch_bounds__(SCAN_THREADS)
 ssd_finish_kernel(const float* __restrict__ o_raw, const float* __restrict__ prep, int prep_stride, int x_at,
                   const float* __restrict__ proj, int proj_stride, int z_at, const float* __restrict__ skip, int p,
@@ -421,13 +474,34 @@ ssd_finish_kernel(const float* __restrict__ o_raw, const float* __restrict__ pre
     const float* o = o_raw + t * width + c0;
     const float* x = prep + t * prep_stride + x_at + c0;
     const float* z = proj + t * proj_stride + z_at + c0;
+    float ov[ITEMS], xv[ITEMS], zv[ITEMS], sv[ITEMS], wv[ITEMS];
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+        const int e = min((int)threadIdx.x + i * SCAN_THREADS, span - 1);
+        ov[i] = o[e];
+        xv[i] = x[e];
+        zv[i] = z[e];
+        sv[i] = skip[(c0 + e) / p];
+        wv[i] = w[c0 + e];
+    }
+    __builtin_amdgcn_sched_barrier(0);
     float ss = 0.0f;
-    for (int e = threadIdx.x; e < span; e += SCAN_THREADS) {
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+        ov[i] = fmaf(sv[i], xv[i], ov[i]) * silu_f(zv[i]);
+        if ((int)threadIdx.x + i * SCAN_THREADS < span) ss = fmaf(ov[i], ov[i], ss);
+    }
+    for (int e = threadIdx.x + ITEMS * SCAN_THREADS; e < span; e += SCAN_THREADS) {
         const float y = fmaf(skip[(c0 + e) / p], x[e], o[e]) * silu_f(z[e]);
         ss = fmaf(y, y, ss);
     }
     const float inv = 1.0f / sqrtf(block_sum(ss, scratch) / (float)span + eps);
-    for (int e = threadIdx.x; e < span; e += SCAN_THREADS) {
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+        const int e = threadIdx.x + i * SCAN_THREADS;
+        if (e < span) store_f(out, t * width + c0 + e, ov[i] * inv * wv[i]);
+    }
+    for (int e = threadIdx.x + ITEMS * SCAN_THREADS; e < span; e += SCAN_THREADS) {
         const float y = fmaf(skip[(c0 + e) / p], x[e], o[e]) * silu_f(z[e]);
         store_f(out, t * width + c0 + e, y * inv * w[c0 + e]);
     }
@@ -439,14 +513,22 @@ extern "C" int kipp_ssd_finish(const float* o_raw, const float* prep, int prep_s
     if (tokens <= 0) return 0;
     if (width <= 0 || span <= 0 || width % span || p <= 0 || width % p || prep_stride < x_at + width || proj_stride < z_at + width) return -1;
     dim3 grid(width / span, tokens), block(SCAN_THREADS);
-    if (out_dtype == KIPP_F32)
-        hipLaunchKernelGGL((ssd_finish_kernel<float>), grid, block, 0, stream, o_raw, prep, prep_stride, x_at, proj, proj_stride, z_at, skip, p,
-                           w, eps, (float*)out, width, span);
-    else if (out_dtype == KIPP_BF16)
-        hipLaunchKernelGGL((ssd_finish_kernel<bf16_t>), grid, block, 0, stream, o_raw, prep, prep_stride, x_at, proj, proj_stride, z_at, skip, p,
-                           w, eps, (bf16_t*)out, width, span);
-    else
+#define KIPP_SF(TO, ITEMS)                                                                                                             \
+    hipLaunchKernelGGL((ssd_finish_kernel<TO, ITEMS>), grid, block, 0, stream, o_raw, prep, prep_stride, x_at, proj, proj_stride, z_at, skip, p, \
+                       w, eps, (TO*)out, width, span)
+#define KIPP_SFT(TO)                                                                                                                   \
+    if (span <= SCAN_THREADS) KIPP_SF(TO, 1);                                                                                          \
+    else if (span <= 4 * SCAN_THREADS) KIPP_SF(TO, 4);                                                                                 \
+    else KIPP_SF(TO, 20)
+    if (out_dtype == KIPP_F32) {
+        KIPP_SFT(float);
+    } else if (out_dtype == KIPP_BF16) {
+        KIPP_SFT(bf16_t);
+    } else {
         return -2;
+    }
+#undef KIPP_SFT
+#undef KIPP_SF
     return KIPP_LAUNCH_CHECK();
 }
 
