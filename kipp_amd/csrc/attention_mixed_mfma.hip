@@ -81,6 +81,16 @@ union Frag {
     bf16_t h[8];
 };
 
+typedef __attribute__((ext_vector_type(2))) float f32x2;
+typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
+
+__device__ __forceinline__ uint32_t to_bf16_pair(float a, float b) {
+    const f32x2 f = {a, b};
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, bf16x2));
+}
+
+#define LOG2E 1.4426950408889634f
+
 struct MixedGeometry {
     const int32_t* item_entry;      // [items] entry of the batch
     const int32_t* item_row0;       // [items] first row of the tile within its entry
@@ -127,19 +137,25 @@ __device__ __forceinline__ int key_tile(const Tile& t, int index) {
     return index < t.kept_tiles ? index : t.window_tile0 + index - t.kept_tiles;
 }
 
+// The page of a lane's key among the 16 from `key0` on.
+__device__ __forceinline__ int page_of(const MixedGeometry& g, const Tile& t, int key0) {
+    return t.table[min(key0 + (int)(threadIdx.x & 15), t.last) / g.page];
+}
+
 // The 16 keys from `key0` on of key/value head `c` as A operands: lane l holds key l % 16, columns 32 s + 8 (l / 16) ..
-__device__ __forceinline__ void load_keys(const MixedGeometry& g, const Tile& t, const bf16_t* __restrict__ k_cache, int c, int key0,
+// `page`: the lane's page_of them.
+__device__ __forceinline__ void load_keys(const MixedGeometry& g, const Tile& t, const bf16_t* __restrict__ k_cache, int c, int key0, int page,
                                           Frag* kf) {
     const int lane = threadIdx.x & (KIPP_WAVE - 1), l16 = lane & 15, quarter = lane >> 4;
     const int key = min(key0 + l16, t.last);            // rows beyond the context are masked later; their loads stay inside it
-    const bf16_t* row = k_cache + (((size_t)t.table[key / g.page] * g.n_kv + c) * g.page + key % g.page) * HEAD_DIM + 8 * quarter;
+    const bf16_t* row = k_cache + (((size_t)page * g.n_kv + c) * g.page + key % g.page) * HEAD_DIM + 8 * quarter;
 #pragma unroll
     for (int s = 0; s < KSTEPS; ++s) kf[s].u = *(const u32x4*)(row + 32 * s);
 }
 
 // S^T[key][row] of one head for the 16 keys from `key0` on: lane l gets keys key0 + 4 (l / 16) + v of row l % 16,
-// already scaled, biased by distance and masked (-inf).  `kf`: the keys as A operands, `qf`: the head's query rows
-// as B operands.
+// already scaled, biased by distance and masked (-inf), in base 2 (2^score is the weight: `scale2` is the scale times log2 e, and
+// e^(-a ln u) is 2^(-a log2 u)).  `kf`: the keys as A operands, `qf`: the head's query rows as B operands.
 template <bool INSIDE>
 __device__ __forceinline__ void scores16(const MixedGeometry& g, const Tile& t, int key0, const Frag* kf, const Frag* qf,
                                          float a, float b, float sc[4]) {
@@ -147,13 +163,14 @@ __device__ __forceinline__ void scores16(const MixedGeometry& g, const Tile& t, 
     f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int s = 0; s < KSTEPS; ++s) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[s].v, qf[s].v, acc, 0, 0, 0);
-    const int i = t.pos0 + l16;
+    const int i = t.pos0 + l16, away = i - key0 - 4 * quarter;
+    const float scale2 = g.scale * LOG2E, away0 = (float)away;
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-        const int j = key0 + 4 * quarter + v;
         // INSIDE: every row of the tile sees all 16 keys (rows that only fill the tile up compute unused numbers)
-        const bool sees = INSIDE || (l16 < t.rows && j <= i && (g.window <= 0 || i - j < g.window || j < g.keep_first));
-        sc[v] = sees ? acc[v] * g.scale - a * __logf(1.0f + b * (float)(i - j)) : -INFINITY;
+        const bool sees = INSIDE || (l16 < t.rows && away >= v && (g.window <= 0 || away - v < g.window || i - away + v < g.keep_first));
+        const float s = fmaf(acc[v], scale2, -a * __builtin_amdgcn_logf(fmaf(b, away0 - (float)v, 1.0f)));
+        sc[v] = sees ? s : -INFINITY;
     }
 }
 
@@ -172,7 +189,9 @@ __device__ __forceinline__ void load_queries(const Tile& t, const bf16_t* __rest
     for (int s = 0; s < KSTEPS; ++s) qf[s].u = *(const u32x4*)(at + 32 * s);
 }
 
-// stats [items][n_q][16][2]: (maximum, sum of exp(score - maximum)) over the item's keys, without the sink.
+// stats [items][n_q][16][2]: (maximum, sum of 2^(score - maximum)) over the item's keys, without the sink.
+// Bound by vector instructions (a logarithm and an exponential a score): 1,500 rows of 32 heads 51 us with both in base 2 and the pages
+// asked for a tile ahead of the keys, 68 in base e.
 __global__ void __launch_bounds__(MX_THREADS) mixed_stats_kernel(MixedGeometry g, const bf16_t* __restrict__ q,
                                                                  const bf16_t* __restrict__ k_cache, float* __restrict__ stats) {
     const int item = blockIdx.x;
@@ -193,9 +212,15 @@ __global__ void __launch_bounds__(MX_THREADS) mixed_stats_kernel(MixedGeometry g
         l[hh] = 0.0f;
     }
     Frag kf[MX_KEYS / 16][KSTEPS], next[MX_KEYS / 16][KSTEPS];
+    int page[MX_KEYS / 16], page_next[MX_KEYS / 16];        // of this tile's keys and of the next's: asked for a tile ahead of the keys
     if (t.begin < t.end) {
 #pragma unroll
-        for (int kb = 0; kb < MX_KEYS / 16; ++kb) load_keys(g, t, k_cache, h0 / group, key_tile(t, t.begin) * MX_KEYS + 16 * kb, next[kb]);
+        for (int kb = 0; kb < MX_KEYS / 16; ++kb) {
+            page[kb] = page_of(g, t, key_tile(t, t.begin) * MX_KEYS + 16 * kb);
+            page_next[kb] = page_of(g, t, key_tile(t, min(t.begin + 1, t.end - 1)) * MX_KEYS + 16 * kb);
+        }
+#pragma unroll
+        for (int kb = 0; kb < MX_KEYS / 16; ++kb) load_keys(g, t, k_cache, h0 / group, key_tile(t, t.begin) * MX_KEYS + 16 * kb, page[kb], next[kb]);
     }
     for (int index = t.begin; index < t.end; ++index) {
         const int key0 = key_tile(t, index) * MX_KEYS;
@@ -204,9 +229,16 @@ __global__ void __launch_bounds__(MX_THREADS) mixed_stats_kernel(MixedGeometry g
 #pragma unroll
             for (int s = 0; s < KSTEPS; ++s) kf[kb][s] = next[kb][s];
         const bool inside = all_seen(g, t, key0);
+        int own_page[MX_KEYS / 16];
+#pragma unroll
+        for (int kb = 0; kb < MX_KEYS / 16; ++kb) own_page[kb] = page[kb];
         if (index + 1 < t.end) {            // the next tile's keys are on their way while this one is scored
 #pragma unroll
-            for (int kb = 0; kb < MX_KEYS / 16; ++kb) load_keys(g, t, k_cache, h0 / group, key_tile(t, index + 1) * MX_KEYS + 16 * kb, next[kb]);
+            for (int kb = 0; kb < MX_KEYS / 16; ++kb) {
+                page[kb] = page_next[kb];
+                load_keys(g, t, k_cache, h0 / group, key_tile(t, index + 1) * MX_KEYS + 16 * kb, page[kb], next[kb]);
+                page_next[kb] = page_of(g, t, key_tile(t, min(index + 2, t.end - 1)) * MX_KEYS + 16 * kb);
+            }
         }
 #pragma unroll
         for (int hh = 0; hh < HPW; ++hh) {
@@ -214,7 +246,7 @@ __global__ void __launch_bounds__(MX_THREADS) mixed_stats_kernel(MixedGeometry g
 #pragma unroll
             for (int kb = 0; kb < MX_KEYS / 16; ++kb) {
                 Frag own[KSTEPS];
-                if (!shared && hh > 0) load_keys(g, t, k_cache, (h0 + hh) / group, key0 + 16 * kb, own);
+                if (!shared && hh > 0) load_keys(g, t, k_cache, (h0 + hh) / group, key0 + 16 * kb, own_page[kb], own);
                 float sc[4];
                 if (inside) scores16<true>(g, t, key0 + 16 * kb, (!shared && hh > 0) ? own : kf[kb], qf[hh], a[hh], b[hh], sc);
                 else scores16<false>(g, t, key0 + 16 * kb, (!shared && hh > 0) ? own : kf[kb], qf[hh], a[hh], b[hh], sc);
@@ -222,8 +254,8 @@ __global__ void __launch_bounds__(MX_THREADS) mixed_stats_kernel(MixedGeometry g
                 if (m_new != -INFINITY) {
                     float sum = 0.0f;
 #pragma unroll
-                    for (int v = 0; v < 4; ++v) sum += __expf(sc[v] - m_new);       // exp(-inf) = 0
-                    l[hh] = l[hh] * __expf(m[hh] - m_new) + sum;
+                    for (int v = 0; v < 4; ++v) sum += __builtin_amdgcn_exp2f(sc[v] - m_new);       // exp(-inf) = 0
+                    l[hh] = l[hh] * __builtin_amdgcn_exp2f(m[hh] - m_new) + sum;
                     m[hh] = m_new;
                 }
             }
@@ -238,7 +270,7 @@ __global__ void __launch_bounds__(MX_THREADS) mixed_stats_kernel(MixedGeometry g
         for (int off = 16; off <= 32; off <<= 1) {
             const float m_o = __shfl_xor(mm, off, KIPP_WAVE), l_o = __shfl_xor(ll, off, KIPP_WAVE);
             const float m_new = fmaxf(mm, m_o);
-            if (m_new != -INFINITY) ll = ll * __expf(mm - m_new) + l_o * __expf(m_o - m_new);
+            if (m_new != -INFINITY) ll = ll * __builtin_amdgcn_exp2f(mm - m_new) + l_o * __builtin_amdgcn_exp2f(m_o - m_new);
             mm = m_new;
         }
         if (lane < 16) {
@@ -249,6 +281,8 @@ __global__ void __launch_bounds__(MX_THREADS) mixed_stats_kernel(MixedGeometry g
     }
 }
 
+// Bound by vector instructions, LDS and two barriers a tile: 1,500 rows of 32 heads of 128 181 us (186 with weights in base e).  Values and
+// pages asked for ahead as well: 198 (no registers are left: they spill).
 // LDS: p_hi, p_lo [16 rows][32 keys][32 heads] bfloat16, then p' [32 heads][16 rows][32 keys] bfloat16, with the padded strides above.
 __global__ void __launch_bounds__(MX_THREADS) mixed_values_kernel(
     MixedGeometry g, const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache,
@@ -284,14 +318,13 @@ __global__ void __launch_bounds__(MX_THREADS) mixed_values_kernel(
         }
     }
 
-    // this wave's heads: queries, bias numbers, and every row's maximum and 1 / denominator over ALL runs of the tile
+    // this wave's heads: queries, bias numbers, and every row's maximum and denominator over ALL runs of the tile
     Frag qf[HPW][KSTEPS];
-    float bias_a[HPW], bias_b[HPW], top[HPW], inv[HPW];
+    float bias_a[HPW], bias_b[HPW], under[HPW];         // a weight is 2^(score + under)
 #pragma unroll
     for (int hh = 0; hh < HPW; ++hh) {
         const int h = wave * HPW + hh;
-        top[hh] = 0.0f;
-        inv[hh] = 0.0f;
+        under[hh] = -INFINITY;
         bias_a[hh] = bias_b[hh] = 0.0f;
         if (h < n_q) {
             load_queries(t, q, n_q, h, qf[hh]);
@@ -309,7 +342,7 @@ __global__ void __launch_bounds__(MX_THREADS) mixed_values_kernel(
 #pragma unroll
                 for (int s = 0; s < 4; ++s) {
                     const float m_new = fmaxf(m, st[s].x);
-                    if (m_new != -INFINITY) l = l * __expf(m - m_new) + st[s].y * __expf(st[s].x - m_new);
+                    if (m_new != -INFINITY) l = l * __builtin_amdgcn_exp2f(m - m_new) + st[s].y * __builtin_amdgcn_exp2f(st[s].x - m_new);
                     m = m_new;
                 }
             }
@@ -317,16 +350,15 @@ __global__ void __launch_bounds__(MX_THREADS) mixed_values_kernel(
             for (int off = 16; off <= 32; off <<= 1) {
                 const float m_o = __shfl_xor(m, off, KIPP_WAVE), l_o = __shfl_xor(l, off, KIPP_WAVE);
                 const float m_new = fmaxf(m, m_o);
-                if (m_new != -INFINITY) l = l * __expf(m - m_new) + l_o * __expf(m_o - m_new);
+                if (m_new != -INFINITY) l = l * __builtin_amdgcn_exp2f(m - m_new) + l_o * __builtin_amdgcn_exp2f(m_o - m_new);
                 m = m_new;
             }
             if (sink != nullptr) {
-                const float m_new = fmaxf(m, sink[h]);
-                l = (m == -INFINITY ? 0.0f : l * __expf(m - m_new)) + __expf(sink[h] - m_new);
+                const float sunk = sink[h] * LOG2E, m_new = fmaxf(m, sunk);
+                l = (m == -INFINITY ? 0.0f : l * __builtin_amdgcn_exp2f(m - m_new)) + __builtin_amdgcn_exp2f(sunk - m_new);
                 m = m_new;
             }
-            top[hh] = m;
-            inv[hh] = l > 0.0f ? 1.0f / l : 0.0f;
+            under[hh] = l > 0.0f ? -m - __builtin_amdgcn_logf(l) : -INFINITY;
         }
     }
 
@@ -346,7 +378,7 @@ __global__ void __launch_bounds__(MX_THREADS) mixed_values_kernel(
         for (int kb = 0; kb < MX_KEYS / 16; ++kb) {
             if (wave * HPW < n_q) {
                 Frag kf[KSTEPS];
-                load_keys(g, t, k_cache, wave * HPW / group, key0 + 16 * kb, kf);
+                load_keys(g, t, k_cache, wave * HPW / group, key0 + 16 * kb, page_of(g, t, key0 + 16 * kb), kf);
                 float p[HPW][4];
 #pragma unroll
                 for (int hh = 0; hh < HPW; ++hh) {
@@ -354,34 +386,38 @@ __global__ void __launch_bounds__(MX_THREADS) mixed_values_kernel(
 #pragma unroll
                     for (int v = 0; v < 4; ++v) p[hh][v] = 0.0f;
                     if (h < n_q) {
-                        if (!shared && hh > 0) load_keys(g, t, k_cache, h / group, key0 + 16 * kb, kf);
+                        if (!shared && hh > 0) load_keys(g, t, k_cache, h / group, key0 + 16 * kb, page_of(g, t, key0 + 16 * kb), kf);
                         float sc[4];
                         if (inside) scores16<true>(g, t, key0 + 16 * kb, kf, qf[hh], bias_a[hh], bias_b[hh], sc);
                         else scores16<false>(g, t, key0 + 16 * kb, kf, qf[hh], bias_a[hh], bias_b[hh], sc);
 #pragma unroll
-                        for (int v = 0; v < 4; ++v) p[hh][v] = sc[v] == -INFINITY ? 0.0f : __expf(sc[v] - top[hh]) * inv[hh];
+                        for (int v = 0; v < 4; ++v) p[hh][v] = __builtin_amdgcn_exp2f(sc[v] + under[hh]);
                     }
                 }
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
                     const int at = l16 * P_ROW + (16 * kb + 4 * quarter + v) * P_KEY + wave * HPW;
-                    bf16_t hi[HPW], lo[HPW];
+                    if (HPW == 4 || HPW == 2) {
+                        uint32_t hi[(HPW + 1) / 2], lo[(HPW + 1) / 2];
 #pragma unroll
-                    for (int hh = 0; hh < HPW; ++hh) {
-                        hi[hh] = to_bf16(p[hh][v]);
-                        lo[hh] = to_bf16(p[hh][v] - bf16_to_f32(hi[hh]));
-                    }
-                    if (HPW == 4) {
-                        *(uint2*)(p_hi + at) = make_uint2((uint32_t)hi[0] | ((uint32_t)hi[1 % HPW] << 16), (uint32_t)hi[2 % HPW] | ((uint32_t)hi[3 % HPW] << 16));
-                        *(uint2*)(p_lo + at) = make_uint2((uint32_t)lo[0] | ((uint32_t)lo[1 % HPW] << 16), (uint32_t)lo[2 % HPW] | ((uint32_t)lo[3 % HPW] << 16));
-                    } else if (HPW == 2) {
-                        *(uint32_t*)(p_hi + at) = (uint32_t)hi[0] | ((uint32_t)hi[1 % HPW] << 16);
-                        *(uint32_t*)(p_lo + at) = (uint32_t)lo[0] | ((uint32_t)lo[1 % HPW] << 16);
+                        for (int two = 0; two < HPW / 2; ++two) {
+                            const float a = p[2 * two % HPW][v], b = p[(2 * two + 1) % HPW][v];
+                            hi[two] = to_bf16_pair(a, b);
+                            lo[two] = to_bf16_pair(a - __uint_as_float(hi[two] << 16), b - __uint_as_float(hi[two] & 0xffff0000u));
+                        }
+                        if (HPW == 4) {
+                            *(uint2*)(p_hi + at) = make_uint2(hi[0], hi[HPW / 2 - 1]);
+                            *(uint2*)(p_lo + at) = make_uint2(lo[0], lo[HPW / 2 - 1]);
+                        } else {
+                            *(uint32_t*)(p_hi + at) = hi[0];
+                            *(uint32_t*)(p_lo + at) = lo[0];
+                        }
                     } else {
 #pragma unroll
                         for (int hh = 0; hh < HPW; ++hh) {
-                            p_hi[at + hh] = hi[hh];
-                            p_lo[at + hh] = lo[hh];
+                            const bf16_t hi = to_bf16(p[hh][v]);
+                            p_hi[at + hh] = hi;
+                            p_lo[at + hh] = to_bf16(p[hh][v] - bf16_to_f32(hi));
                         }
                     }
                 }
@@ -406,8 +442,8 @@ __global__ void __launch_bounds__(MX_THREADS) mixed_values_kernel(
                     const int h = 16 * nb + l16;        // d[v]: keys 16 kb + 4 quarter + v of `row`, head h
                     if (h < n_q) {
                         uint2 w;
-                        w.x = (uint32_t)to_bf16(d[0]) | ((uint32_t)to_bf16(d[1]) << 16);
-                        w.y = (uint32_t)to_bf16(d[2]) | ((uint32_t)to_bf16(d[3]) << 16);
+                        w.x = to_bf16_pair(d[0], d[1]);
+                        w.y = to_bf16_pair(d[2], d[3]);
                         *(uint2*)(p_mixed + (h * M_HEAD + row * M_ROW + 16 * kb + 4 * quarter)) = w;
                     }
                 }
