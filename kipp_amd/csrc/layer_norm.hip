@@ -6,28 +6,32 @@
 //     norm   out = scale * LN(sum of the slabs of u)                                  (any output type)
 //     step   x <- x + mult * LN_post(sum of the slabs of delta) [+ extra];  out = LN_next(x)   (out optional)
 //
-// One workgroup a row; the row stays in registers (a lane holds every 256th column), so a row is read once.  The
+// One workgroup a row; the row stays in registers (a lane holds every 256th column), so a row is read once, and what the step reads beside
+// it is asked for before the first sum (built for rows of up to 10, 20 and 32 of a lane's columns: a lane that asks for
+// columns beyond the row's waits for them too).  Bound by its reads: 2,048 rows of 2,560, 2 or 3 slabs (about 100 MB) 33 us; 39 with the
+// residual stream asked for behind the sums and a slab behind the other.  The
 // mean is taken first and the variance from the deviations, both summed over the workgroup in an order that the
 // width alone fixes: a row's result does not depend on what else is in the launch.  All arithmetic is float32.
 #include "common.h"
 #include <math.h>
 
 #define LN_THREADS 256
-#define LN_ITEMS 32     // columns a lane holds: rows of up to 8,192 numbers
+#define LN_ITEMS 32     // columns a lane holds at most: rows of up to 8,192 numbers
 
 struct RowStats {
     float mean, inv;
 };
 
-__device__ __forceinline__ RowStats row_stats(const float (&v)[LN_ITEMS], int width, float eps, float* scratch) {
+template <int ITEMS>
+__device__ __forceinline__ RowStats row_stats(const float (&v)[ITEMS], int width, float eps, float* scratch) {
     float s = 0.0f;
 #pragma unroll
-    for (int i = 0; i < LN_ITEMS; ++i)
+    for (int i = 0; i < ITEMS; ++i)
         if ((int)threadIdx.x + i * LN_THREADS < width) s += v[i];
     const float mean = block_sum(s, scratch) / (float)width;
     float ss = 0.0f;
 #pragma unroll
-    for (int i = 0; i < LN_ITEMS; ++i)
+    for (int i = 0; i < ITEMS; ++i)
         if ((int)threadIdx.x + i * LN_THREADS < width) {
             const float dlt = v[i] - mean;
             ss = fmaf(dlt, dlt, ss);
@@ -39,37 +43,52 @@ __device__ __forceinline__ RowStats row_stats(const float (&v)[LN_ITEMS], int wi
     return r;
 }
 
-__device__ __forceinline__ void load_slabs(float (&v)[LN_ITEMS], const float* __restrict__ src, int parts, size_t part_stride, int width) {
+// v[i] = src at this lane's columns (columns beyond the row's read its last one and are not used)
+template <int ITEMS>
+__device__ __forceinline__ void load_row(float (&v)[ITEMS], const float* __restrict__ src, int width) {
 #pragma unroll
-    for (int i = 0; i < LN_ITEMS; ++i) {
-        const int c = (int)threadIdx.x + i * LN_THREADS;
-        float a = 0.0f;
-        if (c < width) {
-            a = src[c];
-            for (int p = 1; p < parts; ++p) a += src[p * part_stride + c];
+    for (int i = 0; i < ITEMS; ++i) v[i] = src[min((int)threadIdx.x + i * LN_THREADS, width - 1)];
+}
+
+// The slabs added in order: the first four are asked for before any is used.
+template <int ITEMS>
+__device__ __forceinline__ void load_slabs(float (&v)[ITEMS], const float* __restrict__ src, int parts, size_t part_stride, int width) {
+    load_row(v, src, width);
+    float more[3][ITEMS];
+#pragma unroll
+    for (int p = 1; p < 4; ++p)
+        if (p < parts) load_row(more[p - 1], src + p * part_stride, width);
+#pragma unroll
+    for (int p = 1; p < 4; ++p)
+        if (p < parts) {
+#pragma unroll
+            for (int i = 0; i < ITEMS; ++i) v[i] += more[p - 1][i];
         }
-        v[i] = a;
+    for (int p = 4; p < parts; ++p) {
+        load_row(more[0], src + p * part_stride, width);
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i) v[i] += more[0][i];
     }
 }
 
-template <typename TO>
+template <typename TO, int ITEMS>
 __global__ void __launch_bounds__(LN_THREADS)
 layer_norm_kernel(const float* __restrict__ u, int parts, size_t part_stride, const float* __restrict__ w,
                   const float* __restrict__ b, float eps, float scale, TO* __restrict__ out, int width) {
     __shared__ float scratch[16];
     const size_t row = blockIdx.x;
-    float v[LN_ITEMS];
+    float v[ITEMS];
     load_slabs(v, u + row * width, parts, part_stride, width);
     const RowStats st = row_stats(v, width, eps, scratch);
     TO* dst = out + row * width;
 #pragma unroll
-    for (int i = 0; i < LN_ITEMS; ++i) {
+    for (int i = 0; i < ITEMS; ++i) {
         const int c = (int)threadIdx.x + i * LN_THREADS;
         if (c < width) store_f(dst, c, ((v[i] - st.mean) * st.inv * w[c] + b[c]) * scale);
     }
 }
 
-template <typename TO>
+template <typename TO, int ITEMS>
 __global__ void __launch_bounds__(LN_THREADS)
 sandwich_step_kernel(float* __restrict__ x, const float* __restrict__ delta, int parts, size_t part_stride,
                      const float* __restrict__ post_w, const float* __restrict__ post_b, float post_eps, float mult,
@@ -77,15 +96,16 @@ sandwich_step_kernel(float* __restrict__ x, const float* __restrict__ delta, int
                      float next_eps, TO* __restrict__ out, int width) {
     __shared__ float scratch[16];
     const size_t row = blockIdx.x;
-    float v[LN_ITEMS];
+    float* xr = x + row * width;
+    float v[ITEMS], old[ITEMS];
+    load_row(old, xr, width);
     load_slabs(v, delta + row * width, parts, part_stride, width);
     const RowStats st = row_stats(v, width, post_eps, scratch);
-    float* xr = x + row * width;
 #pragma unroll
-    for (int i = 0; i < LN_ITEMS; ++i) {
+    for (int i = 0; i < ITEMS; ++i) {
         const int c = (int)threadIdx.x + i * LN_THREADS;
         if (c < width) {
-            float nx = xr[c] + mult * ((v[i] - st.mean) * st.inv * post_w[c] + post_b[c]);
+            float nx = old[i] + mult * ((v[i] - st.mean) * st.inv * post_w[c] + post_b[c]);
             if (extra != nullptr) nx += extra[row * width + c];
             xr[c] = nx;
             v[i] = nx;
@@ -95,25 +115,40 @@ sandwich_step_kernel(float* __restrict__ x, const float* __restrict__ delta, int
     const RowStats nt = row_stats(v, width, next_eps, scratch);
     TO* dst = out + row * width;
 #pragma unroll
-    for (int i = 0; i < LN_ITEMS; ++i) {
+    for (int i = 0; i < ITEMS; ++i) {
         const int c = (int)threadIdx.x + i * LN_THREADS;
         if (c < width) store_f(dst, c, (v[i] - nt.mean) * nt.inv * next_w[c] + next_b[c]);
     }
 }
+
+// the build whose lanes hold the fewest columns that make up the row
+#define KIPP_LN_ITEMS(LAUNCH)                              \
+    do {                                                   \
+        if (width <= 10 * LN_THREADS) LAUNCH(10);          \
+        else if (width <= 20 * LN_THREADS) LAUNCH(20);     \
+        else LAUNCH(LN_ITEMS);                             \
+    } while (0)
 
 extern "C" int kipp_layer_norm(const float* u, int parts, const float* w, const float* b, float eps, float scale, void* out,
                                int out_dtype, int rows, int width, hipStream_t stream) {
     if (rows <= 0) return 0;
     if (width <= 0 || width > LN_THREADS * LN_ITEMS || parts <= 0) return -1;
     const size_t part_stride = (size_t)rows * width;
-    if (out_dtype == KIPP_F32)
-        hipLaunchKernelGGL((layer_norm_kernel<float>), dim3(rows), dim3(LN_THREADS), 0, stream, u, parts, part_stride, w, b, eps, scale,
-                           (float*)out, width);
-    else if (out_dtype == KIPP_BF16)
-        hipLaunchKernelGGL((layer_norm_kernel<bf16_t>), dim3(rows), dim3(LN_THREADS), 0, stream, u, parts, part_stride, w, b, eps, scale,
-                           (bf16_t*)out, width);
-    else
+#define KIPP_LN(ITEMS)                                                                                                             \
+    hipLaunchKernelGGL((layer_norm_kernel<KIPP_LN_TO, ITEMS>), dim3(rows), dim3(LN_THREADS), 0, stream, u, parts, part_stride, w, b, eps, \
+                       scale, (KIPP_LN_TO*)out, width)
+    if (out_dtype == KIPP_F32) {
+#define KIPP_LN_TO float
+        KIPP_LN_ITEMS(KIPP_LN);
+#undef KIPP_LN_TO
+    } else if (out_dtype == KIPP_BF16) {
+#define KIPP_LN_TO bf16_t
+        KIPP_LN_ITEMS(KIPP_LN);
+#undef KIPP_LN_TO
+    } else {
         return -2;
+    }
+#undef KIPP_LN
     return KIPP_LAUNCH_CHECK();
 }
 
@@ -124,13 +159,20 @@ extern "C" int kipp_sandwich_step(float* x, const float* delta, int parts, const
     if (width <= 0 || width > LN_THREADS * LN_ITEMS || parts <= 0) return -1;
     if (out != nullptr && (next_w == nullptr || next_b == nullptr)) return -1;
     const size_t part_stride = (size_t)rows * width;
-    if (out == nullptr || out_dtype == KIPP_F32)
-        hipLaunchKernelGGL((sandwich_step_kernel<float>), dim3(rows), dim3(LN_THREADS), 0, stream, x, delta, parts, part_stride, post_w,
-                           post_b, post_eps, mult, extra, next_w, next_b, next_eps, (float*)out, width);
-    else if (out_dtype == KIPP_BF16)
-        hipLaunchKernelGGL((sandwich_step_kernel<bf16_t>), dim3(rows), dim3(LN_THREADS), 0, stream, x, delta, parts, part_stride, post_w,
-                           post_b, post_eps, mult, extra, next_w, next_b, next_eps, (bf16_t*)out, width);
-    else
+#define KIPP_SS(ITEMS)                                                                                                             \
+    hipLaunchKernelGGL((sandwich_step_kernel<KIPP_SS_TO, ITEMS>), dim3(rows), dim3(LN_THREADS), 0, stream, x, delta, parts, part_stride, \
+                       post_w, post_b, post_eps, mult, extra, next_w, next_b, next_eps, (KIPP_SS_TO*)out, width)
+    if (out == nullptr || out_dtype == KIPP_F32) {
+#define KIPP_SS_TO float
+        KIPP_LN_ITEMS(KIPP_SS);
+#undef KIPP_SS_TO
+    } else if (out_dtype == KIPP_BF16) {
+#define KIPP_SS_TO bf16_t
+        KIPP_LN_ITEMS(KIPP_SS);
+#undef KIPP_SS_TO
+    } else {
         return -2;
+    }
+#undef KIPP_SS
     return KIPP_LAUNCH_CHECK();
 }
