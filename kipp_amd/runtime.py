@@ -266,8 +266,33 @@ class Runtime:
 
     @staticmethod
     def _rows_class(m: int) -> int:
-        """Rows of a prompt product, in classes of a factor of two (193-256, 257-512, 513-1024, ...): one decision a class."""
+        """Rows of a prompt product, in classes of a factor of two (193-256, 257-512, 513-1024, ...): timed once a class."""
         return 1 << (max(m, 1) - 1).bit_length()
+
+    @staticmethod
+    def _rounds_of(name, m: int, cols: int, pairs: bool) -> float:
+        """What a way to compute a product costs at m rows, in units of its own: the rounds of its tiles over the 256 compute units (of
+        the library's: 256 rows at a time; of the planned way: of what the plan would take).  A class is timed at the first rows that come; the others' times
+        are taken in proportion to this.  (1,193 rows against [gate; up] of 2 x 12,288 x 4,096: whole rounds of 256 x 256 and the rest in
+        128 x 64 were level with one cut at the class's first 2,048 rows, three rounds and no rest; there 281 us against 231.)"""
+        if name == "plan":
+            if pairs and m >= 512:
+                return Runtime._rounds_of(2421, m, cols, pairs)
+            return min(Runtime._rounds_of(cut, m, cols, pairs) / (cut % 10) for cut in Runtime.TILE_CUTS_SLABS if cut < 1000 and not (pairs and cut % 10 > 1))
+        if name == "library":
+            return float(-(-m // 256))
+
+        def rounds(wm, wn, across, parts, width):
+            tiles = -(-m // (64 * wm)) * -(-width // ((16 if pairs else 32) * wn * across))
+            return -(-tiles * parts // 256) * (0.1 + 0.022 * wm * wn * across)       # times a tile's, from the measured steps
+        rest, code = divmod(name, 10000)
+        if code < 2000:
+            return rounds(code // 100 % 10, code // 10 % 10, 4 if code >= 1000 else 2, code % 10, cols)
+        wide, rows = (16 if pairs else 32) * 8, -(-m // 256)
+        first = rows * (cols // wide) // 256 * 256 // rows * wide
+        if not 0 < first < cols:
+            return rounds(4, 2, 4, 1, cols)
+        return rounds(4, 2, 4, 1, first) + rounds(*((2, 2, 4), (4, 2, 2), (2, 4, 2), (2, 2, 2))[rest], 1, cols - first)
 
     # Cuts of our kernel that are timed beside the planned one: 100 x (wave tile rows / 32) + 10 x (wave tile
     # columns / 32) + parts of K (+ 1000: workgroups of 8 waves, two a SIMD, on the same 256 x 256 tile; + 2000: those for
@@ -275,13 +300,13 @@ class Runtime:
     # plan's cost model is linear; the GPU under its power limit is not (a round that leaves compute units idle
     # clocks the others higher), so the plan is not always the fastest.  An output element is summed over K in
     # the same order whatever the tile, so cuts with the same parts of K give the same bits.
-    _choices_of_process: dict = {}
-    TILE_CUTS_SLABS = (441, 442, 444, 431, 432, 421, 422, 1421, 1422, 1424)
+    _choices_of_process: dict = {}      # what the engines of a process timed: (choice, rows, milliseconds of every way, the choice for other rows)
+    TILE_CUTS_SLABS = (441, 442, 444, 431, 432, 433, 421, 422, 423, 1421, 1422, 1423, 1424)
     TILE_CUTS_BF16 = (441, 421, 241, 1421, 2421, 32421)
 
-    def _fastest(self, key, ways: dict, same_bits, extra_ms=None):
-        """Which of several ways to compute one product is taken for the shape `key`: decided once, by timing
-        them on the operands at hand (three runs each after a first one).  `ways`: name -> callable, "library"
+    def _fastest(self, key, ways: dict, same_bits, m: int, cols: int, pairs: bool = False, extra_ms=None):
+        """Which of several ways to compute one product of `m` rows and `cols` output columns is taken for the shape `key`: timed once,
+        on the operands at hand (three runs each after a first one), and for other rows of the class by those times (`_rounds_of`).  `ways`: name -> callable, "library"
         and "plan" among them; `same_bits`: the names whose results are those of "plan" bit for bit;
         `extra_ms`: name -> milliseconds that a way costs its consumer beyond its own kernel (the slabs of a split
         product are read by the kernel that adds them).
@@ -292,46 +317,50 @@ class Runtime:
             # a step that is to be recorded keeps to our own kernels (the library's calls stay out of HIP graphs)
             key = key + ("for a graph",)
             ways = {name: run for name, run in ways.items() if name != "library"}
-        choice = self.prompt_product_choices.get(key)
-        if choice is None:
-            choice = self._choices_of_process.get((self.own_prompt_products, key))      # every engine of a process decides alike
-        if choice is not None:
+        timed = self._choices_of_process.get((self.own_prompt_products, key))      # every engine of a process decides alike
+        if timed is not None:
+            choice, rows, took, by_rows = timed
             self.prompt_product_choices[key] = choice
-        if choice is None:
-            if self.own_prompt_products is False:
-                choice = "library" if "library" in ways else "plan"
-            else:
-                # The chip is at its power limit while products follow each other, and a product that wins from
-                # a standing start need not win then: every candidate runs a few times first, then they are
-                # timed in turn, twice round, without a pause between them
-                runs = {}
-                for name, run in ways.items():
-                    if self.own_prompt_products != "auto" and name not in same_bits:
-                        continue
-                    try:
-                        for _ in range(3):
-                            run()
-                    except self.ops.KernelError:
-                        continue                      # a cut this shape does not take
-                    runs[name] = run
-                marks = []
-                for _ in range(2):
-                    for name, run in runs.items():
-                        begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-                        begin.record()
-                        for _ in range(4):
-                            run()
-                        end.record()
-                        marks.append((name, begin, end))
-                torch.cuda.current_stream().synchronize()
-                took = {}
-                for name, begin, end in marks:
-                    took[name] = took.get(name, 0.0) + begin.elapsed_time(end) / 4
-                for name in took:
-                    took[name] += 2 * (extra_ms or {}).get(name, 0.0)
-                choice = min(took, key=took.get) if took else "plan"
-            self.prompt_product_choices[key] = choice
-            self._choices_of_process[(self.own_prompt_products, key)] = choice
+            if m in by_rows:
+                return by_rows[m]
+            if took:        # (at most as many entries as the class has numbers of rows)
+                choice = min(took, key=lambda name: took[name] * self._rounds_of(name, m, cols, pairs) / self._rounds_of(name, rows, cols, pairs))
+            by_rows[m] = choice
+            return choice
+        took = {}
+        if self.own_prompt_products is False:
+            choice = "library" if "library" in ways else "plan"
+        else:
+            # The chip is at its power limit while products follow each other, and a product that wins from
+            # a standing start need not win then: every candidate runs a few times first, then they are
+            # timed in turn, twice round, without a pause between them
+            runs = {}
+            for name, run in ways.items():
+                if self.own_prompt_products != "auto" and name not in same_bits:
+                    continue
+                try:
+                    for _ in range(3):
+                        run()
+                except self.ops.KernelError:
+                    continue                      # a cut this shape does not take
+                runs[name] = run
+            marks = []
+            for _ in range(2):
+                for name, run in runs.items():
+                    begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+                    begin.record()
+                    for _ in range(4):
+                        run()
+                    end.record()
+                    marks.append((name, begin, end))
+            torch.cuda.current_stream().synchronize()
+            for name, begin, end in marks:
+                took[name] = took.get(name, 0.0) + begin.elapsed_time(end) / 4
+            for name in took:
+                took[name] += 2 * (extra_ms or {}).get(name, 0.0)
+            choice = min(took, key=took.get) if took else "plan"
+        self.prompt_product_choices[key] = choice
+        self._choices_of_process[(self.own_prompt_products, key)] = (choice, m, took, {m: choice})
         return choice
 
     def _library_product(self, x, w):
@@ -367,7 +396,8 @@ class Runtime:
         if self.ops.gemm_tiles_ok(m, k, rows.shape[0]):
             ways = {"library": library, "plan": ours}
             ways.update({cut: (lambda cut=cut: ours(cut)) for cut in self.TILE_CUTS_BF16})
-            choice = self._fastest(("gated" if plain else "glu", self._rows_class(m), rows.shape[0], k), ways, ("plan",) + self.TILE_CUTS_BF16)
+            choice = self._fastest(("gated" if plain else "glu", self._rows_class(m), rows.shape[0], k), ways, ("plan",) + self.TILE_CUTS_BF16,
+                                   m, rows.shape[0] // 2, pairs=True)
             if choice != "library":
                 self.tile_products += 1
                 return ours(0 if choice == "plan" else choice)
@@ -388,7 +418,7 @@ class Runtime:
         if self.ops.gemm_tiles_ok(m, k, rows.shape[0]):
             ways = {"library": library, "plan": ours}
             ways.update({cut: (lambda cut=cut: ours(cut)) for cut in self.TILE_CUTS_BF16})
-            choice = self._fastest(("relu2", self._rows_class(m), rows.shape[0], k), ways, ("plan",) + self.TILE_CUTS_BF16)
+            choice = self._fastest(("relu2", self._rows_class(m), rows.shape[0], k), ways, ("plan",) + self.TILE_CUTS_BF16, m, rows.shape[0])
             if choice != "library":
                 self.tile_products += 1
                 return ours(0 if choice == "plan" else choice)
@@ -452,7 +482,7 @@ class Runtime:
             # every slab beyond the first is read once more by the kernel that adds them (at about 5 TB/s)
             slab_ms = m * n * 4 / 5e12 * 1e3
             extra = {name: ((planned if name == "plan" else name % 10) - 1) * slab_ms for name in ways if name != "library"}
-            choice = self._fastest(("linear", self._rows_class(m), n, x.shape[1], most), ways, same, extra)
+            choice = self._fastest(("linear", self._rows_class(m), n, x.shape[1], most), ways, same, m, n, extra_ms=extra)
             if choice != "library":
                 self.tile_products += 1
                 return ours(0 if choice == "plan" else choice)

@@ -1,0 +1,41 @@
+"""How a prompt product is cut at rows that its class was not timed at: by the times of the rows it was timed at, in proportion to the rounds
+of tiles over the compute units."""
+import math
+
+import pytest
+
+from kipp_amd.runtime import Runtime
+
+
+@pytest.mark.parametrize("m", [193, 256, 257, 1193, 2048])
+@pytest.mark.parametrize("cols,pairs", [(12288, True), (4096, False), (100, False)])
+def test_rounds(m, cols, pairs):
+    half = 2 if pairs else 1
+    big = 0.1 + 0.022 * 32
+    tiles = math.ceil(m / 256) * math.ceil(cols * half / 256)
+    assert Runtime._rounds_of(441, m, cols, pairs) == pytest.approx(math.ceil(tiles / 256) * big)
+    assert Runtime._rounds_of(1423, m, cols, pairs) == pytest.approx(math.ceil(tiles * 3 / 256) * big)
+    assert Runtime._rounds_of("library", m, cols, pairs) == math.ceil(m / 256)
+    # whole rounds and a rest: as many columns in whole rounds as fit; one cut where there is none, or nothing left
+    if tiles <= 256 or tiles % 256 == 0:
+        assert Runtime._rounds_of(32421, m, cols, pairs) == pytest.approx(Runtime._rounds_of(1421, m, cols, pairs))
+    else:
+        rows = math.ceil(m / 256)
+        first = tiles // 256 * 256 // rows
+        rest = math.ceil(m / 128) * math.ceil((cols * half - first * 256) / 128)
+        assert Runtime._rounds_of(32421, m, cols, pairs) == pytest.approx(math.ceil(rows * first / 256) * big + math.ceil(rest / 256) * (0.1 + 0.022 * 8))
+
+
+def test_other_rows_take_the_times_in_proportion(monkeypatch):
+    rt = Runtime.__new__(Runtime)
+    rt.own_prompt_products, rt.for_a_graph, rt.prompt_product_choices = "auto", False, {}
+    took = {"library": 0.4, "plan": 0.36, 1421: 0.351, 32421: 0.350}
+    monkeypatch.setattr(Runtime, "_choices_of_process", {("auto", ("gated",)): (32421, 2048, took, {2048: 32421})})
+
+    def never():
+        raise AssertionError("nothing is run once a class has been timed")
+    ways = {name: never for name in took}
+    for _ in range(2):
+        assert rt._fastest(("gated",), ways, (), 2048, 12288, pairs=True) == 32421       # level there: what was measured
+        assert rt._fastest(("gated",), ways, (), 1193, 12288, pairs=True) == 1421        # two rounds of three, against one and four small ones
+    assert rt.prompt_product_choices == {("gated",): 32421}
