@@ -323,8 +323,10 @@ class Runtime:
             self.prompt_product_choices[key] = choice
             if m in by_rows:
                 return by_rows[m]
-            if took:        # (at most as many entries as the class has numbers of rows)
-                choice = min(took, key=lambda name: took[name] * self._rounds_of(name, m, cols, pairs) / self._rounds_of(name, rows, cols, pairs))
+            # (what gives the plan's bits at the rows it was timed at need not at others, where the plan may take other parts of K)
+            names = [name for name in took if self.own_prompt_products == "auto" or name in same_bits]
+            if names:       # (at most as many entries as the class has numbers of rows)
+                choice = min(names, key=lambda name: took[name] * self._rounds_of(name, m, cols, pairs) / self._rounds_of(name, rows, cols, pairs))
             by_rows[m] = choice
             return choice
         took = {}

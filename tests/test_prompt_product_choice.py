@@ -39,3 +39,13 @@ def test_other_rows_take_the_times_in_proportion(monkeypatch):
         assert rt._fastest(("gated",), ways, (), 2048, 12288, pairs=True) == 32421       # level there: what was measured
         assert rt._fastest(("gated",), ways, (), 1193, 12288, pairs=True) == 1421        # two rounds of three, against one and four small ones
     assert rt.prompt_product_choices == {("gated",): 32421}
+
+
+def test_own_products_keep_the_plans_bits_at_every_number_of_rows(monkeypatch):
+    """A cut that gives the plan's bits at the rows a class was timed at is not taken at rows where the plan takes other parts of K."""
+    rt = Runtime.__new__(Runtime)
+    rt.own_prompt_products, rt.for_a_graph, rt.prompt_product_choices = True, False, {}
+    took = {"plan": 0.4, 443: 0.1, 1423: 0.2}
+    monkeypatch.setattr(Runtime, "_choices_of_process", {(True, ("linear",)): (443, 2048, took, {2048: 443})})
+    assert rt._fastest(("linear",), {}, ("plan", 442, 1422), 1100, 4096) == "plan"
+    assert rt._fastest(("linear",), {}, ("plan", 443, 1423), 1101, 4096) == 443
