@@ -60,14 +60,102 @@ __device__ __forceinline__ float activate(float z, int act) {
     }
 }
 
+// What the sort of a step's pairs reads and leaves.  tiles: int32 [max_tiles][3] = (expert, first row, rows); rows 0 marks an unused tile.
+// `row_weight` (or null) receives every sorted row's weight.  Choices from `experts` on are identity experts: no row, place -1.
+struct Sort {
+    int pairs, experts, top;
+    int32_t *pair_token, *place_of_pair, *tiles;
+    int max_tiles, tile_rows;
+    float* row_weight;
+};
+
+// One workgroup sorts all pairs.
+__device__ __forceinline__ void sort_pairs(const Sort& sort, const int32_t* chosen, const float* weight) {
+    const int pairs = sort.pairs, experts = sort.experts, top = sort.top, max_tiles = sort.max_tiles, tile_rows = sort.tile_rows;
+    int32_t *pair_token = sort.pair_token, *place_of_pair = sort.place_of_pair, *tiles = sort.tiles;
+    float* row_weight = sort.row_weight;
+    __shared__ int count[MAX_EXPERTS];
+    __shared__ int first[MAX_EXPERTS + 1];
+    __shared__ int tile_first[MAX_EXPERTS + 1];
+    for (int e = threadIdx.x; e < experts; e += blockDim.x) count[e] = 0;
+    __syncthreads();
+    for (int p = threadIdx.x; p < pairs; p += blockDim.x) {
+        const int e = chosen[p];
+        if (e < experts) atomicAdd(&count[e], 1);
+    }
+    __syncthreads();
+    if (threadIdx.x < KIPP_WAVE) {          // where every expert's rows and tiles begin: running sums over 64 experts at a time
+        int rows = 0, tl = 0;
+        for (int e0 = 0; e0 < experts; e0 += KIPP_WAVE) {
+            const int e = e0 + threadIdx.x;
+            const int n = e < experts ? count[e] : 0, mine = (n + tile_rows - 1) / tile_rows;
+            int up_rows = n, up_tl = mine;
+            for (int off = 1; off < KIPP_WAVE; off <<= 1) {
+                const int r = __shfl_up(up_rows, off, KIPP_WAVE), t = __shfl_up(up_tl, off, KIPP_WAVE);
+                if ((int)threadIdx.x >= off) {
+                    up_rows += r;
+                    up_tl += t;
+                }
+            }
+            if (e < experts) {
+                first[e] = rows + up_rows - n;
+                tile_first[e] = tl + up_tl - mine;
+            }
+            rows += __shfl(up_rows, KIPP_WAVE - 1, KIPP_WAVE);
+            tl += __shfl(up_tl, KIPP_WAVE - 1, KIPP_WAVE);
+        }
+        if (threadIdx.x == 0) {
+            first[experts] = rows;
+            tile_first[experts] = tl;
+        }
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < experts; e += blockDim.x) {
+        const int n = count[e], parts = (n + tile_rows - 1) / tile_rows;
+        // whole tiles: an expert's rows shared out evenly, in what the waves' products take
+        const int grain = tile_rows == MANY_ROWS ? 64 : 32;     // of the products that read these tiles
+        const int each = tile_rows >= MFMA_ROWS && parts > 0 ? ((n + parts - 1) / parts + grain - 1) / grain * grain : tile_rows;
+        for (int j = 0; j < parts; ++j) {
+            int32_t* tile = tiles + (size_t)(tile_first[e] + j) * 3;
+            tile[0] = e;
+            tile[1] = first[e] + j * each;
+            tile[2] = min(each, n - j * each);
+        }
+    }
+    for (int i = tile_first[experts] + threadIdx.x; i < max_tiles; i += blockDim.x) {
+        tiles[(size_t)i * 3] = 0;
+        tiles[(size_t)i * 3 + 1] = 0;
+        tiles[(size_t)i * 3 + 2] = 0;
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < experts; e += blockDim.x) count[e] = 0;     // now the next free place of a run
+    __syncthreads();
+    for (int p = threadIdx.x; p < pairs; p += blockDim.x) {
+        const int e = chosen[p];
+        if (e >= experts) {
+            place_of_pair[p] = -1;
+            continue;
+        }
+        const int at = first[e] + atomicAdd(&count[e], 1);
+        pair_token[at] = p / top;
+        place_of_pair[p] = at;
+        if (row_weight != nullptr) row_weight[at] = weight[p];
+    }
+}
+
+__global__ void __launch_bounds__(1024) moe_sort_kernel(Sort sort, const int32_t* chosen, const float* weight) { sort_pairs(sort, chosen, weight); }
+
+// Few tokens (one workgroup's) are chosen for and sorted in one launch (`SORT`): at 1 token 7.5 + 5.6 us as two kernels, 9.86 as one.
+#define ROUTE_SORT_TOKENS 16        // a wave each
 // One wave a token, a lane REGS of the experts.  z: float32 [tokens][stride] (or slabs of it, added in order).
-template <int REGS>
-__global__ void __launch_bounds__(ROUTE_WAVES * KIPP_WAVE)
-moe_route_kernel(const float* __restrict__ z, int parts, size_t part_stride, int stride, int32_t* __restrict__ chosen,
-                 float* __restrict__ weight, int tokens, int experts, int top, float eps) {
+template <int REGS, int WAVES, bool SORT>
+__global__ void __launch_bounds__(WAVES * KIPP_WAVE)
+moe_route_kernel(const float* __restrict__ z, int parts, size_t part_stride, int stride, int32_t* chosen,
+                 float* weight, int tokens, int experts, int top, float eps, Sort sort) {
     const int wave = threadIdx.x / KIPP_WAVE, lane = threadIdx.x & (KIPP_WAVE - 1);
-    const int t = blockIdx.x * ROUTE_WAVES + wave;
-    if (t >= tokens) return;        // no barrier below
+    int t = blockIdx.x * WAVES + wave;
+    const bool live = t < tokens;
+    if (!live) t = tokens - 1;
     float p[REGS];
     float m = -INFINITY;
 #pragma unroll
@@ -110,23 +198,27 @@ moe_route_kernel(const float* __restrict__ z, int parts, size_t part_stride, int
         picked_sum += s;
         if (lane == j) { mine = s; mine_e = best_e; }
     }
-    if (lane < top) {
+    if (live && lane < top) {
         chosen[(size_t)t * top + lane] = mine_e;
         weight[(size_t)t * top + lane] = mine / (picked_sum + eps);
+    }
+    if (SORT) {
+        __syncthreads();
+        sort_pairs(sort, chosen, weight);
     }
 }
 
 // One wave a token: sigmoid scores (`softmax`: a softmax over all of them), a correction for the choice alone, groups of
 // neighbouring experts of which the best stay (by the sum of their two largest, or, `by_largest`, by their largest).
-template <int REGS>
-__global__ void __launch_bounds__(ROUTE_WAVES * KIPP_WAVE)
+template <int REGS, int WAVES, bool SORT>
+__global__ void __launch_bounds__(WAVES * KIPP_WAVE)
 moe_route_grouped_kernel(const float* __restrict__ z, int parts, size_t part_stride, int stride, const float* __restrict__ correction,
-                         int32_t* __restrict__ chosen, float* __restrict__ weight, int tokens, int experts, int top, float eps,
-                         int group_count, int group_keep, float scale, int renormalize, int softmax, int by_largest) {
-    __shared__ float c_s[ROUTE_WAVES][REGS * KIPP_WAVE];     // choice scores, then -inf for experts of groups that do not stay
-    __shared__ float g_s[ROUTE_WAVES][REGS * KIPP_WAVE];     // group scores, -inf once a group is taken
+                         int32_t* chosen, float* weight, int tokens, int experts, int top, float eps,
+                         int group_count, int group_keep, float scale, int renormalize, int softmax, int by_largest, Sort sort) {
+    __shared__ float c_s[WAVES][REGS * KIPP_WAVE];     // choice scores, then -inf for experts of groups that do not stay
+    __shared__ float g_s[WAVES][REGS * KIPP_WAVE];     // group scores, -inf once a group is taken
     const int wave = threadIdx.x / KIPP_WAVE, lane = threadIdx.x & (KIPP_WAVE - 1);
-    int t = blockIdx.x * ROUTE_WAVES + wave;
+    int t = blockIdx.x * WAVES + wave;
     const bool live = t < tokens;
     if (!live) t = tokens - 1;      // stay in step with the barriers
     const int size = experts / group_count;
@@ -234,66 +326,9 @@ moe_route_grouped_kernel(const float* __restrict__ z, int parts, size_t part_str
         chosen[(size_t)t * top + lane] = mine_e;
         weight[(size_t)t * top + lane] = renormalize ? mine / (picked_sum + eps) * scale : mine * scale;
     }
-}
-
-// One workgroup sorts all pairs.  tiles: int32 [max_tiles][3] = (expert, first row, rows); rows 0 marks an unused tile.
-// `row_weight` (or null) receives every sorted row's weight.  Choices from `experts` on are identity experts: no row, place -1.
-__global__ void __launch_bounds__(1024)
-moe_sort_kernel(const int32_t* __restrict__ chosen, int pairs, int experts, int top, int32_t* __restrict__ pair_token,
-                int32_t* __restrict__ place_of_pair, int32_t* __restrict__ tiles, int max_tiles, int tile_rows,
-                const float* __restrict__ weight, float* __restrict__ row_weight) {
-    __shared__ int count[MAX_EXPERTS];
-    __shared__ int first[MAX_EXPERTS + 1];
-    __shared__ int tile_first[MAX_EXPERTS + 1];
-    for (int e = threadIdx.x; e < experts; e += blockDim.x) count[e] = 0;
-    __syncthreads();
-    for (int p = threadIdx.x; p < pairs; p += blockDim.x) {
-        const int e = chosen[p];
-        if (e < experts) atomicAdd(&count[e], 1);
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int rows = 0, tl = 0;
-        for (int e = 0; e < experts; ++e) {
-            first[e] = rows;
-            tile_first[e] = tl;
-            rows += count[e];
-            tl += (count[e] + tile_rows - 1) / tile_rows;
-        }
-        first[experts] = rows;
-        tile_first[experts] = tl;
-    }
-    __syncthreads();
-    for (int e = threadIdx.x; e < experts; e += blockDim.x) {
-        const int n = count[e], parts = (n + tile_rows - 1) / tile_rows;
-        // whole tiles: an expert's rows shared out evenly, in what the waves' products take
-        const int grain = tile_rows == MANY_ROWS ? 64 : 32;     // of the products that read these tiles
-        const int each = tile_rows >= MFMA_ROWS && parts > 0 ? ((n + parts - 1) / parts + grain - 1) / grain * grain : tile_rows;
-        for (int j = 0; j < parts; ++j) {
-            int32_t* tile = tiles + (size_t)(tile_first[e] + j) * 3;
-            tile[0] = e;
-            tile[1] = first[e] + j * each;
-            tile[2] = min(each, n - j * each);
-        }
-    }
-    for (int i = tile_first[experts] + threadIdx.x; i < max_tiles; i += blockDim.x) {
-        tiles[(size_t)i * 3] = 0;
-        tiles[(size_t)i * 3 + 1] = 0;
-        tiles[(size_t)i * 3 + 2] = 0;
-    }
-    __syncthreads();
-    for (int e = threadIdx.x; e < experts; e += blockDim.x) count[e] = 0;     // now the next free place of a run
-    __syncthreads();
-    for (int p = threadIdx.x; p < pairs; p += blockDim.x) {
-        const int e = chosen[p];
-        if (e >= experts) {
-            place_of_pair[p] = -1;
-            continue;
-        }
-        const int at = first[e] + atomicAdd(&count[e], 1);
-        pair_token[at] = p / top;
-        place_of_pair[p] = at;
-        if (row_weight != nullptr) row_weight[at] = weight[p];
+    if (SORT) {
+        __syncthreads();
+        sort_pairs(sort, chosen, weight);
     }
 }
 
@@ -802,15 +837,21 @@ extern "C" int kipp_moe_route(const float* z, int parts, int stride, int32_t* ch
     const int pairs = tokens * top;
     if (tile_rows != TILE_ROWS && tile_rows != ROWS_TILE && tile_rows != MFMA_ROWS && tile_rows != MANY_ROWS) return -1;
     if (max_tiles < (pairs + tile_rows - 1) / tile_rows + (experts < pairs ? experts : pairs)) return -1;
-#define KIPP_RT(REGS)                                                                                                                  \
-    hipLaunchKernelGGL(moe_route_kernel<REGS>, dim3((tokens + ROUTE_WAVES - 1) / ROUTE_WAVES), dim3(ROUTE_WAVES * KIPP_WAVE), 0, stream, z, \
-                       parts, (size_t)tokens * stride, stride, chosen, weight, tokens, experts, top, eps)
-    if (experts <= KIPP_WAVE) KIPP_RT(1);
-    else if (experts <= 4 * KIPP_WAVE) KIPP_RT(4);
-    else KIPP_RT(MAX_EXPERTS / KIPP_WAVE);
+    const Sort sort = {pairs, experts, top, pair_token, place_of_pair, tiles, max_tiles, tile_rows, row_weight};
+#define KIPP_RT(REGS, WAVES, SORT)                                                                                                     \
+    hipLaunchKernelGGL((moe_route_kernel<REGS, WAVES, SORT>), dim3((tokens + WAVES - 1) / WAVES), dim3(WAVES * KIPP_WAVE), 0, stream, z, \
+                       parts, (size_t)tokens * stride, stride, chosen, weight, tokens, experts, top, eps, sort)
+    if (tokens <= ROUTE_SORT_TOKENS && experts <= 4 * KIPP_WAVE) {
+        if (tokens <= ROUTE_WAVES && experts <= KIPP_WAVE) KIPP_RT(1, ROUTE_WAVES, true);
+        else if (experts <= KIPP_WAVE) KIPP_RT(1, ROUTE_SORT_TOKENS, true);
+        else KIPP_RT(4, ROUTE_SORT_TOKENS, true);
+        return KIPP_LAUNCH_CHECK();
+    }
+    if (experts <= KIPP_WAVE) KIPP_RT(1, ROUTE_WAVES, false);
+    else if (experts <= 4 * KIPP_WAVE) KIPP_RT(4, ROUTE_WAVES, false);
+    else KIPP_RT(MAX_EXPERTS / KIPP_WAVE, ROUTE_WAVES, false);
 #undef KIPP_RT
-    hipLaunchKernelGGL(moe_sort_kernel, dim3(1), dim3(1024), 0, stream, (const int32_t*)chosen, pairs, experts, top, pair_token,
-                       place_of_pair, tiles, max_tiles, tile_rows, (const float*)weight, row_weight);
+    hipLaunchKernelGGL(moe_sort_kernel, dim3(1), dim3(1024), 0, stream, sort, (const int32_t*)chosen, (const float*)weight);
     return KIPP_LAUNCH_CHECK();
 }
 
@@ -829,16 +870,22 @@ extern "C" int kipp_moe_route_grouped(const float* z, int parts, int stride, con
     const int pairs = tokens * top, real = experts - identity;
     if (tile_rows != TILE_ROWS && tile_rows != ROWS_TILE && tile_rows != MFMA_ROWS && tile_rows != MANY_ROWS) return -1;
     if (max_tiles < (pairs + tile_rows - 1) / tile_rows + (real < pairs ? real : pairs)) return -1;
-#define KIPP_RG(REGS)                                                                                                                     \
-    hipLaunchKernelGGL(moe_route_grouped_kernel<REGS>, dim3((tokens + ROUTE_WAVES - 1) / ROUTE_WAVES), dim3(ROUTE_WAVES * KIPP_WAVE), 0, stream, \
+    const Sort sort = {pairs, real, top, pair_token, place_of_pair, tiles, max_tiles, tile_rows, row_weight};
+#define KIPP_RG(REGS, WAVES, SORT)                                                                                                     \
+    hipLaunchKernelGGL((moe_route_grouped_kernel<REGS, WAVES, SORT>), dim3((tokens + WAVES - 1) / WAVES), dim3(WAVES * KIPP_WAVE), 0, stream, \
                        z, parts, (size_t)tokens * stride, stride, correction, chosen, weight, tokens, experts, top, eps, group_count, group_keep, \
-                       scale, renormalize, softmax, by_largest)
-    if (experts <= KIPP_WAVE) KIPP_RG(1);
-    else if (experts <= 4 * KIPP_WAVE) KIPP_RG(4);
-    else KIPP_RG(MAX_EXPERTS / KIPP_WAVE);
+                       scale, renormalize, softmax, by_largest, sort)
+    if (tokens <= ROUTE_SORT_TOKENS && experts <= 4 * KIPP_WAVE) {
+        if (tokens <= ROUTE_WAVES && experts <= KIPP_WAVE) KIPP_RG(1, ROUTE_WAVES, true);
+        else if (experts <= KIPP_WAVE) KIPP_RG(1, ROUTE_SORT_TOKENS, true);
+        else KIPP_RG(4, ROUTE_SORT_TOKENS, true);
+        return KIPP_LAUNCH_CHECK();
+    }
+    if (experts <= KIPP_WAVE) KIPP_RG(1, ROUTE_WAVES, false);
+    else if (experts <= 4 * KIPP_WAVE) KIPP_RG(4, ROUTE_WAVES, false);
+    else KIPP_RG(MAX_EXPERTS / KIPP_WAVE, ROUTE_WAVES, false);
 #undef KIPP_RG
-    hipLaunchKernelGGL(moe_sort_kernel, dim3(1), dim3(1024), 0, stream, (const int32_t*)chosen, pairs, real, top, pair_token,
-                       place_of_pair, tiles, max_tiles, tile_rows, (const float*)weight, row_weight);
+    hipLaunchKernelGGL(moe_sort_kernel, dim3(1), dim3(1024), 0, stream, sort, (const int32_t*)chosen, (const float*)weight);
     return KIPP_LAUNCH_CHECK();
 }
 

@@ -77,3 +77,33 @@ def test_the_sort_shares_rows_out(tile_rows):
         assert 0 <= n <= tile_rows and np.all(expert_of_row[first:first + n] == e)
         covered[first:first + n] += 1
     assert np.all(covered == 1)
+
+
+@pytest.mark.parametrize("experts, tokens", [(5, 1), (64, 4), (64, 5), (65, 4), (200, 16), (200, 17), (257, 3)])
+def test_choice_and_sort_in_one_launch_and_in_two(experts, tokens):
+    """On both sides of the tokens and experts up to which one launch chooses and sorts: the choices of the written-out softmax, every
+    pair in a row of its expert's run, the runs in the order of the experts."""
+    import torch
+    from kipp_amd.csrc import ops
+    rng = np.random.default_rng(experts + tokens)
+    top = 4
+    z = rng.normal(size=(tokens, experts)).astype(np.float32)
+    new = lambda *shape: torch.full(shape, -7, dtype=torch.int32, device=DEV)  # noqa: E731
+    for grouped in (False, True):
+        chosen, weight, pair_token, place = new(tokens, top), torch.empty((tokens, top), device=DEV), new(tokens * top), new(tokens * top)
+        tiles = new(ops.moe_max_tiles(tokens, experts, top, 64), 3)
+        ops.moe_route(torch.tensor(z, device=DEV), experts, top, 1e-20, chosen, weight, pair_token, place, tiles, tile_rows=64,
+                      router="sigmoid" if grouped else "softmax")
+        picked = np.argsort(-z, axis=1, kind="stable")[:, :top]
+        assert np.array_equal(chosen.cpu().numpy(), picked)
+        s = np.take_along_axis(1 / (1 + np.exp(-z.astype(np.float64))) if grouped else np.exp(z.astype(np.float64)), picked, axis=1)
+        assert np.allclose(weight.cpu().numpy(), s / s.sum(axis=1, keepdims=True), rtol=1e-5)      # float32 exponentials, a few of them
+        at = place.cpu().numpy()
+        assert np.array_equal(np.sort(at), np.arange(tokens * top))
+        assert np.array_equal(pair_token.cpu().numpy()[at], np.arange(tokens * top) // top)
+        expert_of_row = np.empty(tokens * top, dtype=int)
+        expert_of_row[at] = picked.reshape(-1)
+        assert np.all(np.diff(expert_of_row) >= 0)
+        listed = tiles.cpu().numpy()
+        used = listed[listed[:, 2] > 0]
+        assert np.array_equal(np.repeat(used[:, 0], used[:, 2]), expert_of_row) and np.array_equal(np.cumsum(used[:, 2]) - used[:, 2], used[:, 1])
