@@ -927,10 +927,11 @@ static int launch_expert(const void* x, int x_dtype, const int32_t* gather, cons
         return KIPP_LAUNCH_CHECK();
     }
     if (tile_rows == MFMA_ROWS || tile_rows == MANY_ROWS) {
-        if (x_dtype != KIPP_BF16 || w_dtype != KIPP_BF16 || k % 32 || (((uintptr_t)x | (uintptr_t)w) & 15)) return -2;
-        // a lane's offsets into x and into an expert's matrix are 32 bits wide
-        if ((long long)max_tiles * tile_rows * k >= (1ll << 31) || (long long)(GLU ? 2 : 1) * n_out * k >= (1ll << 31)) return -2;
-        if (tile_rows == MFMA_ROWS && sorted_rows <= WALK_FROM * (long long)experts) {
+        if (x_dtype != KIPP_BF16 || w_dtype != KIPP_BF16 || k % 32) return -2;
+        // the walk brings 16 bytes a lane, from offsets into x and into an expert's matrix that are 32 bits wide
+        const bool walks = (((uintptr_t)x | (uintptr_t)w) & 15) == 0 && (long long)max_tiles * tile_rows * k < (1ll << 31) &&
+                           (long long)(GLU ? 2 : 1) * n_out * k < (1ll << 31);
+        if (tile_rows == MFMA_ROWS && (!walks || sorted_rows <= WALK_FROM * (long long)experts)) {
             const int cols = GLU ? MFMA_COLS / 2 : MFMA_COLS;
             dim3 grid(max_tiles, (n_out + cols - 1) / cols), block(MFMA_THREADS);
             if (out_dtype == KIPP_BF16)
@@ -943,6 +944,7 @@ static int launch_expert(const void* x, int x_dtype, const int32_t* gather, cons
                 return -2;
             return KIPP_LAUNCH_CHECK();
         }
+        if (!walks) return -2;
         if (out_dtype == KIPP_BF16)
             return tile_rows == MFMA_ROWS ? launch_tiles<bf16_t, GLU, 1, TILE_STAGES>(x, gather, row_weight, w, tiles, max_tiles, out, n_out, k, act, stream)
                                           : launch_tiles<bf16_t, GLU, 2, MANY_STAGES>(x, gather, row_weight, w, tiles, max_tiles, out, n_out, k, act, stream);

@@ -1039,8 +1039,8 @@ def moe_tile_rows(dtype: torch.dtype, *contractions: int, pairs: Optional[int] =
     if pairs is not None and pairs <= MOE_FEW_PAIRS * experts:
         return MOE_FEW_ROWS
     many = pairs is not None and pairs > (MOE_MANY_PAIRS if gated else MOE_MANY_PAIRS_UNGATED) * experts
-    # (a lane's offset into the rows is 32 bits wide, for as many rows as the tiles could hold)
-    if many and (-(-pairs // MOE_MANY_ROWS) + experts) * MOE_MANY_ROWS * max(contractions) < 1 << 31:
+    # (a lane's offsets into the rows, as many as the tiles could hold, and into an expert's matrix are 32 bits wide)
+    if many and (-(-pairs // MOE_MANY_ROWS) + experts) * MOE_MANY_ROWS * max(contractions) < 1 << 31 and 2 * max(contractions) * min(contractions) < 1 << 31:
         return MOE_MANY_ROWS
     return MOE_MFMA_ROWS
 

@@ -107,3 +107,21 @@ def test_choice_and_sort_in_one_launch_and_in_two(experts, tokens):
         listed = tiles.cpu().numpy()
         used = listed[listed[:, 2] > 0]
         assert np.array_equal(np.repeat(used[:, 0], used[:, 2]), expert_of_row) and np.array_equal(np.cumsum(used[:, 2]) - used[:, 2], used[:, 1])
+
+
+def test_operands_at_any_offset():
+    """Rows that begin at no multiple of 16 bytes take the staged kernel, whatever the rows an expert: as if they lay at one."""
+    import torch
+    from kipp_amd.csrc import ops
+    rng = np.random.default_rng(2)
+    rows, k, n_out = 120, 96, 64
+    flat = torch.tensor(rng.normal(size=rows * k + 8), dtype=torch.bfloat16, device=DEV)
+    w = torch.tensor(rng.normal(size=(1, n_out, k)), dtype=torch.bfloat16, device=DEV)
+    tiles = torch.tensor([[0, 0, rows]], dtype=torch.int32, device=DEV)
+    results = []
+    for x in (flat[2:2 + rows * k].view(rows, k), flat[2:2 + rows * k].view(rows, k).clone()):
+        results.append(ops.moe_expert(x, None, w, tiles, torch.empty((rows, n_out), device=DEV), tile_rows=128))
+    ref = flat[2:2 + rows * k].view(rows, k).double() @ w[0].double().T
+    size = flat[2:2 + rows * k].view(rows, k).double().abs() @ w[0].double().abs().T
+    for out in results:
+        assert bool(((out.double() - ref).abs() <= (k + 4) * 2.0 ** -24 * size).all())
