@@ -276,7 +276,7 @@ struct Filter {
 
 // A wave a head of q or k, or 64 channels of v (and, first of all, the gates); a token's waves are shared out over gridDim.y workgroups: one
 // for prompts, for single tokens as many as there are (one token, 32 heads in all, us: 12 workgroups 5.2, one 29; a prompt of 1,801 tokens 42 before the loads were asked for together, 28).
-// conv_w [channels][taps]; kept [slot][taps - 1][channels] at `kept_at` floats into the slot.  `single`: every entry brings one
+// conv_w [channels][taps]; kept [slot][taps - 1][channels] at `kept_at` floats into the slot.  `single`: no entry brings more than one
 // token, whose inputs go into the slot here.
 template <int TAPS>
 __global__ void __launch_bounds__(SCAN_THREADS)
@@ -341,10 +341,11 @@ __global__ void conv_keep_kernel(const float* __restrict__ proj, int stride, int
         if (i < taps - 1) kept[(size_t)i * channels + c] = vals[i];
 }
 
+// `single`: no entry brings more than one token.
 extern "C" int kipp_delta_prepare(const float* proj, int stride, const float* conv_w, int taps, const float* a_log, const float* dt_bias,
                                   float* state, size_t state_stride, size_t kept_at, const int32_t* seq_of_token, const int32_t* q_start,
                                   const int32_t* q_len, const int32_t* slots, float* prep, int prep_stride, int tokens, int entries,
-                                  int heads, int kv_heads, int d, int dv, int beta_col, int a_col, float unit_eps, hipStream_t stream) {
+                                  int heads, int kv_heads, int d, int dv, int beta_col, int a_col, float unit_eps, int single, hipStream_t stream) {
     if (tokens <= 0) return 0;
     const int channels = 2 * kv_heads * d + heads * dv;
     if (taps < 1 || taps > MAX_TAPS || heads <= 0 || kv_heads <= 0 || d <= 0 || dv <= 0) return -1;
@@ -352,7 +353,6 @@ extern "C" int kipp_delta_prepare(const float* proj, int stride, const float* co
     const int waves = SCAN_THREADS / KIPP_WAVE, units = 2 * kv_heads + (heads * dv + KIPP_WAVE - 1) / KIPP_WAVE;
     const int most = (units + waves - 1) / waves, fill = (2 * 256 + tokens - 1) / tokens;      // two workgroups a compute unit
     const dim3 grid(tokens, most < fill ? most : fill);
-    const int single = tokens == entries;
 #define KIPP_DP(TAPS)                                                                                                                  \
     hipLaunchKernelGGL(delta_prepare_kernel<TAPS>, grid, dim3(SCAN_THREADS), 0, stream, proj, stride, conv_w, taps, a_log, dt_bias, state,  \
                        state_stride, kept_at, seq_of_token, q_start, slots, prep, prep_stride, heads, kv_heads, d, dv, beta_col, a_col,   \
@@ -381,7 +381,7 @@ extern "C" int kipp_gated_scan(const float* prep, int stride, float* state, size
 // A thread a channel, for TOKENS tokens in a row.  proj: [z: inner | x: inner | B: groups n | C: groups n | dt: heads] (inner =
 // heads p); the channels x | B | C pass a causal filter (conv_w [channels][taps] with conv_b [channels], the slot's kept inputs
 // ahead of a portion; kept [taps - 1][channels] at `kept_at` floats into the slot) and silu.  prep as `kipp_gated_scan` reads it.
-// `single`: every entry brings one token, whose inputs go into the slot here.
+// `single`: no entry brings more than one token, whose inputs go into the slot here.
 template <int TOKENS, int TAPS>
 __global__ void __launch_bounds__(SCAN_THREADS)
 ssd_prepare_kernel(const float* __restrict__ proj, int stride, const float* __restrict__ conv_w, const float* __restrict__ conv_b, int taps,
@@ -430,17 +430,17 @@ ssd_prepare_kernel(const float* __restrict__ proj, int stride, const float* __re
     }
 }
 
+// `single`: no entry brings more than one token.
 extern "C" int kipp_ssd_prepare(const float* proj, int stride, const float* conv_w, const float* conv_b, int taps, const float* a_log,
                                 const float* dt_bias, float* state, size_t state_stride, size_t kept_at, const int32_t* seq_of_token,
                                 const int32_t* q_start, const int32_t* q_len, const int32_t* slots, float* prep, int prep_stride,
-                                int tokens, int entries, int heads, int groups, int n, int p, hipStream_t stream) {
+                                int tokens, int entries, int heads, int groups, int n, int p, int single, hipStream_t stream) {
     if (tokens <= 0) return 0;
     if (taps < 1 || taps > MAX_TAPS || heads <= 0 || heads > SSD_MAX_HEADS || groups <= 0 || heads % groups || n <= 0 || p <= 0) return -1;
     const int inner = heads * p, channels = inner + 2 * groups * n;
     if (stride < inner + channels + heads || prep_stride < 2 * groups * n + 2 * inner + heads ||
         state_stride < kept_at + (size_t)(taps - 1) * channels) return -1;
     const int cols = (channels + SCAN_THREADS - 1) / SCAN_THREADS;
-    const int single = tokens == entries;
 #define KIPP_SP(TOKENS, TAPS)                                                                                                         \
     hipLaunchKernelGGL((ssd_prepare_kernel<TOKENS, TAPS>), dim3((tokens + TOKENS - 1) / TOKENS, cols), dim3(SCAN_THREADS), 0, stream, proj, \
                        stride, conv_w, conv_b, taps, a_log, dt_bias, state, state_stride, kept_at, seq_of_token, q_start, slots, prep, \

@@ -781,12 +781,13 @@ def delta_state_size(heads: int, kv_heads: int, d: int, dv: int, taps: int) -> i
 
 def delta_prepare(proj: torch.Tensor, conv_w: torch.Tensor, a_log: torch.Tensor, dt_bias: torch.Tensor, state: torch.Tensor,
                   seq_of_token: torch.Tensor, q_start: torch.Tensor, q_len: torch.Tensor, slots: torch.Tensor, prep: torch.Tensor,
-                  heads: int, kv_heads: int, d: int, dv: int, beta_col: int, a_col: int, unit_eps: float) -> torch.Tensor:
+                  heads: int, kv_heads: int, d: int, dv: int, beta_col: int, a_col: int, unit_eps: float,
+                  longest: int = 0) -> torch.Tensor:
     """The gated delta rule's inputs from its input product `proj` (float32 [tokens, >= channels], columns q | k | v first,
     the beta and decay pre-activations at `beta_col` and `a_col`): `prep` [tokens, channels + 2 heads] receives q | k | v
     behind their short convolutions (`conv_w` [channels, taps], the slot's kept inputs in front of a portion) and silu, every
     q and k head a unit vector (q also over sqrt(d)), then beta = sigmoid and g = exp(-exp(a_log) softplus(. + dt_bias)) a
-    head.  The slot's kept inputs are then moved on by the portion."""
+    head.  The slot's kept inputs are then moved on by the portion (`longest` 1, no entry brings more than one token: in the same launch)."""
     _dev(proj, conv_w, a_log, dt_bias, state, seq_of_token, q_start, q_len, slots, prep)
     for t, name in ((seq_of_token, "seq_of_token"), (q_start, "q_start"), (q_len, "q_len"), (slots, "slots")):
         _i32(t, name)
@@ -800,10 +801,10 @@ def delta_prepare(proj: torch.Tensor, conv_w: torch.Tensor, a_log: torch.Tensor,
     _need(state.dim() == 2 and state.dtype == torch.float32 and state.shape[1] >= delta_state_size(heads, kv_heads, d, dv, taps), "delta_prepare: state is float32 [slots, size]")
     _need(q_start.numel() == q_len.numel() == slots.numel(), "delta_prepare: one start, length and slot an entry")
     fn = _fn("linear_scan", "kipp_delta_prepare", [_c_ptr, _c_int, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_size, _c_size, _c_ptr, _c_ptr, _c_ptr, _c_ptr,
-                                                   _c_ptr, _c_int] + [_c_int] * 8 + [_c_float, _c_ptr])
+                                                   _c_ptr, _c_int] + [_c_int] * 8 + [_c_float, _c_int, _c_ptr])
     _check(fn(_ptr(proj), proj.shape[1], _ptr(conv_w), taps, _ptr(a_log), _ptr(dt_bias), _ptr(state), state.shape[1], heads * d * dv,
               _ptr(seq_of_token), _ptr(q_start), _ptr(q_len), _ptr(slots), _ptr(prep), prep.shape[1], n, q_start.numel(), heads, kv_heads, d, dv,
-              int(beta_col), int(a_col), float(unit_eps), _stream()), "delta_prepare")
+              int(beta_col), int(a_col), float(unit_eps), int(longest == 1), _stream()), "delta_prepare")
     return prep
 
 
@@ -838,12 +839,12 @@ def ssd_prep_width(heads: int, groups: int, n: int, p: int) -> int:
 
 def ssd_prepare(proj: torch.Tensor, conv_w: torch.Tensor, conv_b: torch.Tensor, a_log: torch.Tensor, dt_bias: torch.Tensor,
                 state: torch.Tensor, seq_of_token: torch.Tensor, q_start: torch.Tensor, q_len: torch.Tensor, slots: torch.Tensor,
-                prep: torch.Tensor, heads: int, groups: int, n: int, p: int) -> torch.Tensor:
+                prep: torch.Tensor, heads: int, groups: int, n: int, p: int, longest: int = 0) -> torch.Tensor:
     """The state space recurrence's inputs from its input product `proj` (float32 [tokens, z | x | B | C | dt], z and x of
     heads p columns, B and C of groups n, dt of heads): x, B and C behind their short causal filter (`conv_w` [channels,
     taps], `conv_b` [channels], the slot's kept inputs ahead of a portion) and silu; dt = softplus(dt + dt_bias);
     `prep` [tokens, `ssd_prep_width`] receives C | B | dt x | x | g with g = exp(-exp(a_log) dt) a head.  The slot's kept
-    inputs are then moved on by the portion."""
+    inputs are then moved on by the portion (`longest` 1, no entry brings more than one token: in the same launch)."""
     _dev(proj, conv_w, conv_b, a_log, dt_bias, state, seq_of_token, q_start, q_len, slots, prep)
     for t, name in ((seq_of_token, "seq_of_token"), (q_start, "q_start"), (q_len, "q_len"), (slots, "slots")):
         _i32(t, name)
@@ -860,10 +861,10 @@ def ssd_prepare(proj: torch.Tensor, conv_w: torch.Tensor, conv_b: torch.Tensor, 
     _need(state.dim() == 2 and state.dtype == torch.float32 and state.shape[1] >= ssd_state_size(heads, groups, n, p, taps), "ssd_prepare: state is float32 [slots, size]")
     _need(q_start.numel() == q_len.numel() == slots.numel(), "ssd_prepare: one start, length and slot an entry")
     fn = _fn("linear_scan", "kipp_ssd_prepare", [_c_ptr, _c_int, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_size, _c_size, _c_ptr, _c_ptr, _c_ptr,
-                                                 _c_ptr, _c_ptr, _c_int] + [_c_int] * 6 + [_c_ptr])
+                                                 _c_ptr, _c_ptr, _c_int] + [_c_int] * 7 + [_c_ptr])
     _check(fn(_ptr(proj), proj.shape[1], _ptr(conv_w), _ptr(conv_b), taps, _ptr(a_log), _ptr(dt_bias), _ptr(state), state.shape[1], heads * n * p,
               _ptr(seq_of_token), _ptr(q_start), _ptr(q_len), _ptr(slots), _ptr(prep), prep.shape[1], tokens, q_start.numel(), heads, groups, n, p,
-              _stream()), "ssd_prepare")
+              int(longest == 1), _stream()), "ssd_prepare")
     return prep
 
 

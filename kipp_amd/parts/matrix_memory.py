@@ -153,7 +153,8 @@ class GatedDelta:
         proj = rt.linear(x, self.w_in)                    # float32 [n, q | k | v | gate | b | a]
         prep = rt.empty((n, channels + 2 * s.num_heads), torch.float32)
         ops.delta_prepare(proj, self.conv, self.a_log, self.dt_bias, state, batch.seq_of_token, batch.q_start, batch.q_len, batch.slots, prep,
-                          s.num_heads, s.num_kv_heads, s.head_dim, s.v_head_dim, channels + hv, channels + hv + s.num_heads, s.unit_eps)
+                          s.num_heads, s.num_kv_heads, s.head_dim, s.v_head_dim, channels + hv, channels + hv + s.num_heads, s.unit_eps,
+                          longest=batch.max_q_len)
         o_raw = rt.empty((n, hv), torch.float32)
         ops.delta_scan(prep, state, batch.q_start, batch.q_len, batch.slots, o_raw, s.num_heads, s.num_kv_heads, s.head_dim, s.v_head_dim, longest=batch.max_q_len,
                        chunks=rt.dtype == "bfloat16")
@@ -221,7 +222,7 @@ class SSD:
         proj = rt.linear(x, self.w_in)                    # float32 [n, z | u | B | C | dt]
         prep = rt.empty((n, ops.ssd_prep_width(s.num_heads, s.groups, s.state_size, s.head_dim)), torch.float32)
         ops.ssd_prepare(proj, self.conv, self.conv_b, self.a_log, self.dt_bias, state, batch.seq_of_token, batch.q_start, batch.q_len,
-                        batch.slots, prep, s.num_heads, s.groups, s.state_size, s.head_dim)
+                        batch.slots, prep, s.num_heads, s.groups, s.state_size, s.head_dim, longest=batch.max_q_len)
         o_raw = rt.empty((n, s.inner), torch.float32)
         ops.gated_scan(prep, state, batch.q_start, batch.q_len, batch.slots, o_raw, s.num_heads, s.groups, s.state_size, s.head_dim,
                        longest=batch.max_q_len, chunks=rt.dtype == "bfloat16")

@@ -30,17 +30,18 @@ def test_single_tokens_are_portions_of_one(taps, kind, heads, groups, d, dv):
     size = (ops.delta_state_size if kind == "delta" else ops.ssd_state_size)(heads, groups, d, dv, taps)
     kept = torch.tensor(rng.normal(size=(3, size)), dtype=torch.float32, device="cuda:0")
 
-    def run(state, first, lens, slots):
+    def run(state, first, lens, slots, longest=None):
         n = sum(lens)
         prep = torch.full((n, width), float("nan"), dtype=torch.float32, device="cuda:0")
         starts = [sum(lens[:i]) for i in range(len(lens))]
         seq = i32(*[e for e, m in enumerate(lens) for _ in range(m)])
         rows = proj[first:first + n].contiguous()
+        said = {} if longest == 0 else {"longest": longest or max(lens)}
         batch = (seq, i32(*starts), i32(*lens), i32(*slots))
         if kind == "delta":
-            ops.delta_prepare(rows, conv_w, a_log, dt_bias, state, *batch, prep, heads, groups, d, dv, channels, channels + heads, 1e-6)
+            ops.delta_prepare(rows, conv_w, a_log, dt_bias, state, *batch, prep, heads, groups, d, dv, channels, channels + heads, 1e-6, **said)
         else:
-            ops.ssd_prepare(rows, conv_w, conv_b, a_log, dt_bias, state, *batch, prep, heads, groups, d, dv)
+            ops.ssd_prepare(rows, conv_w, conv_b, a_log, dt_bias, state, *batch, prep, heads, groups, d, dv, **said)
         return prep
 
     one, many, both = kept.clone(), kept.clone(), kept.clone()
@@ -52,6 +53,9 @@ def test_single_tokens_are_portions_of_one(taps, kind, heads, groups, d, dv):
     pair = run(both, 0, [1, 1], [2, 0])                                          # two entries of one token each
     again = torch.cat([run(kept, 0, [1], [2]), run(kept, 1, [1], [0])])
     assert torch.equal(pair, again) and torch.equal(both, kept)
+    # an entry without a token beside one of two: as many tokens as entries, and nothing said of the longest
+    empty, plain = kept.clone(), kept.clone()
+    assert torch.equal(run(empty, 0, [2, 0], [1, 2], longest=0), run(plain, 0, [2], [1])) and torch.equal(empty, plain)
 
 
 # spans on both sides of what a thread's registers hold
