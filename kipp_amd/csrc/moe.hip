@@ -910,7 +910,7 @@ static int launch_tiles(const void* x, const int32_t* gather, const float* row_w
 template <bool GLU>
 static int launch_expert(const void* x, int x_dtype, const int32_t* gather, const float* row_weight, const void* w, int w_dtype,
                          const int32_t* tiles, int max_tiles, void* out, int out_dtype, int n_out, int k, int act, int tile_rows,
-                         int sorted_rows, int experts, hipStream_t stream) {
+                         int x_rows, int sorted_rows, int experts, hipStream_t stream) {
     if (max_tiles <= 0) return 0;
     if (n_out <= 0 || k <= 0 || act < ACT_NONE || act > ACT_RELU2) return -1;
     if (tile_rows == ROWS_TILE) {
@@ -928,9 +928,11 @@ static int launch_expert(const void* x, int x_dtype, const int32_t* gather, cons
     }
     if (tile_rows == MFMA_ROWS || tile_rows == MANY_ROWS) {
         if (x_dtype != KIPP_BF16 || w_dtype != KIPP_BF16 || k % 32) return -2;
-        // the walk brings 16 bytes a lane, from offsets into x and into an expert's matrix that are 32 bits wide
-        const bool walks = (((uintptr_t)x | (uintptr_t)w) & 15) == 0 && (long long)max_tiles * tile_rows * k < (1ll << 31) &&
-                           (long long)(GLU ? 2 : 1) * n_out * k < (1ll << 31);
+        // a lane's offsets into x and into an expert's matrix are 32 bits wide in either kernel: numbers in the staged one, bytes in the walk
+        if ((long long)max_tiles * tile_rows * k >= (1ll << 31) || (long long)(GLU ? 2 : 1) * n_out * k >= (1ll << 31) ||
+            (long long)x_rows * k >= (1ll << 32)) return -2;
+        // the walk brings 16 bytes a lane; rows of x that `gather` may name reach as far as x does
+        const bool walks = (((uintptr_t)x | (uintptr_t)w) & 15) == 0 && (long long)x_rows * k < (1ll << 31);
         if (tile_rows == MFMA_ROWS && (!walks || sorted_rows <= WALK_FROM * (long long)experts)) {
             const int cols = GLU ? MFMA_COLS / 2 : MFMA_COLS;
             dim3 grid(max_tiles, (n_out + cols - 1) / cols), block(MFMA_THREADS);
@@ -967,19 +969,19 @@ static int launch_expert(const void* x, int x_dtype, const int32_t* gather, cons
 }
 
 // `tile_rows`: the rows of the tiles that `kipp_moe_route` was asked for: 64, 128 and 256 take the matrix cores (bfloat16 x and w, K a
-// multiple of 32), 16 the plain kernel.  `sorted_rows` of `experts` experts in all: which kernel for whole tiles is the faster.
+// multiple of 32), 16 the plain kernel.  `x_rows`: rows that x has.  `sorted_rows` of `experts` experts in all: which kernel for whole tiles is the faster.
 extern "C" int kipp_moe_expert(const void* x, int x_dtype, const int32_t* gather, const void* w, int w_dtype, const int32_t* tiles,
-                               int max_tiles, void* out, int out_dtype, int n_out, int k, int act, int tile_rows, int sorted_rows, int experts,
-                               hipStream_t stream) {
-    return launch_expert<false>(x, x_dtype, gather, nullptr, w, w_dtype, tiles, max_tiles, out, out_dtype, n_out, k, act, tile_rows, sorted_rows,
+                               int max_tiles, void* out, int out_dtype, int n_out, int k, int act, int tile_rows, int x_rows, int sorted_rows,
+                               int experts, hipStream_t stream) {
+    return launch_expert<false>(x, x_dtype, gather, nullptr, w, w_dtype, tiles, max_tiles, out, out_dtype, n_out, k, act, tile_rows, x_rows, sorted_rows,
                                 experts, stream);
 }
 
 // The same against w [experts][2 n_out][k] = [gate; up] with a weight a sorted row (or null): out = act(s gate) * (s up).
 extern "C" int kipp_moe_expert_gated(const void* x, int x_dtype, const int32_t* gather, const float* row_weight, const void* w, int w_dtype,
                                      const int32_t* tiles, int max_tiles, void* out, int out_dtype, int n_out, int k, int act,
-                                     int tile_rows, int sorted_rows, int experts, hipStream_t stream) {
-    return launch_expert<true>(x, x_dtype, gather, row_weight, w, w_dtype, tiles, max_tiles, out, out_dtype, n_out, k, act, tile_rows, sorted_rows,
+                                     int tile_rows, int x_rows, int sorted_rows, int experts, hipStream_t stream) {
+    return launch_expert<true>(x, x_dtype, gather, row_weight, w, w_dtype, tiles, max_tiles, out, out_dtype, n_out, k, act, tile_rows, x_rows, sorted_rows,
                                experts, stream);
 }
 

@@ -1110,9 +1110,9 @@ def moe_expert(x: torch.Tensor, gather: Optional[torch.Tensor], w: torch.Tensor,
     _need(activation is None or activation in ACTIVATIONS, f"moe_expert: activation is one of {sorted(ACTIVATIONS)}")
     _need(tile_rows == MOE_TILE_ROWS or (tile_rows in (MOE_FEW_ROWS, MOE_MFMA_ROWS, MOE_MANY_ROWS) and x.dtype == torch.bfloat16 and w.shape[2] % 32 == 0),
           "moe_expert: tiles of 16 rows, or of 64, 128 or 256 for bfloat16 with K a multiple of 32")
-    fn = _fn("moe", "kipp_moe_expert", [_c_ptr, _c_int, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_int, _c_ptr] + [_c_int] * 7 + [_c_ptr])
+    fn = _fn("moe", "kipp_moe_expert", [_c_ptr, _c_int, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_int, _c_ptr] + [_c_int] * 8 + [_c_ptr])
     _check(fn(_ptr(x), _code(x), _ptr(gather), _ptr(w), _code(w), _ptr(tiles), tiles.shape[0], _ptr(out), _code(out), w.shape[1], w.shape[2],
-              -1 if activation is None else ACTIVATIONS[activation], int(tile_rows), out.shape[0], w.shape[0], _stream()), "moe_expert")
+              -1 if activation is None else ACTIVATIONS[activation], int(tile_rows), x.shape[0], out.shape[0], w.shape[0], _stream()), "moe_expert")
     return out
 
 
@@ -1133,9 +1133,9 @@ def moe_expert_gated(x: torch.Tensor, gather: Optional[torch.Tensor], row_weight
     _need(activation in ACTIVATIONS, f"moe_expert_gated: activation is one of {sorted(ACTIVATIONS)}")
     _need(tile_rows == MOE_TILE_ROWS or (tile_rows in (MOE_FEW_ROWS, MOE_MFMA_ROWS, MOE_MANY_ROWS) and x.dtype == torch.bfloat16 and w.shape[2] % 32 == 0),
           "moe_expert_gated: tiles of 16 rows, or of 64, 128 or 256 for bfloat16 with K a multiple of 32")
-    fn = _fn("moe", "kipp_moe_expert_gated", [_c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_int, _c_ptr] + [_c_int] * 7 + [_c_ptr])
+    fn = _fn("moe", "kipp_moe_expert_gated", [_c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_int, _c_ptr] + [_c_int] * 8 + [_c_ptr])
     _check(fn(_ptr(x), _code(x), _ptr(gather), _ptr(row_weight), _ptr(w), _code(w), _ptr(tiles), tiles.shape[0], _ptr(out), _code(out), inner, w.shape[2],
-              ACTIVATIONS[activation], int(tile_rows), out.shape[0], w.shape[0], _stream()), "moe_expert_gated")
+              ACTIVATIONS[activation], int(tile_rows), x.shape[0], out.shape[0], w.shape[0], _stream()), "moe_expert_gated")
     return out
 
 
