@@ -139,7 +139,7 @@ class MixedHeadAttention:
         Made by the first layer of a geometry and kept while the batch object lives: a recorded step keeps its own,
         made for the longest context of its class (the kernels take the true lengths from the device)."""
         s, ops = self.spec, self.rt.ops
-        key = ("mixed_attention_work", s.num_heads, s.v_head_dim, s.window, s.keep_first)
+        key = ("mixed_attention_work", s.num_heads, s.num_kv_heads, s.v_head_dim, s.window, s.keep_first)
         work = batch.host.get(key)
         if work is None:
             rows_tile, keys_tile = ops.MIXED_ROWS, ops.MIXED_KEYS

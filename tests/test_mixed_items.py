@@ -1,0 +1,32 @@
+"""What layers with mixed heads make of a step: which form takes which tokens, and the space that is made for it."""
+from types import SimpleNamespace
+
+import torch
+
+from kipp_amd.csrc import ops
+from kipp_amd.engine.batch import StepBatch
+from kipp_amd.parts.mixed_attention import MixedHeadAttention
+
+
+def batch_of(q_len, ctx_len):
+    starts = [sum(q_len[:i]) for i in range(len(q_len))]
+    single = [c for n, c in zip(q_len, ctx_len) if n == 1]
+    return StepBatch(sum(q_len), len(q_len), 0, torch.zeros(sum(q_len), dtype=torch.int32), *[None] * 7, {}, n_decode=len(single),
+                     n_portions=len(q_len) - len(single), max_decode_ctx=max(single, default=0), max_q_len=max(q_len),
+                     host={"q_start": starts, "q_len": q_len, "ctx_len": ctx_len})
+
+
+def layer_of(heads, kv_heads, window=None):
+    layer = MixedHeadAttention.__new__(MixedHeadAttention)
+    layer.spec = SimpleNamespace(num_heads=heads, num_kv_heads=kv_heads, v_head_dim=32, window=window, keep_first=0)
+    layer.rt = SimpleNamespace(ops=ops, device=torch.device("cpu"))
+    return layer
+
+
+def test_layers_of_other_groups_in_one_step():
+    """Query heads a key/value head decide whether single tokens take their own form: a layer's answer is not another's."""
+    for first, then in ((8, 1), (1, 8)):
+        batch = batch_of([1, 1, 1], [40, 300, 7])
+        for kv_heads in (first, then):
+            single, tiles = layer_of(32, kv_heads)._items(batch)
+            assert (single is not None) == (kv_heads == 8) and (tiles is not None) == (kv_heads == 1)
