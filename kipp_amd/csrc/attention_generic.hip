@@ -74,11 +74,11 @@ struct Merged {
 #pragma unroll
         for (int c = 0; c < C; ++c) acc[c] = 0.0f;
     }
-    // the scales of what is here and of the next block
+    // the scales of what is here and of the next block (a block whose scores are all -inf weighs nothing: mb = -inf, lb = 0)
     __device__ __forceinline__ void turn(float mb, float lb, float& a, float& b) {
         const float top = fmaxf(m, mb);
-        a = expf(m - top);
-        b = expf(mb - top);
+        a = m == top ? 1.0f : expf(m - top);
+        b = mb == top ? 1.0f : expf(mb - top);
         m = top;
         l = fmaf(l, a, __fmul_rn(lb, b));
     }
@@ -155,7 +155,7 @@ __global__ void __launch_bounds__(WAVES * KIPP_WAVE) paged_attention_generic_ker
 #pragma unroll
             for (int h = 0; h < HPW; ++h) {
                 mb[h] = wave_max(score[h]);
-                const float p = valid ? expf(score[h] - mb[h]) : 0.0f;
+                const float p = score[h] != -INFINITY ? expf(score[h] - mb[h]) : 0.0f;      // -inf: not seen, or of no weight
                 lb[h] = wave_sum(p);
                 p_w[lane * HPW + h] = p;
 #pragma unroll

@@ -94,3 +94,27 @@ def test_attention_of_a_token_alone_and_among_others(n_q, n_kv, d, dv, shared, p
             moved = 2 * d * EPS * scale * (np.abs(keys[lo:p + 1, g]) @ np.abs(q[i, h * d:(h + 1) * d])).max() + (p + 20) * EPS
             bound = 2 * moved * (p_ @ np.abs(values[lo:p + 1, g]))
             assert np.all(np.abs(every[i, h * dv:(h + 1) * dv] - p_ @ values[lo:p + 1, g]) <= bound + 1e-30), (p, h)
+
+
+@pytest.mark.parametrize("block", [0, 1, 3, 6])
+@pytest.mark.parametrize("tokens", [1, 300, 4200])
+def test_a_block_of_keys_whose_scores_overflow(block, tokens):
+    """64 keys of one block score -inf: they weigh nothing, wherever the block lies and however many waves share the keys."""
+    import torch
+    from kipp_amd.csrc import ops
+    rng = np.random.default_rng(block)
+    length, d, n_q, page = 450, 16, 2, 16
+    k, v = rng.normal(size=(length, d)).astype(np.float32), rng.normal(size=(length, d)).astype(np.float32)
+    q = rng.normal(size=(tokens, n_q, d)).astype(np.float32)
+    k[:, 0], q[:, :, 0] = 0.0, 2e38
+    k[64 * block:64 * (block + 1), 0] = -2e38
+    seen = np.arange(length) // 64 != block
+    cache = lambda a: torch.tensor(np.concatenate([a, np.zeros((-length % page, d), dtype=np.float32)]).reshape(-1, 1, page, d), device=DEV)  # noqa: E731
+    i32 = lambda a: torch.tensor(np.asarray(a), dtype=torch.int32, device=DEV)  # noqa: E731
+    out = ops.paged_attention_wide(torch.tensor(q.reshape(tokens, -1), device=DEV), cache(k), cache(v), torch.empty((tokens, n_q * d), device=DEV),
+                                   i32(np.full(tokens, length - 1)), i32(np.zeros(tokens)), i32(np.arange(-(-length // page)))[None], n_q, 1, d, d, 0.25)
+    s = q[:, :, 1:].astype(np.float64) @ k[seen, 1:].astype(np.float64).T * 0.25
+    p = np.exp(s - s.max(axis=-1, keepdims=True))
+    ref = p / p.sum(axis=-1, keepdims=True) @ v[seen].astype(np.float64)
+    # scores of size up to ~ 10, off by d float32 products; weights likewise, then `length` weighted values of size up to ~ 4
+    assert np.all(np.abs(out.cpu().numpy().reshape(ref.shape) - ref) <= (10 * d + length) * EPS * 4)
