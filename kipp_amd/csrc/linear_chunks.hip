@@ -27,6 +27,10 @@
 // A position's bits depend on its place in the chunk, so this is for activations that are rounded to bfloat16 behind it; the walk
 // token by token keeps the float32 path, where a portion gives the bits of single tokens.
 //
+// Entries of fewer than `from` tokens are left to that walk: a request's single token gives the same bits, and costs the same, whether
+// another request's prompt is in the step or not.  (128 single tokens beside a prompt of 64: a step of 7 layers, five of them with keys of
+// 128, takes 3,400 us; 4,010 with every entry through the chunks, 3,590 with every entry walked.)
+//
 // Rows beyond an entry's last token: g = 1, beta = 0, V = 0, and the last token's q and k in place of theirs.
 #include "common.h"
 #include <math.h>
@@ -52,8 +56,35 @@ __device__ __forceinline__ f32x4 mul16(f32x4 a, f32x4 b, f32x4 acc) {
 
 __device__ __forceinline__ f32x4 zero4() { return (f32x4){0.0f, 0.0f, 0.0f, 0.0f}; }
 
-// Chunks of an entry lie at `chunk_base` of it in the work space: entries before it have no more than that.
-__device__ __forceinline__ int chunk_base(int first, int entry) { return first / CHUNK + entry; }
+// The nth of the entries that bring `from` tokens or more (-1: there are fewer), and how many chunks those before it make:
+// its own lie behind them in the work space.  The same in every lane.
+struct Portion {
+    int entry, base;
+};
+__device__ __forceinline__ Portion portion_of(const int32_t* __restrict__ q_len, int entries, int from, int nth) {
+    Portion p = {-1, 0};
+    for (int e0 = 0; e0 < entries; e0 += KIPP_WAVE) {
+        const int lane = threadIdx.x & (KIPP_WAVE - 1);
+        const int n = e0 + lane < entries ? q_len[e0 + lane] : 0;
+        unsigned long long found = __ballot(n > 0 && n >= from);
+        const int here = __popcll(found);
+        int upto = KIPP_WAVE;
+        if (nth < here) {
+            for (int i = 0; i < nth; ++i) found &= found - 1;
+            upto = __ffsll((long long)found) - 1;
+        }
+        int chunks = lane < upto && n > 0 && n >= from ? (n + CHUNK - 1) / CHUNK : 0;
+#pragma unroll
+        for (int off = KIPP_WAVE / 2; off > 0; off >>= 1) chunks += __shfl_xor(chunks, off, KIPP_WAVE);
+        p.base += chunks;
+        if (nth < here) {
+            p.entry = e0 + upto;
+            return p;
+        }
+        nth -= here;
+    }
+    return p;
+}
 
 struct ChunkArgs {
     const float* q;             // row t, head hh: q + t * qk_stride + hh * d
@@ -67,7 +98,7 @@ struct ChunkArgs {
     const int32_t *q_start, *q_len, *slots;
     float* o_raw;
     float *a, *t, *vec;         // [chunk][head][64][64], the same (delta), [chunk][head][3][64]: G, D[last], beta
-    int heads, qk_rep, dv;
+    int heads, qk_rep, dv, entries, from;
 };
 
 __global__ void __launch_bounds__(THREADS)
@@ -86,13 +117,16 @@ __global__ void __launch_bounds__(THREADS) chunks_prepare_kernel(const ChunkArgs
     __shared__ float d_s[CHUNK][CHUNK + 1];
     __shared__ __attribute__((aligned(16))) float l_s[MODE == MODE_DELTA ? CHUNK : 1][UP];
     __shared__ float beta_s[CHUNK];
-    const int entry = blockIdx.z, head = blockIdx.y, chunk = blockIdx.x;
+    const int head = blockIdx.y, chunk = blockIdx.x;
+    const Portion portion = portion_of(p.q_len, p.entries, p.from, blockIdx.z);
+    if (portion.entry < 0) return;          // uniform over the workgroup, as below
+    const int entry = portion.entry;
     const int n = p.q_len[entry], first = p.q_start[entry];
-    if (chunk * CHUNK >= n) return;         // uniform over the workgroup
+    if (chunk * CHUNK >= n) return;
     const int m = min(CHUNK, n - chunk * CHUNK);
     const int t0 = first + chunk * CHUNK;
     const int tid = threadIdx.x, wave = tid / KIPP_WAVE, lane = tid & (KIPP_WAVE - 1), l16 = lane & 15, h4 = 4 * (lane >> 4);
-    const size_t at = (size_t)(chunk_base(first, entry) + chunk) * p.heads + head;
+    const size_t at = (size_t)(portion.base + chunk) * p.heads + head;
     float* a_out = p.a + at * CHUNK * CHUNK;
     float* vec = p.vec + at * 3 * CHUNK;
     if (wave == 0) {
@@ -185,7 +219,10 @@ __global__ void __launch_bounds__(THREADS) chunks_walk_kernel(const ChunkArgs p)
     __shared__ __attribute__((aligned(16))) float s_s[COLS * SP];           // [column][row]
     __shared__ __attribute__((aligned(16))) float u_s[COLS * UP];           // [column][token]
     __shared__ __attribute__((aligned(16))) float r_s[MODE == MODE_DELTA ? COLS * UP : 4];
-    const int entry = blockIdx.z, head = blockIdx.y;
+    const int head = blockIdx.y;
+    const Portion portion = portion_of(p.q_len, p.entries, p.from, blockIdx.z);
+    if (portion.entry < 0) return;          // uniform over the workgroup
+    const int entry = portion.entry;
     const int tid = threadIdx.x, wave = tid / KIPP_WAVE, lane = tid & (KIPP_WAVE - 1), l16 = lane & 15, h4 = 4 * (lane >> 4);
     const int n = p.q_len[entry], first = p.q_start[entry];
     const int col = blockIdx.x * COLS + l16;
@@ -216,7 +253,7 @@ __global__ void __launch_bounds__(THREADS) chunks_walk_kernel(const ChunkArgs p)
     };
     auto rest_of = [&](int c) {
         const int m = min(CHUNK, n - c * CHUNK), t0 = first + c * CHUNK;
-        const size_t at = (size_t)(chunk_base(first, entry) + c) * p.heads + head;
+        const size_t at = (size_t)(portion.base + c) * p.heads + head;
         const float* vec = p.vec + at * 3 * CHUNK;
         if (own < m) {
             const float* a_row = p.a + at * CHUNK * CHUNK + (own + l16) * CHUNK + h4;
@@ -317,29 +354,31 @@ __global__ void __launch_bounds__(THREADS) chunks_walk_kernel(const ChunkArgs p)
 
 extern "C" {
 
-// Chunks that `tokens` tokens of `entries` entries make, whatever their lengths.
-static long long chunk_count(int tokens, int entries) { return (long long)tokens / CHUNK + entries + 1; }
+// Chunks that `tokens` tokens of `portions` entries make at most, whatever their lengths.
+static long long chunk_count(int tokens, int portions) { return (long long)tokens / CHUNK + portions; }
 
 // Floats of work space, or 0 where this kernel does not take the sizes: keys of 64, 128, 192 or 256 numbers.
-long long kipp_matrix_chunks_work(int mode, int tokens, int entries, int heads, int d) {
-    if (mode < MODE_DECAY || mode > MODE_GATED || tokens <= 0 || entries <= 0 || heads <= 0 || d <= 0 || d % 64 || d > 256) return 0;
+long long kipp_matrix_chunks_work(int mode, int tokens, int portions, int heads, int d) {
+    if (mode < MODE_DECAY || mode > MODE_GATED || tokens <= 0 || portions <= 0 || heads <= 0 || d <= 0 || d % 64 || d > 256) return 0;
     const long long each = (mode == MODE_DELTA ? 2 : 1) * CHUNK * CHUNK + 3 * CHUNK;
-    return chunk_count(tokens, entries) * heads * each + (mode == MODE_DECAY ? (long long)tokens * 2 * heads * d : 0);
+    return chunk_count(tokens, portions) * heads * each + (mode == MODE_DECAY ? (long long)tokens * 2 * heads * d : 0);
 }
 
 // src: float32 [tokens][stride] with q, k, v (and beta, g) at the given columns, as `kipp_decay_scan`, `kipp_delta_scan` and `kipp_gated_scan` read it
-// (mode 0, 1, 2); q and k of a head at q_at + (head / qk_rep) d.  `longest`: the most tokens an entry brings.
+// (mode 0, 1, 2); q and k of a head at q_at + (head / qk_rep) d.  Of the entries only those of `from` tokens and more, at most `portions` of
+// them; `longest`: the most tokens an entry brings.
 int kipp_matrix_chunks(int mode, const float* src, int stride, int q_at, int k_at, int v_at, int beta_at, int g_at, const float* decays,
                        float* state, size_t state_stride, const int32_t* q_start, const int32_t* q_len, const int32_t* slots, float* o_raw,
-                       int tokens, int entries, int heads, int qk_rep, int d, int dv, int longest, float* work, long long work_floats,
+                       int tokens, int entries, int heads, int qk_rep, int d, int dv, int longest, int from, int portions, float* work,
+                       long long work_floats,
                        hipStream_t stream) {
-    if (entries <= 0 || tokens <= 0) return 0;
-    const long long need = kipp_matrix_chunks_work(mode, tokens, entries, heads, d);
+    if (entries <= 0 || tokens <= 0 || portions <= 0) return 0;
+    const long long need = kipp_matrix_chunks_work(mode, tokens, portions, heads, d);
     if (need == 0 || work_floats < need || longest <= 0 || qk_rep <= 0 || heads % qk_rep || dv <= 0) return -1;
     if (state_stride < (size_t)heads * d * dv || (state_stride & 3) || (stride & 3) || (q_at & 3) || (k_at & 3)) return -1;
     if (((uintptr_t)src | (uintptr_t)state | (uintptr_t)work) & 15) return -1;
     ChunkArgs p;
-    const long long slots_all = chunk_count(tokens, entries) * heads;
+    const long long slots_all = chunk_count(tokens, portions) * heads;
     p.a = work;
     p.t = mode == MODE_DELTA ? p.a + slots_all * CHUNK * CHUNK : p.a;
     p.vec = p.t + slots_all * CHUNK * CHUNK;
@@ -370,7 +409,9 @@ int kipp_matrix_chunks(int mode, const float* src, int stride, int q_at, int k_a
     p.heads = heads;
     p.qk_rep = qk_rep;
     p.dv = dv;
-    const dim3 prepare((longest + CHUNK - 1) / CHUNK, heads, entries), walk((dv + COLS - 1) / COLS, heads, entries), block(THREADS);
+    p.entries = entries;
+    p.from = from;
+    const dim3 prepare((longest + CHUNK - 1) / CHUNK, heads, portions), walk((dv + COLS - 1) / COLS, heads, portions), block(THREADS);
 #define KIPP_CHUNKS(MODE, DT)                                                              \
     do {                                                                                   \
         hipLaunchKernelGGL((chunks_prepare_kernel<MODE, DT>), prepare, block, 0, stream, p); \

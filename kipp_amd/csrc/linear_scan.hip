@@ -74,7 +74,7 @@ __global__ void __launch_bounds__(SCAN_THREADS)
 matrix_scan_kernel(const float* __restrict__ src, int stride, int q_at, int k_at, int v_at, int beta_at, int g_at,
                    const float* __restrict__ decays, float* __restrict__ state, size_t state_stride,
                    const int32_t* __restrict__ q_start, const int32_t* __restrict__ q_len, const int32_t* __restrict__ slots,
-                   float* __restrict__ o_raw, int heads, int qk_rep, int d, int dv, int chunk) {
+                   float* __restrict__ o_raw, int heads, int qk_rep, int d, int dv, int chunk, int below) {
     extern __shared__ __attribute__((aligned(16))) float lds[];
     constexpr int COLS = SCAN_THREADS / LANES;
     constexpr int DP = R * LANES;           // a key's numbers in LDS, filled up with zeros
@@ -89,6 +89,7 @@ matrix_scan_kernel(const float* __restrict__ src, int stride, int q_at, int k_at
     const bool live = col < dv;
     const int qk_head = head / qk_rep;
     const int first = q_start[entry], n = q_len[entry];
+    if (below > 0 && n >= below) return;    // uniform over the workgroup: another kernel's entry
     float* S_col = state + (size_t)slots[entry] * state_stride + ((size_t)head * dv + (live ? col : 0)) * d;
 
     // a lane's rows lie together: 16 bytes at a time where every column begins at a multiple of 16 bytes
@@ -195,16 +196,16 @@ static bool scan_shape(int d, int longest, int* lanes, int* rows, int* chunk) {
 template <int MODE>
 static int launch_scan(const float* src, int stride, int q_at, int k_at, int v_at, int beta_at, int g_at, const float* decays,
                        float* state, size_t state_stride, const int32_t* q_start, const int32_t* q_len, const int32_t* slots,
-                       float* o_raw, int entries, int heads, int qk_rep, int d, int dv, int longest, hipStream_t stream) {
+                       float* o_raw, int entries, int heads, int qk_rep, int d, int dv, int longest, int below, hipStream_t stream) {
     int lanes, rows, chunk;
-    if (!scan_shape(d, longest, &lanes, &rows, &chunk) || heads <= 0 || dv <= 0 || qk_rep <= 0 || heads % qk_rep) return -1;
+    if (!scan_shape(d, below > 0 && (longest <= 0 || longest >= below) ? below - 1 : longest, &lanes, &rows, &chunk) || heads <= 0 || dv <= 0 || qk_rep <= 0 || heads % qk_rep) return -1;
     if (state_stride < (size_t)heads * d * dv) return -1;
     const int cols = SCAN_THREADS / lanes;
     dim3 grid((dv + cols - 1) / cols, heads, entries), block(SCAN_THREADS);
     const size_t lds = ((size_t)2 * chunk * lanes * rows + (size_t)chunk * cols + 2 * chunk) * sizeof(float);
 #define KIPP_SCAN(R, L)                                                                                                        \
     hipLaunchKernelGGL((matrix_scan_kernel<MODE, R, L>), grid, block, lds, stream, src, stride, q_at, k_at, v_at, beta_at, g_at, \
-                       decays, state, state_stride, q_start, q_len, slots, o_raw, heads, qk_rep, d, dv, chunk)
+                       decays, state, state_stride, q_start, q_len, slots, o_raw, heads, qk_rep, d, dv, chunk, below)
     if (rows == 16) KIPP_SCAN(16, 64);
     else if (lanes == 1) KIPP_SCAN(8, 1);
     else if (lanes == 2) KIPP_SCAN(8, 2);
@@ -218,25 +219,26 @@ static int launch_scan(const float* src, int stride, int q_at, int k_at, int v_a
 }
 
 // proj: float32 [tokens][stride], columns q [heads d] | k [heads d] | v [heads dv] | ... before their silu.
-// `longest`: the most tokens an entry brings, if the host knows (0: it does not); it only sizes the chunks.
+// `longest`: the most tokens an entry brings, if the host knows (0: it does not); it only sizes the chunks.  `below`: entries of so many
+// tokens and more are left alone (0: none is).
 extern "C" int kipp_decay_scan(const float* proj, int stride, const float* decays, float* state, size_t state_stride,
                                const int32_t* q_start, const int32_t* q_len, const int32_t* slots, float* o_raw, int entries,
-                               int heads, int d, int dv, int longest, hipStream_t stream) {
+                               int heads, int d, int dv, int longest, int below, hipStream_t stream) {
     if (entries <= 0) return 0;
     if (stride < 2 * heads * d + heads * dv) return -1;
     return launch_scan<0>(proj, stride, 0, heads * d, 2 * heads * d, 0, 0, decays, state, state_stride, q_start, q_len, slots, o_raw,
-                          entries, heads, 1, d, dv, longest, stream);
+                          entries, heads, 1, d, dv, longest, below, stream);
 }
 
 // prep: float32 [tokens][stride], columns q [kv_heads d] | k [kv_heads d] | v [heads dv] | beta [heads] | g [heads], ready.
 extern "C" int kipp_delta_scan(const float* prep, int stride, float* state, size_t state_stride, const int32_t* q_start,
                                const int32_t* q_len, const int32_t* slots, float* o_raw, int entries, int heads, int kv_heads,
-                               int d, int dv, int longest, hipStream_t stream) {
+                               int d, int dv, int longest, int below, hipStream_t stream) {
     if (entries <= 0) return 0;
     if (kv_heads <= 0 || heads % kv_heads || stride < 2 * kv_heads * d + heads * dv + 2 * heads) return -1;
     const int c = 2 * kv_heads * d + heads * dv;
     return launch_scan<1>(prep, stride, 0, kv_heads * d, 2 * kv_heads * d, c, c + heads, nullptr, state, state_stride, q_start, q_len,
-                          slots, o_raw, entries, heads, heads / kv_heads, d, dv, longest, stream);
+                          slots, o_raw, entries, heads, heads / kv_heads, d, dv, longest, below, stream);
 }
 
 // The causal filter of one channel at token t: in[j] = its input `taps - 1 - j` tokens back (column `col` of proj; ahead of the portion,
@@ -369,11 +371,11 @@ extern "C" int kipp_delta_prepare(const float* proj, int stride, const float* co
 // prep: float32 [tokens][stride], columns q = C [groups n] | k = B [groups n] | v = dt x [heads p] | x [heads p] | g [heads], ready.
 extern "C" int kipp_gated_scan(const float* prep, int stride, float* state, size_t state_stride, const int32_t* q_start,
                                const int32_t* q_len, const int32_t* slots, float* o_raw, int entries, int heads, int groups,
-                               int n, int p, int longest, hipStream_t stream) {
+                               int n, int p, int longest, int below, hipStream_t stream) {
     if (entries <= 0) return 0;
     if (groups <= 0 || heads % groups || stride < 2 * groups * n + 2 * heads * p + heads) return -1;
     return launch_scan<2>(prep, stride, 0, groups * n, 2 * groups * n, 0, 2 * groups * n + 2 * heads * p, nullptr, state, state_stride,
-                          q_start, q_len, slots, o_raw, entries, heads, heads / groups, n, p, longest, stream);
+                          q_start, q_len, slots, o_raw, entries, heads, heads / groups, n, p, longest, below, stream);
 }
 
 #define SSD_MAX_HEADS 1024

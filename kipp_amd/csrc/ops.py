@@ -727,8 +727,8 @@ def _scan_args(state, q_start, q_len, slots, o_raw, tokens, heads, d, dv, what):
     _need(q_start.numel() == q_len.numel() == slots.numel(), f"{what}: one start, length and slot an entry")
 
 
-# Entries of so many tokens and more go through a matrix memory a chunk of 64 at a time (`chunks` below).  A chunk costs
-# about what the walk takes for a dozen tokens, whether it is full or not.
+# Entries of so many tokens and more go through a matrix memory a chunk of 64 at a time (`chunks` below), each for itself: the
+# others of the launch walk.  A chunk costs about what the walk takes for a dozen tokens, whether it is full or not.
 CHUNKS_FROM = 16
 
 
@@ -737,39 +737,49 @@ def matrix_chunks_ok(d: int) -> bool:
     return d % 64 == 0 and 0 < d <= 256
 
 
-def _matrix_chunks(mode, src, q_at, k_at, v_at, beta_at, g_at, decays, state, q_start, q_len, slots, o_raw, heads, qk_rep, d, dv, longest) -> bool:
-    """The scan by chunks where it takes the sizes (False: it does not, nothing was launched)."""
+def _matrix_chunks(mode, src, q_at, k_at, v_at, beta_at, g_at, decays, state, q_start, q_len, slots, o_raw, heads, qk_rep, d, dv, longest,
+                   portions) -> int:
+    """The scan by chunks, for the entries of `CHUNKS_FROM` tokens and more, where it takes the sizes.  Returns the tokens below which
+    entries are left for the walk: 0, it took none; -1, there are no others."""
     if longest < CHUNKS_FROM or not matrix_chunks_ok(d) or src.shape[1] % 4 or q_at % 4 or k_at % 4 or state.shape[1] % 4 \
             or src.data_ptr() % 16 or state.data_ptr() % 16 or src.shape[0] == 0:
-        return False
+        return 0
     tokens, entries = src.shape[0], q_start.numel()
-    size = _fn("linear_chunks", "kipp_matrix_chunks_work", [_c_int] * 5, restype=ctypes.c_longlong)(mode, tokens, entries, heads, d)
+    every = portions is not None and portions >= entries
+    portions = min(entries if portions is None else int(portions), entries, tokens // CHUNKS_FROM)
+    if portions <= 0:
+        return 0
+    size = _fn("linear_chunks", "kipp_matrix_chunks_work", [_c_int] * 5, restype=ctypes.c_longlong)(mode, tokens, portions, heads, d)
     _need(size > 0, "matrix_chunks: sizes the kernel refuses")
     work = torch.empty(size, dtype=torch.float32, device=src.device)
-    fn = _fn("linear_chunks", "kipp_matrix_chunks", [_c_int, _c_ptr] + [_c_int] * 6 + [_c_ptr, _c_ptr, _c_size] + [_c_ptr] * 4 + [_c_int] * 7
+    fn = _fn("linear_chunks", "kipp_matrix_chunks", [_c_int, _c_ptr] + [_c_int] * 6 + [_c_ptr, _c_ptr, _c_size] + [_c_ptr] * 4 + [_c_int] * 9
              + [_c_ptr, ctypes.c_longlong, _c_ptr])
     _check(fn(mode, _ptr(src), src.shape[1], q_at, k_at, v_at, beta_at, g_at, _ptr(decays), _ptr(state), state.shape[1], _ptr(q_start), _ptr(q_len),
-              _ptr(slots), _ptr(o_raw), tokens, entries, heads, qk_rep, d, dv, int(longest), _ptr(work), size, _stream()), "matrix_chunks")
-    return True
+              _ptr(slots), _ptr(o_raw), tokens, entries, heads, qk_rep, d, dv, int(longest), CHUNKS_FROM, portions, _ptr(work), size, _stream()), "matrix_chunks")
+    return -1 if every else CHUNKS_FROM
 
 
 def decay_scan(proj: torch.Tensor, decays: torch.Tensor, state: torch.Tensor, q_start: torch.Tensor, q_len: torch.Tensor,
-               slots: torch.Tensor, o_raw: torch.Tensor, heads: int, d: int, dv: int, longest: int = 0, chunks: bool = False) -> torch.Tensor:
+               slots: torch.Tensor, o_raw: torch.Tensor, heads: int, d: int, dv: int, longest: int = 0, chunks: bool = False,
+               portions: Optional[int] = None) -> torch.Tensor:
     """Linear attention with a fixed decay a head over every entry's tokens, in order, from and into the entry's slot of
     `state` [slots, size] (float32, S as [head][column][row]).  `proj`: float32 [tokens, >= 2 heads d + heads dv], columns
     q | k | v before their silu; `o_raw` float32 [tokens, heads dv] receives S^T q.  `longest`: the most tokens an entry
-    brings, if known (it sizes the kernel's chunks and changes no result).  `chunks`: entries (which lie one after the other) of many
-    tokens may be taken 64 tokens at a time on the matrix cores, the same float32 sums in another order: a token's last bits
-    then depend on its place in the portion."""
+    brings, if known (it sizes the kernel's chunks and changes no result).  `chunks`: entries of `CHUNKS_FROM` tokens and more
+    may be taken 64 tokens at a time on the matrix cores, the same float32 sums in another order: a token's last bits then depend on
+    its place in its own entry, and on nothing else in the step (for that `longest` must be known).  `portions`: how many entries bring
+    so many tokens, if known."""
     _dev(proj, decays, state, q_start, q_len, slots, o_raw)
     _need(proj.dim() == 2 and proj.dtype == torch.float32 and proj.shape[1] >= 2 * heads * d + heads * dv, "decay_scan: proj is float32 [tokens, q | k | v ...]")
     _need(decays.dtype == torch.float32 and decays.numel() == heads, "decay_scan: float32 decays [heads]")
     _scan_args(state, q_start, q_len, slots, o_raw, proj.shape[0], heads, d, dv, "decay_scan")
-    if chunks and _matrix_chunks(0, proj, 0, heads * d, 2 * heads * d, 0, 0, decays, state, q_start, q_len, slots, o_raw, heads, 1, d, dv, longest):
+    below = _matrix_chunks(0, proj, 0, heads * d, 2 * heads * d, 0, 0, decays, state, q_start, q_len, slots, o_raw, heads, 1, d, dv, longest,
+                           portions) if chunks else 0
+    if below < 0:
         return o_raw
-    fn = _fn("linear_scan", "kipp_decay_scan", [_c_ptr, _c_int, _c_ptr, _c_ptr, _c_size, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr])
+    fn = _fn("linear_scan", "kipp_decay_scan", [_c_ptr, _c_int, _c_ptr, _c_ptr, _c_size, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr])
     _check(fn(_ptr(proj), proj.shape[1], _ptr(decays), _ptr(state), state.shape[1], _ptr(q_start), _ptr(q_len), _ptr(slots), _ptr(o_raw),
-              q_start.numel(), heads, d, dv, max(0, int(longest)), _stream()), "decay_scan")
+              q_start.numel(), heads, d, dv, max(0, int(longest)), below, _stream()), "decay_scan")
     return o_raw
 
 
@@ -809,20 +819,22 @@ def delta_prepare(proj: torch.Tensor, conv_w: torch.Tensor, a_log: torch.Tensor,
 
 
 def delta_scan(prep: torch.Tensor, state: torch.Tensor, q_start: torch.Tensor, q_len: torch.Tensor, slots: torch.Tensor,
-               o_raw: torch.Tensor, heads: int, kv_heads: int, d: int, dv: int, longest: int = 0, chunks: bool = False) -> torch.Tensor:
+               o_raw: torch.Tensor, heads: int, kv_heads: int, d: int, dv: int, longest: int = 0, chunks: bool = False,
+               portions: Optional[int] = None) -> torch.Tensor:
     """The gated delta rule over every entry's tokens, in order, from and into the entry's slot: S <- g S; u = beta (v - S^T k);
-    S <- S + k u^T; o = S^T q, with `prep` as `delta_prepare` leaves it.  `longest` and `chunks` as for `decay_scan`."""
+    S <- S + k u^T; o = S^T q, with `prep` as `delta_prepare` leaves it.  `longest`, `chunks` and `portions` as for `decay_scan`."""
     _dev(prep, state, q_start, q_len, slots, o_raw)
     _need(prep.dim() == 2 and prep.dtype == torch.float32 and prep.shape[1] >= 2 * kv_heads * d + heads * dv + 2 * heads and heads % kv_heads == 0,
           "delta_scan: prep is float32 [tokens, q | k | v | beta | g]")
     _scan_args(state, q_start, q_len, slots, o_raw, prep.shape[0], heads, d, dv, "delta_scan")
     at = 2 * kv_heads * d + heads * dv
-    if chunks and _matrix_chunks(1, prep, 0, kv_heads * d, 2 * kv_heads * d, at, at + heads, None, state, q_start, q_len, slots, o_raw, heads,
-                                 heads // kv_heads, d, dv, longest):
+    below = _matrix_chunks(1, prep, 0, kv_heads * d, 2 * kv_heads * d, at, at + heads, None, state, q_start, q_len, slots, o_raw, heads,
+                           heads // kv_heads, d, dv, longest, portions) if chunks else 0
+    if below < 0:
         return o_raw
-    fn = _fn("linear_scan", "kipp_delta_scan", [_c_ptr, _c_int, _c_ptr, _c_size, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr])
+    fn = _fn("linear_scan", "kipp_delta_scan", [_c_ptr, _c_int, _c_ptr, _c_size, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr])
     _check(fn(_ptr(prep), prep.shape[1], _ptr(state), state.shape[1], _ptr(q_start), _ptr(q_len), _ptr(slots), _ptr(o_raw), q_start.numel(),
-              heads, kv_heads, d, dv, max(0, int(longest)), _stream()), "delta_scan")
+              heads, kv_heads, d, dv, max(0, int(longest)), below, _stream()), "delta_scan")
     return o_raw
 
 
@@ -869,20 +881,22 @@ def ssd_prepare(proj: torch.Tensor, conv_w: torch.Tensor, conv_b: torch.Tensor, 
 
 
 def gated_scan(prep: torch.Tensor, state: torch.Tensor, q_start: torch.Tensor, q_len: torch.Tensor, slots: torch.Tensor,
-               o_raw: torch.Tensor, heads: int, groups: int, n: int, p: int, longest: int = 0, chunks: bool = False) -> torch.Tensor:
+               o_raw: torch.Tensor, heads: int, groups: int, n: int, p: int, longest: int = 0, chunks: bool = False,
+               portions: Optional[int] = None) -> torch.Tensor:
     """The recurrence with a decay a token and head over every entry's tokens, in order, from and into the entry's slot:
     S <- g S + k v^T; o = S^T q, with `prep` as `ssd_prepare` leaves it (q = C, k = B shared by the heads of a group, v = dt x).
-    `longest` and `chunks` as for `decay_scan`."""
+    `longest`, `chunks` and `portions` as for `decay_scan`."""
     _dev(prep, state, q_start, q_len, slots, o_raw)
     _need(prep.dim() == 2 and prep.dtype == torch.float32 and prep.shape[1] >= ssd_prep_width(heads, groups, n, p) and heads % groups == 0,
           "gated_scan: prep is float32 [tokens, C | B | dt x | x | g]")
     _scan_args(state, q_start, q_len, slots, o_raw, prep.shape[0], heads, n, p, "gated_scan")
-    if chunks and _matrix_chunks(2, prep, 0, groups * n, 2 * groups * n, 0, 2 * groups * n + 2 * heads * p, None, state, q_start, q_len, slots, o_raw,
-                                 heads, heads // groups, n, p, longest):
+    below = _matrix_chunks(2, prep, 0, groups * n, 2 * groups * n, 0, 2 * groups * n + 2 * heads * p, None, state, q_start, q_len, slots, o_raw,
+                           heads, heads // groups, n, p, longest, portions) if chunks else 0
+    if below < 0:
         return o_raw
-    fn = _fn("linear_scan", "kipp_gated_scan", [_c_ptr, _c_int, _c_ptr, _c_size, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr])
+    fn = _fn("linear_scan", "kipp_gated_scan", [_c_ptr, _c_int, _c_ptr, _c_size, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr])
     _check(fn(_ptr(prep), prep.shape[1], _ptr(state), state.shape[1], _ptr(q_start), _ptr(q_len), _ptr(slots), _ptr(o_raw), q_start.numel(),
-              heads, groups, n, p, max(0, int(longest)), _stream()), "gated_scan")
+              heads, groups, n, p, max(0, int(longest)), below, _stream()), "gated_scan")
     return o_raw
 
 

@@ -14,8 +14,8 @@ dual form (`SSDSpec`).
 
 The recurrences, the gates and the norms run in float32 under either precision; the state is float32.  Under float32 a
 prompt portion walks its tokens in order inside one launch, a single token is a walk of one step of the same kernel, so a
-position's result does not depend on how the tokens were cut.  Under bfloat16 a portion goes 64 tokens at a time where the
-key size allows: the same float32 sums in another order.
+position's result does not depend on how the tokens were cut.  Under bfloat16 a portion of 16 tokens and more goes 64 tokens at
+a time where the key size allows: the same float32 sums in another order, which depends on the portion alone.
 """
 from __future__ import annotations
 
@@ -40,6 +40,15 @@ def _scan_variants(key_size, dtype):
     """The walk, and under bfloat16 its form for prompt portions where that takes the key size."""
     from ..csrc.ops import matrix_chunks_ok
     return [("linear_scan", None)] + ([("linear_chunks", None)] if dtype == "bfloat16" and matrix_chunks_ok(key_size) else [])
+
+
+def _portions(batch):
+    """How many entries of the step bring as many tokens as a portion's chunks ask for."""
+    from ..csrc.ops import CHUNKS_FROM
+    n = batch.host.get("chunk_portions")
+    if n is None:
+        n = batch.host["chunk_portions"] = sum(n >= CHUNKS_FROM for n in batch.host["q_len"])
+    return n
 
 
 @register("mixer", "decay_attention")
@@ -89,7 +98,7 @@ class DecayAttention:
         proj = rt.linear(x, self.w_in)                    # float32 [n, q | k | v | gate]
         o_raw = rt.empty((n, hv), torch.float32)
         ops.decay_scan(proj, self.decays, state, batch.q_start, batch.q_len, batch.slots, o_raw, s.num_heads, s.head_dim, s.v_head_dim, longest=batch.max_q_len,
-                       chunks=rt.dtype == "bfloat16")
+                       chunks=rt.dtype == "bfloat16", portions=_portions(batch))
         out = ops.scan_finish(o_raw, proj, 2 * s.num_heads * s.head_dim + hv, self.norm, s.norm_eps, "sigmoid", hv, rt.empty((n, hv), rt.act_dtype))
         return rt.linear(out, self.w_o, slabs=True, defer=True)
 
@@ -157,7 +166,7 @@ class GatedDelta:
                           longest=batch.max_q_len)
         o_raw = rt.empty((n, hv), torch.float32)
         ops.delta_scan(prep, state, batch.q_start, batch.q_len, batch.slots, o_raw, s.num_heads, s.num_kv_heads, s.head_dim, s.v_head_dim, longest=batch.max_q_len,
-                       chunks=rt.dtype == "bfloat16")
+                       chunks=rt.dtype == "bfloat16", portions=_portions(batch))
         out = ops.scan_finish(o_raw, proj, channels, self.norm, s.norm_eps, "silu", s.v_head_dim, rt.empty((n, hv), rt.act_dtype))
         return rt.linear(out, self.w_o, slabs=True, defer=True)
 
@@ -225,7 +234,7 @@ class SSD:
                         batch.slots, prep, s.num_heads, s.groups, s.state_size, s.head_dim, longest=batch.max_q_len)
         o_raw = rt.empty((n, s.inner), torch.float32)
         ops.gated_scan(prep, state, batch.q_start, batch.q_len, batch.slots, o_raw, s.num_heads, s.groups, s.state_size, s.head_dim,
-                       longest=batch.max_q_len, chunks=rt.dtype == "bfloat16")
+                       longest=batch.max_q_len, chunks=rt.dtype == "bfloat16", portions=_portions(batch))
         out = ops.ssd_finish(o_raw, prep, 2 * s.groups * s.state_size + s.inner, proj, 0, self.skip, s.head_dim, self.norm, s.norm_eps,
                              s.inner // s.norm_groups, rt.empty((n, s.inner), rt.act_dtype))
         return rt.linear(out, self.w_o, slabs=True, defer=True)

@@ -99,3 +99,40 @@ def test_few_tokens_and_other_sizes_walk():
             got.append(ops.decay_scan(src, torch.tensor([0.9, 1.0], device=DEV), state, one(0), one(n), one(0), torch.empty((n, heads * dv), device=DEV),
                                       heads, d, dv, longest=n, chunks=chunks))
         assert torch.equal(*got)
+
+
+@pytest.mark.parametrize("mode", ["decay", "delta", "gated"])
+def test_an_entry_beside_others_is_as_alone(mode):
+    """Every entry of a launch, short or long, in any order of the entries, gives the bits it gives alone: the walk's below
+    `CHUNKS_FROM` tokens, the chunks' from there on."""
+    import torch
+    from kipp_amd.csrc import ops
+    rng = np.random.default_rng(1)
+    d, dv, heads = 64, 24, 2
+    lengths = [1, 70, 15, 16, 1, 1, 129, 0, 3] + [1] * 70 + [64]       # (more entries than a wave has lanes)
+    tokens, n = sum(lengths), len(lengths)
+    starts = np.concatenate([[0], np.cumsum(lengths)[:-1]])
+    width = {"decay": heads * (2 * d + dv), "delta": heads * (2 * d + dv + 2), "gated": heads * (2 * d + 2 * dv + 1) + 2}[mode]
+    src = rng.normal(size=(tokens, width)).astype(np.float32) * 0.3
+    src[:, heads * (2 * d + dv):] = rng.uniform(0.3, 1.0, size=src[:, heads * (2 * d + dv):].shape)
+    kept = rng.normal(size=(n, heads * d * dv)).astype(np.float32)
+    dev = lambda a, ty=torch.float32: torch.tensor(np.asarray(a), dtype=ty, device=DEV)  # noqa: E731
+
+    def run(rows, starts, lens, slots, chunks, portions):
+        state, o = dev(kept), torch.zeros((len(rows), heads * dv), device=DEV)
+        where = [state] + [dev(a, torch.int32) for a in (starts, lens, slots)] + [o]
+        said = dict(longest=max(lens), chunks=chunks, portions=portions)
+        if mode == "decay":
+            ops.decay_scan(dev(src[rows]), dev([0.9, 0.99]), *where, heads, d, dv, **said)
+        else:
+            (ops.delta_scan if mode == "delta" else ops.gated_scan)(dev(src[rows]), *where, heads, heads, d, dv, **said)
+        return o.cpu().numpy(), state.cpu().numpy()
+    many = sum(m >= ops.CHUNKS_FROM for m in lengths)
+    order = rng.permutation(n)
+    together = [run(np.arange(tokens), starts[o], np.array(lengths)[o], o, True, portions) for o in (np.arange(n), order) for portions in (None, many)]
+    for o, state in together[1:]:
+        assert np.array_equal(o, together[0][0]) and np.array_equal(state, together[0][1])
+    for e in [0, 1, 2, 3, 6, 8, 40, n - 1]:
+        rows = np.arange(starts[e], starts[e] + lengths[e])
+        o, state = run(rows, [0], [lengths[e]], [e], lengths[e] >= ops.CHUNKS_FROM, None)
+        assert np.array_equal(o, together[0][0][rows]) and np.array_equal(state[e], together[0][1][e]), e
