@@ -873,28 +873,32 @@ int kipp_mixed_attention_mfma(const void* q, const void* k_cache, const void* v_
     return KIPP_LAUNCH_CHECK();
 }
 
-// Single tokens: rows[i] of the batch for i < n_tokens.  scores: float32 [n_tokens][max_tiles][64][32]; stats: float32
-// [n_tokens][n_runs][32][2]; partial: float32 [n_runs][n_tokens][n_q V_DIM]; out: bfloat16 [n_rows][n_q V_DIM], the rows named.
+// Single tokens: rows[i] of the batch for i < n_tokens, `at_a_time` of them after another.  scores: float32
+// [at_a_time][max_tiles][64][32]; stats: float32 [at_a_time][n_runs][32][2]; partial: float32 [n_runs][at_a_time][n_q V_DIM]; out: bfloat16 [n_rows][n_q V_DIM], the rows named.
 // max_tiles: tiles of 64 keys that a token can see at most.
 int kipp_mixed_attention_single(const void* q, const void* k_cache, const void* v_cache, void* out, const float* gate, int gate_stride,
-                                int gate_parts, const int32_t* rows, int n_tokens, const int32_t* positions, const int32_t* seq_of_token,
+                                int gate_parts, const int32_t* rows, int n_tokens, int at_a_time, const int32_t* positions, const int32_t* seq_of_token,
                                 const int32_t* block_table, int max_blocks, const float* r1, const float* r2, const float* sink,
                                 const float* mix, float* scores, float* stats, float* partial, int n_runs, int max_tiles, int n_rows, int n_q,
                                 int n_kv, int d, int dv, int page, float scale, int window, int keep_first, hipStream_t stream) {
     if (n_tokens <= 0 || n_rows <= 0) return 0;
     if (d != HEAD_DIM || dv != V_DIM || n_kv <= 0 || n_q % n_kv || n_q > MX_HPAD || n_q / n_kv > 16) return -1;
-    if (page <= 0 || page % 16 || n_runs < 1 || max_tiles < 1) return -2;
+    if (page <= 0 || page % 16 || n_runs < 1 || max_tiles < 1 || at_a_time < 1) return -2;
     SingleGeometry g;
-    g.rows = rows; g.positions = positions; g.seq_of_token = seq_of_token; g.block_table = block_table;
+    g.positions = positions; g.seq_of_token = seq_of_token; g.block_table = block_table;
     g.max_blocks = max_blocks; g.page = page; g.n_q = n_q; g.n_kv = n_kv; g.window = window; g.keep_first = keep_first;
     g.n_runs = n_runs; g.max_tiles = max_tiles; g.scale = scale; g.r1 = r1; g.r2 = r2;
-    hipLaunchKernelGGL(mixed_single_scores_kernel, dim3(n_runs, n_tokens), dim3(MX_THREADS), 0, stream, g, (const bf16_t*)q, (const bf16_t*)k_cache,
-                       scores, stats);
-    hipLaunchKernelGGL(mixed_single_values_kernel, dim3(n_runs, n_tokens), dim3(MX_THREADS), 0, stream, g, (const bf16_t*)v_cache,
-                       (const float*)scores, (const float*)stats, sink, mix, partial);
-    hipLaunchKernelGGL(mixed_finish_kernel, dim3((n_q * V_DIM / 4 + 255) / 256, n_tokens), dim3(256), 0, stream, (const float*)partial,
-                       (size_t)n_tokens * n_q * V_DIM, (const int32_t*)nullptr, rows, n_runs, gate, gate_stride, gate_parts,
-                       (size_t)n_rows * gate_stride, (bf16_t*)out, n_q * V_DIM);
+    for (int from = 0; from < n_tokens; from += at_a_time) {
+        const int n = n_tokens - from < at_a_time ? n_tokens - from : at_a_time;
+        g.rows = rows + from;
+        hipLaunchKernelGGL(mixed_single_scores_kernel, dim3(n_runs, n), dim3(MX_THREADS), 0, stream, g, (const bf16_t*)q, (const bf16_t*)k_cache,
+                           scores, stats);
+        hipLaunchKernelGGL(mixed_single_values_kernel, dim3(n_runs, n), dim3(MX_THREADS), 0, stream, g, (const bf16_t*)v_cache,
+                           (const float*)scores, (const float*)stats, sink, mix, partial);
+        hipLaunchKernelGGL(mixed_finish_kernel, dim3((n_q * V_DIM / 4 + 255) / 256, n), dim3(256), 0, stream, (const float*)partial,
+                           (size_t)n * n_q * V_DIM, (const int32_t*)nullptr, g.rows, n_runs, gate, gate_stride, gate_parts,
+                           (size_t)n_rows * gate_stride, (bf16_t*)out, n_q * V_DIM);
+    }
     return KIPP_LAUNCH_CHECK();
 }
 

@@ -1357,7 +1357,16 @@ def mixed_attention_mfma(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.
 
 
 MIXED_SINGLE_KEYS = 64          # keys of a tile of the form for single tokens
-MIXED_SINGLE_BYTES = 512 << 20  # most bytes of scores it may keep between its two walks
+# Bytes of scores that it keeps between its two walks, for as many tokens at a time as they hold (one at least): every recorded step
+# keeps a space of its own, and nobody counts it against the cache's.  256 tokens behind 1,500 keys fit (64 MiB in all, 230 us a layer; with
+# half the space 323), behind 4,000 they go by halves: 761 us, 630 with all of their scores at once (126 MiB).
+MIXED_SINGLE_BYTES = 64 << 20
+
+
+def mixed_single_tokens(n_tokens: int, tiles: int) -> int:
+    """How many of the single tokens go at a time: equal shares of no more than the space for scores holds."""
+    most = max(1, MIXED_SINGLE_BYTES // (tiles * MIXED_SINGLE_KEYS * 32 * 4))
+    return -(-n_tokens // -(-n_tokens // most)) if n_tokens else 1
 
 
 def mixed_single_plan(n_tokens: int, max_ctx: int, window: int, keep_first: int):
@@ -1367,16 +1376,18 @@ def mixed_single_plan(n_tokens: int, max_ctx: int, window: int, keep_first: int)
     tiles = -(-max_ctx // keys)
     if window:
         tiles = min(tiles, -(-keep_first // keys) + -(-window // keys) + 1)
-    return max(tiles, 1), max(1, min(tiles, 128, -(-4 * COMPUTE_UNITS // max(n_tokens, 1))))
+    tiles = max(tiles, 1)
+    return tiles, max(1, min(tiles, 128, -(-4 * COMPUTE_UNITS // mixed_single_tokens(n_tokens, tiles))))
 
 
 def mixed_single_ok(n_q: int, n_kv: int, n_tokens: int, tiles: int) -> bool:
-    """Whether single tokens take their own form: up to 16 query heads a key/value head, and scores that fit the space for them."""
-    return n_q // n_kv <= 16 and n_tokens * tiles * MIXED_SINGLE_KEYS * 32 * 4 <= MIXED_SINGLE_BYTES
+    """Whether `n_tokens` single tokens that see up to `tiles` tiles take their own form: up to 16 query heads a key/value head."""
+    return n_q // n_kv <= 16
 
 
 def mixed_single_workspace(n_tokens: int, n_q: int, dv: int, tiles: int, runs: int, device) -> tuple:
-    """(scores, statistics, partial sums) of the form for single tokens."""
+    """(scores, statistics, partial sums) of the form for single tokens, for as many of them as go at a time."""
+    n_tokens = mixed_single_tokens(n_tokens, tiles)
     new = lambda *shape: torch.empty(shape, dtype=torch.float32, device=device)  # noqa: E731
     return new(n_tokens, tiles, MIXED_SINGLE_KEYS, 32), new(n_tokens, runs, 32, 2), new(runs, n_tokens, n_q * dv)
 
@@ -1396,17 +1407,18 @@ def mixed_attention_single(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torc
     n, gate_parts, gate_stride = _mixed_common(q, k_cache, v_cache, out, gate, gate_at, n_q, n_kv, d, dv, r1, r2, sink, mix,
                                                "mixed_attention_single")
     tokens, tiles, runs = rows.numel(), scores.shape[1], stats.shape[1]
+    at_a_time = min(scores.shape[0], stats.shape[0], partial.shape[1])
     _need(all(t.dtype == torch.bfloat16 for t in (q, k_cache, v_cache, out)), "mixed_attention_single: bfloat16 queries, caches and output")
     _need(mixed_attention_fast_ok(n_q, d, dv, k_cache.shape[2]) and n_q // n_kv <= 16, "mixed_attention_single: sizes refused (the other forms take them)")
-    _need(scores.shape[0] >= tokens and stats.shape[0] >= tokens and partial.shape[0] >= runs and partial.numel() >= runs * tokens * n_q * dv,
-          "mixed_attention_single: the workspace is too small")
+    _need(at_a_time >= 1 and scores.shape[2:] == (MIXED_SINGLE_KEYS, 32) and stats.shape[2:] == (32, 2) and partial.shape[0] >= runs
+          and partial.shape[2] == n_q * dv, "mixed_attention_single: the workspace is too small")
     _need(positions.numel() == n and seq_of_token.numel() == n and block_table.dim() == 2, "mixed_attention_single: one position and sequence a row")
     fn = _fn("attention_mixed_mfma", "kipp_mixed_attention_single",
-             [_c_ptr] * 5 + [_c_int, _c_int, _c_ptr, _c_int] + [_c_ptr] * 3 + [_c_int] + [_c_ptr] * 7 + [_c_int] * 8 + [_c_float, _c_int, _c_int, _c_ptr],
+             [_c_ptr] * 5 + [_c_int, _c_int, _c_ptr, _c_int, _c_int] + [_c_ptr] * 3 + [_c_int] + [_c_ptr] * 7 + [_c_int] * 8 + [_c_float, _c_int, _c_int, _c_ptr],
              mixed_attention_defines(n_q, n_kv, d, dv))
     gate_ptr = gate.data_ptr() + 4 * gate_at if gate is not None else None
-    _check(fn(_ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(out), gate_ptr, gate_stride, gate_parts, _ptr(rows), tokens, _ptr(positions),
-              _ptr(seq_of_token), _ptr(block_table), block_table.shape[1], _ptr(r1), _ptr(r2), _ptr(sink), _ptr(mix), _ptr(scores), _ptr(stats),
+    _check(fn(_ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(out), gate_ptr, gate_stride, gate_parts, _ptr(rows), tokens, at_a_time,
+              _ptr(positions), _ptr(seq_of_token), _ptr(block_table), block_table.shape[1], _ptr(r1), _ptr(r2), _ptr(sink), _ptr(mix), _ptr(scores), _ptr(stats),
               _ptr(partial), runs, tiles, n, n_q, n_kv, d, dv, k_cache.shape[2], float(scale), int(window), int(keep_first), _stream()),
            "mixed_attention_single")
     return out

@@ -56,3 +56,14 @@ def test_a_key_that_stands_out_at_every_edge(monkeypatch):
         assert (np.abs(ref[query]).max() > 20.0) == (query - key < window or key < keep)
         got, rows = single_run(case, monkeypatch, [query])
         close(got, ref[rows], KERNEL_TOL["bfloat16"] * 10, f"key {key}")
+
+
+@pytest.mark.parametrize("tokens", [1, 3, 13, 14])
+def test_some_tokens_at_a_time(monkeypatch, tokens):
+    """Space for the scores of a few tokens only: they go one after another through it (14 tokens of up to five tiles of keys here)."""
+    from kipp_amd.csrc import ops
+    monkeypatch.setattr(ops, "MIXED_SINGLE_BYTES", tokens * 5 * 64 * 32 * 4)
+    assert ops.mixed_single_tokens(14, 5) == {1: 1, 3: 3, 13: 7, 14: 14}[tokens]
+    case = MixerCase(6, 3, 32, 16, None, 0, T=260, seed=5)
+    got, rows = single_run(case, monkeypatch, [0, 1, 15, 16, 62, 63, 64, 65, 127, 128, 129, 191, 192, 259], slabs=2)
+    close(got, case.plain(True)[rows], KERNEL_TOL["bfloat16"], tokens)

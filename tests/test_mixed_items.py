@@ -30,3 +30,13 @@ def test_layers_of_other_groups_in_one_step():
         for kv_heads in (first, then):
             single, tiles = layer_of(32, kv_heads)._items(batch)
             assert (single is not None) == (kv_heads == 8) and (tiles is not None) == (kv_heads == 1)
+
+
+def test_space_for_scores_is_bounded():
+    """Many requests behind long contexts, as a recorded step of theirs keeps it: no more than the bound, or one token's scores."""
+    for requests, context in ((256, 8192), (512, 4096), (64, 100_000), (1, 1_000_000)):
+        (scores, stats, partial), _ = layer_of(32, 8)._items(batch_of([1] * requests, [context] * requests))
+        one = -(-context // ops.MIXED_SINGLE_KEYS) * ops.MIXED_SINGLE_KEYS * 32 * 4
+        assert scores.numel() * 4 <= max(64 << 20, one) and scores.numel() * 4 >= one
+        # four workgroups a compute unit at a time, or one for each token of a share
+        assert stats.shape[0] == partial.shape[1] == scores.shape[0] and partial.shape[0] * partial.shape[1] < 1024 + partial.shape[1]
