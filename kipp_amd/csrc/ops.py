@@ -1380,9 +1380,17 @@ def mixed_single_plan(n_tokens: int, max_ctx: int, window: int, keep_first: int)
     return tiles, max(1, min(tiles, 128, -(-4 * COMPUTE_UNITS // mixed_single_tokens(n_tokens, tiles))))
 
 
-def mixed_single_ok(n_q: int, n_kv: int, n_tokens: int, tiles: int) -> bool:
-    """Whether `n_tokens` single tokens that see up to `tiles` tiles take their own form: up to 16 query heads a key/value head."""
-    return n_q // n_kv <= 16
+# Single tokens beside portions: from so many on (a tile that a token sees counts one, the token itself one more) they take their own
+# form; fewer ride along in the tiles of rows, whose launches are there anyway.  One layer's share of a step of four, us, own form / as
+# tiles, beside a portion of 200: 16 tokens of one tile (32) 398 / 372, 64 (128) 418 / 403, 128 (256) 486 / 514; of 16 tiles: 1 token (17)
+# 382 / 365, 8 (136) 398 / 380, 16 (272) 416 / 436, 64 (1,088) 533 / 636.
+MIXED_SINGLE_BESIDE = 256
+
+
+def mixed_single_ok(n_q: int, n_kv: int, n_tokens: int, tiles: int, portions: int = 0) -> bool:
+    """Whether `n_tokens` single tokens that see up to `tiles` tiles of keys take their own form in a step with so many `portions`: up to 16
+    query heads a key/value head, and beside portions work enough for launches of its own."""
+    return n_q // n_kv <= 16 and (portions == 0 or n_tokens * (tiles + 1) >= MIXED_SINGLE_BESIDE)
 
 
 def mixed_single_workspace(n_tokens: int, n_q: int, dv: int, tiles: int, runs: int, device) -> tuple:

@@ -147,7 +147,7 @@ class MixedHeadAttention:
             single = None
             if batch.n_decode:
                 seen, runs = ops.mixed_single_plan(batch.n_decode, batch.max_decode_ctx, window, keep)
-                if ops.mixed_single_ok(s.num_heads, s.num_kv_heads, batch.n_decode, seen):
+                if ops.mixed_single_ok(s.num_heads, s.num_kv_heads, batch.n_decode, seen, batch.n_portions):
                     single = ops.mixed_single_workspace(batch.n_decode, s.num_heads, s.v_head_dim, seen, runs, self.rt.device)
             tiles = []
             for e, (n, ctx) in enumerate(zip(batch.host["q_len"], batch.host["ctx_len"])):

@@ -40,3 +40,15 @@ def test_space_for_scores_is_bounded():
         assert scores.numel() * 4 <= max(64 << 20, one) and scores.numel() * 4 >= one
         # four workgroups a compute unit at a time, or one for each token of a share
         assert stats.shape[0] == partial.shape[1] == scores.shape[0] and partial.shape[0] * partial.shape[1] < 1024 + partial.shape[1]
+
+
+def test_single_tokens_beside_a_portion():
+    """They ride along in the portion's tiles until they are work enough for launches of their own; alone they always have those."""
+    layer = layer_of(32, 8)
+    for tokens, context, own in ((1, 60, False), (64, 60, False), (127, 60, False), (128, 60, True), (8, 1000, False), (16, 1000, True), (1, 16_400, True)):
+        single, tiles = layer._items(batch_of([1] * tokens + [40], [context] * tokens + [40]))
+        assert (single is not None) == own and tiles is not None
+        entries = tiles[0][0].tolist()
+        assert set(entries) == ({tokens} if own else set(range(tokens + 1)))
+        single, tiles = layer._items(batch_of([1] * tokens, [context] * tokens))
+        assert single is not None and tiles is None
