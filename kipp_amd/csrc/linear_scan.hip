@@ -464,9 +464,11 @@ extern "C" int kipp_ssd_prepare(const float* proj, int stride, const float* conv
 // y[t][c] = (o[t][c] + skip[c / p] x[t][c]) * silu(z[t][c]); out = y * rsqrt(mean over c's span of y^2 + eps) * w[c]: the gate
 // comes before the norm.  x at column `x_at` of prep, z at column `z_at` of proj.
 // ITEMS columns a thread (beyond: read for the sum, and again), all asked for at once: for single tokens the loads' latencies are the time
-// (a token of 5,120 columns 6.6 us; 10.9 with a column after the other).
-template <typename TO, int ITEMS>
-__global__ void __launch_bounds__(SCAN_THREADS)
+// (a token of 5,120 columns 5.5 us; 10.9 with a column after the other).  Five columns a thread at most, and threads for about as many as
+// the span has: 2,048 tokens of 5,120 columns in spans of 1,280 take 27 us; with twenty columns a thread, three of four of them beyond the
+// span, 57, and with a column after the other 38.
+template <typename TO, int THREADS, int ITEMS>
+__global__ void __launch_bounds__(THREADS)
 ssd_finish_kernel(const float* __restrict__ o_raw, const float* __restrict__ prep, int prep_stride, int x_at,
                   const float* __restrict__ proj, int proj_stride, int z_at, const float* __restrict__ skip, int p,
                   const float* __restrict__ w, float eps, TO* __restrict__ out, int width, int span) {
@@ -479,7 +481,7 @@ ssd_finish_kernel(const float* __restrict__ o_raw, const float* __restrict__ pre
     float ov[ITEMS], xv[ITEMS], zv[ITEMS], sv[ITEMS], wv[ITEMS];
 #pragma unroll
     for (int i = 0; i < ITEMS; ++i) {
-        const int e = min((int)threadIdx.x + i * SCAN_THREADS, span - 1);
+        const int e = min((int)threadIdx.x + i * THREADS, span - 1);
         ov[i] = o[e];
         xv[i] = x[e];
         zv[i] = z[e];
@@ -491,19 +493,19 @@ ssd_finish_kernel(const float* __restrict__ o_raw, const float* __restrict__ pre
 #pragma unroll
     for (int i = 0; i < ITEMS; ++i) {
         ov[i] = fmaf(sv[i], xv[i], ov[i]) * silu_f(zv[i]);
-        if ((int)threadIdx.x + i * SCAN_THREADS < span) ss = fmaf(ov[i], ov[i], ss);
+        if ((int)threadIdx.x + i * THREADS < span) ss = fmaf(ov[i], ov[i], ss);
     }
-    for (int e = threadIdx.x + ITEMS * SCAN_THREADS; e < span; e += SCAN_THREADS) {
+    for (int e = threadIdx.x + ITEMS * THREADS; e < span; e += THREADS) {
         const float y = fmaf(skip[(c0 + e) / p], x[e], o[e]) * silu_f(z[e]);
         ss = fmaf(y, y, ss);
     }
     const float inv = 1.0f / sqrtf(block_sum(ss, scratch) / (float)span + eps);
 #pragma unroll
     for (int i = 0; i < ITEMS; ++i) {
-        const int e = threadIdx.x + i * SCAN_THREADS;
+        const int e = threadIdx.x + i * THREADS;
         if (e < span) store_f(out, t * width + c0 + e, ov[i] * inv * wv[i]);
     }
-    for (int e = threadIdx.x + ITEMS * SCAN_THREADS; e < span; e += SCAN_THREADS) {
+    for (int e = threadIdx.x + ITEMS * THREADS; e < span; e += THREADS) {
         const float y = fmaf(skip[(c0 + e) / p], x[e], o[e]) * silu_f(z[e]);
         store_f(out, t * width + c0 + e, y * inv * w[c0 + e]);
     }
@@ -514,14 +516,19 @@ extern "C" int kipp_ssd_finish(const float* o_raw, const float* prep, int prep_s
                                int width, int span, hipStream_t stream) {
     if (tokens <= 0) return 0;
     if (width <= 0 || span <= 0 || width % span || p <= 0 || width % p || prep_stride < x_at + width || proj_stride < z_at + width) return -1;
-    dim3 grid(width / span, tokens), block(SCAN_THREADS);
-#define KIPP_SF(TO, ITEMS)                                                                                                             \
-    hipLaunchKernelGGL((ssd_finish_kernel<TO, ITEMS>), grid, block, 0, stream, o_raw, prep, prep_stride, x_at, proj, proj_stride, z_at, skip, p, \
-                       w, eps, (TO*)out, width, span)
+    dim3 grid(width / span, tokens);
+#define KIPP_SF(TO, THREADS, ITEMS)                                                                                                    \
+    hipLaunchKernelGGL((ssd_finish_kernel<TO, THREADS, ITEMS>), grid, dim3(THREADS), 0, stream, o_raw, prep, prep_stride, x_at, proj,      \
+                       proj_stride, z_at, skip, p, w, eps, (TO*)out, width, span)
 #define KIPP_SFT(TO)                                                                                                                   \
-    if (span <= SCAN_THREADS) KIPP_SF(TO, 1);                                                                                          \
-    else if (span <= 4 * SCAN_THREADS) KIPP_SF(TO, 4);                                                                                 \
-    else KIPP_SF(TO, 20)
+    if (span <= 64) KIPP_SF(TO, 64, 1);                                                                                                \
+    else if (span <= 256) KIPP_SF(TO, 256, 1);                                                                                         \
+    else if (span <= 512) KIPP_SF(TO, 256, 2);                                                                                         \
+    else if (span <= 1024) KIPP_SF(TO, 256, 4);                                                                                        \
+    else if (span <= 1536) KIPP_SF(TO, 512, 3);                                                                                        \
+    else if (span <= 2560) KIPP_SF(TO, 512, 5);                                                                                        \
+    else if (span <= 4096) KIPP_SF(TO, 1024, 4);                                                                                       \
+    else KIPP_SF(TO, 1024, 5)
     if (out_dtype == KIPP_F32) {
         KIPP_SFT(float);
     } else if (out_dtype == KIPP_BF16) {

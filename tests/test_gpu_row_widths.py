@@ -39,6 +39,35 @@ def test_layer_norm_and_step(width, parts):
         assert float((out.double() - layer_norm64(x.double(), w2.double(), b2.double(), 1e-5)).abs().max()) <= bound
 
 
+@pytest.mark.parametrize("span", [1, 16, 64, 65, 256, 257, 512, 513, 1024, 1025, 1536, 1537, 2560, 2561, 4096, 4097, 5120, 5121, 11000])
+@pytest.mark.parametrize("spans", [1, 3])
+def test_state_space_finish(span, spans):
+    from kipp_amd.csrc import ops
+    rng = np.random.default_rng(span)
+    width = span * spans
+    o, prep, proj, skip, w = f32(rng, 3, width), f32(rng, 3, width + 5), f32(rng, 3, width + 7), f32(rng, spans), f32(rng, width)
+    out = ops.ssd_finish(o, prep, 5, proj, 7, skip, span, w, 1e-5, span, torch.empty((3, width), device=DEV))
+    z = proj[:, 7:].double()
+    y = (o.double() + skip.double().repeat_interleave(span) * prep[:, 5:].double()) * z * torch.sigmoid(z)
+    ref = (y.view(3, spans, -1) / (y.view(3, spans, -1).square().mean(-1, keepdim=True) + 1e-5).sqrt()).reshape(3, width) * w.double()
+    # a handful of float32 roundings and a sum of `span` squares, at most `span` / 256 of them a thread: halved by the root
+    assert ((out.double() - ref).abs() <= (ref.abs() + 1e-3) * 2.0 ** -24 * (span / 256 + 30)).all()
+
+
+def fastest(run):
+    """Milliseconds of 40 runs, the best of eight times."""
+    marks = []
+    for _ in range(8):
+        begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        begin.record()
+        for _ in range(40):
+            run()
+        end.record()
+        marks.append((begin, end))
+    torch.cuda.synchronize()
+    return min(a.elapsed_time(b) for a, b in marks)
+
+
 def test_wide_rows_take_their_share_of_the_time():
     """Rows of 8,192 are 3.2 times as many bytes as rows of 2,560, and take no more than four times as long."""
     from kipp_amd.csrc import ops
@@ -47,14 +76,15 @@ def test_wide_rows_take_their_share_of_the_time():
     for width in (2560, 8192):
         x, u, w = torch.randn(2048, width, device=DEV), torch.randn(2048, width, device=DEV), f32(rng, width)
         out = torch.empty((2048, width), dtype=torch.bfloat16, device=DEV)
-        marks = []
-        for _ in range(8):
-            begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-            begin.record()
-            for _ in range(40):
-                ops.sandwich_step(x, u, w, w, 1e-5, 0.01, next_w=w, next_b=w, next_eps=1e-5, out=out)
-            end.record()
-            marks.append((begin, end))
-        torch.cuda.synchronize()
-        took[width] = min(a.elapsed_time(b) for a, b in marks)
+        took[width] = fastest(lambda: ops.sandwich_step(x, u, w, w, 1e-5, 0.01, next_w=w, next_b=w, next_eps=1e-5, out=out))
     assert took[8192] <= 4.0 * took[2560], took
+
+
+def test_spans_take_their_share_of_the_time():
+    """The same columns in spans of 1,280 take no more than one and a half times what they take in spans of 640."""
+    from kipp_amd.csrc import ops
+    rng = np.random.default_rng(0)
+    o, prep, proj, skip, w = f32(rng, 2048, 5120), f32(rng, 2048, 5120), f32(rng, 2048, 5120), f32(rng, 80), f32(rng, 5120)
+    out = torch.empty((2048, 5120), dtype=torch.bfloat16, device=DEV)
+    took = {span: fastest(lambda: ops.ssd_finish(o, prep, 0, proj, 0, skip, 64, w, 1e-5, span, out)) for span in (640, 1280)}
+    assert took[1280] <= 1.5 * took[640], took
