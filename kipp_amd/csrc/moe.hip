@@ -45,6 +45,8 @@
 #define MANY_STAGES 4       // one workgroup (two waves a SIMD) a compute unit
 #define ROWS_TILE 64        // rows of a tile of the product for few rows
 #define ROWS_WAVES 8        // waves of its workgroup
+#define ROWS_SHORT_K 1024   // K up to which a workgroup of it has two steps a wave at most, and is the slower one
+#define ROWS_SHORT_GROUPS 2048      // in a launch of more workgroups than this
 #define XCDS 8              // dies of the chip; consecutive workgroups of a launch go to them in turn
 
 enum { ACT_NONE = -1, ACT_SILU = 0, ACT_RELU = 1, ACT_GELU = 2, ACT_GELU_TANH = 3, ACT_RELU2 = 4 };
@@ -913,7 +915,15 @@ static int launch_expert(const void* x, int x_dtype, const int32_t* gather, cons
                          int x_rows, int sorted_rows, int experts, hipStream_t stream) {
     if (max_tiles <= 0) return 0;
     if (n_out <= 0 || k <= 0 || act < ACT_NONE || act > ACT_RELU2) return -1;
-    if (tile_rows == ROWS_TILE) {
+    // a lane's offsets into x and into an expert's matrix are 32 bits wide in the kernels for whole tiles: numbers in the staged one, bytes
+    // in the walk; rows of x that `gather` may name reach as far as x does
+    const bool fits = (long long)max_tiles * tile_rows * k < (1ll << 31) && (long long)(GLU ? 2 : 1) * n_out * k < (1ll << 31) &&
+                      (long long)x_rows * k < (1ll << 32);
+    // Tiles of few rows whose workgroups would have little of K each, and be many, are the staged kernel's: beside it the one for few rows
+    // takes, 256 experts of 1,024 x 512 and 10 pairs an expert, 1.25 and 1.5 of the time (gated, and back); 64 of 2,048 x 704, up 0.8, back 1.35.
+    const long long hit = sorted_rows < experts ? sorted_rows : experts;
+    const bool short_k = k <= ROWS_SHORT_K && hit * ((n_out + 15) / 16) > ROWS_SHORT_GROUPS;
+    if (tile_rows == ROWS_TILE && !(short_k && fits)) {
         if (x_dtype != KIPP_BF16 || w_dtype != KIPP_BF16 || k % 32 || (((uintptr_t)x | (uintptr_t)w) & 15)) return -2;
         dim3 grid((n_out + 15) / 16, max_tiles), block(ROWS_WAVES * KIPP_WAVE);
         if (out_dtype == KIPP_BF16)
@@ -926,14 +936,11 @@ static int launch_expert(const void* x, int x_dtype, const int32_t* gather, cons
             return -2;
         return KIPP_LAUNCH_CHECK();
     }
-    if (tile_rows == MFMA_ROWS || tile_rows == MANY_ROWS) {
-        if (x_dtype != KIPP_BF16 || w_dtype != KIPP_BF16 || k % 32) return -2;
-        // a lane's offsets into x and into an expert's matrix are 32 bits wide in either kernel: numbers in the staged one, bytes in the walk
-        if ((long long)max_tiles * tile_rows * k >= (1ll << 31) || (long long)(GLU ? 2 : 1) * n_out * k >= (1ll << 31) ||
-            (long long)x_rows * k >= (1ll << 32)) return -2;
-        // the walk brings 16 bytes a lane; rows of x that `gather` may name reach as far as x does
+    if (tile_rows == ROWS_TILE || tile_rows == MFMA_ROWS || tile_rows == MANY_ROWS) {
+        if (x_dtype != KIPP_BF16 || w_dtype != KIPP_BF16 || k % 32 || !fits) return -2;
+        // the walk brings 16 bytes a lane
         const bool walks = (((uintptr_t)x | (uintptr_t)w) & 15) == 0 && (long long)x_rows * k < (1ll << 31);
-        if (tile_rows == MFMA_ROWS && (!walks || sorted_rows <= WALK_FROM * (long long)experts)) {
+        if (tile_rows == ROWS_TILE || (tile_rows == MFMA_ROWS && (!walks || sorted_rows <= WALK_FROM * (long long)experts))) {
             const int cols = GLU ? MFMA_COLS / 2 : MFMA_COLS;
             dim3 grid(max_tiles, (n_out + cols - 1) / cols), block(MFMA_THREADS);
             if (out_dtype == KIPP_BF16)

@@ -1039,11 +1039,16 @@ MOE_TILE_ROWS = 16
 MOE_MFMA_ROWS = 128    # rows of a tile of the experts' products on the matrix cores
 MOE_FEW_ROWS = 64      # the same in the kernel for few rows an expert, which reads the experts' matrices straight into the products
 MOE_MANY_ROWS = 256    # the same where an expert has many rows: its matrix is read less often, a compute unit has one workgroup
-# Pairs an expert (all of them) up to which a step takes the kernel for few rows, and from which on a gated one, or one without a
-# gate, takes tiles of 256.  32 experts, inner 2,432, width 2,560, both products, us: 256 pairs gated 251 with tiles of 64, 276 with 128;
-# 512 pairs 314 and 281; gated with tiles of 128 / 256: 2,048 pairs 314 / 316, 3,200 341 / 343, 4,300 428 / 377, 8,192 564 / 490; without
-# a gate 6,400 340 / 362, 7,600 362 / 362, 8,192 414 / 363, 10,000 409 / 412, 12,288 511 / 458.
-MOE_FEW_PAIRS, MOE_MANY_PAIRS, MOE_MANY_PAIRS_UNGATED = 12, 96, 240
+# Pairs an expert (all of them) up to which a step takes the kernel for few rows, in its time over that of tiles of 128, both products,
+# at 4, 6, 8 and 12 pairs: 32 experts of 2,560 x 2,432 gated 0.84 0.88 0.96 1.11, 32 of 4,096 x 3,072 gated 0.98 1.04 1.10 1.21,
+# 16 of 5,120 x 3,200 without a gate 0.89 0.92 1.01 1.13, 8 of 4,096 x 3,584 0.70 0.74 0.79 0.89 (a product with little of K goes by its
+# own rule, in the kernel's launch).
+MOE_FEW_PAIRS = 6
+# From how many pairs on a gated step, or one without a gate, takes tiles of 256.  32 experts of 2,560 x 2,432, both products, us: gated with
+# tiles of 128 / 256: 2,048 pairs 314 / 316, 3,200 341 / 343, 4,300 428 / 377, 8,192 564 / 490; without a gate 6,400 340 / 362,
+# 7,600 362 / 362, 8,192 414 / 363, 10,000 409 / 412, 12,288 511 / 458: rounds of workgroups, which the number of tiles decides, and
+# the device alone knows that.
+MOE_MANY_PAIRS, MOE_MANY_PAIRS_UNGATED = 96, 240
 
 
 def moe_tile_rows(dtype: torch.dtype, *contractions: int, pairs: Optional[int] = None, experts: int = 1, gated: bool = False) -> int:

@@ -125,3 +125,78 @@ def test_operands_at_any_offset():
     size = flat[2:2 + rows * k].view(rows, k).double().abs() @ w[0].double().abs().T
     for out in results:
         assert bool(((out.double() - ref).abs() <= (k + 4) * 2.0 ** -24 * size).all())
+
+
+@pytest.mark.parametrize("k, n_out", [(512, 1040), (1024, 528), (1056, 528)])
+@pytest.mark.parametrize("gated", [False, True])
+def test_lists_of_few_rows_in_products_of_little_k(k, n_out, gated):
+    """On both sides of the K up to which a launch of many workgroups takes the staged kernel for tiles of up to 64 rows: lists of 64
+    and of 128 rows against float64."""
+    import torch
+    from kipp_amd.csrc import ops
+    rng = np.random.default_rng(k)
+    counts = list(rng.integers(0, 9, 64)) + [64, 33, 65, 17]
+    experts, rows = len(counts), int(sum(counts))
+    x = torch.tensor(rng.normal(size=(rows, k)).astype(np.float32), device=DEV).bfloat16()
+    w = torch.tensor((rng.normal(size=(experts, n_out * (2 if gated else 1), k)) * k ** -0.5).astype(np.float32), device=DEV).bfloat16()
+    starts = np.concatenate([[0], np.cumsum(counts)[:-1]])
+    ref = torch.empty((rows, n_out), dtype=torch.float64, device=DEV)
+    size = torch.empty_like(ref)
+    for e, (at, n) in enumerate(zip(starts, counts)):
+        p, a = x[at:at + n].double() @ w[e].double().T, x[at:at + n].double().abs() @ w[e].double().abs().T
+        if gated:
+            g, u = p[:, :n_out], p[:, n_out:]
+            ref[at:at + n] = torch.relu(g) * u
+            size[at:at + n] = a[:, :n_out] * u.abs() + g.abs() * a[:, n_out:]
+        else:
+            ref[at:at + n], size[at:at + n] = p, a
+    for tile_rows in (64, 128):
+        tiles = [(e, at + j, min(tile_rows, n - j)) for e, (at, n) in enumerate(zip(starts, counts)) for j in range(0, n, tile_rows)] + [(0, 0, 0)] * 3
+        td = torch.tensor(np.array(tiles, dtype=np.int32), device=DEV)
+        out = torch.full((rows, n_out), float("nan"), device=DEV)
+        if gated:
+            ops.moe_expert_gated(x, None, None, w, td, out, "relu", tile_rows=tile_rows)
+        else:
+            ops.moe_expert(x, None, w, td, out, tile_rows=tile_rows)
+        # sums of k exact products in float32, in any order
+        assert bool(((out.double() - ref).abs() <= (k + 4) * 2.0 ** -24 * size + 2.0 ** -22 * ref.abs()).all()), tile_rows
+
+
+def both_products(experts, width, inner, top, tokens, gated, tile_rows):
+    """Milliseconds of 12 runs of a step's two products with tiles of so many rows, the best of six times."""
+    import torch
+    from kipp_amd.csrc import ops
+    torch.manual_seed(tokens)
+    pairs = tokens * top
+    i32 = lambda *shape: torch.empty(shape, dtype=torch.int32, device=DEV)  # noqa: E731
+    bf = lambda *shape: torch.randn(*shape, device=DEV).bfloat16()  # noqa: E731
+    x, up, down = bf(tokens, width), bf(experts, inner * (2 if gated else 1), width), bf(experts, width, inner)
+    mid, out = bf(pairs, inner), torch.empty((pairs, width), device=DEV)
+    pair_token, place, tiles = i32(pairs), i32(pairs), i32(ops.moe_max_tiles(tokens, experts, top, tile_rows), 3)
+    z = torch.randn(tokens, experts, device=DEV) + 0.4 * torch.randn(experts, device=DEV)
+    ops.moe_route(z, experts, top, 1e-20, i32(tokens, top), torch.empty((tokens, top), device=DEV), pair_token, place, tiles, tile_rows=tile_rows)
+    marks = []
+    for _ in range(7):
+        begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        begin.record()
+        for _ in range(12):
+            if gated:
+                ops.moe_expert_gated(x, pair_token, None, up, tiles, mid, "silu", tile_rows=tile_rows)
+            else:
+                ops.moe_expert(x, pair_token, up, tiles, mid, "gelu", tile_rows=tile_rows)
+            ops.moe_expert(mid, None, down, tiles, out, tile_rows=tile_rows)
+        end.record()
+        marks.append((begin, end))
+    torch.cuda.synchronize()
+    return min(a.elapsed_time(b) for a, b in marks[1:])
+
+
+@pytest.mark.parametrize("experts, width, inner, top, tokens, gated", [(256, 1024, 512, 8, 333, True), (64, 2048, 704, 6, 128, False),
+                                                                       (32, 4096, 3072, 4, 96, True)])
+def test_the_tiles_chosen_are_not_much_slower_than_those_of_128(experts, width, inner, top, tokens, gated):
+    """Sizes away from 32 experts of 2,432 x 2,560, at 10 to 12 pairs an expert."""
+    import torch
+    from kipp_amd.csrc import ops
+    rows = ops.moe_tile_rows(torch.bfloat16, width, inner, pairs=tokens * top, experts=experts, gated=gated)
+    chosen, whole = (both_products(experts, width, inner, top, tokens, gated, r) for r in (rows, 128))
+    assert chosen <= 1.12 * whole, (rows, chosen, whole)
