@@ -1049,16 +1049,21 @@ MOE_FEW_PAIRS = 6
 # 7,600 362 / 362, 8,192 414 / 363, 10,000 409 / 412, 12,288 511 / 458: rounds of workgroups, which the number of tiles decides, and
 # the device alone knows that.
 MOE_MANY_PAIRS, MOE_MANY_PAIRS_UNGATED = 96, 240
+# Workgroups of the first product (half a tile an expert more than its pairs fill) below which tiles of 256 leave too much of the chip idle:
+# 8 experts of 1,024 x 1,024 without a gate, 2,256 pairs, both products 78 us with tiles of 256 (about 50 workgroups), 67 with tiles of 128.
+MOE_MANY_GROUPS = 128
 
 
 def moe_tile_rows(dtype: torch.dtype, *contractions: int, pairs: Optional[int] = None, experts: int = 1, gated: bool = False) -> int:
     """Rows of the tiles that the experts' products take: 128 on the matrix cores (bfloat16, every contraction a multiple of
-    32), else 16.  With `pairs`, the (token, choice) pairs of the step: 64 for few of them an expert, 256 for many."""
+    32), else 16.  With `pairs`, the (token, choice) pairs of the step: 64 for few of them an expert, 256 for many and for
+    columns enough of the first product (as many as the last contraction)."""
     if dtype != torch.bfloat16 or any(k % 32 for k in contractions):
         return MOE_TILE_ROWS
     if pairs is not None and pairs <= MOE_FEW_PAIRS * experts:
         return MOE_FEW_ROWS
-    many = pairs is not None and pairs > (MOE_MANY_PAIRS if gated else MOE_MANY_PAIRS_UNGATED) * experts
+    many = pairs is not None and pairs > (MOE_MANY_PAIRS if gated else MOE_MANY_PAIRS_UNGATED) * experts \
+        and (pairs / MOE_MANY_ROWS + experts / 2) * -(-contractions[-1] // (128 if gated else 256)) >= MOE_MANY_GROUPS
     # (a lane's offsets into the rows, as many as the tiles could hold, and into an expert's matrix are 32 bits wide)
     if many and (-(-pairs // MOE_MANY_ROWS) + experts) * MOE_MANY_ROWS * max(contractions) < 1 << 31 and 2 * max(contractions) * min(contractions) < 1 << 31:
         return MOE_MANY_ROWS

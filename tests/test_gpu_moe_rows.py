@@ -192,9 +192,9 @@ def both_products(experts, width, inner, top, tokens, gated, tile_rows):
 
 
 @pytest.mark.parametrize("experts, width, inner, top, tokens, gated", [(256, 1024, 512, 8, 333, True), (64, 2048, 704, 6, 128, False),
-                                                                       (32, 4096, 3072, 4, 96, True)])
+                                                                       (32, 4096, 3072, 4, 96, True), (8, 1024, 1024, 2, 1128, False)])
 def test_the_tiles_chosen_are_not_much_slower_than_those_of_128(experts, width, inner, top, tokens, gated):
-    """Sizes away from 32 experts of 2,432 x 2,560, at 10 to 12 pairs an expert."""
+    """Sizes away from 32 experts of 2,432 x 2,560, at 10 to 12 pairs an expert and at 282."""
     import torch
     from kipp_amd.csrc import ops
     rows = ops.moe_tile_rows(torch.bfloat16, width, inner, pairs=tokens * top, experts=experts, gated=gated)
