@@ -1054,12 +1054,16 @@ MOE_MANY_PAIRS, MOE_MANY_PAIRS_UNGATED = 96, 240
 MOE_MANY_GROUPS = 128
 
 
-def moe_tile_rows(dtype: torch.dtype, *contractions: int, pairs: Optional[int] = None, experts: int = 1, gated: bool = False) -> int:
+def moe_tile_rows(dtype: torch.dtype, *contractions: int, pairs: Optional[int] = None, experts: int = 1, gated: bool = False,
+                  aligned: bool = True) -> int:
     """Rows of the tiles that the experts' products take: 128 on the matrix cores (bfloat16, every contraction a multiple of
     32), else 16.  With `pairs`, the (token, choice) pairs of the step: 64 for few of them an expert, 256 for many and for
-    columns enough of the first product (as many as the last contraction)."""
+    columns enough of the first product (as many as the last contraction), unless rows or matrices do not begin at multiples of 16
+    bytes (`aligned`): those are taken in tiles of 128."""
     if dtype != torch.bfloat16 or any(k % 32 for k in contractions):
         return MOE_TILE_ROWS
+    if not aligned:
+        return MOE_MFMA_ROWS
     if pairs is not None and pairs <= MOE_FEW_PAIRS * experts:
         return MOE_FEW_ROWS
     many = pairs is not None and pairs > (MOE_MANY_PAIRS if gated else MOE_MANY_PAIRS_UNGATED) * experts \

@@ -200,3 +200,23 @@ def test_the_tiles_chosen_are_not_much_slower_than_those_of_128(experts, width, 
     rows = ops.moe_tile_rows(torch.bfloat16, width, inner, pairs=tokens * top, experts=experts, gated=gated)
     chosen, whole = (both_products(experts, width, inner, top, tokens, gated, r) for r in (rows, 128))
     assert chosen <= 1.12 * whole, (rows, chosen, whole)
+
+
+@pytest.mark.parametrize("tokens", [1, 40, 700])
+@pytest.mark.parametrize("gated", [False, True])
+def test_feed_forward_of_rows_at_any_offset(tokens, gated):
+    """The whole part over rows that begin at no multiple of 16 bytes: for steps of few pairs an expert, of some and of many."""
+    import torch
+    from kipp_amd.config import RoutedMLPSpec
+    from kipp_amd.parts import build_part
+    from kipp_amd.runtime import Runtime
+    rng = np.random.default_rng(tokens)
+    width, inner = 96, 16512 if gated else 33024        # (columns enough for tiles of 256 rows at so few experts)
+    spec = RoutedMLPSpec(hidden_size=width, experts=3, top=2, expert_size=inner, activation="silu" if gated else "relu2", gate_name="gate" if gated else None)
+    part = build_part("feed_forward", spec, Runtime("bfloat16"))
+    part.load({name: torch.tensor(rng.normal(size=p.shape) / np.sqrt(p.shape[-1]), dtype=torch.bfloat16, device=DEV) for name, p in part.params(spec).items()})
+    flat = torch.tensor(rng.normal(size=tokens * width + 8), dtype=torch.bfloat16, device=DEV)
+    x = flat[1:1 + tokens * width].view(tokens, width)
+    got, ref = part.forward(x), part.forward(x.clone())
+    # the products in two orders of their sums, the inner rows rounded to bfloat16 in between
+    assert float((got - ref).norm() / ref.norm()) < 4e-3

@@ -18,3 +18,5 @@ def test_many_rows_an_expert():
     assert [rows(32, 2560, 2432, 32 * n, False) for n in (240, 241)] == [128, 256]
     assert [rows(8, 1024, 1024, 8 * n, False) for n in (282, 512, 7000)] == [128, 128, 256]
     assert [rows(8, 1024, 1024, 8 * n, True) for n in (100, 282, 1024)] == [128, 128, 256]
+    assert ops.moe_tile_rows(torch.bfloat16, 2560, 2432, pairs=1, experts=32, aligned=False) == 128
+    assert ops.moe_tile_rows(torch.bfloat16, 2560, 2432, pairs=32 * 500, experts=32, aligned=False) == 128
