@@ -484,7 +484,9 @@ class Runtime:
             # every slab beyond the first is read once more by the kernel that adds them (at about 5 TB/s)
             slab_ms = m * n * 4 / 5e12 * 1e3
             extra = {name: ((planned if name == "plan" else name % 10) - 1) * slab_ms for name in ways if name != "library"}
-            choice = self._fastest(("linear", self._rows_class(m), n, x.shape[1], most), ways, same, m, n, extra_ms=extra)
+            # with our own products alone, rows that the plan cuts into other parts of K have other ways: they are timed by themselves
+            key = ("linear", self._rows_class(m), n, x.shape[1], most) + ((planned,) if self.own_prompt_products is True else ())
+            choice = self._fastest(key, ways, same, m, n, extra_ms=extra)
             if choice != "library":
                 self.tile_products += 1
                 return ours(0 if choice == "plan" else choice)

@@ -1,8 +1,10 @@
 """How a prompt product is cut at rows that its class was not timed at: by the times of the rows it was timed at, in proportion to the rounds
 of tiles over the compute units."""
 import math
+from types import SimpleNamespace
 
 import pytest
+import torch
 
 from kipp_amd.runtime import Runtime
 
@@ -49,3 +51,24 @@ def test_own_products_keep_the_plans_bits_at_every_number_of_rows(monkeypatch):
     monkeypatch.setattr(Runtime, "_choices_of_process", {(True, ("linear",)): (443, 2048, took, {2048: 443})})
     assert rt._fastest(("linear",), {}, ("plan", 442, 1422), 1100, 4096) == "plan"
     assert rt._fastest(("linear",), {}, ("plan", 443, 1423), 1101, 4096) == 443
+
+
+@pytest.mark.parametrize("own", [True, "auto"])
+def test_own_products_are_timed_for_every_number_of_parts(monkeypatch, own):
+    """Rows of one class that the plan cuts into one, two and three parts of K: each finds the cuts with its parts among the ways, timed; where
+    any way may be taken, the class is timed once."""
+    rt = Runtime.__new__(Runtime)
+    rt.own_prompt_products, rt.for_a_graph, rt.prompt_product_choices = own, False, {}
+    rt.staged_rows, rt.few_rows, rt.tile_products, rt.library_products = 192, 64, 0, 0
+    parts = {1100: 1, 1300: 2, 1500: 3, 1101: 1}
+    asked = []
+    rt.ops = SimpleNamespace(gemm_rows_ok=lambda m, k: False, gemm_tiles_ok=lambda m, k, n: True, gemm_tiles_parts=lambda m, *a: parts[m],
+                             gemm_tiles=lambda x, w, **k: torch.zeros(1, 1, 1))
+    monkeypatch.setattr(Runtime, "_fastest", lambda self, key, ways, same, m, cols, **k: asked.append((key, same)) or "plan")
+    w = torch.zeros((64, 32), dtype=torch.bfloat16)
+    for m in parts:
+        rt.linear(torch.zeros((m, 32), dtype=torch.bfloat16), w, slabs=True)
+    keys = {m: key for m, (key, _) in zip(parts, asked)}
+    assert keys[1100] == keys[1101] and len(set(keys.values())) == (3 if own is True else 1)
+    for m, (_, same) in zip(parts, asked):
+        assert all(cut % 10 == parts[m] for cut in same if cut != "plan")
