@@ -272,8 +272,8 @@ class Runtime:
     @staticmethod
     def _rounds_of(name, m: int, cols: int, pairs: bool) -> float:
         """What a way to compute a product costs at m rows, in units of its own: the rounds of its tiles over the 256 compute units (of
-        the library's: 256 rows at a time; of the planned way: of what the plan would take).  A class is timed at the first rows that come; the others' times
-        are taken in proportion to this.  (1,193 rows against [gate; up] of 2 x 12,288 x 4,096: whole rounds of 256 x 256 and the rest in
+        the library's: 256 rows at a time; of the planned way: of what the plan would take).  A class is timed at the first rows that come; the times
+        of our cuts at others are taken in proportion to this.  (1,193 rows against [gate; up] of 2 x 12,288 x 4,096: whole rounds of 256 x 256 and the rest in
         128 x 64 were level with one cut at the class's first 2,048 rows, three rounds and no rest; there 281 us against 231.)"""
         if name == "plan":
             if pairs and m >= 512:
@@ -294,6 +294,20 @@ class Runtime:
             return rounds(4, 2, 4, 1, cols)
         return rounds(4, 2, 4, 1, first) + rounds(*((2, 2, 4), (4, 2, 2), (2, 4, 2), (2, 2, 2))[rest], 1, cols - first)
 
+    @staticmethod
+    def _at_rows(choice, took: dict, rows: int, m: int, cols: int, pairs: bool):
+        """What a class timed at `rows` rows (`took`: milliseconds) takes at m: one of our cuts by its time in proportion to the rounds of its
+        tiles, where that promises 5 % more than the class's choice.  The library's times do not go by rounds, nor do those of the plan that
+        may split K: chosen, they stay, and they are chosen by times alone.  (Four products of each of the 4B, 8B and 32B shapes at 25
+        numbers of rows up to 2,048, a class first timed at every other of its numbers: 2.1 % over the fastest way in the mean, 3.5 with the
+        class's choice at all its rows, 4.6 with every way in proportion, where a product took up to 1.7 times the class's choice.)"""
+        if choice in took and (choice == "library" or (choice == "plan" and not pairs)):
+            return choice
+        names = [name for name in took if name != "library" and (pairs or name != "plan")] or list(took)
+        there = {name: took[name] * Runtime._rounds_of(name, m, cols, pairs) / Runtime._rounds_of(name, rows, cols, pairs) for name in names}
+        best = min(names, key=there.get)
+        return best if choice not in there or there[best] < 0.95 * there[choice] else choice
+
     # Cuts of our kernel that are timed beside the planned one: 100 x (wave tile rows / 32) + 10 x (wave tile
     # columns / 32) + parts of K (+ 1000: workgroups of 8 waves, two a SIMD, on the same 256 x 256 tile; + 2000: those for
     # the whole rounds of 256 tiles and smaller tiles for the columns that are left, + 30000: the smallest for those).  The
@@ -306,7 +320,7 @@ class Runtime:
 
     def _fastest(self, key, ways: dict, same_bits, m: int, cols: int, pairs: bool = False, extra_ms=None):
         """Which of several ways to compute one product of `m` rows and `cols` output columns is taken for the shape `key`: timed once,
-        on the operands at hand (three runs each after a first one), and for other rows of the class by those times (`_rounds_of`).  `ways`: name -> callable, "library"
+        on the operands at hand (three runs each after a first one), and for other rows of the class by those times (`_at_rows`).  `ways`: name -> callable, "library"
         and "plan" among them; `same_bits`: the names whose results are those of "plan" bit for bit;
         `extra_ms`: name -> milliseconds that a way costs its consumer beyond its own kernel (the slabs of a split
         product are read by the kernel that adds them).
@@ -325,10 +339,8 @@ class Runtime:
                 return by_rows[m]
             # (what gives the plan's bits at the rows it was timed at need not at others, where the plan may take other parts of K)
             names = [name for name in took if self.own_prompt_products == "auto" or name in same_bits]
-            if names:       # (at most as many entries as the class has numbers of rows)
-                choice = min(names, key=lambda name: took[name] * self._rounds_of(name, m, cols, pairs) / self._rounds_of(name, rows, cols, pairs))
-            by_rows[m] = choice
-            return choice
+            by_rows[m] = self._at_rows(choice, {name: took[name] for name in names}, rows, m, cols, pairs) if names else choice
+            return by_rows[m]       # (at most as many entries as the class has numbers of rows)
         took = {}
         if self.own_prompt_products is False:
             choice = "library" if "library" in ways else "plan"

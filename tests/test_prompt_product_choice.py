@@ -72,3 +72,16 @@ def test_own_products_are_timed_for_every_number_of_parts(monkeypatch, own):
     assert keys[1100] == keys[1101] and len(set(keys.values())) == (3 if own is True else 1)
     for m, (_, same) in zip(parts, asked):
         assert all(cut % 10 == parts[m] for cut in same if cut != "plan")
+
+
+def test_ways_whose_times_do_not_go_by_rounds_keep_their_rows():
+    """[2,560 x 9,728] as measured at 2,048 rows, the library's the fastest: so it is at 1,536 (157 us; the plan 265).  One of our cuts is
+    left for another where that promises more than 5 %."""
+    took = {"library": 0.186, "plan": 0.205, 441: 0.363, 442: 0.233, 1421: 0.353, 1423: 0.209}
+    for m in (1100, 1536, 1900):
+        assert Runtime._at_rows("library", took, 2048, m, 2560, False) == "library"
+        assert Runtime._at_rows("plan", took, 2048, m, 2560, False) == "plan"
+    ours = {"library": 0.4, 442: 0.1, 444: 0.104}       # tiles in half a round and parts in one: 160 and 320 at 2,048 rows
+    assert Runtime._at_rows(442, ours, 2048, 2047, 2560, False) == 442
+    assert Runtime._at_rows(442, ours, 2048, 1500, 2560, False) == 444              # 240 in one round where 320 were two
+    assert Runtime._at_rows(441, {"plan": 0.4}, 2048, 1500, 2560, False) == "plan"       # nothing else of the same bits
