@@ -27,9 +27,9 @@
 // A position's bits depend on its place in the chunk, so this is for activations that are rounded to bfloat16 behind it; the walk
 // token by token keeps the float32 path, where a portion gives the bits of single tokens.
 //
-// Entries of fewer than `from` tokens are left to that walk: a request's single token gives the same bits, and costs the same, whether
-// another request's prompt is in the step or not.  (128 single tokens beside a prompt of 64: a step of 7 layers, five of them with keys of
-// 128, takes 3,400 us; 4,010 with every entry through the chunks, 3,590 with every entry walked.)
+// Entries of fewer than `from` tokens are left to that walk: a request's single token costs the same whether another request's prompt
+// is in the step or not.  (64 single tokens beside a prompt of 512: a step of 7 layers, five of them with keys of 128, takes 3,750 us;
+// 4,180 with every entry through the chunks, 4,590 with every entry walked.)
 //
 // Rows beyond an entry's last token: g = 1, beta = 0, V = 0, and the last token's q and k in place of theirs.
 #include "common.h"

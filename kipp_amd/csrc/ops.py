@@ -727,9 +727,21 @@ def _scan_args(state, q_start, q_len, slots, o_raw, tokens, heads, d, dv, what):
     _need(q_start.numel() == q_len.numel() == slots.numel(), f"{what}: one start, length and slot an entry")
 
 
-# Entries of so many tokens and more go through a matrix memory a chunk of 64 at a time (`chunks` below), each for itself: the
-# others of the launch walk.  A chunk costs about what the walk takes for a dozen tokens, whether it is full or not.
+# Entries of so many tokens and more go through a matrix memory a chunk of 64 at a time (`chunks` below) in a step whose longest entry
+# pays for the chunks' launches (`matrix_chunks_from`); the others of the step walk.
 CHUNKS_FROM = 16
+
+
+def matrix_chunks_from(mode: int, d: int, state: int) -> int:
+    """Tokens of a step's longest entry from which on chunks are the faster way (mode 0 fixed decays, 1 the delta rule, 2 a decay a token;
+    `state`: numbers of the memories of all the entries that would go by chunks).  In the walk's time, one entry of 16 / 64 / 128 / 256
+    tokens: 8 heads of 128 x 320, fixed 1.63 1.05 0.70 0.47, delta 2.76 1.48 0.99 0.70; 8 of 64 x 128, 1.80 0.95 0.64 0.45 and 2.81 1.43 0.96
+    0.66; 16 of 256 x 256, 1.57 0.98 0.53 0.36 and 2.42 1.42 0.73 0.51.  Sixteen entries: 1.49 0.70 0.56 0.46 and 2.57 1.13 0.94 0.83; 2.09 1.39 0.96 0.81
+    and 2.90 1.69 1.15 0.93; 0.97 0.40 0.34 0.28 and 1.23 0.54 0.46 0.38.  Where single tokens walk beside them that launch comes on top."""
+    many = state >= 1 << 22
+    if mode == 1:
+        return (48 if many else 112) if d >= 192 else 224
+    return 144 if d < 128 else (48 if many else (64 if d >= 192 else 112))
 
 
 def matrix_chunks_ok(d: int) -> bool:
@@ -739,15 +751,15 @@ def matrix_chunks_ok(d: int) -> bool:
 
 def _matrix_chunks(mode, src, q_at, k_at, v_at, beta_at, g_at, decays, state, q_start, q_len, slots, o_raw, heads, qk_rep, d, dv, longest,
                    portions) -> int:
-    """The scan by chunks, for the entries of `CHUNKS_FROM` tokens and more, where it takes the sizes.  Returns the tokens below which
-    entries are left for the walk: 0, it took none; -1, there are no others."""
+    """The scan by chunks, for the entries of `CHUNKS_FROM` tokens and more, where it takes the sizes and is the faster way.  Returns the
+    tokens below which entries are left for the walk: 0, it took none; -1, there are no others."""
     if longest < CHUNKS_FROM or not matrix_chunks_ok(d) or src.shape[1] % 4 or q_at % 4 or k_at % 4 or state.shape[1] % 4 \
             or src.data_ptr() % 16 or state.data_ptr() % 16 or src.shape[0] == 0:
         return 0
     tokens, entries = src.shape[0], q_start.numel()
     every = portions is not None and portions >= entries
     portions = min(entries if portions is None else int(portions), entries, tokens // CHUNKS_FROM)
-    if portions <= 0:
+    if portions <= 0 or longest < matrix_chunks_from(mode, d, portions * heads * d * dv):
         return 0
     size = _fn("linear_chunks", "kipp_matrix_chunks_work", [_c_int] * 5, restype=ctypes.c_longlong)(mode, tokens, portions, heads, d)
     _need(size > 0, "matrix_chunks: sizes the kernel refuses")
@@ -766,9 +778,9 @@ def decay_scan(proj: torch.Tensor, decays: torch.Tensor, state: torch.Tensor, q_
     `state` [slots, size] (float32, S as [head][column][row]).  `proj`: float32 [tokens, >= 2 heads d + heads dv], columns
     q | k | v before their silu; `o_raw` float32 [tokens, heads dv] receives S^T q.  `longest`: the most tokens an entry
     brings, if known (it sizes the kernel's chunks and changes no result).  `chunks`: entries of `CHUNKS_FROM` tokens and more
-    may be taken 64 tokens at a time on the matrix cores, the same float32 sums in another order: a token's last bits then depend on
-    its place in its own entry, and on nothing else in the step (for that `longest` must be known).  `portions`: how many entries bring
-    so many tokens, if known."""
+    may be taken 64 tokens at a time on the matrix cores, the same float32 sums in another order, in steps where that is the faster
+    way (`matrix_chunks_from`; `longest` must be known): a token's last bits then depend on its place in its entry and on which way the
+    step takes; shorter entries always walk.  `portions`: how many entries bring so many tokens, if known."""
     _dev(proj, decays, state, q_start, q_len, slots, o_raw)
     _need(proj.dim() == 2 and proj.dtype == torch.float32 and proj.shape[1] >= 2 * heads * d + heads * dv, "decay_scan: proj is float32 [tokens, q | k | v ...]")
     _need(decays.dtype == torch.float32 and decays.numel() == heads, "decay_scan: float32 decays [heads]")

@@ -9,6 +9,13 @@ DEV = "cuda:0"
 LENGTHS = [64, 1, 65, 15, 16, 130, 17, 63, 200]
 
 
+@pytest.fixture(autouse=True)
+def chunks_wherever_an_entry_may_take_them(monkeypatch):
+    """Here chunks are taken from their first token count on, not from where they are the faster way."""
+    from kipp_amd.csrc import ops
+    monkeypatch.setattr(ops, "matrix_chunks_from", lambda mode, d, state: ops.CHUNKS_FROM)
+
+
 def _plain(mode, q, k, v, beta, g, s):
     """The recurrence over one head's tokens in float64: (o [T, dv], S [d, dv])."""
     out = np.zeros(v.shape)
@@ -103,7 +110,7 @@ def test_few_tokens_and_other_sizes_walk():
 
 @pytest.mark.parametrize("mode", ["decay", "delta", "gated"])
 def test_an_entry_beside_others_is_as_alone(mode):
-    """Every entry of a launch, short or long, in any order of the entries, gives the bits it gives alone: the walk's below
+    """Every entry of a launch by chunks, short or long, in any order of the entries, gives the bits it gives alone: the walk's below
     `CHUNKS_FROM` tokens, the chunks' from there on."""
     import torch
     from kipp_amd.csrc import ops
