@@ -213,8 +213,6 @@ __global__ void __launch_bounds__(KIPP_WAVE) attention_shared_merge_kernel(
 
 extern "C" {
 
-int kipp_attention_shared_runs() { return SH_MAX_RUNS; }
-
 // Rows rows[i] of the batch, i < n_tokens: out [batch rows][heads][d] over cache [pages][1][page][d] (keys and values).  part_acc: float32
 // [n_tokens][n_runs][16][d], part_ml: [n_tokens][n_runs][16][2].  d a multiple of 16 up to 256, at most 16 heads, pages of a power of two.
 int kipp_attention_shared(const void* q, const void* cache, void* out, float* part_acc, float* part_ml, const int32_t* rows, int n_tokens,
