@@ -6,16 +6,19 @@
 //     route (grouped)  s = sigmoid(z), or softmax(z); choice scores c = s + correction; experts in equal groups of neighbours, a
 //              group's score the sum of its two largest c, or its largest; only experts of the `keep` best groups can be chosen; the
 //              `top` largest c among them; weight = s / (sum of the chosen s + eps) * scale, or s * scale (not renormalized)
-//     sort     the (token, choice) pairs in runs of one expert each, cut into tiles of up to 16 (or 128) rows; the list of tiles
+//     sort     the (token, choice) pairs in runs of one expert each, cut into tiles of up to 16 (64, 128, 256) rows; the list of tiles
 //              is made on the device, so the host never learns the counts and the launches have a fixed shape.  The router may
 //              have more outputs than there are experts with matrices: those behind are identity experts, whose pairs get no
 //              row (place -1)
 //     expert   a tile's rows against its expert's matrix: out[row][n] = act(sum_k W_e[n][k] x[row][k]).  bfloat16 with K a
-//              multiple of 32: on the matrix cores, a workgroup a (tile of up to 128 rows, 128 columns), a wave 32 of the
-//              columns in 8 x 2 fragments of 16 x 16 (two workgroups share a compute unit's registers); steps of 64 numbers of k come from memory 128 bytes a row (eight
-//              lanes side by side) into registers while the step before is multiplied out of LDS; a tile of a few rows
-//              (single tokens) multiplies only the fragments it has, and is then bound by the read of its expert's matrix.  Else (float32, other K): a lane takes a column of a tile of 16 rows.
-//              Either way the sum over k runs in one order for every row, so a row's result does not depend on its tile
+//              multiple of 32: on the matrix cores, in three forms.  Few rows an expert (tiles of up to 64): a workgroup 16 columns,
+//              its eight waves every eighth 64 numbers of k each, whose sums are added in order.  Staged (tiles of up to 128): a workgroup
+//              128 columns, 64 numbers of k a step through registers and LDS, one chain of 16 x 16 x 32 products along k.  Walking (tiles of
+//              up to 128 or 256): the walk of the prompt products, 32 x 32 x 16 products along k.  Else (float32, other K): a
+//              lane takes a column of a tile of 16 rows, one chain along k.
+//              A form sums over k in one order for every row, whichever tile the row is in; the forms' orders differ, and the form
+//              follows from the pairs of the whole step and the matrices' sizes: under bfloat16 a token's last bits depend on how
+//              many tokens share its step
 //     gated expert  the same against an expert's [gate; up] matrix with a weight s a row of x:
 //              out[row][n] = act(s (W_gate x)[n]) * s (W_up x)[n], which is the expert applied to s x; on the matrix cores a wave's
 //              two fragments of 16 columns are the gate's and the up's of the same 16 inner columns

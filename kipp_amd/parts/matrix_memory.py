@@ -15,7 +15,8 @@ dual form (`SSDSpec`).
 The recurrences, the gates and the norms run in float32 under either precision; the state is float32.  Under float32 a
 prompt portion walks its tokens in order inside one launch, a single token is a walk of one step of the same kernel, so a
 position's result does not depend on how the tokens were cut.  Under bfloat16 portions of 16 tokens and more go 64 tokens at
-a time where the key size allows and the step's longest portion is long enough: the same float32 sums in another order.
+a time where the key size allows and the step's longest portion is long enough: the same float32 sums in another order, so a
+position's last bits depend on its place in its portion and on the longest portion of its step.
 """
 from __future__ import annotations
 
