@@ -87,7 +87,7 @@ __global__ void latent_prepare_kernel(
         if (e >= q_rank) q_v[i] = 0.0f;
         if (e >= rank) c_v[i] = 0.0f;
         q_w[i] = e < q_rank ? q_norm_w[e] : 0.0f;
-        c_w[i] = e < rank ? c_norm_w[e] : 0.0f;
+        c_w[i] = write_kv && e < rank ? c_norm_w[e] : 0.0f;         // (who writes no row need not have its weights)
     }
     // the shared rotated part, and the numbers of it that are not turned, one by one
     const int pairs = rot_dims / 2;

@@ -73,3 +73,22 @@ def test_ssd_finish(heads, dv, spans):
     ref = (y.view(3, spans, -1) / (y.view(3, spans, -1).square().mean(-1, keepdim=True) + 1e-5).sqrt()).reshape(3, width) * w.double()
     # a handful of float32 roundings and a sum of `span` squares: its relative error at most span / 256 + 10 of them, halved by the root
     assert ((out.double() - ref).abs() <= (ref.abs() + 1e-3) * 2.0 ** -24 * (width / 256 + 30)).all()
+
+
+def test_latent_prepare_without_a_row_to_write():
+    """A run that reads another's cache brings no weights for the row it does not write: the query latent is what it is beside a row, and
+    the cache stays as it was."""
+    from kipp_amd.csrc import ops
+    rng = np.random.default_rng(5)
+    f = lambda *shape: torch.tensor(rng.normal(size=shape), dtype=torch.float32, device="cuda:0")  # noqa: E731
+    i32 = lambda *a: torch.tensor(a, dtype=torch.int32, device="cuda:0")  # noqa: E731
+    proj, q_w, c_w, cache = f(3, 40 + 24 + 8), f(40), f(24), f(2, 1, 16, 32)
+    positions, seq, table, freq = i32(3, 4, 17), i32(0, 0, 0), i32(1, 0).view(1, 2), f(4)
+    there = ops.latent_prepare(proj, torch.empty((3, 40), device="cuda:0"), cache.clone(), positions, seq, table, 40, 24, 8, q_w, c_w, 1e-6, freq, 8, 1.0)
+    before, cq = cache.clone(), torch.empty((3, 40), device="cuda:0")
+    fn = ops._fn("latent", "kipp_latent_prepare", [ops._c_ptr, ops._c_int, ops._c_int, ops._c_ptr, ops._c_ptr, ops._c_float, ops._c_ptr, ops._c_int, ops._c_ptr,
+                                                   ops._c_int, ops._c_ptr, ops._c_ptr, ops._c_ptr, ops._c_int, ops._c_ptr, ops._c_int, ops._c_float]
+                 + [ops._c_int] * 8 + [ops._c_ptr])
+    rc = fn(proj.data_ptr(), 1, proj.shape[1], q_w.data_ptr(), None, 1e-6, cq.data_ptr(), ops._code(cq), cache.data_ptr(), ops._code(cache), positions.data_ptr(),
+            seq.data_ptr(), table.data_ptr(), 2, freq.data_ptr(), 8, 1.0, 0, 3, 40, 40, 24, 8, 16, 0, ops._stream())
+    assert rc == 0 and torch.equal(cq, there) and torch.equal(cache, before)
