@@ -1406,17 +1406,22 @@ def mixed_single_plan(n_tokens: int, max_ctx: int, window: int, keep_first: int)
     return tiles, max(1, min(tiles, 128, -(-4 * COMPUTE_UNITS // mixed_single_tokens(n_tokens, tiles))))
 
 
-# Single tokens beside portions: from so many on (a tile that a token sees counts one, the token itself one more) they take their own
-# form; fewer ride along in the tiles of rows, whose launches are there anyway.  One layer's share of a step of four, us, own form / as
-# tiles, beside a portion of 200: 16 tokens of one tile (32) 398 / 372, 64 (128) 418 / 403, 128 (256) 486 / 514; of 16 tiles: 1 token (17)
-# 382 / 365, 8 (136) 398 / 380, 16 (272) 416 / 436, 64 (1,088) 533 / 636.
-MIXED_SINGLE_BESIDE = 256
+# Single tokens beside portions take their own form from so much work on (a tile of keys that a token sees counts one, the token itself one
+# more), or from less beside this many rows of portions; lighter ones ride along in the tiles of rows, whose launches are there anyway.  A
+# step of four layers (32 heads over 8 of 128), own form / as tiles, us: work 240, 24 tokens behind 500 keys: beside 16 rows 882 / 813, 200 rows 1,422 /
+# 1,336, 456 rows 1,753 / 1,792, 1,000 rows 2,260 / 2,437; 288, 96 behind 60: 1,201 / 1,113, 1,443 / 1,363, 1,910 / 1,903, 2,575 / 2,813, 1,900 rows 4,454 / 4,607;
+# 396, 12 behind 2,000: 960 / 964, 1,502 / 1,514, 1,832 / 1,846, 2,343 / 2,436; 576, 96 behind 250: 1,290 / 1,314, 1,532 / 1,551, 1,976 / 1,977, 2,660 / 2,943;
+# 144, 24 behind 250: 864 / 812, 1,399 / 1,315, 1,734 / 1,640, 2,233 / 2,422, 1,900 rows 4,153 / 4,063.
+MIXED_SINGLE_BESIDE = 400
+MIXED_SINGLE_BESIDE_ROWS, MIXED_SINGLE_BESIDE_MANY = 768, 240
 
 
-def mixed_single_ok(n_q: int, n_kv: int, n_tokens: int, tiles: int, portions: int = 0) -> bool:
-    """Whether `n_tokens` single tokens that see up to `tiles` tiles of keys take their own form in a step with so many `portions`: up to 16
-    query heads a key/value head, and beside portions work enough for launches of its own."""
-    return n_q // n_kv <= 16 and (portions == 0 or n_tokens * (tiles + 1) >= MIXED_SINGLE_BESIDE)
+def mixed_single_ok(n_q: int, n_kv: int, n_tokens: int, tiles: int, portion_rows: int = 0, work: Optional[int] = None) -> bool:
+    """Whether `n_tokens` single tokens that see up to `tiles` tiles of keys take their own form in a step whose portions have so many rows: up
+    to 16 query heads a key/value head, and beside portions work enough (`work`, or every token sees `tiles`) for launches of its own."""
+    work = n_tokens * (tiles + 1) if work is None else work
+    least = 0 if portion_rows == 0 else (MIXED_SINGLE_BESIDE if portion_rows < MIXED_SINGLE_BESIDE_ROWS else MIXED_SINGLE_BESIDE_MANY)
+    return n_q // n_kv <= 16 and work >= least
 
 
 def mixed_single_workspace(n_tokens: int, n_q: int, dv: int, tiles: int, runs: int, device) -> tuple:
