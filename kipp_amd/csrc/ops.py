@@ -1051,11 +1051,15 @@ MOE_TILE_ROWS = 16
 MOE_MFMA_ROWS = 128    # rows of a tile of the experts' products on the matrix cores
 MOE_FEW_ROWS = 64      # the same in the kernel for few rows an expert, which reads the experts' matrices straight into the products
 MOE_MANY_ROWS = 256    # the same where an expert has many rows: its matrix is read less often, a compute unit has one workgroup
-# Pairs an expert (all of them) up to which a step takes the kernel for few rows, in its time over that of tiles of 128, both products,
-# at 4, 6, 8 and 12 pairs: 32 experts of 2,560 x 2,432 gated 0.84 0.88 0.96 1.11, 32 of 4,096 x 3,072 gated 0.98 1.04 1.10 1.21,
-# 16 of 5,120 x 3,200 without a gate 0.89 0.92 1.01 1.13, 8 of 4,096 x 3,584 0.70 0.74 0.79 0.89 (a product with little of K goes by its
-# own rule, in the kernel's launch).
-MOE_FEW_PAIRS = 6
+# A step takes the kernel for few rows up to so many pairs an expert (all of them), and fewer where there is more of the experts' matrices: each 16
+# rows more of an expert are its matrix once more from the caches.  Whole steps of four layers, kernel for few rows over tiles of 128, routed
+# as a trained model routes, at 5, 7, 9, 11, 13 pairs.  Without a gate: 32 experts of 2,560 x 2,432 0.88 0.92 0.95 0.97 0.99, 32 of 4,096 x 3,072
+# 0.94 0.99 1.03 1.06 1.09, 16 of 5,120 x 3,200 0.95 0.98 1.01 1.03 1.05, 16 of 2,560 x 2,432 0.93 .. 1.00; gated: 0.90 0.94 0.98 1.02 1.04, 0.98 1.02 1.07
+# 1.11 1.14, 0.94 0.98 1.02 1.04 1.09, 0.85 .. 0.97; 32 of 5,120 x 6,400, evenly routed, at 3, 5, 7: 1.04 1.09 1.18, gated 0.97 1.05 1.10.  So the
+# pairs times an expert's numbers decide; of many small experts the sides differ (64 of 2,560 x 1,408 0.96 0.98 1.00, gated 1.02 1.05 1.08, 128 of 2,560 x
+# 768 0.97 to 1.00 and 0.94 to 0.99, 256 of 2,560 x 512 0.95 to 0.98, gated 1.02 1.04 1.06): six pairs at most.
+MOE_FEW_PAIRS, MOE_FEW_PAIRS_MANY, MOE_FEW_PAIRS_ALWAYS = 12, 6, 3      # up to 32 experts; more of them; however large
+MOE_FEW_WORK, MOE_FEW_WORK_GATED = 2.4e9, 2.0e9         # pairs of the step times numbers of an expert's way back
 # From how many pairs on a gated step, or one without a gate, takes tiles of 256.  32 experts of 2,560 x 2,432, both products, us: gated with
 # tiles of 128 / 256: 2,048 pairs 314 / 316, 3,200 341 / 343, 4,300 428 / 377, 8,192 564 / 490; without a gate 6,400 340 / 362,
 # 7,600 362 / 362, 8,192 414 / 363, 10,000 409 / 412, 12,288 511 / 458: rounds of workgroups, which the number of tiles decides, and
@@ -1067,16 +1071,19 @@ MOE_MANY_GROUPS = 128
 
 
 def moe_tile_rows(dtype: torch.dtype, *contractions: int, pairs: Optional[int] = None, experts: int = 1, gated: bool = False,
-                  aligned: bool = True) -> int:
+                  aligned: bool = True, identity: int = 0) -> int:
     """Rows of the tiles that the experts' products take: 128 on the matrix cores (bfloat16, every contraction a multiple of
-    32), else 16.  With `pairs`, the (token, choice) pairs of the step: 64 for few of them an expert, 256 for many and for
+    32), else 16.  With `pairs`, the (token, choice) pairs of the step: 64 for few of them an expert (without the share of the
+    `identity` experts, which have no matrices), 256 for many and for
     columns enough of the first product (as many as the last contraction), unless rows or matrices do not begin at multiples of 16
     bytes (`aligned`): those are taken in tiles of 128."""
     if dtype != torch.bfloat16 or any(k % 32 for k in contractions):
         return MOE_TILE_ROWS
     if not aligned:
         return MOE_MFMA_ROWS
-    if pairs is not None and pairs <= MOE_FEW_PAIRS * experts:
+    most = (MOE_FEW_PAIRS if experts <= 32 else MOE_FEW_PAIRS_MANY) * experts
+    work = (MOE_FEW_WORK_GATED if gated else MOE_FEW_WORK) / (max(contractions) * min(contractions))
+    if pairs is not None and pairs * experts / (experts + identity) <= max(min(most, work), MOE_FEW_PAIRS_ALWAYS * experts):
         return MOE_FEW_ROWS
     many = pairs is not None and pairs > (MOE_MANY_PAIRS if gated else MOE_MANY_PAIRS_UNGATED) * experts \
         and (pairs / MOE_MANY_ROWS + experts / 2) * -(-contractions[-1] // (128 if gated else 256)) >= MOE_MANY_GROUPS

@@ -5,10 +5,18 @@ import torch
 from kipp_amd.csrc import ops
 
 
-@pytest.mark.parametrize("experts", [8, 32, 256])
-def test_few_rows_an_expert(experts):
-    for pairs, rows in ((1, 64), (6 * experts, 64), (6 * experts + 1, 128), (12 * experts, 128)):
-        assert ops.moe_tile_rows(torch.bfloat16, 4096, 3072, pairs=pairs, experts=experts) == rows
+@pytest.mark.parametrize("experts,width,inner,gated,most", [(32, 2560, 2432, False, 384), (32, 2560, 2432, True, 321), (8, 4096, 3584, False, 96),
+                                                            (32, 4096, 3072, False, 190), (32, 4096, 3072, True, 158), (32, 5120, 6400, False, 96),
+                                                            (256, 2560, 512, False, 1536), (1, 64, 64, True, 12)])
+def test_few_rows_an_expert(experts, width, inner, gated, most):
+    """Up to a number of pairs that falls with the experts' sizes: by pairs an expert, by the work, never below three an expert."""
+    for pairs, rows in ((1, 64), (most, 64), (most + 1, 128)):
+        assert ops.moe_tile_rows(torch.bfloat16, width, inner, pairs=pairs, experts=experts, gated=gated) == rows
+
+
+def test_identity_experts_take_a_share_of_the_pairs():
+    rows = [ops.moe_tile_rows(torch.bfloat16, 2560, 2432, pairs=n, experts=32, identity=8) for n in (480, 481)]
+    assert rows == [64, 128]
 
 
 def test_many_rows_an_expert():
