@@ -737,11 +737,13 @@ def matrix_chunks_from(mode: int, d: int, state: int) -> int:
     `state`: numbers of the memories of all the entries that would go by chunks).  In the walk's time, one entry of 16 / 64 / 128 / 256
     tokens: 8 heads of 128 x 320, fixed 1.63 1.05 0.70 0.47, delta 2.76 1.48 0.99 0.70; 8 of 64 x 128, 1.80 0.95 0.64 0.45 and 2.81 1.43 0.96
     0.66; 16 of 256 x 256, 1.57 0.98 0.53 0.36 and 2.42 1.42 0.73 0.51.  Sixteen entries: 1.49 0.70 0.56 0.46 and 2.57 1.13 0.94 0.83; 2.09 1.39 0.96 0.81
-    and 2.90 1.69 1.15 0.93; 0.97 0.40 0.34 0.28 and 1.23 0.54 0.46 0.38.  Where single tokens walk beside them that launch comes on top."""
+    and 2.90 1.69 1.15 0.93; 0.97 0.40 0.34 0.28 and 1.23 0.54 0.46 0.38.  Where single tokens walk beside them that launch comes on top.
+    Whole steps of a prompt of 64, 80, 96, 112 tokens, us that chunks take more: two memories of 8 heads of 128 x 320, fixed -7 -21 -36 -53, two with
+    40 of 128 x 64, a decay a token, -1 -9 -15 -21; the delta rule 27 18 2 -7, four prompts of 64, 96, 128, 176 tokens 32 24 18 9."""
     many = state >= 1 << 22
     if mode == 1:
-        return (48 if many else 112) if d >= 192 else 224
-    return 144 if d < 128 else (48 if many else (64 if d >= 192 else 112))
+        return (48 if many else 112) if d >= 192 else (128 if state < 1 << 19 else 224)
+    return 144 if d < 128 else (48 if many else (64 if d >= 192 else 80))
 
 
 def matrix_chunks_ok(d: int) -> bool:

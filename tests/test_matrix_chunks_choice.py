@@ -7,11 +7,11 @@ DECAY, DELTA, GATED = 0, 1, 2
 
 
 @pytest.mark.parametrize("mode, heads, d, dv, entries, walks, chunks", [
-    (DECAY, 8, 128, 320, 1, 96, 128), (DELTA, 8, 128, 320, 1, 128, 256), (GATED, 40, 128, 64, 1, 96, 128), (GATED, 40, 128, 64, 16, 32, 48),
+    (DECAY, 8, 128, 320, 1, 64, 96), (DELTA, 8, 128, 320, 1, 112, 128), (DELTA, 8, 128, 320, 4, 176, 256), (GATED, 40, 128, 64, 1, 64, 96), (GATED, 40, 128, 64, 16, 32, 48),
     (DECAY, 8, 64, 128, 16, 112, 160), (DELTA, 8, 64, 128, 16, 192, 256), (DECAY, 16, 256, 256, 1, 48, 64), (DELTA, 16, 256, 256, 4, 32, 48),
     (DELTA, 4, 192, 64, 1, 96, 128), (DELTA, 32, 128, 128, 4, 160, 256)])
 def test_where_chunks_were_the_faster_way(mode, heads, d, dv, entries, walks, chunks):
-    """Steps whose longest entry has `walks` tokens walk, with `chunks` they take chunks: at those the chunks were the faster way by themselves
-    and with a walk of single tokens beside them; at a few of the former they were by themselves."""
+    """Steps whose longest entry has `walks` tokens walk, with `chunks` they take chunks: at those the chunks were the faster way, and no
+    slower with a walk of single tokens beside them; at a few of the former they were by themselves."""
     start = ops.matrix_chunks_from(mode, d, entries * heads * d * dv)
     assert walks < start <= chunks and start >= ops.CHUNKS_FROM
