@@ -8,22 +8,28 @@
 // instructions, four numbers of k each (16 j + i, + 4, + 8, + 12 for i = 0..3, j counting up from the run's start), and the runs' sums are added
 // in order.  Both kernels below do exactly that, W always the instruction's first operand and X its second.
 //
-//   rows   up to 64 rows of X a workgroup: 16 rows of W, a wave a run of K, straight from memory into the instruction's
+//   rows   up to 16 rows of X a workgroup: 16 rows of W, a wave a run of K, straight from memory into the instruction's
 //          operands (16 bytes a lane), the runs' sums added through LDS.  Bound by the read of W.  A 16-column fragment of
 //          X is multiplied whether its rows are there or not: at one row the matrix cores could feed 19 TB/s.
-//   tiles  64 x 64 outputs a workgroup, a wave 32 x 32, X and W staged through LDS 32 numbers of k at a time, the next
-//          step's on their way in registers.  Bound by the instruction's rate and, below a few hundred tiles, by idle
-//          compute units.
-// Measured at the 4B shape, before (one plain FMA chain an output, 64 x 64 tiles at every M) and now: one row against 19,456 x 2,560
-// 402 and 46 us (4.3 TB/s), 2,560 x 9,728 1,160 and 34 us, the head's 151,936 x 2,560 913 and 325 us (4.8 TB/s);
-// 333 rows against 19,456 x 2,560 614 and 422 us (79 TFLOP/s), 2,560 x 9,728 1,220 and 274 us (240 tiles for 256 compute units).
+//   tiles  more rows: 64 or 32 rows of W times 64, 48 or 32 of X a workgroup, a wave a run of K here too, so that every wave of a
+//          workgroup multiplies all of its outputs and none waits for another in the walk.  Bound by the instruction's rate (80 %
+//          of it at 1,024 rows) and, below a few rounds of tiles, by what the last round leaves idle: the shape goes by that.
+// Measured at the 4B shape, W in turn from three copies, us: one row against 19,456 x 2,560 46 (4.3 TB/s), 2,560 x 9,728 34, the head's
+// 151,936 x 2,560 325 (4.8 TB/s).  The tiles, against 19,456 x 2,560 / 6,144 x 2,560 / 2,560 x 4,096 / 2,560 x 9,728, beside what these
+// rows took before (up to 64 rows of X through the kernel for rows, 64 x 64 tiles of four waves that share a step of K beyond):
+//      32 rows    56 / 16 / 20 / 49      106 / 36 / 28 / 73
+//      64 rows    78 / 27 / 21 / 49      171 / 64 / 46 / 115
+//     128 rows   125 / 45 / 31 / 68      156 / 71 / 92 / 219
+//     333 rows   305 / 100 / 69 / 157    402 / 153 / 114 / 271     (110 TFLOP/s; 68 to 83)
+//   1,024 rows   814 / 257 / 183 / 454   957 / 308 / 240 / 566
+// Without the walk's requests for the next steps the same tiles reach 127 TFLOP/s, without its writes into LDS either 139; operands straight
+// from memory into registers, 16 rows of 64 bytes a request, 65 to 85; all sixteen requests of a step behind one another 77 to 100.
 #include "common.h"
 
 #define KPARTS 8
-#define STEP 32             // numbers of k a tile step brings into LDS; a run is a multiple of it
-#define TILE 64
-#define PITCH 36            // floats from a row to the next in LDS: 16 bytes a lane spread over the banks
-#define THREADS 256
+#define STEP 32             // numbers of k a tile's wave asks for together; a run is a multiple of it
+#define UNITS 256           // compute units
+#define XCDS 8              // dies of the chip; consecutive workgroups of a launch go to them in turn
 #define ROWS_THREADS (KPARTS * KIPP_WAVE)
 
 typedef __attribute__((ext_vector_type(4))) float f32x4;
@@ -66,6 +72,20 @@ __device__ __forceinline__ f32x4 four(const bf16_t* __restrict__ row, int k, int
     return v;
 }
 
+// The same where all four are inside the row.
+template <bool VEC>
+__device__ __forceinline__ f32x4 four_inside(const float* __restrict__ at) {
+    if (VEC) return *reinterpret_cast<const f32x4*>(at);
+    return (f32x4){at[0], at[1], at[2], at[3]};
+}
+
+template <bool VEC>
+__device__ __forceinline__ f32x4 four_inside(const bf16_t* __restrict__ at) {
+    if (!VEC) return (f32x4){bf16_to_f32(at[0]), bf16_to_f32(at[1]), bf16_to_f32(at[2]), bf16_to_f32(at[3])};
+    const uint2 u = *reinterpret_cast<const uint2*>(at);
+    return (f32x4){__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xffff0000u), __uint_as_float(u.y << 16), __uint_as_float(u.y & 0xffff0000u)};
+}
+
 // 16 numbers of k: lane l holds those at 4 (l / 16) .. + 3 of row l % 16 of either operand.
 __device__ __forceinline__ f32x4 mul16(f32x4 w, f32x4 x, f32x4 acc) {
 #pragma unroll
@@ -74,167 +94,212 @@ __device__ __forceinline__ f32x4 mul16(f32x4 w, f32x4 x, f32x4 acc) {
 }
 
 // The sums of a fragment lie in lane l as rows 4 (l / 16) .. + 3 (of W) of column l % 16 (a row of X).
-template <typename TW, int MT, bool VEC>
+template <typename TW, bool VEC>
 __global__ void __launch_bounds__(ROWS_THREADS)
 gemm_f32_rows_kernel(const float* __restrict__ X, const TW* __restrict__ W, float* __restrict__ Y, int M, int N, int K) {
-    __shared__ __attribute__((aligned(16))) float part_s[KPARTS][MT][KIPP_WAVE][4];
+    __shared__ __attribute__((aligned(16))) float part_s[KPARTS][KIPP_WAVE][4];
     const int wave = threadIdx.x / KIPP_WAVE, lane = threadIdx.x & (KIPP_WAVE - 1);
     const int l16 = lane & 15, h4 = 4 * (lane >> 4);
-    const int n0 = blockIdx.x * 16, m0 = blockIdx.y * (16 * MT);
+    const int blocks = (N + 15) / 16, n0 = blockIdx.x % blocks * 16, m0 = blockIdx.x / blocks * 16;
     const TW* w_row = W + (size_t)min(n0 + l16, N - 1) * K;         // rows beyond the last read it and are not stored
-    const float* x_row[MT];
-#pragma unroll
-    for (int i = 0; i < MT; ++i) x_row[i] = X + (size_t)min(m0 + 16 * i + l16, M - 1) * K;
+    const float* x_row = X + (size_t)min(m0 + l16, M - 1) * K;
     const int part = part_of(K);
     const int k_lo = wave * part, k_hi = min(K, k_lo + part);
-    f32x4 acc[MT];
-#pragma unroll
-    for (int i = 0; i < MT; ++i) acc[i] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
-    constexpr int AHEAD = MT == 1 ? 8 : (MT == 2 ? 6 : 4);       // 16-number pieces asked for together
+    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    constexpr int AHEAD = 8;       // 16-number pieces asked for together
     int k = k_lo;
     for (; k + 16 * AHEAD <= k_hi; k += 16 * AHEAD) {
-        f32x4 w[AHEAD], x[AHEAD][MT];
+        f32x4 w[AHEAD], x[AHEAD];
 #pragma unroll
         for (int j = 0; j < AHEAD; ++j) {
             w[j] = four<VEC>(w_row, k + 16 * j + h4, K);
-#pragma unroll
-            for (int i = 0; i < MT; ++i) x[j][i] = four<VEC>(x_row[i], k + 16 * j + h4, K);
+            x[j] = four<VEC>(x_row, k + 16 * j + h4, K);
         }
 #pragma unroll
-        for (int j = 0; j < AHEAD; ++j)
-#pragma unroll
-            for (int i = 0; i < MT; ++i) acc[i] = mul16(w[j], x[j][i], acc[i]);
+        for (int j = 0; j < AHEAD; ++j) acc = mul16(w[j], x[j], acc);
     }
     for (; k < k_hi; k += 16) {
         const f32x4 w = four<VEC>(w_row, k + h4, K);
-#pragma unroll
-        for (int i = 0; i < MT; ++i) acc[i] = mul16(w, four<VEC>(x_row[i], k + h4, K), acc[i]);
+        acc = mul16(w, four<VEC>(x_row, k + h4, K), acc);
     }
-#pragma unroll
-    for (int i = 0; i < MT; ++i) *reinterpret_cast<f32x4*>(part_s[wave][i][lane]) = acc[i];
+    *reinterpret_cast<f32x4*>(part_s[wave][lane]) = acc;
     __syncthreads();
     // a thread an output: the runs' sums in order
-    for (int e = threadIdx.x; e < MT * 256; e += ROWS_THREADS) {
-        const int i = e >> 8, at = e & 255;             // fragment; place in it: column 16 numbers of n long
-        const int n = n0 + (at & 15), m = m0 + 16 * i + (at >> 4);
+    if (threadIdx.x < 256) {
+        const int at = threadIdx.x;             // place in the fragment: column 16 numbers of n long
+        const int n = n0 + (at & 15), m = m0 + (at >> 4);
         const int from = 16 * ((at & 15) >> 2) + (at >> 4);
         float total = 0.0f;
 #pragma unroll
-        for (int p = 0; p < KPARTS; ++p) total += part_s[p][i][from][at & 3];
+        for (int p = 0; p < KPARTS; ++p) total += part_s[p][from][at & 3];
         if (m < M && n < N) Y[(size_t)m * N + n] = total;
     }
 }
 
-template <typename TW, bool VEC>
-__global__ void __launch_bounds__(THREADS)
-gemm_f32_tiles_kernel(const float* __restrict__ X, const TW* __restrict__ W, float* __restrict__ Y, int M, int N, int K) {
-    __shared__ __attribute__((aligned(16))) float w_s[2][TILE * PITCH];
-    __shared__ __attribute__((aligned(16))) float x_s[2][TILE * PITCH];
-    const int tid = threadIdx.x;
-    const int wave = tid / KIPP_WAVE, lane = tid & (KIPP_WAVE - 1);
+// A wave stages its own steps of 32 numbers of k in its own part of LDS, so no wave waits for another before the sums.  A row's 128
+// bytes lie at 128 times the row in it, 16 byte piece c at place c ^ (row / 2 mod 8): reads and writes then meet every bank once.
+template <typename TW, int NT, int MT, bool VEC>
+__global__ void __launch_bounds__(ROWS_THREADS, 2)
+gemm_f32_tiles_kernel(const float* __restrict__ X, const TW* __restrict__ W, float* __restrict__ Y, int M, int N, int K, int n_tiles, int m_tiles) {
+    constexpr int ROWS = 16 * (NT + MT), LOADS = ROWS / 8, READS = NT + MT, STAGE = ROWS * STEP, PRODUCTS = 4 * NT * MT;
+    __shared__ __attribute__((aligned(16))) float lds[KPARTS * (STAGE > NT * MT * 256 ? STAGE : NT * MT * 256)];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / KIPP_WAVE), lane = threadIdx.x & (KIPP_WAVE - 1);
     const int l16 = lane & 15, h4 = 4 * (lane >> 4);
-    const int n0 = blockIdx.x * TILE, m0 = blockIdx.y * TILE;
-    const int wn = (wave & 1) * 32, wm = (wave >> 1) * 32;
-    // from memory a thread takes 16 bytes of rows tid / 8 and tid / 8 + 32: eight lanes a row's 128 bytes
-    const int ld_row = tid >> 3, ld_k = (tid & 7) * 4;
-    const TW* w_row[2];
-    const float* x_row[2];
+    // workgroups id, id + 8, .. share a die and its L2: a die takes a run of tiles, those of the same rows of W one after the other
+    const int tiles = n_tiles * m_tiles, per_die = (tiles + XCDS - 1) / XCDS;
+    const int turn = blockIdx.x / XCDS, tile = (blockIdx.x % XCDS) * per_die + turn;
+    if (turn >= per_die || tile >= tiles) return;       // uniform over the workgroup
+    // The last rows of W are a whole tile that ends with them (the launcher has checked that there are so many): outputs that two
+    // tiles have are the same bits in both.
+    const int n0 = min(tile / m_tiles * (16 * NT), N - 16 * NT), m0 = tile % m_tiles * (16 * MT);
+    // From memory a lane takes four numbers, eight lanes a row's 32: load i brings rows 8 i + lane / 8, first W's, then X's.
+    const TW* w_base = W + (size_t)n0 * K;
+    const float* x_base = X + (size_t)m0 * K;
+    const int ld_row = lane >> 3, ld_k = 4 * (lane & 7);
+    const uint32_t w_src = (uint32_t)ld_row * (uint32_t)K + ld_k;
+    uint32_t x_src[2 * MT];             // rows of X beyond the last read it and are not stored
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        w_row[i] = W + (size_t)min(n0 + ld_row + 32 * i, N - 1) * K;
-        x_row[i] = X + (size_t)min(m0 + ld_row + 32 * i, M - 1) * K;
+    for (int i = 0; i < 2 * MT; ++i) x_src[i] = (uint32_t)min(8 * i + ld_row, M - 1 - m0) * (uint32_t)K + ld_k;
+    float* stage = lds + wave * STAGE;
+    float* put_at[2];                   // of even and odd i
+    const float* take_at[2];            // of a step's two halves
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        put_at[j] = stage + ld_row * STEP + (ld_k ^ (4 * ((4 * j + (ld_row >> 1)) & 7)));
+        take_at[j] = stage + l16 * STEP + ((16 * j + h4) ^ (4 * ((l16 >> 1) & 7)));
     }
-    f32x4 w_r[2], x_r[2];
-    auto fetch = [&](int k0) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            w_r[i] = four<VEC>(w_row[i], k0 + ld_k, K);
-            x_r[i] = four<VEC>(x_row[i], k0 + ld_k, K);
-        }
-    };
-    auto stage = [&](int buf) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            *reinterpret_cast<f32x4*>(&w_s[buf][(ld_row + 32 * i) * PITCH + ld_k]) = w_r[i];
-            *reinterpret_cast<f32x4*>(&x_s[buf][(ld_row + 32 * i) * PITCH + ld_k]) = x_r[i];
-        }
-    };
-    f32x4 acc[2][2], total[2][2];
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b) acc[a][b] = total[a][b] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
     const int part = part_of(K);
-    int until = part;           // where the run under way ends
-    fetch(0);
-    stage(0);
-    __syncthreads();
-    int buf = 0;
-    for (int k0 = 0; k0 < K; k0 += STEP, buf ^= 1) {
-        const bool more = k0 + STEP < K;
-        if (more) fetch(k0 + STEP);
+    const int k_lo = wave * part, k_hi = min(K, k_lo + part);
+    f32x4 acc[NT][MT];
 #pragma unroll
-        for (int j = 0; j < STEP; j += 16) {
-            if (k0 + j >= K) break;
-            f32x4 w[2], x[2];
+    for (int a = 0; a < NT; ++a)
 #pragma unroll
-            for (int a = 0; a < 2; ++a) {
-                w[a] = *reinterpret_cast<const f32x4*>(&w_s[buf][(wn + 16 * a + l16) * PITCH + j + h4]);
-                x[a] = *reinterpret_cast<const f32x4*>(&x_s[buf][(wm + 16 * a + l16) * PITCH + j + h4]);
-            }
-            // the four sums side by side: an instruction does not wait for the one before
+        for (int b = 0; b < MT; ++b) acc[a][b] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+    f32x4 next[LOADS], op[2][READS];    // a step on its way; operands of the two halves of the one that is multiplied, W's and then X's
+    auto fetch = [&](int i, int k0) {
+        next[i] = i < 2 * NT ? four_inside<VEC>(w_base + ((size_t)(8 * i) * K + k0) + w_src)
+                             : four_inside<VEC>(x_base + k0 + x_src[i < 2 * NT ? 0 : i - 2 * NT]);
+    };
+    auto put = [&](int i) { *reinterpret_cast<f32x4*>(put_at[i & 1] + 8 * i * STEP) = next[i]; };
+    auto take = [&](int j, int r) { op[j][r] = *reinterpret_cast<const f32x4*>(take_at[j] + 16 * r * STEP); };
+    // The sums side by side: an instruction does not wait for the one before.
+    auto product = [&](int j, int p) {
+        const int i = p / (NT * MT), a = p / MT % NT, b = p % MT;
+        acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(op[j][a][i], op[j][NT + b][i], acc[a][b], 0, 0, 0);
+    };
+    // A step's first half is in registers when its products begin.  Behind them go, one at a time, the reads of its second half, then a
+    // write of the next step into LDS with the request for the same piece of the one after it; behind the second half's products the
+    // reads of the next step's first half.  (The two waves of a SIMD begin together, so neither fills the other's gaps, and sixteen
+    // requests behind one another held every wave up for a quarter of its step.)  The order is pinned, or the compiler gathers them.
+    const int steps = k_hi > k_lo ? (k_hi - k_lo) / STEP : 0, last = k_lo + (steps - 1) * STEP;
+    if (steps > 0) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < LOADS; ++i) fetch(i, k_lo);
 #pragma unroll
-                for (int a = 0; a < 2; ++a)
-#pragma unroll
-                    for (int b = 0; b < 2; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[a][i], x[b][i], acc[a][b], 0, 0, 0);
+        for (int i = 0; i < LOADS; ++i) {
+            put(i);
+            fetch(i, min(k_lo + STEP, last));
         }
-        if (k0 + STEP == until || !more) {
-            until += part;
 #pragma unroll
-            for (int a = 0; a < 2; ++a)
+        for (int r = 0; r < READS; ++r) take(0, r);
+        for (int k0 = k_lo; k0 <= last; k0 += STEP) {       // behind the last step it is asked for again
+            const int ahead = min(k0 + 2 * STEP, last);
+            constexpr int ITEMS = READS + LOADS;
 #pragma unroll
-                for (int b = 0; b < 2; ++b) {
-                    total[a][b] += acc[a][b];
-                    acc[a][b] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+            for (int p = 0; p < PRODUCTS; ++p) {
+                product(0, p);
+#pragma unroll
+                for (int q = p * ITEMS / PRODUCTS; q < (p + 1) * ITEMS / PRODUCTS; ++q) {
+                    if (q < READS) {
+                        take(1, q);
+                    } else {
+                        put(q - READS);
+                        fetch(q - READS, ahead);
+                    }
                 }
-        }
-        if (more) stage(buf ^ 1);
-        __syncthreads();
-    }
+                __builtin_amdgcn_sched_barrier(0);
+            }
 #pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b) {
-            const int m = m0 + wm + 16 * b + l16, n = n0 + wn + 16 * a + h4;
-            if (m >= M) continue;
-            float* y = Y + (size_t)m * N + n;
-            if ((N & 3) == 0 && ((uintptr_t)Y & 15) == 0) {
-                if (n < N) *reinterpret_cast<f32x4*>(y) = total[a][b];
-            } else {
-#pragma unroll
-                for (int v = 0; v < 4; ++v)
-                    if (n + v < N) y[v] = total[a][b][v];
+            for (int p = 0; p < PRODUCTS; ++p) {
+                product(1, p);
+                if (p < READS) take(0, p);
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
+    }
+    const int rest = k_lo + steps * STEP;
+    if (rest < k_hi) {                              // what K leaves of a step
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) {
+            next[i] = i < 2 * NT ? four<VEC>(w_base + (size_t)(8 * i + ld_row) * K, rest + ld_k, K)
+                                 : four<VEC>(x_base + x_src[i < 2 * NT ? 0 : i - 2 * NT] - ld_k, rest + ld_k, K);
+            put(i);
+        }
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            if (rest + 16 * j >= k_hi) continue;
+#pragma unroll
+            for (int r = 0; r < READS; ++r) take(j, r);
+#pragma unroll
+            for (int p = 0; p < PRODUCTS; ++p) product(j, p);
+        }
+    }
+    __syncthreads();                                // every wave is done with its part of LDS
+    f32x4(*part_s)[NT * MT][KIPP_WAVE] = reinterpret_cast<f32x4(*)[NT * MT][KIPP_WAVE]>(lds);
+#pragma unroll
+    for (int a = 0; a < NT; ++a)
+#pragma unroll
+        for (int b = 0; b < MT; ++b) part_s[wave][a * MT + b][lane] = acc[a][b];
+    __syncthreads();
+    const bool fours = (N & 3) == 0 && ((uintptr_t)Y & 15) == 0;
+    for (int f = wave; f < NT * MT; f += KPARTS) {      // a wave a fragment: the runs' sums in order
+        f32x4 total = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int p = 0; p < KPARTS; ++p) total += part_s[p][f][lane];
+        const int m = m0 + 16 * (f % MT) + l16, n = n0 + 16 * (f / MT) + h4;
+        if (m >= M) continue;
+        float* y = Y + (size_t)m * N + n;
+        if (fours) {
+            *reinterpret_cast<f32x4*>(y) = total;
+        } else {
+#pragma unroll
+            for (int v = 0; v < 4; ++v) y[v] = total[v];
+        }
+    }
+}
+
+template <typename TW, int NT, int MT, bool VEC>
+static void launch_tiles(const float* X, const TW* W, float* Y, int M, int N, int K, hipStream_t stream) {
+    const int n_tiles = (N + 16 * NT - 1) / (16 * NT), m_tiles = (M + 16 * MT - 1) / (16 * MT);
+    const int grid = (n_tiles * m_tiles + XCDS - 1) / XCDS * XCDS;
+    hipLaunchKernelGGL((gemm_f32_tiles_kernel<TW, NT, MT, VEC>), dim3(grid), dim3(ROWS_THREADS), 0, stream, X, W, Y, M, N, K, n_tiles, m_tiles);
+}
+
+// What the busiest compute unit takes for its tiles of nt x mt, one after the other, in products of one fragment: a tile's first requests
+// and its sums cost two of them whatever it is (measured with K of 2,560, 4,096 and 9,728, us a round of tiles: 4 x 4 45, 64, 146;
+// 4 x 3 35, 50, 114; 4 x 2 25, 36, 81; 2 x 3 20, 29, 65; 2 x 2 15, 21, 49).
+static long long tile_price(int M, int N, int nt, int mt) {
+    const long long tiles = (long long)((N + 16 * nt - 1) / (16 * nt)) * ((M + 16 * mt - 1) / (16 * mt));
+    return (tiles + UNITS - 1) / UNITS * (nt * mt + 2);
 }
 
 template <typename TW, bool VEC>
 static int launch(const float* X, const TW* W, float* Y, int M, int N, int K, hipStream_t stream) {
-    const int m_tiles = (M + TILE - 1) / TILE, n_tiles = (N + TILE - 1) / TILE;
-    // Tiles need a workgroup for most of the 256 compute units; the other kernel has N / 16 workgroups for 64 rows, but
-    // reads each of its operands from the caches for 16 rows of W only.
-    if (M <= 64 || (M <= 256 && m_tiles * n_tiles < 192)) {
-        const dim3 block(ROWS_THREADS);
-        const int nb = (N + 15) / 16;
-#define KIPP_ROWS(MT) hipLaunchKernelGGL((gemm_f32_rows_kernel<TW, MT, VEC>), dim3(nb, (M + 16 * MT - 1) / (16 * MT)), block, 0, stream, X, W, Y, M, N, K)
-        if (M <= 16) KIPP_ROWS(1);
-        else if (M <= 32) KIPP_ROWS(2);
-        else KIPP_ROWS(4);
-#undef KIPP_ROWS
-    } else {
-        hipLaunchKernelGGL((gemm_f32_tiles_kernel<TW, VEC>), dim3(n_tiles, m_tiles), dim3(THREADS), 0, stream, X, W, Y, M, N, K);
+    if (M <= 16 || N < 32) {        // tiles hold 32 rows of W or more
+        hipLaunchKernelGGL((gemm_f32_rows_kernel<TW, VEC>), dim3((N + 15) / 16 * ((M + 15) / 16)), dim3(ROWS_THREADS), 0, stream, X, W, Y, M, N, K);
+        return KIPP_LAUNCH_CHECK();
+    }
+    static const int shapes[5][2] = {{4, 4}, {4, 3}, {4, 2}, {2, 3}, {2, 2}};
+    int best = 4;
+    for (int i = 3; i >= 0; --i)
+        if (N >= 64 || shapes[i][0] == 2)
+            if (tile_price(M, N, shapes[i][0], shapes[i][1]) <= tile_price(M, N, shapes[best][0], shapes[best][1])) best = i;
+    switch (best) {
+        case 0: launch_tiles<TW, 4, 4, VEC>(X, W, Y, M, N, K, stream); break;
+        case 1: launch_tiles<TW, 4, 3, VEC>(X, W, Y, M, N, K, stream); break;
+        case 2: launch_tiles<TW, 4, 2, VEC>(X, W, Y, M, N, K, stream); break;
+        case 3: launch_tiles<TW, 2, 3, VEC>(X, W, Y, M, N, K, stream); break;
+        default: launch_tiles<TW, 2, 2, VEC>(X, W, Y, M, N, K, stream); break;
     }
     return KIPP_LAUNCH_CHECK();
 }

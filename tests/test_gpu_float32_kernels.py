@@ -36,6 +36,20 @@ def test_product_rows_are_the_same_in_both_kernels(n, k):
     assert torch.equal(got, again)          # a weight in bfloat16 is widened exactly
 
 
+@pytest.mark.parametrize("m, n", [(17, 32), (33, 47), (49, 2579), (97, 2570), (350, 3001), (333, 2570), (200, 6155)])
+@pytest.mark.parametrize("k", [40, 268])
+def test_product_in_every_shape_of_tiles(m, n, k):
+    """Sizes that the rule gives to tiles of 32 x 32, 32 x 48, 64 x 32, 64 x 48 and 64 x 64, with parts of tiles at both ends and
+    of a step of K: every row as the kernel for up to 16 rows makes it, whose sums the test above holds to float64."""
+    import torch
+    from kipp_amd.csrc import ops
+    gen = torch.Generator().manual_seed(m + n + k)
+    x, w = torch.randn((m, k), generator=gen).to(DEV), torch.randn((n, k), generator=gen).to(DEV)
+    full = ops.gemm_f32(x, w, torch.empty((m, n), device=DEV))
+    for lo in sorted({0, m // 2, m - 16}):
+        assert torch.equal(ops.gemm_f32(x[lo:lo + 16].contiguous(), w, torch.empty((min(16, m - lo), n), device=DEV)), full[lo:lo + 16]), lo
+
+
 def test_product_of_rows_that_begin_anywhere():
     """Operands at addresses that 16-byte loads do not take."""
     import torch
