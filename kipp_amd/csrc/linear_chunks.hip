@@ -8,10 +8,14 @@
 //     o = G (Q S) + A U                          A[t][s] = D[t][s] q_t . k_s for s <= t
 //     S <- G_last S + K^T (D[last][s] U)
 //
-// which is the walk's sums in another order.  D is made by running products (a decay of zero stays one), never by
-// quotients.  Three launches:
+// and an mLSTM is a decay a token and head, g = exp(lf + m - m'), with U = exp(li - m') V and one more column of S, of values of one: n, whose
+// o is what the others are divided by.
+//
+// These are the walk's sums in another order.  D is made by running products (a decay of zero stays one), never by
+// quotients.  Two or three launches:
 //
 //     ready    (decay only) silu of q and k, once
+//     gates    (mLSTM only) m, and what follows from it
 //     prepare  a workgroup (chunk, head, entry): A, T = (I + L)^-1 by forward substitution (a lane a column), G and
 //              D[last]; every chunk of the launch at once
 //     walk     a workgroup (16 columns of S, head, entry) takes its chunks in order.  S stays in registers as the
@@ -22,7 +26,8 @@
 // Bound by the walk's chain: at keys of 128 a chunk is 80 instructions of 32 cycles a wave (delta: 128), the sums in between
 // and two or three barriers, 3.8 us a chunk with 160 workgroups on 256 compute units.  2,048 tokens of 8 heads, keys of 128,
 // values of 320: 145 us (124 the walk) with a fixed decay, 193 (168) for the delta rule, where the walk token by token takes 772
-// and 663; 1,801 tokens of 40 heads with a state of 128 x 64: 120 (99), was 560.
+// and 663; 1,801 tokens of 40 heads with a state of 128 x 64: 120 (99), was 560.  An mLSTM of 8 heads of 128 x 320, all launches: one entry of 64,
+// 1,024, 2,048 tokens 22, 80, 137, eight of 150 70, where its walk takes 29, 378, 751, 186; of 256 x 512 39, 206, 376, 175 and 42, 591, 1,178, 722.
 //
 // A position's bits depend on its place in the chunk, so this is for activations that are rounded to bfloat16 behind it; the walk
 // token by token keeps the float32 path, where a portion gives the bits of single tokens.
@@ -40,7 +45,14 @@
 #define UP 68               // floats from a column to the next of U and R in LDS
 #define COLS 16             // columns of S a workgroup of the walk
 
-enum { MODE_DECAY = 0, MODE_DELTA = 1, MODE_GATED = 2 };
+#define VECS 4              // vectors of 64 numbers a chunk and head
+
+enum { MODE_DECAY = 0, MODE_DELTA = 1, MODE_GATED = 2, MODE_MLSTM = 3 };
+
+// Runs that a contraction over the key size is summed in, every RUNS-th 16 numbers one, then in pairs: an mLSTM divides by a sum that may
+// almost cancel, so its sums are kept as short as the walk's (errors of its rows against 64 bits, median over 1,100 tokens of 128 x 320: 1.66e-7
+// in one run, 1.44e-7 in two, 1.31e-7 in four, 1.52e-7 by the walk; 600 tokens of 256 x 64: 2.6e-7, 2.1e-7, 1.8e-7, 1.5e-7 in eight, 1.5e-7).
+constexpr int runs_of(int mode, int dt) { return mode != MODE_MLSTM ? 1 : (dt == 4 ? 8 : 4); }
 
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 
@@ -52,6 +64,18 @@ __device__ __forceinline__ f32x4 mul16(f32x4 a, f32x4 b, f32x4 acc) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[i], acc, 0, 0, 0);
     return acc;
+}
+
+template <int RUNS, int N>
+__device__ __forceinline__ f32x4 sum_runs(const f32x4 (&runs)[RUNS][N], int n) {
+    f32x4 sum[RUNS];
+#pragma unroll
+    for (int h = 0; h < RUNS; ++h) sum[h] = runs[h][n];
+#pragma unroll
+    for (int w = 1; w < RUNS; w <<= 1)
+#pragma unroll
+        for (int h = 0; h + w < RUNS; h += 2 * w) sum[h] += sum[h + w];
+    return sum[0];
 }
 
 __device__ __forceinline__ f32x4 zero4() { return (f32x4){0.0f, 0.0f, 0.0f, 0.0f}; }
@@ -97,8 +121,14 @@ struct ChunkArgs {
     size_t state_stride;
     const int32_t *q_start, *q_len, *slots;
     float* o_raw;
-    float *a, *t, *vec;         // [chunk][head][64][64], the same (delta), [chunk][head][3][64]: G, D[last], beta
-    int heads, qk_rep, dv, entries, from;
+    float *a, *t, *vec;         // [chunk][head][64][64], the same (delta), [chunk][head][4][64]: G, D[last], beta (mLSTM: the input gate), mLSTM's floor of a denominator
+    int heads, qk_rep, d, dv, entries, from;
+    // mLSTM: the gates' columns and biases, their cap, where a slot's copies of n begin and how many there are, 1 / sqrt(d), and what a
+    // token's sums are divided by, [token][head]
+    const float *bias_i, *bias_f;
+    int i_at, f_at, n_at, copies;
+    float cap, q_scale;
+    float* den;
 };
 
 __global__ void __launch_bounds__(THREADS)
@@ -109,6 +139,75 @@ chunks_ready_kernel(const float* __restrict__ src, int stride, float* __restrict
 #pragma unroll
     for (int i = 0; i < 4; ++i) v[i] = silu_f(v[i]);
     *reinterpret_cast<f32x4*>(out + (size_t)blockIdx.y * width + c) = v;
+}
+
+__device__ __forceinline__ float log_sigmoid(float z) { return fminf(z, 0.0f) - log1pf(expf(-fabsf(z))); }
+
+#define GATE_WAVES 16
+
+// The gates of an mLSTM head: m' = max(lf + m, li) is an affine step of (max, +), so a wave scans 64 tokens in six exchanges and the
+// waves' results are joined through LDS: 1,024 tokens a turn.  Leaves a token's decay (in G's place), input gate and floor.  For an entry
+// that walks it writes the ones that its finished sums are divided by.
+__global__ void __launch_bounds__(GATE_WAVES * KIPP_WAVE) chunks_gates_kernel(const ChunkArgs p) {
+    __shared__ float a_s[GATE_WAVES], b_s[GATE_WAVES];
+    const int head = blockIdx.x, entry = blockIdx.y, tid = threadIdx.x;
+    const int wave = tid / KIPP_WAVE, lane = tid & (KIPP_WAVE - 1);
+    const int n = p.q_len[entry], first = p.q_start[entry];
+    if (n <= 0) return;
+    if (n < p.from) {
+        if (tid < n) p.den[(size_t)(first + tid) * p.heads + head] = 1.0f;      // `from` is less than the threads
+        return;
+    }
+    int base = 0;       // chunks of the entries ahead, as `portion_of` counts them
+    for (int e0 = 0; e0 < entry; e0 += KIPP_WAVE) {
+        const int len = e0 + lane < entry ? p.q_len[e0 + lane] : 0;
+        int chunks = len > 0 && len >= p.from ? (len + CHUNK - 1) / CHUNK : 0;
+#pragma unroll
+        for (int off = KIPP_WAVE / 2; off > 0; off >>= 1) chunks += __shfl_xor(chunks, off, KIPP_WAVE);
+        base += chunks;
+    }
+    float* m_all = p.state + (size_t)p.slots[entry] * p.state_stride + p.n_at + (size_t)p.copies * p.heads * (p.d);
+    float m = m_all[head];
+    const float bi = p.bias_i[head], bf = p.bias_f[head];
+    for (int t0 = 0; t0 < n; t0 += GATE_WAVES * CHUNK) {
+        const int chunk = t0 / CHUNK + wave, t = chunk * CHUNK + lane;
+        float lf = 0.0f, li = -INFINITY;        // beyond the last token: m stays
+        if (t < n) {
+            const float* row = p.src + (size_t)(first + t) * p.stride;
+            li = p.cap * tanhf((row[p.i_at + head] + bi) / p.cap);
+            lf = log_sigmoid(p.cap * tanhf((row[p.f_at + head] + bf) / p.cap));
+        }
+        float a = lf, b = li;                   // tokens up to this one: m -> max(a + m, b)
+#pragma unroll
+        for (int off = 1; off < KIPP_WAVE; off <<= 1) {
+            const float a0 = __shfl_up(a, off, KIPP_WAVE), b0 = __shfl_up(b, off, KIPP_WAVE);
+            if (lane >= off) {
+                b = fmaxf(b0 + a, b);
+                a += a0;
+            }
+        }
+        __syncthreads();                        // the turn before has been read
+        if (lane == KIPP_WAVE - 1) {
+            a_s[wave] = a;
+            b_s[wave] = b;
+        }
+        __syncthreads();
+        float mine = m;
+        for (int w = 0; w < GATE_WAVES; ++w) {
+            if (w == wave) mine = m;
+            m = fmaxf(a_s[w] + m, b_s[w]);
+        }
+        const float after = fmaxf(a + mine, b);
+        float before = __shfl_up(after, 1, KIPP_WAVE);
+        if (lane == 0) before = mine;
+        if (chunk * CHUNK < n) {
+            float* vec = p.vec + ((size_t)(base + chunk) * p.heads + head) * VECS * CHUNK;
+            vec[lane] = t < n ? expf(lf + before - after) : 1.0f;
+            vec[2 * CHUNK + lane] = t < n ? expf(li - after) : 0.0f;
+            vec[3 * CHUNK + lane] = expf(-after);
+        }
+    }
+    for (int c = tid; c < p.copies; c += GATE_WAVES * KIPP_WAVE) m_all[(size_t)c * p.heads + head] = m;
 }
 
 template <int MODE, int DT>
@@ -128,11 +227,11 @@ __global__ void __launch_bounds__(THREADS) chunks_prepare_kernel(const ChunkArgs
     const int tid = threadIdx.x, wave = tid / KIPP_WAVE, lane = tid & (KIPP_WAVE - 1), l16 = lane & 15, h4 = 4 * (lane >> 4);
     const size_t at = (size_t)(portion.base + chunk) * p.heads + head;
     float* a_out = p.a + at * CHUNK * CHUNK;
-    float* vec = p.vec + at * 3 * CHUNK;
+    float* vec = p.vec + at * VECS * CHUNK;
     if (wave == 0) {
         // the wave with the fewest products below: D column by column, a lane a column
         const float* row = p.src + (size_t)(t0 + min(lane, m - 1)) * p.stride;
-        const float g = lane >= m ? 1.0f : (MODE == MODE_DECAY ? p.decays[head] : row[p.g_at + head]);
+        const float g = lane >= m ? 1.0f : (MODE == MODE_DECAY ? p.decays[head] : (MODE == MODE_MLSTM ? vec[lane] : row[p.g_at + head]));
         if (MODE == MODE_DELTA) {
             const float b = lane < m ? row[p.beta_at + head] : 0.0f;
             beta_s[lane] = b;
@@ -151,38 +250,46 @@ __global__ void __launch_bounds__(THREADS) chunks_prepare_kernel(const ChunkArgs
     }
     const float* q = p.q + (size_t)(head / p.qk_rep) * D;
     const float* k = p.k + (size_t)(head / p.qk_rep) * D;
-    f32x4 qk[4], kk[4];
+    constexpr int RUNS = runs_of(MODE, DT);
+    f32x4 qk[RUNS][4], kk[RUNS][4];
 #pragma unroll
-    for (int s = 0; s < 4; ++s) qk[s] = kk[s] = zero4();
+    for (int h = 0; h < RUNS; ++h)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) qk[h][s] = kk[h][s] = zero4();
     if (16 * wave < m) {
         const float* q_row = q + (size_t)(t0 + min(16 * wave + l16, m - 1)) * p.qk_stride + h4;
         const float* k_row = k + (size_t)(t0 + min(16 * wave + l16, m - 1)) * p.qk_stride + h4;
         const float* s_row[4];
 #pragma unroll
         for (int s = 0; s < 4; ++s) s_row[s] = k + (size_t)(t0 + min(16 * s + l16, m - 1)) * p.qk_stride + h4;
-#pragma unroll 2
-        for (int j = 0; j < D; j += 16) {
-            const f32x4 qv = *reinterpret_cast<const f32x4*>(q_row + j);
-            const f32x4 kv = MODE == MODE_DELTA ? *reinterpret_cast<const f32x4*>(k_row + j) : zero4();
+#pragma unroll(RUNS == 1 ? 2 : 1)
+        for (int j0 = 0; j0 < D; j0 += 16 * RUNS)
 #pragma unroll
-            for (int s = 0; s < 4; ++s)
-                if (s <= wave) {
-                    const f32x4 sv = *reinterpret_cast<const f32x4*>(s_row[s] + j);
-                    qk[s] = mul16(qv, sv, qk[s]);
-                    if (MODE == MODE_DELTA) kk[s] = mul16(kv, sv, kk[s]);
-                }
-        }
+            for (int h = 0; h < RUNS; ++h) {
+                const int j = j0 + 16 * h;
+                const f32x4 qv = *reinterpret_cast<const f32x4*>(q_row + j);
+                const f32x4 kv = MODE == MODE_DELTA ? *reinterpret_cast<const f32x4*>(k_row + j) : zero4();
+#pragma unroll
+                for (int s = 0; s < 4; ++s)
+                    if (s <= wave) {
+                        const f32x4 sv = *reinterpret_cast<const f32x4*>(s_row[s] + j);
+                        qk[h][s] = mul16(qv, sv, qk[h][s]);
+                        if (MODE == MODE_DELTA) kk[h][s] = mul16(kv, sv, kk[h][s]);
+                    }
+            }
     }
     __syncthreads();
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
         if (s > wave) continue;
+        qk[0][s] = sum_runs(qk, s);
+        if (MODE == MODE_DELTA) kk[0][s] = sum_runs(kk, s);
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
             const int t = 16 * wave + h4 + v, c = 16 * s + l16;
             const float decay = c <= t && t < m ? d_s[t][c] : 0.0f;
-            a_out[t * CHUNK + c] = decay != 0.0f ? qk[s][v] * decay : 0.0f;
-            if (MODE == MODE_DELTA) l_s[t][c] = c < t && decay != 0.0f ? beta_s[t] * decay * kk[s][v] : 0.0f;
+            a_out[t * CHUNK + c] = decay != 0.0f ? (MODE == MODE_MLSTM ? qk[0][s][v] * p.q_scale : qk[0][s][v]) * decay : 0.0f;
+            if (MODE == MODE_DELTA) l_s[t][c] = c < t && decay != 0.0f ? beta_s[t] * decay * kk[0][s][v] : 0.0f;
         }
     }
     if (MODE != MODE_DELTA) return;
@@ -209,7 +316,7 @@ __global__ void __launch_bounds__(THREADS) chunks_prepare_kernel(const ChunkArgs
 // What a wave multiplies in a chunk: its own rows of q, k, T and A, its rows of K^T, the values of its tokens.
 template <int MODE, int DT>
 struct Operands {
-    f32x4 q[4 * DT], k[MODE == MODE_DELTA ? 4 * DT : 1], a[4], t[MODE == MODE_DELTA ? 4 : 1], e[4], kt[DT][4], v, g, b;
+    f32x4 q[4 * DT], k[MODE == MODE_DELTA ? 4 * DT : 1], a[4], t[MODE == MODE_DELTA ? 4 : 1], e[4], kt[DT][4], v, g, b, f;
     float g_last;
 };
 
@@ -226,13 +333,15 @@ __global__ void __launch_bounds__(THREADS) chunks_walk_kernel(const ChunkArgs p)
     const int tid = threadIdx.x, wave = tid / KIPP_WAVE, lane = tid & (KIPP_WAVE - 1), l16 = lane & 15, h4 = 4 * (lane >> 4);
     const int n = p.q_len[entry], first = p.q_start[entry];
     const int col = blockIdx.x * COLS + l16;
-    const bool live = col < p.dv;
+    const bool norm = MODE == MODE_MLSTM && col == p.dv;        // n: one more column of S, of values of one
+    const bool live = col < p.dv || norm;
     const int own = 16 * wave;              // the wave's tokens of a chunk
     const int row0 = D / 4 * wave;          // its rows of S
-    float* S_col = p.state + (size_t)p.slots[entry] * p.state_stride + ((size_t)head * p.dv + (live ? col : 0)) * D + row0 + h4;
+    float* S_col = p.state + (size_t)p.slots[entry] * p.state_stride + row0 + h4 +
+                   (norm ? p.n_at + (size_t)head * D : ((size_t)head * p.dv + (live ? col : 0)) * D);
     const float* q = p.q + (size_t)(head / p.qk_rep) * D;
     const float* k = p.k + (size_t)(head / p.qk_rep) * D;
-    const float* v_src = p.src + p.v_at + (size_t)head * p.dv + (live ? col : 0);
+    const float* v_src = p.src + p.v_at + (size_t)head * p.dv + (live && !norm ? col : 0);
 
     f32x4 S[DT];
 #pragma unroll
@@ -254,14 +363,15 @@ __global__ void __launch_bounds__(THREADS) chunks_walk_kernel(const ChunkArgs p)
     auto rest_of = [&](int c) {
         const int m = min(CHUNK, n - c * CHUNK), t0 = first + c * CHUNK;
         const size_t at = (size_t)(portion.base + c) * p.heads + head;
-        const float* vec = p.vec + at * 3 * CHUNK;
+        const float* vec = p.vec + at * VECS * CHUNK;
         if (own < m) {
             const float* a_row = p.a + at * CHUNK * CHUNK + (own + l16) * CHUNK + h4;
             const float* t_row = p.t + at * CHUNK * CHUNK + (own + l16) * CHUNK + h4;
 #pragma unroll
             for (int i = 0; i < 4; ++i) x.v[i] = own + h4 + i < m ? v_src[(size_t)(t0 + own + h4 + i) * p.stride] : 0.0f;
             x.g = *reinterpret_cast<const f32x4*>(vec + own + h4);
-            if (MODE == MODE_DELTA) x.b = *reinterpret_cast<const f32x4*>(vec + 2 * CHUNK + own + h4);
+            if (MODE == MODE_DELTA || MODE == MODE_MLSTM) x.b = *reinterpret_cast<const f32x4*>(vec + 2 * CHUNK + own + h4);
+            if (MODE == MODE_MLSTM) x.f = *reinterpret_cast<const f32x4*>(vec + 3 * CHUNK + own + h4);
 #pragma unroll
             for (int j = 0; j < 4; ++j)
                 if (j <= wave) {
@@ -293,16 +403,30 @@ __global__ void __launch_bounds__(THREADS) chunks_walk_kernel(const ChunkArgs p)
         __syncthreads();
         f32x4 inter = zero4(), read = zero4();
         if (mine) {
+            constexpr int RUNS = runs_of(MODE, DT);
+            f32x4 in[RUNS][1], rd[RUNS][1];
 #pragma unroll
-            for (int j = 0; j < 4 * DT; ++j) {
-                const f32x4 sv = *reinterpret_cast<const f32x4*>(&s_s[l16 * SP + 16 * j + h4]);
-                inter = mul16(x.q[j], sv, inter);
-                if (MODE == MODE_DELTA) read = mul16(x.k[j], sv, read);
+            for (int h = 0; h < RUNS; ++h) in[h][0] = rd[h][0] = zero4();
+#pragma unroll
+            for (int j = 0; j < 4 * DT; j += RUNS) {
+                f32x4 sv[RUNS];
+#pragma unroll
+                for (int h = 0; h < RUNS; ++h) sv[h] = *reinterpret_cast<const f32x4*>(&s_s[l16 * SP + 16 * (j + h) + h4]);
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int h = 0; h < RUNS; ++h) {
+                        in[h][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.q[j + h][i], sv[h][i], in[h][0], 0, 0, 0);
+                        if (MODE == MODE_DELTA) rd[h][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.k[j + h][i], sv[h][i], rd[h][0], 0, 0, 0);
+                    }
             }
+            inter = sum_runs(in, 0);
+            if (MODE == MODE_DELTA) read = sum_runs(rd, 0);
             f32x4 u = x.v;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 if (MODE == MODE_DECAY) u[i] = silu_f(u[i]);        // silu(0) = 0
+                if (MODE == MODE_MLSTM) u[i] = x.b[i] * (norm ? 1.0f : u[i]);       // a gate of zero beyond the last token
                 if (MODE == MODE_DELTA) u[i] = own + h4 + i < m ? x.b[i] * (x.v[i] - x.g[i] * read[i]) : 0.0f;
             }
             *reinterpret_cast<f32x4*>((MODE == MODE_DELTA ? r_s : u_s) + l16 * UP + own + h4) = u;
@@ -324,11 +448,16 @@ __global__ void __launch_bounds__(THREADS) chunks_walk_kernel(const ChunkArgs p)
         for (int j = 0; j < 4; ++j)
             if (16 * j < m) u[j] = *reinterpret_cast<const f32x4*>(u_s + l16 * UP + 16 * j + h4);
         if (mine) {
-            f32x4 o = inter * x.g;
+            f32x4 o = MODE == MODE_MLSTM ? zero4() : inter * x.g;
 #pragma unroll
             for (int j = 0; j < 4; ++j)
                 if (j <= wave) o = mul16(x.a[j], u[j], o);
-            if (live) {
+            if (MODE == MODE_MLSTM) o += inter * (x.g * p.q_scale);
+            if (norm) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (own + h4 + i < m) p.den[(size_t)(first + c * CHUNK + own + h4 + i) * p.heads + head] = fmaxf(fabsf(o[i]), x.f[i]) + 1e-6f;
+            } else if (live) {
                 float* o_at = p.o_raw + (size_t)(first + c * CHUNK + own + h4) * p.heads * p.dv + (size_t)head * p.dv + col;
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
@@ -347,8 +476,9 @@ __global__ void __launch_bounds__(THREADS) chunks_walk_kernel(const ChunkArgs p)
         if (more) rest_of(c + 1);
     }
     if (live) {
+        for (int c = 0; c < (norm ? p.copies : 1); ++c)         // every copy of n
 #pragma unroll
-        for (int a = 0; a < DT; ++a) *reinterpret_cast<f32x4*>(S_col + 16 * a) = S[a];
+            for (int a = 0; a < DT; ++a) *reinterpret_cast<f32x4*>(S_col + (size_t)c * p.heads * D + 16 * a) = S[a];
     }
 }
 
@@ -359,10 +489,37 @@ static long long chunk_count(int tokens, int portions) { return (long long)token
 
 // Floats of work space, or 0 where this kernel does not take the sizes: keys of 64, 128, 192 or 256 numbers.
 long long kipp_matrix_chunks_work(int mode, int tokens, int portions, int heads, int d) {
-    if (mode < MODE_DECAY || mode > MODE_GATED || tokens <= 0 || portions <= 0 || heads <= 0 || d <= 0 || d % 64 || d > 256) return 0;
-    const long long each = (mode == MODE_DELTA ? 2 : 1) * CHUNK * CHUNK + 3 * CHUNK;
+    if (mode < MODE_DECAY || mode > MODE_MLSTM || tokens <= 0 || portions <= 0 || heads <= 0 || d <= 0 || d % 64 || d > 256) return 0;
+    const long long each = (mode == MODE_DELTA ? 2 : 1) * CHUNK * CHUNK + VECS * CHUNK;
     return chunk_count(tokens, portions) * heads * each + (mode == MODE_DECAY ? (long long)tokens * 2 * heads * d : 0);
 }
+
+}  // extern "C"
+
+// The work space's parts, and the launches behind what a mode puts ahead of them.
+static void lay_out(ChunkArgs& p, int mode, long long slots_all, float* work) {
+    p.a = work;
+    p.t = mode == MODE_DELTA ? p.a + slots_all * CHUNK * CHUNK : p.a;
+    p.vec = p.t + slots_all * CHUNK * CHUNK;
+}
+
+template <int MODE, int DT>
+static void launch_chunks(const ChunkArgs& p, int longest, int portions, hipStream_t stream) {
+    const int cols = p.dv + (MODE == MODE_MLSTM ? 1 : 0);
+    const dim3 prepare((longest + CHUNK - 1) / CHUNK, p.heads, portions), walk((cols + COLS - 1) / COLS, p.heads, portions), block(THREADS);
+    hipLaunchKernelGGL((chunks_prepare_kernel<MODE, DT>), prepare, block, 0, stream, p);
+    hipLaunchKernelGGL((chunks_walk_kernel<MODE, DT>), walk, block, 0, stream, p);
+}
+
+template <int MODE>
+static void launch_mode(const ChunkArgs& p, int longest, int portions, hipStream_t stream) {
+    if (p.d == 64) launch_chunks<MODE, 1>(p, longest, portions, stream);
+    else if (p.d == 128) launch_chunks<MODE, 2>(p, longest, portions, stream);
+    else if (p.d == 192) launch_chunks<MODE, 3>(p, longest, portions, stream);
+    else launch_chunks<MODE, 4>(p, longest, portions, stream);
+}
+
+extern "C" {
 
 // src: float32 [tokens][stride] with q, k, v (and beta, g) at the given columns, as `kipp_decay_scan`, `kipp_delta_scan` and `kipp_gated_scan` read it
 // (mode 0, 1, 2); q and k of a head at q_at + (head / qk_rep) d.  Of the entries only those of `from` tokens and more, at most `portions` of
@@ -374,20 +531,18 @@ int kipp_matrix_chunks(int mode, const float* src, int stride, int q_at, int k_a
                        hipStream_t stream) {
     if (entries <= 0 || tokens <= 0 || portions <= 0) return 0;
     const long long need = kipp_matrix_chunks_work(mode, tokens, portions, heads, d);
-    if (need == 0 || work_floats < need || longest <= 0 || qk_rep <= 0 || heads % qk_rep || dv <= 0) return -1;
+    if (mode == MODE_MLSTM || need == 0 || work_floats < need || longest <= 0 || qk_rep <= 0 || heads % qk_rep || dv <= 0) return -1;
     if (state_stride < (size_t)heads * d * dv || (state_stride & 3) || (stride & 3) || (q_at & 3) || (k_at & 3)) return -1;
     if (((uintptr_t)src | (uintptr_t)state | (uintptr_t)work) & 15) return -1;
-    ChunkArgs p;
+    ChunkArgs p = {};
     const long long slots_all = chunk_count(tokens, portions) * heads;
-    p.a = work;
-    p.t = mode == MODE_DELTA ? p.a + slots_all * CHUNK * CHUNK : p.a;
-    p.vec = p.t + slots_all * CHUNK * CHUNK;
+    lay_out(p, mode, slots_all, work);
     p.q = src + q_at;
     p.k = src + k_at;
     p.qk_stride = stride;
     if (mode == MODE_DECAY) {
         if (q_at != 0 || k_at != heads * d || qk_rep != 1) return -1;
-        float* ready = p.vec + slots_all * 3 * CHUNK;
+        float* ready = p.vec + slots_all * VECS * CHUNK;
         const int width = 2 * heads * d;
         hipLaunchKernelGGL(chunks_ready_kernel, dim3((width / 4 + THREADS - 1) / THREADS, tokens), dim3(THREADS), 0, stream, src, stride, ready, width);
         p.q = ready;
@@ -408,27 +563,58 @@ int kipp_matrix_chunks(int mode, const float* src, int stride, int q_at, int k_a
     p.o_raw = o_raw;
     p.heads = heads;
     p.qk_rep = qk_rep;
+    p.d = d;
     p.dv = dv;
     p.entries = entries;
     p.from = from;
-    const dim3 prepare((longest + CHUNK - 1) / CHUNK, heads, portions), walk((dv + COLS - 1) / COLS, heads, portions), block(THREADS);
-#define KIPP_CHUNKS(MODE, DT)                                                              \
-    do {                                                                                   \
-        hipLaunchKernelGGL((chunks_prepare_kernel<MODE, DT>), prepare, block, 0, stream, p); \
-        hipLaunchKernelGGL((chunks_walk_kernel<MODE, DT>), walk, block, 0, stream, p);       \
-    } while (0)
-#define KIPP_CHUNKS_D(MODE)                     \
-    do {                                        \
-        if (d == 64) KIPP_CHUNKS(MODE, 1);      \
-        else if (d == 128) KIPP_CHUNKS(MODE, 2); \
-        else if (d == 192) KIPP_CHUNKS(MODE, 3); \
-        else KIPP_CHUNKS(MODE, 4);              \
-    } while (0)
-    if (mode == MODE_DECAY) KIPP_CHUNKS_D(MODE_DECAY);
-    else if (mode == MODE_DELTA) KIPP_CHUNKS_D(MODE_DELTA);
-    else KIPP_CHUNKS_D(MODE_GATED);
-#undef KIPP_CHUNKS_D
-#undef KIPP_CHUNKS
+    if (mode == MODE_DECAY) launch_mode<MODE_DECAY>(p, longest, portions, stream);
+    else if (mode == MODE_DELTA) launch_mode<MODE_DELTA>(p, longest, portions, stream);
+    else launch_mode<MODE_GATED>(p, longest, portions, stream);
+    return KIPP_LAUNCH_CHECK();
+}
+
+// The same for an mLSTM: `proj` and `state` as `kipp_mlstm_scan` has them, `copies` of n and m in a slot.  o_raw receives the sums before they
+// are divided, den [tokens][heads] what they are to be divided by (ones for the entries of fewer than `from` tokens, at most 1,024, which
+// are left to the walk).
+int kipp_mlstm_chunks(const float* proj, int stride, const float* bias_i, const float* bias_f, float cap, float* state, size_t state_stride,
+                      int copies, const int32_t* q_start, const int32_t* q_len, const int32_t* slots, float* o_raw, float* den, int tokens, int entries,
+                      int heads, int d, int dv, int longest, int from, int portions, float* work, long long work_floats, hipStream_t stream) {
+    if (entries <= 0 || tokens <= 0 || portions <= 0) return 0;
+    const long long need = kipp_matrix_chunks_work(MODE_MLSTM, tokens, portions, heads, d);
+    if (need == 0 || work_floats < need || longest <= 0 || dv <= 0 || copies <= 0 || from > GATE_WAVES * KIPP_WAVE || !(cap > 0.0f)) return -1;
+    if (stride < 2 * heads * d + 2 * heads * dv + 2 * heads || state_stride < (size_t)heads * d * dv + (size_t)copies * (heads * d + heads)) return -1;
+    if ((state_stride & 3) || (stride & 3) || (((uintptr_t)proj | (uintptr_t)state | (uintptr_t)work) & 15)) return -1;
+    ChunkArgs p = {};
+    lay_out(p, MODE_MLSTM, chunk_count(tokens, portions) * heads, work);
+    p.q = proj;
+    p.k = proj + heads * d;
+    p.qk_stride = stride;
+    p.src = proj;
+    p.stride = stride;
+    p.v_at = 2 * heads * d;
+    p.i_at = 2 * heads * d + 2 * heads * dv;
+    p.f_at = p.i_at + heads;
+    p.bias_i = bias_i;
+    p.bias_f = bias_f;
+    p.cap = cap;
+    p.q_scale = 1.0f / sqrtf((float)d);
+    p.state = state;
+    p.state_stride = state_stride;
+    p.n_at = heads * d * dv;
+    p.copies = copies;
+    p.q_start = q_start;
+    p.q_len = q_len;
+    p.slots = slots;
+    p.o_raw = o_raw;
+    p.den = den;
+    p.heads = heads;
+    p.qk_rep = 1;
+    p.d = d;
+    p.dv = dv;
+    p.entries = entries;
+    p.from = from;
+    hipLaunchKernelGGL(chunks_gates_kernel, dim3(heads, entries), dim3(GATE_WAVES * KIPP_WAVE), 0, stream, p);
+    launch_mode<MODE_MLSTM>(p, longest, portions, stream);
     return KIPP_LAUNCH_CHECK();
 }
 

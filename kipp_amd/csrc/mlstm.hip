@@ -1,5 +1,5 @@
-// The matrix memory of an mLSTM layer: the recurrence itself, for prompt portions and single tokens alike, and
-// the step between it and the output projection.
+// The matrix memory of an mLSTM layer: the recurrence itself, for prompt portions and single tokens alike (under bfloat16 longer
+// portions go by `linear_chunks.hip`), and the step between it and the output projection.
 //
 // Per head, with a query q (already times d^(-1/2)), key k (d numbers), value v (dv numbers) and the two gate
 // pre-activations zi, zf of a token:
@@ -48,7 +48,7 @@ template <int ROWS, int PARTS, int BASE>
 __global__ void __launch_bounds__(SCAN_THREADS) mlstm_scan_kernel(
     const float* __restrict__ proj, int stride, const float* __restrict__ bias_i, const float* __restrict__ bias_f, float cap,
     float* __restrict__ state, size_t state_stride, const int32_t* __restrict__ q_start, const int32_t* __restrict__ q_len,
-    const int32_t* __restrict__ slots, float* __restrict__ o_raw, int heads, int d, int dv, int chunk, int unit, int copies) {
+    const int32_t* __restrict__ slots, float* __restrict__ o_raw, int heads, int d, int dv, int chunk, int unit, int copies, int below) {
     constexpr int COLS = SCAN_THREADS / PARTS;
     constexpr int DP = ROWS * PARTS;                        // a staged row of k or q
     constexpr int PER = SCAN_STAGE / SCAN_THREADS;          // staged numbers of k, and of q, a thread
@@ -65,6 +65,7 @@ __global__ void __launch_bounds__(SCAN_THREADS) mlstm_scan_kernel(
     const bool live = col < dv;
     const int row0 = part * ROWS;
     const int first = q_start[seq], count = q_len[seq];
+    if (below > 0 && count >= below) return;        // uniform over the workgroup: another kernel's entry
     float* slot = state + (size_t)slots[seq] * state_stride;
     float* S_g = slot + ((size_t)head * dv + (live ? col : 0)) * d;
     float* n_all = slot + (size_t)heads * d * dv;
@@ -250,20 +251,24 @@ __global__ void __launch_bounds__(SCAN_THREADS) mlstm_scan_kernel(
 #define FINISH_HEADS 4
 
 template <typename TO>
-__global__ void mlstm_finish_kernel(const float* __restrict__ o_raw, const float* __restrict__ proj, int stride, int gate_at,
+__global__ void mlstm_finish_kernel(const float* __restrict__ o_raw, const float* __restrict__ den, const float* __restrict__ proj, int stride, int gate_at,
                                     const float* __restrict__ norm_w, float eps, TO* __restrict__ out, int heads, int dv) {
     const int wave = threadIdx.x / KIPP_WAVE, lane = threadIdx.x & (KIPP_WAVE - 1);
     const int t = blockIdx.y, head = blockIdx.x * FINISH_HEADS + wave;
     if (head >= heads) return;
     const float* src = o_raw + ((size_t)t * heads + head) * dv;
+    const float below = den != nullptr ? den[(size_t)t * heads + head] : 1.0f;
     float ss = 0.0f;
-    for (int e = lane; e < dv; e += KIPP_WAVE) ss = fmaf(src[e], src[e], ss);
+    for (int e = lane; e < dv; e += KIPP_WAVE) {
+        const float o = src[e] / below;
+        ss = fmaf(o, o, ss);
+    }
     ss = wave_sum(ss);
     const float scale = 1.0f / sqrtf(ss / (float)dv + eps);
     const float* gate = proj + (size_t)t * stride + gate_at + head * dv;
     TO* dst = out + ((size_t)t * heads + head) * dv;
     for (int e = lane; e < dv; e += KIPP_WAVE)
-        store_f(dst, e, src[e] * scale * norm_w[head * dv + e] * (1.0f / (1.0f + expf(-gate[e]))));
+        store_f(dst, e, src[e] / below * scale * norm_w[head * dv + e] * (1.0f / (1.0f + expf(-gate[e]))));
 }
 
 // Lanes that share a column of the memory in the walk over prompt portions: 8 rows a lane (16 for keys of 129 to 256 and
@@ -273,10 +278,11 @@ static int kipp_mlstm_parts(int d) { return d <= 32 ? 4 : (d <= 256 ? 16 : 64); 
 extern "C" {
 
 // `few`: every entry brings few tokens (single decoded tokens): where the key size allows, a workgroup takes 64 columns
-// with 4 lanes each, a quarter of the workgroups, each reading longer runs of the state.
+// with 4 lanes each, a quarter of the workgroups, each reading longer runs of the state.  `below`: entries of so many tokens and more
+// are left alone (0: none).
 int kipp_mlstm_scan(const float* proj, int stride, const float* bias_i, const float* bias_f, float cap, float* state,
                     size_t state_stride, const int32_t* q_start, const int32_t* q_len, const int32_t* slots, float* o_raw,
-                    int n_seqs, int heads, int d, int dv, int few, hipStream_t stream) {
+                    int n_seqs, int heads, int d, int dv, int few, int below, hipStream_t stream) {
     if (n_seqs <= 0) return 0;
     if (heads <= 0 || d <= 0 || d > 1024 || dv <= 0 || !(cap > 0.0f)) return -1;
     const int unit = SCAN_THREADS / kipp_mlstm_parts(d);
@@ -294,7 +300,7 @@ int kipp_mlstm_scan(const float* proj, int stride, const float* bias_i, const fl
     const size_t lds = ((size_t)chunk * (2 * rows * parts + cols + 4) + 4) * sizeof(float);
 #define KIPP_SCAN(R, P, B)                                                                                                          \
     hipLaunchKernelGGL((mlstm_scan_kernel<R, P, B>), grid, block, lds, stream, proj, stride, bias_i, bias_f, cap, state, state_stride, \
-                       q_start, q_len, slots, o_raw, heads, d, dv, chunk, unit, copies)
+                       q_start, q_len, slots, o_raw, heads, d, dv, chunk, unit, copies, below)
     if (parts == 4 && rows == 8) KIPP_SCAN(8, 4, 8);
     else if (parts == 4) KIPP_SCAN(32, 4, 8);
     else if (parts == 8) KIPP_SCAN(32, 8, 16);
@@ -306,15 +312,16 @@ int kipp_mlstm_scan(const float* proj, int stride, const float* bias_i, const fl
     return KIPP_LAUNCH_CHECK();
 }
 
-int kipp_mlstm_finish(const float* o_raw, const float* proj, int stride, int gate_at, const float* norm_w, float eps,
+// `den` [tokens][heads] (or null): what a head's sums are divided by first.
+int kipp_mlstm_finish(const float* o_raw, const float* den, const float* proj, int stride, int gate_at, const float* norm_w, float eps,
                       void* out, int out_dtype, int n_tokens, int heads, int dv, hipStream_t stream) {
     if (n_tokens <= 0) return 0;
     if (heads <= 0 || dv <= 0 || stride < gate_at + heads * dv) return -1;
     dim3 grid((heads + FINISH_HEADS - 1) / FINISH_HEADS, n_tokens), block(FINISH_HEADS * KIPP_WAVE);
     if (out_dtype == KIPP_BF16)
-        hipLaunchKernelGGL(mlstm_finish_kernel<bf16_t>, grid, block, 0, stream, o_raw, proj, stride, gate_at, norm_w, eps, (bf16_t*)out, heads, dv);
+        hipLaunchKernelGGL(mlstm_finish_kernel<bf16_t>, grid, block, 0, stream, o_raw, den, proj, stride, gate_at, norm_w, eps, (bf16_t*)out, heads, dv);
     else
-        hipLaunchKernelGGL(mlstm_finish_kernel<float>, grid, block, 0, stream, o_raw, proj, stride, gate_at, norm_w, eps, (float*)out, heads, dv);
+        hipLaunchKernelGGL(mlstm_finish_kernel<float>, grid, block, 0, stream, o_raw, den, proj, stride, gate_at, norm_w, eps, (float*)out, heads, dv);
     return KIPP_LAUNCH_CHECK();
 }
 

@@ -644,9 +644,10 @@ def mlstm_state_size(heads: int, d: int, dv: int) -> int:
 
 def mlstm_scan(proj: torch.Tensor, bias_i: torch.Tensor, bias_f: torch.Tensor, cap: float, state: torch.Tensor,
                q_start: torch.Tensor, q_len: torch.Tensor, slots: torch.Tensor, o_raw: torch.Tensor,
-               heads: int, d: int, dv: int, few: bool = False) -> torch.Tensor:
+               heads: int, d: int, dv: int, few: bool = False, below: int = 0) -> torch.Tensor:
     """The recurrence over every entry's tokens, in order, from and into the entry's slot of `state` [slots, size]
-    (float32).  `few`: every entry brings few tokens (single decoded tokens): fewer, larger workgroups; the same bits.  `proj`: float32 [tokens, >= 2 heads d + 2 heads dv + 2 heads], columns q | k | v | gate | zi | zf;
+    (float32).  `few`: every entry brings few tokens (single decoded tokens): fewer, larger workgroups; the same bits.  `below`: entries of
+    so many tokens and more are left alone (0: none; what `mlstm_chunks` took).  `proj`: float32 [tokens, >= 2 heads d + 2 heads dv + 2 heads], columns q | k | v | gate | zi | zf;
     `o_raw` float32 [tokens, heads dv] receives S^T q over its denominator."""
     _dev(proj, bias_i, bias_f, state, q_start, q_len, slots, o_raw)
     for t, name in ((q_start, "q_start"), (q_len, "q_len"), (slots, "slots")):
@@ -660,23 +661,50 @@ def mlstm_scan(proj: torch.Tensor, bias_i: torch.Tensor, bias_f: torch.Tensor, c
           "mlstm_scan: o_raw is float32 [tokens, heads dv]; key size up to 1,024")
     _need(q_start.numel() == q_len.numel() == slots.numel(), "mlstm_scan: one start, length and slot an entry")
     fn = _fn("mlstm", "kipp_mlstm_scan", [_c_ptr, _c_int, _c_ptr, _c_ptr, _c_float, _c_ptr, _c_size, _c_ptr, _c_ptr, _c_ptr, _c_ptr,
-                                          _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr])
+                                          _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr])
     _check(fn(_ptr(proj), proj.shape[1], _ptr(bias_i), _ptr(bias_f), float(cap), _ptr(state), state.shape[1], _ptr(q_start),
-              _ptr(q_len), _ptr(slots), _ptr(o_raw), q_start.numel(), heads, d, dv, int(bool(few)), _stream()), "mlstm_scan")
+              _ptr(q_len), _ptr(slots), _ptr(o_raw), q_start.numel(), heads, d, dv, int(bool(few)), max(0, int(below)), _stream()), "mlstm_scan")
     return o_raw
 
 
+def mlstm_chunks(proj: torch.Tensor, bias_i: torch.Tensor, bias_f: torch.Tensor, cap: float, state: torch.Tensor,
+                 q_start: torch.Tensor, q_len: torch.Tensor, slots: torch.Tensor, o_raw: torch.Tensor,
+                 heads: int, d: int, dv: int, longest: int, portions: Optional[int] = None):
+    """`mlstm_scan` for entries of `CHUNKS_FROM` tokens and more, 64 tokens at a time on the matrix cores: the same float32 sums in another
+    order, in steps where that is the faster way (`matrix_chunks_from`; `longest`: the most tokens an entry brings, `portions`: how many
+    bring so many, if known).  Returns (den, below): `den` float32 [tokens, heads] is what `mlstm_finish` divides the rows of `o_raw` by, or
+    None where it took no entry; the entries of fewer than `below` tokens are left for `mlstm_scan(..., below=below)` (0: every entry is; -1: there are no others)."""
+    _dev(proj, bias_i, bias_f, state, q_start, q_len, slots, o_raw)
+    _need(proj.dim() == 2 and proj.dtype == torch.float32 and proj.shape[1] >= 2 * heads * d + 2 * heads * dv + 2 * heads,
+          "mlstm_chunks: proj is float32 [tokens, q | k | v | gate | zi | zf]")
+    _need(state.shape[1] >= mlstm_state_size(heads, d, dv) and cap > 0, "mlstm_chunks: state is float32 [slots, size]")
+    _need(bias_i.dtype == bias_f.dtype == torch.float32 and bias_i.numel() == heads and bias_f.numel() == heads, "mlstm_chunks: float32 gate biases [heads]")
+    _scan_args(state, q_start, q_len, slots, o_raw, proj.shape[0], heads, d, dv, "mlstm_chunks")
+    portions, below = _chunk_portions(3, proj, 0, heads * d, state, q_start, heads, d, dv, longest, portions)
+    if not portions:
+        return None, 0
+    size, work = _chunk_work(3, proj.shape[0], portions, heads, d, proj.device)
+    den = torch.empty((proj.shape[0], heads), dtype=torch.float32, device=proj.device)
+    fn = _fn("linear_chunks", "kipp_mlstm_chunks", [_c_ptr, _c_int, _c_ptr, _c_ptr, _c_float, _c_ptr, _c_size, _c_int] + [_c_ptr] * 5 + [_c_int] * 8
+             + [_c_ptr, ctypes.c_longlong, _c_ptr])
+    _check(fn(_ptr(proj), proj.shape[1], _ptr(bias_i), _ptr(bias_f), float(cap), _ptr(state), state.shape[1], -(-dv // mlstm_columns(d)), _ptr(q_start),
+              _ptr(q_len), _ptr(slots), _ptr(o_raw), _ptr(den), proj.shape[0], q_start.numel(), heads, d, dv, int(longest), CHUNKS_FROM, portions,
+              _ptr(work), size, _stream()), "mlstm_chunks")
+    return den, below
+
+
 def mlstm_finish(o_raw: torch.Tensor, proj: torch.Tensor, gate_at: int, norm_w: torch.Tensor, eps: float, out: torch.Tensor,
-                 heads: int, dv: int) -> torch.Tensor:
-    """out [tokens, heads dv] = every head of `o_raw` over its root mean square, times `norm_w`, times
-    sigmoid(proj[:, gate_at:gate_at + heads dv])."""
-    _dev(o_raw, proj, norm_w, out)
+                 heads: int, dv: int, den: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """out [tokens, heads dv] = every head of `o_raw` (over `den` [tokens, heads] first, if given) over its root mean square, times
+    `norm_w`, times sigmoid(proj[:, gate_at:gate_at + heads dv])."""
+    _dev(o_raw, proj, norm_w, out, den)
+    _need(den is None or (den.dtype == torch.float32 and den.shape == (o_raw.shape[0], heads)), "mlstm_finish: den is float32 [tokens, heads]")
     n = o_raw.shape[0]
     _need(o_raw.dtype == proj.dtype == norm_w.dtype == torch.float32 and o_raw.shape == (n, heads * dv) and out.shape == o_raw.shape
           and proj.dim() == 2 and proj.shape[0] == n and proj.shape[1] >= gate_at + heads * dv and norm_w.numel() == heads * dv,
           "mlstm_finish: float32 [tokens, heads dv] rows, gate columns inside proj")
-    fn = _fn("mlstm", "kipp_mlstm_finish", [_c_ptr, _c_ptr, _c_int, _c_int, _c_ptr, _c_float, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_ptr])
-    _check(fn(_ptr(o_raw), _ptr(proj), proj.shape[1], int(gate_at), _ptr(norm_w), float(eps), _ptr(out), _code(out), n, heads, dv,
+    fn = _fn("mlstm", "kipp_mlstm_finish", [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_ptr, _c_float, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_ptr])
+    _check(fn(_ptr(o_raw), _ptr(den), _ptr(proj), proj.shape[1], int(gate_at), _ptr(norm_w), float(eps), _ptr(out), _code(out), n, heads, dv,
               _stream()), "mlstm_finish")
     return out
 
@@ -733,14 +761,18 @@ CHUNKS_FROM = 16
 
 
 def matrix_chunks_from(mode: int, d: int, state: int) -> int:
-    """Tokens of a step's longest entry from which on chunks are the faster way (mode 0 fixed decays, 1 the delta rule, 2 a decay a token;
+    """Tokens of a step's longest entry from which on chunks are the faster way (mode 0 fixed decays, 1 the delta rule, 2 a decay a token, 3 an mLSTM;
     `state`: numbers of the memories of all the entries that would go by chunks).  In the walk's time, one entry of 16 / 64 / 128 / 256
     tokens: 8 heads of 128 x 320, fixed 1.63 1.05 0.70 0.47, delta 2.76 1.48 0.99 0.70; 8 of 64 x 128, 1.80 0.95 0.64 0.45 and 2.81 1.43 0.96
     0.66; 16 of 256 x 256, 1.57 0.98 0.53 0.36 and 2.42 1.42 0.73 0.51.  Sixteen entries: 1.49 0.70 0.56 0.46 and 2.57 1.13 0.94 0.83; 2.09 1.39 0.96 0.81
     and 2.90 1.69 1.15 0.93; 0.97 0.40 0.34 0.28 and 1.23 0.54 0.46 0.38.  Where single tokens walk beside them that launch comes on top.
     Whole steps of a prompt of 64, 80, 96, 112 tokens, us that chunks take more: two memories of 8 heads of 128 x 320, fixed -7 -21 -36 -53, two with
-    40 of 128 x 64, a decay a token, -1 -9 -15 -21; the delta rule 27 18 2 -7, four prompts of 64, 96, 128, 176 tokens 32 24 18 9."""
+    40 of 128 x 64, a decay a token, -1 -9 -15 -21; the delta rule 27 18 2 -7, four prompts of 64, 96, 128, 176 tokens 32 24 18 9.
+    An mLSTM, us walk / chunks, one entry of 32, 48, 64 tokens: 8 heads of 128 x 320 17 / 21, 23 / 21, 28 / 22, of 256 x 512 24 / 30, 34 / 34, 42 / 39, 4 of
+    64 x 128 18 / 20, 26 / 21, 31 / 20; eight entries of 16, 32: 29 / 29, 46 / 34; 100 / 64, 173 / 75; 12 / 21, 17 / 21."""
     many = state >= 1 << 22
+    if mode == 3:
+        return 32 if many else 64
     if mode == 1:
         return (48 if many else 112) if d >= 192 else (128 if state < 1 << 19 else 224)
     return 144 if d < 128 else (48 if many else (64 if d >= 192 else 80))
@@ -751,26 +783,40 @@ def matrix_chunks_ok(d: int) -> bool:
     return d % 64 == 0 and 0 < d <= 256
 
 
+def _chunk_portions(mode, src, q_at, k_at, state, q_start, heads, d, dv, longest, portions):
+    """(entries that may go by chunks, tokens below which entries are left for the walk): (0, 0) where chunks do not take the sizes or are not the
+    faster way; below is -1 where there are no others."""
+    if longest < CHUNKS_FROM or not matrix_chunks_ok(d) or src.shape[1] % 4 or q_at % 4 or k_at % 4 or state.shape[1] % 4 \
+            or src.data_ptr() % 16 or state.data_ptr() % 16 or src.shape[0] == 0:
+        return 0, 0
+    entries = q_start.numel()
+    every = portions is not None and portions >= entries
+    portions = min(entries if portions is None else int(portions), entries, src.shape[0] // CHUNKS_FROM)
+    if portions <= 0 or longest < matrix_chunks_from(mode, d, portions * heads * d * dv):
+        return 0, 0
+    return portions, -1 if every else CHUNKS_FROM
+
+
+def _chunk_work(mode, tokens, portions, heads, d, device):
+    size = _fn("linear_chunks", "kipp_matrix_chunks_work", [_c_int] * 5, restype=ctypes.c_longlong)(mode, tokens, portions, heads, d)
+    _need(size > 0, "matrix_chunks: sizes the kernel refuses")
+    return size, torch.empty(size, dtype=torch.float32, device=device)
+
+
 def _matrix_chunks(mode, src, q_at, k_at, v_at, beta_at, g_at, decays, state, q_start, q_len, slots, o_raw, heads, qk_rep, d, dv, longest,
                    portions) -> int:
     """The scan by chunks, for the entries of `CHUNKS_FROM` tokens and more, where it takes the sizes and is the faster way.  Returns the
     tokens below which entries are left for the walk: 0, it took none; -1, there are no others."""
-    if longest < CHUNKS_FROM or not matrix_chunks_ok(d) or src.shape[1] % 4 or q_at % 4 or k_at % 4 or state.shape[1] % 4 \
-            or src.data_ptr() % 16 or state.data_ptr() % 16 or src.shape[0] == 0:
+    portions, below = _chunk_portions(mode, src, q_at, k_at, state, q_start, heads, d, dv, longest, portions)
+    if not portions:
         return 0
     tokens, entries = src.shape[0], q_start.numel()
-    every = portions is not None and portions >= entries
-    portions = min(entries if portions is None else int(portions), entries, tokens // CHUNKS_FROM)
-    if portions <= 0 or longest < matrix_chunks_from(mode, d, portions * heads * d * dv):
-        return 0
-    size = _fn("linear_chunks", "kipp_matrix_chunks_work", [_c_int] * 5, restype=ctypes.c_longlong)(mode, tokens, portions, heads, d)
-    _need(size > 0, "matrix_chunks: sizes the kernel refuses")
-    work = torch.empty(size, dtype=torch.float32, device=src.device)
+    size, work = _chunk_work(mode, tokens, portions, heads, d, src.device)
     fn = _fn("linear_chunks", "kipp_matrix_chunks", [_c_int, _c_ptr] + [_c_int] * 6 + [_c_ptr, _c_ptr, _c_size] + [_c_ptr] * 4 + [_c_int] * 9
              + [_c_ptr, ctypes.c_longlong, _c_ptr])
     _check(fn(mode, _ptr(src), src.shape[1], q_at, k_at, v_at, beta_at, g_at, _ptr(decays), _ptr(state), state.shape[1], _ptr(q_start), _ptr(q_len),
               _ptr(slots), _ptr(o_raw), tokens, entries, heads, qk_rep, d, dv, int(longest), CHUNKS_FROM, portions, _ptr(work), size, _stream()), "matrix_chunks")
-    return -1 if every else CHUNKS_FROM
+    return below
 
 
 def decay_scan(proj: torch.Tensor, decays: torch.Tensor, state: torch.Tensor, q_start: torch.Tensor, q_len: torch.Tensor,

@@ -43,7 +43,7 @@ def _scan_variants(key_size, dtype):
     return [("linear_scan", None)] + ([("linear_chunks", None)] if dtype == "bfloat16" and matrix_chunks_ok(key_size) else [])
 
 
-def _portions(batch):
+def chunk_portions(batch):
     """How many entries of the step bring as many tokens as a portion's chunks ask for."""
     from ..csrc.ops import CHUNKS_FROM
     n = batch.host.get("chunk_portions")
@@ -99,7 +99,7 @@ class DecayAttention:
         proj = rt.linear(x, self.w_in)                    # float32 [n, q | k | v | gate]
         o_raw = rt.empty((n, hv), torch.float32)
         ops.decay_scan(proj, self.decays, state, batch.q_start, batch.q_len, batch.slots, o_raw, s.num_heads, s.head_dim, s.v_head_dim, longest=batch.max_q_len,
-                       chunks=rt.dtype == "bfloat16", portions=_portions(batch))
+                       chunks=rt.dtype == "bfloat16", portions=chunk_portions(batch))
         out = ops.scan_finish(o_raw, proj, 2 * s.num_heads * s.head_dim + hv, self.norm, s.norm_eps, "sigmoid", hv, rt.empty((n, hv), rt.act_dtype))
         return rt.linear(out, self.w_o, slabs=True, defer=True)
 
@@ -167,7 +167,7 @@ class GatedDelta:
                           longest=batch.max_q_len)
         o_raw = rt.empty((n, hv), torch.float32)
         ops.delta_scan(prep, state, batch.q_start, batch.q_len, batch.slots, o_raw, s.num_heads, s.num_kv_heads, s.head_dim, s.v_head_dim, longest=batch.max_q_len,
-                       chunks=rt.dtype == "bfloat16", portions=_portions(batch))
+                       chunks=rt.dtype == "bfloat16", portions=chunk_portions(batch))
         out = ops.scan_finish(o_raw, proj, channels, self.norm, s.norm_eps, "silu", s.v_head_dim, rt.empty((n, hv), rt.act_dtype))
         return rt.linear(out, self.w_o, slabs=True, defer=True)
 
@@ -235,7 +235,7 @@ class SSD:
                         batch.slots, prep, s.num_heads, s.groups, s.state_size, s.head_dim, longest=batch.max_q_len)
         o_raw = rt.empty((n, s.inner), torch.float32)
         ops.gated_scan(prep, state, batch.q_start, batch.q_len, batch.slots, o_raw, s.num_heads, s.groups, s.state_size, s.head_dim,
-                       longest=batch.max_q_len, chunks=rt.dtype == "bfloat16", portions=_portions(batch))
+                       longest=batch.max_q_len, chunks=rt.dtype == "bfloat16", portions=chunk_portions(batch))
         out = ops.ssd_finish(o_raw, prep, 2 * s.groups * s.state_size + s.inner, proj, 0, self.skip, s.head_dim, self.norm, s.norm_eps,
                              s.inner // s.norm_groups, rt.empty((n, s.inner), rt.act_dtype))
         return rt.linear(out, self.w_o, slabs=True, defer=True)

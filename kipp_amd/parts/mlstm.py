@@ -7,9 +7,10 @@ request's slot.
                                   o = S'^T (q / sqrt(d)) / (max(|n' . q / sqrt(d)|, e^(-m')) + 1e-6)
     delta = W_o (o / rms(o) per head * w * sigmoid(gate))
 
-The recurrence, the gates and the norms run in float32 under either precision; the state is float32.  A prompt
+The recurrence, the gates and the norms run in float32 under either precision; the state is float32.  Under float32 a prompt
 portion walks its tokens in order inside one kernel launch, a single token is a walk of one step: the same kernel,
-so a position's result does not depend on how the tokens were cut.
+so a position's result does not depend on how the tokens were cut.  Under bfloat16 portions of 16 tokens and more go 64 tokens at
+a time where the key size allows and the step's longest portion is long enough, as the other matrix memories do.
 """
 from __future__ import annotations
 
@@ -17,6 +18,7 @@ import torch
 
 from ..cache.needs import StateNeed
 from .base import ParamSpec, register
+from .matrix_memory import chunk_portions
 
 
 @register("mixer", "mlstm")
@@ -52,7 +54,8 @@ class MLSTM:
 
     @staticmethod
     def variants(spec, dtype):
-        return [("mlstm", None)]
+        from ..csrc.ops import matrix_chunks_ok
+        return [("mlstm", None)] + ([("linear_chunks", None)] if dtype == "bfloat16" and matrix_chunks_ok(spec.head_dim) else [])
 
     def load(self, tensors):
         n = self._names(self.spec)
@@ -80,8 +83,10 @@ class MLSTM:
         hv = s.num_heads * s.v_head_dim
         proj = rt.linear(x, self.w_in)                    # float32 [n, q | k | v | gate | zi | zf]
         o_raw = rt.empty((n, hv), torch.float32)
-        ops.mlstm_scan(proj, self.bias_i, self.bias_f, s.gate_cap, state, batch.q_start, batch.q_len, batch.slots, o_raw,
-                       s.num_heads, s.head_dim, s.v_head_dim, few=batch.max_q_len <= 4)
+        args = (proj, self.bias_i, self.bias_f, s.gate_cap, state, batch.q_start, batch.q_len, batch.slots, o_raw, s.num_heads, s.head_dim, s.v_head_dim)
+        den, below = ops.mlstm_chunks(*args, longest=batch.max_q_len, portions=chunk_portions(batch)) if rt.dtype == "bfloat16" else (None, 0)
+        if below >= 0:
+            ops.mlstm_scan(*args, few=batch.max_q_len <= 4, below=below)
         out = ops.mlstm_finish(o_raw, proj, 2 * s.num_heads * s.head_dim + hv, self.norm, s.norm_eps, rt.empty((n, hv), rt.act_dtype),
-                               s.num_heads, s.v_head_dim)
+                               s.num_heads, s.v_head_dim, den=den)
         return rt.linear(out, self.w_o, slabs=True, defer=True)

@@ -143,3 +143,65 @@ def test_an_entry_beside_others_is_as_alone(mode):
         rows = np.arange(starts[e], starts[e] + lengths[e])
         o, state = run(rows, [0], [lengths[e]], [e], lengths[e] >= ops.CHUNKS_FROM, None)
         assert np.array_equal(o, together[0][0][rows]) and np.array_equal(state[e], together[0][1][e]), e
+
+
+@pytest.mark.parametrize("d, dv, heads", [(64, 16, 3), (128, 40, 2), (192, 31, 2), (256, 33, 1)])
+def test_mlstm_chunks_beside_the_walk(d, dv, heads):
+    """The mLSTM's running maximum, normalizer and floor by chunks: entries longer than the gates' turn of 1,024 tokens and shorter than
+    what chunks take, from states that the walk left, a column of n beside whole and partial tiles of columns.  Both forms against
+    float64; S, every copy of n and m as the walk leaves them."""
+    import torch
+    from kipp_amd.csrc import ops
+    rng = np.random.default_rng(d)
+    cap, lengths = 15.0, [64, 1, 65, 15, 16, 1100]
+    tokens, n = sum(lengths), len(lengths)
+    starts = np.concatenate([[0], np.cumsum(lengths)[:-1]]).astype(np.int32)
+    width = 2 * heads * d + 2 * heads * dv + 2 * heads
+    proj = rng.normal(size=(tokens, width + -width % 4)).astype(np.float32)
+    proj[:, width - 2 * heads:width] *= 4.0
+    bi, bf = rng.normal(size=heads).astype(np.float32), (2.0 + rng.normal(size=heads)).astype(np.float32)
+    to = lambda x: torch.tensor(x, device=DEV)  # noqa: E731
+    args = lambda p, state, o, at, count, slots: (to(p), to(bi), to(bf), cap, state, to(at), to(count), to(slots), o, heads, d, dv)  # noqa: E731
+    size, slots = ops.mlstm_state_size(heads, d, dv), np.arange(n, dtype=np.int32)[::-1].copy()
+    before = torch.zeros((n, size), device=DEV)
+    lead = rng.normal(size=(n, proj.shape[1])).astype(np.float32)
+    ops.mlstm_scan(*args(lead, before, torch.empty((n, heads * dv), device=DEV), np.arange(n, dtype=np.int32), np.ones(n, dtype=np.int32), slots))
+    walked, chunked = before.clone(), before.clone()
+    o_walk, o = (torch.full((tokens, heads * dv), np.nan, device=DEV) for _ in range(2))
+    lens = np.array(lengths, dtype=np.int32)
+    ops.mlstm_scan(*args(proj, walked, o_walk, starts, lens, slots))
+    den, below = ops.mlstm_chunks(*args(proj, chunked, o, starts, lens, slots), longest=max(lengths), portions=4)
+    assert below == ops.CHUNKS_FROM
+    ops.mlstm_scan(*args(proj, chunked, o, starts, lens, slots), below=below)
+    got = (o.view(tokens, heads, dv) / den[:, :, None]).double().cpu().numpy()
+    o_walk, walked, chunked = o_walk.view(tokens, heads, dv).double().cpu().numpy(), walked.double().cpu().numpy(), chunked.double().cpu().numpy()
+    q, k, v = (proj[:, a:b].reshape(tokens, heads, -1).astype(np.float64) for a, b in ((0, heads * d), (heads * d, 2 * heads * d), (2 * heads * d, 2 * heads * d + heads * dv)))
+    z = proj[:, width - 2 * heads:width].astype(np.float64)
+    li, lf = (cap * np.tanh((z[:, a:a + heads] + b) / cap) for a, b in ((0, bi), (heads, bf)))
+    lf = -np.logaddexp(0.0, -lf)
+    copies = (size - heads * d * dv) // (heads * d + heads)
+    before = before.double().cpu().numpy()
+    for i in range(n):
+        at, state, row = slice(starts[i], starts[i] + lengths[i]), before[slots[i]], slots[i]
+        n_all, m_all = heads * d * dv, heads * d * dv + copies * heads * d
+        for h in range(heads):
+            size_s, size_n = 0.0, 0.0       # the same sums over the numbers' sizes
+            s, nv, m = state[h * dv * d:(h + 1) * dv * d].reshape(dv, d).T, state[n_all + h * d:n_all + (h + 1) * d], state[m_all + h]
+            ref, bound = np.zeros((lengths[i], dv)), np.zeros((lengths[i], dv))
+            for j, t in enumerate(range(at.start, at.stop)):
+                new = max(lf[t, h] + m, li[t, h])
+                keep, take, m = np.exp(lf[t, h] + m - new), np.exp(li[t, h] - new), new
+                s, nv = keep * s + take * np.outer(k[t, h], v[t, h]), keep * nv + take * k[t, h]
+                qt = q[t, h] * d ** -0.5
+                size_s, size_n = keep * size_s + take * np.abs(np.outer(k[t, h], v[t, h])), keep * size_n + take * np.abs(k[t, h])
+                den = max(abs(nv @ qt), np.exp(-m)) + 1e-6
+                ref[j] = s.T @ qt / den
+                # numerator and denominator each off by less than 64 roundings of the sums of their terms' sizes (runs of up to 32
+                # terms in one chain, 16 in the next, and the roundings of gates and decays)
+                bound[j] = 64 * 2.0 ** -24 * (size_s.T + np.abs(ref[j])[:, None] * size_n) @ np.abs(qt) / den + 1e-6 * np.abs(ref[j])
+            assert np.all(np.abs(got[at, h] - ref) <= bound), (i, h)
+            assert np.all(np.abs(o_walk[at, h] - ref) <= bound), (i, h)
+            for c in range(copies):
+                assert _off(chunked[row, n_all + (c * heads + h) * d:n_all + (c * heads + h + 1) * d], nv) <= 4e-6, (i, h, c)
+                assert abs(chunked[row, m_all + c * heads + h] - m) <= 4e-6 * max(1.0, abs(m)), (i, h, c)
+            assert _off(chunked[row, h * dv * d:(h + 1) * dv * d].reshape(dv, d), s.T) <= 4e-6, (i, h)
