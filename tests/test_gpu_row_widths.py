@@ -39,6 +39,29 @@ def test_layer_norm_and_step(width, parts):
         assert float((out.double() - layer_norm64(x.double(), w2.double(), b2.double(), 1e-5)).abs().max()) <= bound
 
 
+@pytest.mark.parametrize("width", [4, 260, 2564, 4100, 8188])
+def test_rows_at_multiples_of_16_bytes_and_elsewhere(width):
+    """Widths of four columns a load: rows that begin elsewhere take a column a load, with the same result up to the order of the sums; a
+    bfloat16 result is the float32 one rounded."""
+    from kipp_amd.csrc import ops
+    rng = np.random.default_rng(width)
+
+    def moved(t):
+        return torch.cat([t.new_zeros(1), t.flatten()])[1:].view(t.shape)
+    x, u, w, b = f32(rng, 5, width), f32(rng, 2, 5, width), f32(rng, width), f32(rng, width)
+    steps = []
+    for place in (lambda t: t, moved):
+        xs, out = place(x.clone()), torch.empty((5, width), device=DEV)
+        ops.sandwich_step(xs, place(u), place(w), place(b), 1e-5, 0.5, None, place(w), place(b), 1e-5, out)
+        steps.append((xs, out, ops.layer_norm(place(u), place(w), place(b), 1e-5, torch.empty((5, width), device=DEV))))
+    for one, other in zip(*steps):      # both within the bound of the test above
+        assert float((one - other).abs().max()) <= 2 * 82 * 2.0 ** -24 * 25 * (4.0 if width == 4 else 1.0)      # (four numbers can be close to each other)
+    half, x2 = torch.empty((5, width), dtype=torch.bfloat16, device=DEV), x.clone()
+    ops.sandwich_step(x2, u, w, b, 1e-5, 0.5, None, w, b, 1e-5, half)
+    assert torch.equal(half, steps[0][1].bfloat16()) and torch.equal(x2, steps[0][0])
+    assert torch.equal(ops.layer_norm(u, w, b, 1e-5, torch.empty((5, width), dtype=torch.bfloat16, device=DEV)), steps[0][2].bfloat16())
+
+
 @pytest.mark.parametrize("span", [1, 16, 64, 65, 256, 257, 512, 513, 1024, 1025, 1536, 1537, 2560, 2561, 4096, 4097, 5120, 5121, 11000])
 @pytest.mark.parametrize("spans", [1, 3])
 def test_state_space_finish(span, spans):
