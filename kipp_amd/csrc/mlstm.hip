@@ -248,6 +248,99 @@ __global__ void __launch_bounds__(SCAN_THREADS) mlstm_scan_kernel(
     if (writes_copy && part == 0) m_all[(size_t)(col / unit) * heads + head] = m_s[0];
 }
 
+#define STEP_UNIT 16
+#define STEP_ROWS 8
+
+// Single tokens with keys of 33 to 128 numbers, a multiple of 8: a unit of 16 columns is one wave's, or two waves' of one workgroup, PASSES times four columns
+// by 16 lanes each, eight rows a lane, all of it asked for at once and straight from memory; gates and denominator are every wave's own.
+// Nothing goes through LDS and no wave waits for another.  The order of the sums is that of the build with eight rows a lane and 16 lanes a
+// column.  Bound by a chain of loads (lengths, slot, state) and gates up to a few entries, then by the state's bytes.  8 heads of 128 x 320, in
+// a recorded step, us, 1, 2, 4, 8, 16, 24 entries: two waves a unit 6.9, 6.7, 10.3, 14.7, 21.9, 31.3, one wave 8.7, 8.9, 9.8, 16.2, 22.2, 28.6,
+// through the walk 8.7, 8.9, 9.8, 18.7, 28.0, 37.2: two where all workgroups are resident at once, one beyond.  Keys of 256 (16 rows a lane)
+// gained nothing up to eight entries: they walk.
+template <int PASSES>
+__global__ void __launch_bounds__(SCAN_THREADS) mlstm_step_kernel(
+    const float* __restrict__ proj, int stride, const float* __restrict__ bias_i, const float* __restrict__ bias_f, float cap,
+    float* __restrict__ state, size_t state_stride, const int32_t* __restrict__ q_start, const int32_t* __restrict__ q_len,
+    const int32_t* __restrict__ slots, float* __restrict__ o_raw, int heads, int d, int dv, int copies) {
+    constexpr int ROWS = STEP_ROWS, HALVES = STEP_UNIT / 4 / PASSES;     // waves that share a unit
+    const int seq = blockIdx.x, head = blockIdx.y, lane = threadIdx.x & (KIPP_WAVE - 1), part = lane & 15;
+    const int wave = threadIdx.x / KIPP_WAVE, unit_of_wave = blockIdx.z * (SCAN_THREADS / KIPP_WAVE / HALVES) + wave / HALVES;
+    const int first = q_start[seq], count = q_len[seq];
+    if (count <= 0) return;                 // uniform over the workgroup
+    const int unit = min(unit_of_wave, copies - 1);
+    const bool mine = unit_of_wave < copies;
+    const int row0 = part * ROWS;
+    const bool rows = row0 < d;             // a lane's rows are all there or none
+    float* slot = state + (size_t)slots[seq] * state_stride;
+    float* n_g = slot + (size_t)heads * d * dv + ((size_t)unit * heads + head) * d + row0;
+    float* m_g = slot + (size_t)heads * d * dv + (size_t)copies * heads * d + (size_t)unit * heads + head;
+    const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    float S[PASSES][ROWS], nv[ROWS];
+    int col[PASSES];
+    float* S_g[PASSES];
+#pragma unroll
+    for (int c = 0; c < PASSES; ++c) {
+        col[c] = unit * STEP_UNIT + 4 * (PASSES * (wave % HALVES) + c) + (lane >> 4);
+        S_g[c] = slot + ((size_t)head * dv + min(col[c], dv - 1)) * d + row0;
+#pragma unroll
+        for (int r = 0; r < ROWS; r += 4) *reinterpret_cast<float4*>(S[c] + r) = rows ? *reinterpret_cast<const float4*>(S_g[c] + r) : zero;
+    }
+#pragma unroll
+    for (int r = 0; r < ROWS; r += 4) *reinterpret_cast<float4*>(nv + r) = rows ? *reinterpret_cast<const float4*>(n_g + r) : zero;
+    float m = *m_g;
+    const float q_scale = 1.0f / sqrtf((float)d), bi = bias_i[head], bf = bias_f[head];
+    for (int t = 0; t < count; ++t) {
+        const float* row = proj + (size_t)(first + t) * stride;
+        float kk[ROWS], qq[ROWS], v[PASSES];
+#pragma unroll
+        for (int r = 0; r < ROWS; r += 4) {
+            *reinterpret_cast<float4*>(kk + r) = rows ? *reinterpret_cast<const float4*>(row + (heads + head) * d + row0 + r) : zero;
+            *reinterpret_cast<float4*>(qq + r) = rows ? *reinterpret_cast<const float4*>(row + head * d + row0 + r) : zero;
+        }
+#pragma unroll
+        for (int c = 0; c < PASSES; ++c) v[c] = row[2 * heads * d + head * dv + min(col[c], dv - 1)];
+        const float* z = row + 2 * heads * d + 2 * heads * dv + head;
+        float li = cap * tanhf((z[0] + bi) / cap);
+        asm volatile("" : "+v"(li));        // a product for itself, as in the walk: not contracted into the difference below
+        const float lf = log_sigmoid(cap * tanhf((z[heads] + bf) / cap));
+        const float m_new = fmaxf(lf + m, li);
+        const float keep = expf(lf + m - m_new), take = expf(li - m_new), floor_p = expf(-m_new);
+        m = m_new;
+        float den = 0.0f;
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r) {
+            qq[r] *= q_scale;
+            nv[r] = fmaf(keep, nv[r], take * kk[r]);
+            den = fmaf(nv[r], qq[r], den);
+        }
+        den = fmaxf(fabsf(column_sum<16>(den)), floor_p) + 1e-6f;
+#pragma unroll
+        for (int c = 0; c < PASSES; ++c) {
+            const float tv = take * v[c];
+            float num = 0.0f;
+#pragma unroll
+            for (int r = 0; r < ROWS; ++r) {
+                S[c][r] = fmaf(keep, S[c][r], kk[r] * tv);
+                num = fmaf(S[c][r], qq[r], num);
+            }
+            num = column_sum<16>(num);
+            if (mine && part == 0 && col[c] < dv) o_raw[((size_t)(first + t) * heads + head) * dv + col[c]] = num / den;
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < PASSES; ++c)
+        if (mine && rows && col[c] < dv)
+#pragma unroll
+            for (int r = 0; r < ROWS; r += 4) *reinterpret_cast<float4*>(S_g[c] + r) = *reinterpret_cast<float4*>(S[c] + r);
+    __syncthreads();                        // the waves of a unit have read n and m
+    if (!mine || wave % HALVES != 0) return;
+    if (rows && lane < 16)
+#pragma unroll
+        for (int r = 0; r < ROWS; r += 4) *reinterpret_cast<float4*>(n_g + r) = *reinterpret_cast<float4*>(nv + r);
+    if (lane == 0) *m_g = m;
+}
+
 #define FINISH_HEADS 4
 
 template <typename TO>
@@ -278,7 +371,8 @@ static int kipp_mlstm_parts(int d) { return d <= 32 ? 4 : (d <= 256 ? 16 : 64); 
 extern "C" {
 
 // `few`: every entry brings few tokens (single decoded tokens): where the key size allows, a workgroup takes 64 columns
-// with 4 lanes each, a quarter of the workgroups, each reading longer runs of the state.  `below`: entries of so many tokens and more
+// with 4 lanes each, a quarter of the workgroups, each reading longer runs of the state.  `few` 2: every entry brings one token (`mlstm_step_kernel`
+// where it takes the sizes; `below` is not for that).  `below`: entries of so many tokens and more
 // are left alone (0: none).
 int kipp_mlstm_scan(const float* proj, int stride, const float* bias_i, const float* bias_f, float cap, float* state,
                     size_t state_stride, const int32_t* q_start, const int32_t* q_len, const int32_t* slots, float* o_raw,
@@ -291,6 +385,16 @@ int kipp_mlstm_scan(const float* proj, int stride, const float* bias_i, const fl
     const int base_parts = kipp_mlstm_parts(d);
     const int base_rows = d <= 128 ? 8 : (d <= 256 ? 16 : (d <= 512 ? 8 : 16));
     int parts = base_parts, rows = base_rows;
+    if (few == 2 && d > 32 && d <= 128 && d % STEP_ROWS == 0 && stride % 4 == 0 && state_stride % 4 == 0 && (((uintptr_t)proj | (uintptr_t)state) & 15) == 0) {
+        const int waves = SCAN_THREADS / KIPP_WAVE, pairs = (2 * copies + waves - 1) / waves;
+        if ((long long)n_seqs * heads * pairs <= 256)
+            hipLaunchKernelGGL(mlstm_step_kernel<2>, dim3(n_seqs, heads, pairs), dim3(SCAN_THREADS), 0, stream, proj, stride, bias_i, bias_f, cap, state, state_stride,
+                               q_start, q_len, slots, o_raw, heads, d, dv, copies);
+        else
+            hipLaunchKernelGGL(mlstm_step_kernel<4>, dim3(n_seqs, heads, (copies + waves - 1) / waves), dim3(SCAN_THREADS), 0, stream, proj, stride, bias_i, bias_f, cap,
+                               state, state_stride, q_start, q_len, slots, o_raw, heads, d, dv, copies);
+        return KIPP_LAUNCH_CHECK();
+    }
     if (few && d > 32 && d <= 128) parts = 4, rows = 32;
     else if (few && d > 128 && d <= 256) parts = 8, rows = 32;
     const int cols = SCAN_THREADS / parts;

@@ -644,9 +644,10 @@ def mlstm_state_size(heads: int, d: int, dv: int) -> int:
 
 def mlstm_scan(proj: torch.Tensor, bias_i: torch.Tensor, bias_f: torch.Tensor, cap: float, state: torch.Tensor,
                q_start: torch.Tensor, q_len: torch.Tensor, slots: torch.Tensor, o_raw: torch.Tensor,
-               heads: int, d: int, dv: int, few: bool = False, below: int = 0) -> torch.Tensor:
+               heads: int, d: int, dv: int, few: bool = False, below: int = 0, single: bool = False) -> torch.Tensor:
     """The recurrence over every entry's tokens, in order, from and into the entry's slot of `state` [slots, size]
-    (float32).  `few`: every entry brings few tokens (single decoded tokens): fewer, larger workgroups; the same bits.  `below`: entries of
+    (float32).  `few`: every entry brings few tokens (single decoded tokens): fewer, larger workgroups; the same bits.  `single`: every entry brings
+    one token at most; the same bits.  `below`: entries of
     so many tokens and more are left alone (0: none; what `mlstm_chunks` took).  `proj`: float32 [tokens, >= 2 heads d + 2 heads dv + 2 heads], columns q | k | v | gate | zi | zf;
     `o_raw` float32 [tokens, heads dv] receives S^T q over its denominator."""
     _dev(proj, bias_i, bias_f, state, q_start, q_len, slots, o_raw)
@@ -663,7 +664,7 @@ def mlstm_scan(proj: torch.Tensor, bias_i: torch.Tensor, bias_f: torch.Tensor, c
     fn = _fn("mlstm", "kipp_mlstm_scan", [_c_ptr, _c_int, _c_ptr, _c_ptr, _c_float, _c_ptr, _c_size, _c_ptr, _c_ptr, _c_ptr, _c_ptr,
                                           _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr])
     _check(fn(_ptr(proj), proj.shape[1], _ptr(bias_i), _ptr(bias_f), float(cap), _ptr(state), state.shape[1], _ptr(q_start),
-              _ptr(q_len), _ptr(slots), _ptr(o_raw), q_start.numel(), heads, d, dv, int(bool(few)), max(0, int(below)), _stream()), "mlstm_scan")
+              _ptr(q_len), _ptr(slots), _ptr(o_raw), q_start.numel(), heads, d, dv, 2 if single and below <= 0 else int(bool(few)), max(0, int(below)), _stream()), "mlstm_scan")
     return o_raw
 
 

@@ -86,7 +86,7 @@ class MLSTM:
         args = (proj, self.bias_i, self.bias_f, s.gate_cap, state, batch.q_start, batch.q_len, batch.slots, o_raw, s.num_heads, s.head_dim, s.v_head_dim)
         den, below = ops.mlstm_chunks(*args, longest=batch.max_q_len, portions=chunk_portions(batch)) if rt.dtype == "bfloat16" else (None, 0)
         if below >= 0:
-            ops.mlstm_scan(*args, few=batch.max_q_len <= 4, below=below)
+            ops.mlstm_scan(*args, few=batch.max_q_len <= 4, below=below, single=batch.max_q_len == 1)
         out = ops.mlstm_finish(o_raw, proj, 2 * s.num_heads * s.head_dim + hv, self.norm, s.norm_eps, rt.empty((n, hv), rt.act_dtype),
                                s.num_heads, s.v_head_dim, den=den)
         return rt.linear(out, self.w_o, slabs=True, defer=True)

@@ -205,3 +205,27 @@ def test_mlstm_chunks_beside_the_walk(d, dv, heads):
                 assert _off(chunked[row, n_all + (c * heads + h) * d:n_all + (c * heads + h + 1) * d], nv) <= 4e-6, (i, h, c)
                 assert abs(chunked[row, m_all + c * heads + h] - m) <= 4e-6 * max(1.0, abs(m)), (i, h, c)
             assert _off(chunked[row, h * dv * d:(h + 1) * dv * d].reshape(dv, d), s.T) <= 4e-6, (i, h)
+
+
+@pytest.mark.parametrize("d, dv, heads", [(40, 5, 2), (64, 16, 3), (128, 320, 2), (96, 33, 1), (88, 300, 8)])
+def test_mlstm_single_tokens_have_the_walks_bits(d, dv, heads):
+    """Steps of single tokens, an entry without one among them: results, S, every copy of n and of m as the walk leaves them."""
+    import torch
+    from kipp_amd.csrc import ops
+    gen = torch.Generator().manual_seed(d)
+    n, size = 5, ops.mlstm_state_size(heads, d, dv)
+    width = 2 * heads * d + 2 * heads * dv + 2 * heads
+    width += -width % 4
+    b = torch.randn((2, heads), generator=gen).to(DEV)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)  # noqa: E731
+    states = [torch.zeros((n + 1, size), device=DEV) for _ in range(2)]
+    for step in range(3):
+        proj = torch.randn((n, width), generator=gen).to(DEV)
+        got = []
+        for state, single in zip(states, (False, True)):
+            o = torch.zeros((n, heads * dv), device=DEV)
+            # (the walk takes every entry with a token; an entry without one is left alone by the other form)
+            entries = [0, 1, 3, 4] if not single else [0, 1, 2, 3, 4]
+            lens = [0 if e == 2 else 1 for e in entries]
+            got.append(ops.mlstm_scan(proj, b[0], b[1], 15.0, state, i32(entries), i32(lens), i32([5 - e for e in entries]), o, heads, d, dv, few=True, single=single))
+        assert torch.equal(*got) and torch.equal(*states), step
