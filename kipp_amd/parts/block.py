@@ -17,6 +17,7 @@ Interface of a block:
 """
 from __future__ import annotations
 
+from ..runtime import WeightedDelta
 from .base import build_part, register
 
 
@@ -168,8 +169,8 @@ class SandwichNormMixerBlock(SandwichNormBlock):
 @register("block", "parallel")
 class ParallelBlock:
     """One norm whose output both sublayers read: h = mixer_norm(x); x += mixer(h) + ffn(h).  The mixer's result is added
-    at once (a weighted sum of deltas term by term, where it lies); the feed-forward's is handed on and added inside the next
-    block's norm."""
+    at once, where it lies; the feed-forward's is handed on and added inside the next block's norm.  Where both are weighted
+    sums of deltas, which no norm adds in its own kernel, their terms are handed on together and added in one launch."""
 
     roles = (("mixer_norm", "norm"), ("mixer", "mixer"), ("ffn", "feed_forward"))
 
@@ -186,13 +187,14 @@ class ParallelBlock:
         h = norm.forward(x, rt.act_dtype) if pending is None else norm.add_forward(x, pending, rt.act_dtype)
         h = rt.rows_of(h)       # two readers: the rows are finished once
         delta = self.mixer.forward(h, batch, cache, state)
+        more = self.parts["ffn"].forward(h, batch) if "ffn" in self.parts else None
+        if isinstance(delta, WeightedDelta) and isinstance(more, WeightedDelta):
+            return x, delta.plus(more)
         if hasattr(delta, "add_to"):
             delta.add_to(x)
         else:
             rt.ops.residual_add(x, rt.settle(delta))
-        if "ffn" not in self.parts:
-            return x, None
-        return x, self.parts["ffn"].forward(h, batch)
+        return x, more
 
 
 @register("block", "parallel_mixer")

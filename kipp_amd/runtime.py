@@ -104,7 +104,7 @@ class Deferred(Pending):
 class WeightedDelta(Pending):
     """A weighted sum of deltas, each with the bias of the product that made it (or none): sum_i scale_i (delta_i + bias_i).
     `terms`: (delta, scale, bias) with delta a tensor, slabs of one or another `Pending`.  `add_to(x)` adds every term to
-    the residual stream where it lies (one launch a term, nothing kept in between); `run()` gives the sum as a tensor."""
+    the residual stream where it lies, several of them a launch; `run()` gives the sum as a tensor."""
     __slots__ = ("rt", "terms")
 
     def __init__(self, rt, terms):
@@ -121,17 +121,11 @@ class WeightedDelta(Pending):
         return WeightedDelta(self.rt, self.terms + WeightedDelta.of(self.rt, other).terms)
 
     def add_to(self, x):
-        for delta, scale, bias in self.terms:
-            self.rt.ops.residual_add_scaled(x, self.rt.settle(delta), scale, bias)
-        return x
+        return self.rt.ops.residual_add_terms(x, [(self.rt.settle(delta), scale, bias) for delta, scale, bias in self.terms])
 
     def run(self):
-        first = self.rt.settle(self.terms[0][0])
-        out = self.rt.ops.fill_zero(self.rt.empty(tuple(first.shape[-2:]), torch.float32))
-        self.rt.ops.residual_add_scaled(out, first, self.terms[0][1], self.terms[0][2])
-        for delta, scale, bias in self.terms[1:]:
-            self.rt.ops.residual_add_scaled(out, self.rt.settle(delta), scale, bias)
-        return out
+        self.terms = [(self.rt.settle(delta), scale, bias) for delta, scale, bias in self.terms]
+        return self.add_to(self.rt.ops.fill_zero(self.rt.empty(tuple(self.terms[0][0].shape[-2:]), torch.float32)))
 
 
 class ColumnScaled(Pending):

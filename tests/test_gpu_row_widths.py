@@ -62,6 +62,28 @@ def test_rows_at_multiples_of_16_bytes_and_elsewhere(width):
     assert torch.equal(ops.layer_norm(u, w, b, 1e-5, torch.empty((5, width), dtype=torch.bfloat16, device=DEV)), steps[0][2].bfloat16())
 
 
+@pytest.mark.parametrize("width", [1, 4, 63, 512, 516, 2560, 2561])
+def test_terms_of_a_weighted_sum_together(width):
+    """One to six terms, in slabs and not, with biases and without: the bits of a launch a term, also where rows begin anywhere."""
+    from kipp_amd.csrc import ops
+    rng = np.random.default_rng(width)
+    x = f32(rng, 5, width)
+    every = [(f32(rng, *((p,) if p > 1 else ()), 5, width), s, f32(rng, width) if b else None)
+             for p, s, b in ((1, 1.25, False), (3, 0.8, True), (6, -0.5, False), (2, 1.0, True), (1, 0.3, True), (4, 2.0, False))]
+    for count in range(1, 7):
+        one, together = x.clone(), x.clone()
+        for term in every[:count]:
+            ops.residual_add_scaled(one, *term)
+        ops.residual_add_terms(together, every[:count])
+        assert torch.equal(one, together), count
+        store = torch.zeros(x.numel() + 1, device=DEV)[1:].view(x.shape).copy_(x)
+        assert torch.equal(ops.residual_add_terms(store, every[:count]), one), count
+    ref = x.double()
+    for delta, scale, bias in every:
+        ref = ref + scale * ((delta.double().sum(0) if delta.dim() == 3 else delta.double()) + (0.0 if bias is None else bias.double()))
+    assert float((one.double() - ref).abs().max()) <= 24 * 2.0 ** -24 * 30      # 24 additions of numbers up to about 30
+
+
 @pytest.mark.parametrize("span", [1, 16, 64, 65, 256, 257, 512, 513, 1024, 1025, 1536, 1537, 2560, 2561, 4096, 4097, 5120, 5121, 11000])
 @pytest.mark.parametrize("spans", [1, 3])
 def test_state_space_finish(span, spans):
