@@ -134,19 +134,19 @@ class Model:
                     pending = pending.also_add(first)       # the norm that carries the pending delta out adds this as well
                 else:
                     if pending is not None:
-                        ops.residual_add(x, self.rt.settle(pending))
+                        self.rt.add(x, pending)
                         pending = None
                     ops.residual_add(x, first)
             x, pending = block.forward(x, pending, batch, view, cache.state(index))
             if self.residual_probe is not None:
                 if pending is not None:
-                    ops.residual_add(x, self.rt.settle(pending))
+                    self.rt.add(x, pending)
                     pending = None
                 self.residual_probe(index, x)
         if batch.n_want == 0:
             return None
         if pending is not None and not (batch.want_every_row and getattr(self.final_norm, "fuses_products", False)):
-            pending = self.rt.settle(pending)
+            pending = self.rt.settle_onto(x, pending)
         if batch.want_every_row:
             # every row in order (a step of single tokens): no gather, and the last delta is added inside the norm
             normed = (self.final_norm.forward(x, self.rt.act_dtype) if pending is None

@@ -38,7 +38,7 @@ class PreNormBlock:
         act = self.rt.act_dtype
         rt, norm1 = self.rt, self.parts["mixer_norm"]
         if pending is not None and not getattr(norm1, "fuses_products", False):
-            pending = rt.settle(pending)
+            pending = rt.settle_onto(x, pending)
         h = norm1.forward(x, act) if pending is None else norm1.add_forward(x, pending, act)
         if not getattr(self.mixer, "takes_scaled_rows", False):
             h = rt.rows_of(h)
@@ -110,7 +110,7 @@ class PostNormBlock:
     def forward(self, x, pending, batch, cache, state):
         rt = self.rt
         if pending is not None:
-            rt.ops.residual_add(x, rt.settle(pending))
+            rt.add(x, pending)
         h = self._rows(x, batch)
         h = self.parts["mixer_norm"].post_forward(x, self.mixer.forward(h, batch, cache, state), self.alpha, rt.act_dtype)
         if "ffn" in self.parts:
@@ -147,7 +147,7 @@ class SandwichNormBlock:
         from .norm import NormedDelta
         rt, act = self.rt, self.rt.act_dtype
         if pending is not None and not getattr(norm, "fuses_products", False):
-            pending = rt.settle(pending)
+            pending = rt.settle_onto(x, pending)
         h = rt.rows_of(norm.forward(x, act) if pending is None else norm.add_forward(x, pending, act))
         return NormedDelta(rt, rt.settle(run(h)), post_norm, self.alpha)
 
@@ -183,7 +183,7 @@ class ParallelBlock:
     def forward(self, x, pending, batch, cache, state):
         rt, norm = self.rt, self.parts["mixer_norm"]
         if pending is not None and not getattr(norm, "fuses_products", False):
-            pending = rt.settle(pending)
+            pending = rt.settle_onto(x, pending)
         h = norm.forward(x, rt.act_dtype) if pending is None else norm.add_forward(x, pending, rt.act_dtype)
         h = rt.rows_of(h)       # two readers: the rows are finished once
         delta = self.mixer.forward(h, batch, cache, state)

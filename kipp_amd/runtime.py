@@ -223,6 +223,19 @@ class Runtime:
         """The tensor of a delta, launched now if it was deferred."""
         return delta.run() if isinstance(delta, Pending) else delta
 
+    def settle_onto(self, x, delta):
+        """`settle` for a delta that is added to x next: a weighted sum is added here, term by term as a norm adds it (None is left to add)."""
+        if isinstance(delta, WeightedDelta):
+            delta.add_to(x)
+            return None
+        return self.settle(delta)
+
+    def add(self, x, delta):
+        """x += delta, pending or not."""
+        delta = self.settle_onto(x, delta)
+        if delta is not None:
+            self.ops.residual_add(x, delta)
+
     def rows_of(self, h):
         """The tensor of norm output, scaled now if the scale was left to a product."""
         if not isinstance(h, ScaledRows):
