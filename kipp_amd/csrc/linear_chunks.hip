@@ -122,7 +122,7 @@ struct ChunkArgs {
     const int32_t *q_start, *q_len, *slots;
     float* o_raw;
     float *a, *t, *vec;         // [chunk][head][64][64], the same (delta), [chunk][head][4][64]: G, D[last], beta (mLSTM: the input gate), mLSTM's floor of a denominator
-    int heads, qk_rep, d, dv, entries, from;
+    int heads, qk_rep, d, dv, entries, from, portions;
     // mLSTM: the gates' columns and biases, their cap, where a slot's copies of n begin and how many there are, 1 / sqrt(d), and what a
     // token's sums are divided by, [token][head]
     const float *bias_i, *bias_f;
@@ -158,14 +158,17 @@ __global__ void __launch_bounds__(GATE_WAVES * KIPP_WAVE) chunks_gates_kernel(co
         if (tid < n) p.den[(size_t)(first + tid) * p.heads + head] = 1.0f;      // `from` is less than the threads
         return;
     }
-    int base = 0;       // chunks of the entries ahead, as `portion_of` counts them
+    int base = 0, ahead = 0;        // chunks of the entries ahead, as `portion_of` counts them, and how many entries those are
     for (int e0 = 0; e0 < entry; e0 += KIPP_WAVE) {
         const int len = e0 + lane < entry ? p.q_len[e0 + lane] : 0;
-        int chunks = len > 0 && len >= p.from ? (len + CHUNK - 1) / CHUNK : 0;
+        const bool portion = len > 0 && len >= p.from;
+        int chunks = portion ? (len + CHUNK - 1) / CHUNK : 0;
 #pragma unroll
         for (int off = KIPP_WAVE / 2; off > 0; off >>= 1) chunks += __shfl_xor(chunks, off, KIPP_WAVE);
         base += chunks;
+        ahead += __popcll(__ballot(portion));
     }
+    if (ahead >= p.portions) return;        // beyond what the work space is laid out for and the other kernels take; uniform over the workgroup
     float* m_all = p.state + (size_t)p.slots[entry] * p.state_stride + p.n_at + (size_t)p.copies * p.heads * (p.d);
     float m = m_all[head];
     const float bi = p.bias_i[head], bf = p.bias_f[head];
@@ -567,6 +570,7 @@ int kipp_matrix_chunks(int mode, const float* src, int stride, int q_at, int k_a
     p.dv = dv;
     p.entries = entries;
     p.from = from;
+    p.portions = portions;
     if (mode == MODE_DECAY) launch_mode<MODE_DECAY>(p, longest, portions, stream);
     else if (mode == MODE_DELTA) launch_mode<MODE_DELTA>(p, longest, portions, stream);
     else launch_mode<MODE_GATED>(p, longest, portions, stream);
@@ -613,6 +617,7 @@ int kipp_mlstm_chunks(const float* proj, int stride, const float* bias_i, const 
     p.dv = dv;
     p.entries = entries;
     p.from = from;
+    p.portions = portions;
     hipLaunchKernelGGL(chunks_gates_kernel, dim3(heads, entries), dim3(GATE_WAVES * KIPP_WAVE), 0, stream, p);
     launch_mode<MODE_MLSTM>(p, longest, portions, stream);
     return KIPP_LAUNCH_CHECK();

@@ -229,3 +229,28 @@ def test_mlstm_single_tokens_have_the_walks_bits(d, dv, heads):
             lens = [0 if e == 2 else 1 for e in entries]
             got.append(ops.mlstm_scan(proj, b[0], b[1], 15.0, state, i32(entries), i32(lens), i32([5 - e for e in entries]), o, heads, d, dv, few=True, single=single))
         assert torch.equal(*got) and torch.equal(*states), step
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_mlstm_entries_beyond_the_portions_are_left_alone(d):
+    """Fewer `portions` than entries that bring so many tokens: the first are as they are without the others, and of the others neither
+    S nor n nor m moves."""
+    import torch
+    from kipp_amd.csrc import ops
+    heads, dv, lens = 2, 20, [64, 1, 65, 64]
+    gen = torch.Generator().manual_seed(d)
+    proj = torch.randn((sum(lens), 2 * heads * (d + dv) + 2 * heads), generator=gen).to(DEV)
+    bias = torch.randn((2, heads), generator=gen).to(DEV)
+    kept = torch.randn((len(lens), ops.mlstm_state_size(heads, d, dv)), generator=gen).to(DEV)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)  # noqa: E731
+
+    def run(lens, portions):
+        state, o = kept.clone(), torch.zeros((proj.shape[0], heads * dv), device=DEV)
+        den, below = ops.mlstm_chunks(proj, bias[0], bias[1], 15.0, state, i32([0, 64, 65, 130][:len(lens)]), i32(lens), i32([3, 2, 1, 0][:len(lens)]), o, heads, d, dv,
+                                      longest=65, portions=portions)
+        assert below == ops.CHUNKS_FROM
+        return state, o[:64], den[:65]
+    some, alone = run(lens, 1), run(lens[:2], 1)
+    for a, b in zip(some, alone):
+        assert torch.equal(a, b)
+    assert not torch.equal(some[0][3], kept[3]) and torch.equal(some[0][:3], kept[:3])
