@@ -137,7 +137,8 @@ gemm_f32_rows_kernel(const float* __restrict__ X, const TW* __restrict__ W, floa
 }
 
 // A wave stages its own steps of 32 numbers of k in its own part of LDS, so no wave waits for another before the sums.  A row's 128
-// bytes lie at 128 times the row in it, 16 byte piece c at place c ^ (row / 2 mod 8): reads and writes then meet every bank once.
+// bytes lie at 128 times the row in it, 16 byte piece c at place c ^ (row / 2 mod 8): reads and writes then meet every bank once.  A lane
+// reads what others of its wave wrote: LDS is in order within a wave, and the wave's barriers keep the compiler to that order.
 template <typename TW, int NT, int MT, bool VEC>
 __global__ void __launch_bounds__(ROWS_THREADS, 2)
 gemm_f32_tiles_kernel(const float* __restrict__ X, const TW* __restrict__ W, float* __restrict__ Y, int M, int N, int K, int n_tiles, int m_tiles) {
@@ -200,6 +201,7 @@ gemm_f32_tiles_kernel(const float* __restrict__ X, const TW* __restrict__ W, flo
             put(i);
             fetch(i, min(k_lo + STEP, last));
         }
+        __builtin_amdgcn_wave_barrier();
 #pragma unroll
         for (int r = 0; r < READS; ++r) take(0, r);
         for (int k0 = k_lo; k0 <= last; k0 += STEP) {       // behind the last step it is asked for again
@@ -213,12 +215,14 @@ gemm_f32_tiles_kernel(const float* __restrict__ X, const TW* __restrict__ W, flo
                     if (q < READS) {
                         take(1, q);
                     } else {
+                        if (q == READS) __builtin_amdgcn_wave_barrier();
                         put(q - READS);
                         fetch(q - READS, ahead);
                     }
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
+            __builtin_amdgcn_wave_barrier();
 #pragma unroll
             for (int p = 0; p < PRODUCTS; ++p) {
                 product(1, p);
@@ -229,12 +233,14 @@ gemm_f32_tiles_kernel(const float* __restrict__ X, const TW* __restrict__ W, flo
     }
     const int rest = k_lo + steps * STEP;
     if (rest < k_hi) {                              // what K leaves of a step
+        __builtin_amdgcn_wave_barrier();
 #pragma unroll
         for (int i = 0; i < LOADS; ++i) {
             next[i] = i < 2 * NT ? four<VEC>(w_base + (size_t)(8 * i + ld_row) * K, rest + ld_k, K)
                                  : four<VEC>(x_base + x_src[i < 2 * NT ? 0 : i - 2 * NT] - ld_k, rest + ld_k, K);
             put(i);
         }
+        __builtin_amdgcn_wave_barrier();
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
             if (rest + 16 * j >= k_hi) continue;
