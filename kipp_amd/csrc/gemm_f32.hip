@@ -6,14 +6,16 @@
 // An output's bits depend on its two rows and K alone, not on M, on the tile it falls in or on what else is in the
 // batch.  K is cut into KPARTS runs of `part_of(K)` numbers (the last ones shorter or empty); a run is one chain of
 // instructions, four numbers of k each (16 j + i, + 4, + 8, + 12 for i = 0..3, j counting up from the run's start), and the runs' sums are added
-// in order.  Both kernels below do exactly that, W always the instruction's first operand and X its second.
+// in order.  All kernels below do exactly that, W always the instruction's first operand and X its second.
 //
-//   rows   up to 16 rows of X a workgroup: 16 rows of W, a wave a run of K, straight from memory into the instruction's
+//   rows   up to 16 rows of X a workgroup (32 or 64 for short K): 16 rows of W, a wave a run of K, straight from memory into the instruction's
 //          operands (16 bytes a lane), the runs' sums added through LDS.  Bound by the read of W.  A 16-column fragment of
 //          X is multiplied whether its rows are there or not: at one row the matrix cores could feed 19 TB/s.
 //   tiles  more rows: 64 or 32 rows of W times 64, 48 or 32 of X a workgroup, a wave a run of K here too, so that every wave of a
 //          workgroup multiplies all of its outputs and none waits for another in the walk.  Bound by the instruction's rate (80 %
 //          of it at 1,024 rows) and, below a few rounds of tiles, by what the last round leaves idle: the shape goes by that.
+//   shared 64 x 64 outputs a workgroup of four waves, which meet at a barrier every 32 numbers of k: short K in many tiles, where a run a wave
+//          does not pay (`form_of`).
 // Measured at the 4B shape, W in turn from three copies, us: one row against 19,456 x 2,560 46 (4.3 TB/s), 2,560 x 9,728 34, the head's
 // 151,936 x 2,560 325 (4.8 TB/s).  The tiles, against 19,456 x 2,560 / 6,144 x 2,560 / 2,560 x 4,096 / 2,560 x 9,728, beside what these
 // rows took before (up to 64 rows of X through the kernel for rows, 64 x 64 tiles of four waves that share a step of K beyond):
@@ -31,6 +33,9 @@
 #define UNITS 256           // compute units
 #define XCDS 8              // dies of the chip; consecutive workgroups of a launch go to them in turn
 #define ROWS_THREADS (KPARTS * KIPP_WAVE)
+#define SHARED_TILE 64
+#define SHARED_THREADS 256
+#define PITCH 36            // floats from a row to the next of a shared tile's operands in LDS: 16 bytes a lane spread over the banks
 
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 
@@ -94,44 +99,53 @@ __device__ __forceinline__ f32x4 mul16(f32x4 w, f32x4 x, f32x4 acc) {
 }
 
 // The sums of a fragment lie in lane l as rows 4 (l / 16) .. + 3 (of W) of column l % 16 (a row of X).
-template <typename TW, bool VEC>
+template <typename TW, int MT, bool VEC>
 __global__ void __launch_bounds__(ROWS_THREADS)
 gemm_f32_rows_kernel(const float* __restrict__ X, const TW* __restrict__ W, float* __restrict__ Y, int M, int N, int K) {
-    __shared__ __attribute__((aligned(16))) float part_s[KPARTS][KIPP_WAVE][4];
+    __shared__ __attribute__((aligned(16))) float part_s[KPARTS][MT][KIPP_WAVE][4];
     const int wave = threadIdx.x / KIPP_WAVE, lane = threadIdx.x & (KIPP_WAVE - 1);
     const int l16 = lane & 15, h4 = 4 * (lane >> 4);
-    const int blocks = (N + 15) / 16, n0 = blockIdx.x % blocks * 16, m0 = blockIdx.x / blocks * 16;
+    const int blocks = (N + 15) / 16, n0 = blockIdx.x % blocks * 16, m0 = blockIdx.x / blocks * (16 * MT);
     const TW* w_row = W + (size_t)min(n0 + l16, N - 1) * K;         // rows beyond the last read it and are not stored
-    const float* x_row = X + (size_t)min(m0 + l16, M - 1) * K;
+    const float* x_row[MT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i) x_row[i] = X + (size_t)min(m0 + 16 * i + l16, M - 1) * K;
     const int part = part_of(K);
     const int k_lo = wave * part, k_hi = min(K, k_lo + part);
-    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-    constexpr int AHEAD = 8;       // 16-number pieces asked for together
+    f32x4 acc[MT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i) acc[i] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+    constexpr int AHEAD = MT == 1 ? 8 : (MT == 2 ? 6 : 4);       // 16-number pieces asked for together
     int k = k_lo;
     for (; k + 16 * AHEAD <= k_hi; k += 16 * AHEAD) {
-        f32x4 w[AHEAD], x[AHEAD];
+        f32x4 w[AHEAD], x[AHEAD][MT];
 #pragma unroll
         for (int j = 0; j < AHEAD; ++j) {
             w[j] = four<VEC>(w_row, k + 16 * j + h4, K);
-            x[j] = four<VEC>(x_row, k + 16 * j + h4, K);
+#pragma unroll
+            for (int i = 0; i < MT; ++i) x[j][i] = four<VEC>(x_row[i], k + 16 * j + h4, K);
         }
 #pragma unroll
-        for (int j = 0; j < AHEAD; ++j) acc = mul16(w[j], x[j], acc);
+        for (int j = 0; j < AHEAD; ++j)
+#pragma unroll
+            for (int i = 0; i < MT; ++i) acc[i] = mul16(w[j], x[j][i], acc[i]);
     }
     for (; k < k_hi; k += 16) {
         const f32x4 w = four<VEC>(w_row, k + h4, K);
-        acc = mul16(w, four<VEC>(x_row, k + h4, K), acc);
+#pragma unroll
+        for (int i = 0; i < MT; ++i) acc[i] = mul16(w, four<VEC>(x_row[i], k + h4, K), acc[i]);
     }
-    *reinterpret_cast<f32x4*>(part_s[wave][lane]) = acc;
+#pragma unroll
+    for (int i = 0; i < MT; ++i) *reinterpret_cast<f32x4*>(part_s[wave][i][lane]) = acc[i];
     __syncthreads();
     // a thread an output: the runs' sums in order
-    if (threadIdx.x < 256) {
-        const int at = threadIdx.x;             // place in the fragment: column 16 numbers of n long
-        const int n = n0 + (at & 15), m = m0 + (at >> 4);
+    for (int e = threadIdx.x; e < MT * 256; e += ROWS_THREADS) {
+        const int i = e >> 8, at = e & 255;             // fragment; place in it: column 16 numbers of n long
+        const int n = n0 + (at & 15), m = m0 + 16 * i + (at >> 4);
         const int from = 16 * ((at & 15) >> 2) + (at >> 4);
         float total = 0.0f;
 #pragma unroll
-        for (int p = 0; p < KPARTS; ++p) total += part_s[p][from][at & 3];
+        for (int p = 0; p < KPARTS; ++p) total += part_s[p][i][from][at & 3];
         if (m < M && n < N) Y[(size_t)m * N + n] = total;
     }
 }
@@ -274,6 +288,102 @@ gemm_f32_tiles_kernel(const float* __restrict__ X, const TW* __restrict__ W, flo
     }
 }
 
+// Four waves of 32 x 32 share a step of 64 rows of either operand, the next one's on its way in registers; a run's sums are added where it ends.
+template <typename TW, bool VEC>
+__global__ void __launch_bounds__(SHARED_THREADS)
+gemm_f32_shared_kernel(const float* __restrict__ X, const TW* __restrict__ W, float* __restrict__ Y, int M, int N, int K) {
+    __shared__ __attribute__((aligned(16))) float w_s[2][SHARED_TILE * PITCH];
+    __shared__ __attribute__((aligned(16))) float x_s[2][SHARED_TILE * PITCH];
+    const int tid = threadIdx.x;
+    const int wave = tid / KIPP_WAVE, lane = tid & (KIPP_WAVE - 1);
+    const int l16 = lane & 15, h4 = 4 * (lane >> 4);
+    const int n0 = blockIdx.x * SHARED_TILE, m0 = blockIdx.y * SHARED_TILE;
+    const int wn = (wave & 1) * 32, wm = (wave >> 1) * 32;
+    // from memory a thread takes 16 bytes of rows tid / 8 and tid / 8 + 32: eight lanes a row's 128 bytes
+    const int ld_row = tid >> 3, ld_k = (tid & 7) * 4;
+    const TW* w_row[2];
+    const float* x_row[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        w_row[i] = W + (size_t)min(n0 + ld_row + 32 * i, N - 1) * K;
+        x_row[i] = X + (size_t)min(m0 + ld_row + 32 * i, M - 1) * K;
+    }
+    f32x4 w_r[2], x_r[2];
+    auto fetch = [&](int k0) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            w_r[i] = four<VEC>(w_row[i], k0 + ld_k, K);
+            x_r[i] = four<VEC>(x_row[i], k0 + ld_k, K);
+        }
+    };
+    auto stage = [&](int buf) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            *reinterpret_cast<f32x4*>(&w_s[buf][(ld_row + 32 * i) * PITCH + ld_k]) = w_r[i];
+            *reinterpret_cast<f32x4*>(&x_s[buf][(ld_row + 32 * i) * PITCH + ld_k]) = x_r[i];
+        }
+    };
+    f32x4 acc[2][2], total[2][2];
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b) acc[a][b] = total[a][b] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+    const int part = part_of(K);
+    int until = part;           // where the run under way ends
+    fetch(0);
+    stage(0);
+    __syncthreads();
+    int buf = 0;
+    for (int k0 = 0; k0 < K; k0 += STEP, buf ^= 1) {
+        const bool more = k0 + STEP < K;
+        if (more) fetch(k0 + STEP);
+#pragma unroll
+        for (int j = 0; j < STEP; j += 16) {
+            if (k0 + j >= K) break;
+            f32x4 w[2], x[2];
+#pragma unroll
+            for (int a = 0; a < 2; ++a) {
+                w[a] = *reinterpret_cast<const f32x4*>(&w_s[buf][(wn + 16 * a + l16) * PITCH + j + h4]);
+                x[a] = *reinterpret_cast<const f32x4*>(&x_s[buf][(wm + 16 * a + l16) * PITCH + j + h4]);
+            }
+            // the four sums side by side: an instruction does not wait for the one before
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int a = 0; a < 2; ++a)
+#pragma unroll
+                    for (int b = 0; b < 2; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[a][i], x[b][i], acc[a][b], 0, 0, 0);
+        }
+        if (k0 + STEP == until || !more) {
+            until += part;
+#pragma unroll
+            for (int a = 0; a < 2; ++a)
+#pragma unroll
+                for (int b = 0; b < 2; ++b) {
+                    total[a][b] += acc[a][b];
+                    acc[a][b] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+                }
+        }
+        if (more) stage(buf ^ 1);
+        __syncthreads();
+    }
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            const int m = m0 + wm + 16 * b + l16, n = n0 + wn + 16 * a + h4;
+            if (m >= M) continue;
+            float* y = Y + (size_t)m * N + n;
+            if ((N & 3) == 0 && ((uintptr_t)Y & 15) == 0) {
+                if (n < N) *reinterpret_cast<f32x4*>(y) = total[a][b];
+            } else {
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+                    if (n + v < N) y[v] = total[a][b][v];
+            }
+        }
+}
+
 template <typename TW, int NT, int MT, bool VEC>
 static void launch_tiles(const float* X, const TW* W, float* Y, int M, int N, int K, hipStream_t stream) {
     const int n_tiles = (N + 16 * NT - 1) / (16 * NT), m_tiles = (M + 16 * MT - 1) / (16 * MT);
@@ -289,26 +399,66 @@ static long long tile_price(int M, int N, int nt, int mt) {
     return (tiles + UNITS - 1) / UNITS * (nt * mt + 2);
 }
 
-template <typename TW, bool VEC>
-static int launch(const float* X, const TW* W, float* Y, int M, int N, int K, hipStream_t stream) {
-    if (M <= 16 || N < 32) {        // tiles hold 32 rows of W or more
-        hipLaunchKernelGGL((gemm_f32_rows_kernel<TW, VEC>), dim3((N + 15) / 16 * ((M + 15) / 16)), dim3(ROWS_THREADS), 0, stream, X, W, Y, M, N, K);
-        return KIPP_LAUNCH_CHECK();
+// The kernel of a product: 1, 2 or 4 (rows, so many fragments of X), 0 (shared tiles) or 10 nt + mt (tiles).
+// A short K is a few steps for every wave of a tile, or none for most: its eight sums through LDS, the requests ahead of what is there and the part of a
+// step that K ends with then cost more than the products.  Up to 32 rows the kernel for rows is the faster one up to the K below (17 rows and K of 256 by
+// 19 %, 500 by 30 %, 32 rows and 512 by 5 %).  With more rows the prices, in us, were fitted to 3,773 products (32 to 19,456 rows of W, 65 to 4,096 of
+// X, K from 16 to 4,100; shared tiles 5 % off, tiles 8 %): a round of shared tiles by its steps, and of tiles by the steps of a run, fragments, runs and what
+// the last run takes longer where K ends inside a step; numbers one at a time (`vec` false) cost both more.  By them 8,422 products take 0.2 % more than
+// the faster way in the mean, 25 % at most; tiles alone take up to 4.2 times as long (2,048 rows against 9,728 x 16 / 64 / 256 / 768, us, shared and
+// tiles: 23 / 95, 41 / 106, 114 / 158, 302 / 327; against 2,560 x 192 30 / 40, and 2,560 x 1,100 122 / 137).
+static int form_of(int M, int N, int K, bool vec) {
+    if (M <= 16 || N < 32) return 1;        // tiles hold 32 rows of W or more
+    const long long shared = (long long)((M + SHARED_TILE - 1) / SHARED_TILE) * ((N + SHARED_TILE - 1) / SHARED_TILE);
+    const bool few = M <= 64 || (M <= 256 && shared < 192), rest = K % STEP != 0;
+    if (M <= 32) {
+        const int most = vec ? (rest ? 1616 : 1040) - 16 * M : 224, most_wide = vec && rest ? 320 : 64;
+        if (K <= (N <= 4096 ? most : min(most, most_wide))) return 2;
     }
+    if (few && K < STEP) return M <= 32 ? 2 : 4;
     static const int shapes[5][2] = {{4, 4}, {4, 3}, {4, 2}, {2, 3}, {2, 2}};
     int best = 4;
     for (int i = 3; i >= 0; --i)
         if (N >= 64 || shapes[i][0] == 2)
             if (tile_price(M, N, shapes[i][0], shapes[i][1]) <= tile_price(M, N, shapes[best][0], shapes[best][1])) best = i;
-    switch (best) {
-        case 0: launch_tiles<TW, 4, 4, VEC>(X, W, Y, M, N, K, stream); break;
-        case 1: launch_tiles<TW, 4, 3, VEC>(X, W, Y, M, N, K, stream); break;
-        case 2: launch_tiles<TW, 4, 2, VEC>(X, W, Y, M, N, K, stream); break;
-        case 3: launch_tiles<TW, 2, 3, VEC>(X, W, Y, M, N, K, stream); break;
-        default: launch_tiles<TW, 2, 2, VEC>(X, W, Y, M, N, K, stream); break;
+    const int nt = shapes[best][0], mt = shapes[best][1];
+    if (!few) {
+        const int part = part_of(K), steps = part / STEP, runs = (K + part - 1) / part;
+        const int longer = rest ? max(0, (K - (runs - 1) * part) / STEP + 2 - (runs > 1 ? steps : 0)) : 0;
+        const long long rounds = tile_price(M, N, nt, mt) / (nt * mt + 2), shared_rounds = (shared + UNITS - 1) / UNITS;
+        const double tile = 0.18 + 0.50 * steps + (0.217 * steps + 0.038 * runs) * nt * mt + 0.29 * longer + (vec ? 0.0 : (0.56 + 0.02 * nt * mt) * steps);
+        const double shared_tile = 1.21 + (vec ? 0.876 : 1.42) * ((K + STEP - 1) / STEP);
+        if (2.23 + shared_tile * (1.0 + 0.664 * (shared_rounds - 1)) < 2.15 + tile * (1.0 + 0.968 * (rounds - 1))) return 0;
+    }
+    return 10 * nt + mt;
+}
+
+template <typename TW, int MT, bool VEC>
+static void launch_rows(const float* X, const TW* W, float* Y, int M, int N, int K, hipStream_t stream) {
+    const dim3 grid((N + 15) / 16 * ((M + 16 * MT - 1) / (16 * MT)));
+    hipLaunchKernelGGL((gemm_f32_rows_kernel<TW, MT, VEC>), grid, dim3(ROWS_THREADS), 0, stream, X, W, Y, M, N, K);
+}
+
+template <typename TW, bool VEC>
+static int launch(const float* X, const TW* W, float* Y, int M, int N, int K, hipStream_t stream) {
+    switch (form_of(M, N, K, VEC)) {
+        case 1: launch_rows<TW, 1, VEC>(X, W, Y, M, N, K, stream); break;
+        case 2: launch_rows<TW, 2, VEC>(X, W, Y, M, N, K, stream); break;
+        case 4: launch_rows<TW, 4, VEC>(X, W, Y, M, N, K, stream); break;
+        case 44: launch_tiles<TW, 4, 4, VEC>(X, W, Y, M, N, K, stream); break;
+        case 43: launch_tiles<TW, 4, 3, VEC>(X, W, Y, M, N, K, stream); break;
+        case 42: launch_tiles<TW, 4, 2, VEC>(X, W, Y, M, N, K, stream); break;
+        case 23: launch_tiles<TW, 2, 3, VEC>(X, W, Y, M, N, K, stream); break;
+        case 22: launch_tiles<TW, 2, 2, VEC>(X, W, Y, M, N, K, stream); break;
+        default: {
+            const dim3 grid((N + SHARED_TILE - 1) / SHARED_TILE, (M + SHARED_TILE - 1) / SHARED_TILE);
+            hipLaunchKernelGGL((gemm_f32_shared_kernel<TW, VEC>), grid, dim3(SHARED_THREADS), 0, stream, X, W, Y, M, N, K);
+        }
     }
     return KIPP_LAUNCH_CHECK();
 }
+
+extern "C" int kipp_gemm_f32_form(int M, int N, int K) { return form_of(M, N, K, K % 4 == 0); }
 
 extern "C" int kipp_gemm_f32(const float* X, const void* W, int w_dtype, float* Y, int M, int N, int K,
                              hipStream_t stream) {

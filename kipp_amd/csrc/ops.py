@@ -2160,6 +2160,12 @@ def gemm_f32(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> torch.Tenso
     return out
 
 
+def gemm_f32_form(m: int, n: int, k: int) -> int:
+    """Which kernel `gemm_f32` launches for operands that begin at multiples of 16 bytes: 1, 2 or 4 for the one for rows with so many fragments of x, 0 for 64 x 64 tiles that four waves
+    share, 10 a + b for tiles of 16 a rows of w and 16 b of x in which a wave has a run of K."""
+    return _fn("gemm_f32", "kipp_gemm_f32_form", [_c_int] * 3)(m, n, k)
+
+
 # --------------------------------------------------------------------------- probe
 
 def stream_read(buffer: torch.Tensor, workgroups: int, depth: int = 8) -> int:

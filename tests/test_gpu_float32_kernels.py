@@ -50,6 +50,39 @@ def test_product_in_every_shape_of_tiles(m, n, k):
         assert torch.equal(ops.gemm_f32(x[lo:lo + 16].contiguous(), w, torch.empty((min(16, m - lo), n), device=DEV)), full[lo:lo + 16]), lo
 
 
+@pytest.mark.parametrize("m, n, form", [(33, 47, 22), (97, 2570, 23), (64, 6144, 42), (31, 9731, 42), (200, 6155, 43), (333, 2570, 44)])
+@pytest.mark.parametrize("k", [1068, 1069])
+def test_tiles_over_several_steps_of_k(m, n, form, k):
+    """Every shape of tiles where a wave's run has more steps than are asked for ahead and the last run ends inside one; weights in both
+    types, rows that begin anywhere (K of 1,069): every row as the kernel for up to 16 rows makes it."""
+    import torch
+    from kipp_amd.csrc import ops
+    assert ops.gemm_f32_form(m, n, k) == form
+    gen = torch.Generator().manual_seed(m + n + k)
+    x, wf = torch.randn((m, k), generator=gen).to(DEV), torch.randn((n, k), generator=gen).to(DEV)
+    for w in (wf, wf.bfloat16()):
+        full = ops.gemm_f32(x, w, torch.empty((m, n), device=DEV))
+        for lo in range(0, m, 16):
+            part = x[lo:lo + 16].contiguous()
+            assert torch.equal(ops.gemm_f32(part, w, torch.empty((len(part), n), device=DEV)), full[lo:lo + 16]), (w.dtype, lo)
+
+
+@pytest.mark.parametrize("m, n, k, form", [(17, 32, 40, 2), (32, 2563, 268, 2), (31, 100, 500, 2), (19, 100, 201, 2), (33, 130, 31, 4), (130, 1000, 16, 4), (350, 3001, 40, 0), (333, 2570, 268, 0),
+                                           (700, 2561, 257, 0), (2000, 1030, 33, 0)])
+def test_products_of_a_short_k(m, n, k, form):
+    """The kernels that short K goes through, at ends of tiles, steps and runs: every row as the kernel for up to 16 rows makes it."""
+    import torch
+    from kipp_amd.csrc import ops
+    assert ops.gemm_f32_form(m, n, k) == form
+    gen = torch.Generator().manual_seed(m + n + k)
+    x, wf = torch.randn((m, k), generator=gen).to(DEV), torch.randn((n, k), generator=gen).to(DEV)
+    for w in (wf, wf.bfloat16()):
+        full = ops.gemm_f32(x, w, torch.empty((m, n), device=DEV))
+        for lo in sorted({0, m // 32 * 16, m - 16}):
+            part = x[lo:lo + 16].contiguous()
+            assert torch.equal(ops.gemm_f32(part, w, torch.empty((16, n), device=DEV)), full[lo:lo + 16]), (w.dtype, lo)
+
+
 def test_product_of_rows_that_begin_anywhere():
     """Operands at addresses that 16-byte loads do not take."""
     import torch
