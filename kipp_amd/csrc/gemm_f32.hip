@@ -422,7 +422,10 @@ static int form_of(int M, int N, int K, bool vec) {
         if (N >= 64 || shapes[i][0] == 2)
             if (tile_price(M, N, shapes[i][0], shapes[i][1]) <= tile_price(M, N, shapes[best][0], shapes[best][1])) best = i;
     const int nt = shapes[best][0], mt = shapes[best][1];
-    if (!few) {
+    // a tile's offsets into X have 32 bits, and a launch less than 2^32 threads, 2^16 tiles down a grid's second side
+    const long long tiles = tile_price(M, N, nt, mt) / (nt * mt + 2) * UNITS;
+    if (K > 1 << 26 || tiles >= 1LL << 23) return 0;
+    if (!few && (M + SHARED_TILE - 1) / SHARED_TILE < 1 << 16) {
         const int part = part_of(K), steps = part / STEP, runs = (K + part - 1) / part;
         const int longer = rest ? max(0, (K - (runs - 1) * part) / STEP + 2 - (runs > 1 ? steps : 0)) : 0;
         const long long rounds = tile_price(M, N, nt, mt) / (nt * mt + 2), shared_rounds = (shared + UNITS - 1) / UNITS;

@@ -12,3 +12,11 @@ from kipp_amd.csrc import ops
 def test_the_form_that_was_the_faster_one(m, n, k, form):
     """Sizes at which one kernel took 5 % less than the other, and the 4B shape's."""
     assert ops.gemm_f32_form(m, n, k) == form
+
+
+@pytest.mark.parametrize("m, n, k, form", [
+    (64, 6144, 1 << 26, 42), (20, 64, (1 << 26) + 4, 0), (64, 6144, (1 << 26) + 4, 0),      # 63 rows of x in 32 bits, and not
+    (1 << 18, 1 << 16, 4096, 44), (1 << 18, 1 << 17, 4096, 0),                              # workgroups of 512 threads that one launch holds, and not
+    (5_000_000, 64, 64, 44), (4_000_000, 64, 64, 0)])                                       # 64 x 64 tiles that a grid's second side holds, and not
+def test_sizes_beyond_what_a_kernel_addresses(m, n, k, form):
+    assert ops.gemm_f32_form(m, n, k) == form
