@@ -10,9 +10,10 @@
 // first sum.  Bound by its reads and, at these sizes, by their number: a lane takes eight columns as two loads of 16 bytes.  2,048 rows of 2,560 / 4,096 / 5,120 /
 // 8,192, three slabs, us, in turn from three copies: step 25, 36, 52, 74, norm 13, 23, 31, 45; one slab 21, 24, 35, 55 and 9, 11, 16.5, 24.  With a
 // column a load, which is five times the requests: step 28, 43, 58, 84, norm 16, 26, 31.5, 49; 22, 28, 40, 59 and 11, 13, 15.5, 30.
-// Rows whose width is no multiple of 4, or that begin at no multiple of 16 bytes, are taken a column a load (up to ten columns a lane of 256).  The
+// Rows whose width is no multiple of 4, or that begin at no multiple of 16 bytes, are taken a column a load: up to ten columns a lane, wider rows more lanes
+// (2,048 rows of 2,561 / 4,097 / 5,118, one slab, us: step 20, 35, 42, norm 11.5, 15, 17; with 1,024 lanes for all of them 30, 35, 42 and 17, 19, 20).  The
 // mean is taken first and the variance from the deviations, both summed over the workgroup in an order that the
-// width alone fixes: a row's result does not depend on what else is in the launch.  All arithmetic is float32.
+// width and that alignment fix: a row's result does not depend on what else is in the launch.  All arithmetic is float32.
 #include "common.h"
 #include <math.h>
 
@@ -210,7 +211,7 @@ layer_norm_wide_kernel(const float* __restrict__ u, int parts, size_t part_strid
     lane.store(out + row * width, v);
 }
 
-// CROWDED: rows of more than 4,096 columns, 640 lanes and more: 64 registers, so that two and three workgroups share a compute unit, for which the
+// CROWDED: rows of more than 4,096 columns, 576 lanes and more: 64 registers, so that two and three workgroups share a compute unit, for which the
 // weights and the fourth slab are asked for when they are wanted.
 template <typename TO, bool CROWDED>
 __global__ void __launch_bounds__(1024, CROWDED ? 8 : 4)
@@ -259,11 +260,14 @@ static bool wide_rows(int width, const void* a, const void* b, const void* c, co
 
 static dim3 wide_lanes(int width) { return dim3((width / 8 + KIPP_WAVE - 1 + (width % 8 != 0)) / KIPP_WAVE * KIPP_WAVE); }
 
-// LAUNCH(lanes, columns a lane, slabs asked for behind the first): rows a column a load.
-#define KIPP_LN_BUILDS(LAUNCH)                             \
+// LAUNCH(lanes, columns a lane, slabs asked for behind the first): rows a column a load.  FIVE: which build rows of up to 5,120 take.
+#define KIPP_LN_BUILDS(LAUNCH, FIVE)                       \
     do {                                                   \
         if (width <= 256 * 10) LAUNCH(256, 10, 3);         \
-        else if (width <= 5120) LAUNCH(1024, 5, 2);        \
+        else if (width <= 512 * 6) LAUNCH(512, 6, 2);      \
+        else if (width <= 512 * 8) LAUNCH(512, 8, 2);      \
+        else if (width <= 5120) FIVE;                      \
+        else if (width <= 1024 * 6) LAUNCH(1024, 6, 2);    \
         else LAUNCH(1024, 8, 1);                           \
     } while (0)
 
@@ -286,11 +290,11 @@ extern "C" int kipp_layer_norm(const float* u, int parts, const float* w, const 
                        scale, (KIPP_LN_TO*)out, width)
     if (out_dtype == KIPP_F32) {
 #define KIPP_LN_TO float
-        KIPP_LN_BUILDS(KIPP_LN);
+        KIPP_LN_BUILDS(KIPP_LN, KIPP_LN(512, 10, 2));
 #undef KIPP_LN_TO
     } else if (out_dtype == KIPP_BF16) {
 #define KIPP_LN_TO bf16_t
-        KIPP_LN_BUILDS(KIPP_LN);
+        KIPP_LN_BUILDS(KIPP_LN, KIPP_LN(512, 10, 2));
 #undef KIPP_LN_TO
     } else {
         return -2;
@@ -324,11 +328,11 @@ extern "C" int kipp_sandwich_step(float* x, const float* delta, int parts, const
                        post_w, post_b, post_eps, mult, extra, next_w, next_b, next_eps, (KIPP_SS_TO*)out, width)
     if (out == nullptr || out_dtype == KIPP_F32) {
 #define KIPP_SS_TO float
-        KIPP_LN_BUILDS(KIPP_SS);
+        KIPP_LN_BUILDS(KIPP_SS, KIPP_SS(1024, 5, 2));
 #undef KIPP_SS_TO
     } else if (out_dtype == KIPP_BF16) {
 #define KIPP_SS_TO bf16_t
-        KIPP_LN_BUILDS(KIPP_SS);
+        KIPP_LN_BUILDS(KIPP_SS, KIPP_SS(1024, 5, 2));
 #undef KIPP_SS_TO
     } else {
         return -2;
