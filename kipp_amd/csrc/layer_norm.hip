@@ -211,8 +211,9 @@ layer_norm_wide_kernel(const float* __restrict__ u, int parts, size_t part_strid
     lane.store(out + row * width, v);
 }
 
-// CROWDED: rows of more than 4,096 columns, 576 lanes and more: 64 registers, so that two and three workgroups share a compute unit, for which the
-// weights and the fourth slab are asked for when they are wanted.
+// CROWDED: rows of more than 4,096 columns, 576 lanes and more, and of 2,564 to 3,584, six and seven waves, of which 94 registers leave room for two or
+// three workgroups: 64 registers, so that two and three, and four and five, share a compute unit, for which the weights and the fourth slab are asked
+// for when they are wanted (2,048 rows of 3,072, one and three slabs, us: 20.8, 28.5; with 94 registers 25.0, 32.0; a column a load 22.1, 30.5).
 template <typename TO, bool CROWDED>
 __global__ void __launch_bounds__(1024, CROWDED ? 8 : 4)
 sandwich_step_wide_kernel(float* __restrict__ x, const float* __restrict__ delta, int parts, size_t part_stride,
@@ -315,7 +316,7 @@ extern "C" int kipp_sandwich_step(float* x, const float* delta, int parts, const
     hipLaunchKernelGGL((sandwich_step_wide_kernel<TO, CROWDED>), dim3(rows), wide_lanes(width), 0, stream, x, delta, parts, part_stride, post_w, post_b, \
                        post_eps, mult, extra, next_w, next_b, next_eps, (TO*)out, width)
         if (out != nullptr && out_dtype != KIPP_F32 && out_dtype != KIPP_BF16) return -2;
-        const bool crowded = width > 4096, narrow = out != nullptr && out_dtype == KIPP_BF16;
+        const bool crowded = width > 4096 || (width > 2560 && width <= 3584), narrow = out != nullptr && out_dtype == KIPP_BF16;
         if (crowded && narrow) KIPP_SW(bf16_t, true);
         else if (crowded) KIPP_SW(float, true);
         else if (narrow) KIPP_SW(bf16_t, false);

@@ -39,7 +39,7 @@ def test_layer_norm_and_step(width, parts):
         assert float((out.double() - layer_norm64(x.double(), w2.double(), b2.double(), 1e-5)).abs().max()) <= bound
 
 
-@pytest.mark.parametrize("width", [4, 260, 2564, 4100, 8188])
+@pytest.mark.parametrize("width", [4, 260, 2564, 3584, 3588, 4100, 8188])
 def test_rows_at_multiples_of_16_bytes_and_elsewhere(width):
     """Widths of four columns a load: rows that begin elsewhere take a column a load, with the same result up to the order of the sums; a
     bfloat16 result is the float32 one rounded."""
