@@ -343,17 +343,18 @@ __global__ void __launch_bounds__(SCAN_THREADS) mlstm_step_kernel(
 
 #define FINISH_HEADS 4
 
-template <typename TO>
+// DIVIDED: the sums are still to be divided by `den` (two divisions a number, which cost a fifth of 2,048 tokens' time: not for those that are).
+template <typename TO, bool DIVIDED>
 __global__ void mlstm_finish_kernel(const float* __restrict__ o_raw, const float* __restrict__ den, const float* __restrict__ proj, int stride, int gate_at,
                                     const float* __restrict__ norm_w, float eps, TO* __restrict__ out, int heads, int dv) {
     const int wave = threadIdx.x / KIPP_WAVE, lane = threadIdx.x & (KIPP_WAVE - 1);
     const int t = blockIdx.y, head = blockIdx.x * FINISH_HEADS + wave;
     if (head >= heads) return;
     const float* src = o_raw + ((size_t)t * heads + head) * dv;
-    const float below = den != nullptr ? den[(size_t)t * heads + head] : 1.0f;
+    const float below = DIVIDED ? den[(size_t)t * heads + head] : 1.0f;
     float ss = 0.0f;
     for (int e = lane; e < dv; e += KIPP_WAVE) {
-        const float o = src[e] / below;
+        const float o = DIVIDED ? src[e] / below : src[e];
         ss = fmaf(o, o, ss);
     }
     ss = wave_sum(ss);
@@ -361,7 +362,7 @@ __global__ void mlstm_finish_kernel(const float* __restrict__ o_raw, const float
     const float* gate = proj + (size_t)t * stride + gate_at + head * dv;
     TO* dst = out + ((size_t)t * heads + head) * dv;
     for (int e = lane; e < dv; e += KIPP_WAVE)
-        store_f(dst, e, src[e] / below * scale * norm_w[head * dv + e] * (1.0f / (1.0f + expf(-gate[e]))));
+        store_f(dst, e, (DIVIDED ? src[e] / below : src[e]) * scale * norm_w[head * dv + e] * (1.0f / (1.0f + expf(-gate[e]))));
 }
 
 // Lanes that share a column of the memory in the walk over prompt portions: 8 rows a lane (16 for keys of 129 to 256 and
@@ -422,10 +423,16 @@ int kipp_mlstm_finish(const float* o_raw, const float* den, const float* proj, i
     if (n_tokens <= 0) return 0;
     if (heads <= 0 || dv <= 0 || stride < gate_at + heads * dv) return -1;
     dim3 grid((heads + FINISH_HEADS - 1) / FINISH_HEADS, n_tokens), block(FINISH_HEADS * KIPP_WAVE);
-    if (out_dtype == KIPP_BF16)
-        hipLaunchKernelGGL(mlstm_finish_kernel<bf16_t>, grid, block, 0, stream, o_raw, den, proj, stride, gate_at, norm_w, eps, (bf16_t*)out, heads, dv);
-    else
-        hipLaunchKernelGGL(mlstm_finish_kernel<float>, grid, block, 0, stream, o_raw, den, proj, stride, gate_at, norm_w, eps, (float*)out, heads, dv);
+#define KIPP_FINISH(TO, DIVIDED) \
+    hipLaunchKernelGGL((mlstm_finish_kernel<TO, DIVIDED>), grid, block, 0, stream, o_raw, den, proj, stride, gate_at, norm_w, eps, (TO*)out, heads, dv)
+    if (out_dtype == KIPP_BF16) {
+        if (den != nullptr) KIPP_FINISH(bf16_t, true);
+        else KIPP_FINISH(bf16_t, false);
+    } else {
+        if (den != nullptr) KIPP_FINISH(float, true);
+        else KIPP_FINISH(float, false);
+    }
+#undef KIPP_FINISH
     return KIPP_LAUNCH_CHECK();
 }
 

@@ -254,3 +254,24 @@ def test_mlstm_entries_beyond_the_portions_are_left_alone(d):
     for a, b in zip(some, alone):
         assert torch.equal(a, b)
     assert not torch.equal(some[0][3], kept[3]) and torch.equal(some[0][:3], kept[:3])
+
+
+@pytest.mark.parametrize("heads, dv", [(1, 1), (5, 63), (8, 320), (3, 65)])
+def test_mlstm_finish_with_and_without_a_division(heads, dv):
+    """Sums that are still to be divided give the bits of divided ones, and those the norm, weight and gate of float64."""
+    import torch
+    from kipp_amd.csrc import ops
+    gen = torch.Generator().manual_seed(dv)
+    n, at = 7, 3
+    o, proj, w = (torch.randn(shape, generator=gen).to(DEV) for shape in ((n, heads * dv), (n, at + heads * dv + 2), (heads * dv,)))
+    den = torch.empty((n, heads)).uniform_(0.1, 20.0, generator=gen).to(DEV)
+    o[0] = 0.0
+    divided = (o.view(n, heads, dv) / den[:, :, None]).view(n, heads * dv)
+    for dtype in (torch.float32, torch.bfloat16):
+        out = [ops.mlstm_finish(sums, proj, at, w, 1e-6, torch.empty((n, heads * dv), dtype=dtype, device=DEV), heads, dv, den=d)
+               for sums, d in ((o, den), (divided, None))]
+        assert torch.equal(*out), dtype
+        x = divided.double().view(n, heads, dv)
+        ref = (x / (x.square().mean(-1, keepdim=True) + 1e-6).sqrt()).view(n, heads * dv) * w.double() * torch.sigmoid(proj.double()[:, at:at + heads * dv])
+        # ten numbers a lane and six exchanges of the square's sum, a root, two quotients, an exponential and four products
+        assert torch.all((out[0].double() - ref).abs() <= ref.abs() * (32 * 2.0 ** -24 if dtype == torch.float32 else 2.0 ** -8))
