@@ -44,7 +44,8 @@ __device__ __forceinline__ float log_sigmoid(float z) { return fminf(z, 0.0f) - 
 // workgroup.  BASE: the rows a lane has in the build for prompt portions of this key size; a build with more rows a lane
 // adds them in runs of BASE and the runs pairwise, which is the order in which the lanes of that build add theirs.  `unit`: columns that share one copy of n and m in the state (a workgroup's columns are a multiple of it).
 // LDS: chunk * (2 ROWS PARTS + columns + 4) + 4 floats; rows of k and q are padded with zeros to ROWS * PARTS numbers.
-template <int ROWS, int PARTS, int BASE>
+// SOME: only entries of fewer than `below` tokens (a build of its own: a look at the length ahead of the loads took 3 % of 64 single tokens' time).
+template <int ROWS, int PARTS, int BASE, bool SOME>
 __global__ void __launch_bounds__(SCAN_THREADS) mlstm_scan_kernel(
     const float* __restrict__ proj, int stride, const float* __restrict__ bias_i, const float* __restrict__ bias_f, float cap,
     float* __restrict__ state, size_t state_stride, const int32_t* __restrict__ q_start, const int32_t* __restrict__ q_len,
@@ -65,7 +66,7 @@ __global__ void __launch_bounds__(SCAN_THREADS) mlstm_scan_kernel(
     const bool live = col < dv;
     const int row0 = part * ROWS;
     const int first = q_start[seq], count = q_len[seq];
-    if (below > 0 && count >= below) return;        // uniform over the workgroup: another kernel's entry
+    if (SOME && count >= below) return;             // uniform over the workgroup: another kernel's entry
     float* slot = state + (size_t)slots[seq] * state_stride;
     float* S_g = slot + ((size_t)head * dv + (live ? col : 0)) * d;
     float* n_all = slot + (size_t)heads * d * dv;
@@ -373,8 +374,8 @@ extern "C" {
 
 // `few`: every entry brings few tokens (single decoded tokens): where the key size allows, a workgroup takes 64 columns
 // with 4 lanes each, a quarter of the workgroups, each reading longer runs of the state.  `few` 2: every entry brings one token (`mlstm_step_kernel`
-// where it takes the sizes; `below` is not for that).  `below`: entries of so many tokens and more
-// are left alone (0: none).
+// where it takes the sizes).  `below`: entries of so many tokens and more
+// are left alone (0: none; `few` is not for that).
 int kipp_mlstm_scan(const float* proj, int stride, const float* bias_i, const float* bias_f, float cap, float* state,
                     size_t state_stride, const int32_t* q_start, const int32_t* q_len, const int32_t* slots, float* o_raw,
                     int n_seqs, int heads, int d, int dv, int few, int below, hipStream_t stream) {
@@ -386,6 +387,7 @@ int kipp_mlstm_scan(const float* proj, int stride, const float* bias_i, const fl
     const int base_parts = kipp_mlstm_parts(d);
     const int base_rows = d <= 128 ? 8 : (d <= 256 ? 16 : (d <= 512 ? 8 : 16));
     int parts = base_parts, rows = base_rows;
+    if (below > 0) few = 0;         // the builds for few tokens take every entry
     if (few == 2 && d > 32 && d <= 128 && d % STEP_ROWS == 0 && stride % 4 == 0 && state_stride % 4 == 0 && (((uintptr_t)proj | (uintptr_t)state) & 15) == 0) {
         const int waves = SCAN_THREADS / KIPP_WAVE, pairs = (2 * copies + waves - 1) / waves;
         if ((long long)n_seqs * heads * pairs <= 256)
@@ -403,16 +405,22 @@ int kipp_mlstm_scan(const float* proj, int stride, const float* bias_i, const fl
     int chunk = SCAN_STAGE / (rows * parts);          // tokens whose k and q fit the staging registers
     if (chunk > 32) chunk = 32;
     const size_t lds = ((size_t)chunk * (2 * rows * parts + cols + 4) + 4) * sizeof(float);
-#define KIPP_SCAN(R, P, B)                                                                                                          \
-    hipLaunchKernelGGL((mlstm_scan_kernel<R, P, B>), grid, block, lds, stream, proj, stride, bias_i, bias_f, cap, state, state_stride, \
+#define KIPP_SCAN(R, P, B, SOME)                                                                                                          \
+    hipLaunchKernelGGL((mlstm_scan_kernel<R, P, B, SOME>), grid, block, lds, stream, proj, stride, bias_i, bias_f, cap, state, state_stride, \
                        q_start, q_len, slots, o_raw, heads, d, dv, chunk, unit, copies, below)
-    if (parts == 4 && rows == 8) KIPP_SCAN(8, 4, 8);
-    else if (parts == 4) KIPP_SCAN(32, 4, 8);
-    else if (parts == 8) KIPP_SCAN(32, 8, 16);
-    else if (parts == 16 && rows == 8) KIPP_SCAN(8, 16, 8);
-    else if (parts == 16) KIPP_SCAN(16, 16, 16);
-    else if (rows == 8) KIPP_SCAN(8, 64, 8);
-    else KIPP_SCAN(16, 64, 16);
+#define KIPP_SCAN_OF(R, P, B)                    \
+    do {                                         \
+        if (below > 0) KIPP_SCAN(R, P, B, true); \
+        else KIPP_SCAN(R, P, B, false);          \
+    } while (0)
+    if (parts == 4 && rows == 8) KIPP_SCAN_OF(8, 4, 8);
+    else if (parts == 4) KIPP_SCAN(32, 4, 8, false);
+    else if (parts == 8) KIPP_SCAN(32, 8, 16, false);
+    else if (parts == 16 && rows == 8) KIPP_SCAN_OF(8, 16, 8);
+    else if (parts == 16) KIPP_SCAN_OF(16, 16, 16);
+    else if (rows == 8) KIPP_SCAN_OF(8, 64, 8);
+    else KIPP_SCAN_OF(16, 64, 16);
+#undef KIPP_SCAN_OF
 #undef KIPP_SCAN
     return KIPP_LAUNCH_CHECK();
 }

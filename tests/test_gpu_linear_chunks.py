@@ -275,3 +275,27 @@ def test_mlstm_finish_with_and_without_a_division(heads, dv):
         ref = (x / (x.square().mean(-1, keepdim=True) + 1e-6).sqrt()).view(n, heads * dv) * w.double() * torch.sigmoid(proj.double()[:, at:at + heads * dv])
         # ten numbers a lane and six exchanges of the square's sum, a root, two quotients, an exponential and four products
         assert torch.all((out[0].double() - ref).abs() <= ref.abs() * (32 * 2.0 ** -24 if dtype == torch.float32 else 2.0 ** -8))
+
+
+@pytest.mark.parametrize("d, dv", [(20, 9), (128, 40), (200, 17), (300, 5), (600, 6)])
+@pytest.mark.parametrize("few", [False, True])
+def test_mlstm_walk_of_some_entries(d, dv, few):
+    """`below`: the short entries' bits are those of a walk over every entry, the others' rows and states stay."""
+    import torch
+    from kipp_amd.csrc import ops
+    gen = torch.Generator().manual_seed(d)
+    heads, lens = 2, [3, 10, 0, 9, 40]
+    proj = torch.randn((sum(lens), 2 * heads * (d + dv) + 2 * heads), generator=gen).to(DEV)
+    bias, kept = torch.randn((2, heads), generator=gen).to(DEV), torch.randn((len(lens), ops.mlstm_state_size(heads, d, dv)), generator=gen).to(DEV)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)  # noqa: E731
+    got = []
+    for below in (0, 10):
+        state, o = kept.clone(), torch.full((sum(lens), heads * dv), 7.0, device=DEV)
+        ops.mlstm_scan(proj, bias[0], bias[1], 15.0, state, i32([0, 3, 13, 13, 22]), i32(lens), i32([0, 1, 2, 3, 4]), o, heads, d, dv, few=few and below > 0, below=below)
+        got.append((o, state))
+    (o, state), (o_some, state_some) = got
+    for e, (at, n) in enumerate(zip((0, 3, 13, 13, 22), lens)):
+        if n < 10:
+            assert torch.equal(o_some[at:at + n], o[at:at + n]) and torch.equal(state_some[e], state[e]), e
+        else:
+            assert bool((o_some[at:at + n] == 7.0).all()) and torch.equal(state_some[e], kept[e]), e
