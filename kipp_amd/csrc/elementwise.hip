@@ -884,8 +884,8 @@ int kipp_scale_values(float* x, float s, size_t n, hipStream_t stream) {
 // Up to MAX_TERMS terms: float32 delta[i] of x's rows, or parts[i] slabs of them, scale[i], and bias[i] (or null).
 int kipp_residual_add_terms(float* x, int count, const float* const* delta, const int* parts, const float* scale, const float* const* bias, int rows,
                             int width, hipStream_t stream) {
-    if (rows <= 0 || count == 0) return 0;
-    if (width <= 0 || count < 0 || count > MAX_TERMS) return -1;
+    if (rows <= 0 || width == 0 || count == 0) return 0;
+    if (width < 0 || count < 0 || count > MAX_TERMS) return -1;
     Terms terms = {};
     uintptr_t at = (uintptr_t)x;
     for (int i = 0; i < count; ++i) {

@@ -205,7 +205,7 @@ def residual_add(x: torch.Tensor, delta: torch.Tensor) -> torch.Tensor:
 
 def residual_add_scaled(x: torch.Tensor, delta: torch.Tensor, scale: float = 1.0, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """x += scale * (delta + bias): `delta` float32 of x's shape or slabs of it (added in order), `bias` float32 [width] or none."""
-    return residual_add_terms(x, [(delta, scale, bias)])
+    return _residual_add(x, [(delta, scale, bias)], "residual_add_scaled")
 
 
 RESIDUAL_TERMS = 4      # a launch
@@ -213,11 +213,15 @@ RESIDUAL_TERMS = 4      # a launch
 
 def residual_add_terms(x: torch.Tensor, terms) -> torch.Tensor:
     """`residual_add_scaled` for every (delta, scale, bias) of `terms` in turn, up to `RESIDUAL_TERMS` of them a launch: the same bits."""
+    return _residual_add(x, terms, "residual_add_terms")
+
+
+def _residual_add(x, terms, what):
     for delta, _, bias in terms:
         _dev(x, delta, bias)
         _need(x.dtype == delta.dtype == torch.float32 and x.dim() == 2 and tuple(delta.shape[-2:]) == tuple(x.shape) and delta.dim() in (2, 3),
-              "residual_add_scaled: float32 x [rows, width] and a float32 delta of its shape (or slabs of it)")
-        _need(bias is None or (bias.dtype == torch.float32 and bias.numel() == x.shape[1]), "residual_add_scaled: float32 bias [width]")
+              f"{what}: float32 x [rows, width] and a float32 delta of its shape (or slabs of it)")
+        _need(bias is None or (bias.dtype == torch.float32 and bias.numel() == x.shape[1]), f"{what}: float32 bias [width]")
     fn = _fn("elementwise", "kipp_residual_add_terms", [_c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_ptr])
     for i in range(0, len(terms), RESIDUAL_TERMS):
         some = terms[i:i + RESIDUAL_TERMS]
@@ -225,7 +229,7 @@ def residual_add_terms(x: torch.Tensor, terms) -> torch.Tensor:
         deltas, biases = ((ctypes.c_void_p * n)(*(_ptr(t[j]) for t in some)) for j in (0, 2))
         parts = (ctypes.c_int * n)(*(t[0].shape[0] if t[0].dim() == 3 else 1 for t in some))
         scales = (ctypes.c_float * n)(*(float(t[1]) for t in some))
-        _check(fn(_ptr(x), n, deltas, parts, scales, biases, x.shape[0], x.shape[1], _stream()), "residual_add_scaled")
+        _check(fn(_ptr(x), n, deltas, parts, scales, biases, x.shape[0], x.shape[1], _stream()), what)
     return x
 
 

@@ -84,6 +84,19 @@ def test_terms_of_a_weighted_sum_together(width):
     assert float((one.double() - ref).abs().max()) <= 24 * 2.0 ** -24 * 30      # 24 additions of numbers up to about 30
 
 
+def test_terms_without_rows_or_columns():
+    """Nothing to add to is no error, with slabs and biases and without."""
+    from kipp_amd.csrc import ops
+    for shape in ((5, 0), (0, 5), (0, 0)):
+        x, bias = torch.zeros(shape, device=DEV), torch.zeros(shape[1], device=DEV)
+        assert ops.residual_add_scaled(x, torch.zeros(shape, device=DEV)) is x
+        assert ops.residual_add_terms(x, [(torch.zeros((2, *shape), device=DEV), 0.5, bias), (torch.zeros(shape, device=DEV), 1.0, None)]) is x
+    with pytest.raises(Exception, match="residual_add_terms"):
+        ops.residual_add_terms(torch.zeros((2, 3), device=DEV), [(torch.zeros((3, 2), device=DEV), 1.0, None)])
+    with pytest.raises(Exception, match="residual_add_scaled"):
+        ops.residual_add_scaled(torch.zeros((2, 3), device=DEV), torch.zeros((3, 2), device=DEV))
+
+
 @pytest.mark.parametrize("span", [1, 16, 64, 65, 256, 257, 512, 513, 1024, 1025, 1536, 1537, 2560, 2561, 4096, 4097, 5120, 5121, 11000])
 @pytest.mark.parametrize("spans", [1, 3])
 def test_state_space_finish(span, spans):
