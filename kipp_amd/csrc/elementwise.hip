@@ -615,10 +615,12 @@ __global__ void scale_values_kernel(float* __restrict__ x, float s, size_t n) {
 }
 
 // x[r][c] += scale * (sum of the slabs of delta[r][c] + bias[c]), term after term of a weighted sum of deltas, each with the bias of
-// the product that made it (or none).  A lane takes four columns (one where rows do not begin at multiples of 16 bytes), and what all terms
-// bring is asked for before the first is added.  Bound by its launch for few rows, by its reads for many.  Three
+// the product that made it (or none).  A lane takes four columns of a row, and narrow rows share a workgroup; where rows do not begin at multiples of 16
+// bytes it takes one number, wherever rows end.  What all terms bring is asked for before the first is added.  Bound by its launch for few rows, by its
+// reads for many.  Three
 // terms, one launch / a launch a term and a column a lane, us in a recorded step: 16 rows of 2,560 3.5 / 6.5; 1,285 rows, one slab each 11.5 / 25.2, three
-// each 21.7 / 44.6; 2,048 rows of 5,120 45 / 89, 83 / 128.
+// each 21.7 / 44.6; 2,048 rows of 5,120 45 / 89, 83 / 128.  One term by itself, 333 rows of 2,561 3.5, 2,048 of 64 and of
+// 255 in three slabs 2.8, 3.0; with workgroups for every row's own lanes 4.6, 3.0, 4.0.
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 
 #define MAX_TERMS 4
@@ -633,17 +635,19 @@ struct Terms {
 };
 
 template <int N, typename V>
-__global__ void __launch_bounds__(TERM_LANES) residual_add_terms_kernel(float* __restrict__ x, const Terms terms, size_t part_stride, int width) {
-    const int c = (blockIdx.y * TERM_LANES + threadIdx.x) * (int)(sizeof(V) / sizeof(float));
-    if (c >= width) return;
-    const size_t at = (size_t)blockIdx.x * width + c;
+__global__ void __launch_bounds__(256) residual_add_terms_kernel(float* __restrict__ x, const Terms terms, size_t part_stride, int rows, int width) {
+    constexpr bool WIDE = sizeof(V) > sizeof(float);
+    const int row = blockIdx.x * blockDim.y + threadIdx.y, c = 4 * (blockIdx.y * blockDim.x + threadIdx.x);       // WIDE
+    if (WIDE && (row >= rows || c >= width)) return;
+    const size_t at = WIDE ? (size_t)row * width + c : (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (!WIDE && at >= part_stride) return;
     V v = *reinterpret_cast<const V*>(x + at), d[N][TERM_SLABS], b[N];
 #pragma unroll
     for (int i = 0; i < N; ++i) {
 #pragma unroll
         for (int p = 0; p < TERM_SLABS; ++p)
             if (p < terms.parts[i]) d[i][p] = *reinterpret_cast<const V*>(terms.delta[i] + p * part_stride + at);
-        if (terms.bias[i] != nullptr) b[i] = *reinterpret_cast<const V*>(terms.bias[i] + c);
+        if (terms.bias[i] != nullptr) b[i] = *reinterpret_cast<const V*>(terms.bias[i] + (WIDE ? c : at % width));
     }
 #pragma unroll
     for (int i = 0; i < N; ++i) {
@@ -653,11 +657,11 @@ __global__ void __launch_bounds__(TERM_LANES) residual_add_terms_kernel(float* _
             if (p < terms.parts[i]) sum += d[i][p];
         for (int p = TERM_SLABS; p < terms.parts[i]; ++p) sum += *reinterpret_cast<const V*>(terms.delta[i] + p * part_stride + at);
         if (terms.bias[i] != nullptr) sum += b[i];
-        if constexpr (sizeof(V) == sizeof(float)) {
-            v = fmaf(terms.scale[i], sum, v);
-        } else {
+        if constexpr (WIDE) {
 #pragma unroll
             for (int j = 0; j < 4; ++j) v[j] = fmaf(terms.scale[i], sum[j], v[j]);
+        } else {
+            v = fmaf(terms.scale[i], sum, v);
         }
     }
     *reinterpret_cast<V*>(x + at) = v;
@@ -897,12 +901,16 @@ int kipp_residual_add_terms(float* x, int count, const float* const* delta, cons
         at |= (uintptr_t)delta[i] | (uintptr_t)bias[i];
     }
     const bool wide = width % 4 == 0 && (at & 15) == 0;
-    const int lanes = wide ? width / 4 : width;
-    const dim3 grid(rows, (lanes + TERM_LANES - 1) / TERM_LANES), block(TERM_LANES);
-#define KIPP_TERMS(N)                                                                                                                   \
-    do {                                                                                                                                \
-        if (wide) hipLaunchKernelGGL((residual_add_terms_kernel<N, f32x4>), grid, block, 0, stream, x, terms, (size_t)rows * width, width);  \
-        else hipLaunchKernelGGL((residual_add_terms_kernel<N, float>), grid, block, 0, stream, x, terms, (size_t)rows * width, width);       \
+    const size_t n = (size_t)rows * width;
+    int lanes = TERM_LANES;         // of a row, wide
+    while (lanes > 4 && lanes >= width / 2) lanes /= 2;
+    const int together = TERM_LANES / lanes;
+    const dim3 grid = wide ? dim3((rows + together - 1) / together, (width + 4 * lanes - 1) / (4 * lanes)) : dim3((unsigned)((n + 255) / 256));
+    const dim3 block = wide ? dim3(lanes, together) : dim3(256);
+#define KIPP_TERMS(N)                                                                                                            \
+    do {                                                                                                                         \
+        if (wide) hipLaunchKernelGGL((residual_add_terms_kernel<N, f32x4>), grid, block, 0, stream, x, terms, n, rows, width);   \
+        else hipLaunchKernelGGL((residual_add_terms_kernel<N, float>), grid, block, 0, stream, x, terms, n, rows, width);        \
     } while (0)
     switch (count) {
         case 1: KIPP_TERMS(1); break;

@@ -84,6 +84,18 @@ def test_terms_of_a_weighted_sum_together(width):
     assert float((one.double() - ref).abs().max()) <= 24 * 2.0 ** -24 * 30      # 24 additions of numbers up to about 30
 
 
+@pytest.mark.parametrize("rows", [1, 33, 70])
+@pytest.mark.parametrize("width", [3, 4, 8, 12, 16, 100, 255, 256, 260])
+def test_terms_of_narrow_rows(rows, width):
+    """Rows that share a workgroup, more and fewer than it holds, and numbers taken wherever rows end."""
+    from kipp_amd.csrc import ops
+    rng = np.random.default_rng(rows * width)
+    x, one, slabs, bias = f32(rng, rows, width), f32(rng, rows, width), f32(rng, 3, rows, width), f32(rng, width)
+    ref = x.double() + 0.7 * (one.double() + bias.double()) - 0.4 * slabs.double().sum(0)
+    got = ops.residual_add_terms(x.clone(), [(one, 0.7, bias), (slabs, -0.4, None)])
+    assert float((got.double() - ref).abs().max()) <= 6 * 2.0 ** -24 * 16       # six additions of numbers up to about 16
+
+
 def test_terms_without_rows_or_columns():
     """Nothing to add to is no error, with slabs and biases and without."""
     from kipp_amd.csrc import ops
