@@ -170,9 +170,11 @@ class SandwichNormMixerBlock(SandwichNormBlock):
 class ParallelBlock:
     """One norm whose output both sublayers read: h = mixer_norm(x); x += mixer(h) + ffn(h).  The mixer's result is added
     at once, where it lies; the feed-forward's is handed on and added inside the next block's norm.  Where both are weighted
-    sums of deltas, which no norm adds in its own kernel, their terms are handed on together and added in one launch."""
+    sums of deltas, which no norm adds in its own kernel, and the rows are few, their terms are handed on together and added
+    in one launch, in the same order."""
 
     roles = (("mixer_norm", "norm"), ("mixer", "mixer"), ("ffn", "feed_forward"))
+    TOGETHER = 1 << 20      # most numbers of x: with more, a launch costs less than x again, and the mixer's slabs would lie beside the feed-forward's work
 
     def __init__(self, layer_spec, runtime):
         self.rt = runtime
@@ -187,13 +189,18 @@ class ParallelBlock:
         h = norm.forward(x, rt.act_dtype) if pending is None else norm.add_forward(x, pending, rt.act_dtype)
         h = rt.rows_of(h)       # two readers: the rows are finished once
         delta = self.mixer.forward(h, batch, cache, state)
-        more = self.parts["ffn"].forward(h, batch) if "ffn" in self.parts else None
-        if isinstance(delta, WeightedDelta) and isinstance(more, WeightedDelta):
-            return x, delta.plus(more)
+        more = None
+        if isinstance(delta, WeightedDelta) and x.numel() <= self.TOGETHER and "ffn" in self.parts:
+            more = self.parts["ffn"].forward(h, batch)
+            if isinstance(more, WeightedDelta):
+                return x, delta.plus(more)
         if hasattr(delta, "add_to"):
             delta.add_to(x)
         else:
             rt.ops.residual_add(x, rt.settle(delta))
+        del delta               # its slabs are free for the feed-forward
+        if more is None and "ffn" in self.parts:
+            more = self.parts["ffn"].forward(h, batch)
         return x, more
 
 

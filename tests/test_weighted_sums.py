@@ -1,4 +1,5 @@
 """In which order a weighted sum of deltas is added to the residual stream: term after term, whoever adds it."""
+import weakref
 from types import SimpleNamespace
 
 import pytest
@@ -64,3 +65,30 @@ def test_mixer_and_feed_forward_keep_their_order(norm):
     x, pending = block.forward(start.clone(), None, None, None, None)
     block.parts["mixer_norm"].add_forward(x, pending, torch.float32)
     assert torch.equal(x, _in_turn(start, mixed, fed))
+
+
+@pytest.mark.parametrize("fed_is_a_sum", [True, False])
+@pytest.mark.parametrize("rows_are_few", [True, False])
+def test_many_rows_are_added_ahead_of_the_feed_forward(rows_are_few, fed_is_a_sum):
+    """With more numbers than `TOGETHER` the mixer's result is in x, and nobody holds it, when the feed-forward runs; the sum is the same."""
+    rt = PlainRuntime()
+    block = ParallelBlock.__new__(ParallelBlock)
+    mixed, fed = _terms(rt, 2), _terms(rt, 3)
+    start = torch.full((2, 4), 0.7)
+    held = weakref.ref(mixed.terms[0][0])
+    want = _in_turn(_in_turn(start, mixed), fed) if fed_is_a_sum else _in_turn(start, mixed) + 0.3
+    seen = []
+
+    def feed(h, batch):
+        seen.append((held() is None, x.clone()))
+        return fed if fed_is_a_sum else torch.full((2, 4), 0.3)
+    box = [mixed]
+    block.rt, block.mixer, block.TOGETHER = rt, SimpleNamespace(forward=lambda h, batch, cache, state: box.pop()), 8 if rows_are_few else 7
+    block.parts = {"mixer_norm": RMSNorm(SimpleNamespace(eps=1e-5), rt), "ffn": SimpleNamespace(forward=feed)}
+    added = _in_turn(start, mixed)
+    del mixed
+    x = start.clone()
+    _, pending = block.forward(x, None, None, None, None)
+    assert len(seen) == 1 and seen[0][0] == (not rows_are_few) and torch.equal(seen[0][1], start if rows_are_few else added)
+    rt.add(x, pending)
+    assert torch.equal(x, want)
