@@ -461,6 +461,36 @@ def test_long_decoding_through_a_small_pool_and_one_slot(tmp_path, dtype):
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_mlstm_portions_by_chunks(tmp_path, monkeypatch, dtype):
+    """Keys of 64 and 128, which bfloat16 portions take by chunks: prompts alone (nothing is left to walk), a portion beside single tokens
+    and a short one (which walk), then single tokens, recorded, in their own kernel; a slot used again."""
+    from kipp_amd.csrc import ops
+    from kipp_amd.weights import write_random_model
+    cfg = _one_layer("mlstm", {"heads": 2, "dim": 64, "vdim": 48, "gate_cap": 8.0})
+    cfg["layers"].append({"type": "mlstm", "mixer": {"heads": 1, "dim": 128, "vdim": 70, "gate_cap": 5.0}, "mlp": None})
+    folder = write_random_model(str(tmp_path / "keys"), cfg, seed=9, dtype=dtype)
+    tokens = {"a": H.random_tokens(1, 165, 90), "b": H.random_tokens(2, 115, 90), "c": H.random_tokens(3, 160, 90), "d": H.random_tokens(4, 80, 90)}
+    steps = [([("a", 130), ("b", 70)], []), ([("a", 1), ("c", 100), ("b", 1), ("d", 9)], []), ([("a", 1), ("b", 15), ("d", 70)], [])]
+    steps += [([("a", 1), ("b", 1), ("c", 1), ("d", 1)], ["d"])] + [([("a", 1), ("b", 1), ("c", 1)], []) for _ in range(28)]
+    steps += [([("a", 4)], ["a"]), ([("c", 31)], ["c"])]
+    taken, chunks = [], ops.mlstm_chunks
+
+    def watched(*args, **kw):
+        out = chunks(*args, **kw)
+        taken.append((kw["longest"], out[1], out[0] is not None))
+        return out
+    monkeypatch.setattr(ops, "mlstm_chunks", watched)
+    got = H.replay(engine_of(folder, dtype, max_tokens=None, num_pages=64, max_requests=4), tokens, steps)
+    for rid in tokens:
+        close(got[rid], plain_logits(folder, tokens[rid])[:len(got[rid])], TOL[dtype], f"{dtype}/{rid}")
+    if dtype == "float32":
+        assert not taken
+        return
+    assert taken[:6] == 2 * [(130, -1, True)] + 2 * [(100, ops.CHUNKS_FROM, True)] + 2 * [(70, ops.CHUNKS_FROM, True)]
+    assert all(not by_chunks and below == 0 for longest, below, by_chunks in taken[6:])
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 def test_other_sizes_and_branches(tmp_path, dtype):
     """Widths that are no multiple of 8 or of 32, a latent too wide and heads too many for the matrix-core attention, a mLSTM
     key wider than 256, one stream, four streams, no logit scale, attention without a query factor, a layer that reads
