@@ -18,8 +18,10 @@
 // halves.  Measured with the shader clock around the walk: 37.5 cycles a
 // product where the matrix core needs 32; 33.5 with the DMA taken out: a wave that issues
 // a DMA instruction cannot issue its next product in time, which a second wave on the SIMD hides.  In the
-// run of a prefill the chip is at its power limit, and the time of a product is set by that, not by the
-// cycles: the cuts differ by a few per cent, and which is fastest for a shape is found by the clock.
+// run of a prefill the clock comes down as well, to 1.3 to 1.8 GHz; how much of the distance to what the matrix cores
+// sustain by themselves (1.55 to 1.8 PFLOP/s on such operands) is the clock's and how much the walk's was not told apart, and the
+// library's 1.45 at 8,192 x 9,728 shows that it is not all the clock's.  The cuts differ by a few per cent, and which is
+// fastest for a shape is found by timing.
 //
 // An output element is summed over K in the same order whatever the tile and the number of waves: cuts
 // with the same parts of K give the same bits.
