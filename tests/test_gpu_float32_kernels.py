@@ -39,8 +39,8 @@ def test_product_rows_are_the_same_in_both_kernels(n, k):
 @pytest.mark.parametrize("m, n", [(17, 32), (33, 47), (49, 2579), (97, 2570), (350, 3001), (333, 2570), (200, 6155)])
 @pytest.mark.parametrize("k", [40, 268])
 def test_product_in_every_shape_of_tiles(m, n, k):
-    """Sizes that the rule gives to tiles of 32 x 32, 32 x 48, 64 x 32, 64 x 48 and 64 x 64, with parts of tiles at both ends and
-    of a step of K: every row as the kernel for up to 16 rows makes it, whose sums the test above holds to float64."""
+    """Sizes around the tiles of every kernel at a K of a step or two a run, with parts of tiles at both ends and of a step of K: every row
+    as the kernel for up to 16 rows makes it, whose sums the test above holds to float64.  (The test below names every shape of tiles.)"""
     import torch
     from kipp_amd.csrc import ops
     gen = torch.Generator().manual_seed(m + n + k)
