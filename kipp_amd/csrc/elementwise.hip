@@ -618,9 +618,9 @@ __global__ void scale_values_kernel(float* __restrict__ x, float s, size_t n) {
 // the product that made it (or none).  A lane takes four columns of a row, and narrow rows share a workgroup; where rows do not begin at multiples of 16
 // bytes it takes one number, wherever rows end.  What all terms bring is asked for before the first is added.  Bound by its launch for few rows, by its
 // reads for many.  Three
-// terms, one launch / a launch a term and a column a lane, us in a recorded step: 16 rows of 2,560 3.5 / 6.5; 1,285 rows, one slab each 11.5 / 25.2, three
-// each 21.7 / 44.6; 2,048 rows of 5,120 45 / 89, 83 / 128.  One term by itself, 333 rows of 2,561 3.5, 2,048 of 64 and of
-// 255 in three slabs 2.8, 3.0; with workgroups for every row's own lanes 4.6, 3.0, 4.0.
+// terms, one launch / a launch a term and a column a lane, us in a recorded step: 8 rows of 2,560 3.2 / 6.7; 1,285 rows, one slab each 11.8 / 24.2, three
+// each 22.0 / 40.5.  One term by itself: 333 rows of 2,561 3.4 (with lanes in rows of their own 4.6), 2,048 of 255 in three slabs 3.0 (4.0), 33 of 1,000
+// in five 3.4 (3.8 with every slab's request behind a condition).
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 
 #define MAX_TERMS 4
@@ -634,29 +634,37 @@ struct Terms {
     int parts[MAX_TERMS];
 };
 
-template <int N, typename V>
+// SLABS: the most slabs a term has, or TERM_SLABS where one has more; BIAS: a term has one.  Nothing is asked for behind a condition (the compiler waits
+// for a request ahead of the next one then): a term of fewer slabs has its last, and one without a bias x, asked for once more, and not added.
+template <int N, int SLABS, bool BIAS, typename V>
 __global__ void __launch_bounds__(256) residual_add_terms_kernel(float* __restrict__ x, const Terms terms, size_t part_stride, int rows, int width) {
     constexpr bool WIDE = sizeof(V) > sizeof(float);
     const int row = blockIdx.x * blockDim.y + threadIdx.y, c = 4 * (blockIdx.y * blockDim.x + threadIdx.x);       // WIDE
     if (WIDE && (row >= rows || c >= width)) return;
     const size_t at = WIDE ? (size_t)row * width + c : (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (!WIDE && at >= part_stride) return;
-    V v = *reinterpret_cast<const V*>(x + at), d[N][TERM_SLABS], b[N];
+    const size_t at_bias = !BIAS ? 0 : (WIDE ? c : at % width);
+    V v = *reinterpret_cast<const V*>(x + at), d[N][SLABS], b[N];
 #pragma unroll
     for (int i = 0; i < N; ++i) {
 #pragma unroll
-        for (int p = 0; p < TERM_SLABS; ++p)
-            if (p < terms.parts[i]) d[i][p] = *reinterpret_cast<const V*>(terms.delta[i] + p * part_stride + at);
-        if (terms.bias[i] != nullptr) b[i] = *reinterpret_cast<const V*>(terms.bias[i] + (WIDE ? c : at % width));
+        for (int p = 0; p < SLABS; ++p) d[i][p] = *reinterpret_cast<const V*>(terms.delta[i] + (p == 0 ? 0 : min(p, terms.parts[i] - 1) * part_stride) + at);
+        if (BIAS) b[i] = *reinterpret_cast<const V*>(terms.bias[i] != nullptr ? terms.bias[i] + at_bias : x + at);
     }
 #pragma unroll
     for (int i = 0; i < N; ++i) {
         V sum = d[i][0];
 #pragma unroll
-        for (int p = 1; p < TERM_SLABS; ++p)
-            if (p < terms.parts[i]) sum += d[i][p];
-        for (int p = TERM_SLABS; p < terms.parts[i]; ++p) sum += *reinterpret_cast<const V*>(terms.delta[i] + p * part_stride + at);
-        if (terms.bias[i] != nullptr) sum += b[i];
+        for (int p = 1; p < SLABS; ++p) {
+            const V more = sum + d[i][p];
+            sum = p < terms.parts[i] ? more : sum;
+        }
+        if (SLABS == TERM_SLABS)
+            for (int p = TERM_SLABS; p < terms.parts[i]; ++p) sum += *reinterpret_cast<const V*>(terms.delta[i] + p * part_stride + at);
+        if (BIAS) {
+            const V more = sum + b[i];
+            sum = terms.bias[i] != nullptr ? more : sum;
+        }
         if constexpr (WIDE) {
 #pragma unroll
             for (int j = 0; j < 4; ++j) v[j] = fmaf(terms.scale[i], sum[j], v[j]);
@@ -665,6 +673,28 @@ __global__ void __launch_bounds__(256) residual_add_terms_kernel(float* __restri
         }
     }
     *reinterpret_cast<V*>(x + at) = v;
+}
+
+template <int N, int SLABS>
+static void launch_terms(float* x, const Terms& terms, bool biased, bool wide, int rows, int width, hipStream_t stream) {
+    const size_t n = (size_t)rows * width;
+    int lanes = TERM_LANES;         // of a row, wide
+    while (lanes > 4 && lanes >= width / 2) lanes /= 2;
+    const int together = TERM_LANES / lanes;
+    const dim3 grid = wide ? dim3((rows + together - 1) / together, (width + 4 * lanes - 1) / (4 * lanes)) : dim3((unsigned)((n + 255) / 256));
+    const dim3 block = wide ? dim3(lanes, together) : dim3(256);
+    if (wide && biased) hipLaunchKernelGGL((residual_add_terms_kernel<N, SLABS, true, f32x4>), grid, block, 0, stream, x, terms, n, rows, width);
+    else if (wide) hipLaunchKernelGGL((residual_add_terms_kernel<N, SLABS, false, f32x4>), grid, block, 0, stream, x, terms, n, rows, width);
+    else if (biased) hipLaunchKernelGGL((residual_add_terms_kernel<N, SLABS, true, float>), grid, block, 0, stream, x, terms, n, rows, width);
+    else hipLaunchKernelGGL((residual_add_terms_kernel<N, SLABS, false, float>), grid, block, 0, stream, x, terms, n, rows, width);
+}
+
+template <int N>
+static void launch_terms_of(float* x, const Terms& terms, int slabs, bool biased, bool wide, int rows, int width, hipStream_t stream) {
+    if (slabs == 1) launch_terms<N, 1>(x, terms, biased, wide, rows, width, stream);
+    else if (slabs == 2) launch_terms<N, 2>(x, terms, biased, wide, rows, width, stream);
+    else if (slabs == 3) launch_terms<N, 3>(x, terms, biased, wide, rows, width, stream);
+    else launch_terms<N, TERM_SLABS>(x, terms, biased, wide, rows, width, stream);
 }
 
 // out[r][c] = scale[c] * (sum of the slabs of delta[r][c]), or x[r][c] += that where `add`.
@@ -892,8 +922,12 @@ int kipp_residual_add_terms(float* x, int count, const float* const* delta, cons
     if (width < 0 || count < 0 || count > MAX_TERMS) return -1;
     Terms terms = {};
     uintptr_t at = (uintptr_t)x;
+    int slabs = 1;
+    bool biased = false;
     for (int i = 0; i < count; ++i) {
         if (parts[i] <= 0) return -1;
+        slabs = max(slabs, parts[i]);
+        biased = biased || bias[i] != nullptr;
         terms.delta[i] = delta[i];
         terms.parts[i] = parts[i];
         terms.scale[i] = scale[i];
@@ -901,24 +935,12 @@ int kipp_residual_add_terms(float* x, int count, const float* const* delta, cons
         at |= (uintptr_t)delta[i] | (uintptr_t)bias[i];
     }
     const bool wide = width % 4 == 0 && (at & 15) == 0;
-    const size_t n = (size_t)rows * width;
-    int lanes = TERM_LANES;         // of a row, wide
-    while (lanes > 4 && lanes >= width / 2) lanes /= 2;
-    const int together = TERM_LANES / lanes;
-    const dim3 grid = wide ? dim3((rows + together - 1) / together, (width + 4 * lanes - 1) / (4 * lanes)) : dim3((unsigned)((n + 255) / 256));
-    const dim3 block = wide ? dim3(lanes, together) : dim3(256);
-#define KIPP_TERMS(N)                                                                                                            \
-    do {                                                                                                                         \
-        if (wide) hipLaunchKernelGGL((residual_add_terms_kernel<N, f32x4>), grid, block, 0, stream, x, terms, n, rows, width);   \
-        else hipLaunchKernelGGL((residual_add_terms_kernel<N, float>), grid, block, 0, stream, x, terms, n, rows, width);        \
-    } while (0)
     switch (count) {
-        case 1: KIPP_TERMS(1); break;
-        case 2: KIPP_TERMS(2); break;
-        case 3: KIPP_TERMS(3); break;
-        default: KIPP_TERMS(4); break;
+        case 1: launch_terms_of<1>(x, terms, slabs, biased, wide, rows, width, stream); break;
+        case 2: launch_terms_of<2>(x, terms, slabs, biased, wide, rows, width, stream); break;
+        case 3: launch_terms_of<3>(x, terms, slabs, biased, wide, rows, width, stream); break;
+        default: launch_terms_of<4>(x, terms, slabs, biased, wide, rows, width, stream); break;
     }
-#undef KIPP_TERMS
     return KIPP_LAUNCH_CHECK();
 }
 
