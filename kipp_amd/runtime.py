@@ -315,15 +315,15 @@ class Runtime:
         best = min(names, key=there.get)
         return best if choice not in there or there[best] < 0.95 * there[choice] else choice
 
-    # Cuts of our kernel that are timed beside the planned one: 100 x (wave tile rows / 32) + 10 x (wave tile
-    # columns / 32) + parts of K (+ 1000: workgroups of 8 waves, two a SIMD, on the same 256 x 256 tile; + 2000: those for
-    # the whole rounds of 256 tiles and smaller tiles for the columns that are left, + 30000: the smallest for those).  The
+    # Cuts of our kernel that are timed beside the planned one: 100 x (tile rows / 64) + 10 x (tile
+    # columns / 64) + parts of K (+ 2000: tiles of 256 x 256 for
+    # the whole rounds of 256 tiles and smaller tiles for the columns that are left, 128 x 256 or, + 10000, 256 x 128, + 30000, 128 x 128).  The
     # plan's cost model is linear; the GPU under its power limit is not (a round that leaves compute units idle
     # clocks the others higher), so the plan is not always the fastest.  An output element is summed over K in
     # the same order whatever the tile, so cuts with the same parts of K give the same bits.
     _choices_of_process: dict = {}      # what the engines of a process timed: (choice, rows, milliseconds of every way, the choice for other rows)
-    TILE_CUTS_SLABS = (441, 442, 444, 431, 432, 433, 421, 422, 423, 1421, 1422, 1423, 1424)
-    TILE_CUTS_BF16 = (441, 421, 241, 1421, 2421, 32421)
+    TILE_CUTS_SLABS = (441, 442, 443, 444, 431, 432, 433, 421, 422, 241, 242, 221, 222)
+    TILE_CUTS_BF16 = (441, 421, 241, 2421, 12421, 32421)
 
     def _fastest(self, key, ways: dict, same_bits, m: int, cols: int, pairs: bool = False, extra_ms=None):
         """Which of several ways to compute one product of `m` rows and `cols` output columns is taken for the shape `key`: timed once,

@@ -1077,6 +1077,25 @@ def test_gemm_tiles_cuts_with_the_same_parts_give_the_same_bits():
         assert torch.equal(ops.gemm_tiles(x, w, "swiglu", force=cut), gated), cut
 
 
+@pytest.mark.parametrize("k,parts", [(32, 1), (64, 1), (64, 2), (96, 1), (96, 3), (160, 2), (224, 4), (1056, 1), (1056, 3)])
+def test_gemm_tiles_walks_of_whole_and_half_steps(k, parts):
+    """K of whole and half steps of 64 columns, cut where a part begins and ends inside a line or is a half step alone, in every tile (12 DMA
+    instructions over eight waves where a half has 96 rows): exactly on small integers, the same bits in every tile on others; rows beyond
+    eight tiles' (bands of them)."""
+    ops = _ops()
+    rng = np.random.default_rng(k + parts)
+    m, n = 1100, 388
+    xi, wi = (torch.tensor(rng.integers(-3, 4, size=(a, k)), dtype=torch.bfloat16) for a in (m, n))
+    x, w = (torch.tensor(rng.normal(size=(a, k)), dtype=torch.bfloat16).to(DEV) for a in (m, n))
+    base = None
+    for tile in (44, 43, 42, 24, 23, 22):
+        got = ops.gemm_tiles(xi.to(DEV), wi.to(DEV), "slabs", max_parts=4, force=10 * tile + parts)
+        assert torch.equal(got.sum(dim=0).cpu(), xi.float() @ wi.float().T), tile
+        got = ops.gemm_tiles(x, w, "slabs", max_parts=4, force=10 * tile + parts)
+        base = got if base is None else base
+        assert torch.equal(got, base), tile
+
+
 def test_gemm_tiles_refuses_what_it_cannot_do():
     ops = _ops()
     x = torch.zeros(300, 40, dtype=torch.bfloat16, device=DEV)
