@@ -12,9 +12,10 @@
 //              row (place -1)
 //     expert   a tile's rows against its expert's matrix: out[row][n] = act(sum_k W_e[n][k] x[row][k]).  bfloat16 with K a
 //              multiple of 32: on the matrix cores, in three forms.  Few rows an expert (tiles of up to 64): a workgroup 16 columns,
-//              its eight waves every eighth 64 numbers of k each, whose sums are added in order.  Staged (tiles of up to 128): a workgroup
-//              128 columns, 64 numbers of k a step through registers and LDS, one chain of 16 x 16 x 32 products along k.  Walking (tiles of
-//              up to 128 or 256): the walk of the prompt products, 32 x 32 x 16 products along k.  Else (float32, other K): a
+//              its eight waves every eighth 64 numbers of k each, whose sums are added in order.  Walking (tiles of
+//              up to 64, 128 or 256): the walk of the prompt products, one chain of 16 x 16 x 32 products along k.  Staged (tiles of up to
+//              128, for rows and matrices that begin at no multiple of 16 bytes): a workgroup
+//              128 columns, 64 numbers of k a step through registers and LDS, the same chain.  Else (float32, other K): a
 //              lane takes a column of a tile of 16 rows, one chain along k.
 //              A form sums over k in one order for every row, whichever tile the row is in; the forms' orders differ, and the form
 //              follows from the pairs of the whole step and the matrices' sizes: under bfloat16 a token's last bits depend on how
@@ -24,7 +25,7 @@
 //              two fragments of 16 columns are the gate's and the up's of the same 16 inner columns
 //     combine  out[t] = sum_j weight[t][j] y[place of (t, j)], or weight[t][j] x[t] for an identity expert (+ the shared expert's
 //              result, slabs added in order, maybe times the sigmoid of a logit of its own)
-#include "tile_walk.h"
+#include "line_walk.h"
 #include <math.h>
 
 #define ROUTE_WAVES 4
@@ -40,16 +41,13 @@
 #define MFMA_PITCH 72       // bfloat16 numbers from a row to the next in LDS
 #define MFMA_THREADS 256
 #define MANY_ROWS 256       // rows of a tile of the walking one where an expert has many
-#define WALK_FROM 48        // rows an expert (all of them) beyond which the walking one is the faster
-#define TILE_ACROSS 4       // waves of its workgroup across the columns (one or two down)
-#ifndef TILE_STAGES
-#define TILE_STAGES 3       // steps of K that are in LDS or on their way there: two workgroups share a compute unit
-#endif
-#define MANY_STAGES 4       // one workgroup (two waves a SIMD) a compute unit
+#define TILE_ACROSS 4       // waves of its workgroup across the columns, two down
+#define TILE_COLS(GLU) (((GLU) ? 32 : 64) * TILE_ACROSS)     // output columns of its tile
 #define ROWS_TILE 64        // rows of a tile of the product for few rows
 #define ROWS_WAVES 8        // waves of its workgroup
 #define ROWS_SHORT_K 1024   // K up to which a workgroup of it has two steps a wave at most, and is the slower one
 #define ROWS_SHORT_GROUPS 2048      // in a launch of more workgroups than this
+#define DIE_UNITS 32        // compute units of a die
 #define XCDS 8              // dies of the chip; consecutive workgroups of a launch go to them in turn
 
 enum { ACT_NONE = -1, ACT_SILU = 0, ACT_RELU = 1, ACT_GELU = 2, ACT_GELU_TANH = 3, ACT_RELU2 = 4 };
@@ -525,59 +523,67 @@ moe_expert_mfma_kernel(const bf16_t* __restrict__ x, const int32_t* __restrict__
         }
 }
 
-// The same for experts of many rows, tiles of up to 128 DOWN rows.  A workgroup takes a tile's rows
-// and 256 rows of the expert's matrix (GLU: 128 of the gate's and the 128 of the up's that belong to them), DOWN x 4 waves, each
-// 1 / DOWN of the rows against 64 of them, as many products of 32 rows as its part has.  The walk over K is the one of the products for
-// prompt portions (`tile_walk.h`), its rows of X taken through `gather`.  Bound by what a compute unit draws (a matrix of an
-// expert meets its 100 to 300 rows only) and by whole rounds of workgroups.  32 experts, matrices of 2,432 x 2,560 and back,
-// us: staged kernel / this one with 128 rows: 8,192 rows 251 / 212 and 230 / 201, gated 417 / 363; 5,120 rows 198 / 165, 172 / 152,
-// 329 / 300; 2,048 rows 137 / 128, 125 / 119, 197 / 195; 1,024 rows 116 / 119, 105 / 108, 175 / 185: its lines of 64
-// bytes of a row are the slower way to read a matrix once, so the staged kernel keeps experts of up to 48 rows.
-// 256 rows: 8,192 rows 193, 170, gated 320; 5,120 rows 171, 153, 243; with four waves of all 256 rows, one a SIMD, instead of
-// eight: 237, 195, 365; 196, 157, 264 (whatever holds up a SIMD's one wave idles its matrix core).
-template <typename TO, bool GLU, int DOWN, int STAGES, int WM>
+// The same by the walk of the products for prompt portions (`line_walk.h`), its rows of x taken through `gather`: eight waves take a tile's rows
+// (up to 64 XF) and 128 WF rows of the expert's matrix (GLU: 64 WF of the gate's and the 64 WF of the up's that belong to them), two waves down and four
+// across.  Bound by the experts' matrices, which arrive at 4.9 to 5.5 TB/s where an expert has up to 100 rows, and by whole rounds of
+// workgroups.  32 experts, [gate; up] of 2 x 2,432 x 2,560, one such matrix, and back, us: the staged kernel or a walk in steps of half
+// lines with tiles of 128 or 256, the best of them / now: 416 rows 161 / 145, 104 / 85, 94 / 77; 2,048 rows 195 / 159, 130 / 101, 119 / 89;
+// 4,000 rows 225 / 181, 149 / 123, 132 / 105; 8,192 rows 345 / 276, 203 / 172, 176 / 142; 128 experts of 768, 3,968 rows 201 / 182, 124 / 100, 127 / 115.
+template <typename TO, bool GLU, int XF, int WF>
 __device__ __forceinline__ void expert_tile(const bf16_t* __restrict__ x, const int32_t* __restrict__ gather, const float* __restrict__ row_weight,
                                             const bf16_t* __restrict__ w_e, TO* __restrict__ out, int row0, int rows, int col0, int n_out, int k,
                                             int act, unsigned char* lds) {
-    constexpr int WAVES = TILE_ACROSS * DOWN, WN = 2;
-    constexpr int TM = 64 * DOWN * ((WM + 1) / 2), TN = 32 * WN * TILE_ACROSS;     // rows of the pieces of a step (of X: whole instructions a wave)
-    constexpr int X_PIECE = TM * BK * 2, W_PIECE = TN * BK * 2, STAGE_BYTES = X_PIECE + W_PIECE;
-    constexpr int XI = TM / INSTR_ROWS / WAVES, WI = TN / INSTR_ROWS / WAVES;
+    using Walk = LineWalk<XF, WF, 2, TILE_ACROSS>;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int l32 = lane & 31, hh = lane >> 5, across = wave % TILE_ACROSS, first = 32 * WM * (wave / TILE_ACROSS);     // this wave's columns and rows
-    int lane_row, col8;
-    dma_place(lane, lane_row, col8);
+    const int l16 = lane & 15, quarter = lane >> 4, across = wave % TILE_ACROSS, first = 32 * XF * (wave / TILE_ACROSS);     // this wave's columns and rows
     // a lane's rows begin at 32-bit offsets from x and from the expert's matrix (the launcher has checked that they fit)
-    uint32_t x_src[XI], w_src[WI];
+    uint32_t x_src[2][Walk::X_MOST], w_src[2][Walk::W_MOST];
 #pragma unroll
-    for (int i = 0; i < XI; ++i) {
-        const int r = row0 + min((TM / WAVES) * wave + INSTR_ROWS * i + lane_row, rows - 1);     // rows beyond the tile's read its last one and are not stored
-        x_src[i] = (uint32_t)(((size_t)(gather != nullptr ? gather[r] : r) * k + col8) * 2);
-    }
+    for (int h = 0; h < 2; ++h) {
 #pragma unroll
-    for (int i = 0; i < WI; ++i) {
-        const int r = (TN / WAVES) * wave + INSTR_ROWS * i + lane_row;      // of the piece; 64 a wave multiplies: under GLU 32 of the gate's, then the up's
-        const int wr = GLU ? min(col0 + 32 * (r / 64) + (r & 31), n_out - 1) + (r & 32 ? n_out : 0) : min(col0 + r, n_out - 1);
-        w_src[i] = (uint32_t)(((size_t)wr * k + col8) * 2);
+        for (int n = 0; n < Walk::X_MOST; ++n) {
+            const int p = Walk::x_row(n, wave, lane), r = row0 + min(Walk::x_tile_row(h, p), rows - 1);     // rows beyond the tile's read its last one and are not stored
+            x_src[h][n] = (uint32_t)(((size_t)(gather != nullptr ? gather[r] : r) * k + line_col(lane, p, k / BK)) * 2);
+        }
+#pragma unroll
+        for (int n = 0; n < Walk::W_MOST; ++n) {
+            const int p = Walk::w_row(n, wave, lane);       // of the half; 16 WF of either half a wave multiplies: under GLU the gate's and the up's
+            const int wr = GLU ? min(col0 + p, n_out - 1) + h * n_out : min(col0 + Walk::w_tile_row(h, p), n_out - 1);
+            w_src[h][n] = (uint32_t)(((size_t)wr * k + line_col(lane, p, k / BK)) * 2);
+        }
     }
-    f32x16 acc[WM][WN];
-    tile_walk<WM, WN, XI, WI, STAGES, STAGE_BYTES>(lds, lane, (const unsigned char*)x, (const unsigned char*)w_e, x_src, w_src,
-                                                   wave * (X_PIECE / WAVES), X_PIECE + wave * (W_PIECE / WAVES), first * BK * 2,
-                                                   X_PIECE + across * (W_PIECE / TILE_ACROSS), k / BK, acc);
-    // In accumulator tile (i, j) a lane holds column l32 and rows 8 (v / 4) + 4 hh + v % 4.  32 rows at a time go through the wave's own
+    f32x4 acc[2 * XF][2 * WF];
+    line_walk<XF, WF, 2, TILE_ACROSS>(lds, lane, wave, (const unsigned char*)x, (const unsigned char*)w_e, x_src, w_src, k / BK, acc);
+    // Of fragment (i, j) a lane holds row l16 and columns 16 j + 4 quarter .. + 3.  Sums that are stored as they are go straight from there.
+    if constexpr (!GLU && sizeof(TO) == 4) {
+        if (act == ACT_NONE && (n_out & 7) == 0) {
+#pragma unroll
+            for (int i = 0; i < 2 * XF; ++i) {
+                const int r = first + 16 * i + l16;
+                if (r >= rows) continue;
+#pragma unroll
+                for (int j = 0; j < 2 * WF; ++j) {
+                    const int c = col0 + 32 * WF * across + 16 * j + 4 * quarter;
+                    if (c < n_out) *(f32x4*)(out + (size_t)(row0 + r) * n_out + c) = acc[i][j];
+                }
+            }
+            return;
+        }
+    }
+    // Others: 32 rows at a time go through the wave's own
     // corner of LDS (now free) as they are; a lane then takes 8 neighbouring columns of a row, activates and stores them (the
     // activations written out for every accumulator register were hundreds of KB of code that ran once).
-    constexpr int WCOLS = GLU ? 32 : 64, PITCH = 68, LANES_PER_ROW = WCOLS / 8, ROWS_PER_PASS = 64 / LANES_PER_ROW;
-    static_assert(32 * PITCH * 4 * WAVES <= STAGES * STAGE_BYTES, "a wave's staging fits its share of LDS");
+    constexpr int WCOLS = (GLU ? 16 : 32) * WF, PITCH = 32 * WF + 4, LANES_PER_ROW = WCOLS / 8, ROWS_PER_PASS = 64 / LANES_PER_ROW;
+    static_assert(32 * PITCH * 4 * Walk::WAVES <= Walk::LDS_BYTES, "a wave's staging fits its share of LDS");
     __syncthreads();                                               // every wave is done reading operands
     float* stage = (float*)lds + wave * 32 * PITCH;
     const int c_in = (lane % LANES_PER_ROW) * 8, c = col0 + WCOLS * across + c_in;
 #pragma unroll
-    for (int i = 0; i < WM; ++i) {
+    for (int i = 0; i < XF; ++i) {
 #pragma unroll
-        for (int v = 0; v < 16; ++v)
+        for (int f = 0; f < 2; ++f)
 #pragma unroll
-            for (int j = 0; j < WN; ++j) stage[(8 * (v / 4) + 4 * hh + (v % 4)) * PITCH + 32 * j + l32] = acc[i][j][v];
+            for (int j = 0; j < 2 * WF; ++j) *(f32x4*)(stage + (16 * f + l16) * PITCH + 16 * j + 4 * quarter) = acc[2 * i + f][j];
         __builtin_amdgcn_s_waitcnt(0xC07F);                        // lgkmcnt(0): what the wave wrote it reads back
         __builtin_amdgcn_wave_barrier();
 #pragma unroll 1
@@ -588,7 +594,7 @@ __device__ __forceinline__ void expert_tile(const bf16_t* __restrict__ x, const 
 #pragma unroll
             for (int q = 0; q < 8; q += 4) {
                 *(f32x4*)(y + q) = *(const f32x4*)(at + q);
-                if (GLU) *(f32x4*)(u + q) = *(const f32x4*)(at + 32 + q);
+                if (GLU) *(f32x4*)(u + q) = *(const f32x4*)(at + 16 * WF + q);
             }
             const float s = GLU && row_weight != nullptr ? row_weight[row0 + first + 32 * i + r] : 1.0f;
 #pragma unroll
@@ -614,33 +620,46 @@ __device__ __forceinline__ void expert_tile(const bf16_t* __restrict__ x, const 
     }
 }
 
-template <typename TO, bool GLU, int DOWN, int STAGES>
-__global__ void __launch_bounds__(64 * TILE_ACROSS * DOWN, 2)
+template <typename TO, bool GLU>
+__global__ void __launch_bounds__(512, 2)
 moe_expert_tiles_kernel(const bf16_t* __restrict__ x, const int32_t* __restrict__ gather, const float* __restrict__ row_weight,
                         const bf16_t* __restrict__ w, const int32_t* __restrict__ tiles, int max_tiles, int col_tiles, TO* __restrict__ out,
                         int n_out, int k, int act) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
-    // Used tiles come first in the list.  Workgroups id, id + 8, .. run on one die of the chip, each with an L2 of its own: a die
-    // takes a run of (tile, columns) pairs, columns fastest, so that its workgroups share rows of x and, from tile to tile of one
-    // expert, rows of w.
+    // Used tiles come first in the list, an expert's beside each other.  Workgroups id, id + 8, .. run on one die of the chip, each with an
+    // L2 of its own: a die takes a run of (expert, columns, tile), the expert's tiles fastest, so that workgroups which need the same rows of
+    // w walk over them at the same time.
+    const int lane = threadIdx.x & 63;
     int used = 0;
-    for (int at = 0; at < max_tiles; at += KIPP_WAVE) {
-        const int i = at + (threadIdx.x & 63);
-        used += __popcll(__ballot(i < max_tiles && tiles[(size_t)i * 3 + 2] > 0));
+    for (int at = 0; at < max_tiles; at += KIPP_WAVE) used += __popcll(__ballot(at + lane < max_tiles && tiles[(size_t)(at + lane) * 3 + 2] > 0));
+    const int items = used * col_tiles, per_die = (items + XCDS - 1) / XCDS, die = blockIdx.x % XCDS, turn = blockIdx.x / XCDS;
+    // What a die has beyond whole rounds of its compute units goes in halves of the columns where those take one round of half the time
+    // (7,204 rows of the experts above, 608 whole ones in three rounds / 512 and 192 halves: 238 and 223 us)
+    const int mine = min(per_die, items - die * per_die), whole = mine / DIE_UNITS * DIE_UNITS, rest = mine - whole;
+    const bool halved = turn >= whole && 2 * rest <= DIE_UNITS;
+    const int at_die = halved ? whole + (turn - whole) / 2 : turn, half = halved ? (turn - whole) & 1 : 0;
+    if (at_die >= mine) return;                         // uniform over the workgroup
+    const int item = die * per_die + at_die;
+    const int one = item / col_tiles, expert = __builtin_amdgcn_readfirstlane(tiles[(size_t)one * 3]);       // a tile of this item's expert
+    int before = 0, beside = 0;                         // the expert's tiles ahead of that one, and all of them
+    for (int at = 0; at < used; at += KIPP_WAVE) {
+        const unsigned long long same = __ballot(at + lane < used && tiles[(size_t)(at + lane) * 3] == expert);
+        beside += __popcll(same);
+        before += one - at >= KIPP_WAVE ? __popcll(same) : (one > at ? __popcll(same & ((1ull << (one - at)) - 1)) : 0);
     }
-    const int items = used * col_tiles, per_die = (items + XCDS - 1) / XCDS;
-    const int turn = blockIdx.x / XCDS, item = (blockIdx.x % XCDS) * per_die + turn;
-    if (turn >= per_die || item >= items) return;       // uniform over the workgroup
-    const int32_t* tile = tiles + (size_t)(item / col_tiles) * 3;
-    const int expert = __builtin_amdgcn_readfirstlane(tile[0]), row0 = __builtin_amdgcn_readfirstlane(tile[1]), rows = __builtin_amdgcn_readfirstlane(tile[2]);
-    const int col0 = (item % col_tiles) * (GLU ? 32 : 64) * TILE_ACROSS;
+    const int within = item - (one - before) * col_tiles;
+    const int32_t* tile = tiles + (size_t)(one - before + within % beside) * 3;
+    const int row0 = __builtin_amdgcn_readfirstlane(tile[1]), rows = __builtin_amdgcn_readfirstlane(tile[2]);
+    const int col0 = within / beside * TILE_COLS(GLU) + half * TILE_COLS(GLU) / 2;
+    if (col0 >= n_out) return;                          // the last columns may fill less than half a tile
     const bf16_t* w_e = w + (size_t)expert * (GLU ? 2 : 1) * n_out * k;
-    // a wave's products: as many of 32 rows as its part of the tile has
+    // a wave's fragments: as many as the tile's rows ask for
 #define KIPP_ET(N)                                                                                                                     \
     case N:                                                                                                                            \
-        expert_tile<TO, GLU, DOWN, STAGES, N>(x, gather, row_weight, w_e, out, row0, rows, col0, n_out, k, act, lds);           \
+        if (halved) expert_tile<TO, GLU, N, 1>(x, gather, row_weight, w_e, out, row0, rows, col0, n_out, k, act, lds);                  \
+        else expert_tile<TO, GLU, N, 2>(x, gather, row_weight, w_e, out, row0, rows, col0, n_out, k, act, lds);                          \
         break
-    switch ((rows + 32 * DOWN - 1) / (32 * DOWN)) {
+    switch ((rows + 63) / 64) {
         KIPP_ET(1);
         KIPP_ET(2);
         KIPP_ET(3);
@@ -894,20 +913,20 @@ extern "C" int kipp_moe_route_grouped(const float* z, int parts, int stride, con
     return KIPP_LAUNCH_CHECK();
 }
 
-template <typename TO, bool GLU, int DOWN, int STAGES>
+template <typename TO, bool GLU>
 static int launch_tiles(const void* x, const int32_t* gather, const float* row_weight, const void* w, const int32_t* tiles, int max_tiles,
                         void* out, int n_out, int k, int act, hipStream_t stream) {
-    constexpr int lds_bytes = STAGES * (128 * DOWN + 64 * TILE_ACROSS) * BK * 2;
+    constexpr int lds_bytes = LineWalk<MANY_ROWS / 64, 2, 2, TILE_ACROSS>::LDS_BYTES;
     static bool prepared = false;
     if (!prepared) {
-        if (hipFuncSetAttribute((const void*)moe_expert_tiles_kernel<TO, GLU, DOWN, STAGES>, hipFuncAttributeMaxDynamicSharedMemorySize,
+        if (hipFuncSetAttribute((const void*)moe_expert_tiles_kernel<TO, GLU>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 lds_bytes) != hipSuccess)
             return -6;
         prepared = true;
     }
-    const int cols = (GLU ? 32 : 64) * TILE_ACROSS, col_tiles = (n_out + cols - 1) / cols;
-    const int grid = (max_tiles * col_tiles + XCDS - 1) / XCDS * XCDS;
-    hipLaunchKernelGGL((moe_expert_tiles_kernel<TO, GLU, DOWN, STAGES>), dim3(grid), dim3(64 * TILE_ACROSS * DOWN), lds_bytes, stream, (const bf16_t*)x,
+    const int col_tiles = (n_out + TILE_COLS(GLU) - 1) / TILE_COLS(GLU);
+    const int grid = XCDS * ((max_tiles * col_tiles + XCDS - 1) / XCDS + DIE_UNITS / 2);        // halves: as many more
+    hipLaunchKernelGGL((moe_expert_tiles_kernel<TO, GLU>), dim3(grid), dim3(512), lds_bytes, stream, (const bf16_t*)x,
                        gather, row_weight, (const bf16_t*)w, tiles, max_tiles, col_tiles, (TO*)out, n_out, k, act);
     return KIPP_LAUNCH_CHECK();
 }
@@ -922,8 +941,8 @@ static int launch_expert(const void* x, int x_dtype, const int32_t* gather, cons
     // in the walk; rows of x that `gather` may name reach as far as x does
     const bool fits = (long long)max_tiles * tile_rows * k < (1ll << 31) && (long long)(GLU ? 2 : 1) * n_out * k < (1ll << 31) &&
                       (long long)x_rows * k < (1ll << 32);
-    // Tiles of few rows whose workgroups would have little of K each, and be many, are the staged kernel's: beside it the one for few rows
-    // takes, 256 experts of 1,024 x 512 and 10 pairs an expert, 1.25 and 1.5 of the time (gated, and back); 64 of 2,048 x 704, up 0.8, back 1.35.
+    // Tiles of few rows whose workgroups would have little of K each, and be many, are the walk's: beside the staged kernel, which the walk is as fast as here,
+    // the one for few rows takes, 256 experts of 1,024 x 512 and 10 pairs an expert, 1.25 and 1.5 of the time (gated, and back); 64 of 2,048 x 704, up 0.8, back 1.35.
     const long long hit = sorted_rows < experts ? sorted_rows : experts;
     const bool short_k = k <= ROWS_SHORT_K && hit * ((n_out + 15) / 16) > ROWS_SHORT_GROUPS;
     if (tile_rows == ROWS_TILE && !(short_k && fits)) {
@@ -943,7 +962,7 @@ static int launch_expert(const void* x, int x_dtype, const int32_t* gather, cons
         if (x_dtype != KIPP_BF16 || w_dtype != KIPP_BF16 || k % 32 || !fits) return -2;
         // the walk brings 16 bytes a lane
         const bool walks = (((uintptr_t)x | (uintptr_t)w) & 15) == 0 && (long long)x_rows * k < (1ll << 31);
-        if (tile_rows == ROWS_TILE || (tile_rows == MFMA_ROWS && (!walks || sorted_rows <= WALK_FROM * (long long)experts))) {
+        if (!walks && tile_rows != MANY_ROWS) {
             const int cols = GLU ? MFMA_COLS / 2 : MFMA_COLS;
             dim3 grid(max_tiles, (n_out + cols - 1) / cols), block(MFMA_THREADS);
             if (out_dtype == KIPP_BF16)
@@ -957,12 +976,8 @@ static int launch_expert(const void* x, int x_dtype, const int32_t* gather, cons
             return KIPP_LAUNCH_CHECK();
         }
         if (!walks) return -2;
-        if (out_dtype == KIPP_BF16)
-            return tile_rows == MFMA_ROWS ? launch_tiles<bf16_t, GLU, 1, TILE_STAGES>(x, gather, row_weight, w, tiles, max_tiles, out, n_out, k, act, stream)
-                                          : launch_tiles<bf16_t, GLU, 2, MANY_STAGES>(x, gather, row_weight, w, tiles, max_tiles, out, n_out, k, act, stream);
-        if (out_dtype == KIPP_F32)
-            return tile_rows == MFMA_ROWS ? launch_tiles<float, GLU, 1, TILE_STAGES>(x, gather, row_weight, w, tiles, max_tiles, out, n_out, k, act, stream)
-                                          : launch_tiles<float, GLU, 2, MANY_STAGES>(x, gather, row_weight, w, tiles, max_tiles, out, n_out, k, act, stream);
+        if (out_dtype == KIPP_BF16) return launch_tiles<bf16_t, GLU>(x, gather, row_weight, w, tiles, max_tiles, out, n_out, k, act, stream);
+        if (out_dtype == KIPP_F32) return launch_tiles<float, GLU>(x, gather, row_weight, w, tiles, max_tiles, out, n_out, k, act, stream);
         return -2;
     }
     if (tile_rows != TILE_ROWS) return -1;

@@ -1160,6 +1160,28 @@ def moe_tile_rows(dtype: torch.dtype, *contractions: int, pairs: Optional[int] =
     return MOE_MFMA_ROWS
 
 
+# Pairs an expert up to which a step stays with the kernel for few rows where the walk could take it: 32 experts of 2,560 x 2,432, both
+# products, few rows / walk, us: 3 an expert 141 / 153, gated 201 / 213; 5 an expert 162 / 159, 229 / 222; of 4,096 x 3,072 252 / 261, 378 / 388; 293 / 280, 433 / 427.
+# Gated experts of few numbers keep it as long as `moe_tile_rows` says (a walk's start counts there: 64 of 2,048 x 704, 5 an expert 97 / 118).
+MOE_STEP_FEW_PAIRS, MOE_STEP_FEW_NUMBERS = 4, 200_000_000
+
+
+def moe_step_tile_rows(dtype: torch.dtype, *contractions: int, pairs: int, experts: int = 1, gated: bool = False, aligned: bool = True,
+                       identity: int = 0) -> int:
+    """Rows of the tiles for the experts' products of a step: as `moe_tile_rows`, but the walk takes steps of fewer rows an expert, and always with
+    tiles of 256 where those are workgroups enough (an expert of 125 rows, both products without a gate, tiles of 128 / 256: 234 / 228 us; 225 rows 315 / 279,
+    gated 408 / 350)."""
+    rows = moe_tile_rows(dtype, *contractions, pairs=pairs, experts=experts, gated=gated, aligned=aligned, identity=identity)
+    if rows == MOE_TILE_ROWS or not aligned:
+        return rows
+    small = gated and 2 * experts * max(contractions) * min(contractions) <= MOE_STEP_FEW_NUMBERS
+    if rows == MOE_FEW_ROWS and (small or pairs * experts / (experts + identity) <= MOE_STEP_FEW_PAIRS * experts):
+        return rows
+    groups = (pairs / MOE_MANY_ROWS + experts / 2) * -(-contractions[-1] // (128 if gated else 256))
+    fits = (-(-pairs // MOE_MANY_ROWS) + experts) * MOE_MANY_ROWS * max(contractions) < 1 << 31 and 2 * max(contractions) * min(contractions) < 1 << 31
+    return MOE_MANY_ROWS if groups >= MOE_MANY_GROUPS and fits else MOE_MFMA_ROWS
+
+
 def moe_max_tiles(tokens: int, experts: int, top: int, tile_rows: int = 16) -> int:
     """Tiles of up to `tile_rows` rows that the sorted pairs of a step can need at most (every expert may end in a partial one)."""
     pairs = tokens * top

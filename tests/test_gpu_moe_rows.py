@@ -220,3 +220,37 @@ def test_feed_forward_of_rows_at_any_offset(tokens, gated):
     got, ref = part.forward(x), part.forward(x.clone())
     # the products in two orders of their sums, the inner rows rounded to bfloat16 in between
     assert float((got - ref).norm() / ref.norm()) < 4e-3
+
+
+@pytest.mark.parametrize("gated", [False, True])
+@pytest.mark.parametrize("k, n_out", [(32, 2040), (96, 1160), (160, 900)])
+def test_the_walk_over_many_tiles(gated, k, n_out):
+    """Experts of one to three tiles in every number of fragments, and of none, with more workgroups than compute units: whole rounds, and what is left
+    in halves of the columns (or not).  Small whole numbers, so that the sums are exact in any order."""
+    import torch
+    from kipp_amd.csrc import ops
+    rng = np.random.default_rng(k + n_out)
+    sizes = [0, 1, 63, 64, 65, 128, 129, 192, 193, 256, 257, 300, 520]
+    counts = [int(rng.choice(sizes)) for _ in range(33)]
+    starts = np.cumsum([0] + counts[:-1])
+    rows = int(np.sum(counts))
+    x = torch.tensor(rng.integers(-3, 4, size=(rows, k)), dtype=torch.bfloat16, device=DEV)
+    w = torch.tensor(rng.integers(-2, 3, size=(33, (2 if gated else 1) * n_out, k)), dtype=torch.bfloat16, device=DEV)
+    weight = torch.tensor(rng.integers(1, 3, size=rows), dtype=torch.float32, device=DEV)
+    tiles = []
+    for e, (at, n) in enumerate(zip(starts, counts)):
+        parts = -(-n // 256)
+        each = -(-(-(-n // parts)) // 64) * 64 if parts else 0
+        tiles += [(e, at + j * each, min(each, n - j * each)) for j in range(parts)]
+    td = torch.tensor(np.array(tiles + [(0, 0, 0)] * 70, dtype=np.int32), device=DEV)
+    out = torch.full((rows, n_out), float("nan"), device=DEV)
+    if gated:
+        ops.moe_expert_gated(x, None, weight, w, td, out, "relu", tile_rows=256)
+    else:
+        ops.moe_expert(x, None, w, td, out, tile_rows=256)
+    for e, (at, n) in enumerate(zip(starts, counts)):
+        p = x[at:at + n].float() @ w[e].float().T
+        if gated:
+            s = weight[at:at + n, None]
+            p = torch.relu(s * p[:, :n_out]) * (s * p[:, n_out:])
+        assert torch.equal(out[at:at + n], p), (e, n)

@@ -28,3 +28,15 @@ def test_many_rows_an_expert():
     assert [rows(8, 1024, 1024, 8 * n, True) for n in (100, 282, 1024)] == [128, 128, 256]
     assert ops.moe_tile_rows(torch.bfloat16, 2560, 2432, pairs=1, experts=32, aligned=False) == 128
     assert ops.moe_tile_rows(torch.bfloat16, 2560, 2432, pairs=32 * 500, experts=32, aligned=False) == 128
+
+
+def test_rows_of_a_step():
+    """The kernel for few rows up to four pairs an expert, or as long as it may where a gated step has few numbers; then the walk, in tiles of 256
+    where those are workgroups enough; what begins at no multiple of 16 bytes, and float32, as ever."""
+    rows = lambda experts, width, inner, pairs, gated, **k: ops.moe_step_tile_rows(k.pop("dtype", torch.bfloat16), width, inner, pairs=pairs, experts=experts, gated=gated, **k)  # noqa: E731
+    assert [rows(32, 2560, 2432, n, g) for g in (False, True) for n in (128, 129)] == [64, 256, 64, 256]
+    assert [rows(32, 2560, 2432, n, False, identity=8) for n in (160, 161)] == [64, 256]
+    assert [rows(64, 2048, 704, 64 * 6 + n, g) for g in (False, True) for n in (0, 1)] == [128, 128, 64, 256]
+    assert [rows(8, 1024, 1024, n, False) for n in (30, 200, 8 * 512, 8 * 900)] == [64, 128, 128, 256]
+    assert [rows(32, 2560, 2432, n, True, aligned=False) for n in (1, 500, 9000)] == [128, 128, 128]
+    assert rows(32, 2560, 2432, 9000, True, dtype=torch.float32) == 16
