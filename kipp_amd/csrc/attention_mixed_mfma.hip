@@ -69,12 +69,6 @@ typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
 
-// float32 -> bfloat16 by the hardware's conversion (round to nearest even, as f32_to_bf16 does for finite values)
-__device__ __forceinline__ bf16_t to_bf16(float f) {
-    const __bf16 b = (__bf16)f;
-    return __builtin_bit_cast(bf16_t, b);
-}
-
 union Frag {
     u32x4 u;
     bf16x8 v;
@@ -415,9 +409,9 @@ __global__ void __launch_bounds__(MX_THREADS) mixed_values_kernel(
                     } else {
 #pragma unroll
                         for (int hh = 0; hh < HPW; ++hh) {
-                            const bf16_t hi = to_bf16(p[hh][v]);
+                            const bf16_t hi = f32_to_bf16(p[hh][v]);
                             p_hi[at + hh] = hi;
-                            p_lo[at + hh] = to_bf16(p[hh][v] - bf16_to_f32(hi));
+                            p_lo[at + hh] = f32_to_bf16(p[hh][v] - bf16_to_f32(hi));
                         }
                     }
                 }
@@ -744,15 +738,15 @@ __global__ void __launch_bounds__(MX_THREADS) mixed_single_values_kernel(SingleG
                 for (int j = 0; j < 8; ++j) {
                     // (heads that do not exist were never written)
                     const float p = 8 * quarter + j < n_q && sc[j] != -INFINITY ? __expf(sc[j] - of_head[j].x) * of_head[j].y : 0.0f;
-                    hi.h[j] = to_bf16(p);
-                    lo.h[j] = to_bf16(p - bf16_to_f32(hi.h[j]));
+                    hi.h[j] = f32_to_bf16(p);
+                    lo.h[j] = f32_to_bf16(p - bf16_to_f32(hi.h[j]));
                 }
                 f32x4 d = {0.0f, 0.0f, 0.0f, 0.0f};
                 d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lo.v, mf.v, d, 0, 0, 0);
                 d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hi.v, mf.v, d, 0, 0, 0);
                 uint2 w;                                    // d[v]: key 16 kb + 4 quarter + v, head 16 nb + l16
-                w.x = (uint32_t)to_bf16(d[0]) | ((uint32_t)to_bf16(d[1]) << 16);
-                w.y = (uint32_t)to_bf16(d[2]) | ((uint32_t)to_bf16(d[3]) << 16);
+                w.x = (uint32_t)f32_to_bf16(d[0]) | ((uint32_t)f32_to_bf16(d[1]) << 16);
+                w.y = (uint32_t)f32_to_bf16(d[2]) | ((uint32_t)f32_to_bf16(d[3]) << 16);
                 *(uint2*)(pm + (16 * nb + l16) * SG_PITCH + 16 * kb + 4 * quarter) = w;
             }
             __syncthreads();

@@ -1397,3 +1397,18 @@ def test_window_edge(kernel):
             want = v[table[0, far // page], g, far % page, :].float().numpy()
             close = np.abs(got[4 * g] - want).max() < 0.02
             assert close == seen, f"{kernel}: key at distance {offset} (window {window}) seen={close}, expected {seen}"
+
+
+@pytest.mark.parametrize("sign", [0, 1 << 31])
+def test_rounding_to_bfloat16(sign):
+    """Every upper half of a float with lower halves around the tie, of the smallest, the largest and what overflows: the bits of the nearest bfloat16,
+    the even one of two; NaN stays NaN."""
+    ops = _ops()
+    low = torch.tensor([0, 1, 0x7fff, 0x8000, 0x8001, 0xffff], dtype=torch.int64)
+    bits = (torch.arange(0, 1 << 15, dtype=torch.int64)[:, None] * 65536 + low + sign).reshape(-1)
+    x = torch.where(bits >= 1 << 31, bits - (1 << 32), bits).to(torch.int32).view(torch.float32)
+    got = ops.cast(x.to(DEV), torch.empty(x.shape, dtype=torch.bfloat16, device=DEV)).cpu()
+    want = ((bits + 0x7fff + ((bits >> 16) & 1)) >> 16).to(torch.int32)
+    nan = torch.isnan(x)
+    assert torch.equal(got.view(torch.int16).to(torch.int32)[~nan] & 0xffff, want[~nan] & 0xffff)
+    assert bool(torch.isnan(got[nan]).all())
