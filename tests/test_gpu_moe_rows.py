@@ -254,3 +254,24 @@ def test_the_walk_over_many_tiles(gated, k, n_out):
             s = weight[at:at + n, None]
             p = torch.relu(s * p[:, :n_out]) * (s * p[:, n_out:])
         assert torch.equal(out[at:at + n], p), (e, n)
+
+
+@pytest.mark.parametrize("inner", [8, 7])
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("name", ["silu", "gelu", "gelu_tanh"])
+def test_activations_over_their_range(name, dtype, inner):
+    """Where exponentials vanish, overflow and cancel, infinities and NaN, four columns a thread and one: within the rounding of the result and of
+    float32 arithmetic (1 + erf and its like cancel below zero: an absolute error of some 2^-24 times z)."""
+    import torch
+    from kipp_amd.csrc import ops
+    x = torch.cat([torch.linspace(-20, 20, 4001), torch.logspace(-30, 38, 700), -torch.logspace(-30, 38, 700), torch.randn(2207)]).float()
+    x = x[:x.numel() // 56 * 56].reshape(-1, inner)
+    got = ops.activate(x.to(DEV), torch.empty(x.shape, dtype=getattr(torch, dtype), device=DEV), name).cpu().double()
+    z = x.double()
+    u = 0.79788456080286535588 * (z + 0.044715 * z * z * z)
+    ref = z * {"silu": torch.sigmoid(z), "gelu": torch.special.ndtr(z), "gelu_tanh": torch.sigmoid(2 * u)}[name]
+    bound = 2.0 ** -22 * ref.abs() + 2.0 ** -23 * z.abs().clamp(max=20) + (2.0 ** -8 * ref.abs() if dtype == "bfloat16" else 0) + 1e-37
+    assert bool(((got - ref).abs() <= bound).all())
+    ends = torch.tensor([[float("inf"), float("nan"), 0.0, -3e38] + [1.0] * (inner - 4)])
+    out = ops.activate(ends.to(DEV), torch.empty(ends.shape, dtype=getattr(torch, dtype), device=DEV), name).cpu()[0]
+    assert out[0] == float("inf") and torch.isnan(out[1]) and out[2] == 0 and out[3] == 0
