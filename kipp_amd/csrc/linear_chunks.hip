@@ -18,16 +18,16 @@
 //     gates    (mLSTM only) m, and what follows from it
 //     prepare  a workgroup (chunk, head, entry): A, T = (I + L)^-1 by forward substitution (a lane a column), G and
 //              D[last]; every chunk of the launch at once
-//     walk     a workgroup (16 columns of S, head, entry) takes its chunks in order.  S stays in registers as the
-//              instruction leaves it (a wave a quarter of its rows) and is shown to all waves through LDS; a wave takes 16 of the
-//              chunk's tokens for Q S, K S, T R and A U.  Q, K, T and A are operands straight from memory: a wave reads its own
-//              rows only, and the next chunk's are asked for as soon as this one's have been multiplied.
+//     walk     a workgroup (16 columns of S, head, entry) takes its chunks in order.  Four waves keep S in registers as the
+//              instruction leaves it (a wave a quarter of its rows), take it through the chunk (U first, for the delta rule) and show it
+//              through LDS for the next one; four others sum o for 16 of the chunk's tokens each, Q S and A U, meanwhile: what S waits for
+//              is a chain of 16 instructions a chunk (delta: 80), not of 80 (128).  One barrier a chunk (delta: three).  Q, K, T and A are operands
+//              straight from memory, the next chunk's asked for as soon as this one's have been multiplied.
 //
-// Bound by the walk's chain: at keys of 128 a chunk is 80 instructions of 32 cycles a wave (delta: 128), the sums in between
-// and two or three barriers, 3.8 us a chunk with 160 workgroups on 256 compute units.  2,048 tokens of 8 heads, keys of 128,
-// values of 320: 145 us (124 the walk) with a fixed decay, 193 (168) for the delta rule, where the walk token by token takes 772
-// and 663; 1,801 tokens of 40 heads with a state of 128 x 64: 120 (99), was 560.  An mLSTM of 8 heads of 128 x 320, all launches: one entry of 64,
-// 1,024, 2,048 tokens 22, 80, 137, eight of 150 70, where its walk takes 29, 378, 751, 186; of 256 x 512 39, 206, 376, 175 and 42, 591, 1,178, 722.
+// Bound by the walk's chain and the latency of its operands: 2,048 tokens of 8 heads, keys of 128, values of 320, all launches, us, with four
+// waves that do both / now: fixed decay 145 / 101, delta rule 185 / 154, an mLSTM 137 / 113; keys of 256, values of 512: 229 / 193, 293 / 250, 378 / 303;
+// 40 heads with a state of 128 x 64 127 / 98.  Token by token they take 772, 663 and 751, and 560.  More workgroups than the chip has places for are
+// the other way round (16 entries of 80 tokens, gated, 73 / 77): those keep the four waves.
 //
 // A position's bits depend on its place in the chunk, so this is for activations that are rounded to bfloat16 behind it; the walk
 // token by token keeps the float32 path, where a portion gives the bits of single tokens.
@@ -44,6 +44,7 @@
 #define THREADS 256
 #define UP 68               // floats from a column to the next of U and R in LDS
 #define COLS 16             // columns of S a workgroup of the walk
+#define EIGHT_GROUPS 1024   // workgroups of a walk up to which eight waves each are the faster way with keys of up to 128 (always with longer ones)
 
 #define VECS 4              // vectors of 64 numbers a chunk and head
 
@@ -316,19 +317,281 @@ __global__ void __launch_bounds__(THREADS) chunks_prepare_kernel(const ChunkArgs
     }
 }
 
-// What a wave multiplies in a chunk: its own rows of q, k, T and A, its rows of K^T, the values of its tokens.
+template <bool B>
+struct Bool {
+    static constexpr bool value = B;
+};
+
+// What a wave needs in a chunk to sum o for 16 of its tokens (q, a, g, f), or to keep 16 DT rows of S and, for the delta rule, make R and U of 16
+// tokens.  The delta rule's two share their places, which a wave uses in one way only.
 template <int MODE, int DT>
 struct Operands {
-    f32x4 q[4 * DT], k[MODE == MODE_DELTA ? 4 * DT : 1], a[4], t[MODE == MODE_DELTA ? 4 : 1], e[4], kt[DT][4], v, g, b, f;
+    static constexpr bool SHARED = MODE == MODE_DELTA;
+    f32x4 kt[4 * DT], k[SHARED ? 4 * DT : 1], t[SHARED ? 4 : 1], e[4], v, g, b, f;
+    f32x4 q_own[SHARED ? 1 : 4 * DT], a_own[SHARED ? 1 : 4];
+    float g_last;
+    __device__ __forceinline__ f32x4* q() { return SHARED ? kt : q_own; }
+    __device__ __forceinline__ f32x4* a() { return SHARED ? t : a_own; }
+};
+
+// Eight waves: four keep S, four sum o.
+template <int MODE, int DT>
+__global__ void __launch_bounds__(2 * THREADS, 2) chunks_walk_kernel(const ChunkArgs p) {
+    constexpr int D = 64 * DT, SP = D + 4;
+    __shared__ __attribute__((aligned(16))) float s_s[2][COLS * SP];        // [chunk's parity][column][row]
+    __shared__ __attribute__((aligned(16))) float u_s[2][COLS * UP];        // [chunk's parity][column][token]
+    __shared__ __attribute__((aligned(16))) float r_s[MODE == MODE_DELTA ? COLS * UP : 4];
+    const int head = blockIdx.y;
+    const Portion portion = portion_of(p.q_len, p.entries, p.from, blockIdx.z);
+    if (portion.entry < 0) return;          // uniform over the workgroup
+    const int entry = portion.entry;
+    const int lane = threadIdx.x & (KIPP_WAVE - 1), l16 = lane & 15, h4 = 4 * (lane >> 4);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / KIPP_WAVE) & 3;
+    const bool keeps = __builtin_amdgcn_readfirstlane(threadIdx.x / KIPP_WAVE) < 4;
+    const int n = p.q_len[entry], first = p.q_start[entry];
+    const int col = blockIdx.x * COLS + l16;
+    const bool norm = MODE == MODE_MLSTM && col == p.dv;        // n: one more column of S, of values of one
+    const bool live = col < p.dv || norm;
+    const int own = 16 * wave;              // the wave's tokens of a chunk
+    const int row0 = D / 4 * wave;          // its rows of S
+    float* S_col = p.state + (size_t)p.slots[entry] * p.state_stride + row0 + h4 +
+                   (norm ? p.n_at + (size_t)head * D : ((size_t)head * p.dv + (live ? col : 0)) * D);
+    const float* q = p.q + (size_t)(head / p.qk_rep) * D;
+    const float* k = p.k + (size_t)(head / p.qk_rep) * D;
+    const float* v_src = p.src + p.v_at + (size_t)head * p.dv + (live && !norm ? col : 0);
+    const int chunks = (n + CHUNK - 1) / CHUNK;
+
+    // A chunk's operands are asked for as soon as the one before has used its own; always all of them (rows beyond the last token are the last
+    // one's): behind a branch the compiler waits for everything that is on its way, so the last chunk, which asks for none, is code of its own.
+    Operands<MODE, DT> x;
+    f32x4 S[DT];
+    auto vec_of = [&](int c) { return p.vec + ((size_t)(portion.base + c) * p.heads + head) * VECS * CHUNK; };
+    auto own_rows = [&](int c, const float* from, f32x4* to) {          // of q or k
+        const int m = min(CHUNK, n - c * CHUNK);
+        const size_t row = (size_t)(first + c * CHUNK + min(own + l16, m - 1)) * p.qk_stride + h4;
+#pragma unroll
+        for (int j = 0; j < 4 * DT; ++j) to[j] = *reinterpret_cast<const f32x4*>(from + row + 16 * j);
+    };
+    auto square_of = [&](int c, const float* from, f32x4* to) {         // of A or T
+        const float* row = from + ((size_t)(portion.base + c) * p.heads + head) * CHUNK * CHUNK + (own + l16) * CHUNK + h4;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) to[j] = *reinterpret_cast<const f32x4*>(row + 16 * min(j, wave));       // (none above the diagonal)
+    };
+    auto gates_of = [&](int c) {
+        x.g = *reinterpret_cast<const f32x4*>(vec_of(c) + own + h4);
+        if (MODE == MODE_MLSTM) x.f = *reinterpret_cast<const f32x4*>(vec_of(c) + 3 * CHUNK + own + h4);
+    };
+    auto values_of = [&](int c) {
+        c = min(c, chunks - 1);
+        const int m = min(CHUNK, n - c * CHUNK), t0 = first + c * CHUNK;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x.v[i] = v_src[(size_t)(t0 + min(own + h4 + i, m - 1)) * p.stride];
+        if (MODE == MODE_DELTA) x.g = *reinterpret_cast<const f32x4*>(vec_of(c) + own + h4);
+        if (MODE == MODE_DELTA || MODE == MODE_MLSTM) x.b = *reinterpret_cast<const f32x4*>(vec_of(c) + 2 * CHUNK + own + h4);
+    };
+    auto keys_of = [&](int c) {
+        const int m = min(CHUNK, n - c * CHUNK), t0 = first + c * CHUNK;
+        const float* vec = vec_of(c);
+        x.g_last = vec[CHUNK - 1];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            x.e[j] = *reinterpret_cast<const f32x4*>(vec + CHUNK + 16 * j + h4);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float* k_row = k + (size_t)(t0 + min(16 * j + h4 + i, m - 1)) * p.qk_stride + row0 + l16;
+#pragma unroll
+                for (int a = 0; a < DT; ++a) x.kt[4 * a + j][i] = k_row[16 * a];
+            }
+        }
+    };
+    auto show_state = [&](int c) {
+#pragma unroll
+        for (int a = 0; a < DT; ++a) *reinterpret_cast<f32x4*>(&s_s[c & 1][l16 * SP + row0 + 16 * a + h4]) = S[a];
+    };
+    auto show_values = [&](int c) {         // U of the wave's tokens, where it does not hang on S
+        const int m = min(CHUNK, n - c * CHUNK);
+        f32x4 u = x.v;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            if (own + h4 + i >= m) u[i] = 0.0f;
+            if (MODE == MODE_DECAY) u[i] = silu_f(u[i]);        // silu(0) = 0
+            if (MODE == MODE_MLSTM) u[i] = x.b[i] * (norm ? 1.0f : u[i]);       // a gate of zero beyond the last token
+        }
+        *reinterpret_cast<f32x4*>(&u_s[c & 1][l16 * UP + own + h4]) = u;
+    };
+    auto values_shown = [&](int c, int m, f32x4 (&u)[4]) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (16 * j < m) u[j] = *reinterpret_cast<const f32x4*>(&u_s[c & 1][l16 * UP + 16 * j + h4]);
+    };
+    // the 16 columns of S against the wave's rows of q or k
+    auto with_state = [&](int c, const f32x4* rows) {
+        constexpr int RUNS = runs_of(MODE, DT);
+        f32x4 sum[RUNS][1];
+#pragma unroll
+        for (int h = 0; h < RUNS; ++h) sum[h][0] = zero4();
+#pragma unroll
+        for (int j = 0; j < 4 * DT; j += RUNS) {
+            f32x4 sv[RUNS];
+#pragma unroll
+            for (int h = 0; h < RUNS; ++h) sv[h] = *reinterpret_cast<const f32x4*>(&s_s[c & 1][l16 * SP + 16 * (j + h) + h4]);
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int h = 0; h < RUNS; ++h) sum[h][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(rows[j + h][i], sv[h][i], sum[h][0], 0, 0, 0);
+        }
+        return sum_runs(sum, 0);
+    };
+
+    f32x4 u_all[4];         // (the delta rule's, in one place for both kinds of waves: 14 registers fewer, and next to no spills at keys of 256)
+    // ---- S: through a chunk, and shown for the next one
+    auto begin_keeping = [&]() {
+#pragma unroll
+        for (int a = 0; a < DT; ++a) S[a] = live ? *reinterpret_cast<const f32x4*>(S_col + 16 * a) : zero4();
+        values_of(0);
+        if (MODE == MODE_DELTA) {
+            own_rows(0, k, x.k);
+            square_of(0, p.t, x.t);
+        }
+        keys_of(0);
+        show_state(0);
+        if (MODE != MODE_DELTA) {
+            show_values(0);
+            values_of(1);
+        }
+    };
+    auto keep = [&](int c, auto there_are_more) __attribute__((always_inline)) {
+        constexpr bool MORE = decltype(there_are_more)::value;
+        const int m = min(CHUNK, n - c * CHUNK);
+        if constexpr (MODE == MODE_DELTA) {
+            const bool mine = own < m;
+            if (mine) {
+                const f32x4 read = with_state(c, x.k);
+                f32x4 r;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) r[i] = own + h4 + i < m ? x.b[i] * (x.v[i] - x.g[i] * read[i]) : 0.0f;
+                *reinterpret_cast<f32x4*>(r_s + l16 * UP + own + h4) = r;
+            }
+            if (MORE) {
+                own_rows(c + 1, k, x.k);
+                values_of(c + 1);
+            }
+            __syncthreads();
+            if (mine) {
+                f32x4 w = zero4();
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    if (j <= wave) w = mul16(x.t[j], *reinterpret_cast<const f32x4*>(r_s + l16 * UP + 16 * j + h4), w);
+                *reinterpret_cast<f32x4*>(&u_s[c & 1][l16 * UP + own + h4]) = w;
+            }
+            if (MORE) square_of(c + 1, p.t, x.t);
+            __syncthreads();
+        }
+        f32x4 u_own[4];
+        f32x4 (&u)[4] = MODE == MODE_DELTA ? u_all : u_own;
+        values_shown(c, m, u);
+#pragma unroll
+        for (int a = 0; a < DT; ++a) S[a] *= x.g_last;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            if (16 * j >= m) continue;
+            const f32x4 eu = u[j] * x.e[j];
+#pragma unroll
+            for (int a = 0; a < DT; ++a) S[a] = mul16(x.kt[4 * a + j], eu, S[a]);
+        }
+        if (MORE) {
+            keys_of(c + 1);
+            show_state(c + 1);
+            if (MODE != MODE_DELTA) {
+                show_values(c + 1);
+                values_of(c + 2);
+            }
+        }
+    };
+    auto end_keeping = [&]() {
+        if (!live) return;
+        for (int c = 0; c < (norm ? p.copies : 1); ++c)         // every copy of n
+#pragma unroll
+            for (int a = 0; a < DT; ++a) *reinterpret_cast<f32x4*>(S_col + (size_t)c * p.heads * D + 16 * a) = S[a];
+    };
+    // ---- o of a chunk
+    auto begin_summing = [&]() {
+        own_rows(0, q, x.q());
+        gates_of(0);
+        square_of(0, p.a, x.a());
+    };
+    auto sum_up = [&](int c, auto there_are_more) __attribute__((always_inline)) {
+        constexpr bool MORE = decltype(there_are_more)::value;
+        const int m = min(CHUNK, n - c * CHUNK);
+        const bool mine = own < m;
+        f32x4 inter = zero4();
+        if (mine) inter = with_state(c, x.q());
+        if (MORE) own_rows(c + 1, q, x.q());
+        if (MODE == MODE_DELTA) {
+            __syncthreads();
+            __syncthreads();
+        }
+        f32x4 u_own[4];
+        f32x4 (&u)[4] = MODE == MODE_DELTA ? u_all : u_own;
+        values_shown(c, m, u);
+        if (mine) {
+            f32x4 o = MODE == MODE_MLSTM ? zero4() : inter * x.g;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (j <= wave) o = mul16(x.a()[j], u[j], o);
+            if (MODE == MODE_MLSTM) o += inter * (x.g * p.q_scale);
+            if (norm) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (own + h4 + i < m) p.den[(size_t)(first + c * CHUNK + own + h4 + i) * p.heads + head] = fmaxf(fabsf(o[i]), x.f[i]) + 1e-6f;
+            } else if (live) {
+                float* o_at = p.o_raw + (size_t)(first + c * CHUNK + own + h4) * p.heads * p.dv + (size_t)head * p.dv + col;
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (own + h4 + i < m) o_at[(size_t)i * p.heads * p.dv] = o[i];
+            }
+        }
+        if (MORE) {
+            gates_of(c + 1);
+            square_of(c + 1, p.a, x.a());
+        }
+    };
+
+    // All waves meet once a chunk (S ahead of it is shown, and U where that does not hang on S), and for the delta rule behind R and behind U.
+    if (keeps) {
+        begin_keeping();
+        for (int c = 0; c + 1 < chunks; ++c) {
+            __syncthreads();
+            keep(c, Bool<true>{});
+        }
+        __syncthreads();
+        keep(chunks - 1, Bool<false>{});
+        end_keeping();
+    } else {
+        begin_summing();
+        for (int c = 0; c + 1 < chunks; ++c) {
+            __syncthreads();
+            sum_up(c, Bool<true>{});
+        }
+        __syncthreads();
+        sum_up(chunks - 1, Bool<false>{});
+    }
+}
+
+// The walk of many short portions: four waves that do both, one behind the other.  Its workgroups are half as large, and more than fill the chip;
+// where they do not, a chunk's chain is what counts, and the eight waves are faster.
+// What one of four waves multiplies in a chunk: its own rows of q and A, its rows of K^T, the values of its tokens.
+template <int MODE, int DT>
+struct FourOperands {
+    f32x4 q[4 * DT], a[4], e[4], kt[DT][4], v, g, b, f;
     float g_last;
 };
 
 template <int MODE, int DT>
-__global__ void __launch_bounds__(THREADS) chunks_walk_kernel(const ChunkArgs p) {
+__global__ void __launch_bounds__(THREADS) chunks_walk_four_kernel(const ChunkArgs p) {
     constexpr int D = 64 * DT, SP = D + 4;
     __shared__ __attribute__((aligned(16))) float s_s[COLS * SP];           // [column][row]
     __shared__ __attribute__((aligned(16))) float u_s[COLS * UP];           // [column][token]
-    __shared__ __attribute__((aligned(16))) float r_s[MODE == MODE_DELTA ? COLS * UP : 4];
     const int head = blockIdx.y;
     const Portion portion = portion_of(p.q_len, p.entries, p.from, blockIdx.z);
     if (portion.entry < 0) return;          // uniform over the workgroup
@@ -352,7 +615,7 @@ __global__ void __launch_bounds__(THREADS) chunks_walk_kernel(const ChunkArgs p)
 
     // The next chunk's operands are asked for as soon as this one's have been used.  (A second set of registers, asked for
     // a whole chunk ahead, changed nothing and left a compute unit one workgroup instead of two.)
-    Operands<MODE, DT> x;
+    FourOperands<MODE, DT> x;
     auto rows_of = [&](int c) {
         const int m = min(CHUNK, n - c * CHUNK);
         if (own >= m) return;
@@ -360,7 +623,6 @@ __global__ void __launch_bounds__(THREADS) chunks_walk_kernel(const ChunkArgs p)
 #pragma unroll
         for (int j = 0; j < 4 * DT; ++j) {
             x.q[j] = *reinterpret_cast<const f32x4*>(q + row + 16 * j);
-            if (MODE == MODE_DELTA) x.k[j] = *reinterpret_cast<const f32x4*>(k + row + 16 * j);
         }
     };
     auto rest_of = [&](int c) {
@@ -369,18 +631,14 @@ __global__ void __launch_bounds__(THREADS) chunks_walk_kernel(const ChunkArgs p)
         const float* vec = p.vec + at * VECS * CHUNK;
         if (own < m) {
             const float* a_row = p.a + at * CHUNK * CHUNK + (own + l16) * CHUNK + h4;
-            const float* t_row = p.t + at * CHUNK * CHUNK + (own + l16) * CHUNK + h4;
 #pragma unroll
             for (int i = 0; i < 4; ++i) x.v[i] = own + h4 + i < m ? v_src[(size_t)(t0 + own + h4 + i) * p.stride] : 0.0f;
             x.g = *reinterpret_cast<const f32x4*>(vec + own + h4);
-            if (MODE == MODE_DELTA || MODE == MODE_MLSTM) x.b = *reinterpret_cast<const f32x4*>(vec + 2 * CHUNK + own + h4);
+            if (MODE == MODE_MLSTM) x.b = *reinterpret_cast<const f32x4*>(vec + 2 * CHUNK + own + h4);
             if (MODE == MODE_MLSTM) x.f = *reinterpret_cast<const f32x4*>(vec + 3 * CHUNK + own + h4);
 #pragma unroll
             for (int j = 0; j < 4; ++j)
-                if (j <= wave) {
-                    if (MODE == MODE_DELTA) x.t[j] = *reinterpret_cast<const f32x4*>(t_row + 16 * j);
-                    x.a[j] = *reinterpret_cast<const f32x4*>(a_row + 16 * j);
-                }
+                if (j <= wave) x.a[j] = *reinterpret_cast<const f32x4*>(a_row + 16 * j);
         }
         x.g_last = vec[CHUNK - 1];
 #pragma unroll
@@ -404,12 +662,12 @@ __global__ void __launch_bounds__(THREADS) chunks_walk_kernel(const ChunkArgs p)
 #pragma unroll
         for (int a = 0; a < DT; ++a) *reinterpret_cast<f32x4*>(&s_s[l16 * SP + row0 + 16 * a + h4]) = S[a];
         __syncthreads();
-        f32x4 inter = zero4(), read = zero4();
+        f32x4 inter = zero4();
         if (mine) {
             constexpr int RUNS = runs_of(MODE, DT);
-            f32x4 in[RUNS][1], rd[RUNS][1];
+            f32x4 in[RUNS][1];
 #pragma unroll
-            for (int h = 0; h < RUNS; ++h) in[h][0] = rd[h][0] = zero4();
+            for (int h = 0; h < RUNS; ++h) in[h][0] = zero4();
 #pragma unroll
             for (int j = 0; j < 4 * DT; j += RUNS) {
                 f32x4 sv[RUNS];
@@ -418,34 +676,19 @@ __global__ void __launch_bounds__(THREADS) chunks_walk_kernel(const ChunkArgs p)
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
 #pragma unroll
-                    for (int h = 0; h < RUNS; ++h) {
-                        in[h][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.q[j + h][i], sv[h][i], in[h][0], 0, 0, 0);
-                        if (MODE == MODE_DELTA) rd[h][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.k[j + h][i], sv[h][i], rd[h][0], 0, 0, 0);
-                    }
+                    for (int h = 0; h < RUNS; ++h) in[h][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.q[j + h][i], sv[h][i], in[h][0], 0, 0, 0);
             }
             inter = sum_runs(in, 0);
-            if (MODE == MODE_DELTA) read = sum_runs(rd, 0);
             f32x4 u = x.v;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 if (MODE == MODE_DECAY) u[i] = silu_f(u[i]);        // silu(0) = 0
                 if (MODE == MODE_MLSTM) u[i] = x.b[i] * (norm ? 1.0f : u[i]);       // a gate of zero beyond the last token
-                if (MODE == MODE_DELTA) u[i] = own + h4 + i < m ? x.b[i] * (x.v[i] - x.g[i] * read[i]) : 0.0f;
             }
-            *reinterpret_cast<f32x4*>((MODE == MODE_DELTA ? r_s : u_s) + l16 * UP + own + h4) = u;
+            *reinterpret_cast<f32x4*>(u_s + l16 * UP + own + h4) = u;
         }
         if (more) rows_of(c + 1);
         __syncthreads();
-        if (MODE == MODE_DELTA) {
-            if (mine) {
-                f32x4 u = zero4();
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    if (j <= wave) u = mul16(x.t[j], *reinterpret_cast<const f32x4*>(r_s + l16 * UP + 16 * j + h4), u);
-                *reinterpret_cast<f32x4*>(u_s + l16 * UP + own + h4) = u;
-            }
-            __syncthreads();
-        }
         f32x4 u[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j)
@@ -511,7 +754,13 @@ static void launch_chunks(const ChunkArgs& p, int longest, int portions, hipStre
     const int cols = p.dv + (MODE == MODE_MLSTM ? 1 : 0);
     const dim3 prepare((longest + CHUNK - 1) / CHUNK, p.heads, portions), walk((cols + COLS - 1) / COLS, p.heads, portions), block(THREADS);
     hipLaunchKernelGGL((chunks_prepare_kernel<MODE, DT>), prepare, block, 0, stream, p);
-    hipLaunchKernelGGL((chunks_walk_kernel<MODE, DT>), walk, block, 0, stream, p);
+    if constexpr (MODE != MODE_DELTA && DT <= 2) {
+        if ((long long)walk.x * walk.y * walk.z > EIGHT_GROUPS) {
+            hipLaunchKernelGGL((chunks_walk_four_kernel<MODE, DT>), walk, block, 0, stream, p);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((chunks_walk_kernel<MODE, DT>), walk, dim3(2 * THREADS), 0, stream, p);
 }
 
 template <int MODE>

@@ -299,3 +299,50 @@ def test_mlstm_walk_of_some_entries(d, dv, few):
             assert torch.equal(o_some[at:at + n], o[at:at + n]) and torch.equal(state_some[e], state[e]), e
         else:
             assert bool((o_some[at:at + n] == 7.0).all()) and torch.equal(state_some[e], kept[e]), e
+
+
+@pytest.mark.parametrize("mode, d", [("decay", 64), ("decay", 128), ("gated", 64), ("gated", 128), ("mlstm", 64), ("mlstm", 128)])
+def test_many_portions_have_the_bits_of_few(mode, d):
+    """More than 1,024 workgroups of a walk go by four waves that do both, fewer by eight: the same bits, of portions of one, two and three chunks, whole
+    and not."""
+    import torch
+    from kipp_amd.csrc import ops
+    heads, dv = 40, 64
+    lengths = [64, 65, 127, 128, 130, 150, 96, 192]
+    tokens, n = sum(lengths), len(lengths)
+    starts = np.concatenate([[0], np.cumsum(lengths)[:-1]])
+    gen = torch.Generator(device=DEV).manual_seed(d)
+    i32 = lambda x: torch.tensor(np.asarray(x), dtype=torch.int32, device=DEV)  # noqa: E731
+    if mode == "mlstm":
+        src = torch.randn(tokens, 2 * heads * d + 2 * heads * dv + 2 * heads, device=DEV, generator=gen)
+        bias, size = torch.randn(heads, device=DEV, generator=gen), ops.mlstm_state_size(heads, d, dv)
+    elif mode == "decay":
+        src = torch.randn(tokens, 2 * heads * d + heads * dv, device=DEV, generator=gen)
+        decays, size = torch.rand(heads, device=DEV, generator=gen), heads * d * dv
+    else:
+        src = torch.randn(tokens, ops.ssd_prep_width(heads, 1, d, dv), device=DEV, generator=gen)
+        src[:, 2 * d + 2 * heads * dv:].uniform_(0.5, 1.0, generator=gen)
+        size = heads * d * dv
+    begin = torch.randn(n, size, device=DEV, generator=gen)
+
+    def run(entries):
+        state, o = begin.clone(), torch.full((tokens, heads * dv), float("nan"), device=DEV)
+        where = (state, i32(starts[entries]), i32(np.asarray(lengths)[entries]), i32(entries), o)
+        longest, portions = max(lengths[e] for e in entries), len(entries)
+        if mode == "mlstm":
+            den, _ = ops.mlstm_chunks(src, bias, bias, 15.0, *where, heads, d, dv, longest=longest, portions=portions)
+            return state, o, den
+        if mode == "decay":
+            ops.decay_scan(src, decays, *where, heads, d, dv, longest=longest, chunks=True, portions=portions)
+        else:
+            ops.gated_scan(src, *where, heads, 1, d, dv, longest=longest, chunks=True, portions=portions)
+        return state, o, torch.zeros(tokens, heads, device=DEV)
+    real, ops.matrix_chunks_from = ops.matrix_chunks_from, lambda *a: 16
+    try:
+        together = run(list(range(n)))
+        for e in range(n):
+            alone = run([e])
+            rows = slice(starts[e], starts[e] + lengths[e])
+            assert torch.equal(together[0][e], alone[0][e]) and torch.equal(together[1][rows], alone[1][rows]) and torch.equal(together[2][rows], alone[2][rows]), e
+    finally:
+        ops.matrix_chunks_from = real
