@@ -208,17 +208,19 @@ __global__ void __launch_bounds__(512, (LineWalk<XF, WF, GM, GN>::LDS_BYTES <= 6
 // How a product is cut: the workgroup's tile (tm rows of X by tn rows of W) and the parts of K, for a range of output columns.
 // The cost of a cut is what its slowest compute unit does: rounds of tiles over the 256 units, each a fixed cost
 // (first data, the stores of the end) plus the steps of its part of K, and for every slab beyond the first what the kernel that adds them
-// reads once more.  Microseconds, fitted to the times of all cuts of seven products (4B and 8B shapes) at 256 to 1,800 rows: the plan is 0.4 %
-// over the fastest cut in the mean.
+// reads once more.  Microseconds, fitted to the times of all cuts of seven products (4B and 8B shapes) at 256 to 1,800 rows.
 struct Cut {
     int tm, tn, parts;
     int col_begin, col_end;     // output columns
 };
 
-#define N_SHAPES 5
-static const int kShapes[N_SHAPES][2] = {{256, 256}, {256, 192}, {256, 128}, {128, 256}, {128, 128}};
-static const double kStep[N_SHAPES] = {0.581, 0.510, 0.339, 0.315, 0.217};    // 32 columns of one tile
-static const double kFixed[N_SHAPES] = {12.9, 9.7, 7.5, 9.9, 4.6};            // start and end of a tile
+// Tiles 192 wide are there for the slabs alone (a gate's half would be 96).  128 x 192 fills the last round where 128 x 256 leaves 96
+// units idle: 2,048 x 2,560 x 2,560 34.0 -> 30.6 us (214 tiles for 160), 1,024 x 5,120 x 2,560 34.2 -> 30.6, 600 x 7,168 x 2,560
+// 33.5 -> 29.7.  129 sizes from 200 to 2,048 rows: the plan is 0.44 % over the fastest cut in the mean, without that tile 1.56.
+#define N_SHAPES 6
+static const int kShapes[N_SHAPES][2] = {{256, 256}, {256, 192}, {256, 128}, {128, 256}, {128, 192}, {128, 128}};
+static const double kStep[N_SHAPES] = {0.581, 0.510, 0.339, 0.315, 0.269, 0.217};    // 32 columns of one tile
+static const double kFixed[N_SHAPES] = {12.9, 9.7, 7.5, 9.9, 7.7, 4.6};              // start and end of a tile
 
 static double cut_cost(int M, int cols, int steps, int end, int shape, int parts) {
     const int tm = kShapes[shape][0], tn = pairs_columns(end) ? kShapes[shape][1] / 2 : kShapes[shape][1];
@@ -268,6 +270,7 @@ static int plan(int M, int N, int K, int end, int max_parts, Cut* cuts) {
         const int first_cols = (int)(whole / tiles_m) * tn;
         if (first_cols > 0 && first_cols < cols) {
             for (int s = 2; s < N_SHAPES; ++s) {
+                if (kShapes[s][1] == 192) continue;
                 const double cost = cut_cost(M, first_cols, steps, end, 0, 1) + cut_cost(M, cols - first_cols, steps, end, s, 1);
                 if (cost < best - 1e-9) {
                     best = cost;

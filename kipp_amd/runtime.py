@@ -322,7 +322,7 @@ class Runtime:
     # clocks the others higher), so the plan is not always the fastest.  An output element is summed over K in
     # the same order whatever the tile, so cuts with the same parts of K give the same bits.
     _choices_of_process: dict = {}      # what the engines of a process timed: (choice, rows, milliseconds of every way, the choice for other rows)
-    TILE_CUTS_SLABS = (441, 442, 443, 444, 431, 432, 433, 421, 422, 241, 242, 221, 222)
+    TILE_CUTS_SLABS = (441, 442, 443, 444, 431, 432, 433, 421, 422, 241, 242, 231, 232, 221, 222)
     TILE_CUTS_BF16 = (441, 421, 241, 2421, 12421, 32421)
 
     def _fastest(self, key, ways: dict, same_bits, m: int, cols: int, pairs: bool = False, extra_ms=None):

@@ -1096,6 +1096,19 @@ def test_gemm_tiles_walks_of_whole_and_half_steps(k, parts):
         assert torch.equal(got, base), tile
 
 
+@pytest.mark.parametrize("m,n", [(2048, 2560), (600, 7168), (1000, 2740)])
+def test_gemm_tiles_plans_where_tiles_of_192_columns_fit_best(m, n):
+    """Sizes at which the plan for slabs takes 128 x 192: the bits of other tiles; the other ends, which that width is not there for, plan
+    around it."""
+    ops = _ops()
+    rng = np.random.default_rng(m + n)
+    x = torch.tensor(rng.normal(size=(m, 160)), dtype=torch.bfloat16).to(DEV)
+    w = torch.tensor(rng.normal(size=(n, 160)) * 0.1, dtype=torch.bfloat16).to(DEV)
+    for end in ("slabs", "bf16", "relu2", "swiglu"):
+        assert torch.equal(ops.gemm_tiles(x, w, end), ops.gemm_tiles(x, w, end, force=441)), end
+    assert torch.equal(ops.gemm_tiles(x, w), ops.gemm_tiles(x, w, force=231))
+
+
 def test_gemm_tiles_refuses_what_it_cannot_do():
     ops = _ops()
     x = torch.zeros(300, 40, dtype=torch.bfloat16, device=DEV)
