@@ -584,8 +584,8 @@ moe_expert_mfma_kernel(const bf16_t* __restrict__ x, const int32_t* __restrict__
 // (up to 64 XF) and 128 WF rows of the expert's matrix (GLU: 64 WF of the gate's and the 64 WF of the up's that belong to them), two waves down and four
 // across.  Bound by the experts' matrices, which arrive at 4.9 to 5.5 TB/s where an expert has up to 100 rows, and by whole rounds of
 // workgroups.  32 experts, [gate; up] of 2 x 2,432 x 2,560, one such matrix, and back, us: the staged kernel or a walk in steps of half
-// lines with tiles of 128 or 256, the best of them / now: 416 rows 161 / 145, 104 / 85, 94 / 77; 2,048 rows 195 / 159, 130 / 101, 119 / 89;
-// 4,000 rows 225 / 181, 149 / 123, 132 / 105; 8,192 rows 345 / 276, 203 / 172, 176 / 142; 128 experts of 768, 3,968 rows 201 / 182, 124 / 100, 127 / 115.
+// lines with tiles of 128 or 256, the best of them / now: 416 rows 161 / 148, 104 / 84, 94 / 82; 2,048 rows 195 / 154, 130 / 91, 119 / 89;
+// 4,000 rows 225 / 175, 149 / 108, 132 / 106; 8,192 rows 345 / 264, 203 / 149, 176 / 143; 128 experts of 768, 3,968 rows 201 / 178, 124 / 94, 127 / 114.
 template <typename TO, bool GLU, int XF, int WF>
 __device__ __forceinline__ void expert_tile(const bf16_t* __restrict__ x, const int32_t* __restrict__ gather, const float* __restrict__ row_weight,
                                             const bf16_t* __restrict__ w_e, TO* __restrict__ out, int row0, int rows, int col0, int n_out, int k,
