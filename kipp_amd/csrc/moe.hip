@@ -689,12 +689,15 @@ moe_expert_tiles_kernel(const bf16_t* __restrict__ x, const int32_t* __restrict_
                         const bf16_t* __restrict__ w, const int32_t* __restrict__ tiles, int max_tiles, int col_tiles, TO* __restrict__ out,
                         int n_out, int k, int act) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
-    // Used tiles come first in the list, an expert's beside each other.  Workgroups id, id + 8, .. run on one die of the chip, each with an
-    // L2 of its own: a die takes a run of (expert, columns, tile), the expert's tiles fastest, so that workgroups which need the same rows of
-    // w walk over them at the same time.
+    // Workgroups id, id + 8, .. run on one die of the chip, each with an L2 of its own: a die takes a run of (tiles of one expert that lie side by
+    // side in the list, columns), those tiles fastest, so that workgroups which need the same rows of w walk over them at the same time.  (The sort
+    // lists an expert's tiles side by side and the used ones first; any other order is as right.)
     const int lane = threadIdx.x & 63;
-    int used = 0;
-    for (int at = 0; at < max_tiles; at += KIPP_WAVE) used += __popcll(__ballot(at + lane < max_tiles && tiles[(size_t)(at + lane) * 3 + 2] > 0));
+    int used = 0;                                       // up to the last tile with rows
+    for (int at = 0; at < max_tiles; at += KIPP_WAVE) {
+        const unsigned long long some = __ballot(at + lane < max_tiles && tiles[(size_t)(at + lane) * 3 + 2] > 0);
+        if (some != 0) used = at + KIPP_WAVE - __clzll((long long)some);
+    }
     const int items = used * col_tiles, per_die = (items + XCDS - 1) / XCDS, die = blockIdx.x % XCDS, turn = blockIdx.x / XCDS;
     // What a die has beyond whole rounds of its compute units goes in halves of the columns where those take one round of half the time
     // (7,204 rows of the experts above, 608 whole ones in three rounds / 512 and 192 halves: 238 and 223 us)
@@ -704,14 +707,15 @@ moe_expert_tiles_kernel(const bf16_t* __restrict__ x, const int32_t* __restrict_
     if (at_die >= mine) return;                         // uniform over the workgroup
     const int item = die * per_die + at_die;
     const int one = item / col_tiles, expert = __builtin_amdgcn_readfirstlane(tiles[(size_t)one * 3]);       // a tile of this item's expert
-    int before = 0, beside = 0;                         // the expert's tiles ahead of that one, and all of them
+    int begin = 0, end = used;                          // the tiles of that expert which lie side by side with it
     for (int at = 0; at < used; at += KIPP_WAVE) {
-        const unsigned long long same = __ballot(at + lane < used && tiles[(size_t)(at + lane) * 3] == expert);
-        beside += __popcll(same);
-        before += one - at >= KIPP_WAVE ? __popcll(same) : (one > at ? __popcll(same & ((1ull << (one - at)) - 1)) : 0);
+        const unsigned long long others = __ballot(at + lane < used && tiles[(size_t)(at + lane) * 3] != expert);
+        const unsigned long long ahead = one - at >= KIPP_WAVE ? others : (one > at ? others & ((1ull << (one - at)) - 1) : 0), behind = others ^ ahead;
+        if (ahead != 0) begin = at + KIPP_WAVE - __clzll((long long)ahead);
+        if (behind != 0 && end == used) end = at + __ffsll((long long)behind) - 1;
     }
-    const int within = item - (one - before) * col_tiles;
-    const int32_t* tile = tiles + (size_t)(one - before + within % beside) * 3;
+    const int beside = end - begin, within = item - begin * col_tiles;
+    const int32_t* tile = tiles + (size_t)(begin + within % beside) * 3;
     const int row0 = __builtin_amdgcn_readfirstlane(tile[1]), rows = __builtin_amdgcn_readfirstlane(tile[2]);
     const int col0 = within / beside * TILE_COLS(GLU) + half * TILE_COLS(GLU) / 2;
     if (col0 >= n_out) return;                          // the last columns may fill less than half a tile

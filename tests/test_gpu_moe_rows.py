@@ -256,6 +256,43 @@ def test_the_walk_over_many_tiles(gated, k, n_out):
         assert torch.equal(out[at:at + n], p), (e, n)
 
 
+@pytest.mark.parametrize("order", ["mixed", "largest first", "gaps", "two in turn"])
+@pytest.mark.parametrize("gated", [False, True])
+@pytest.mark.parametrize("tile_rows", [64, 128, 256])
+def test_lists_of_tiles_in_any_order(order, gated, tile_rows):
+    """Tiles of one expert that do not lie side by side in the list, and unused ones between them: every tile is done once, with its own expert's
+    matrix.  Small whole numbers, so that the sums are exact in any order."""
+    import torch
+    from kipp_amd.csrc import ops
+    rng = np.random.default_rng(tile_rows)
+    k, n_out, experts = 96, 1160, 33
+    counts = [int(rng.choice([0, 1, 64, 65, 130, 257, 520])) for _ in range(experts)]
+    starts = np.cumsum([0] + counts[:-1])
+    rows = int(np.sum(counts))
+    x = torch.tensor(rng.integers(-3, 4, size=(rows, k)), dtype=torch.bfloat16, device=DEV)
+    w = torch.tensor(rng.integers(-2, 3, size=(experts, (2 if gated else 1) * n_out, k)), dtype=torch.bfloat16, device=DEV)
+    tiles = [(e, at + j, min(tile_rows, n - j)) for e, (at, n) in enumerate(zip(starts, counts)) for j in range(0, n, tile_rows)]
+    if order == "largest first":
+        tiles.sort(key=lambda t: -t[2])
+    elif order == "two in turn":
+        tiles = tiles[0::2] + tiles[1::2]
+    else:
+        tiles = [tiles[i] for i in rng.permutation(len(tiles))]
+    if order == "gaps":
+        tiles = [t for tile in tiles for t in ((0, 0, 0), tile)] + [(0, 0, 0)] * 70
+    td = torch.tensor(np.array(tiles, dtype=np.int32), device=DEV)
+    out = torch.full((rows, n_out), float("nan"), device=DEV)
+    if gated:
+        ops.moe_expert_gated(x, None, None, w, td, out, "relu", tile_rows=tile_rows)
+    else:
+        ops.moe_expert(x, None, w, td, out, tile_rows=tile_rows)
+    for e, (at, n) in enumerate(zip(starts, counts)):
+        p = x[at:at + n].float() @ w[e].float().T
+        if gated:
+            p = torch.relu(p[:, :n_out]) * p[:, n_out:]
+        assert torch.equal(out[at:at + n], p), (e, n)
+
+
 @pytest.mark.parametrize("inner", [8, 7])
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("name", ["silu", "gelu", "gelu_tanh"])
