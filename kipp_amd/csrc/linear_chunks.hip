@@ -44,7 +44,6 @@
 #define THREADS 256
 #define UP 68               // floats from a column to the next of U and R in LDS
 #define COLS 16             // columns of S a workgroup of the walk
-#define EIGHT_GROUPS 1024   // workgroups of a walk up to which eight waves each are the faster way with keys of up to 128 (always with longer ones)
 
 #define VECS 4              // vectors of 64 numbers a chunk and head
 
@@ -578,12 +577,12 @@ __global__ void __launch_bounds__(2 * THREADS, 2) chunks_walk_kernel(const Chunk
     }
 }
 
-// The walk of many short portions: four waves that do both, one behind the other.  Its workgroups are half as large, and more than fill the chip;
-// where they do not, a chunk's chain is what counts, and the eight waves are faster.
-// What one of four waves multiplies in a chunk: its own rows of q and A, its rows of K^T, the values of its tokens.
+// The walk of many short portions: four waves that do both, one behind the other (`walk_waves` says when).  Its workgroups are half as large, and more
+// of them than the chip has places for run beside each other; where they do not, a chunk's chain is what counts, and the eight waves are faster.
+// What one of four waves multiplies in a chunk: its own rows of q, k, T and A, its rows of K^T, the values of its tokens.
 template <int MODE, int DT>
 struct FourOperands {
-    f32x4 q[4 * DT], a[4], e[4], kt[DT][4], v, g, b, f;
+    f32x4 q[4 * DT], k[MODE == MODE_DELTA ? 4 * DT : 1], a[4], t[MODE == MODE_DELTA ? 4 : 1], e[4], kt[DT][4], v, g, b, f;
     float g_last;
 };
 
@@ -592,6 +591,7 @@ __global__ void __launch_bounds__(THREADS) chunks_walk_four_kernel(const ChunkAr
     constexpr int D = 64 * DT, SP = D + 4;
     __shared__ __attribute__((aligned(16))) float s_s[COLS * SP];           // [column][row]
     __shared__ __attribute__((aligned(16))) float u_s[COLS * UP];           // [column][token]
+    __shared__ __attribute__((aligned(16))) float r_s[MODE == MODE_DELTA ? COLS * UP : 4];
     const int head = blockIdx.y;
     const Portion portion = portion_of(p.q_len, p.entries, p.from, blockIdx.z);
     if (portion.entry < 0) return;          // uniform over the workgroup
@@ -623,6 +623,7 @@ __global__ void __launch_bounds__(THREADS) chunks_walk_four_kernel(const ChunkAr
 #pragma unroll
         for (int j = 0; j < 4 * DT; ++j) {
             x.q[j] = *reinterpret_cast<const f32x4*>(q + row + 16 * j);
+            if (MODE == MODE_DELTA) x.k[j] = *reinterpret_cast<const f32x4*>(k + row + 16 * j);
         }
     };
     auto rest_of = [&](int c) {
@@ -631,14 +632,18 @@ __global__ void __launch_bounds__(THREADS) chunks_walk_four_kernel(const ChunkAr
         const float* vec = p.vec + at * VECS * CHUNK;
         if (own < m) {
             const float* a_row = p.a + at * CHUNK * CHUNK + (own + l16) * CHUNK + h4;
+            const float* t_row = p.t + at * CHUNK * CHUNK + (own + l16) * CHUNK + h4;
 #pragma unroll
             for (int i = 0; i < 4; ++i) x.v[i] = own + h4 + i < m ? v_src[(size_t)(t0 + own + h4 + i) * p.stride] : 0.0f;
             x.g = *reinterpret_cast<const f32x4*>(vec + own + h4);
-            if (MODE == MODE_MLSTM) x.b = *reinterpret_cast<const f32x4*>(vec + 2 * CHUNK + own + h4);
+            if (MODE == MODE_DELTA || MODE == MODE_MLSTM) x.b = *reinterpret_cast<const f32x4*>(vec + 2 * CHUNK + own + h4);
             if (MODE == MODE_MLSTM) x.f = *reinterpret_cast<const f32x4*>(vec + 3 * CHUNK + own + h4);
 #pragma unroll
             for (int j = 0; j < 4; ++j)
-                if (j <= wave) x.a[j] = *reinterpret_cast<const f32x4*>(a_row + 16 * j);
+                if (j <= wave) {
+                    if (MODE == MODE_DELTA) x.t[j] = *reinterpret_cast<const f32x4*>(t_row + 16 * j);
+                    x.a[j] = *reinterpret_cast<const f32x4*>(a_row + 16 * j);
+                }
         }
         x.g_last = vec[CHUNK - 1];
 #pragma unroll
@@ -662,12 +667,12 @@ __global__ void __launch_bounds__(THREADS) chunks_walk_four_kernel(const ChunkAr
 #pragma unroll
         for (int a = 0; a < DT; ++a) *reinterpret_cast<f32x4*>(&s_s[l16 * SP + row0 + 16 * a + h4]) = S[a];
         __syncthreads();
-        f32x4 inter = zero4();
+        f32x4 inter = zero4(), read = zero4();
         if (mine) {
             constexpr int RUNS = runs_of(MODE, DT);
-            f32x4 in[RUNS][1];
+            f32x4 in[RUNS][1], rd[RUNS][1];
 #pragma unroll
-            for (int h = 0; h < RUNS; ++h) in[h][0] = zero4();
+            for (int h = 0; h < RUNS; ++h) in[h][0] = rd[h][0] = zero4();
 #pragma unroll
             for (int j = 0; j < 4 * DT; j += RUNS) {
                 f32x4 sv[RUNS];
@@ -676,19 +681,34 @@ __global__ void __launch_bounds__(THREADS) chunks_walk_four_kernel(const ChunkAr
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
 #pragma unroll
-                    for (int h = 0; h < RUNS; ++h) in[h][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.q[j + h][i], sv[h][i], in[h][0], 0, 0, 0);
+                    for (int h = 0; h < RUNS; ++h) {
+                        in[h][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.q[j + h][i], sv[h][i], in[h][0], 0, 0, 0);
+                        if (MODE == MODE_DELTA) rd[h][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.k[j + h][i], sv[h][i], rd[h][0], 0, 0, 0);
+                    }
             }
             inter = sum_runs(in, 0);
+            if (MODE == MODE_DELTA) read = sum_runs(rd, 0);
             f32x4 u = x.v;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 if (MODE == MODE_DECAY) u[i] = silu_f(u[i]);        // silu(0) = 0
                 if (MODE == MODE_MLSTM) u[i] = x.b[i] * (norm ? 1.0f : u[i]);       // a gate of zero beyond the last token
+                if (MODE == MODE_DELTA) u[i] = own + h4 + i < m ? x.b[i] * (x.v[i] - x.g[i] * read[i]) : 0.0f;
             }
-            *reinterpret_cast<f32x4*>(u_s + l16 * UP + own + h4) = u;
+            *reinterpret_cast<f32x4*>((MODE == MODE_DELTA ? r_s : u_s) + l16 * UP + own + h4) = u;
         }
         if (more) rows_of(c + 1);
         __syncthreads();
+        if (MODE == MODE_DELTA) {
+            if (mine) {
+                f32x4 u = zero4();
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    if (j <= wave) u = mul16(x.t[j], *reinterpret_cast<const f32x4*>(r_s + l16 * UP + 16 * j + h4), u);
+                *reinterpret_cast<f32x4*>(u_s + l16 * UP + own + h4) = u;
+            }
+            __syncthreads();
+        }
         f32x4 u[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j)
@@ -749,18 +769,41 @@ static void lay_out(ChunkArgs& p, int mode, long long slots_all, float* work) {
     p.vec = p.t + slots_all * CHUNK * CHUNK;
 }
 
+// Eight waves a workgroup of the walk, or four.  Eight shorten the chain of a chunk; four start and end sooner and fit twice or more often on a
+// compute unit (registers; from keys of 256 on, 128 for the delta rule, they fit once only and eight always win).  So four have many short
+// portions: more workgroups than compute units (fixed decays of short keys, whose values are work ahead of the chain: three or four to a unit) and two
+// chunks a portion ahead for every one a unit.  Calls of four / eight waves, us: 64 portions of 80 tokens, 16 heads of 192 x 128, a decay a token 225 / 307, an mLSTM 347 /
+// 442; delta rule, 32 heads of 64 x 64, 64 portions of 64 176 / 235, 4 of 64 30.5 / 32.4; 4 of 80, 16 heads of 128 x 128, a decay a token 22 / 25; and the other
+// way 16 heads of 128 x 128, 10 portions of 1,000 tokens 12 % and one of 2,048 26 % less with eight.  1,350 calls of both, from 16 to 12,800 workgroups and 64 to 2,048
+// tokens: this choice is 0.2 % over the faster one in the mean, eight waves up to 1,024 workgroups (keys of 128) or always were 2.6.
+static int walk_waves(int mode, int dt, long long groups, int chunks) {
+    if (dt >= (mode == MODE_DELTA ? 2 : 4)) return 8;
+    const int units = 256, places = dt == 1 && (mode == MODE_DECAY || mode == MODE_GATED) ? 2 * units : units;        // of eight waves: two fit where they have 128 registers
+    const int always = mode != MODE_DECAY || dt > 2 ? units : (dt == 1 ? 4 * units : 3 * units);
+    // (an mLSTM's eight waves have 130 registers with keys of 64: what is one round of four waves is two of eight)
+    if (mode == MODE_MLSTM && dt == 1 && groups > units && groups <= 2 * units) return 4;
+    return groups <= always || groups <= (long long)places * (chunks - 2) ? 8 : 4;
+}
+
 template <int MODE, int DT>
 static void launch_chunks(const ChunkArgs& p, int longest, int portions, hipStream_t stream) {
     const int cols = p.dv + (MODE == MODE_MLSTM ? 1 : 0);
     const dim3 prepare((longest + CHUNK - 1) / CHUNK, p.heads, portions), walk((cols + COLS - 1) / COLS, p.heads, portions), block(THREADS);
     hipLaunchKernelGGL((chunks_prepare_kernel<MODE, DT>), prepare, block, 0, stream, p);
-    if constexpr (MODE != MODE_DELTA && DT <= 2) {
-        if ((long long)walk.x * walk.y * walk.z > EIGHT_GROUPS) {
+    if constexpr (DT < (MODE == MODE_DELTA ? 2 : 4)) {
+        if (walk_waves(MODE, DT, (long long)walk.x * walk.y * walk.z, (longest + CHUNK - 1) / CHUNK) == 4) {
             hipLaunchKernelGGL((chunks_walk_four_kernel<MODE, DT>), walk, block, 0, stream, p);
             return;
         }
     }
     hipLaunchKernelGGL((chunks_walk_kernel<MODE, DT>), walk, dim3(2 * THREADS), 0, stream, p);
+}
+
+// Waves of a workgroup of the walk, 4 or 8, as a launch of these sizes has them; 0 where chunks do not take them.
+extern "C" int kipp_matrix_chunks_waves(int mode, int heads, int d, int dv, int longest, int portions) {
+    if (kipp_matrix_chunks_work(mode, 1, 1, heads, d) == 0 || dv <= 0 || longest <= 0 || portions <= 0) return 0;
+    const int cols = dv + (mode == MODE_MLSTM ? 1 : 0);
+    return walk_waves(mode, d / 64, (long long)((cols + COLS - 1) / COLS) * heads * portions, (longest + CHUNK - 1) / CHUNK);
 }
 
 template <int MODE>

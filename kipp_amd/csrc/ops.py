@@ -802,6 +802,11 @@ def matrix_chunks_ok(d: int) -> bool:
     return d % 64 == 0 and 0 < d <= 256
 
 
+def matrix_chunks_waves(mode: int, heads: int, d: int, dv: int, longest: int, portions: int) -> int:
+    """Waves of a workgroup of the walk over chunks, 4 or 8, in a step of so many portions whose longest has `longest` tokens (`mode` as above)."""
+    return _fn("linear_chunks", "kipp_matrix_chunks_waves", [_c_int] * 6)(int(mode), int(heads), int(d), int(dv), int(longest), int(portions))
+
+
 def _chunk_portions(mode, src, q_at, k_at, state, q_start, heads, d, dv, longest, portions):
     """(entries that may go by chunks, tokens below which entries are left for the walk): (0, 0) where chunks do not take the sizes or are not the
     faster way; below is -1 where there are no others."""

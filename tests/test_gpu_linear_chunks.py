@@ -301,9 +301,10 @@ def test_mlstm_walk_of_some_entries(d, dv, few):
             assert bool((o_some[at:at + n] == 7.0).all()) and torch.equal(state_some[e], kept[e]), e
 
 
-@pytest.mark.parametrize("mode, d", [("decay", 64), ("decay", 128), ("gated", 64), ("gated", 128), ("mlstm", 64), ("mlstm", 128)])
+@pytest.mark.parametrize("mode, d", [("decay", 64), ("decay", 128), ("decay", 192), ("gated", 64), ("gated", 128), ("gated", 192), ("mlstm", 64), ("mlstm", 128),
+                                     ("mlstm", 192), ("delta", 64)])
 def test_many_portions_have_the_bits_of_few(mode, d):
-    """More than 1,024 workgroups of a walk go by four waves that do both, fewer by eight: the same bits, of portions of one, two and three chunks, whole
+    """Many workgroups of a walk go by four waves that do both, few by eight: the same bits, of portions of one, two and three chunks, whole
     and not."""
     import torch
     from kipp_amd.csrc import ops
@@ -319,6 +320,11 @@ def test_many_portions_have_the_bits_of_few(mode, d):
     elif mode == "decay":
         src = torch.randn(tokens, 2 * heads * d + heads * dv, device=DEV, generator=gen)
         decays, size = torch.rand(heads, device=DEV, generator=gen), heads * d * dv
+    elif mode == "delta":
+        src = torch.randn(tokens, heads * d + heads * dv + 2 * heads, device=DEV, generator=gen)
+        src[:, :heads * d] *= d ** -0.5
+        src[:, heads * d + heads * dv:].uniform_(0.5, 1.0, generator=gen)
+        size = heads * d * dv
     else:
         src = torch.randn(tokens, ops.ssd_prep_width(heads, 1, d, dv), device=DEV, generator=gen)
         src[:, 2 * d + 2 * heads * dv:].uniform_(0.5, 1.0, generator=gen)
@@ -334,9 +340,13 @@ def test_many_portions_have_the_bits_of_few(mode, d):
             return state, o, den
         if mode == "decay":
             ops.decay_scan(src, decays, *where, heads, d, dv, longest=longest, chunks=True, portions=portions)
+        elif mode == "delta":
+            ops.delta_scan(src, *where, heads, heads // 2, d, dv, longest=longest, chunks=True, portions=portions)
         else:
             ops.gated_scan(src, *where, heads, 1, d, dv, longest=longest, chunks=True, portions=portions)
         return state, o, torch.zeros(tokens, heads, device=DEV)
+    kind = ["decay", "delta", "gated", "mlstm"].index(mode)
+    assert ops.matrix_chunks_waves(kind, heads, d, dv, max(lengths), n) == 4 and all(ops.matrix_chunks_waves(kind, heads, d, dv, e, 1) == 8 for e in lengths)
     real, ops.matrix_chunks_from = ops.matrix_chunks_from, lambda *a: 16
     try:
         together = run(list(range(n)))
