@@ -1109,6 +1109,39 @@ def test_gemm_tiles_plans_where_tiles_of_192_columns_fit_best(m, n):
     assert torch.equal(ops.gemm_tiles(x, w), ops.gemm_tiles(x, w, force=231))
 
 
+def _microseconds(run, calls=10):
+    """The shortest of six groups of calls."""
+    run()
+    marks = [(torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)) for _ in range(6)]
+    for begin, end in marks:
+        begin.record()
+        for _ in range(calls):
+            run()
+        end.record()
+    torch.cuda.synchronize()
+    return 1000 * min(a.elapsed_time(b) for a, b in marks) / calls
+
+
+@pytest.mark.parametrize("parts", [1, 2])
+@pytest.mark.parametrize("n", [389, 390, 391, 513])
+def test_gemm_tiles_odd_columns(n, parts):
+    """Rows of the float32 result that begin at no multiple of 16 bytes, and end inside a run of four columns: every tile, exactly on small integers."""
+    ops = _ops()
+    rng = np.random.default_rng(n)
+    xi, wi = (torch.tensor(rng.integers(-3, 4, size=(a, 96)), dtype=torch.bfloat16) for a in (301, n))
+    for tile in (44, 43, 42, 24, 23, 22):
+        got = ops.gemm_tiles(xi.to(DEV), wi.to(DEV), "slabs", max_parts=4, force=10 * tile + parts)
+        assert torch.equal(got.sum(dim=0).cpu(), xi.float() @ wi.float().T), tile
+
+
+def test_gemm_tiles_odd_columns_are_not_much_slower():
+    """A product of few steps of K is its stores: one column more takes no number of them apart (2.6 times as long where it did)."""
+    ops = _ops()
+    x, w = torch.randn(1923, 64, device=DEV).bfloat16(), torch.randn(15473, 64, device=DEV).bfloat16()
+    odd, even = (_microseconds(lambda: ops.gemm_tiles(x, w[:n])) for n in (15473, 15472))
+    assert odd < 1.5 * even, (odd, even)
+
+
 def test_gemm_tiles_refuses_what_it_cannot_do():
     ops = _ops()
     x = torch.zeros(300, 40, dtype=torch.bfloat16, device=DEV)
