@@ -683,12 +683,16 @@ __device__ __forceinline__ void expert_tile(const bf16_t* __restrict__ x, const 
     }
 }
 
-template <typename TO, bool GLU>
-__global__ void __launch_bounds__(512, 2)
+// FEW: tiles of up to 64 rows alone.  Their 80 KB of LDS (128 KB where tiles of 256 may come) and 128 registers let two workgroups share a compute unit, one's
+// start and end beside the other's walk: 256 experts of 2 rows each, gated 704 x 384 43 us, alone on a compute unit 59 (the staged kernel 48); 2,048 x 256 of
+// 12 rows 55, 78 (71); 6,400 x 64 gated of 2 153, 226 (152); 102 such products of K from 32 to 1,024: 0.83 of the time in the mean.
+template <typename TO, bool GLU, bool FEW>
+__global__ void __launch_bounds__(512, FEW ? 4 : 2)
 moe_expert_tiles_kernel(const bf16_t* __restrict__ x, const int32_t* __restrict__ gather, const float* __restrict__ row_weight,
                         const bf16_t* __restrict__ w, const int32_t* __restrict__ tiles, int max_tiles, int col_tiles, TO* __restrict__ out,
                         int n_out, int k, int act) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
+    constexpr int PLACES = DIE_UNITS * (FEW ? 2 : 1);       // of a die
     // Workgroups id, id + 8, .. run on one die of the chip, each with an L2 of its own: a die takes a run of (tiles of one expert that lie side by
     // side in the list, columns), those tiles fastest, so that workgroups which need the same rows of w walk over them at the same time.  (The sort
     // lists an expert's tiles side by side and the used ones first; any other order is as right.)
@@ -701,8 +705,8 @@ moe_expert_tiles_kernel(const bf16_t* __restrict__ x, const int32_t* __restrict_
     const int items = used * col_tiles, per_die = (items + XCDS - 1) / XCDS, die = blockIdx.x % XCDS, turn = blockIdx.x / XCDS;
     // What a die has beyond whole rounds of its compute units goes in halves of the columns where those take one round of half the time
     // (7,204 rows of the experts above, 608 whole ones in three rounds / 512 and 192 halves: 238 and 223 us)
-    const int mine = min(per_die, items - die * per_die), whole = mine / DIE_UNITS * DIE_UNITS, rest = mine - whole;
-    const bool halved = turn >= whole && 2 * rest <= DIE_UNITS;
+    const int mine = min(per_die, items - die * per_die), whole = mine / PLACES * PLACES, rest = mine - whole;
+    const bool halved = turn >= whole && 2 * rest <= PLACES;
     const int at_die = halved ? whole + (turn - whole) / 2 : turn, half = halved ? (turn - whole) & 1 : 0;
     if (at_die >= mine) return;                         // uniform over the workgroup
     const int item = die * per_die + at_die;
@@ -726,6 +730,10 @@ moe_expert_tiles_kernel(const bf16_t* __restrict__ x, const int32_t* __restrict_
         if (halved) expert_tile<TO, GLU, N, 1>(x, gather, row_weight, w_e, out, row0, rows, col0, n_out, k, act, lds);                  \
         else expert_tile<TO, GLU, N, 2>(x, gather, row_weight, w_e, out, row0, rows, col0, n_out, k, act, lds);                          \
         break
+    if constexpr (FEW) {
+        switch ((rows + 63) / 64) { KIPP_ET(1); }
+        return;
+    }
     switch ((rows + 63) / 64) {
         KIPP_ET(1);
         KIPP_ET(2);
@@ -980,20 +988,20 @@ extern "C" int kipp_moe_route_grouped(const float* z, int parts, int stride, con
     return KIPP_LAUNCH_CHECK();
 }
 
-template <typename TO, bool GLU>
+template <typename TO, bool GLU, bool FEW>
 static int launch_tiles(const void* x, const int32_t* gather, const float* row_weight, const void* w, const int32_t* tiles, int max_tiles,
                         void* out, int n_out, int k, int act, hipStream_t stream) {
-    constexpr int lds_bytes = LineWalk<MANY_ROWS / 64, 2, 2, TILE_ACROSS>::LDS_BYTES;
+    constexpr int lds_bytes = LineWalk<FEW ? 1 : MANY_ROWS / 64, 2, 2, TILE_ACROSS>::LDS_BYTES;
     static bool prepared = false;
     if (!prepared) {
-        if (hipFuncSetAttribute((const void*)moe_expert_tiles_kernel<TO, GLU>, hipFuncAttributeMaxDynamicSharedMemorySize,
+        if (hipFuncSetAttribute((const void*)moe_expert_tiles_kernel<TO, GLU, FEW>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 lds_bytes) != hipSuccess)
             return -6;
         prepared = true;
     }
     const int col_tiles = (n_out + TILE_COLS(GLU) - 1) / TILE_COLS(GLU);
-    const int grid = XCDS * ((max_tiles * col_tiles + XCDS - 1) / XCDS + DIE_UNITS / 2);        // halves: as many more
-    hipLaunchKernelGGL((moe_expert_tiles_kernel<TO, GLU>), dim3(grid), dim3(512), lds_bytes, stream, (const bf16_t*)x,
+    const int grid = XCDS * ((max_tiles * col_tiles + XCDS - 1) / XCDS + DIE_UNITS / (FEW ? 1 : 2));        // halves: as many more
+    hipLaunchKernelGGL((moe_expert_tiles_kernel<TO, GLU, FEW>), dim3(grid), dim3(512), lds_bytes, stream, (const bf16_t*)x,
                        gather, row_weight, (const bf16_t*)w, tiles, max_tiles, col_tiles, (TO*)out, n_out, k, act);
     return KIPP_LAUNCH_CHECK();
 }
@@ -1008,7 +1016,7 @@ static int launch_expert(const void* x, int x_dtype, const int32_t* gather, cons
     // in the walk; rows of x that `gather` may name reach as far as x does
     const bool fits = (long long)max_tiles * tile_rows * k < (1ll << 31) && (long long)(GLU ? 2 : 1) * n_out * k < (1ll << 31) &&
                       (long long)x_rows * k < (1ll << 32);
-    // Tiles of few rows whose workgroups would have little of K each, and be many, are the walk's: beside the staged kernel, which the walk is as fast as here,
+    // Tiles of few rows whose workgroups would have little of K each, and be many, are the walk's: beside the staged kernel, in whose time the walk takes 0.78 here,
     // the one for few rows takes, 256 experts of 1,024 x 512 and 10 pairs an expert, 1.25 and 1.5 of the time (gated, and back); 64 of 2,048 x 704, up 0.8, back 1.35.
     const long long hit = sorted_rows < experts ? sorted_rows : experts;
     const bool short_k = k <= ROWS_SHORT_K && hit * ((n_out + 15) / 16) > ROWS_SHORT_GROUPS;
@@ -1043,8 +1051,10 @@ static int launch_expert(const void* x, int x_dtype, const int32_t* gather, cons
             return KIPP_LAUNCH_CHECK();
         }
         if (!walks) return -2;
-        if (out_dtype == KIPP_BF16) return launch_tiles<bf16_t, GLU>(x, gather, row_weight, w, tiles, max_tiles, out, n_out, k, act, stream);
-        if (out_dtype == KIPP_F32) return launch_tiles<float, GLU>(x, gather, row_weight, w, tiles, max_tiles, out, n_out, k, act, stream);
+        if (out_dtype == KIPP_BF16) return tile_rows == ROWS_TILE ? launch_tiles<bf16_t, GLU, true>(x, gather, row_weight, w, tiles, max_tiles, out, n_out, k, act, stream)
+                                       : launch_tiles<bf16_t, GLU, false>(x, gather, row_weight, w, tiles, max_tiles, out, n_out, k, act, stream);
+        if (out_dtype == KIPP_F32) return tile_rows == ROWS_TILE ? launch_tiles<float, GLU, true>(x, gather, row_weight, w, tiles, max_tiles, out, n_out, k, act, stream)
+                                       : launch_tiles<float, GLU, false>(x, gather, row_weight, w, tiles, max_tiles, out, n_out, k, act, stream);
         return -2;
     }
     if (tile_rows != TILE_ROWS) return -1;

@@ -293,6 +293,39 @@ def test_lists_of_tiles_in_any_order(order, gated, tile_rows):
         assert torch.equal(out[at:at + n], p), (e, n)
 
 
+@pytest.mark.parametrize("k, n_out, each, gated", [(384, 704, 2, True), (256, 2048, 12, False)])
+def test_many_tiles_of_few_rows_share_compute_units(k, n_out, each, gated):
+    """Products of little K over many tiles of up to 64 rows are their starts and ends, which two workgroups a compute unit hide from each other: faster than
+    the same tiles where larger ones may come (level with those, and slower than the staged kernel, where they had a compute unit each)."""
+    import torch
+    from kipp_amd.csrc import ops
+    experts = 256
+    x = torch.randn(experts * each, k, device=DEV).bfloat16()
+    w = torch.randn(experts, (2 if gated else 1) * n_out, k, device=DEV).bfloat16()
+    td = torch.tensor([(e, e * each, each) for e in range(experts)], dtype=torch.int32, device=DEV)
+    out = torch.empty(experts * each, n_out, dtype=torch.bfloat16, device=DEV)
+
+    def run(rows):
+        if gated:
+            ops.moe_expert_gated(x, None, None, w, td, out, "silu", tile_rows=rows)
+        else:
+            ops.moe_expert(x, None, w, td, out, "silu", tile_rows=rows)
+        return out
+    assert torch.equal(run(64).clone(), run(128))
+    took = {64: [], 128: []}
+    for _ in range(6):
+        for rows in took:
+            begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            begin.record()
+            for _ in range(20):
+                run(rows)
+            end.record()
+            took[rows].append((begin, end))
+    torch.cuda.synchronize()
+    few, whole = (min(a.elapsed_time(b) for a, b in took[rows]) for rows in (64, 128))
+    assert few < 0.9 * whole, (few, whole)
+
+
 @pytest.mark.parametrize("inner", [8, 7])
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("name", ["silu", "gelu", "gelu_tanh"])
