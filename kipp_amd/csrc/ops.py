@@ -1165,10 +1165,13 @@ def moe_tile_rows(dtype: torch.dtype, *contractions: int, pairs: Optional[int] =
     return MOE_MFMA_ROWS
 
 
-# Pairs an expert up to which a step stays with the kernel for few rows where the walk could take it: 32 experts of 2,560 x 2,432, both
-# products, few rows / walk, us: 3 an expert 141 / 153, gated 201 / 213; 5 an expert 162 / 159, 229 / 222; of 4,096 x 3,072 252 / 261, 378 / 388; 293 / 280, 433 / 427.
-# Gated experts of few numbers keep it as long as `moe_tile_rows` says (a walk's start counts there: 64 of 2,048 x 704, 5 an expert 97 / 118).
-MOE_STEP_FEW_PAIRS, MOE_STEP_FEW_NUMBERS = 4, 200_000_000
+# Pairs an expert up to which a step stays with the kernel for few rows where the walk could take it, and how many numbers one matrix of all the experts has
+# where it stays as long as `moe_tile_rows` says: an item of the walk takes its start and end whatever it multiplies, and few or small experts are few items.
+# Both products, few rows / walk, us: 1 expert of 4,096 x 3,072, 6 pairs 21 / 45; 3 of 4,096 x 768, 9 an expert 17 / 26; 8 of 4,096 x 96, 5 an expert 21 / 31; and
+# the other way 32 of 5,120 x 1,024, 9 an expert 155 / 129, 16 of 5,120 x 1,408 gated, 10 an expert 172 / 142.  2,162 steps of 1 to 256 experts that
+# `moe_tile_rows` leaves to few rows: 0.8 % over the faster one in the mean and 1.09 of few rows' time at worst; with the walk beyond four pairs an
+# expert whatever the size those without a gate took 17 % and up to 2.1 times.
+MOE_STEP_FEW_PAIRS, MOE_STEP_FEW_NUMBERS = 6, 120_000_000
 
 
 def moe_step_tile_rows(dtype: torch.dtype, *contractions: int, pairs: int, experts: int = 1, gated: bool = False, aligned: bool = True,
@@ -1179,7 +1182,7 @@ def moe_step_tile_rows(dtype: torch.dtype, *contractions: int, pairs: int, exper
     rows = moe_tile_rows(dtype, *contractions, pairs=pairs, experts=experts, gated=gated, aligned=aligned, identity=identity)
     if rows == MOE_TILE_ROWS or not aligned:
         return rows
-    small = gated and 2 * experts * max(contractions) * min(contractions) <= MOE_STEP_FEW_NUMBERS
+    small = experts * max(contractions) * min(contractions) <= MOE_STEP_FEW_NUMBERS
     if rows == MOE_FEW_ROWS and (small or pairs * experts / (experts + identity) <= MOE_STEP_FEW_PAIRS * experts):
         return rows
     groups = (pairs / MOE_MANY_ROWS + experts / 2) * -(-contractions[-1] // (128 if gated else 256))

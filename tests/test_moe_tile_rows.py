@@ -31,12 +31,20 @@ def test_many_rows_an_expert():
 
 
 def test_rows_of_a_step():
-    """The kernel for few rows up to four pairs an expert, or as long as it may where a gated step has few numbers; then the walk, in tiles of 256
+    """The kernel for few rows up to six pairs an expert, or as long as it may where the experts have few numbers; then the walk, in tiles of 256
     where those are workgroups enough; what begins at no multiple of 16 bytes, and float32, as ever."""
     rows = lambda experts, width, inner, pairs, gated, **k: ops.moe_step_tile_rows(k.pop("dtype", torch.bfloat16), width, inner, pairs=pairs, experts=experts, gated=gated, **k)  # noqa: E731
-    assert [rows(32, 2560, 2432, n, g) for g in (False, True) for n in (128, 129)] == [64, 256, 64, 256]
-    assert [rows(32, 2560, 2432, n, False, identity=8) for n in (160, 161)] == [64, 256]
-    assert [rows(64, 2048, 704, 64 * 6 + n, g) for g in (False, True) for n in (0, 1)] == [128, 128, 64, 256]
-    assert [rows(8, 1024, 1024, n, False) for n in (30, 200, 8 * 512, 8 * 900)] == [64, 128, 128, 256]
+    assert [rows(32, 2560, 2432, n, g) for g in (False, True) for n in (192, 193)] == [64, 256, 64, 256]
+    assert [rows(32, 2560, 2432, n, False, identity=8) for n in (240, 241)] == [64, 256]
+    assert [rows(64, 2048, 704, 64 * 6 + n, g) for g in (False, True) for n in (0, 1)] == [64, 128, 64, 256]
+    assert [rows(32, 2048, 1408, 32 * n, g) for g in (False, True) for n in (12, 13)] == [64, 128, 64, 256]      # 92 million numbers
+    assert [rows(8, 1024, 1024, n, False) for n in (30, 96, 97, 8 * 512, 8 * 900)] == [64, 64, 128, 128, 256]
     assert [rows(32, 2560, 2432, n, True, aligned=False) for n in (1, 500, 9000)] == [128, 128, 128]
     assert rows(32, 2560, 2432, 9000, True, dtype=torch.float32) == 16
+
+
+@pytest.mark.parametrize("experts, width, inner, pairs", [(1, 4096, 3072, 6), (3, 4096, 768, 26), (1, 64, 96, 7), (16, 512, 4096, 88), (8, 4096, 96, 36), (2, 5120, 4096, 20), (16, 2048, 2432, 130)])
+@pytest.mark.parametrize("gated", [False, True])
+def test_few_or_small_experts_keep_the_kernel_for_few_rows(experts, width, inner, pairs, gated):
+    """Sizes at which the walk took 1.1 to 2.1 times as long."""
+    assert ops.moe_step_tile_rows(torch.bfloat16, width, inner, pairs=pairs, experts=experts, gated=gated) == 64
