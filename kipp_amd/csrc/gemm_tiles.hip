@@ -70,10 +70,10 @@ __global__ void __launch_bounds__(512, (LineWalk<XF, WF, GM, GN>::LDS_BYTES <= 6
     using Walk = LineWalk<XF, WF, GM, GN>;
     constexpr bool PAIRS = pairs_columns(END);
     constexpr int OUT_N = PAIRS ? Walk::TN / 2 : Walk::TN;         // output columns of a tile
-    // The bfloat16 ends of fragments that come in pairs: rows 4 q .. + 3 of the two fragments are W's rows 8 q .. + 7 of the
+    // The bfloat16 ends: rows 4 q .. + 3 of two neighbouring fragments are W's rows 8 q .. + 7 of the
     // pair's 32, so that a lane holds 8 neighbouring columns of its row.
-    constexpr bool EIGHT = END != END_SLABS && WF % 2 == 0;
-    static_assert(WF != 3 || END == END_SLABS, "three fragments across only for the float32 end");
+    constexpr bool EIGHT = END != END_SLABS;
+    static_assert(WF % 2 == 0 || !EIGHT, "pairs of fragments across for the bfloat16 ends");
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
 
     const int lane = threadIdx.x & 63;
@@ -150,12 +150,14 @@ __global__ void __launch_bounds__(512, (LineWalk<XF, WF, GM, GN>::LDS_BYTES <= 6
             }
         }
     } else {
-        constexpr int RUN = EIGHT ? 8 : 4;                         // neighbouring columns a lane holds
+        constexpr int RUN = 8;                                     // neighbouring columns a lane holds
         constexpr int RUNS = (PAIRS ? 1 : 2) * 16 * WF / (4 * RUN);  // runs of columns of a row
         const int width = PAIRS ? inner : N;
         const int col0 = col_begin + tn * OUT_N + wave % GN * (PAIRS ? 16 * WF : 32 * WF) + RUN * quarter;
         bf16_t* out = (bf16_t*)Y;
-        const bool whole = (width & (RUN - 1)) == 0;
+        // (rows begin at any multiple of 2 bytes where the width is no multiple of 8: 16 bytes a store there too, as above.  1,016 x 12,980 x 32 with
+        // relu^2 36 -> 13 us, 2,534 x 8,394 x 256 60 -> 23; 120 such sizes of all ends 0.76 of the time in the mean)
+        typedef u32x4 __attribute__((aligned(2))) u32x4_any;
 #pragma unroll
         for (int g = 0; g < RUNS; ++g) {
             const int col = col0 + 4 * RUN * g;
@@ -189,14 +191,11 @@ __global__ void __launch_bounds__(512, (LineWalk<XF, WF, GM, GN>::LDS_BYTES <= 6
                 }
                 if (row >= M) continue;
                 bf16_t* at = out + (size_t)row * width + col;
-                if (whole && col + RUN <= col_end) {
+                if (col + RUN <= col_end) {
                     uint32_t packed[RUN / 2];
 #pragma unroll
                     for (int c = 0; c < RUN / 2; ++c) packed[c] = (uint32_t)value_of[2 * c] | ((uint32_t)value_of[2 * c + 1] << 16);
-                    if constexpr (RUN == 8)
-                        *(u32x4*)at = (u32x4){packed[0], packed[1], packed[2], packed[3]};
-                    else
-                        *(uint2*)at = make_uint2(packed[0], packed[1]);
+                    *(u32x4_any*)at = (u32x4){packed[0], packed[1], packed[2], packed[3]};
                 } else {
 #pragma unroll
                     for (int c = 0; c < RUN; ++c)

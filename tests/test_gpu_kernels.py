@@ -1134,11 +1134,33 @@ def test_gemm_tiles_odd_columns(n, parts):
         assert torch.equal(got.sum(dim=0).cpu(), xi.float() @ wi.float().T), tile
 
 
-def test_gemm_tiles_odd_columns_are_not_much_slower():
-    """A product of few steps of K is its stores: one column more takes no number of them apart (2.6 times as long where it did)."""
+@pytest.mark.parametrize("end", ["bf16", "relu2", "swiglu", "glu"])
+@pytest.mark.parametrize("n", [386, 388, 389, 391, 519])
+def test_gemm_tiles_odd_columns_of_bfloat16(n, end):
+    """Rows of the bfloat16 results that begin at any multiple of 2 bytes, and end inside a run of eight columns: every tile."""
     ops = _ops()
-    x, w = torch.randn(1923, 64, device=DEV).bfloat16(), torch.randn(15473, 64, device=DEV).bfloat16()
-    odd, even = (_microseconds(lambda: ops.gemm_tiles(x, w[:n])) for n in (15473, 15472))
+    rng = np.random.default_rng(n)
+    pairs = end in ("swiglu", "glu")
+    x, w = (torch.tensor(rng.integers(-3, 4, size=(a, 96)), dtype=torch.bfloat16).to(DEV) for a in (301, 2 * n if pairs else n))
+    exact = (x.float() @ w.float().T).double()
+    ref = {"bf16": exact, "relu2": torch.relu(exact) ** 2, "swiglu": exact[:, :n] * torch.sigmoid(exact[:, :n]) * exact[:, n:] if pairs else None,
+           "glu": torch.relu(exact[:, :n]) * exact[:, n:] if pairs else None}[end]
+    for tile in (44, 42, 24, 22):
+        got = ops.gemm_tiles(x, w, end, force=10 * tile + 1, **({"activation": "relu"} if end == "glu" else {}))
+        assert got.shape == ref.shape
+        if end == "swiglu":     # a float32 sigmoid and two products ahead of the rounding
+            assert bool(((got.double() - ref).abs() <= (2.0 ** -8 + 1e-5) * ref.abs() + 1e-30).all()), tile
+        else:                   # whole numbers below 2^24: rounded once
+            assert torch.equal(got, ref.float().bfloat16()), tile
+
+
+@pytest.mark.parametrize("end, m, n, k", [("slabs", 1923, 15473, 64), ("relu2", 1016, 12980, 32), ("swiglu", 2534, 4197, 64)])
+def test_gemm_tiles_odd_columns_are_not_much_slower(end, m, n, k):
+    """A product of few steps of K is its stores: some columns more take no number of them apart (2.6 times as long where they did)."""
+    ops = _ops()
+    x, w = torch.randn(m, k, device=DEV).bfloat16(), torch.randn(2 * n, k, device=DEV).bfloat16()
+    rows = 2 if end == "swiglu" else 1
+    odd, even = (_microseconds(lambda: ops.gemm_tiles(x, w[:rows * c], end)) for c in (n, n // 16 * 16))
     assert odd < 1.5 * even, (odd, even)
 
 
