@@ -1123,21 +1123,19 @@ MOE_TILE_ROWS = 16
 MOE_MFMA_ROWS = 128    # rows of a tile of the experts' products on the matrix cores
 MOE_FEW_ROWS = 64      # the same in the kernel for few rows an expert, which reads the experts' matrices straight into the products
 MOE_MANY_ROWS = 256    # the same where an expert has many rows: its matrix is read less often, a compute unit has one workgroup
-# A step takes the kernel for few rows up to so many pairs an expert (all of them), and fewer where there is more of the experts' matrices: each 16
-# rows more of an expert are its matrix once more from the caches.  Whole steps of four layers, kernel for few rows over tiles of 128, routed
-# as a trained model routes, at 5, 7, 9, 11, 13 pairs.  Without a gate: 32 experts of 2,560 x 2,432 0.88 0.92 0.95 0.97 0.99, 32 of 4,096 x 3,072
-# 0.94 0.99 1.03 1.06 1.09, 16 of 5,120 x 3,200 0.95 0.98 1.01 1.03 1.05, 16 of 2,560 x 2,432 0.93 .. 1.00; gated: 0.90 0.94 0.98 1.02 1.04, 0.98 1.02 1.07
-# 1.11 1.14, 0.94 0.98 1.02 1.04 1.09, 0.85 .. 0.97; 32 of 5,120 x 6,400, evenly routed, at 3, 5, 7: 1.04 1.09 1.18, gated 0.97 1.05 1.10.  So the
-# pairs times an expert's numbers decide; of many small experts the sides differ (64 of 2,560 x 1,408 0.96 0.98 1.00, gated 1.02 1.05 1.08, 128 of 2,560 x
-# 768 0.97 to 1.00 and 0.94 to 0.99, 256 of 2,560 x 512 0.95 to 0.98, gated 1.02 1.04 1.06): six pairs at most.
-MOE_FEW_PAIRS, MOE_FEW_PAIRS_MANY, MOE_FEW_PAIRS_ALWAYS = 12, 6, 3      # up to 32 experts; more of them; however large
+# A step takes the kernel for few rows up to so many pairs an expert.  It reads an expert's matrix once more from the caches for each 16 rows
+# more; an item of the walk takes its start and end whatever it multiplies, and few or small experts are few items.  Both products, few rows / walk, us: 1
+# expert of 4,096 x 3,072, 6 pairs 21 / 45; 3 of 4,096 x 768, 9 an expert 17 / 26; 8 of 4,096 x 96, 5 an expert 21 / 31; and the other way 32 of 5,120 x 1,024, 9 an
+# expert 155 / 129, 16 of 5,120 x 1,408 gated, 10 an expert 172 / 142.  So as long as one matrix of all the experts has few numbers up to 12 pairs, else
+# (and of more than 32 experts) up to 6.  2,162 steps of 1 to 256 experts that few rows might take: 0.8 % over the faster one in the mean and 1.09 of few
+# rows' time at worst; with the walk beyond four pairs whatever the size those without a gate took 17 % and up to 2.1 times.
+# Fewer where there is still more of the experts' matrices.  Whole steps of four layers, kernel for few rows over an earlier walk in tiles of 128, evenly routed,
+# at 3, 5, 7 pairs: 32 experts of 5,120 x 6,400 1.04 1.09 1.18, gated 0.97 1.05 1.10; three pairs always.
+MOE_FEW_PAIRS, MOE_FEW_PAIRS_MANY, MOE_FEW_PAIRS_ALWAYS = 12, 6, 3      # few numbers and up to 32 experts; more of either; however large
+MOE_FEW_NUMBERS = 120_000_000
 MOE_FEW_WORK, MOE_FEW_WORK_GATED = 2.4e9, 2.0e9         # pairs of the step times numbers of an expert's way back
-# From how many pairs on a gated step, or one without a gate, takes tiles of 256.  32 experts of 2,560 x 2,432, both products, us: gated with
-# tiles of 128 / 256: 2,048 pairs 314 / 316, 3,200 341 / 343, 4,300 428 / 377, 8,192 564 / 490; without a gate 6,400 340 / 362,
-# 7,600 362 / 362, 8,192 414 / 363, 10,000 409 / 412, 12,288 511 / 458: rounds of workgroups, which the number of tiles decides, and
-# the device alone knows that.
-MOE_MANY_PAIRS, MOE_MANY_PAIRS_UNGATED = 96, 240
-# Workgroups of the first product (half a tile an expert more than its pairs fill) below which tiles of 256 leave too much of the chip idle:
+# The walk takes tiles of 256 where those are workgroups enough (an expert of 125 rows, both products without a gate, tiles of 128 / 256: 234 / 228 us; 225 rows
+# 315 / 279, gated 408 / 350): so many workgroups of the first product, half a tile an expert more than its pairs fill.
 # 8 experts of 1,024 x 1,024 without a gate, 2,256 pairs, both products 78 us with tiles of 256 (about 50 workgroups), 67 with tiles of 128.
 MOE_MANY_GROUPS = 128
 
@@ -1146,47 +1144,20 @@ def moe_tile_rows(dtype: torch.dtype, *contractions: int, pairs: Optional[int] =
                   aligned: bool = True, identity: int = 0) -> int:
     """Rows of the tiles that the experts' products take: 128 on the matrix cores (bfloat16, every contraction a multiple of
     32), else 16.  With `pairs`, the (token, choice) pairs of the step: 64 for few of them an expert (without the share of the
-    `identity` experts, which have no matrices), 256 for many and for
-    columns enough of the first product (as many as the last contraction), unless rows or matrices do not begin at multiples of 16
-    bytes (`aligned`): those are taken in tiles of 128."""
+    `identity` experts, which have no matrices), else 256 for columns enough of the first product (as many as the last contraction), unless rows or
+    matrices do not begin at multiples of 16 bytes (`aligned`): those are taken in tiles of 128."""
     if dtype != torch.bfloat16 or any(k % 32 for k in contractions):
         return MOE_TILE_ROWS
-    if not aligned:
+    if pairs is None or not aligned:
         return MOE_MFMA_ROWS
-    most = (MOE_FEW_PAIRS if experts <= 32 else MOE_FEW_PAIRS_MANY) * experts
-    work = (MOE_FEW_WORK_GATED if gated else MOE_FEW_WORK) / (max(contractions) * min(contractions))
-    if pairs is not None and pairs * experts / (experts + identity) <= max(min(most, work), MOE_FEW_PAIRS_ALWAYS * experts):
+    numbers = max(contractions) * min(contractions)
+    most = (MOE_FEW_PAIRS if experts <= 32 and experts * numbers <= MOE_FEW_NUMBERS else MOE_FEW_PAIRS_MANY) * experts
+    work = (MOE_FEW_WORK_GATED if gated else MOE_FEW_WORK) / numbers
+    if pairs * experts / (experts + identity) <= max(min(most, work), MOE_FEW_PAIRS_ALWAYS * experts):
         return MOE_FEW_ROWS
-    many = pairs is not None and pairs > (MOE_MANY_PAIRS if gated else MOE_MANY_PAIRS_UNGATED) * experts \
-        and (pairs / MOE_MANY_ROWS + experts / 2) * -(-contractions[-1] // (128 if gated else 256)) >= MOE_MANY_GROUPS
-    # (a lane's offsets into the rows, as many as the tiles could hold, and into an expert's matrix are 32 bits wide)
-    if many and (-(-pairs // MOE_MANY_ROWS) + experts) * MOE_MANY_ROWS * max(contractions) < 1 << 31 and 2 * max(contractions) * min(contractions) < 1 << 31:
-        return MOE_MANY_ROWS
-    return MOE_MFMA_ROWS
-
-
-# Pairs an expert up to which a step stays with the kernel for few rows where the walk could take it, and how many numbers one matrix of all the experts has
-# where it stays as long as `moe_tile_rows` says: an item of the walk takes its start and end whatever it multiplies, and few or small experts are few items.
-# Both products, few rows / walk, us: 1 expert of 4,096 x 3,072, 6 pairs 21 / 45; 3 of 4,096 x 768, 9 an expert 17 / 26; 8 of 4,096 x 96, 5 an expert 21 / 31; and
-# the other way 32 of 5,120 x 1,024, 9 an expert 155 / 129, 16 of 5,120 x 1,408 gated, 10 an expert 172 / 142.  2,162 steps of 1 to 256 experts that
-# `moe_tile_rows` leaves to few rows: 0.8 % over the faster one in the mean and 1.09 of few rows' time at worst; with the walk beyond four pairs an
-# expert whatever the size those without a gate took 17 % and up to 2.1 times.
-MOE_STEP_FEW_PAIRS, MOE_STEP_FEW_NUMBERS = 6, 120_000_000
-
-
-def moe_step_tile_rows(dtype: torch.dtype, *contractions: int, pairs: int, experts: int = 1, gated: bool = False, aligned: bool = True,
-                       identity: int = 0) -> int:
-    """Rows of the tiles for the experts' products of a step: as `moe_tile_rows`, but the walk takes steps of fewer rows an expert, and always with
-    tiles of 256 where those are workgroups enough (an expert of 125 rows, both products without a gate, tiles of 128 / 256: 234 / 228 us; 225 rows 315 / 279,
-    gated 408 / 350)."""
-    rows = moe_tile_rows(dtype, *contractions, pairs=pairs, experts=experts, gated=gated, aligned=aligned, identity=identity)
-    if rows == MOE_TILE_ROWS or not aligned:
-        return rows
-    small = experts * max(contractions) * min(contractions) <= MOE_STEP_FEW_NUMBERS
-    if rows == MOE_FEW_ROWS and (small or pairs * experts / (experts + identity) <= MOE_STEP_FEW_PAIRS * experts):
-        return rows
     groups = (pairs / MOE_MANY_ROWS + experts / 2) * -(-contractions[-1] // (128 if gated else 256))
-    fits = (-(-pairs // MOE_MANY_ROWS) + experts) * MOE_MANY_ROWS * max(contractions) < 1 << 31 and 2 * max(contractions) * min(contractions) < 1 << 31
+    # (a lane's offsets into the rows, as many as the tiles could hold, and into an expert's matrix are 32 bits wide)
+    fits = (-(-pairs // MOE_MANY_ROWS) + experts) * MOE_MANY_ROWS * max(contractions) < 1 << 31 and 2 * numbers < 1 << 31
     return MOE_MANY_ROWS if groups >= MOE_MANY_GROUPS and fits else MOE_MFMA_ROWS
 
 

@@ -247,8 +247,8 @@ class RoutedMLP:
         place = torch.empty((pairs,), dtype=torch.int32, device=dev)
         # bfloat16 experts whose two contractions are multiples of 32 run on the matrix cores, in tiles that suit the step's pairs
         aligned = (x.dtype != self.w_up.dtype or x.data_ptr() % 16 == 0) and (self.w_up.data_ptr() | self.w_down.data_ptr()) % 16 == 0
-        tile_rows = ops.moe_step_tile_rows(self.w_up.dtype, s.hidden_size, s.expert_size, pairs=pairs, experts=s.experts,
-                                           gated=s.gate_name is not None, aligned=aligned, identity=s.identity)
+        tile_rows = ops.moe_tile_rows(self.w_up.dtype, s.hidden_size, s.expert_size, pairs=pairs, experts=s.experts,
+                                      gated=s.gate_name is not None, aligned=aligned, identity=s.identity)
         tiles = torch.empty((ops.moe_max_tiles(n, s.experts, s.top, tile_rows), 3), dtype=torch.int32, device=dev)
         # the weights in the order of the sorted rows, for experts that are given weighed inputs
         row_weight = rt.empty((pairs,), torch.float32) if s.weigh_input else None
