@@ -230,19 +230,14 @@ static double cut_cost(int M, int cols, int steps, int end, int shape, int parts
     return rounds * (kFixed[shape] + kStep[shape] * ((steps + parts - 1) / parts)) + (1.27 + (double)M * cols * 4.0 / 5e6) * (parts - 1);
 }
 
-// Tiles of 256 x 256 for the whole rounds of 256 of them, and the columns that are left, which would hold every compute unit for a
-// round that few of them have a tile in, in smaller ones (`rest` 0 .. 3).  Without whole rounds, or with nothing left, one cut of the large tile.
-static int whole_rounds_then_rest(int M, int cols, int end, int rest, Cut* cuts) {
-    cuts[0] = {256, 256, 1, 0, cols};
+// The output columns of the whole rounds of 256 tiles of 256 x 256 (0 where there are none, or nothing is left beside them).  What is left
+// would hold every compute unit for a round that few of them have a tile in, and goes in smaller tiles.
+static int columns_of_whole_rounds(int M, int cols, int end) {
     const int tn = pairs_columns(end) ? 128 : 256;
     const int tiles_m = (M + 255) / 256;
     const long long whole = ((long long)tiles_m * (cols / tn)) / 256 * 256;
     const int first_cols = (int)(whole / tiles_m) * tn;
-    if (first_cols <= 0 || first_cols >= cols) return 1;
-    cuts[0].col_end = first_cols;
-    static const int tiles[4][2] = {{128, 256}, {256, 128}, {128, 256}, {128, 128}};
-    cuts[1] = {tiles[rest & 3][0], tiles[rest & 3][1], 1, first_cols, cols};
-    return 2;
+    return first_cols < cols ? first_cols : 0;
 }
 
 // Up to two cuts, side by side in the output's columns.  The float32 end takes one cut, whose parts of K may be
@@ -265,11 +260,8 @@ static int plan(int M, int N, int K, int end, int max_parts, Cut* cuts) {
     }
     if (end != END_SLABS) {
         // whole rounds of the largest tile first, the rest of the columns in smaller tiles
-        const int tn = pairs_columns(end) ? 128 : 256;
-        const int tiles_m = (M + 255) / 256;
-        const long long whole = ((long long)tiles_m * (cols / tn)) / 256 * 256;      // tiles of whole rounds
-        const int first_cols = (int)(whole / tiles_m) * tn;
-        if (first_cols > 0 && first_cols < cols) {
+        const int first_cols = columns_of_whole_rounds(M, cols, end);
+        if (first_cols > 0) {
             for (int s = 2; s < N_SHAPES; ++s) {
                 if (kShapes[s][1] == 192) continue;
                 const double cost = cut_cost(M, first_cols, steps, end, 0, 1) + cut_cost(M, cols - first_cols, steps, end, s, 1);
@@ -283,6 +275,21 @@ static int plan(int M, int N, int K, int end, int max_parts, Cut* cuts) {
         }
     }
     return n_cuts;
+}
+
+// The cuts that a product is launched in: the planned ones, or those that `force` names (kipp_gemm_tiles).
+static int cuts_of(int M, int N, int K, int end, int max_parts, int force, Cut* cuts) {
+    if (!force) return plan(M, N, K, end, max_parts, cuts);
+    const int cols = pairs_columns(end) ? N / 2 : N, rest = force / 10000, code = force % 10000;
+    cuts[0] = {64 * (code / 100), 64 * (code / 10 % 10), code % 10, 0, cols};        // (tiles without a kernel are refused where they are launched)
+    if (code != 2421) return 1;
+    const int tile = rest == 0 ? 3 : rest == 1 ? 2 : rest == 3 ? 5 : -1;
+    cuts[0] = {256, 256, tile < 0 ? 0 : 1, 0, cols};
+    const int first_cols = end == END_SLABS ? 0 : columns_of_whole_rounds(M, cols, end);
+    if (first_cols <= 0 || tile < 0) return 1;
+    cuts[0].col_end = first_cols;
+    cuts[1] = {kShapes[tile][0], kShapes[tile][1], 1, first_cols, cols};
+    return 2;
 }
 
 template <int XF, int WF, int GM, int GN, int END>
@@ -327,15 +334,7 @@ static int launch_product(const void* X, const void* W, void* Y, int M, int N, i
     // a lane's offset into an operand is 32 bits wide
     if ((unsigned long long)M * K * 2 >= (1ull << 32) || (unsigned long long)N * K * 2 >= (1ull << 32)) return -6;
     Cut cuts[2];
-    int n_cuts = plan(M, N, K, end, max_parts, cuts);
-    if (force) {
-        const int cols = pairs_columns(end) ? N / 2 : N;
-        n_cuts = 1;
-        const int rest_code = force / 10000;         // + 10000 r: the tile of the columns that + 2000 leaves (below)
-        force %= 10000;
-        cuts[0] = {64 * ((force / 100) % 10), 32 * ((force / 10) % 10) * (force >= 1000 ? 4 : 2), force % 10, 0, cols};
-        if (force >= 2000 && end != END_SLABS) n_cuts = whole_rounds_then_rest(M, cols, end, rest_code, cuts);   // + 2000 (above)
-    }
+    const int n_cuts = cuts_of(M, N, K, end, max_parts, force, cuts);
     for (int c = 0; c < n_cuts; ++c) {
         const Cut& cut = cuts[c];
         if (cut.parts < 1 || cut.parts > K / BK || (end != END_SLABS && cut.parts != 1)) return -2;
@@ -360,8 +359,8 @@ int kipp_gemm_tiles_parts(int M, int N, int K, int end, int max_parts) {
 
 // Y: float32 [parts, M, N] with parts = kipp_gemm_tiles_parts(...) (end 0), bfloat16 [M, N / 2] = silu(gate) * up for
 // W = [gate; up] (end 1), bfloat16 [M, N] (end 2), bfloat16 [M, N] = relu(product)^2 (end 3).  K a multiple of 32.  `force`: 0, or 100 a + 10 b + parts for tiles of 64 a x 64 b
-// (+ 1000: of 64 a x 128 b; + 2000: 256 x 256 for whole rounds of tiles, the rest of the columns in smaller ones, 128 x 256 or, + 10000 r,
-// 256 x 128, 128 x 256, 128 x 128) to take that cut whatever the plan says (the runtime's timed choice, tests).
+// or 2421 (bfloat16 ends: 256 x 256 for whole rounds of tiles, the rest of the columns in 128 x 256; + 10000: the rest in 256 x 128,
+// + 30000: in 128 x 128; the slabs' end: 256 x 256) to take that cut whatever the plan says (the runtime's timed choice, tests).
 int kipp_gemm_tiles(const void* X, const void* W, void* Y, int M, int N, int K, int end, int max_parts, int force,
                     hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;

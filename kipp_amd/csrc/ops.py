@@ -2121,8 +2121,8 @@ def gemm_tiles(x: torch.Tensor, w: torch.Tensor, end: str = "slabs", max_parts: 
     "swiglu": w = [gate; up] of [2 I, K], the result is bfloat16 [M, I] = silu(x . gate^T) * (x . up^T);
     "glu": the same with `activation` silu or relu and a float32 `bias` [2 I] (or none) ahead of it;
     "bf16": bfloat16 [M, N]; "relu2": bfloat16 [M, N] = relu(x . w^T)^2.  `force` = 100 a + 10 b + parts: tiles of 64 a x 64 b
-    outputs (+ 1000: of 64 a x 128 b; + 2000, bfloat16 ends: 256 x 256 for the whole rounds of 256 tiles and smaller tiles for the columns
-    that are left, 128 x 256 or, + 10000 r, 256 x 128, 128 x 256 or 128 x 128 outputs) takes
+    outputs (2421, bfloat16 ends: 256 x 256 for the whole rounds of 256 tiles and smaller tiles for the columns
+    that are left, 128 x 256 or, + 10000, 256 x 128 or, + 30000, 128 x 128 outputs) takes
     that cut instead of the planned one (the runtime's timed choice, tests)."""
     _dev(x, w)
     m, k = x.shape

@@ -1006,13 +1006,13 @@ def test_gemm_rows_swiglu(m, inner, k):
     assert not ops.gemm_rows_swiglu_pays(64, 2 * 512, 2560)          # too few rows of W to go round without splitting K
 
 
-TILE_CUTS = [0, 441, 442, 444, 421, 422, 243, 221, 224, 431, 432, 232, 1421, 1422, 1424, 1221]      # 100 wm + 10 wn + parts (+ 1000: 8 waves; + 2000: whole rounds of those, the rest smaller; + 10000 r: the rest's tile); 0: what the launcher plans
+TILE_CUTS = [0, 441, 442, 443, 444, 421, 422, 424, 241, 243, 221, 224, 431, 432, 231, 232, 233]      # 100 a + 10 b + parts of K: tiles of 64 a x 64 b; 0: what the launcher plans
 
 
 @pytest.mark.parametrize("force", TILE_CUTS)
 @pytest.mark.parametrize("m,n,k", [(257, 300, 64), (300, 2560, 96), (513, 77, 2560), (1000, 640, 352), (64, 16, 32)])
 def test_gemm_tiles_float32_end(m, n, k, force):
-    """The product for prompt portions, every wave tile and split of K, at sizes that end inside tiles on both
+    """The product for prompt portions, every tile and splits of K, at sizes that end inside tiles on both
     sides (and one smaller than any tile): against float64, and exactly on small integers."""
     ops = _ops()
     if force % 10 > k // 32:
@@ -1030,13 +1030,13 @@ def test_gemm_tiles_float32_end(m, n, k, force):
     assert np.array_equal(out.cpu().numpy(), xi.float().numpy() @ wi.float().numpy().T)
 
 
-@pytest.mark.parametrize("force", [0, 441, 421, 241, 221, 1421, 1221, 2421, 32421])
+@pytest.mark.parametrize("force", [0, 441, 421, 241, 221, 2421, 12421, 32421])
 @pytest.mark.parametrize("m,inner,k", [(257, 150, 64), (600, 9728 // 8, 160), (300, 24, 2560), (2050, 1300, 96), (2050, 4804, 64)])
 def test_gemm_tiles_swiglu_and_bfloat16_ends(m, inner, k, force):
     """W = [gate; up]: silu(x . gate^T) * (x . up^T) rounded once, at the end (gate first: the other way round
     gives another result), also where the launcher cuts the columns into two kinds of tiles (as planned, or
-    forced with + 2000: whole rounds of 8-wave tiles and the rest of the columns in smaller ones, which the
-    last size has); and the plain bfloat16 end.  Widths that are no multiple of 8 take the store of single values."""
+    forced with 2421: whole rounds of 256 x 256 and the rest of the columns in smaller ones, which the
+    last size has); and the plain bfloat16 end.  Widths that are no multiple of 8 have rows that begin at no multiple of 16 bytes."""
     ops = _ops()
     rng = np.random.default_rng(m + inner + force)
     x = torch.tensor(rng.normal(size=(m, k)), dtype=torch.bfloat16)
@@ -1055,25 +1055,25 @@ def test_gemm_tiles_swiglu_and_bfloat16_ends(m, inner, k, force):
 
 
 def test_gemm_tiles_cuts_with_the_same_parts_give_the_same_bits():
-    """An output element is summed over K in the same order whatever the wave tile and the number of waves: every
+    """An output element is summed over K in the same order whatever the tile: every
     cut with the same parts of K gives the same bits (the runtime relies on it when it takes the fastest of them)."""
     ops = _ops()
     rng = np.random.default_rng(3)
     x = torch.tensor(rng.normal(size=(700, 2560)), dtype=torch.bfloat16).to(DEV)
     w = torch.tensor(rng.normal(size=(1300, 2560)) * 0.05, dtype=torch.bfloat16).to(DEV)
-    for parts, cuts in ((1, (441, 431, 421, 241, 221, 1421, 1221)), (2, (442, 432, 422, 222, 1422)), (4, (444, 424, 1424))):
+    for parts, cuts in ((1, (441, 431, 421, 241, 231, 221)), (2, (442, 432, 422, 242, 232, 222)), (3, (443, 433, 243, 233)), (4, (444, 424, 224))):
         base = ops.gemm_tiles(x, w, "slabs", max_parts=4, force=cuts[0])
         assert base.shape[0] == parts
         for cut in cuts[1:]:
             assert torch.equal(ops.gemm_tiles(x, w, "slabs", max_parts=4, force=cut), base), cut
     gated = ops.gemm_tiles(x, w, "swiglu", force=441)
-    for cut in (0, 421, 241, 221, 1421):
+    for cut in (0, 421, 241, 221):
         assert torch.equal(ops.gemm_tiles(x, w, "swiglu", force=cut), gated), cut
     # wide enough for whole rounds of tiles and a rest
     x = torch.tensor(rng.normal(size=(2050, 96)), dtype=torch.bfloat16).to(DEV)
     w = torch.tensor(rng.normal(size=(2 * 4800, 96)) * 0.3, dtype=torch.bfloat16).to(DEV)
     gated = ops.gemm_tiles(x, w, "swiglu", force=441)
-    for cut in (0, 1421, 2421, 12421, 22421, 32421):
+    for cut in (0, 421, 2421, 12421, 32421):
         assert torch.equal(ops.gemm_tiles(x, w, "swiglu", force=cut), gated), cut
 
 
