@@ -357,6 +357,22 @@ int kipp_gemm_tiles_parts(int M, int N, int K, int end, int max_parts) {
     return cuts[0].parts;
 }
 
+// Microseconds that the plan's prices give for a product cut as planned, or as `force` says (kipp_gemm_tiles); -1 for a cut that these
+// sizes do not take.
+double kipp_gemm_tiles_cost(int M, int N, int K, int end, int max_parts, int force) {
+    if (K <= 0 || (K % BK) || M <= 0 || N <= 0 || max_parts <= 0) return -1.0;
+    Cut cuts[2];
+    const int n_cuts = cuts_of(M, N, K, end, max_parts, force, cuts);
+    double cost = 0.0;
+    for (int c = 0; c < n_cuts; ++c) {
+        int s = 0;
+        while (s < N_SHAPES && (kShapes[s][0] != cuts[c].tm || kShapes[s][1] != cuts[c].tn)) ++s;
+        if (s == N_SHAPES || cuts[c].parts < 1 || cuts[c].parts > K / BK || (end != END_SLABS && (cuts[c].parts != 1 || kShapes[s][1] == 192))) return -1.0;
+        cost += cut_cost(M, cuts[c].col_end - cuts[c].col_begin, K / BK, end, s, cuts[c].parts);
+    }
+    return cost;
+}
+
 // Y: float32 [parts, M, N] with parts = kipp_gemm_tiles_parts(...) (end 0), bfloat16 [M, N / 2] = silu(gate) * up for
 // W = [gate; up] (end 1), bfloat16 [M, N] (end 2), bfloat16 [M, N] = relu(product)^2 (end 3).  K a multiple of 32.  `force`: 0, or 100 a + 10 b + parts for tiles of 64 a x 64 b
 // or 2421 (bfloat16 ends: 256 x 256 for whole rounds of tiles, the rest of the columns in 128 x 256; + 10000: the rest in 256 x 128,

@@ -2114,6 +2114,12 @@ def gemm_tiles_parts(m: int, n: int, k: int, end: str = "slabs", max_parts: int 
     return int(build.library("gemm_tiles").kipp_gemm_tiles_parts(int(m), int(n), int(k), TILES_END[end], int(max_parts)))
 
 
+def gemm_tiles_cost(m: int, n: int, k: int, end: str = "slabs", max_parts: int = 1, force: int = 0) -> float:
+    """Microseconds that the launcher's prices give for a product cut as planned, or as `force` says (`gemm_tiles`); -1 for a cut that these sizes
+    do not take."""
+    return _fn("gemm_tiles", "kipp_gemm_tiles_cost", [_c_int] * 6, restype=ctypes.c_double)(int(m), int(n), int(k), TILES_END[end], int(max_parts), int(force))
+
+
 def gemm_tiles(x: torch.Tensor, w: torch.Tensor, end: str = "slabs", max_parts: int = 1, force: int = 0, activation: str = "silu",
                bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """x [M, K] . w [N, K]^T on the matrix cores for many rows, bfloat16 operands, float32 accumulation.

@@ -276,48 +276,31 @@ class Runtime:
         """Rows of a prompt product, in classes of a factor of two (193-256, 257-512, 513-1024, ...): timed once a class."""
         return 1 << (max(m, 1) - 1).bit_length()
 
-    @staticmethod
-    def _rounds_of(name, m: int, cols: int, pairs: bool) -> float:
-        """What a way to compute a product costs at m rows, in units of its own: the rounds of its tiles over the 256 compute units (of
-        the library's: 256 rows at a time; of the planned way: of what the plan would take).  A class is timed at the first rows that come; the times
-        of our cuts at others are taken in proportion to this.  (1,193 rows against [gate; up] of 2 x 12,288 x 4,096: whole rounds of 256 x 256 and the rest in
-        128 x 64 were level with one cut at the class's first 2,048 rows, three rounds and no rest; there 281 us against 231.)"""
-        if name == "plan":
-            if pairs and m >= 512:
-                return Runtime._rounds_of(2421, m, cols, pairs)
-            return min(Runtime._rounds_of(cut, m, cols, pairs) / (cut % 10) for cut in Runtime.TILE_CUTS_SLABS if cut < 1000 and not (pairs and cut % 10 > 1))
+    def _price(self, name, m: int, n: int, k: int, end: str, most: int = 1) -> float:
+        """What a way to compute a product costs at m rows, in units of its own: by the prices that the plan goes by, which hold the rounds of its
+        tiles over the 256 compute units (the library's: 256 rows at a time).  A class is timed at the first rows that come; the times
+        of our cuts at others are taken in proportion to this."""
         if name == "library":
             return float(-(-m // 256))
-
-        def rounds(wm, wn, across, parts, width):
-            tiles = -(-m // (64 * wm)) * -(-width // ((16 if pairs else 32) * wn * across))
-            return -(-tiles * parts // 256) * (0.1 + 0.022 * wm * wn * across)       # times a tile's, from the measured steps
-        rest, code = divmod(name, 10000)
-        if code < 2000:
-            return rounds(code // 100 % 10, code // 10 % 10, 4 if code >= 1000 else 2, code % 10, cols)
-        wide, rows = (16 if pairs else 32) * 8, -(-m // 256)
-        first = rows * (cols // wide) // 256 * 256 // rows * wide
-        if not 0 < first < cols:
-            return rounds(4, 2, 4, 1, cols)
-        return rounds(4, 2, 4, 1, first) + rounds(*((2, 2, 4), (4, 2, 2), (2, 4, 2), (2, 2, 2))[rest], 1, cols - first)
+        return self.ops.gemm_tiles_cost(m, n, k, end, most, 0 if name == "plan" else name)
 
     @staticmethod
-    def _at_rows(choice, took: dict, rows: int, m: int, cols: int, pairs: bool):
-        """What a class timed at `rows` rows (`took`: milliseconds) takes at m: one of our cuts by its time in proportion to the rounds of its
-        tiles, where that promises 5 % more than the class's choice.  The library's times do not go by rounds, nor do those of the plan that
-        may split K: chosen, they stay, and they are chosen by times alone.  (Four products of each of the 4B, 8B and 32B shapes at 25
-        numbers of rows up to 2,048, a class first timed at every other of its numbers: 2.1 % over the fastest way in the mean, 3.5 with the
-        class's choice at all its rows, 4.6 with every way in proportion, where a product took up to 1.7 times the class's choice.)"""
-        if choice in took and (choice == "library" or (choice == "plan" and not pairs)):
+    def _at_rows(choice, took: dict, rows: int, m: int, price, slabs: bool):
+        """What a class timed at `rows` rows (`took`: milliseconds) takes at m: one of our cuts by its time in proportion to its `price` (of a way's
+        name and rows), where that promises 5 % more than the class's choice.  The library's times do not go by rounds, nor do those of the plan that
+        may split K (`slabs`): chosen, they stay, and they are chosen by times alone.  (Four products of each of the 4B, 8B and 32B shapes at 25
+        numbers of rows from 200 to 2,048, a class first timed at every one of its numbers: with own products 0.4 % over the fastest way in the mean and
+        13 % at most, 5.1 and 55 with the class's choice at all its rows; with the library's among them 1.1 and 17, 6.7 and 55.)"""
+        if choice in took and (choice == "library" or (choice == "plan" and slabs)):
             return choice
-        names = [name for name in took if name != "library" and (pairs or name != "plan")] or list(took)
-        there = {name: took[name] * Runtime._rounds_of(name, m, cols, pairs) / Runtime._rounds_of(name, rows, cols, pairs) for name in names}
+        names = [name for name in took if name != "library" and not (slabs and name == "plan")] or list(took)
+        there = {name: took[name] * price(name, m) / price(name, rows) for name in names}
         best = min(names, key=there.get)
         return best if choice not in there or there[best] < 0.95 * there[choice] else choice
 
     # Cuts of our kernel that are timed beside the planned one: 100 x (tile rows / 64) + 10 x (tile
-    # columns / 64) + parts of K (+ 2000: tiles of 256 x 256 for
-    # the whole rounds of 256 tiles and smaller tiles for the columns that are left, 128 x 256 or, + 10000, 256 x 128, + 30000, 128 x 128).  The
+    # columns / 64) + parts of K; 2421: tiles of 256 x 256 for
+    # the whole rounds of 256 tiles and smaller tiles for the columns that are left, 128 x 256 or, + 10000, 256 x 128, + 30000, 128 x 128.  The
     # plan's cost model is linear; the GPU under its power limit is not (a round that leaves compute units idle
     # clocks the others higher), so the plan is not always the fastest.  An output element is summed over K in
     # the same order whatever the tile, so cuts with the same parts of K give the same bits.
@@ -325,9 +308,9 @@ class Runtime:
     TILE_CUTS_SLABS = (441, 442, 443, 444, 431, 432, 433, 421, 422, 241, 242, 231, 232, 221, 222)
     TILE_CUTS_BF16 = (441, 421, 241, 2421, 12421, 32421)
 
-    def _fastest(self, key, ways: dict, same_bits, m: int, cols: int, pairs: bool = False, extra_ms=None):
-        """Which of several ways to compute one product of `m` rows and `cols` output columns is taken for the shape `key`: timed once,
-        on the operands at hand (three runs each after a first one), and for other rows of the class by those times (`_at_rows`).  `ways`: name -> callable, "library"
+    def _fastest(self, key, ways: dict, same_bits, m: int, price, slabs: bool = False, extra_ms=None):
+        """Which of several ways to compute one product of `m` rows is taken for the shape `key`: timed once,
+        on the operands at hand (three runs each after a first one), and for other rows of the class by those times and `price` (`_at_rows`).  `ways`: name -> callable, "library"
         and "plan" among them; `same_bits`: the names whose results are those of "plan" bit for bit;
         `extra_ms`: name -> milliseconds that a way costs its consumer beyond its own kernel (the slabs of a split
         product are read by the kernel that adds them).
@@ -346,7 +329,7 @@ class Runtime:
                 return by_rows[m]
             # (what gives the plan's bits at the rows it was timed at need not at others, where the plan may take other parts of K)
             names = [name for name in took if self.own_prompt_products == "auto" or name in same_bits]
-            by_rows[m] = self._at_rows(choice, {name: took[name] for name in names}, rows, m, cols, pairs) if names else choice
+            by_rows[m] = self._at_rows(choice, {name: took[name] for name in names}, rows, m, price, slabs) if names else choice
             return by_rows[m]       # (at most as many entries as the class has numbers of rows)
         took = {}
         if self.own_prompt_products is False:
@@ -418,7 +401,7 @@ class Runtime:
             ways = {"library": library, "plan": ours}
             ways.update({cut: (lambda cut=cut: ours(cut)) for cut in self.TILE_CUTS_BF16})
             choice = self._fastest(("gated" if plain else "glu", self._rows_class(m), rows.shape[0], k), ways, ("plan",) + self.TILE_CUTS_BF16,
-                                   m, rows.shape[0] // 2, pairs=True)
+                                   m, lambda name, at: self._price(name, at, rows.shape[0], k, "swiglu"))
             if choice != "library":
                 self.tile_products += 1
                 return ours(0 if choice == "plan" else choice)
@@ -439,7 +422,8 @@ class Runtime:
         if self.ops.gemm_tiles_ok(m, k, rows.shape[0]):
             ways = {"library": library, "plan": ours}
             ways.update({cut: (lambda cut=cut: ours(cut)) for cut in self.TILE_CUTS_BF16})
-            choice = self._fastest(("relu2", self._rows_class(m), rows.shape[0], k), ways, ("plan",) + self.TILE_CUTS_BF16, m, rows.shape[0])
+            choice = self._fastest(("relu2", self._rows_class(m), rows.shape[0], k), ways, ("plan",) + self.TILE_CUTS_BF16, m,
+                                   lambda name, at: self._price(name, at, rows.shape[0], k, "relu2"))
             if choice != "library":
                 self.tile_products += 1
                 return ours(0 if choice == "plan" else choice)
@@ -505,7 +489,7 @@ class Runtime:
             extra = {name: ((planned if name == "plan" else name % 10) - 1) * slab_ms for name in ways if name != "library"}
             # with our own products alone, rows that the plan cuts into other parts of K have other ways: they are timed by themselves
             key = ("linear", self._rows_class(m), n, x.shape[1], most) + ((planned,) if self.own_prompt_products is True else ())
-            choice = self._fastest(key, ways, same, m, n, extra_ms=extra)
+            choice = self._fastest(key, ways, same, m, lambda name, at: self._price(name, at, n, x.shape[1], "slabs", most), slabs=True, extra_ms=extra)
             if choice != "library":
                 self.tile_products += 1
                 return ours(0 if choice == "plan" else choice)

@@ -6,40 +6,60 @@ from types import SimpleNamespace
 import pytest
 import torch
 
+from kipp_amd.csrc import ops
 from kipp_amd.runtime import Runtime
 
 
+K = 2560
+
+
+def _price(end, n):
+    return lambda name, m: Runtime._price(SimpleNamespace(ops=ops), name, m, n, K, end, 4 if end == "slabs" else 1)
+
+
 @pytest.mark.parametrize("m", [193, 256, 257, 1193, 2048])
-@pytest.mark.parametrize("cols,pairs", [(12288, True), (4096, False), (100, False)])
-def test_rounds(m, cols, pairs):
-    half = 2 if pairs else 1
-    big = 0.1 + 0.022 * 32
-    tiles = math.ceil(m / 256) * math.ceil(cols * half / 256)
-    assert Runtime._rounds_of(441, m, cols, pairs) == pytest.approx(math.ceil(tiles / 256) * big)
-    assert Runtime._rounds_of(1423, m, cols, pairs) == pytest.approx(math.ceil(tiles * 3 / 256) * big)
-    assert Runtime._rounds_of("library", m, cols, pairs) == math.ceil(m / 256)
-    # whole rounds and a rest: as many columns in whole rounds as fit; one cut where there is none, or nothing left
-    if tiles <= 256 or tiles % 256 == 0:
-        assert Runtime._rounds_of(32421, m, cols, pairs) == pytest.approx(Runtime._rounds_of(1421, m, cols, pairs))
-    else:
-        rows = math.ceil(m / 256)
-        first = tiles // 256 * 256 // rows
-        rest = math.ceil(m / 128) * math.ceil((cols * half - first * 256) / 128)
-        assert Runtime._rounds_of(32421, m, cols, pairs) == pytest.approx(math.ceil(rows * first / 256) * big + math.ceil(rest / 256) * (0.1 + 0.022 * 8))
+@pytest.mark.parametrize("cols,end", [(12288, "swiglu"), (4096, "slabs"), (4096, "relu2"), (100, "slabs")])
+def test_prices(m, cols, end):
+    pairs = end == "swiglu"
+    n = 2 * cols if pairs else cols
+    price, one = _price(end, n), _price(end, n if n <= 256 else 256)
+    tiles = math.ceil(m / 256) * math.ceil(n / 256)
+    assert price(441, m) == pytest.approx(math.ceil(tiles / 256) * one(441, 256))
+    assert price("library", m) == math.ceil(m / 256)
+    if end == "slabs":      # three tiles a place, each of a third of K (up to one step), and the slabs that are read once more
+        third = ops.gemm_tiles_cost(256, min(n, 256), 32 * math.ceil(K / 32 / 3), end, 1, 441)
+        assert price(443, m) == pytest.approx(math.ceil(tiles * 3 / 256) * third + 2 * (1.27 + m * n * 4 / 5e6))
+    # the plan's price is that of the cheapest cut that the end takes (for slabs other parts of K are planned too)
+    ways = {cut: price(cut, m) for cut in (Runtime.TILE_CUTS_SLABS if end == "slabs" else (221, *Runtime.TILE_CUTS_BF16))}
+    assert 0 < price("plan", m) <= min(ways.values()) + 1e-9
+    if end != "slabs":
+        assert price("plan", m) == pytest.approx(min(ways.values()))
+        assert price(431, m) == price(231, m) == price(442, m) == -1.0
+        # whole rounds and a rest: as many columns in whole rounds as fit; one cut where there is none, or nothing left
+        if tiles <= 256 or tiles % 256 == 0:
+            assert price(32421, m) == price(441, m)
+        else:
+            rows = math.ceil(m / 256)
+            first = tiles // 256 * 256 // rows
+            rest = math.ceil(m / 128) * math.ceil((n - first * 256) / 128)
+            small = ops.gemm_tiles_cost(128, 128, K, end, 1, 221)
+            assert price(32421, m) == pytest.approx(math.ceil(rows * first / 256) * one(441, 256) + math.ceil(rest / 256) * small)
+    assert price(1421, m) == price(22421, m) == -1.0        # no cut's name
 
 
 def test_other_rows_take_the_times_in_proportion(monkeypatch):
     rt = Runtime.__new__(Runtime)
     rt.own_prompt_products, rt.for_a_graph, rt.prompt_product_choices = "auto", False, {}
-    took = {"library": 0.4, "plan": 0.36, 1421: 0.351, 32421: 0.350}
+    took = {"library": 0.4, "plan": 0.36, 441: 0.351, 32421: 0.350}
     monkeypatch.setattr(Runtime, "_choices_of_process", {("auto", ("gated",)): (32421, 2048, took, {2048: 32421})})
 
     def never():
         raise AssertionError("nothing is run once a class has been timed")
     ways = {name: never for name in took}
+    price = _price("swiglu", 2 * 12288)
     for _ in range(2):
-        assert rt._fastest(("gated",), ways, (), 2048, 12288, pairs=True) == 32421       # level there: what was measured
-        assert rt._fastest(("gated",), ways, (), 1193, 12288, pairs=True) == 1421        # two rounds of three, against one and four small ones
+        assert rt._fastest(("gated",), ways, (), 2048, price) == 32421       # level there: what was measured
+        assert rt._fastest(("gated",), ways, (), 1193, price) == 441        # two rounds of three, against one and three small ones
     assert rt.prompt_product_choices == {("gated",): 32421}
 
 
@@ -47,10 +67,10 @@ def test_own_products_keep_the_plans_bits_at_every_number_of_rows(monkeypatch):
     """A cut that gives the plan's bits at the rows a class was timed at is not taken at rows where the plan takes other parts of K."""
     rt = Runtime.__new__(Runtime)
     rt.own_prompt_products, rt.for_a_graph, rt.prompt_product_choices = True, False, {}
-    took = {"plan": 0.4, 443: 0.1, 1423: 0.2}
+    took = {"plan": 0.4, 443: 0.1, 233: 0.2}
     monkeypatch.setattr(Runtime, "_choices_of_process", {(True, ("linear",)): (443, 2048, took, {2048: 443})})
-    assert rt._fastest(("linear",), {}, ("plan", 442, 1422), 1100, 4096) == "plan"
-    assert rt._fastest(("linear",), {}, ("plan", 443, 1423), 1101, 4096) == 443
+    assert rt._fastest(("linear",), {}, ("plan", 442, 222), 1100, _price("slabs", 4096), slabs=True) == "plan"
+    assert rt._fastest(("linear",), {}, ("plan", 443, 233), 1101, _price("slabs", 4096), slabs=True) == 443
 
 
 @pytest.mark.parametrize("own", [True, "auto"])
@@ -64,7 +84,7 @@ def test_own_products_are_timed_for_every_number_of_parts(monkeypatch, own):
     asked = []
     rt.ops = SimpleNamespace(gemm_rows_ok=lambda m, k: False, gemm_tiles_ok=lambda m, k, n: True, gemm_tiles_parts=lambda m, *a: parts[m],
                              gemm_tiles=lambda x, w, **k: torch.zeros(1, 1, 1))
-    monkeypatch.setattr(Runtime, "_fastest", lambda self, key, ways, same, m, cols, **k: asked.append((key, same)) or "plan")
+    monkeypatch.setattr(Runtime, "_fastest", lambda self, key, ways, same, m, price, **k: asked.append((key, same)) or "plan")
     w = torch.zeros((64, 32), dtype=torch.bfloat16)
     for m in parts:
         rt.linear(torch.zeros((m, 32), dtype=torch.bfloat16), w, slabs=True)
@@ -77,11 +97,16 @@ def test_own_products_are_timed_for_every_number_of_parts(monkeypatch, own):
 def test_ways_whose_times_do_not_go_by_rounds_keep_their_rows():
     """[2,560 x 9,728] as measured at 2,048 rows, the library's the fastest: so it is at 1,536 (157 us; the plan 265).  One of our cuts is
     left for another where that promises more than 5 %."""
-    took = {"library": 0.186, "plan": 0.205, 441: 0.363, 442: 0.233, 1421: 0.353, 1423: 0.209}
+    took = {"library": 0.186, "plan": 0.205, 441: 0.363, 442: 0.233, 431: 0.353, 443: 0.209}
+    price = _price("slabs", 2560)
     for m in (1100, 1536, 1900):
-        assert Runtime._at_rows("library", took, 2048, m, 2560, False) == "library"
-        assert Runtime._at_rows("plan", took, 2048, m, 2560, False) == "plan"
+        assert Runtime._at_rows("library", took, 2048, m, price, True) == "library"
+        assert Runtime._at_rows("plan", took, 2048, m, price, True) == "plan"
     ours = {"library": 0.4, 442: 0.1, 444: 0.104}       # tiles in half a round and parts in one: 160 and 320 at 2,048 rows
-    assert Runtime._at_rows(442, ours, 2048, 2047, 2560, False) == 442
-    assert Runtime._at_rows(442, ours, 2048, 1500, 2560, False) == 444              # 240 in one round where 320 were two
-    assert Runtime._at_rows(441, {"plan": 0.4}, 2048, 1500, 2560, False) == "plan"       # nothing else of the same bits
+    assert Runtime._at_rows(442, ours, 2048, 2047, price, True) == 442
+    assert Runtime._at_rows(442, ours, 2048, 1500, price, True) == 444              # 240 in one round where 320 were two
+    assert Runtime._at_rows(441, {"plan": 0.4}, 2048, 1500, price, True) == "plan"       # nothing else of the same bits
+    # an end that cannot split K: the plan goes by rounds as its cuts do
+    price = _price("relu2", 12288)
+    assert price("plan", 1400) < 0.9 * price("plan", 2048) and price(421, 1400) == price(421, 2048)
+    assert Runtime._at_rows(421, {"plan": 0.3, 421: 0.3}, 2048, 1400, price, False) == "plan"
