@@ -9,14 +9,17 @@
 //   whole lines   a step's 128 bytes of a row are one memory line.  Out of L2 a compute unit draws 64-byte halves at three quarters of the rate of whole
 //                 lines (15.3 against 20.2 TB/s over all of them), and steps of 32 columns met every line twice;
 //   16 x 16       with two waves a SIMD the 32 x 32 x 16 instruction is as fast until the chip meets its power limit, which prompt
-//                 products do: on normal operands a kernel that only multiplies sustains 1.71 PFLOP/s with it and 2.0 with 16 x 16 x 32,
-//                 half of whose accumulator traffic it has (same sums in the same order: the same bits);
+//                 products do: on normal operands a kernel that only multiplies sustains 1.82 PFLOP/s with it and 2.03 with 16 x 16 x 32
+//                 (`python -m kipp_amd.workloads mfma`), half of whose accumulator traffic it has (same sums in the same order: the same bits);
 //   two a SIMD    a wave that issues a DMA instruction or a read cannot issue its next product; the other one does.  With four waves of
-//                 128 x 128, one a SIMD, a step takes 3,840 cycles where its products take 2,048, with eight 2,220;
+//                 128 x 128, one a SIMD, a step takes 3,840 cycles where its products take 2,048, with eight 2,220 (builds that read the shader
+//                 clock around the walk, which are not in the tree);
 //   64 x 128      outputs a wave, of the cuts of 256 x 256 into eight the one that a few per cent are won by (78 us of 128 x 64's 79 at
 //                 2,048 x 2,560 x 9,728).
-// Inside the walk the matrix cores are busy 92 cycles of 100, at 1.75 to 1.9 GHz under the power limit; what a product loses beside is the
-// start and the end of its tiles (2 us until the first step is there, 4 for the stores) and its last round.  2,048 rows of the 4B
+// What bounds it: by that count the matrix cores are busy 92 cycles of 100 inside the walk, at 1.75 to 1.9 GHz under the power limit, but
+// over whole launches of a prefill 47 to 54.  A tile's start and end are 13 us by the fit over all cuts (kFixed), about a quarter of such a
+// product's time (K of 2,560: 40 steps of 1.2 us a round): a compute unit holds one workgroup of the large tile, and nothing
+// runs beside its first data and its stores.  The rest is the last round, which few tiles fill.  2,048 rows of the 4B
 // shape, us, steps of 32 columns (32 x 32 x 16, best cut) / now: QKV 65 / 55, output 49 / 43, gate-up with its end 198 / 163, down 96 / 82;
 // 49 sizes from 256 to 1,800 rows: 1.19 in the mean.
 //

@@ -2194,18 +2194,18 @@ def stream_read(buffer: torch.Tensor, workgroups: int, depth: int = 8) -> int:
     return int(got)
 
 
-def mfma_rate(data: torch.Tensor, workgroups: int, accumulators: int, iters: int) -> int:
-    """Launches the probe that only multiplies (32x32x16 bfloat16 products from registers, `accumulators` = 8 or 16
+def mfma_rate(data: torch.Tensor, workgroups: int, accumulators: int, iters: int, side: int = 32) -> int:
+    """Launches the probe that only multiplies (bfloat16 products from registers, 32x32x16 or, `side` 16, 16x16x32; `accumulators` = 8 or 16
     independent sums a wave, `workgroups` of 4 waves); `data`: 16 KiB whose bits are the operands.  Returns the
     floating-point operations launched."""
     _dev(data)
-    _need(data.is_contiguous() and data.numel() * data.element_size() == 16384 and accumulators in (8, 16),
-          "mfma_rate: 16 KiB of operand bits, 8 or 16 accumulators")
+    _need(data.is_contiguous() and data.numel() * data.element_size() == 16384 and accumulators in (8, 16) and side in (16, 32),
+          "mfma_rate: 16 KiB of operand bits, 8 or 16 accumulators, products of 16 or 32")
     fn = build.library("probe").kipp_probe_mfma_rate
     fn.restype = ctypes.c_longlong
-    fn.argtypes = [_c_ptr, _c_int, _c_int, _c_int, _c_ptr, _c_ptr]
+    fn.argtypes = [_c_ptr, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_ptr]
     sink = torch.zeros(1, dtype=torch.int32, device=data.device)
-    got = fn(_ptr(data), int(workgroups), int(accumulators), int(iters), _ptr(sink), _stream())
+    got = fn(_ptr(data), int(workgroups), int(side), int(accumulators), int(iters), _ptr(sink), _stream())
     _need(got > 0, "mfma_rate: refused")
     return int(got)
 

@@ -157,30 +157,33 @@ def hbm_read(gib: float) -> dict:
 
 def mfma_rate() -> dict:
     """What the matrix cores sustain on operands that stay in registers: by the operands' bits (zeros, values
-    of a normal distribution), the compute units at work, waves a SIMD and the kernel's length."""
+    of a normal distribution), the instruction, the compute units at work, waves a SIMD and the kernel's length.  Both instructions are
+    timed in turn: a chip at its power limit clocks by what ran before."""
     import torch
     from .csrc import ops
     cus = torch.cuda.get_device_properties(0).multi_processor_count
     gen = torch.Generator().manual_seed(0)
     operands = {"zeros": torch.zeros(8192, dtype=torch.bfloat16),
                 "normal": torch.randn(8192, generator=gen).to(torch.bfloat16)}
+    sides = {32: "32x32x16", 16: "16x16x32"}
     table = []
     for name, host in operands.items():
         data = host.to("cuda:0")
         for groups, acc, what in ((cus, 16, "1 wave a SIMD"), (2 * cus, 8, "2 waves a SIMD"), (80, 16, "80 compute units")):
             for iters in (400, 4000, 40000):
-                start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-                ops.mfma_rate(data, groups, acc, iters)
-                best = 0.0
-                for _ in range(3):
-                    start.record()
-                    flops = ops.mfma_rate(data, groups, acc, iters)
-                    end.record()
-                    torch.cuda.synchronize()
-                    ms = start.elapsed_time(end)
-                    best = max(best, flops / (ms * 1e-3) / 1e15)
-                table.append({"operands": name, "grid": what, "ms": round(ms, 3), "PFLOP_s": round(best, 3)})
-                log(f"{name:6s} {what:17s} kernel of {ms:8.3f} ms: {best:5.3f} PFLOP/s")
+                best = dict.fromkeys(sides, 0.0)
+                for run in range(4):
+                    for side in sides:
+                        start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+                        start.record()
+                        flops = ops.mfma_rate(data, groups, acc, iters * 32 // side, side)       # as many operations either way
+                        end.record()
+                        torch.cuda.synchronize()
+                        if run:
+                            best[side] = max(best[side], flops / (start.elapsed_time(end) * 1e-3) / 1e15)
+                for side, instruction in sides.items():
+                    table.append({"operands": name, "instruction": instruction, "grid": what, "ms": round(flops / best[side] / 1e12, 3), "PFLOP_s": round(best[side], 3)})
+                    log(f"{name:6s} {instruction} {what:17s} kernel of {table[-1]['ms']:8.3f} ms: {best[side]:5.3f} PFLOP/s")
     return {"workload": "mfma rate", "compute_units": cus, "all": table}
 
 
