@@ -1808,7 +1808,10 @@ SKINNY_MAX_ROWS = 64     # rows the few-rows kernel takes
 SKINNY_BEST_ROWS = 12    # ... and rows up to which it is the faster one (each wave reads its rows of x itself; beyond, x staged in LDS wins:
                          # with rows in steps-major order a step at 12 rows takes 3.02 ms this way against 3.22, at 16 rows 3.58 against 3.56)
 ROWS_MAX_ROWS = 256      # rows of the kernel that stages x through LDS
-ROWS_BEST_ROWS = 192     # beyond these the product built for hundreds of rows is faster where it takes the shape (measured)
+# Beyond these the product built for hundreds of rows is the faster one where it takes the shape.  Four products of a layer, us, this kernel / that one, at
+# 128, 144 and 192 rows: the 4B shape 90 / 104, 123 / 99, 127 / 107, 8B 137 / 139, 184 / 145, 192 / 155, 32B 257 / 273, 362 / 281, 378 / 304 (from 129 rows on
+# this one stages 64 columns of x at a time).  One of few columns whose K may be split the other loses by up to 2 us to 192 rows (256 x 2,560 7.1 / 8.5).
+ROWS_BEST_ROWS = 128
 
 
 def gemm_rows_ok(m: int, k: int) -> bool:

@@ -489,7 +489,7 @@ static int hip_embed(kipp_runtime *rt, const kipp_weight *table, const int32_t *
 }
 
 #define FEW_ROWS 12           /* up to these the kernel in which every wave reads its rows of x itself is the faster one, and has the fused ends */
-#define STAGED_ROWS 192       /* up to these the kernel that stages x through LDS; beyond, the one built for hundreds of rows where it takes the shape */
+#define STAGED_ROWS 128       /* up to these the kernel that stages x through LDS; beyond, the one built for hundreds of rows where it takes the shape */
 #define FUSE_NORM_X_BYTES 40e6 /* most bytes of x the workgroups of an unsplit product may read together for the fused norm to pay */
 
 /* The few-rows kernel takes this product (and with it the ends that spare a decode step its norm kernels). */
@@ -556,7 +556,7 @@ static int hip_residual_add(kipp_runtime *rt, float *x, kipp_delta *delta, uint3
 }
 
 /* x . w^T.  bfloat16 x bfloat16: up to 12 rows the kernel in which every wave streams its rows of w against all of x (it also
- * applies a scale that the rows still lack), up to 192 rows the one that stages x through LDS, both from the streaming layout
+ * applies a scale that the rows still lack), up to 128 rows the one that stages x through LDS, both from the streaming layout
  * where the weight has it; beyond those the tiled matrix-core kernel (K a multiple of 32) or the staged one over runs of 256
  * rows; a shape none of them takes (K no multiple of 8, or below 32) and every float32 weight go through the plain float32
  * product. */
@@ -628,7 +628,7 @@ static int hip_linear(kipp_runtime *rt, const kipp_rows *rows_in, const kipp_wei
 }
 
 /* Few rows against [gate; up]: both products and the activation in one kernel (and the norm's scale, if it was left to us).
- * Up to 192 rows: the product streamed from the paired tiles, whose columns come out gate tile by gate tile, then the activation
+ * Up to 128 rows: the product streamed from the paired tiles, whose columns come out gate tile by gate tile, then the activation
  * over those pairs.  Beyond: the matrix-core kernel with the activation as its end. */
 static int hip_gated(kipp_runtime *rt, const kipp_rows *x, const kipp_weight *w, const kipp_weight *reader, kipp_rows *act, uint32_t m, bool *done,
                      kipp_error *error) {

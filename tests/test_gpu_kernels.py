@@ -1,5 +1,6 @@
 """Each HIP kernel alone against a plain float64 reference, at sizes other
 than the engine tests use (ragged widths, odd head counts, several head sizes)."""
+import itertools
 import math
 
 import numpy as np
@@ -1120,6 +1121,25 @@ def _microseconds(run, calls=10):
         end.record()
     torch.cuda.synchronize()
     return 1000 * min(a.elapsed_time(b) for a, b in marks) / calls
+
+
+@pytest.mark.parametrize("n,k", [(10240, 5120), (5120, 25600)])
+@pytest.mark.parametrize("m", [128, 129, 192])
+def test_the_product_taken_for_dozens_of_rows_is_not_much_slower_than_the_other(m, n, k):
+    """On both sides of the line between the kernel that stages x whole and the one with tiles of x too (1.3 times as long where it lay at 192),
+    over weights that no cache holds."""
+    ops = _ops()
+    x = torch.randn((m, k), device=DEV).bfloat16()
+    weights = [(torch.randn((n, k), device=DEV) * 0.02).bfloat16() for _ in range(5)]
+    pairs = itertools.cycle([(w, ops.tile_weight(w)) for w in weights])
+
+    def staged_product():
+        w, tiles = next(pairs)
+        ops.gemm_rows(x, w, max_parts=12, tiles=tiles)
+    staged = _microseconds(staged_product)
+    tiled = _microseconds(lambda: ops.gemm_tiles(x, next(pairs)[0], max_parts=4))
+    taken, other = (staged, tiled) if m <= ops.ROWS_BEST_ROWS else (tiled, staged)
+    assert taken < 1.15 * other, (staged, tiled)
 
 
 @pytest.mark.parametrize("parts", [1, 2])

@@ -306,7 +306,7 @@ def test_a_batch_whose_size_changes_replays_one_graph(long_folder, dtype):
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 def test_many_decoding_rows_beside_prompt_portions(long_folder, dtype):
     """Steps that hold 20 to 34 single tokens AND two or three prompt portions of changing size (2 to 290
-    tokens; a few steps pass 192 rows and take the products for many rows), at head size 128: in bfloat16 one
+    tokens; a few steps pass 128 rows and take the products for many rows), at head size 128: in bfloat16 one
     forward pass then runs the rotary kernel, the prefill attention and the split decode attention side
     by side.  The pool holds exactly what live requests need at the peak, so pages are used again while
     others are still read.  Every row of every request against the plain implementation."""

@@ -1,6 +1,7 @@
 """How a prompt product is cut at rows that its class was not timed at: by the times of the rows it was timed at, in proportion to the rounds
 of tiles over the compute units."""
 import math
+import os
 from types import SimpleNamespace
 
 import pytest
@@ -73,13 +74,21 @@ def test_own_products_keep_the_plans_bits_at_every_number_of_rows(monkeypatch):
     assert rt._fastest(("linear",), {}, ("plan", 443, 233), 1101, _price("slabs", 4096), slabs=True) == 443
 
 
+def test_both_hosts_leave_the_kernel_for_dozens_of_rows_at_the_same_number():
+    rt = Runtime.__new__(Runtime)
+    rt.ops, rt.staged_rows = ops, ops.ROWS_BEST_ROWS
+    assert rt.streams(128, 2560, 6144) and not rt.streams(129, 2560, 6144) and rt.streams(129, 2568, 6144)      # (no multiple of 32 stays)
+    source = os.path.join(os.path.dirname(ops.__file__), "..", "host", "backend_hip.c")
+    assert f"#define STAGED_ROWS {ops.ROWS_BEST_ROWS} " in open(source).read()
+
+
 @pytest.mark.parametrize("own", [True, "auto"])
 def test_own_products_are_timed_for_every_number_of_parts(monkeypatch, own):
     """Rows of one class that the plan cuts into one, two and three parts of K: each finds the cuts with its parts among the ways, timed; where
     any way may be taken, the class is timed once."""
     rt = Runtime.__new__(Runtime)
     rt.own_prompt_products, rt.for_a_graph, rt.prompt_product_choices = own, False, {}
-    rt.staged_rows, rt.few_rows, rt.tile_products, rt.library_products = 192, 64, 0, 0
+    rt.staged_rows, rt.few_rows, rt.tile_products, rt.library_products = 128, 64, 0, 0
     parts = {1100: 1, 1300: 2, 1500: 3, 1101: 1}
     asked = []
     rt.ops = SimpleNamespace(gemm_rows_ok=lambda m, k: False, gemm_tiles_ok=lambda m, k, n: True, gemm_tiles_parts=lambda m, *a: parts[m],
