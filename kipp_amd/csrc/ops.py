@@ -782,19 +782,26 @@ CHUNKS_FROM = 16
 def matrix_chunks_from(mode: int, d: int, state: int) -> int:
     """Tokens of a step's longest entry from which on chunks are the faster way (mode 0 fixed decays, 1 the delta rule, 2 a decay a token, 3 an mLSTM;
     `state`: numbers of the memories of all the entries that would go by chunks).  In the walk's time, one entry of 16 / 64 / 128 / 256
-    tokens: 8 heads of 128 x 320, fixed 1.63 1.05 0.70 0.47, delta 2.76 1.48 0.99 0.70; 8 of 64 x 128, 1.80 0.95 0.64 0.45 and 2.81 1.43 0.96
-    0.66; 16 of 256 x 256, 1.57 0.98 0.53 0.36 and 2.42 1.42 0.73 0.51.  Sixteen entries: 1.49 0.70 0.56 0.46 and 2.57 1.13 0.94 0.83; 2.09 1.39 0.96 0.81
-    and 2.90 1.69 1.15 0.93; 0.97 0.40 0.34 0.28 and 1.23 0.54 0.46 0.38.  Where single tokens walk beside them that launch comes on top.
+    tokens: 8 heads of 128 x 320, fixed 1.88 1.00 0.63 0.40, delta 3.15 1.47 0.95 0.58; 8 of 64 x 128, 1.87 0.89 0.57 0.36 and 3.20 1.45 0.91 0.58;
+    16 of 256 x 256, 1.74 0.96 0.49 0.33 and 2.81 1.42 0.70 0.47.  Sixteen entries: 1.52 0.69 0.55 0.47 and 2.67 1.05 0.84 0.72; 2.69 1.20 0.90 0.71
+    and 3.20 1.63 1.19 0.99; 0.94 0.35 0.29 0.23 and 1.41 0.54 0.44 0.33.  Where single tokens walk beside them that launch comes on top.
     Whole steps of a prompt of 64, 80, 96, 112 tokens, us that chunks take more: two memories of 8 heads of 128 x 320, fixed -7 -21 -36 -53, two with
     40 of 128 x 64, a decay a token, -1 -9 -15 -21; the delta rule 27 18 2 -7, four prompts of 64, 96, 128, 176 tokens 32 24 18 9.
     An mLSTM, us walk / chunks, one entry of 32, 48, 64 tokens: 8 heads of 128 x 320 17 / 21, 23 / 21, 28 / 22, of 256 x 512 24 / 30, 34 / 34, 42 / 39, 4 of
-    64 x 128 18 / 20, 26 / 21, 31 / 20; eight entries of 16, 32: 29 / 29, 46 / 34; 100 / 64, 173 / 75; 12 / 21, 17 / 21."""
+    64 x 128 18 / 20, 26 / 21, 31 / 20; eight entries of 16, 32: 29 / 29, 46 / 34; 100 / 64, 173 / 75; 12 / 21, 17 / 21.
+    Many memories of long keys, us walk / chunks, entries of 24, 32, 48 tokens: 16 entries of 16 heads of 192 x 128, fixed 102 / 52, 134 / 56, 187 / 68, a decay a
+    token 85 / 45, 110 / 48, 149 / 60, the delta rule 96 / 78, 123 / 82, 173 / 96, an mLSTM 153 / 54, 181 / 56, 254 / 68; two of 16 heads of 256 x 256, fixed 27 / 31,
+    40 / 32, 65 / 39, the delta rule 24 / 42, 38 / 44, 60 / 51; 48 of 8 heads of 64 x 128, an mLSTM 81 / 49, 100 / 49, 144 / 56.  Over 3,520 calls of
+    16 to 256 tokens the faster way is missed by 1.9 % in the mean."""
     many = state >= 1 << 22
+    wide = d >= 192 and state >= 3 << 19        # (16 heads of 192 x 128, four entries)
     if mode == 3:
-        return 32 if many else 64
+        return 16 if wide and many else (24 if wide or state >= d << 15 else 64)
     if mode == 1:
-        return (48 if many else 112) if d >= 192 else (128 if state < 1 << 19 else 224)
-    return 144 if d < 128 else (48 if many else (64 if d >= 192 else 80))
+        return (40 if many else (48 if wide else 112)) if d >= 192 else (128 if state < 1 << 19 else 224)
+    if d >= 192:
+        return 24 if many else (32 if wide else 64)
+    return (144 if state >= 3 << 18 else 96) if d < 128 else (48 if many else 80)
 
 
 def matrix_chunks_ok(d: int) -> bool:
