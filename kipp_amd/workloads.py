@@ -187,18 +187,28 @@ def mfma_rate() -> dict:
     return {"workload": "mfma rate", "compute_units": cus, "all": table}
 
 
-def _time(fn, runs: int = 20) -> float:
-    """Microseconds a call, over `runs` calls after three that are not timed."""
+def _time_in_turn(ways: dict, rounds: int = 7, runs: int = 4) -> dict:
+    """Microseconds a call of every way: each runs three times first, then all in turn without a pause, there and back, `runs` calls a time
+    behind one that is not timed (a chip at its power limit clocks by what ran before); the median of the rounds."""
     import torch
-    for _ in range(3):
-        fn()
-    start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-    start.record()
-    for _ in range(runs):
-        fn()
-    end.record()
-    end.synchronize()
-    return start.elapsed_time(end) / runs * 1e3
+    for run in ways.values():
+        for _ in range(3):
+            run()
+    marks = []
+    for turn in range(rounds):
+        for name in list(ways)[::-1 if turn % 2 else 1]:
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            ways[name]()
+            start.record()
+            for _ in range(runs):
+                ways[name]()
+            end.record()
+            marks.append((name, start, end))
+    torch.cuda.synchronize()
+    took = {name: [] for name in ways}
+    for name, start, end in marks:
+        took[name].append(start.elapsed_time(end) / runs * 1e3)
+    return {name: sorted(times)[rounds // 2] for name, times in took.items()}
 
 
 def products(shape: str, rows_list) -> dict:
@@ -219,24 +229,25 @@ def products(shape: str, rows_list) -> dict:
             x = torch.randn(rows, k, device="cuda:0", dtype=torch.bfloat16)
             w = torch.randn(n, k, device="cuda:0", dtype=torch.bfloat16) * 0.02
             act = torch.empty(rows, n // 2, device="cuda:0", dtype=torch.bfloat16)
-            ours = _time(lambda: ops.gemm_tiles(x, w, end, max_parts=4))
-            best_cut, best = "plan", ours
+            ways = {"plan": lambda: ops.gemm_tiles(x, w, end, max_parts=4)}
             for cut in (Runtime.TILE_CUTS_SLABS if end == "slabs" else Runtime.TILE_CUTS_BF16):
-                try:
-                    took = _time(lambda: ops.gemm_tiles(x, w, end, max_parts=4, force=cut))
-                except ops.KernelError:
-                    continue
-                if took < best:
-                    best_cut, best = str(cut), took
+                if end != "slabs" or cut % 10 <= k // 32:
+                    ways[str(cut)] = lambda cut=cut: ops.gemm_tiles(x, w, end, max_parts=4, force=cut)
             if end == "swiglu":
-                library = _time(lambda: ops.swiglu(torch.mm(x, w.t(), out_dtype=torch.float32), act))
+                ways["library"] = lambda: ops.swiglu(torch.mm(x, w.t(), out_dtype=torch.float32), act)
             else:
-                library = _time(lambda: torch.mm(x, w.t(), out_dtype=torch.float32))
+                ways["library"] = lambda: torch.mm(x, w.t(), out_dtype=torch.float32)
+            took = _time_in_turn(ways)
+            ours, library = took["plan"], took["library"]
+            best_cut = min((name for name in took if name != "library"), key=took.get)
+            planned = ops.gemm_tiles_cost(rows, n, k, end, 4)
+            planned_cut = next((name for name in took if name.isdigit() and ops.gemm_tiles_cost(rows, n, k, end, 4, int(name)) == planned), "another")
+            best = took[best_cut]
             flops = 2.0 * rows * n * k
-            table[name] = {"ours_us": round(ours, 1), "ours_best_cut": best_cut, "ours_best_us": round(best, 1),
+            table[name] = {"ours_us": round(ours, 1), "ours_cut": planned_cut, "ours_best_cut": best_cut, "ours_best_us": round(best, 1),
                            "library_us": round(library, 1), "ours_PFLOPs": round(flops / best / 1e9, 3),
                            "library_PFLOPs": round(flops / library / 1e9, 3)}
-            log(f"{rows} rows {name:8s} ours as planned {ours:7.1f} us, best cut {best_cut} {best:7.1f} us ({flops / best / 1e9:.2f} PFLOP/s)   "
+            log(f"{rows} rows {name:8s} ours as planned ({planned_cut}) {ours:7.1f} us, best cut {best_cut} {best:7.1f} us ({flops / best / 1e9:.2f} PFLOP/s)   "
                 f"library {library:7.1f} us ({flops / library / 1e9:.2f} PFLOP/s)")
         out["rows"][str(rows)] = table
     return out
