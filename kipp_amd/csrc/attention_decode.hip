@@ -858,14 +858,25 @@ __global__ void __launch_bounds__(THREADS, 2) attention_decode_ring_kernel(
     bf16_t* __restrict__ out, float* __restrict__ part_acc, float* __restrict__ part_ml,
     const int32_t* __restrict__ rows, const int32_t* __restrict__ positions, const int32_t* __restrict__ seq_of_token,
     const int32_t* __restrict__ block_table, int max_blocks, int n_q, int n_kv, int page, float scale_log2e,
-    int window, int max_splits, int range, Projected pj, unsigned* arrivals) {
+    int window, int max_splits, int range, int folded, Projected pj, unsigned* arrivals) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char ring[];
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l16 = lane & 15, h = lane >> 4;
-    const int kvh = blockIdx.y;
-    const int row = rows[blockIdx.x];                 // the grid is (query tokens, key/value heads, ranges): ranges beyond a sequence's position come last
+    // The grid is (query tokens, key/value heads, ranges), or, `folded` > 0, (heads, tokens, ranges): ranges beyond a sequence's position come
+    // last.  Two workgroups share a compute unit, number i of the launch with number i + 256, and with whole contexts the launch lasts as long
+    // as the compute unit that has the most keys to walk.  So every second run of `folded` tokens (256 workgroups) goes the other way round: where `rows`
+    // come by the length of their contexts, the longest lie beside the shortest.
+    int item = blockIdx.x, kvh = blockIdx.y;
+    if (folded > 0) {
+        item = blockIdx.y;
+        kvh = blockIdx.x;
+        int first = 0, odd = 0;                       // of this run
+        for (; item - first >= folded; first += folded) odd ^= 1;
+        if (odd) item = first + min(first + folded, (int)gridDim.y) - 1 - item;
+    }
+    const int row = rows[item];
     const int pos = positions[row];
     const int lo = first_key(pos, window);
     const int first_split = lo / range, last_split = pos / range;
@@ -1106,11 +1117,11 @@ __global__ void __launch_bounds__(THREADS, 2) attention_decode_ring_kernel(
             *(uint32_t*)(out + out_at(row, head * HEAD_DIM + dcol, n_q * HEAD_DIM, FUSED ? pj.out_rows : 0)) =
                 (uint32_t)f32_to_bf16(a0 / (l + sink_term(m))) | ((uint32_t)f32_to_bf16(a1 / (l + sink_term(m))) << 16);
         } else {
-            put_partial2(arrivals, part_acc, part_ml, ((size_t)blockIdx.x * n_q + head) * max_splits + blockIdx.z, dcol, a0, a1, m, l);
+            put_partial2(arrivals, part_acc, part_ml, ((size_t)item * n_q + head) * max_splits + blockIdx.z, dcol, a0, a1, m, l);
         }
     }
     if (arrivals != nullptr && n_splits > 1)
-        merge_by_the_last(arrivals, part_acc, part_ml, out, blockIdx.x, row, kvh, n_q, n_kv, max_splits, n_splits, FUSED ? pj.out_rows : 0);
+        merge_by_the_last(arrivals, part_acc, part_ml, out, item, row, kvh, n_q, n_kv, max_splits, n_splits, FUSED ? pj.out_rows : 0);
 }
 #endif  // RING_OK
 
@@ -1263,9 +1274,15 @@ static int launch_ring(const bf16_t* q, bf16_t* k_cache, bf16_t* v_cache, bf16_t
     const int span = grid_splits * SPLIT;
     const int ring_splits = (span + range - 1) / range + (window > 0 ? 1 : 0);   // a window may straddle one more edge
     if (ring_splits > max_splits) return 0;
-    hipLaunchKernelGGL(attention_decode_ring_kernel<FUSED>, dim3(n_items, n_kv, ring_splits), dim3(THREADS), lds, stream, q,
+    // Up to 256 workgroups have a compute unit each.  Whole steps of eight layers with eight heads, us, tokens in the order of the requests and unfolded / now:
+    // 64 tokens behind 560 to 2,240 keys 2,755 / 2,620, 40 behind 720 to 2,880 2,595 / 2,379, 100 behind 360 to 1,440 3,404 / 3,286; of equal
+    // contexts 64 behind 1,400 2,566 / 2,566, 128 behind 700 3,168 / 3,184 (heads in turn over the dies 3,195).
+    const long long pairs = (long long)n_items * n_kv;
+    const int folded = pairs > 256 && n_items <= 65535 ? 256 / n_kv : 0;
+    const dim3 grid = folded ? dim3(n_kv, n_items, ring_splits) : dim3(n_items, n_kv, ring_splits);
+    hipLaunchKernelGGL(attention_decode_ring_kernel<FUSED>, grid, dim3(THREADS), lds, stream, q,
                        k_cache, v_cache, out, part_acc, part_ml, rows, positions, seq_of_token, block_table, max_blocks, n_q,
-                       n_kv, page, scale_log2e, window, max_splits, range, pj, arrivals);
+                       n_kv, page, scale_log2e, window, max_splits, range, folded, pj, arrivals);
     *rc = KIPP_LAUNCH_CHECK();
     if (*rc != 0 || ring_splits == 1 || arrivals != nullptr) return 1;
     *rc = launch_reduce(part_acc, part_ml, (bf16_t*)out, rows, positions, n_items, n_q, window, max_splits, range, ring_splits, stream,

@@ -81,7 +81,8 @@ def build_batch(entries: Sequence[StepEntry], requests: Sequence[object], n_grou
         positions.extend(range(req.length, req.length + n))
         seq_of.extend([i] * n)
     n_seqs = len(entries)
-    decode_rows = [q_start[i] for i in range(n_seqs) if q_len[i] == 1]
+    # the longest context first: decode attention hands its workgroups out in this order
+    decode_rows = [q_start[i] for i in sorted((i for i in range(n_seqs) if q_len[i] == 1), key=lambda i: -ctx_len[i])]
     decode_ctx = [ctx_len[i] for i in range(n_seqs) if q_len[i] == 1]
     max_blocks = max(1, max(len(req.tables[g]) for req in requests for g in range(n_groups)) if n_groups else 1)
     tables = []

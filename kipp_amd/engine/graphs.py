@@ -58,12 +58,12 @@ class DecodeGraph:
         # a table row is as wide as the contexts of this shape, not as the model's longest possible one:
         # kernels choose by it what they can do, and it is copied whenever a row changes
         self.blocks = [max(1, -(-max_context // g.page_size)) for g in cache.groups]     # of a table row, per group
-        self.table_at = [4 * n + n * sum(self.blocks[:g]) for g in range(self.groups)]     # where a group's tables begin
+        self.table_at = [5 * n + n * sum(self.blocks[:g]) for g in range(self.groups)]     # where a group's tables begin
         self.max_context = max_context
         table_ints = n * sum(self.blocks)
-        # [tokens | positions | ctx_len | slots | tables | arange | ones]
-        self.layout = {"tokens": 0, "positions": n, "ctx_len": 2 * n, "slots": 3 * n, "tables": 4 * n}
-        var_ints = 4 * n + table_ints
+        # [tokens | positions | ctx_len | slots | order | tables | arange | ones]
+        self.layout = {"tokens": 0, "positions": n, "ctx_len": 2 * n, "slots": 3 * n, "order": 4 * n, "tables": 5 * n}
+        var_ints = 5 * n + table_ints
         total = var_ints + 2 * n
         self.var_ints = var_ints
         self.host = torch.zeros(total, dtype=torch.int32).pin_memory()
@@ -80,7 +80,7 @@ class DecodeGraph:
         self.batch = StepBatch(
             n_tokens=n, n_seqs=n, n_want=n, tokens=d[0:n], positions=d[n:2 * n], seq_of_token=arange, q_start=arange,
             q_len=ones, ctx_len=d[2 * n:3 * n], slots=d[3 * n:4 * n], want_rows=arange, block_tables=tables,
-            decode_rows=arange, n_decode=n, n_portions=0,
+            decode_rows=d[4 * n:5 * n], n_decode=n, n_portions=0,
             max_decode_ctx=max_context, max_q_len=1, max_ctx_len=max_context, want_every_row=True,
             host={"q_start": list(range(n)), "q_len": [1] * n, "ctx_len": [max_context] * n})
         self.graph: Optional[torch.cuda.CUDAGraph] = None
@@ -104,6 +104,7 @@ class DecodeGraph:
         h[2 * n:3 * n] = h[n:2 * n] + 1
         h[3 * n:3 * n + live] = [r.slot for r in requests]
         h[3 * n + live:4 * n] = self.scratch_slot
+        h[4 * n:5 * n] = np.argsort(-h[n:2 * n], kind="stable")     # as in `build_batch`: the longest context first
         # a row of a block table changes only when its request got a page (or another request
         # took the row): only then is it written again, and only then are the tables copied
         changed = False
@@ -117,7 +118,7 @@ class DecodeGraph:
                 for g in range(self.groups):
                     at, width = self.table_at[g] + i * self.blocks[g], self.blocks[g]
                     h[at:at + width] = r.rows[g][:width] if r is not None else self.scratch_pages[g]
-        upto = self.var_ints if changed else 4 * n
+        upto = self.var_ints if changed else 5 * n
         self.dev[:upto].copy_(self.host[:upto], non_blocking=True)
         self.copied = torch.cuda.Event()
         self.copied.record()

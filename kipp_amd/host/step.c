@@ -135,6 +135,24 @@ static int batch_room(kipp_model *model, size_t ints, kipp_error *error) {
     return 0;
 }
 
+/* Rows of single tokens, the longest context first (among equals the lower row): decode attention hands its workgroups out in this order. */
+static void order_by_context(int32_t *rows, size_t count, const int32_t *positions) {
+    size_t gap = 1;
+    while (gap < count / 3) gap = 3 * gap + 1;
+    for (; gap > 0; gap /= 3) {
+        for (size_t i = gap; i < count; ++i) {
+            const int32_t row = rows[i];
+            size_t at = i;
+            for (; at >= gap; at -= gap) {
+                const int32_t other = rows[at - gap];
+                if (positions[other] > positions[row] || (positions[other] == positions[row] && other < row)) break;
+                rows[at] = other;
+            }
+            rows[at] = row;
+        }
+    }
+}
+
 /* Flattens the items: the tokens of every item one after the other, with what each operation needs to find a token's
  * sequence, position and pages; all integers go to where the path computes in one copy. */
 static int build_batch(kipp_model *model, const kipp_step_item *items, size_t item_count, bool rounded, kipp_error *error) {
@@ -206,6 +224,7 @@ static int build_batch(kipp_model *model, const kipp_step_item *items, size_t it
             }
         }
     }
+    order_by_context(h_decode, decode_at, h_positions);
     batch->h_q_start = h_q_start;
     batch->h_q_len = h_q_len;
     batch->h_ctx_len = h_ctx_len;
