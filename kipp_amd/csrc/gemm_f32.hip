@@ -9,15 +9,15 @@
 // in order.  All kernels below do exactly that, W always the instruction's first operand and X its second.
 //
 //   rows   up to 16 rows of X a workgroup (32 or 64 for short K): 16 rows of W, a wave a run of K, straight from memory into the instruction's
-//          operands (16 bytes a lane), the runs' sums added through LDS.  Bound by the read of W.  A 16-column fragment of
+//          operands (16 bytes a lane), the runs' sums added through LDS.  Bound by the read of W (5.9 TB/s for the head's matrix).  A 16-column fragment of
 //          X is multiplied whether its rows are there or not: at one row the matrix cores could feed 19 TB/s.
 //   tiles  more rows: 64 or 32 rows of W times 64, 48 or 32 of X a workgroup, a wave a run of K here too, so that every wave of a
 //          workgroup multiplies all of its outputs and none waits for another in the walk.  Bound by the instruction's rate (80 %
 //          of it at 1,024 rows) and, below a few rounds of tiles, by what the last round leaves idle: the shape goes by that.
 //   shared 64 x 64 outputs a workgroup of four waves, which meet at a barrier every 32 numbers of k: short K in many tiles, where a run a wave
 //          does not pay (`form_of`).
-// Measured at the 4B shape, W in turn from three copies, us: one row against 19,456 x 2,560 46 (4.3 TB/s), 2,560 x 9,728 34, the head's
-// 151,936 x 2,560 325 (4.8 TB/s).  The tiles, against 19,456 x 2,560 / 6,144 x 2,560 / 2,560 x 4,096 / 2,560 x 9,728, beside what these
+// Measured at the 4B shape, W in turn from several copies, us: one row against 19,456 x 2,560 39 (5.1 TB/s), 2,560 x 9,728 26, the head's
+// 151,936 x 2,560 264 (5.9 TB/s).  The tiles, against 19,456 x 2,560 / 6,144 x 2,560 / 2,560 x 4,096 / 2,560 x 9,728, beside what these
 // rows took before (up to 64 rows of X through the kernel for rows, 64 x 64 tiles of four waves that share a step of K beyond):
 //      32 rows    56 / 16 / 20 / 49      106 / 36 / 28 / 73
 //      64 rows    78 / 27 / 21 / 49      171 / 64 / 46 / 115
@@ -115,25 +115,47 @@ gemm_f32_rows_kernel(const float* __restrict__ X, const TW* __restrict__ W, floa
     f32x4 acc[MT];
 #pragma unroll
     for (int i = 0; i < MT; ++i) acc[i] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
-    constexpr int AHEAD = MT == 1 ? 8 : (MT == 2 ? 6 : 4);       // 16-number pieces asked for together
-    int k = k_lo;
-    for (; k + 16 * AHEAD <= k_hi; k += 16 * AHEAD) {
-        f32x4 w[AHEAD], x[AHEAD][MT];
+    // Pieces of 16 numbers, AHEAD of them on their way: a piece's place is asked for again as soon as it has been multiplied.  (Eight asked for
+    // together, multiplied, and the run's last ones one after the other before: one row against 151,936 / 19,456 / 6,144 x 2,560 and 2,560 x 4,096 / 9,728, us,
+    // 325 / 46.7 / 19.7 / 14.7 / 33.4, with four on their way 271 / 39 / 17 / 12 / 25, six 264 / 39 / 17 / 12.5 / 26, eight 287 / 42 / 18 / 14 / 29, ten
+    // 257 / 38 / 18 / 15 / 30, twelve 386 / 54 / 21 / 16 / 30; 30 rows against 19,456 x 64 7.0, with three 5.6, four 6.8, six 7.3.)
+    constexpr int AHEAD = MT == 1 ? 6 : 3;
+    const int whole = max(k_hi - k_lo, 0) / 16;
+    f32x4 w[AHEAD], x[AHEAD][MT];
+    auto ask = [&](int j, int piece) {
+        const int k = k_lo + 16 * piece + h4;
+        w[j] = four_inside<VEC>(w_row + k);
+#pragma unroll
+        for (int i = 0; i < MT; ++i) x[j][i] = four_inside<VEC>(x_row[i] + k);
+    };
+    auto take = [&](int j) {
+#pragma unroll
+        for (int i = 0; i < MT; ++i) acc[i] = mul16(w[j], x[j][i], acc[i]);
+    };
+#pragma unroll
+    for (int j = 0; j < AHEAD; ++j)
+        if (j < whole) ask(j, j);
+    int piece = 0;
+    for (; piece + 2 * AHEAD <= whole; piece += AHEAD) {
 #pragma unroll
         for (int j = 0; j < AHEAD; ++j) {
-            w[j] = four<VEC>(w_row, k + 16 * j + h4, K);
-#pragma unroll
-            for (int i = 0; i < MT; ++i) x[j][i] = four<VEC>(x_row[i], k + 16 * j + h4, K);
+            take(j);
+            ask(j, piece + AHEAD + j);
         }
-#pragma unroll
-        for (int j = 0; j < AHEAD; ++j)
-#pragma unroll
-            for (int i = 0; i < MT; ++i) acc[i] = mul16(w[j], x[j][i], acc[i]);
     }
-    for (; k < k_hi; k += 16) {
-        const f32x4 w = four<VEC>(w_row, k + h4, K);
 #pragma unroll
-        for (int i = 0; i < MT; ++i) acc[i] = mul16(w, four<VEC>(x_row[i], k + h4, K), acc[i]);
+    for (int j = 0; j < AHEAD; ++j) {
+        if (piece + j < whole) take(j);
+        if (piece + AHEAD + j < whole) ask(j, piece + AHEAD + j);
+    }
+#pragma unroll
+    for (int j = 0; j < AHEAD; ++j)
+        if (piece + AHEAD + j < whole) take(j);
+    const int k = k_lo + 16 * whole;
+    if (k < k_hi) {                 // what K ends with
+        const f32x4 last = four<VEC>(w_row, k + h4, K);
+#pragma unroll
+        for (int i = 0; i < MT; ++i) acc[i] = mul16(last, four<VEC>(x_row[i], k + h4, K), acc[i]);
     }
 #pragma unroll
     for (int i = 0; i < MT; ++i) *reinterpret_cast<f32x4*>(part_s[wave][i][lane]) = acc[i];

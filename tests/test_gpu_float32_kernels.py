@@ -36,6 +36,24 @@ def test_product_rows_are_the_same_in_both_kernels(n, k):
     assert torch.equal(got, again)          # a weight in bfloat16 is widened exactly
 
 
+@pytest.mark.parametrize("pieces", [0, 1, 2, 3, 5, 6, 7, 8, 11, 12, 13, 18, 19, 24, 25])
+@pytest.mark.parametrize("m", [1, 16, 20])
+def test_few_rows_over_every_number_of_pieces(m, pieces):
+    """The kernel for few rows with up to twice and more of the 16-number pieces that it asks for ahead in the last run of K, whole and with a part
+    of one behind them.  Bound as above."""
+    import torch
+    from kipp_amd.csrc import ops
+    part = -(-max(pieces, 1) // 2) * 32
+    for rest in (0, 4, 5):
+        k = 7 * part + min(16 * pieces + rest, part) if pieces else rest + 1
+        rng = np.random.default_rng(pieces + rest + m)
+        x, w = rng.normal(size=(m, k)).astype(np.float32), rng.normal(size=(37, k)).astype(np.float32)
+        got = ops.gemm_f32(torch.tensor(x, device=DEV), torch.tensor(w, device=DEV), torch.empty((m, 37), device=DEV)).cpu().numpy()
+        exact = x.astype(np.float64) @ w.astype(np.float64).T
+        size = np.abs(x).astype(np.float64) @ np.abs(w).astype(np.float64).T
+        assert np.all(np.abs(got - exact) <= (min(k, _run_of(k)) + 8) * EPS * size), k
+
+
 @pytest.mark.parametrize("m, n", [(17, 32), (33, 47), (49, 2579), (97, 2570), (350, 3001), (333, 2570), (200, 6155)])
 @pytest.mark.parametrize("k", [40, 268])
 def test_product_in_every_shape_of_tiles(m, n, k):
