@@ -58,12 +58,13 @@
 #define P_ROW 1288
 #define M_ROW 40
 #define M_HEAD 656
-#define MX_LDS_BYTES ((2 * MX_ROWS * P_ROW + MX_HPAD * M_HEAD) * 2)
+#define MX_LDS_BYTES ((2 * MX_ROWS * P_ROW + MX_HPAD * M_HEAD) * 2 + HEAD_BLOCKS * KIPP_WAVE * 16)
 #define KSTEPS (HEAD_DIM / 32)
 #ifndef V_SLICE
 #define V_SLICE V_DIM                   // value columns a workgroup sums: V_DIM / V_SLICE workgroups share an item, each
 #endif                                  // with its own columns (their sums then fit a wave's registers) and all of the weights
 #define VBLOCKS (V_SLICE / 16)
+#define HEAD_BLOCKS (MX_WAVES * HPW > 16 ? 2 : 1)       // blocks of 16 mixed heads: a build of more heads a wave has more than 16 in all
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
@@ -84,6 +85,11 @@ __device__ __forceinline__ uint32_t to_bf16_pair(float a, float b) {
 }
 
 #define LOG2E 1.4426950408889634f
+
+template <bool V>
+struct Const {
+    static constexpr bool value = V;
+};
 
 struct MixedGeometry {
     const int32_t* item_entry;      // [items] entry of the batch
@@ -131,20 +137,31 @@ __device__ __forceinline__ int key_tile(const Tile& t, int index) {
     return index < t.kept_tiles ? index : t.window_tile0 + index - t.kept_tiles;
 }
 
-// The page of a lane's key among the 16 from `key0` on.
-__device__ __forceinline__ int page_of(const MixedGeometry& g, const Tile& t, int key0) {
-    return t.table[min(key0 + (int)(threadIdx.x & 15), t.last) / g.page];
+// The 16 keys from a multiple of 16 on lie in one page (whose size is a multiple of 16): where, the same for every lane of a wave, so
+// that the table is read through the scalar cache and a load's address is a scalar base and a lane's own 32-bit offset.
+struct Block {
+    int first;                  // the first of them; the last key of the tile where they all lie beyond it
+    int page, slot;             // of `first`
+};
+
+__device__ __forceinline__ Block block_of(const MixedGeometry& g, const Tile& t, int key0) {
+    Block b;
+    b.first = __builtin_amdgcn_readfirstlane(min(key0, t.last));
+    const int at = __builtin_amdgcn_readfirstlane((int)((uint32_t)b.first / (uint32_t)g.page));
+    b.page = ((const __attribute__((address_space(4))) int32_t*)t.table)[at];
+    b.slot = b.first - at * g.page;
+    return b;
 }
 
-// The 16 keys from `key0` on of key/value head `c` as A operands: lane l holds key l % 16, columns 32 s + 8 (l / 16) ..
-// `page`: the lane's page_of them.
-__device__ __forceinline__ void load_keys(const MixedGeometry& g, const Tile& t, const bf16_t* __restrict__ k_cache, int c, int key0, int page,
-                                          Frag* kf) {
-    const int lane = threadIdx.x & (KIPP_WAVE - 1), l16 = lane & 15, quarter = lane >> 4;
-    const int key = min(key0 + l16, t.last);            // rows beyond the context are masked later; their loads stay inside it
-    const bf16_t* row = k_cache + (((size_t)page * g.n_kv + c) * g.page + key % g.page) * HEAD_DIM + 8 * quarter;
+// A block's keys of key/value head `c` as A operands: lane l holds key l % 16, columns 32 s + 8 (l / 16) ..
+__device__ __forceinline__ void load_keys(const MixedGeometry& g, const Tile& t, const bf16_t* __restrict__ k_cache, int c, const Block& b,
+                                          int lane, Frag* kf) {
+    const int l16 = lane & 15, quarter = lane >> 4;
+    const bf16_t* base = k_cache + (((size_t)b.page * g.n_kv + c) * g.page + b.slot) * HEAD_DIM;
+    // (rows beyond the context are masked later; their loads stay inside it)
+    const uint32_t own = min(l16, t.last - b.first) * HEAD_DIM + 8 * quarter;
 #pragma unroll
-    for (int s = 0; s < KSTEPS; ++s) kf[s].u = *(const u32x4*)(row + 32 * s);
+    for (int s = 0; s < KSTEPS; ++s) kf[s].u = *(const u32x4*)(base + own + 32 * s);
 }
 
 // S^T[key][row] of one head for the 16 keys from `key0` on: lane l gets keys key0 + 4 (l / 16) + v of row l % 16,
@@ -152,8 +169,8 @@ __device__ __forceinline__ void load_keys(const MixedGeometry& g, const Tile& t,
 // e^(-a ln u) is 2^(-a log2 u)).  `kf`: the keys as A operands, `qf`: the head's query rows as B operands.
 template <bool INSIDE>
 __device__ __forceinline__ void scores16(const MixedGeometry& g, const Tile& t, int key0, const Frag* kf, const Frag* qf,
-                                         float a, float b, float sc[4]) {
-    const int lane = threadIdx.x & (KIPP_WAVE - 1), l16 = lane & 15, quarter = lane >> 4;
+                                         float a, float b, int lane, float sc[4]) {
+    const int l16 = lane & 15, quarter = lane >> 4;
     f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int s = 0; s < KSTEPS; ++s) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[s].v, qf[s].v, acc, 0, 0, 0);
@@ -184,13 +201,13 @@ __device__ __forceinline__ void load_queries(const Tile& t, const bf16_t* __rest
 }
 
 // stats [items][n_q][16][2]: (maximum, sum of 2^(score - maximum)) over the item's keys, without the sink.
-// Bound by vector instructions (a logarithm and an exponential a score): 1,500 rows of 32 heads 51 us with both in base 2 and the pages
-// asked for a tile ahead of the keys, 68 in base e.
+// Bound by vector instructions (a logarithm and an exponential a score): 1,500 rows of 32 heads 41 us, as 414 items with a page looked up by
+// every lane 51, in base e 68.
 __global__ void __launch_bounds__(MX_THREADS) mixed_stats_kernel(MixedGeometry g, const bf16_t* __restrict__ q,
                                                                  const bf16_t* __restrict__ k_cache, float* __restrict__ stats) {
     const int item = blockIdx.x;
     const Tile t = tile_of(g, item);
-    const int wave = threadIdx.x / KIPP_WAVE, lane = threadIdx.x & (KIPP_WAVE - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / KIPP_WAVE), lane = threadIdx.x & (KIPP_WAVE - 1);
     const int group = g.n_q / g.n_kv, h0 = wave * HPW;
     if (h0 >= g.n_q) return;
     constexpr bool shared = SHARED_KV != 0;                 // the wave's heads read one key/value head
@@ -206,15 +223,15 @@ __global__ void __launch_bounds__(MX_THREADS) mixed_stats_kernel(MixedGeometry g
         l[hh] = 0.0f;
     }
     Frag kf[MX_KEYS / 16][KSTEPS], next[MX_KEYS / 16][KSTEPS];
-    int page[MX_KEYS / 16], page_next[MX_KEYS / 16];        // of this tile's keys and of the next's: asked for a tile ahead of the keys
+    Block at[MX_KEYS / 16], at_next[MX_KEYS / 16];          // of this tile's keys and of the next's: asked for a tile ahead of the keys
     if (t.begin < t.end) {
 #pragma unroll
         for (int kb = 0; kb < MX_KEYS / 16; ++kb) {
-            page[kb] = page_of(g, t, key_tile(t, t.begin) * MX_KEYS + 16 * kb);
-            page_next[kb] = page_of(g, t, key_tile(t, min(t.begin + 1, t.end - 1)) * MX_KEYS + 16 * kb);
+            at[kb] = block_of(g, t, key_tile(t, t.begin) * MX_KEYS + 16 * kb);
+            at_next[kb] = block_of(g, t, key_tile(t, min(t.begin + 1, t.end - 1)) * MX_KEYS + 16 * kb);
         }
 #pragma unroll
-        for (int kb = 0; kb < MX_KEYS / 16; ++kb) load_keys(g, t, k_cache, h0 / group, key_tile(t, t.begin) * MX_KEYS + 16 * kb, page[kb], next[kb]);
+        for (int kb = 0; kb < MX_KEYS / 16; ++kb) load_keys(g, t, k_cache, h0 / group, at[kb], lane, next[kb]);
     }
     for (int index = t.begin; index < t.end; ++index) {
         const int key0 = key_tile(t, index) * MX_KEYS;
@@ -223,15 +240,15 @@ __global__ void __launch_bounds__(MX_THREADS) mixed_stats_kernel(MixedGeometry g
 #pragma unroll
             for (int s = 0; s < KSTEPS; ++s) kf[kb][s] = next[kb][s];
         const bool inside = all_seen(g, t, key0);
-        int own_page[MX_KEYS / 16];
+        Block own_at[MX_KEYS / 16];
 #pragma unroll
-        for (int kb = 0; kb < MX_KEYS / 16; ++kb) own_page[kb] = page[kb];
+        for (int kb = 0; kb < MX_KEYS / 16; ++kb) own_at[kb] = at[kb];
         if (index + 1 < t.end) {            // the next tile's keys are on their way while this one is scored
 #pragma unroll
             for (int kb = 0; kb < MX_KEYS / 16; ++kb) {
-                page[kb] = page_next[kb];
-                load_keys(g, t, k_cache, h0 / group, key_tile(t, index + 1) * MX_KEYS + 16 * kb, page[kb], next[kb]);
-                page_next[kb] = page_of(g, t, key_tile(t, min(index + 2, t.end - 1)) * MX_KEYS + 16 * kb);
+                at[kb] = at_next[kb];
+                load_keys(g, t, k_cache, h0 / group, at[kb], lane, next[kb]);
+                at_next[kb] = block_of(g, t, key_tile(t, min(index + 2, t.end - 1)) * MX_KEYS + 16 * kb);
             }
         }
 #pragma unroll
@@ -240,10 +257,10 @@ __global__ void __launch_bounds__(MX_THREADS) mixed_stats_kernel(MixedGeometry g
 #pragma unroll
             for (int kb = 0; kb < MX_KEYS / 16; ++kb) {
                 Frag own[KSTEPS];
-                if (!shared && hh > 0) load_keys(g, t, k_cache, (h0 + hh) / group, key0 + 16 * kb, own_page[kb], own);
+                if (!shared && hh > 0) load_keys(g, t, k_cache, (h0 + hh) / group, own_at[kb], lane, own);
                 float sc[4];
-                if (inside) scores16<true>(g, t, key0 + 16 * kb, (!shared && hh > 0) ? own : kf[kb], qf[hh], a[hh], b[hh], sc);
-                else scores16<false>(g, t, key0 + 16 * kb, (!shared && hh > 0) ? own : kf[kb], qf[hh], a[hh], b[hh], sc);
+                if (inside) scores16<true>(g, t, key0 + 16 * kb, (!shared && hh > 0) ? own : kf[kb], qf[hh], a[hh], b[hh], lane, sc);
+                else scores16<false>(g, t, key0 + 16 * kb, (!shared && hh > 0) ? own : kf[kb], qf[hh], a[hh], b[hh], lane, sc);
                 const float m_new = fmaxf(m[hh], fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3])));
                 if (m_new != -INFINITY) {
                     float sum = 0.0f;
@@ -275,8 +292,11 @@ __global__ void __launch_bounds__(MX_THREADS) mixed_stats_kernel(MixedGeometry g
     }
 }
 
-// Bound by vector instructions, LDS and two barriers a tile: 1,500 rows of 32 heads of 128 181 us (186 with weights in base e).  Values and
-// pages asked for ahead as well: 198 (no registers are left: they spill).
+// Bound by vector instructions, LDS and two barriers a tile; a compute unit holds one workgroup, so its loads' latencies show: the table is read
+// through the scalar cache a tile ahead, the values leave memory while the heads are mixed.  Registers (256 a wave) decide: sums and queries take 192, and with a
+// lane's places in LDS kept over tiles, the mix in registers and all heads' scores at once in the scheduler's hands 73 to 175 spilled.  1,500 rows of 32
+// heads of 128, us: 166 as it was (73 spilled, 414 items of up to eight tiles); 89 now (232 items of up to twelve, `ops.mixed_tile_runs`).
+// The first keys of the next tile asked for as well: 75 spill where a workgroup sums all of 128 value columns; there they wait.
 // LDS: p_hi, p_lo [16 rows][32 keys][32 heads] bfloat16, then p' [32 heads][16 rows][32 keys] bfloat16, with the padded strides above.
 __global__ void __launch_bounds__(MX_THREADS) mixed_values_kernel(
     MixedGeometry g, const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache,
@@ -289,7 +309,7 @@ __global__ void __launch_bounds__(MX_THREADS) mixed_values_kernel(
     bf16_t* p_mixed = p_lo + MX_ROWS * P_ROW;
     const int item = blockIdx.x, v0 = blockIdx.y * V_SLICE;        // this workgroup's value columns v0 .. v0 + V_SLICE - 1 of every head
     const Tile t = tile_of(g, item);
-    const int wave = threadIdx.x / KIPP_WAVE, lane = threadIdx.x & (KIPP_WAVE - 1), l16 = lane & 15, quarter = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / KIPP_WAVE), lane_of_wave = threadIdx.x & (KIPP_WAVE - 1), l16 = lane_of_wave & 15, quarter = lane_of_wave >> 4;
     const int nsplits = g.item_nsplits[item], split = g.item_split[item];
     const int n_q = g.n_q, group = g.n_q / g.n_kv;
     constexpr bool shared = SHARED_KV != 0;                 // the wave's heads read one key/value head
@@ -298,18 +318,23 @@ __global__ void __launch_bounds__(MX_THREADS) mixed_values_kernel(
     if (n_q < MX_HPAD)
         for (int e = threadIdx.x; e < 2 * MX_ROWS * P_ROW / 8; e += MX_THREADS) ((u32x4*)p_hi)[e] = (u32x4){0u, 0u, 0u, 0u};
 
-    // mix^T as B operands: lane holds head (column) 16 nb + l % 16, contraction heads 8 (l / 16) ..
-    Frag mf[2];
+    // mix^T as B operands: lane holds head (column) 16 nb + l % 16, contraction heads 8 (l / 16) ..  (asked for whatever the head, inside the
+    // matrix: all loads beside each other)
+    u32x4* mix_frags = (u32x4*)(p_mixed + MX_HPAD * M_HEAD);        // in LDS: in registers they would take the place of keys on their way
+    if (wave < HEAD_BLOCKS) {
+        const int h = 16 * wave + l16;
+        float w[8];
+        if (mix != nullptr) {
 #pragma unroll
-    for (int nb = 0; nb < 2; ++nb) {
-        const int h = 16 * nb + l16;
+            for (int j = 0; j < 8; ++j) w[j] = mix[min(h, n_q - 1) * n_q + min(8 * quarter + j, n_q - 1)];
+        } else {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const int from = 8 * quarter + j;
-            float w = 0.0f;
-            if (h < n_q && from < n_q) w = mix != nullptr ? mix[h * n_q + from] : (h == from ? 1.0f : 0.0f);
-            mf[nb].h[j] = f32_to_bf16(w);
+            for (int j = 0; j < 8; ++j) w[j] = h == 8 * quarter + j ? 1.0f : 0.0f;
         }
+        Frag mf;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) mf.h[j] = f32_to_bf16(h < n_q && 8 * quarter + j < n_q ? w[j] : 0.0f);
+        mix_frags[64 * wave + lane_of_wave] = mf.u;
     }
 
     // this wave's heads: queries, bias numbers, and every row's maximum and denominator over ALL runs of the tile
@@ -317,43 +342,41 @@ __global__ void __launch_bounds__(MX_THREADS) mixed_values_kernel(
     float bias_a[HPW], bias_b[HPW], under[HPW];         // a weight is 2^(score + under)
 #pragma unroll
     for (int hh = 0; hh < HPW; ++hh) {
-        const int h = wave * HPW + hh;
-        under[hh] = -INFINITY;
-        bias_a[hh] = bias_b[hh] = 0.0f;
-        if (h < n_q) {
-            load_queries(t, q, n_q, h, qf[hh]);
-            bias_a[hh] = g.r1 != nullptr ? g.r1[h] : 0.0f;
-            bias_b[hh] = g.r2 != nullptr ? g.r2[h] : 0.0f;
-            // the runs' statistics: each quarter of the wave takes every fourth run (four asked for at once), the
-            // quarters are then merged, the sink last; any order gives the same maximum, and the sums differ in rounding only
-            float m = -INFINITY, l = 0.0f;
-            for (int s0 = quarter; s0 < nsplits; s0 += 16) {
-                float2 st[4];
+        // (heads that do not exist take the last one's queries, and weigh nothing)
+        const int h = min(wave * HPW + hh, n_q - 1);
+        load_queries(t, q, n_q, h, qf[hh]);
+        bias_a[hh] = g.r1 != nullptr ? g.r1[h] : 0.0f;
+        bias_b[hh] = g.r2 != nullptr ? g.r2[h] : 0.0f;
+        const float sunk = sink != nullptr ? sink[h] * LOG2E : -INFINITY;
+        // the runs' statistics: each quarter of the wave takes every fourth run (four asked for at once), the
+        // quarters are then merged, the sink last; any order gives the same maximum, and the sums differ in rounding only
+        float m = -INFINITY, l = 0.0f;
+        for (int s0 = quarter; s0 < nsplits; s0 += 16) {
+            float2 st[4];
 #pragma unroll
-                for (int s = 0; s < 4; ++s)
-                    st[s] = s0 + 4 * s < nsplits ? *(const float2*)(stats + (((size_t)(item - split + s0 + 4 * s) * n_q + h) * MX_ROWS + l16) * 2)
-                                                 : make_float2(-INFINITY, 0.0f);
+            for (int s = 0; s < 4; ++s)
+                st[s] = *(const float2*)(stats + (((size_t)(item - split + min(s0 + 4 * s, nsplits - 1)) * n_q + h) * MX_ROWS + l16) * 2);
 #pragma unroll
-                for (int s = 0; s < 4; ++s) {
-                    const float m_new = fmaxf(m, st[s].x);
-                    if (m_new != -INFINITY) l = l * __builtin_amdgcn_exp2f(m - m_new) + st[s].y * __builtin_amdgcn_exp2f(st[s].x - m_new);
-                    m = m_new;
-                }
-            }
-#pragma unroll
-            for (int off = 16; off <= 32; off <<= 1) {
-                const float m_o = __shfl_xor(m, off, KIPP_WAVE), l_o = __shfl_xor(l, off, KIPP_WAVE);
-                const float m_new = fmaxf(m, m_o);
-                if (m_new != -INFINITY) l = l * __builtin_amdgcn_exp2f(m - m_new) + l_o * __builtin_amdgcn_exp2f(m_o - m_new);
+            for (int s = 0; s < 4; ++s) {
+                if (s0 + 4 * s >= nsplits) st[s] = make_float2(-INFINITY, 0.0f);
+                const float m_new = fmaxf(m, st[s].x);
+                if (m_new != -INFINITY) l = l * __builtin_amdgcn_exp2f(m - m_new) + st[s].y * __builtin_amdgcn_exp2f(st[s].x - m_new);
                 m = m_new;
             }
-            if (sink != nullptr) {
-                const float sunk = sink[h] * LOG2E, m_new = fmaxf(m, sunk);
-                l = (m == -INFINITY ? 0.0f : l * __builtin_amdgcn_exp2f(m - m_new)) + __builtin_amdgcn_exp2f(sunk - m_new);
-                m = m_new;
-            }
-            under[hh] = l > 0.0f ? -m - __builtin_amdgcn_logf(l) : -INFINITY;
         }
+#pragma unroll
+        for (int off = 16; off <= 32; off <<= 1) {
+            const float m_o = __shfl_xor(m, off, KIPP_WAVE), l_o = __shfl_xor(l, off, KIPP_WAVE);
+            const float m_new = fmaxf(m, m_o);
+            if (m_new != -INFINITY) l = l * __builtin_amdgcn_exp2f(m - m_new) + l_o * __builtin_amdgcn_exp2f(m_o - m_new);
+            m = m_new;
+        }
+        if (sink != nullptr) {
+            const float m_new = fmaxf(m, sunk);
+            l = (m == -INFINITY ? 0.0f : l * __builtin_amdgcn_exp2f(m - m_new)) + __builtin_amdgcn_exp2f(sunk - m_new);
+            m = m_new;
+        }
+        under[hh] = wave * HPW + hh < n_q && l > 0.0f ? -m - __builtin_amdgcn_logf(l) : -INFINITY;
     }
 
     f32x4 acc[HPW][VBLOCKS];
@@ -363,30 +386,50 @@ __global__ void __launch_bounds__(MX_THREADS) mixed_values_kernel(
         for (int mb = 0; mb < VBLOCKS; ++mb) acc[hh][mb] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
     __syncthreads();
 
+    Block at_next[MX_KEYS / 16];            // where the next tile's keys and values lie: asked for a tile ahead
+    // where registers are left: the first half of a tile's keys, asked for while the tile before meets its values
+    constexpr bool keys_ahead = shared && 4 * HPW * (VBLOCKS + KSTEPS) <= 128;
+    Frag first_keys[KSTEPS];
+    if (t.begin < t.end) {
+#pragma unroll
+        for (int kb = 0; kb < MX_KEYS / 16; ++kb) at_next[kb] = block_of(g, t, key_tile(t, t.begin) * MX_KEYS + 16 * kb);
+        if (keys_ahead) load_keys(g, t, k_cache, min(wave * HPW, n_q - 1) / group, at_next[0], lane_of_wave, first_keys);
+    }
     for (int index = t.begin; index < t.end; ++index) {
         const int key0 = key_tile(t, index) * MX_KEYS;
         const bool inside = all_seen(g, t, key0);
-        // 1. the final weights of this wave's heads; 16 keys are loaded once for all heads that share them, and a lane
-        //    writes the weights of its heads (they are neighbours in the [row][key][head] layout) with one store
+        // a lane's places in LDS and in the caches are made again for every tile: kept, they take registers that the sums need
+        int lane = lane_of_wave;
+        asm volatile("" : "+v"(lane));
+        const int l16 = lane & 15, quarter = lane >> 4;
+        Block at_key[MX_KEYS / 16];
 #pragma unroll
         for (int kb = 0; kb < MX_KEYS / 16; ++kb) {
-            if (wave * HPW < n_q) {
+            at_key[kb] = at_next[kb];
+            at_next[kb] = block_of(g, t, key_tile(t, min(index + 1, t.end - 1)) * MX_KEYS + 16 * kb);
+        }
+        // 1. the final weights of this wave's heads; 16 keys are loaded once for all heads that share them, and a lane
+        //    writes the weights of its heads (they are neighbours in the [row][key][head] layout) with one store
+        auto weights = [&](auto all) __attribute__((always_inline)) {
+#pragma unroll
+            for (int kb = 0; kb < MX_KEYS / 16; ++kb) {
+                __builtin_amdgcn_sched_barrier(0);
                 Frag kf[KSTEPS];
-                load_keys(g, t, k_cache, wave * HPW / group, key0 + 16 * kb, page_of(g, t, key0 + 16 * kb), kf);
+                if (keys_ahead && kb == 0) {
+#pragma unroll
+                    for (int s = 0; s < KSTEPS; ++s) kf[s] = first_keys[s];
+                } else {
+                    load_keys(g, t, k_cache, min(wave * HPW, n_q - 1) / group, at_key[kb], lane, kf);
+                }
                 float p[HPW][4];
 #pragma unroll
                 for (int hh = 0; hh < HPW; ++hh) {
-                    const int h = wave * HPW + hh;
+                    if (!shared && hh > 0) load_keys(g, t, k_cache, min(wave * HPW + hh, n_q - 1) / group, at_key[kb], lane, kf);
+                    __builtin_amdgcn_sched_barrier(0);      // one head after the other: mixed, their scores fill the registers that the sums need
+                    float sc[4];
+                    scores16<decltype(all)::value>(g, t, key0 + 16 * kb, kf, qf[hh], bias_a[hh], bias_b[hh], lane, sc);
 #pragma unroll
-                    for (int v = 0; v < 4; ++v) p[hh][v] = 0.0f;
-                    if (h < n_q) {
-                        if (!shared && hh > 0) load_keys(g, t, k_cache, h / group, key0 + 16 * kb, page_of(g, t, key0 + 16 * kb), kf);
-                        float sc[4];
-                        if (inside) scores16<true>(g, t, key0 + 16 * kb, kf, qf[hh], bias_a[hh], bias_b[hh], sc);
-                        else scores16<false>(g, t, key0 + 16 * kb, kf, qf[hh], bias_a[hh], bias_b[hh], sc);
-#pragma unroll
-                        for (int v = 0; v < 4; ++v) p[hh][v] = __builtin_amdgcn_exp2f(sc[v] + under[hh]);
-                    }
+                    for (int v = 0; v < 4; ++v) p[hh][v] = __builtin_amdgcn_exp2f(sc[v] + under[hh]);
                 }
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
@@ -416,9 +459,32 @@ __global__ void __launch_bounds__(MX_THREADS) mixed_values_kernel(
                     }
                 }
             }
+        };
+        if (wave * HPW < n_q) {
+            if (inside) weights(Const<true>{});
+            else weights(Const<false>{});
         }
+        // where the values lie, and the first of them asked for while the heads are mixed
+        // (eight keys of one page: those of quarters 0 and 1 lie in the first block, of 2 and 3 in the second)
+        const Block& low = at_key[0];
+        const Block& high = at_key[MX_KEYS / 16 - 1];
+        const size_t v_page = (size_t)(quarter < 2 ? low.page : high.page) * g.n_kv;
+        const int v_slot = ((quarter < 2 ? low.slot : high.slot) & ~15) + 8 * (quarter & 1);
+        constexpr int VB = VBLOCKS < 4 ? VBLOCKS : 4;                // value blocks asked for together
+        constexpr int VGROUPS = (VBLOCKS + VB - 1) / VB;
+        Frag vf[2][VB];
+        const bf16_t* v_at = v_cache + ((v_page + min(wave * HPW, n_q - 1) / group) * V_DIM + v0 + l16) * g.page + v_slot;
+        auto load_values = [&](int m0) __attribute__((always_inline)) {
+#pragma unroll
+            for (int mb = 0; mb < VB; ++mb)
+                if (m0 + mb < VBLOCKS) vf[m0 / VB % 2][mb].u = *(const u32x4*)(v_at + (size_t)16 * (m0 + mb) * g.page);
+        };
+        if (shared) load_values(0);
         __syncthreads();
         // 2. the heads mixed: 32 blocks of 16 (row, key) pairs, four a wave
+        Frag mf[HEAD_BLOCKS];
+#pragma unroll
+        for (int nb = 0; nb < HEAD_BLOCKS; ++nb) mf[nb].u = mix_frags[64 * nb + lane];
 #pragma unroll
         for (int u = 0; u < (MX_ROWS * MX_KEYS / 16) / MX_WAVES; ++u) {
             const int block = wave + MX_WAVES * u;              // row = block / 2, keys 16 (block % 2) ..
@@ -428,45 +494,38 @@ __global__ void __launch_bounds__(MX_THREADS) mixed_values_kernel(
             hi.u = *(const u32x4*)(p_hi + at);
             lo.u = *(const u32x4*)(p_lo + at);
 #pragma unroll
-            for (int nb = 0; nb < 2; ++nb) {
-                if (16 * nb < n_q) {
-                    f32x4 d = {0.0f, 0.0f, 0.0f, 0.0f};
-                    d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lo.v, mf[nb].v, d, 0, 0, 0);
-                    d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hi.v, mf[nb].v, d, 0, 0, 0);
-                    const int h = 16 * nb + l16;        // d[v]: keys 16 kb + 4 quarter + v of `row`, head h
-                    if (h < n_q) {
-                        uint2 w;
-                        w.x = to_bf16_pair(d[0], d[1]);
-                        w.y = to_bf16_pair(d[2], d[3]);
-                        *(uint2*)(p_mixed + (h * M_HEAD + row * M_ROW + 16 * kb + 4 * quarter)) = w;
-                    }
-                }
+            for (int nb = 0; nb < HEAD_BLOCKS; ++nb) {
+                f32x4 d = {0.0f, 0.0f, 0.0f, 0.0f};
+                d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lo.v, mf[nb].v, d, 0, 0, 0);
+                d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hi.v, mf[nb].v, d, 0, 0, 0);
+                uint2 w;                            // d[v]: keys 16 kb + 4 quarter + v of `row`, head 16 nb + l16
+                w.x = to_bf16_pair(d[0], d[1]);
+                w.y = to_bf16_pair(d[2], d[3]);
+                *(uint2*)(p_mixed + ((16 * nb + l16) * M_HEAD + row * M_ROW + 16 * kb + 4 * quarter)) = w;
             }
         }
         __syncthreads();
+        if (shared && VGROUPS > 1) load_values(VB);
         // 3. times the values
-        const int chunk = min(key0 + 8 * quarter, t.last);          // eight keys of one page (a page holds a multiple of 8)
-        const size_t v_page = (size_t)t.table[chunk / g.page] * g.n_kv;
-        const int v_slot = (key0 + 8 * quarter) % g.page;
         if (shared) {
             if (wave * HPW < n_q) {
-                const bf16_t* v_at = v_cache + ((v_page + wave * HPW / group) * V_DIM + v0 + l16) * g.page + v_slot;
-                constexpr int VB = VBLOCKS < 4 ? VBLOCKS : 4;        // value blocks asked for together
 #pragma unroll
                 for (int m0 = 0; m0 < VBLOCKS; m0 += VB) {
-                    Frag vf[VB];
-#pragma unroll
-                    for (int mb = 0; mb < VB; ++mb)
-                        if (m0 + mb < VBLOCKS) vf[mb].u = *(const u32x4*)(v_at + (size_t)16 * (m0 + mb) * g.page);
+                    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                     for (int hh = 0; hh < HPW; ++hh) {
+                        __builtin_amdgcn_sched_barrier(0);
                         Frag pf;
                         pf.u = *(const u32x4*)(p_mixed + (min(wave * HPW + hh, n_q - 1) * M_HEAD + l16 * M_ROW + 8 * quarter));
 #pragma unroll
                         for (int mb = 0; mb < VB; ++mb)
-                            if (m0 + mb < VBLOCKS && wave * HPW + hh < n_q)
-                                acc[hh][m0 + mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[mb].v, pf.v, acc[hh][m0 + mb], 0, 0, 0);
+                            if (m0 + mb < VBLOCKS)
+                                acc[hh][m0 + mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[m0 / VB % 2][mb].v, pf.v, acc[hh][m0 + mb], 0, 0, 0);
                     }
+                    if (m0 + 2 * VB < VBLOCKS) load_values(m0 + 2 * VB);
+                    // (behind the last group but one, whose registers are free)
+                    if (keys_ahead && m0 / VB == (VGROUPS > 1 ? VGROUPS - 2 : 0))
+                        load_keys(g, t, k_cache, min(wave * HPW, n_q - 1) / group, at_next[0], lane, first_keys);
                 }
             }
         } else {
@@ -504,14 +563,16 @@ __global__ void __launch_bounds__(MX_THREADS) mixed_values_kernel(
                 *(f32x4*)(partial + split * partial_stride + row * ((size_t)n_q * V_DIM) + col) = acc[hh][mb];
             } else {
                 float o[4];
+                if (gate != nullptr) {
+                    float z[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+                    for (int p = 0; p < gate_parts; ++p)
 #pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    o[v] = acc[hh][mb][v];
-                    if (gate != nullptr) {
-                        float z = 0.0f;
-                        for (int p = 0; p < gate_parts; ++p) z += gate[p * gate_part_stride + row * gate_stride + col + v];
-                        o[v] *= 1.0f / (1.0f + __expf(-z));
-                    }
+                        for (int v = 0; v < 4; ++v) z[v] += gate[p * gate_part_stride + row * gate_stride + col + v];
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) o[v] = acc[hh][mb][v] * (1.0f / (1.0f + __expf(-z[v])));
+                } else {
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) o[v] = acc[hh][mb][v];
                 }
                 uint2 w;
                 w.x = (uint32_t)f32_to_bf16(o[0]) | ((uint32_t)f32_to_bf16(o[1]) << 16);
@@ -534,7 +595,8 @@ __global__ void __launch_bounds__(MX_THREADS) mixed_values_kernel(
 //                                for before anything else.  Every run leaves float32 partial sums.
 //
 // Bound by its chains of loads (page, keys; statistics, scores), not by bytes: one token behind 1,500 keys of 8 heads (32 query
-// heads of 128 over them) takes 8.9 us for the scores, 15.0 for the values and 5.6 for the sum of the 24 runs.  The tiles of 16 rows
+// heads of 128 over them) takes 8.8 us for the scores, 14.2 for the values (15.0 while their scores, the mix and the sink were asked for behind the
+// statistics) and 5.0 for the sum of the 24 runs (5.5 with the gate asked for behind the sums).  The tiles of 16 rows
 // took 21.5, 41.5 and 4.9 us for it (bias, mask, exponentials and exchanges for 16 rows, at most 16 runs of 128 keys and more).
 #define SG_KEYS 64
 #define SG_PITCH 72                     // bfloat16 values from a head to the next of the mixed weights in LDS
@@ -582,7 +644,7 @@ __global__ void __launch_bounds__(MX_THREADS) mixed_single_scores_kernel(SingleG
                                                                          float* __restrict__ stats) {
     const int token = blockIdx.y, run = blockIdx.x;
     const Single t = single_of(g, token, run);
-    const int wave = threadIdx.x / KIPP_WAVE, lane = threadIdx.x & (KIPP_WAVE - 1), l16 = lane & 15, quarter = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / KIPP_WAVE), lane = threadIdx.x & (KIPP_WAVE - 1), l16 = lane & 15, quarter = lane >> 4;
     const int group = g.n_q / g.n_kv;
     for (int c = wave; c < g.n_kv; c += MX_WAVES) {
         const int h = c * group + min(l16, group - 1);      // lanes beyond the head's group compute what nobody reads
@@ -651,11 +713,11 @@ __global__ void __launch_bounds__(MX_THREADS) mixed_single_values_kernel(SingleG
                                                                          float* __restrict__ partial) {
     constexpr int BLOCKS = V_DIM / 16, KS = SG_KEYS / 32;
     __shared__ __attribute__((aligned(16))) bf16_t p_mixed[2][MX_HPAD * SG_PITCH];
-    __shared__ float2 merged[SG_PARTS][MX_HPAD];
+    __shared__ float2 merged[MX_WAVES][MX_HPAD];
     __shared__ float2 weigh[MX_HPAD];       // a head's maximum and 1 / denominator
     const int token = blockIdx.y, run = blockIdx.x, n_tokens = gridDim.y;
     const Single t = single_of(g, token, run);
-    const int wave = threadIdx.x / KIPP_WAVE, lane = threadIdx.x & (KIPP_WAVE - 1), l16 = lane & 15, quarter = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / KIPP_WAVE), lane = threadIdx.x & (KIPP_WAVE - 1), l16 = lane & 15, quarter = lane >> 4;
     const int n_q = g.n_q, group = g.n_q / g.n_kv;
     auto load_values = [&](int c, int key0, Frag (&vf)[KS][BLOCKS]) {
 #pragma unroll
@@ -668,6 +730,25 @@ __global__ void __launch_bounds__(MX_THREADS) mixed_single_values_kernel(SingleG
     };
     Frag vf[KS][BLOCKS];
     if (t.begin < t.end && wave < g.n_kv) load_values(wave, single_key0(t, t.begin), vf);
+
+    // this wave mixes 16 keys of a tile for 16 of the mixed heads; mix^T as B operand: column 16 nb + l % 16, contraction heads
+    // 8 (l / 16) ..  The first tile's scores and the mix are on their way while the statistics are merged.
+    const int kb = wave & 3, nb = wave >> 2;
+    const int mixed_h = 16 * nb + l16;
+    auto load_scores = [&](int index, float (&sc)[8]) {
+        const float* at = scores + (((size_t)token * g.max_tiles + index) * SG_KEYS + 16 * kb + l16) * MX_HPAD + 8 * quarter;
+        *(f32x4*)sc = *(const f32x4*)at;
+        *(f32x4*)(sc + 4) = *(const f32x4*)(at + 4);
+    };
+    float first_sc[8], mix_w[8];
+    if (t.begin < t.end && 16 * nb < n_q) load_scores(t.begin, first_sc);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const int from = 8 * quarter + j;
+        mix_w[j] = 0.0f;
+        if (mixed_h < n_q && from < n_q) mix_w[j] = mix != nullptr ? mix[mixed_h * n_q + from] : (mixed_h == from ? 1.0f : 0.0f);
+    }
+    const float sunk = sink != nullptr && (int)(threadIdx.x & (MX_HPAD - 1)) < n_q ? sink[threadIdx.x & (MX_HPAD - 1)] : -INFINITY;
 
     // the weights' numbers a head: the runs' statistics, a thread a head and every SG_PARTS-th run; the sink last
     {
@@ -687,37 +768,36 @@ __global__ void __launch_bounds__(MX_THREADS) mixed_single_values_kernel(SingleG
                     m = m_new;
                 }
             }
-        merged[part][h] = make_float2(m, l);
+        {                                   // a wave's two parts
+            const float m_o = __shfl_xor(m, MX_HPAD, KIPP_WAVE), l_o = __shfl_xor(l, MX_HPAD, KIPP_WAVE), m_new = fmaxf(m, m_o);
+            if (m_new != -INFINITY) l = l * __expf(m - m_new) + l_o * __expf(m_o - m_new);
+            m = m_new;
+        }
+        if (lane < MX_HPAD) merged[wave][h] = make_float2(m, l);
         __syncthreads();
         if (threadIdx.x < MX_HPAD) {
+            float2 of_wave[MX_WAVES];
+            float top = sunk;
 #pragma unroll
-            for (int i = 1; i < SG_PARTS; ++i) {
-                const float2 o = merged[i][h];
-                const float m_new = fmaxf(m, o.x);
-                if (m_new != -INFINITY) l = l * __expf(m - m_new) + o.y * __expf(o.x - m_new);
-                m = m_new;
+            for (int i = 0; i < MX_WAVES; ++i) {
+                of_wave[i] = merged[i][h];
+                top = fmaxf(top, of_wave[i].x);
             }
-            if (sink != nullptr && h < n_q) {
-                const float m_new = fmaxf(m, sink[h]);
-                l = (m == -INFINITY ? 0.0f : l * __expf(m - m_new)) + __expf(sink[h] - m_new);
-                m = m_new;
-            }
-            weigh[h] = make_float2(m, l > 0.0f ? 1.0f / l : 0.0f);
+            float sum = sunk != -INFINITY ? __expf(sunk - top) : 0.0f;
+#pragma unroll
+            for (int i = 0; i < MX_WAVES; ++i)
+                if (of_wave[i].x != -INFINITY) sum += of_wave[i].y * __expf(of_wave[i].x - top);
+            weigh[h] = make_float2(top, sum > 0.0f ? 1.0f / sum : 0.0f);
         }
         __syncthreads();
     }
 
-    // this wave mixes 16 keys of a tile for 16 of the mixed heads; mix^T as B operand: column 16 nb + l % 16, contraction heads 8 (l / 16) ..
-    const int kb = wave & 3, nb = wave >> 2;
     float2 of_head[8];
     Frag mf;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-        const int from = 8 * quarter + j, h = 16 * nb + l16;
-        of_head[j] = weigh[from];
-        float w = 0.0f;
-        if (h < n_q && from < n_q) w = mix != nullptr ? mix[h * n_q + from] : (h == from ? 1.0f : 0.0f);
-        mf.h[j] = f32_to_bf16(w);
+        of_head[j] = weigh[8 * quarter + j];
+        mf.h[j] = f32_to_bf16(mix_w[j]);
     }
     for (int c0 = 0; c0 < g.n_kv; c0 += MX_WAVES) {         // (more than eight key/value heads: the weights are made again for each eight)
         const int c = c0 + wave;
@@ -729,10 +809,11 @@ __global__ void __launch_bounds__(MX_THREADS) mixed_single_values_kernel(SingleG
             bf16_t* pm = p_mixed[index & 1];                // the other half is read until every wave is past the barrier
             if ((c0 > 0 || index > t.begin) && c < g.n_kv) load_values(c, key0, vf);
             if (16 * nb < n_q) {
-                const float* at = scores + (((size_t)token * g.max_tiles + index) * SG_KEYS + 16 * kb + l16) * MX_HPAD + 8 * quarter;
                 float sc[8];
-                *(f32x4*)sc = *(const f32x4*)at;
-                *(f32x4*)(sc + 4) = *(const f32x4*)(at + 4);
+                if (c0 > 0 || index > t.begin) load_scores(index, sc);
+                else
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) sc[j] = first_sc[j];
                 Frag hi, lo;
 #pragma unroll
                 for (int j = 0; j < 8; ++j) {
@@ -792,12 +873,23 @@ __global__ void __launch_bounds__(256) mixed_finish_kernel(const float* __restri
     const int n = rows != nullptr ? runs : row_splits[row];
     const int e = 4 * (blockIdx.x * 256 + threadIdx.x);
     if ((rows == nullptr && n <= 1) || e >= width) return;
-    f32x4 o = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int s0 = 0; s0 < n; s0 += 8) {
-        f32x4 part[8];
+    // the gate and eight runs' sums are asked for together, the next eight before those are added
+    f32x4 part[8], next[8], z = {0.0f, 0.0f, 0.0f, 0.0f};
+    auto ask = [&](int s0, f32x4 (&to)[8]) {
 #pragma unroll
         for (int s = 0; s < 8; ++s)
-            part[s] = s0 + s < n ? *(const f32x4*)(partial + (s0 + s) * partial_stride + at_row * width + e) : (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+            to[s] = s0 + s < n ? *(const f32x4*)(partial + (s0 + s) * partial_stride + at_row * width + e) : (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+    };
+    ask(0, next);
+    if (gate != nullptr)
+        for (int p = 0; p < gate_parts; ++p)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) z[v] += gate[p * gate_part_stride + row * gate_stride + e + v];
+    f32x4 o = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int s0 = 0; s0 < n; s0 += 8) {
+#pragma unroll
+        for (int s = 0; s < 8; ++s) part[s] = next[s];
+        if (s0 + 8 < n) ask(s0 + 8, next);
 #pragma unroll
         for (int s = 0; s < 8; ++s) o += part[s];
     }
@@ -805,11 +897,7 @@ __global__ void __launch_bounds__(256) mixed_finish_kernel(const float* __restri
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
         r[v] = o[v];
-        if (gate != nullptr) {
-            float z = 0.0f;
-            for (int p = 0; p < gate_parts; ++p) z += gate[p * gate_part_stride + row * gate_stride + e + v];
-            r[v] *= 1.0f / (1.0f + __expf(-z));
-        }
+        if (gate != nullptr) r[v] *= 1.0f / (1.0f + __expf(-z[v]));
     }
     uint2 w;
     w.x = (uint32_t)f32_to_bf16(r[0]) | ((uint32_t)f32_to_bf16(r[1]) << 16);

@@ -1407,6 +1407,49 @@ def mixed_attention_builds(n_q: int, n_kv: int, d: int, dv: int) -> list:
     return [whole] if whole == sliced else [whole, sliced]
 
 
+def mixed_attention_slices(n_q: int, dv: int) -> int:
+    """Workgroups that share an item in the sliced build."""
+    return dv // mixed_attention_defines(n_q, n_q, 32, dv, sliced=True)["V_SLICE"]
+
+
+# What a cut of the tiles' keys into runs costs, in tiles of 32 keys that a workgroup walks (5.3 us): a round of workgroups its longest item and
+# its start and end (a compute unit holds one workgroup), every item its partial sums' way through memory.  32 heads of 128 over 8, all launches, us, by
+# the longest run of key tiles (items): 1,500 rows 5 (490) 159, 6 (416) 158, 10 (270) 159, 12 (232: one round) 133, 16 (186) 156, 24 (140) 202; 1,900 rows 4 (945)
+# 265, 8 (504: two rounds) 188, 10 (414) 199, 24 (213) 208; 700 rows 2 (264) 98, 3 (184) 72, 4 (144) 76, sliced 5 (120) 72, 6 (104) 76;
+# 200 rows, sliced, 2 (28) 44, 4 (18) 54, 6 (14) 65.
+MIXED_ROUND, MIXED_ROUND_SLICED, MIXED_ITEM, MIXED_SUMS = 3.6, 2.1, 0.02, 1.0
+MIXED_MOST_RUNS = 16
+
+
+def mixed_tile_runs(key_tiles, units: int, slices: int) -> list:
+    """Runs that each tile's keys (`key_tiles[i]` tiles of 32) are cut into: the cut of least cost among those that the longest tile's
+    runs name, by the sizes above.  Up to a round of `units` the workgroups are the sliced ones, `slices` an item."""
+    count = {}
+    for n in key_tiles:
+        count[n] = count.get(n, 0) + 1
+    longest = max(count)
+    best = None
+    for most in range(1, min(MIXED_MOST_RUNS, longest) + 1):
+        chunk = -(-longest // most)
+        items = {}
+        for n, times in count.items():
+            runs = min(MIXED_MOST_RUNS, -(-n // chunk))
+            length = -(-n // runs)
+            items[length] = items.get(length, 0) + runs * times
+        total = sum(items.values())
+        cost = MIXED_ITEM * total + (MIXED_SUMS if most > 1 else 0.0)
+        start = MIXED_ROUND_SLICED if slices > 1 and total * slices <= units else MIXED_ROUND
+        at, turn = 0, 0                         # items go out longest first: a round lasts as long as its first one
+        for length in sorted(items, reverse=True):
+            at += items[length]
+            while turn < at:
+                cost += start + length
+                turn += units
+        if best is None or cost < best[0]:
+            best = (cost, chunk)
+    return [min(MIXED_MOST_RUNS, -(-n // best[1])) for n in key_tiles]
+
+
 def mixed_attention_fast_ok(n_q: int, d: int, dv: int, page: int) -> bool:
     """Whether the matrix-core form takes this geometry: key size a multiple of 32, value size a multiple of 16,
     up to 32 heads whose sums fit a wave's registers, pages of a multiple of 16 keys."""
@@ -1454,7 +1497,7 @@ def mixed_attention_mfma(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.
              [_c_ptr] * 5 + [_c_int, _c_int] + [_c_ptr] * 4 + [_c_int, _c_ptr, _c_int] + [_c_ptr] * 4 + [_c_int] + [_c_ptr] * 6
              + [_c_int] * 6 + [_c_float, _c_int, _c_int, _c_ptr],
              # fewer items than compute units: the value columns are shared out over more workgroups
-             mixed_attention_defines(n_q, n_kv, d, dv, sliced=n_items < COMPUTE_UNITS))
+             mixed_attention_defines(n_q, n_kv, d, dv, sliced=n_items * mixed_attention_slices(n_q, dv) <= COMPUTE_UNITS))
     gate_ptr = gate.data_ptr() + 4 * gate_at if gate is not None else None
     _check(fn(_ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(out), gate_ptr, gate_stride, gate_parts,
               _ptr(items[0]), _ptr(items[1]), _ptr(items[2]), _ptr(items[3]), n_items, _ptr(row_splits), max_splits,

@@ -166,10 +166,11 @@ class MixedHeadAttention:
             if not tiles:
                 batch.host[key] = (single, None)
                 return batch.host[key]
-            want = -(-2 * ops.compute_units(self.rt.device) // len(tiles))
+            runs_of = ops.mixed_tile_runs([t[3] for t in tiles], ops.compute_units(self.rt.device),
+                                          ops.mixed_attention_slices(s.num_heads, s.v_head_dim))
             entry, row0s, split, nsplits, row_splits = [], [], [], [], [1] * batch.n_tokens
-            for e, row0, rows, key_tiles in tiles:
-                runs = max(1, min(16, key_tiles // 4, want))
+            # the longest runs first, so that the short ones fill the last round
+            for (e, row0, rows, _), runs in sorted(zip(tiles, runs_of), key=lambda t: t[0][3] // -t[1]):
                 entry += [e] * runs
                 row0s += [row0] * runs
                 split += list(range(runs))

@@ -61,3 +61,30 @@ def test_work_of_single_tokens_is_their_own_contexts():
     for contexts, own in (([1200] * 24, True), ([300] * 23 + [1200], False)):
         single, tiles = layer._items(batch_of([1] * 24 + [40], contexts + [40]))
         assert (single is not None) == own
+
+
+def test_runs_of_tiles():
+    """Every tile's keys go into 1 to 16 runs none of which is empty, the longest runs come first and a tile's lie together; a
+    prompt fills whole rounds of the chip rather than a round and a part."""
+    for q_len, ctx_len in (([1500], [1500]), ([16], [16]), ([17, 40], [3000, 40]), ([700] * 3, [700, 1400, 9000]), ([2], [2])):
+        layer = layer_of(32, 8)
+        layer.spec.v_head_dim = 128
+        _, (lists, n, row_splits, most, _) = layer._items(batch_of(q_len, ctx_len))
+        entry, row0, split, runs = (x.tolist() for x in lists)
+        at, before, seen = 0, None, {}
+        while at < n:
+            r = runs[at]
+            assert 1 <= r <= 16 and split[at:at + r] == list(range(r)) and {(e, t) for e, t in zip(entry[at:at + r], row0[at:at + r])} == {(entry[at], row0[at])}
+            e = entry[at]
+            rows = min(16, q_len[e] - row0[at])
+            keys = -(-(ctx_len[e] - q_len[e] + row0[at] + rows) // 32)
+            length = -(-keys // r)
+            assert before is None or length <= before
+            before = length
+            seen[(e, row0[at])] = r
+            first = sum(q_len[:e]) + row0[at]
+            assert row_splits[first:first + rows].tolist() == [r] * rows
+            at += r
+        assert at == n and most == max(runs) and set(seen) == {(e, t) for e, m in enumerate(q_len) for t in range(0, m, 16)}
+    tiles = [-(-min(r + 16, 1500) // 32) for r in range(0, 1500, 16)]
+    assert 200 < sum(ops.mixed_tile_runs(tiles, 256, 2)) <= 256
