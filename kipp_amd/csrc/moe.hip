@@ -31,6 +31,7 @@
 #define ROUTE_WAVES 4
 #define MAX_EXPERTS 1024
 #define MAX_TOP 32
+#define SORT_THREADS 1024
 #define TILE_ROWS 16
 #define EXPERT_COLS 256
 #define EXPERT_KC 128
@@ -130,7 +131,9 @@ struct Sort {
     float* row_weight;
 };
 
-// One workgroup sorts all pairs.
+// One workgroup sorts all pairs.  PER > 0: no more than PER pairs a thread, which keeps them in registers, asked for together; a pair's place
+// within its expert's run is what its count returned.  PER 0: any number.
+template <int PER>
 __device__ __forceinline__ void sort_pairs(const Sort& sort, const int32_t* chosen, const float* weight) {
     const int pairs = sort.pairs, experts = sort.experts, top = sort.top, max_tiles = sort.max_tiles, tile_rows = sort.tile_rows;
     int32_t *pair_token = sort.pair_token, *place_of_pair = sort.place_of_pair, *tiles = sort.tiles;
@@ -140,9 +143,23 @@ __device__ __forceinline__ void sort_pairs(const Sort& sort, const int32_t* chos
     __shared__ int tile_first[MAX_EXPERTS + 1];
     for (int e = threadIdx.x; e < experts; e += blockDim.x) count[e] = 0;
     __syncthreads();
-    for (int p = threadIdx.x; p < pairs; p += blockDim.x) {
-        const int e = chosen[p];
-        if (e < experts) atomicAdd(&count[e], 1);
+    int own_e[PER > 0 ? PER : 1], own_place[PER > 0 ? PER : 1];         // (PER) this thread's pairs
+    if (PER > 0) {
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            const int p = threadIdx.x + i * blockDim.x;
+            own_e[i] = chosen[min(p, pairs - 1)];
+            own_place[i] = 0;
+            if (p >= pairs) own_e[i] = experts;
+        }
+#pragma unroll
+        for (int i = 0; i < PER; ++i)
+            if (own_e[i] < experts) own_place[i] = atomicAdd(&count[own_e[i]], 1);
+    } else {
+        for (int p = threadIdx.x; p < pairs; p += blockDim.x) {
+            const int e = chosen[p];
+            if (e < experts) atomicAdd(&count[e], 1);
+        }
     }
     __syncthreads();
     if (threadIdx.x < KIPP_WAVE) {          // where every expert's rows and tiles begin: running sums over 64 experts at a time
@@ -189,6 +206,22 @@ __device__ __forceinline__ void sort_pairs(const Sort& sort, const int32_t* chos
         tiles[(size_t)i * 3 + 1] = 0;
         tiles[(size_t)i * 3 + 2] = 0;
     }
+    if (PER > 0) {
+        float w[PER > 0 ? PER : 1];
+#pragma unroll
+        for (int i = 0; i < PER; ++i) w[i] = row_weight != nullptr ? weight[min((int)(threadIdx.x + i * blockDim.x), pairs - 1)] : 0.0f;
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            const int p = threadIdx.x + i * blockDim.x;
+            if (p >= pairs) break;
+            const int at = own_e[i] < experts ? first[own_e[i]] + own_place[i] : -1;
+            place_of_pair[p] = at;
+            if (at < 0) continue;
+            pair_token[at] = p / top;
+            if (row_weight != nullptr) row_weight[at] = w[i];
+        }
+        return;
+    }
     __syncthreads();
     for (int e = threadIdx.x; e < experts; e += blockDim.x) count[e] = 0;     // now the next free place of a run
     __syncthreads();
@@ -205,7 +238,22 @@ __device__ __forceinline__ void sort_pairs(const Sort& sort, const int32_t* chos
     }
 }
 
-__global__ void __launch_bounds__(1024) moe_sort_kernel(Sort sort, const int32_t* chosen, const float* weight) { sort_pairs(sort, chosen, weight); }
+template <int PER>
+__global__ void __launch_bounds__(SORT_THREADS) moe_sort_kernel(Sort sort, const int32_t* chosen, const float* weight) { sort_pairs<PER>(sort, chosen, weight); }
+
+// The sum of a number's slabs in order, four asked for at once.
+__device__ __forceinline__ float sum_of_slabs(const float* __restrict__ z, int parts, size_t part_stride) {
+    float v = z[0];
+    for (int q0 = 1; q0 < parts; q0 += 4) {
+        float more[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) more[i] = z[min(q0 + i, parts - 1) * part_stride];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (q0 + i < parts) v += more[i];
+    }
+    return v;
+}
 
 // Few tokens (one workgroup's) are chosen for and sorted in one launch (`SORT`): at 1 token 7.5 + 5.6 us as two kernels, 9.86 as one.
 #define ROUTE_SORT_TOKENS 16        // a wave each
@@ -225,8 +273,7 @@ moe_route_kernel(const float* __restrict__ z, int parts, size_t part_stride, int
         const int e = lane + i * KIPP_WAVE;
         float v = -INFINITY;
         if (e < experts) {
-            v = z[(size_t)t * stride + e];
-            for (int q = 1; q < parts; ++q) v += z[q * part_stride + (size_t)t * stride + e];
+            v = sum_of_slabs(z + (size_t)t * stride + e, parts, part_stride);
         }
         p[i] = v;
         m = fmaxf(m, v);
@@ -260,14 +307,18 @@ moe_route_kernel(const float* __restrict__ z, int parts, size_t part_stride, int
         picked_sum += s;
         if (lane == j) { mine = s; mine_e = best_e; }
     }
+    __shared__ int32_t chosen_s[SORT ? WAVES * MAX_TOP : 1];
+    __shared__ float weight_s[SORT ? WAVES * MAX_TOP : 1];
     if (live && lane < top) {
+        const float w = mine / (picked_sum + eps);
         chosen[(size_t)t * top + lane] = mine_e;
-        weight[(size_t)t * top + lane] = mine / (picked_sum + eps);
+        weight[(size_t)t * top + lane] = w;
+        if (SORT) {
+            chosen_s[t * top + lane] = mine_e;
+            weight_s[t * top + lane] = w;
+        }
     }
-    if (SORT) {
-        __syncthreads();
-        sort_pairs(sort, chosen, weight);
-    }
+    if (SORT) sort_pairs<1>(sort, chosen_s, weight_s);
 }
 
 // One wave a token: sigmoid scores (`softmax`: a softmax over all of them), a correction for the choice alone, groups of
@@ -284,15 +335,16 @@ moe_route_grouped_kernel(const float* __restrict__ z, int parts, size_t part_str
     const bool live = t < tokens;
     if (!live) t = tokens - 1;      // stay in step with the barriers
     const int size = experts / group_count;
-    float s[REGS];
+    float s[REGS], correct[REGS];
     float m = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < REGS; ++i) correct[i] = correction != nullptr ? correction[min(lane + i * KIPP_WAVE, experts - 1)] : 0.0f;
 #pragma unroll
     for (int i = 0; i < REGS; ++i) {
         const int e = lane + i * KIPP_WAVE;
         s[i] = 0.0f;
         if (e < experts) {
-            float v = z[(size_t)t * stride + e];
-            for (int q = 1; q < parts; ++q) v += z[q * part_stride + (size_t)t * stride + e];
+            const float v = sum_of_slabs(z + (size_t)t * stride + e, parts, part_stride);
             s[i] = softmax ? v : 1.0f / (1.0f + expf(-v));
             m = fmaxf(m, v);
         }
@@ -313,7 +365,7 @@ moe_route_grouped_kernel(const float* __restrict__ z, int parts, size_t part_str
 #pragma unroll
     for (int i = 0; i < REGS; ++i) {
         const int e = lane + i * KIPP_WAVE;
-        if (e < experts) c_s[wave][e] = s[i] + (correction != nullptr ? correction[e] : 0.0f);
+        if (e < experts) c_s[wave][e] = s[i] + correct[i];
     }
     __syncthreads();
     if (group_keep < group_count) {
@@ -359,39 +411,69 @@ moe_route_grouped_kernel(const float* __restrict__ z, int parts, size_t part_str
             if (g_s[wave][e / size] != -INFINITY) c_s[wave][e] = -INFINITY;             // its group was not taken
         __syncthreads();
     }
-    float c[REGS];
-#pragma unroll
-    for (int i = 0; i < REGS; ++i) {
-        const int e = lane + i * KIPP_WAVE;
-        c[i] = e < experts ? c_s[wave][e] : -INFINITY;
-    }
+    __shared__ int32_t chosen_s[WAVES * MAX_TOP];
+    __shared__ float weight_s[WAVES * MAX_TOP];
     float picked_sum = 0.0f, mine = 0.0f;       // lane j keeps the j-th choice
     int mine_e = 0;
-    for (int j = 0; j < top; ++j) {
-        float best = -INFINITY, best_s = 0.0f;
-        int best_e = MAX_EXPERTS;
-#pragma unroll
-        for (int i = 0; i < REGS; ++i)
-            if (c[i] > best) { best = c[i]; best_e = lane + i * KIPP_WAVE; best_s = s[i]; }     // the lowest index of a lane's largest
-        for (int off = 32; off > 0; off >>= 1) {
-            const float ob = __shfl_xor(best, off, KIPP_WAVE), os = __shfl_xor(best_s, off, KIPP_WAVE);
-            const int oe = __shfl_xor(best_e, off, KIPP_WAVE);
-            if (ob > best || (ob == best && oe < best_e)) { best = ob; best_e = oe; best_s = os; }
+    if constexpr (REGS == 1) {
+        // a lane an expert: its place is the number of experts ahead of it (a larger score, or as large with a lower index)
+        const float own = lane < experts ? c_s[wave][lane] : -INFINITY;
+        int ahead = 0;
+        for (int e = 0; e < experts; ++e) {
+            const float v = c_s[wave][e];
+            ahead += v > own || (v == own && e < lane) ? 1 : 0;
         }
+        if (lane < top) {
+            chosen_s[wave * top + lane] = 0;        // (where fewer can be chosen)
+            weight_s[wave * top + lane] = 0.0f;
+        }
+        __syncthreads();
+        if (own > -INFINITY && ahead < top) {
+            chosen_s[wave * top + ahead] = lane;
+            weight_s[wave * top + ahead] = s[0];
+        }
+        __syncthreads();
+        for (int j = 0; j < top; ++j) picked_sum += weight_s[wave * top + j];
+        if (lane < top) {
+            mine = weight_s[wave * top + lane];
+            mine_e = chosen_s[wave * top + lane];
+        }
+        __syncthreads();
+    } else {
+        float c[REGS];
 #pragma unroll
-        for (int i = 0; i < REGS; ++i)
-            if (lane + i * KIPP_WAVE == best_e) c[i] = -INFINITY;
-        picked_sum += best_s;
-        if (lane == j) { mine = best_s; mine_e = best_e < experts ? best_e : 0; }
+        for (int i = 0; i < REGS; ++i) {
+            const int e = lane + i * KIPP_WAVE;
+            c[i] = e < experts ? c_s[wave][e] : -INFINITY;
+        }
+        for (int j = 0; j < top; ++j) {
+            float best = -INFINITY, best_s = 0.0f;
+            int best_e = MAX_EXPERTS;
+#pragma unroll
+            for (int i = 0; i < REGS; ++i)
+                if (c[i] > best) { best = c[i]; best_e = lane + i * KIPP_WAVE; best_s = s[i]; }     // the lowest index of a lane's largest
+            for (int off = 32; off > 0; off >>= 1) {
+                const float ob = __shfl_xor(best, off, KIPP_WAVE), os = __shfl_xor(best_s, off, KIPP_WAVE);
+                const int oe = __shfl_xor(best_e, off, KIPP_WAVE);
+                if (ob > best || (ob == best && oe < best_e)) { best = ob; best_e = oe; best_s = os; }
+            }
+#pragma unroll
+            for (int i = 0; i < REGS; ++i)
+                if (lane + i * KIPP_WAVE == best_e) c[i] = -INFINITY;
+            picked_sum += best_s;
+            if (lane == j) { mine = best_s; mine_e = best_e < experts ? best_e : 0; }
+        }
     }
     if (live && lane < top) {
+        const float w = renormalize ? mine / (picked_sum + eps) * scale : mine * scale;
         chosen[(size_t)t * top + lane] = mine_e;
-        weight[(size_t)t * top + lane] = renormalize ? mine / (picked_sum + eps) * scale : mine * scale;
+        weight[(size_t)t * top + lane] = w;
+        if (SORT) {
+            chosen_s[t * top + lane] = mine_e;
+            weight_s[t * top + lane] = w;
+        }
     }
-    if (SORT) {
-        __syncthreads();
-        sort_pairs(sort, chosen, weight);
-    }
+    if (SORT) sort_pairs<1>(sort, chosen_s, weight_s);
 }
 
 // x rows are x[gather[row]] (gather null: x[row]); w: [experts][n_out][k]; out[row][n_out].  GLU: w is [experts][2 n_out][k] =
@@ -929,6 +1011,14 @@ moe_combine4_kernel(const float* __restrict__ y, const int32_t* __restrict__ pla
     ((float4*)out)[at] = acc;
 }
 
+static void launch_sort(const Sort& sort, const int32_t* chosen, const float* weight, hipStream_t stream) {
+#define KIPP_SORT(PER) hipLaunchKernelGGL(moe_sort_kernel<PER>, dim3(1), dim3(SORT_THREADS), 0, stream, sort, chosen, weight)
+    if (sort.pairs <= 4 * SORT_THREADS) KIPP_SORT(4);
+    else if (sort.pairs <= 16 * SORT_THREADS) KIPP_SORT(16);
+    else KIPP_SORT(0);
+#undef KIPP_SORT
+}
+
 extern "C" int kipp_moe_route(const float* z, int parts, int stride, int32_t* chosen, float* weight, int tokens, int experts, int top,
                               float eps, int32_t* pair_token, int32_t* place_of_pair, int32_t* tiles, int max_tiles, int tile_rows,
                               float* row_weight, hipStream_t stream) {
@@ -951,7 +1041,7 @@ extern "C" int kipp_moe_route(const float* z, int parts, int stride, int32_t* ch
     else if (experts <= 4 * KIPP_WAVE) KIPP_RT(4, ROUTE_WAVES, false);
     else KIPP_RT(MAX_EXPERTS / KIPP_WAVE, ROUTE_WAVES, false);
 #undef KIPP_RT
-    hipLaunchKernelGGL(moe_sort_kernel, dim3(1), dim3(1024), 0, stream, sort, (const int32_t*)chosen, (const float*)weight);
+    launch_sort(sort, chosen, weight, stream);
     return KIPP_LAUNCH_CHECK();
 }
 
@@ -985,7 +1075,7 @@ extern "C" int kipp_moe_route_grouped(const float* z, int parts, int stride, con
     else if (experts <= 4 * KIPP_WAVE) KIPP_RG(4, ROUTE_WAVES, false);
     else KIPP_RG(MAX_EXPERTS / KIPP_WAVE, ROUTE_WAVES, false);
 #undef KIPP_RG
-    hipLaunchKernelGGL(moe_sort_kernel, dim3(1), dim3(1024), 0, stream, sort, (const int32_t*)chosen, (const float*)weight);
+    launch_sort(sort, chosen, weight, stream);
     return KIPP_LAUNCH_CHECK();
 }
 

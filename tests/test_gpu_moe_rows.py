@@ -349,3 +349,28 @@ def test_activations_over_their_range(name, dtype, inner):
     ends = torch.tensor([[float("inf"), float("nan"), 0.0, -3e38] + [1.0] * (inner - 4)])
     out = ops.activate(ends.to(DEV), torch.empty(ends.shape, dtype=getattr(torch, dtype), device=DEV), name).cpu()[0]
     assert out[0] == float("inf") and torch.isnan(out[1]) and out[2] == 0 and out[3] == 0
+
+
+@pytest.mark.parametrize("router", ["softmax", "sigmoid"])
+@pytest.mark.parametrize("tokens, experts, top, parts", [(16, 32, 32, 1), (4, 64, 32, 5), (1, 1, 1, 6), (1024, 40, 4, 2), (1025, 40, 4, 1), (4096, 33, 4, 1), (4097, 33, 4, 3)])
+def test_choices_and_places_at_the_edges_of_the_sort(router, tokens, experts, top, parts):
+    """Numbers of pairs on both sides of what a thread of the sort keeps, as many choices as experts, equal scores, one to six slabs."""
+    import torch
+    from kipp_amd.csrc import ops
+    rng = np.random.default_rng(tokens + experts)
+    z = rng.integers(-8, 9, size=(parts, tokens, experts)).astype(np.float32) / 8      # sums without rounding, many of them equal
+    new = lambda *shape: torch.full(shape, -7, dtype=torch.int32, device=DEV)  # noqa: E731
+    chosen, weight, pair_token, place = new(tokens, top), torch.empty((tokens, top), device=DEV), new(tokens * top), new(tokens * top)
+    tiles = new(ops.moe_max_tiles(tokens, experts, top, 64), 3)
+    ops.moe_route(torch.tensor(z if parts > 1 else z[0], device=DEV), experts, top, 1e-20, chosen, weight, pair_token, place, tiles, tile_rows=64, router=router)
+    total = z.sum(0).astype(np.float64)
+    picked = np.argsort(-total, axis=1, kind="stable")[:, :top]
+    assert np.array_equal(chosen.cpu().numpy(), picked)
+    s = np.take_along_axis(np.exp(total) if router == "softmax" else 1 / (1 + np.exp(-total)), picked, axis=1)
+    assert np.allclose(weight.cpu().numpy(), s / s.sum(axis=1, keepdims=True), rtol=1e-5)      # float32 exponentials, up to 64 of them
+    at = place.cpu().numpy()
+    assert np.array_equal(np.sort(at), np.arange(tokens * top))
+    assert np.array_equal(pair_token.cpu().numpy()[at], np.arange(tokens * top) // top)
+    expert_of_row = np.empty(tokens * top, dtype=int)
+    expert_of_row[at] = picked.reshape(-1)
+    assert np.all(np.diff(expert_of_row) >= 0)
