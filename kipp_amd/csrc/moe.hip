@@ -832,6 +832,36 @@ moe_expert_tiles_kernel(const bf16_t* __restrict__ x, const int32_t* __restrict_
 // 2,432 (50 MB) 11.1 us.  The kernel for whole tiles above stages 64 numbers of k a step behind two barriers with a workgroup for 128
 // columns: 80 workgroups that walk 38 steps took 44 us for those 50 MB.  One step of 64 numbers ahead for two matrices, two for one: more
 // of them in registers were slower (five: 25.4, 67.8 and 12.7 us), and so were four waves for two matrices.
+// The waves' sums of up to 16 rows, added in order: a lane holds columns 4 (l / 16) .. + 3 of row l % 16.
+template <typename TO, bool GLU>
+__device__ __forceinline__ void expert_rows_end(const f32x4 (&acc)[GLU ? 2 : 1], const float* __restrict__ row_weight, TO* __restrict__ out, int row0, int rows,
+                                                int n0, int n_out, int act, float (*part_s)[GLU ? 2 : 1][KIPP_WAVE][4]) {
+    constexpr int NW = GLU ? 2 : 1;
+    const int wave = threadIdx.x / KIPP_WAVE, lane = threadIdx.x & (KIPP_WAVE - 1);
+#pragma unroll
+    for (int g = 0; g < NW; ++g) *(f32x4*)part_s[wave][g][lane] = acc[g];
+    __syncthreads();
+    const int c = threadIdx.x & 15, m = threadIdx.x >> 4;
+    if (m < 16 && m < rows && n0 + c < n_out) {
+        const int from = 16 * (c >> 2) + m;
+        float total[NW];
+#pragma unroll
+        for (int g = 0; g < NW; ++g) {
+            total[g] = 0.0f;
+#pragma unroll
+            for (int p = 0; p < ROWS_WAVES; ++p) total[g] += part_s[p][g][from][c & 3];
+        }
+        float y;
+        if (GLU) {
+            const float s = row_weight != nullptr ? row_weight[row0 + m] : 1.0f;
+            y = activate<sizeof(TO) == 2>(s * total[0], act) * (s * total[NW - 1]);
+        } else {
+            y = activate<sizeof(TO) == 2>(total[0], act);
+        }
+        store_f(out + (size_t)(row0 + m) * n_out, n0 + c, y);
+    }
+}
+
 template <typename TO, bool GLU, int MT>
 __device__ __forceinline__ void expert_rows(const bf16_t* __restrict__ x, const int32_t* __restrict__ gather, const float* __restrict__ row_weight,
                                             const bf16_t* __restrict__ w_row, TO* __restrict__ out, int row0, int rows, int n0, int n_out, int k,
@@ -874,33 +904,13 @@ __device__ __forceinline__ void expert_rows(const bf16_t* __restrict__ x, const 
                     for (int i = 0; i < MT; ++i)
                         acc[g][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j][half][g].v, xf[j][half][i].v, acc[g][i], 0, 0, 0);
     }
-    // a lane holds columns 4 (l / 16) .. + 3 of row l % 16
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
         if (i > 0) __syncthreads();
+        f32x4 own[NW];
 #pragma unroll
-        for (int g = 0; g < NW; ++g) *(f32x4*)part_s[wave][g][lane] = acc[g][i];
-        __syncthreads();
-        const int c = threadIdx.x & 15, m = threadIdx.x >> 4;
-        if (m < 16 && 16 * i + m < rows && n0 + c < n_out) {
-            const int from = 16 * (c >> 2) + m;
-            float total[NW];
-#pragma unroll
-            for (int g = 0; g < NW; ++g) {
-                total[g] = 0.0f;
-#pragma unroll
-                for (int p = 0; p < ROWS_WAVES; ++p) total[g] += part_s[p][g][from][c & 3];
-            }
-            const int r = row0 + 16 * i + m;
-            float y;
-            if (GLU) {
-                const float s = row_weight != nullptr ? row_weight[r] : 1.0f;
-                y = activate<sizeof(TO) == 2>(s * total[0], act) * (s * total[NW - 1]);
-            } else {
-                y = activate<sizeof(TO) == 2>(total[0], act);
-            }
-            store_f(out + (size_t)r * n_out, n0 + c, y);
-        }
+        for (int g = 0; g < NW; ++g) own[g] = acc[g][i];
+        expert_rows_end<TO, GLU>(own, row_weight, out, row0 + 16 * i, rows - 16 * i, n0, n_out, act, part_s);
     }
 }
 
@@ -917,6 +927,55 @@ moe_expert_rows_kernel(const bf16_t* __restrict__ x, const int32_t* __restrict__
     if (rows <= 16) expert_rows<TO, GLU, 1>(x, gather, row_weight, w_row, out, row0, rows, n0, n_out, k, act, part_s);
     else if (rows <= 32) expert_rows<TO, GLU, 2>(x, gather, row_weight, w_row, out, row0, rows, n0, n_out, k, act, part_s);
     else expert_rows<TO, GLU, 4>(x, gather, row_weight, w_row, out, row0, rows, n0, n_out, k, act, part_s);
+}
+
+// One matrix, steps of up to 16 tokens, whose tiles have no more rows than that (any number is taken, 16 after another): one fragment of rows fits 64
+// registers, four workgroups share a compute unit where the form above has two, and the matrix is asked for before it is known which rows
+// of x the tile has.  A wave's place along k is the same for all its lanes: whole branches, no masks around the loads.  28 experts of 2 rows, 2,432 x
+// 2,560, gathered, 66.6 -> 63.7 us (5.5 TB/s), 2,560 x 2,432 63.7 -> 62.0; 11 experts of one row 28.3 -> 27.1.  Where there are not four workgroups a
+// compute unit it gains nothing (4 experts 11.1, 11.5 so), and neither does a gated one (11 experts 54.8, 54.9; 4 experts 24.4, 24.5; 60 of 768 x 2,048 68.3, 69.7).
+#define FEW_GROUPS (4 * 256)
+template <typename TO>
+__global__ void __launch_bounds__(ROWS_WAVES * KIPP_WAVE, 8)
+moe_expert_few_kernel(const bf16_t* __restrict__ x, const int32_t* __restrict__ gather, const bf16_t* __restrict__ w, const int32_t* __restrict__ tiles,
+                      TO* __restrict__ out, int n_out, int k, int act) {
+    constexpr int STEP = 64, AHEAD = 2;
+    __shared__ __attribute__((aligned(16))) float part_s[ROWS_WAVES][1][KIPP_WAVE][4];
+    const int32_t* tile = tiles + (size_t)blockIdx.y * 3;
+    const int rows = tile[2];
+    if (rows == 0) return;      // uniform over the workgroup
+    const int n0 = 16 * blockIdx.x, row0 = tile[1];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / KIPP_WAVE), lane = threadIdx.x & (KIPP_WAVE - 1), l16 = lane & 15, h8 = 8 * (lane >> 4);
+    const bf16_t* w_row = w + ((size_t)tile[0] * n_out + min(n0 + l16, n_out - 1)) * k + h8;
+    for (int r0 = 0; r0 < rows; r0 += 16) {
+        if (r0 > 0) __syncthreads();
+        f32x4 acc[1] = {(f32x4){0.0f, 0.0f, 0.0f, 0.0f}};
+        Frag wf[AHEAD][2], xf[AHEAD][2];
+        // k is a multiple of 32: the last step may be half a step, whose other half is not multiplied
+        auto fetch = [&](Frag (&to)[2], const bf16_t* row, int from) {
+            if (from >= k) return;
+#pragma unroll
+            for (int half = 0; half < 2; ++half) to[half].u = *(const u32x4*)(row + min(from + 32 * half, k - 32));
+        };
+#pragma unroll
+        for (int j = 0; j < AHEAD; ++j) fetch(wf[j], w_row, STEP * (wave + ROWS_WAVES * j));
+        const int r = row0 + min(r0 + l16, rows - 1);               // rows beyond the last read it and are not stored
+        const bf16_t* x_row = x + (size_t)(gather != nullptr ? gather[r] : r) * k + h8;
+        for (int at = STEP * wave; at < k; at += STEP * ROWS_WAVES * AHEAD) {
+#pragma unroll
+            for (int j = 0; j < AHEAD; ++j) {
+                if (at > STEP * wave) fetch(wf[j], w_row, at + STEP * ROWS_WAVES * j);
+                fetch(xf[j], x_row, at + STEP * ROWS_WAVES * j);
+            }
+#pragma unroll
+            for (int j = 0; j < AHEAD; ++j)
+#pragma unroll
+                for (int half = 0; half < 2; ++half)
+                    if (at + STEP * ROWS_WAVES * j + 32 * half < k)
+                        acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j][half].v, xf[j][half].v, acc[0], 0, 0, 0);
+        }
+        expert_rows_end<TO, false>(acc, nullptr, out, row0 + r0, rows - r0, n0, n_out, act, part_s);
+    }
 }
 
 // A logit that weighs the shared expert's result, by its sigmoid: float32 at column `column` of rows of `stride` (slabs added in
@@ -1100,7 +1159,7 @@ static int launch_tiles(const void* x, const int32_t* gather, const float* row_w
 template <bool GLU>
 static int launch_expert(const void* x, int x_dtype, const int32_t* gather, const float* row_weight, const void* w, int w_dtype,
                          const int32_t* tiles, int max_tiles, void* out, int out_dtype, int n_out, int k, int act, int tile_rows,
-                         int x_rows, int sorted_rows, int experts, hipStream_t stream) {
+                         int x_rows, int sorted_rows, int experts, int most_rows, hipStream_t stream) {
     if (max_tiles <= 0) return 0;
     if (n_out <= 0 || k <= 0 || act < ACT_NONE || act > ACT_RELU2) return -1;
     // a lane's offsets into x and into an expert's matrix are 32 bits wide in the kernels for whole tiles: numbers in the staged one, bytes
@@ -1114,14 +1173,22 @@ static int launch_expert(const void* x, int x_dtype, const int32_t* gather, cons
     if (tile_rows == ROWS_TILE && !(short_k && fits)) {
         if (x_dtype != KIPP_BF16 || w_dtype != KIPP_BF16 || k % 32 || (((uintptr_t)x | (uintptr_t)w) & 15)) return -2;
         dim3 grid((n_out + 15) / 16, max_tiles), block(ROWS_WAVES * KIPP_WAVE);
-        if (out_dtype == KIPP_BF16)
-            hipLaunchKernelGGL((moe_expert_rows_kernel<bf16_t, GLU>), grid, block, 0, stream, (const bf16_t*)x, gather, row_weight,
-                               (const bf16_t*)w, tiles, (bf16_t*)out, n_out, k, act);
-        else if (out_dtype == KIPP_F32)
-            hipLaunchKernelGGL((moe_expert_rows_kernel<float, GLU>), grid, block, 0, stream, (const bf16_t*)x, gather, row_weight,
-                               (const bf16_t*)w, tiles, (float*)out, n_out, k, act);
-        else
+        const bool few = !GLU && most_rows > 0 && most_rows <= 16 && hit * ((n_out + 15) / 16) > FEW_GROUPS;
+#define KIPP_ROWS(TO)                                                                                                                       \
+    if (few)                                                                                                                                \
+        hipLaunchKernelGGL(moe_expert_few_kernel<TO>, grid, block, 0, stream, (const bf16_t*)x, gather, (const bf16_t*)w, tiles, (TO*)out,    \
+                           n_out, k, act);                                                                                                  \
+    else                                                                                                                                    \
+        hipLaunchKernelGGL((moe_expert_rows_kernel<TO, GLU>), grid, block, 0, stream, (const bf16_t*)x, gather, row_weight, (const bf16_t*)w, \
+                           tiles, (TO*)out, n_out, k, act)
+        if (out_dtype == KIPP_BF16) {
+            KIPP_ROWS(bf16_t);
+        } else if (out_dtype == KIPP_F32) {
+            KIPP_ROWS(float);
+        } else {
             return -2;
+        }
+#undef KIPP_ROWS
         return KIPP_LAUNCH_CHECK();
     }
     if (tile_rows == ROWS_TILE || tile_rows == MFMA_ROWS || tile_rows == MANY_ROWS) {
@@ -1163,19 +1230,20 @@ static int launch_expert(const void* x, int x_dtype, const int32_t* gather, cons
 
 // `tile_rows`: the rows of the tiles that `kipp_moe_route` was asked for: 64, 128 and 256 take the matrix cores (bfloat16 x and w, K a
 // multiple of 32), 16 the plain kernel.  `x_rows`: rows that x has.  `sorted_rows` of `experts` experts in all: which kernel for whole tiles is the faster.
+// `most_rows`: the rows that a tile has at most, where the caller knows (else 0): which kernel for few rows is.
 extern "C" int kipp_moe_expert(const void* x, int x_dtype, const int32_t* gather, const void* w, int w_dtype, const int32_t* tiles,
                                int max_tiles, void* out, int out_dtype, int n_out, int k, int act, int tile_rows, int x_rows, int sorted_rows,
-                               int experts, hipStream_t stream) {
+                               int experts, int most_rows, hipStream_t stream) {
     return launch_expert<false>(x, x_dtype, gather, nullptr, w, w_dtype, tiles, max_tiles, out, out_dtype, n_out, k, act, tile_rows, x_rows, sorted_rows,
-                                experts, stream);
+                                experts, most_rows, stream);
 }
 
 // The same against w [experts][2 n_out][k] = [gate; up] with a weight a sorted row (or null): out = act(s gate) * (s up).
 extern "C" int kipp_moe_expert_gated(const void* x, int x_dtype, const int32_t* gather, const float* row_weight, const void* w, int w_dtype,
                                      const int32_t* tiles, int max_tiles, void* out, int out_dtype, int n_out, int k, int act,
-                                     int tile_rows, int x_rows, int sorted_rows, int experts, hipStream_t stream) {
+                                     int tile_rows, int x_rows, int sorted_rows, int experts, int most_rows, hipStream_t stream) {
     return launch_expert<true>(x, x_dtype, gather, row_weight, w, w_dtype, tiles, max_tiles, out, out_dtype, n_out, k, act, tile_rows, x_rows, sorted_rows,
-                               experts, stream);
+                               experts, most_rows, stream);
 }
 
 // `x` (or null): the rows that identity experts hand on.  `gate_z` (or null): rows whose column `gate_column` holds the logit that

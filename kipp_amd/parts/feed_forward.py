@@ -260,10 +260,10 @@ class RoutedMLP:
             x = ops.cast(x, rt.empty(x.shape, self.w_up.dtype))
         inner = rt.empty((pairs, s.expert_size), self.w_up.dtype)
         if s.gate_name is not None:
-            ops.moe_expert_gated(x, pair_token, row_weight, self.w_up, tiles, inner, s.activation, tile_rows=tile_rows)
+            ops.moe_expert_gated(x, pair_token, row_weight, self.w_up, tiles, inner, s.activation, tile_rows=tile_rows, most_rows=n)
         else:
-            ops.moe_expert(x, pair_token, self.w_up, tiles, inner, s.activation, tile_rows=tile_rows)
-        y = ops.moe_expert(inner, None, self.w_down, tiles, rt.empty((pairs, s.hidden_size), torch.float32), tile_rows=tile_rows)
+            ops.moe_expert(x, pair_token, self.w_up, tiles, inner, s.activation, tile_rows=tile_rows, most_rows=n)
+        y = ops.moe_expert(inner, None, self.w_down, tiles, rt.empty((pairs, s.hidden_size), torch.float32), tile_rows=tile_rows, most_rows=n)
         shared = None
         if s.shared_size is not None:
             mid, major = rt.empty((n, s.shared_size), rt.act_dtype), False

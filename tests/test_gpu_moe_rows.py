@@ -374,3 +374,24 @@ def test_choices_and_places_at_the_edges_of_the_sort(router, tokens, experts, to
     expert_of_row = np.empty(tokens * top, dtype=int)
     expert_of_row[at] = picked.reshape(-1)
     assert np.all(np.diff(expert_of_row) >= 0)
+
+
+@pytest.mark.parametrize("k, n_out", [(1056, 530), (1504, 515), (2432, 560), (2560, 512), (4128, 516)])
+@pytest.mark.parametrize("gathered", [False, True])
+def test_few_tokens_have_the_bits_of_more(k, n_out, gathered):
+    """A caller that says how few rows a tile has gets the numbers of one that does not, also where it is wrong: ends of K and of the
+    columns, rows at the edges of 16."""
+    import torch
+    from kipp_amd.csrc import ops
+    rng = np.random.default_rng(k)
+    counts = [1, 2, 15, 16, 17, 0, 33, 64] + [1] * 40
+    experts, rows = len(counts), int(sum(counts))
+    starts = np.concatenate([[0], np.cumsum(counts)[:-1]])
+    tiles = torch.tensor([(e, int(at), n) for e, (at, n) in enumerate(zip(starts, counts))] + [(0, 0, 0)] * 3, dtype=torch.int32, device=DEV)
+    w = torch.tensor((rng.normal(size=(experts, n_out, k)) * k ** -0.5).astype(np.float32), device=DEV).bfloat16()
+    x = torch.tensor(rng.normal(size=(29 if gathered else rows, k)).astype(np.float32), device=DEV).bfloat16()
+    gather = torch.tensor(rng.integers(0, 29, rows), dtype=torch.int32, device=DEV) if gathered else None
+    for dtype, act in ((torch.bfloat16, "relu2"), (torch.float32, None)):
+        want = ops.moe_expert(x, gather, w, tiles, torch.empty((rows, n_out), dtype=dtype, device=DEV), act, tile_rows=64)
+        got = ops.moe_expert(x, gather, w, tiles, torch.full((rows, n_out), float("nan"), dtype=dtype, device=DEV), act, tile_rows=64, most_rows=16)
+        assert torch.equal(got, want), dtype
