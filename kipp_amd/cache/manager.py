@@ -178,8 +178,26 @@ class CacheManager:
         return self.states.get(run)
 
     # -- requests ------------------------------------------------------------------
-    def open(self, request_id, prompt: Optional[Sequence[int]] = None, publish_early: bool = False) -> RequestCache:
-        """Claim a slot (its state zeroed) and, where sharing is on and `prompt`
+    def zero_states(self, slots: Sequence[int]) -> None:
+        """Zero the states of these slots, neighbouring ones in one launch (sixteen requests that come in together over two layers with states of
+        5.4 MB: 32 launches of 2.5 us)."""
+        slots = sorted(slots)
+        runs = []
+        for slot in slots:
+            if runs and runs[-1][1] == slot:
+                runs[-1][1] += 1
+            else:
+                runs.append([slot, slot + 1])
+        for tensor in self.states.values():
+            for first, end in runs:
+                rows = tensor[first:end]
+                if self.rt is not None and (rows[0].numel() * rows.element_size()) % 4 == 0:
+                    self.rt.ops.fill_zero(rows)
+                else:
+                    rows.zero_()
+
+    def open(self, request_id, prompt: Optional[Sequence[int]] = None, publish_early: bool = False, zeroed: bool = True) -> RequestCache:
+        """Claim a slot (its state zeroed, or by the caller with `zero_states` before it is read) and, where sharing is on and `prompt`
         is given, adopt the pages of its longest known beginning.
 
         The reference publishes a session's pages when it ends, which keeps
@@ -192,12 +210,8 @@ class CacheManager:
         if not self.free_slots:
             raise OutOfSlots(f"all {self.max_requests} request slots are taken")
         slot = self.free_slots.pop()
-        for tensor in self.states.values():
-            row = tensor[slot]
-            if self.rt is not None and (row.numel() * row.element_size()) % 4 == 0:
-                self.rt.ops.fill_zero(row)
-            else:
-                row.zero_()
+        if zeroed:
+            self.zero_states([slot])
         self._serial += 1
         req = RequestCache(request_id, slot, tables=[[] for _ in self.groups], adopted=[0 for _ in self.groups],
                            rows=[np.zeros(-(-self.max_position // g.page_size), dtype=np.int32) for g in self.groups],

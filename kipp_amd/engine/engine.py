@@ -124,10 +124,12 @@ class Engine:
         try:
             for e in entries:
                 if e.request not in self.cache.requests:
-                    self.cache.open(e.request)
+                    self.cache.open(e.request, zeroed=False)
                     opened.append(e.request)
                 requests.append(self.cache.requests[e.request])
             self.cache.reserve([(r, len(e.tokens)) for r, e in zip(requests, entries)])
+            if opened and self.cache.states:
+                self.cache.zero_states([self.cache.requests[rid].slot for rid in opened])
         except Exception:
             for rid in opened:
                 self.cache.close(rid)
