@@ -1534,10 +1534,11 @@ def mixed_single_plan(n_tokens: int, max_ctx: int, window: int, keep_first: int)
 
 # Single tokens beside portions take their own form from so much work on (a tile of keys that a token sees counts one, the token itself one
 # more), or from less beside this many rows of portions; lighter ones ride along in the tiles of rows, whose launches are there anyway.  A
-# step of four layers (32 heads over 8 of 128), own form / as tiles, us: work 240, 24 tokens behind 500 keys: beside 16 rows 882 / 813, 200 rows 1,422 /
-# 1,336, 456 rows 1,753 / 1,792, 1,000 rows 2,260 / 2,437; 288, 96 behind 60: 1,201 / 1,113, 1,443 / 1,363, 1,910 / 1,903, 2,575 / 2,813, 1,900 rows 4,454 / 4,607;
-# 396, 12 behind 2,000: 960 / 964, 1,502 / 1,514, 1,832 / 1,846, 2,343 / 2,436; 576, 96 behind 250: 1,290 / 1,314, 1,532 / 1,551, 1,976 / 1,977, 2,660 / 2,943;
-# 144, 24 behind 250: 864 / 812, 1,399 / 1,315, 1,734 / 1,640, 2,233 / 2,422, 1,900 rows 4,153 / 4,063.
+# step of four layers (32 heads over 8 of 128), own form / as tiles, us: work 216, 24 tokens behind 500 keys: beside 16 rows 771 / 703, 200 rows 1,051 /
+# 1,007, 456 rows 1,301 / 1,272, 1,000 rows 1,851 / 1,769; 192, 96 behind 60: 952 / 874, 1,088 / 1,020, 1,351 / 1,302, 1,991 / 1,945; 396, 12 behind
+# 2,000: 858 / 785, 1,153 / 1,075, 1,404 / 1,313, 2,001 / 1,832; 480, 96 behind 250: 1,042 / 1,044, 1,185 / 1,175, 1,457 / 1,392, 2,126 / 2,014; 816, 48
+# behind 1,000: 974 / 883, 1,291 / 1,240, 1,548 / 1,450, 2,179 / 2,090.  The line lies where the two met while a tile's walk cost nearly twice as
+# much; where they meet now (beyond 816) has not been measured, and both sides are faster than they were.
 MIXED_SINGLE_BESIDE = 400
 MIXED_SINGLE_BESIDE_ROWS, MIXED_SINGLE_BESIDE_MANY = 768, 240
 
