@@ -16,7 +16,7 @@
 //          of it at 1,024 rows) and, below a few rounds of tiles, by what the last round leaves idle: the shape goes by that.
 //   shared 64 x 64 outputs a workgroup of four waves, which meet at a barrier every 32 numbers of k: short K in many tiles, where a run a wave
 //          does not pay (`form_of`).
-// Measured at the 4B shape, W in turn from several copies, us: one row against 19,456 x 2,560 39 (5.1 TB/s), 2,560 x 9,728 26, the head's
+// Measured at the 4B shape, W in turn from several copies, us: one row against 19,456 x 2,560 37 (5.4 TB/s), 2,560 x 9,728 25, the head's
 // 151,936 x 2,560 264 (5.9 TB/s).  The tiles, against 19,456 x 2,560 / 6,144 x 2,560 / 2,560 x 4,096 / 2,560 x 9,728, beside what these
 // rows took before (up to 64 rows of X through the kernel for rows, 64 x 64 tiles of four waves that share a step of K beyond):
 //      32 rows    56 / 16 / 20 / 49      106 / 36 / 28 / 73
@@ -100,7 +100,7 @@ __device__ __forceinline__ f32x4 mul16(f32x4 w, f32x4 x, f32x4 acc) {
 
 // The sums of a fragment lie in lane l as rows 4 (l / 16) .. + 3 (of W) of column l % 16 (a row of X).
 template <typename TW, int MT, bool VEC>
-__global__ void __launch_bounds__(ROWS_THREADS)
+__global__ void __launch_bounds__(ROWS_THREADS, MT == 1 ? 6 : 2)
 gemm_f32_rows_kernel(const float* __restrict__ X, const TW* __restrict__ W, float* __restrict__ Y, int M, int N, int K) {
     __shared__ __attribute__((aligned(16))) float part_s[KPARTS][MT][KIPP_WAVE][4];
     const int wave = threadIdx.x / KIPP_WAVE, lane = threadIdx.x & (KIPP_WAVE - 1);
@@ -115,44 +115,51 @@ gemm_f32_rows_kernel(const float* __restrict__ X, const TW* __restrict__ W, floa
     f32x4 acc[MT];
 #pragma unroll
     for (int i = 0; i < MT; ++i) acc[i] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
-    // Pieces of 16 numbers, AHEAD of them on their way: a piece's place is asked for again as soon as it has been multiplied.  (Eight asked for
-    // together, multiplied, and the run's last ones one after the other before: one row against 151,936 / 19,456 / 6,144 x 2,560 and 2,560 x 4,096 / 9,728, us,
-    // 325 / 46.7 / 19.7 / 14.7 / 33.4, with four on their way 271 / 39 / 17 / 12 / 25, six 264 / 39 / 17 / 12.5 / 26, eight 287 / 42 / 18 / 14 / 29, ten
-    // 257 / 38 / 18 / 15 / 30, twelve 386 / 54 / 21 / 16 / 30; 30 rows against 19,456 x 64 7.0, with three 5.6, four 6.8, six 7.3.)
-    constexpr int AHEAD = MT == 1 ? 6 : 3;
+    // Pieces of 16 numbers.  A long run has AHEAD of them on their way: a piece's place is asked for again as soon as it has been multiplied.  The
+    // pieces of a short one are asked for one after the other, and so is what K ends with: asked for under conditions, or with 82 registers (two workgroups a
+    // compute unit; now 80 and three), they cost more than they gain.  The line lies where all of the first AHEAD are there (numbers one at a
+    // time: two pieces of more than a wave's first few, where each is four requests).  One row, us, eight asked for together and the rest one by one / six
+    // ahead whatever the run / now: against 151,936 / 19,456 / 6,144 x 2,560 and 2,560 x 4,096 / 9,728 324 / 46.2 / 19.9 / 14.9 / 33.3, 266 / 38.8 / 17.3 / 12.7 / 26.0,
+    // 264 / 37.5 / 16.2 / 12.2 / 25.3; 19,456 x 16 / 128 / 256 / 768 / 1,024 2.9 / 4.9 / 6.9 / 16.9 / 18.5, 4.9 / 6.5 / 7.8 / 14.4 / 21.3, 2.9 / 4.9 / 6.9 / 11.8 / 16.5; 64 x 16 / 512 1.9 / 2.8,
+    // 2.3 / 3.3, 2.0 / 2.9; 19,456 x 37 / 501 4.8 / 21.3, 4.6 / 12.1, 4.0 / 11.1.  32 rows against 1,024 x 256 3.5, 3.7, 3.5.
+    constexpr int AHEAD = MT > 1 ? 3 : (VEC ? 6 : 5);
     const int whole = max(k_hi - k_lo, 0) / 16;
-    f32x4 w[AHEAD], x[AHEAD][MT];
-    auto ask = [&](int j, int piece) {
-        const int k = k_lo + 16 * piece + h4;
-        w[j] = four_inside<VEC>(w_row + k);
+    int k = k_lo;
+    if (MT == 4 || (whole >= (VEC ? AHEAD : 2) && (VEC || MT == 2 || K > 128))) {
+        constexpr bool full = VEC && MT < 4;        // AHEAD pieces are there
+        f32x4 w[AHEAD], x[AHEAD][MT];
+        auto ask = [&](int j, int piece) {
+            const int at = k_lo + 16 * piece + h4;
+            w[j] = four_inside<VEC>(w_row + at);
 #pragma unroll
-        for (int i = 0; i < MT; ++i) x[j][i] = four_inside<VEC>(x_row[i] + k);
-    };
-    auto take = [&](int j) {
+            for (int i = 0; i < MT; ++i) x[j][i] = four_inside<VEC>(x_row[i] + at);
+        };
+        auto take = [&](int j) {
 #pragma unroll
-        for (int i = 0; i < MT; ++i) acc[i] = mul16(w[j], x[j][i], acc[i]);
-    };
+            for (int i = 0; i < MT; ++i) acc[i] = mul16(w[j], x[j][i], acc[i]);
+        };
 #pragma unroll
-    for (int j = 0; j < AHEAD; ++j)
-        if (j < whole) ask(j, j);
-    int piece = 0;
-    for (; piece + 2 * AHEAD <= whole; piece += AHEAD) {
+        for (int j = 0; j < AHEAD; ++j)
+            if (full || j < whole) ask(j, j);
+        int piece = 0;
+        for (; piece + 2 * AHEAD <= whole; piece += AHEAD) {
+#pragma unroll
+            for (int j = 0; j < AHEAD; ++j) {
+                take(j);
+                ask(j, piece + AHEAD + j);
+            }
+        }
 #pragma unroll
         for (int j = 0; j < AHEAD; ++j) {
-            take(j);
-            ask(j, piece + AHEAD + j);
+            if (full || piece + j < whole) take(j);
+            if (piece + AHEAD + j < whole) ask(j, piece + AHEAD + j);
         }
-    }
 #pragma unroll
-    for (int j = 0; j < AHEAD; ++j) {
-        if (piece + j < whole) take(j);
-        if (piece + AHEAD + j < whole) ask(j, piece + AHEAD + j);
+        for (int j = 0; j < AHEAD; ++j)
+            if (piece + AHEAD + j < whole) take(j);
+        k = k_lo + 16 * whole;
     }
-#pragma unroll
-    for (int j = 0; j < AHEAD; ++j)
-        if (piece + AHEAD + j < whole) take(j);
-    const int k = k_lo + 16 * whole;
-    if (k < k_hi) {                 // what K ends with
+    for (; k < k_hi; k += 16) {
         const f32x4 last = four<VEC>(w_row, k + h4, K);
 #pragma unroll
         for (int i = 0; i < MT; ++i) acc[i] = mul16(last, four<VEC>(x_row[i], k + h4, K), acc[i]);

@@ -54,6 +54,23 @@ def test_few_rows_over_every_number_of_pieces(m, pieces):
         assert np.all(np.abs(got - exact) <= (min(k, _run_of(k)) + 8) * EPS * size), k
 
 
+@pytest.mark.parametrize("k", [1, 17, 31, 33, 127, 128, 129, 131, 190, 255, 256])
+@pytest.mark.parametrize("m", [1, 16, 20, 40])
+def test_few_rows_over_short_runs(m, k):
+    """Both sides of where a run's pieces are asked for ahead, in either kind of weight, numbers four at a time and one at a time.  Bound as above."""
+    import torch
+    from kipp_amd.csrc import ops
+    rng = np.random.default_rng(k + m)
+    x, w = rng.normal(size=(m, k)).astype(np.float32), torch.tensor(rng.normal(size=(37, k)).astype(np.float32)).bfloat16().float().numpy()
+    exact = x.astype(np.float64) @ w.astype(np.float64).T
+    size = np.abs(x).astype(np.float64) @ np.abs(w).astype(np.float64).T
+    outs = []
+    for dtype in (torch.float32, torch.bfloat16):
+        outs.append(ops.gemm_f32(torch.tensor(x, device=DEV), torch.tensor(w, device=DEV, dtype=dtype), torch.empty((m, 37), device=DEV)).cpu().numpy())
+    assert np.all(np.abs(outs[0] - exact) <= (min(k, _run_of(k)) + 8) * EPS * size)
+    assert np.array_equal(outs[0], outs[1])
+
+
 @pytest.mark.parametrize("m, n", [(17, 32), (33, 47), (49, 2579), (97, 2570), (350, 3001), (333, 2570), (200, 6155)])
 @pytest.mark.parametrize("k", [40, 268])
 def test_product_in_every_shape_of_tiles(m, n, k):
