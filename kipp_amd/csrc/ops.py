@@ -1414,12 +1414,14 @@ def mixed_attention_slices(n_q: int, dv: int) -> int:
     return dv // mixed_attention_defines(n_q, n_q, 32, dv, sliced=True)["V_SLICE"]
 
 
-# What a cut of the tiles' keys into runs costs, in tiles of 32 keys that a workgroup walks (5.3 us): a round of workgroups its longest item and
-# its start and end (a compute unit holds one workgroup), every item its partial sums' way through memory.  32 heads of 128 over 8, all launches, us, by
-# the longest run of key tiles (items): 1,500 rows 5 (490) 159, 6 (416) 158, 10 (270) 159, 12 (232: one round) 133, 16 (186) 156, 24 (140) 202; 1,900 rows 4 (945)
-# 265, 8 (504: two rounds) 188, 10 (414) 199, 24 (213) 208; 700 rows 2 (264) 98, 3 (184) 72, 4 (144) 76, sliced 5 (120) 72, 6 (104) 76;
-# 200 rows, sliced, 2 (28) 44, 4 (18) 54, 6 (14) 65.
-MIXED_ROUND, MIXED_ROUND_SLICED, MIXED_ITEM, MIXED_SUMS = 3.6, 2.1, 0.02, 1.0
+# What a cut of the tiles' keys into runs costs, in tiles of 32 keys that a workgroup walks: a round of workgroups its longest item and its start
+# and end (a compute unit holds one workgroup), every item its partial sums' way through memory, any cut the launch that adds them.  A walk takes 2.9 us
+# (12 heads of 32 over 3), 4.9 to 5.7 (16 of 128 over 4, 32 of 64 over 8, 24 of 64 over 8, 16 of 64 over 16), 6.2 (32 of 128 over 8) or 19 (32 of 128 over 32),
+# and the other three fitted to those seven, in walks, round 0.5 to 2, items 0 to 0.014, the launch 0.2 to 1.1.  With the numbers below (the largest for the
+# launch: a cut of two tiles costs the smallest heads more than it gives) the plan of 105 steps (64 to 1,900 rows behind 0 or 3,000 keys, windows of 512)
+# takes 1 % more than the best of eleven cuts in the mean; with a round 3.6, an item 0.02 and the launch 1.0, fitted to the 32 heads of 128 over 8
+# alone, 3 %, and more than runs of at least 128 keys where a window is short: 1,000 rows, window 512, 24 heads of 64 over 8 56 us in 189 items, 51 in 252.
+MIXED_ROUND, MIXED_ROUND_SLICED, MIXED_ITEM, MIXED_SUMS = 1.5, 0.5, 0.005, 1.1
 MIXED_MOST_RUNS = 16
 
 

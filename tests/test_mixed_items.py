@@ -140,3 +140,9 @@ def test_runs_of_a_long_prompt_are_found_quickly():
             took.append(time.perf_counter() - start)
         return min(took)
     assert least(ops.mixed_tile_runs) < 0.5 * least(_runs_cut_by_cut)
+
+
+def test_runs_fill_a_round():
+    """One round of workgroups where a window's few tiles of keys are cut further, and a context of two tiles is not cut."""
+    assert sum(ops.mixed_tile_runs(_key_tiles(1000, 3000, 512), 256, 1)) == 252
+    assert ops.mixed_tile_runs(_key_tiles(64, 0), 256, 1) == [1] * 4
