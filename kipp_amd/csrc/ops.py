@@ -1529,23 +1529,25 @@ def mixed_single_plan(n_tokens: int, max_ctx: int, window: int, keep_first: int)
     return tiles, max(1, min(tiles, 128, -(-4 * COMPUTE_UNITS // mixed_single_tokens(n_tokens, tiles))))
 
 
-# Single tokens beside portions take their own form from so much work on (a tile of keys that a token sees counts one, the token itself one
-# more), or from less beside this many rows of portions; lighter ones ride along in the tiles of rows, whose launches are there anyway.  A
-# step of four layers (32 heads over 8 of 128), own form / as tiles, us: work 216, 24 tokens behind 500 keys: beside 16 rows 771 / 703, 200 rows 1,051 /
-# 1,007, 456 rows 1,301 / 1,272, 1,000 rows 1,851 / 1,769; 192, 96 behind 60: 952 / 874, 1,088 / 1,020, 1,351 / 1,302, 1,991 / 1,945; 396, 12 behind
-# 2,000: 858 / 785, 1,153 / 1,075, 1,404 / 1,313, 2,001 / 1,832; 480, 96 behind 250: 1,042 / 1,044, 1,185 / 1,175, 1,457 / 1,392, 2,126 / 2,014; 816, 48
-# behind 1,000: 974 / 883, 1,291 / 1,240, 1,548 / 1,450, 2,179 / 2,090.  The line lies where the two met while a tile's walk cost nearly twice as
-# much; where they meet now (beyond 816) has not been measured, and both sides are faster than they were.
-MIXED_SINGLE_BESIDE = 400
-MIXED_SINGLE_BESIDE_ROWS, MIXED_SINGLE_BESIDE_MANY = 768, 240
+# Single tokens beside portions take their own form from so much work on (a tile of 64 keys that a token sees counts one, the token itself ten
+# more: in the tiles of rows it is a whole item), or where one of them sees so many tiles of keys that its at most 16 runs outlast the portions'; others
+# ride along in the tiles of rows, whose launches are there anyway.  A step of four layers (32 heads over 8 of 128), own form / as tiles, us, beside
+# 16 rows, 200 and 1,000: work 432, 24 tokens behind 500 keys 772 / 742, 1,051 / 1,031, 1,831 / 1,747; 1,056, 96 behind 60 953 / 870, 1,086 / 1,025, 1,991 / 1,945;
+# 1,248, 48 behind 1,000 971 / 883, 1,291 / 1,229, 2,176 / 2,159; 1,752, 24 behind 4,000 1,166 / 1,080, 1,476 / 1,373, 2,288 / 2,108; 2,496, 96 behind 1,000
+# 1,399 / 1,338, 1,539 / 1,508, 2,454 / 2,525; 2,816, 256 behind 60 1,217 / 1,310, 1,436 / 1,564, 2,286 / 2,359; 3,328, 128 behind 1,000 1,511 / 1,700, 1,654 / 1,823,
+# 2,579 / 2,619; 6,656, 256 behind 1,000 2,170 / 2,497, 2,391 / 2,823, 3,255 / 3,684.  One token behind 5,000 keys (beside 16, 100, 500 and 1,900 rows) 750 / 807, 900 /
+# 936, 1,337 / 1,355, 3,255 / 3,045, behind 6,500 758 / 885, 903 / 1,016, 1,346 / 1,416, 3,250 / 3,051; 8 behind 6,500 984 / 959, 1,204 / 1,120, 1,633 / 1,554,
+# 3,520 / 3,293, behind 16,000 (beside 16, 200, 1,000 rows) 1,262 / 1,579, 1,571 / 1,858, 2,402 / 2,478.  Over 214 such steps, 60 of them with 12 heads of 32 over 3 or 16 of
+# 128 over 4, the two lines take 0.9 % more than the better form in the mean and 9 % at most.
+MIXED_SINGLE_BESIDE, MIXED_SINGLE_TOKEN, MIXED_SINGLE_LONG = 2600, 10, 100
 
 
 def mixed_single_ok(n_q: int, n_kv: int, n_tokens: int, tiles: int, portion_rows: int = 0, work: Optional[int] = None) -> bool:
     """Whether `n_tokens` single tokens that see up to `tiles` tiles of keys take their own form in a step whose portions have so many rows: up
-    to 16 query heads a key/value head, and beside portions work enough (`work`, or every token sees `tiles`) for launches of its own."""
-    work = n_tokens * (tiles + 1) if work is None else work
-    least = 0 if portion_rows == 0 else (MIXED_SINGLE_BESIDE if portion_rows < MIXED_SINGLE_BESIDE_ROWS else MIXED_SINGLE_BESIDE_MANY)
-    return n_q // n_kv <= 16 and work >= least
+    to 16 query heads a key/value head, and beside portions work enough (`work`, or every token sees `tiles`) for launches of its own, or a
+    token whose keys are too many for the tiles' runs."""
+    work = n_tokens * (tiles + MIXED_SINGLE_TOKEN) if work is None else work
+    return n_q // n_kv <= 16 and (portion_rows == 0 or work >= MIXED_SINGLE_BESIDE or tiles >= MIXED_SINGLE_LONG)
 
 
 def mixed_single_workspace(n_tokens: int, n_q: int, dv: int, tiles: int, runs: int, device) -> tuple:

@@ -147,7 +147,7 @@ class MixedHeadAttention:
             single = None
             if batch.n_decode:
                 seen, runs = ops.mixed_single_plan(batch.n_decode, batch.max_decode_ctx, window, keep)
-                work = sum(ops.mixed_single_plan(1, ctx, window, keep)[0] + 1 for n, ctx in zip(batch.host["q_len"], batch.host["ctx_len"])
+                work = sum(ops.mixed_single_plan(1, ctx, window, keep)[0] + ops.MIXED_SINGLE_TOKEN for n, ctx in zip(batch.host["q_len"], batch.host["ctx_len"])
                            if n == 1) if batch.n_portions else None
                 if ops.mixed_single_ok(s.num_heads, s.num_kv_heads, batch.n_decode, seen, batch.n_tokens - batch.n_decode if batch.n_portions else 0, work):
                     single = ops.mixed_single_workspace(batch.n_decode, s.num_heads, s.v_head_dim, seen, runs, self.rt.device)

@@ -47,8 +47,8 @@ def test_space_for_scores_is_bounded():
 def test_single_tokens_beside_a_portion():
     """They ride along in the portion's tiles until they are work enough for launches of their own; alone they always have those."""
     layer = layer_of(32, 8)
-    for tokens, context, rows, own in ((1, 60, 40, False), (199, 60, 40, False), (200, 60, 40, True), (23, 1000, 40, False), (24, 1000, 40, True),
-                                       (1, 25_600, 40, True), (119, 60, 768, False), (120, 60, 768, True), (120, 60, 767, False)):
+    for tokens, context, rows, own in ((1, 60, 40, False), (236, 60, 40, False), (237, 60, 40, True), (99, 1000, 40, False), (100, 1000, 40, True),
+                                       (1, 6336, 40, False), (1, 6337, 40, True), (236, 60, 1000, False), (237, 60, 1000, True)):
         single, tiles = layer._items(batch_of([1] * tokens + [rows], [context] * tokens + [rows]))
         assert (single is not None) == own and tiles is not None
         entries = tiles[0][0].tolist()
@@ -58,10 +58,10 @@ def test_single_tokens_beside_a_portion():
 
 
 def test_work_of_single_tokens_is_their_own_contexts():
-    """One long context among short ones is not what all of them see: 24 tokens behind 300 to 1,200 keys are less work than 24 behind 1,200."""
+    """One long context among short ones is not what all of them see: 90 tokens behind 300 to 1,200 keys are less work than 90 behind 1,200."""
     layer = layer_of(32, 8)
-    for contexts, own in (([1200] * 24, True), ([300] * 23 + [1200], False)):
-        single, tiles = layer._items(batch_of([1] * 24 + [40], contexts + [40]))
+    for contexts, own in (([1200] * 90, True), ([300] * 89 + [1200], False)):
+        single, tiles = layer._items(batch_of([1] * 90 + [40], contexts + [40]))
         assert (single is not None) == own
 
 
