@@ -832,36 +832,6 @@ moe_expert_tiles_kernel(const bf16_t* __restrict__ x, const int32_t* __restrict_
 // 2,432 (50 MB) 11.1 us.  The kernel for whole tiles above stages 64 numbers of k a step behind two barriers with a workgroup for 128
 // columns: 80 workgroups that walk 38 steps took 44 us for those 50 MB.  One step of 64 numbers ahead for two matrices, two for one: more
 // of them in registers were slower (five: 25.4, 67.8 and 12.7 us), and so were four waves for two matrices.
-// The waves' sums of up to 16 rows, added in order: a lane holds columns 4 (l / 16) .. + 3 of row l % 16.
-template <typename TO, bool GLU>
-__device__ __forceinline__ void expert_rows_end(const f32x4 (&acc)[GLU ? 2 : 1], const float* __restrict__ row_weight, TO* __restrict__ out, int row0, int rows,
-                                                int n0, int n_out, int act, float (*part_s)[GLU ? 2 : 1][KIPP_WAVE][4]) {
-    constexpr int NW = GLU ? 2 : 1;
-    const int wave = threadIdx.x / KIPP_WAVE, lane = threadIdx.x & (KIPP_WAVE - 1);
-#pragma unroll
-    for (int g = 0; g < NW; ++g) *(f32x4*)part_s[wave][g][lane] = acc[g];
-    __syncthreads();
-    const int c = threadIdx.x & 15, m = threadIdx.x >> 4;
-    if (m < 16 && m < rows && n0 + c < n_out) {
-        const int from = 16 * (c >> 2) + m;
-        float total[NW];
-#pragma unroll
-        for (int g = 0; g < NW; ++g) {
-            total[g] = 0.0f;
-#pragma unroll
-            for (int p = 0; p < ROWS_WAVES; ++p) total[g] += part_s[p][g][from][c & 3];
-        }
-        float y;
-        if (GLU) {
-            const float s = row_weight != nullptr ? row_weight[row0 + m] : 1.0f;
-            y = activate<sizeof(TO) == 2>(s * total[0], act) * (s * total[NW - 1]);
-        } else {
-            y = activate<sizeof(TO) == 2>(total[0], act);
-        }
-        store_f(out + (size_t)(row0 + m) * n_out, n0 + c, y);
-    }
-}
-
 template <typename TO, bool GLU, int MT>
 __device__ __forceinline__ void expert_rows(const bf16_t* __restrict__ x, const int32_t* __restrict__ gather, const float* __restrict__ row_weight,
                                             const bf16_t* __restrict__ w_row, TO* __restrict__ out, int row0, int rows, int n0, int n_out, int k,
@@ -904,13 +874,33 @@ __device__ __forceinline__ void expert_rows(const bf16_t* __restrict__ x, const 
                     for (int i = 0; i < MT; ++i)
                         acc[g][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j][half][g].v, xf[j][half][i].v, acc[g][i], 0, 0, 0);
     }
+    // a lane holds columns 4 (l / 16) .. + 3 of row l % 16
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
         if (i > 0) __syncthreads();
-        f32x4 own[NW];
 #pragma unroll
-        for (int g = 0; g < NW; ++g) own[g] = acc[g][i];
-        expert_rows_end<TO, GLU>(own, row_weight, out, row0 + 16 * i, rows - 16 * i, n0, n_out, act, part_s);
+        for (int g = 0; g < NW; ++g) *(f32x4*)part_s[wave][g][lane] = acc[g][i];
+        __syncthreads();
+        const int c = threadIdx.x & 15, m = threadIdx.x >> 4;
+        if (m < 16 && 16 * i + m < rows && n0 + c < n_out) {
+            const int from = 16 * (c >> 2) + m;
+            float total[NW];
+#pragma unroll
+            for (int g = 0; g < NW; ++g) {
+                total[g] = 0.0f;
+#pragma unroll
+                for (int p = 0; p < ROWS_WAVES; ++p) total[g] += part_s[p][g][from][c & 3];
+            }
+            const int r = row0 + 16 * i + m;
+            float y;
+            if (GLU) {
+                const float s = row_weight != nullptr ? row_weight[r] : 1.0f;
+                y = activate<sizeof(TO) == 2>(s * total[0], act) * (s * total[NW - 1]);
+            } else {
+                y = activate<sizeof(TO) == 2>(total[0], act);
+            }
+            store_f(out + (size_t)r * n_out, n0 + c, y);
+        }
     }
 }
 
@@ -931,16 +921,13 @@ moe_expert_rows_kernel(const bf16_t* __restrict__ x, const int32_t* __restrict__
 
 // One matrix, steps of up to 16 tokens, whose tiles have no more rows than that (any number is taken, 16 after another): one fragment of rows fits 64
 // registers, four workgroups share a compute unit where the form above has two, and the matrix is asked for before it is known which rows
-// of x the tile has.  A wave's place along k is the same for all its lanes: whole branches, no masks around the loads.  28 experts of 2 rows, 2,432 x
-// 2,560, gathered, 66.6 -> 63.7 us (5.5 TB/s), 2,560 x 2,432 63.7 -> 62.0; 11 experts of one row 28.3 -> 27.1.  Where there are not four workgroups a
-// compute unit it gains nothing (4 experts 11.1, 11.5 so), and neither does a gated one (11 experts 54.8, 54.9; 4 experts 24.4, 24.5; 60 of 768 x 2,048 68.3, 69.7).
-#define FEW_GROUPS (4 * 256)
+// of x the tile has.  A wave's place along k is the same for all its lanes: whole branches, no masks around the loads.  Which K it is for: `few_pays`.
 template <typename TO>
 __global__ void __launch_bounds__(ROWS_WAVES * KIPP_WAVE, 8)
 moe_expert_few_kernel(const bf16_t* __restrict__ x, const int32_t* __restrict__ gather, const bf16_t* __restrict__ w, const int32_t* __restrict__ tiles,
                       TO* __restrict__ out, int n_out, int k, int act) {
     constexpr int STEP = 64, AHEAD = 2;
-    __shared__ __attribute__((aligned(16))) float part_s[ROWS_WAVES][1][KIPP_WAVE][4];
+    __shared__ __attribute__((aligned(16))) float part_s[ROWS_WAVES][KIPP_WAVE][4];
     const int32_t* tile = tiles + (size_t)blockIdx.y * 3;
     const int rows = tile[2];
     if (rows == 0) return;      // uniform over the workgroup
@@ -949,13 +936,12 @@ moe_expert_few_kernel(const bf16_t* __restrict__ x, const int32_t* __restrict__ 
     const bf16_t* w_row = w + ((size_t)tile[0] * n_out + min(n0 + l16, n_out - 1)) * k + h8;
     for (int r0 = 0; r0 < rows; r0 += 16) {
         if (r0 > 0) __syncthreads();
-        f32x4 acc[1] = {(f32x4){0.0f, 0.0f, 0.0f, 0.0f}};
+        f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
         Frag wf[AHEAD][2], xf[AHEAD][2];
-        // k is a multiple of 32: the last step may be half a step, whose other half is not multiplied
-        auto fetch = [&](Frag (&to)[2], const bf16_t* row, int from) {
+        auto fetch = [&](Frag (&to)[2], const bf16_t* row, int from) {          // k is a multiple of a step
             if (from >= k) return;
 #pragma unroll
-            for (int half = 0; half < 2; ++half) to[half].u = *(const u32x4*)(row + min(from + 32 * half, k - 32));
+            for (int half = 0; half < 2; ++half) to[half].u = *(const u32x4*)(row + from + 32 * half);
         };
 #pragma unroll
         for (int j = 0; j < AHEAD; ++j) fetch(wf[j], w_row, STEP * (wave + ROWS_WAVES * j));
@@ -968,13 +954,21 @@ moe_expert_few_kernel(const bf16_t* __restrict__ x, const int32_t* __restrict__ 
                 fetch(xf[j], x_row, at + STEP * ROWS_WAVES * j);
             }
 #pragma unroll
-            for (int j = 0; j < AHEAD; ++j)
+            for (int j = 0; j < AHEAD; ++j) {
+                if (at + STEP * ROWS_WAVES * j >= k) break;
 #pragma unroll
-                for (int half = 0; half < 2; ++half)
-                    if (at + STEP * ROWS_WAVES * j + 32 * half < k)
-                        acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j][half].v, xf[j][half].v, acc[0], 0, 0, 0);
+                for (int half = 0; half < 2; ++half) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j][half].v, xf[j][half].v, acc, 0, 0, 0);
+            }
         }
-        expert_rows_end<TO, false>(acc, nullptr, out, row0 + r0, rows - r0, n0, n_out, act, part_s);
+        *(f32x4*)part_s[wave][lane] = acc;          // a lane holds columns 4 (l / 16) .. + 3 of row l % 16
+        __syncthreads();
+        const int c = threadIdx.x & 15, m = threadIdx.x >> 4;
+        if (m < 16 && r0 + m < rows && n0 + c < n_out) {
+            float total = 0.0f;
+#pragma unroll
+            for (int p = 0; p < ROWS_WAVES; ++p) total += part_s[p][16 * (c >> 2) + m][c & 3];
+            store_f(out + (size_t)(row0 + r0 + m) * n_out, n0 + c, activate<sizeof(TO) == 2>(total, act));
+        }
     }
 }
 
@@ -1156,6 +1150,18 @@ static int launch_tiles(const void* x, const int32_t* gather, const float* row_w
     return KIPP_LAUNCH_CHECK();
 }
 
+// Whether tiles of up to 16 rows of one matrix take the form that four workgroups a compute unit share: where there are two rounds of them (with less
+// up to 3 % slower), in whole steps of k (with half a step at the end 1 to 6 % slower), of more than one turn of the waves (1,024 numbers; up to
+// there the same within 1 %) and up to two and a half: what the rows are waited for is a smaller part of a longer walk.  Not where rows of the
+// matrix lie 4 KiB apart: four workgroups' requests then crowd into the same parts of memory (60 experts of 2,048 x 2,048 88.9 / 98.4 us).
+// The form for up to 64 rows / this, us: 28 experts of 2 rows, 2,432 x 2,560, gathered, 66.3 / 62.6, 2,560 x 2,432 62.5 / 61.1 (5.7 TB/s); 60 of one row,
+// 1,536 x 1,408 51.7 / 45.0; 32 of 8 rows, 2,432 x 2,560 92.0 / 83.2.  1,640 products of 512 to 3,584 rows of W and 1 to 16 of x, two rounds and more:
+// 6 to 13 % less in the mean, 1.3 % more at most.  A gated product gains nothing (11 experts 54.8, 54.9; 60 of 768 x 2,048 68.3, 69.7).
+static bool few_pays(long long groups, int k) {
+    const int step = 64, turn = 2 * step * ROWS_WAVES;
+    return groups > 8 * 256 && k % step == 0 && k > turn && k <= 5 * turn / 2 && k % 2048 != 0;
+}
+
 template <bool GLU>
 static int launch_expert(const void* x, int x_dtype, const int32_t* gather, const float* row_weight, const void* w, int w_dtype,
                          const int32_t* tiles, int max_tiles, void* out, int out_dtype, int n_out, int k, int act, int tile_rows,
@@ -1173,7 +1179,7 @@ static int launch_expert(const void* x, int x_dtype, const int32_t* gather, cons
     if (tile_rows == ROWS_TILE && !(short_k && fits)) {
         if (x_dtype != KIPP_BF16 || w_dtype != KIPP_BF16 || k % 32 || (((uintptr_t)x | (uintptr_t)w) & 15)) return -2;
         dim3 grid((n_out + 15) / 16, max_tiles), block(ROWS_WAVES * KIPP_WAVE);
-        const bool few = !GLU && most_rows > 0 && most_rows <= 16 && hit * ((n_out + 15) / 16) > FEW_GROUPS;
+        const bool few = !GLU && most_rows > 0 && most_rows <= 16 && few_pays(hit * ((n_out + 15) / 16), k);
 #define KIPP_ROWS(TO)                                                                                                                       \
     if (few)                                                                                                                                \
         hipLaunchKernelGGL(moe_expert_few_kernel<TO>, grid, block, 0, stream, (const bf16_t*)x, gather, (const bf16_t*)w, tiles, (TO*)out,    \
@@ -1241,9 +1247,9 @@ extern "C" int kipp_moe_expert(const void* x, int x_dtype, const int32_t* gather
 // The same against w [experts][2 n_out][k] = [gate; up] with a weight a sorted row (or null): out = act(s gate) * (s up).
 extern "C" int kipp_moe_expert_gated(const void* x, int x_dtype, const int32_t* gather, const float* row_weight, const void* w, int w_dtype,
                                      const int32_t* tiles, int max_tiles, void* out, int out_dtype, int n_out, int k, int act,
-                                     int tile_rows, int x_rows, int sorted_rows, int experts, int most_rows, hipStream_t stream) {
+                                     int tile_rows, int x_rows, int sorted_rows, int experts, hipStream_t stream) {
     return launch_expert<true>(x, x_dtype, gather, row_weight, w, w_dtype, tiles, max_tiles, out, out_dtype, n_out, k, act, tile_rows, x_rows, sorted_rows,
-                               experts, most_rows, stream);
+                               experts, 0, stream);
 }
 
 // `x` (or null): the rows that identity experts hand on.  `gate_z` (or null): rows whose column `gate_column` holds the logit that

@@ -1241,7 +1241,7 @@ def moe_expert(x: torch.Tensor, gather: Optional[torch.Tensor], w: torch.Tensor,
 
 
 def moe_expert_gated(x: torch.Tensor, gather: Optional[torch.Tensor], row_weight: Optional[torch.Tensor], w: torch.Tensor, tiles: torch.Tensor,
-                     out: torch.Tensor, activation: str, tile_rows: int = 16, most_rows: int = 0) -> torch.Tensor:
+                     out: torch.Tensor, activation: str, tile_rows: int = 16) -> torch.Tensor:
     """Every tile's rows against its expert's [gate; up] matrix: out[row] = act(s gate x_row) * (s up x_row), x_row as for
     `moe_expert`, s = row_weight[row] (None: one): what the gated expert makes of s x_row.  `w` [experts, 2 inner, k], `out`
     [sorted rows, inner]."""
@@ -1257,9 +1257,9 @@ def moe_expert_gated(x: torch.Tensor, gather: Optional[torch.Tensor], row_weight
     _need(activation in ACTIVATIONS, f"moe_expert_gated: activation is one of {sorted(ACTIVATIONS)}")
     _need(tile_rows == MOE_TILE_ROWS or (tile_rows in (MOE_FEW_ROWS, MOE_MFMA_ROWS, MOE_MANY_ROWS) and x.dtype == torch.bfloat16 and w.shape[2] % 32 == 0),
           "moe_expert_gated: tiles of 16 rows, or of 64, 128 or 256 for bfloat16 with K a multiple of 32")
-    fn = _fn("moe", "kipp_moe_expert_gated", [_c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_int, _c_ptr] + [_c_int] * 9 + [_c_ptr])
+    fn = _fn("moe", "kipp_moe_expert_gated", [_c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_int, _c_ptr] + [_c_int] * 8 + [_c_ptr])
     _check(fn(_ptr(x), _code(x), _ptr(gather), _ptr(row_weight), _ptr(w), _code(w), _ptr(tiles), tiles.shape[0], _ptr(out), _code(out), inner, w.shape[2],
-              ACTIVATIONS[activation], int(tile_rows), x.shape[0], out.shape[0], w.shape[0], int(most_rows), _stream()), "moe_expert_gated")
+              ACTIVATIONS[activation], int(tile_rows), x.shape[0], out.shape[0], w.shape[0], _stream()), "moe_expert_gated")
     return out
 
 

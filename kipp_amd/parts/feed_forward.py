@@ -260,7 +260,7 @@ class RoutedMLP:
             x = ops.cast(x, rt.empty(x.shape, self.w_up.dtype))
         inner = rt.empty((pairs, s.expert_size), self.w_up.dtype)
         if s.gate_name is not None:
-            ops.moe_expert_gated(x, pair_token, row_weight, self.w_up, tiles, inner, s.activation, tile_rows=tile_rows, most_rows=n)
+            ops.moe_expert_gated(x, pair_token, row_weight, self.w_up, tiles, inner, s.activation, tile_rows=tile_rows)
         else:
             ops.moe_expert(x, pair_token, self.w_up, tiles, inner, s.activation, tile_rows=tile_rows, most_rows=n)
         y = ops.moe_expert(inner, None, self.w_down, tiles, rt.empty((pairs, s.hidden_size), torch.float32), tile_rows=tile_rows, most_rows=n)

@@ -376,11 +376,11 @@ def test_choices_and_places_at_the_edges_of_the_sort(router, tokens, experts, to
     assert np.all(np.diff(expert_of_row) >= 0)
 
 
-@pytest.mark.parametrize("k, n_out", [(1056, 530), (1504, 515), (2432, 560), (2560, 512), (4128, 516)])
+@pytest.mark.parametrize("k, n_out", [(1024, 530), (1056, 530), (1088, 513), (1504, 515), (1984, 520), (2048, 516), (2112, 528), (2432, 560), (2560, 512), (2624, 514), (4128, 516)])
 @pytest.mark.parametrize("gathered", [False, True])
 def test_few_tokens_have_the_bits_of_more(k, n_out, gathered):
-    """A caller that says how few rows a tile has gets the numbers of one that does not, also where it is wrong: ends of K and of the
-    columns, rows at the edges of 16."""
+    """A caller that says how few rows a tile has gets the numbers of one that does not, also where it is wrong: both sides of the K whose tiles have a
+    kernel of their own, ends of the columns, rows at the edges of 16."""
     import torch
     from kipp_amd.csrc import ops
     rng = np.random.default_rng(k)
