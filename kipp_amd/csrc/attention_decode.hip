@@ -1277,8 +1277,9 @@ static int launch_ring(const bf16_t* q, bf16_t* k_cache, bf16_t* v_cache, bf16_t
     // Up to 256 workgroups have a compute unit each.  Whole steps of eight layers with eight heads, us, tokens in the order of the requests and unfolded / now:
     // 64 tokens behind 560 to 2,240 keys 2,755 / 2,620, 40 behind 720 to 2,880 2,595 / 2,379, 100 behind 360 to 1,440 3,404 / 3,286; of equal
     // contexts 64 behind 1,400 2,566 / 2,566, 128 behind 700 3,168 / 3,184 (heads in turn over the dies 3,195).
+    // (Up to 512 keys there is little to even out, and heads beside each other cost equal contexts more: 33 tokens behind 300 keys 11.8 us, folded 13.0.)
     const long long pairs = (long long)n_items * n_kv;
-    const int folded = pairs > 256 && n_items <= 65535 ? 256 / n_kv : 0;
+    const int folded = pairs > 256 && grid_splits > 2 && n_items <= 65535 ? 256 / n_kv : 0;
     const dim3 grid = folded ? dim3(n_kv, n_items, ring_splits) : dim3(n_items, n_kv, ring_splits);
     hipLaunchKernelGGL(attention_decode_ring_kernel<FUSED>, grid, dim3(THREADS), lds, stream, q,
                        k_cache, v_cache, out, part_acc, part_ml, rows, positions, seq_of_token, block_table, max_blocks, n_q,
