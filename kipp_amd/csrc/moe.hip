@@ -255,8 +255,11 @@ __device__ __forceinline__ float sum_of_slabs(const float* __restrict__ z, int p
     return v;
 }
 
-// Few tokens (one workgroup's) are chosen for and sorted in one launch (`SORT`): at 1 token 7.5 + 5.6 us as two kernels, 9.86 as one.
+// Few tokens (one workgroup's) are chosen for and sorted in one launch (`SORT`): one token's four of 32 experts 4.3 us by the sigmoid, 5.6 by the softmax.
 #define ROUTE_SORT_TOKENS 16        // a wave each
+// Choices by rank cost a step an expert (up to 64), one after the other a tree of exchanges each.  17 tokens, us, by trees / by rank: one of 32 experts 5.6 / 5.9,
+// four 7.1 / 6.0, one of 64 5.5 / 6.7, two 6.1 / 6.7, eight 9.6 / 6.9.
+#define RANK_EXPERTS 24
 // One wave a token, a lane REGS of the experts.  z: float32 [tokens][stride] (or slabs of it, added in order).
 template <int REGS, int WAVES, bool SORT>
 __global__ void __launch_bounds__(WAVES * KIPP_WAVE)
@@ -415,7 +418,7 @@ moe_route_grouped_kernel(const float* __restrict__ z, int parts, size_t part_str
     __shared__ float weight_s[WAVES * MAX_TOP];
     float picked_sum = 0.0f, mine = 0.0f;       // lane j keeps the j-th choice
     int mine_e = 0;
-    if constexpr (REGS == 1) {
+    if (REGS == 1 && experts <= RANK_EXPERTS * top) {
         // a lane an expert: its place is the number of experts ahead of it (a larger score, or as large with a lower index)
         const float own = lane < experts ? c_s[wave][lane] : -INFINITY;
         int ahead = 0;
@@ -1064,9 +1067,11 @@ moe_combine4_kernel(const float* __restrict__ y, const int32_t* __restrict__ pla
     ((float4*)out)[at] = acc;
 }
 
+// Registers for twice the pairs at hand are asked for and masked: 8,192 pairs in 16 a thread 15.7 us with the routers' launch, in 8 12.6, without 14.5.
 static void launch_sort(const Sort& sort, const int32_t* chosen, const float* weight, hipStream_t stream) {
 #define KIPP_SORT(PER) hipLaunchKernelGGL(moe_sort_kernel<PER>, dim3(1), dim3(SORT_THREADS), 0, stream, sort, chosen, weight)
     if (sort.pairs <= 4 * SORT_THREADS) KIPP_SORT(4);
+    else if (sort.pairs <= 8 * SORT_THREADS) KIPP_SORT(8);
     else if (sort.pairs <= 16 * SORT_THREADS) KIPP_SORT(16);
     else KIPP_SORT(0);
 #undef KIPP_SORT

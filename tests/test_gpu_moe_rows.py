@@ -352,9 +352,11 @@ def test_activations_over_their_range(name, dtype, inner):
 
 
 @pytest.mark.parametrize("router", ["softmax", "sigmoid"])
-@pytest.mark.parametrize("tokens, experts, top, parts", [(16, 32, 32, 1), (4, 64, 32, 5), (1, 1, 1, 6), (1024, 40, 4, 2), (1025, 40, 4, 1), (4096, 33, 4, 1), (4097, 33, 4, 3)])
+@pytest.mark.parametrize("tokens, experts, top, parts", [(16, 32, 32, 1), (4, 64, 32, 5), (1, 1, 1, 6), (16, 24, 1, 2), (5, 25, 1, 1), (16, 48, 2, 3), (17, 49, 2, 4),
+                                                          (1024, 40, 4, 2), (1025, 40, 4, 1), (2048, 40, 4, 1), (2049, 64, 4, 2), (4096, 33, 4, 1), (4097, 33, 4, 3)])
 def test_choices_and_places_at_the_edges_of_the_sort(router, tokens, experts, top, parts):
-    """Numbers of pairs on both sides of what a thread of the sort keeps, as many choices as experts, equal scores, one to six slabs."""
+    """Numbers of pairs on both sides of what a thread of the sort keeps, of experts on both sides of choices by rank, as many choices as experts,
+    equal scores, one to six slabs."""
     import torch
     from kipp_amd.csrc import ops
     rng = np.random.default_rng(tokens + experts)
