@@ -179,11 +179,12 @@ class CacheManager:
 
     # -- requests ------------------------------------------------------------------
     def zero_states(self, slots: Sequence[int]) -> None:
-        """Zero the states of these slots, neighbouring ones in one launch (sixteen requests that come in together over two layers with states of
-        5.4 MB: 32 launches of 2.5 us)."""
-        slots = sorted(slots)
+        """Zero the states of these slots (in any order), neighbouring ones in one launch (sixteen requests that come in together over two layers
+        with states of 5.4 MB: 2 launches for 32 of 2.5 us; where requests have come and gone in between, as many as there are runs of slots)."""
+        if not self.states:
+            return
         runs = []
-        for slot in slots:
+        for slot in sorted(slots):
             if runs and runs[-1][1] == slot:
                 runs[-1][1] += 1
             else:

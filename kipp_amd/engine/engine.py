@@ -128,7 +128,7 @@ class Engine:
                     opened.append(e.request)
                 requests.append(self.cache.requests[e.request])
             self.cache.reserve([(r, len(e.tokens)) for r, e in zip(requests, entries)])
-            if opened and self.cache.states:
+            if opened:
                 self.cache.zero_states([self.cache.requests[rid].slot for rid in opened])
         except Exception:
             for rid in opened:

@@ -227,12 +227,21 @@ class Scheduler:
         return False
 
     def _admit(self) -> None:
+        opened = []
+        try:
+            self._admit_waiting(opened)
+        finally:                                            # together, and before any step reads them
+            if opened:
+                self.cache.zero_states([rc.slot for rc in opened])
+
+    def _admit_waiting(self, opened) -> None:
+        """The requests of the queue that there is room for; `opened` receives what the cache keeps of them, states not yet zeroed."""
         while self.waiting and len(self.running) < self.max_running:
             req = self.waiting[0]
             if self._worth_waiting(req):
                 self.stats.waits_for_prefix += 1
                 return
-            rc = self.cache.open(req.id, req.prompt, publish_early=True)   # adopts the longest known beginning
+            rc = self.cache.open(req.id, req.prompt, publish_early=True, zeroed=False)   # adopts the longest known beginning
             need = self.cache.pages_bound(rc, req.budget_tokens, self._largest_step)
             promised = [0] * len(self.cache.groups)
             for other in self.running:
@@ -243,6 +252,7 @@ class Scheduler:
                 self.cache.close(req.id)                   # undo; stays first in line
                 self.stats.waits_for_pages += 1
                 return
+            opened.append(rc)
             self.waiting.popleft()
             req.admitted_at = time.monotonic()
             self.stats.queue_wait_seconds_sum += req.admitted_at - req.arrived

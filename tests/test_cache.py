@@ -321,3 +321,43 @@ def test_groups_with_page_sizes_and_pool_sizes_of_their_own():
     m.close("r")
     assert m.free_pages() == [10, 7]
     m.check()
+
+
+def _with_states(max_requests, pages=64):
+    """A manager whose states lie in memory, with the launches that zero them counted."""
+    import types
+    import torch
+    launches = []
+
+    def fill_zero(rows):
+        launches.append(rows.shape[0])
+        rows.zero_()
+    rt = types.SimpleNamespace(cache_dtype=torch.float32, device=torch.device("cpu"), ops=types.SimpleNamespace(fill_zero=fill_zero))
+    m = CacheManager([KVNeed(1, 16), None, None], [None, StateNeed((3, 5)), StateNeed((7,))], P, pages, max_requests, 64, runtime=rt)
+    return m, launches
+
+
+def test_states_are_zeroed_slot_by_slot():
+    """Slots in any order with holes between them: theirs alone, neighbours in one launch a layer."""
+    m, launches = _with_states(9)
+    for state in m.states.values():
+        state.fill_(5.0)
+    m.zero_states([7, 2, 4, 1, 8])
+    for state in m.states.values():
+        assert [bool((row == 0).all()) for row in state] == [slot in (1, 2, 4, 7, 8) for slot in range(10)]
+        assert all(bool((state[slot] == 5).all()) for slot in (0, 3, 5, 6, 9))
+    assert sorted(launches) == [1, 1, 2, 2, 2, 2]
+    m.zero_states([])
+    assert len(launches) == 6
+
+
+def test_a_slot_taken_again_is_zeroed_beside_one_that_runs():
+    m, launches = _with_states(3)
+    a, b = m.open("a"), m.open("b")
+    for state in m.states.values():
+        state.fill_(5.0)
+    m.close("a")
+    c = m.open("c")
+    assert c.slot == a.slot
+    for state in m.states.values():
+        assert bool((state[c.slot] == 0).all()) and bool((state[b.slot] == 5).all())

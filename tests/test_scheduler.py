@@ -314,3 +314,36 @@ def test_a_windowed_group_with_a_small_pool_of_its_own():
         big = Scheduler(eng, max_step_tokens=64, prefill_chunk=32)      # steps of 32 tokens: 19 pages of 2 at once
         big.add(Request("d", list(range(40)), 2))
     eng.cache.check()
+
+
+def test_requests_admitted_together_have_their_states_zeroed_together():
+    """One launch a layer and run of slots for what a step admits, whatever was there before; a request that the pools cannot hold is
+    undone and zeroed when it comes in; neighbours that run keep their states."""
+    from tests.test_cache import _with_states
+    cache, launches = _with_states(8, pages=12)
+    seen = []
+
+    class Engine(FakeEngine):
+        def __init__(self):
+            self.cache, self.vocab_size, self.calls = cache, VOCAB, []
+
+        def step(self, entries, borrow=False):
+            for e in entries:
+                req = cache.requests[e.request]
+                for state in cache.states.values():
+                    assert bool((state[req.slot] == (0 if req.length == 0 else 7)).all()), e.request
+                    state[req.slot] = 7.0
+            seen.append(list(launches))
+            return super().step(entries, borrow)
+    for state in cache.states.values():
+        state.fill_(3.0)
+    sched = Scheduler(Engine(), max_step_tokens=32, prefill_chunk=8)
+    for i in range(4):
+        sched.add(Request(f"r{i}", [1 + i, 2, 3], 2))
+    sched.step()
+    assert seen[0] == [4, 4]                                # two layers, four neighbouring slots
+    sched.add(Request("large", list(range(1, 30)), 19))     # all twelve pages: waits until the others are gone
+    sched.add(Request("small", [5], 1))
+    done = sched.run(max_steps=80)
+    assert set(done) == {"r0", "r1", "r2", "r3", "large", "small"} and all(r.finish_reason == "length" for r in done.values())
+    assert not cache.requests
