@@ -3,7 +3,7 @@
  * (the reference builds its own host the same way, /root/reference/Makefile): the JSON reader, checked sizes,
  * the page pool and the cache manager under random orders of sessions, a model folder opened
  * and stepped on the scalar path under several cuttings with scrambled block tables, the error paths
- * of the step function, the scheduler over few pages with cancellations and a failed step, and the sampler.
+ * of the step function, the order of a step's single tokens, the scheduler over few pages with cancellations and a failed step, and the sampler.
  * The GPU's table is not part of this build.
  *
  *   host_test MODEL_DIR [MODEL_DIR ...] [--toy TOY_DIR]      exit code 0 and a last line "ok <checks>" on success
@@ -360,6 +360,54 @@ static void test_scalar_operations(void) {
 
 /* The scheduler over few pages: random requests, some sharing a beginning, cancellations and one failed step.  Greedy
  * output must not depend on the company: each request is run again alone and gives the same tokens. */
+/* The rows of single tokens: all of them, the longest context first, among equals the lower row, beside portions that are not theirs. */
+static void test_decode_order(const char *folder) {
+    enum { SESSIONS = 45 };
+    static const uint32_t counts[] = {1, 2, 3, 4, 5, 13, 14, 40, SESSIONS};
+    kipp_model *model = NULL;
+    kipp_error error;
+    kipp_model_open_config config;
+    memset(&config, 0, sizeof(config));
+    config.path = KIPP_PATH_CPU_FP32;
+    config.page_tokens = 4;
+    config.kv_pool_pages = 400;
+    config.max_sessions = SESSIONS;
+    if (kipp_model_open_ex(folder, &config, &model, &error) != 0) {
+        CHECK(0);
+        return;
+    }
+    kipp_session *sessions[SESSIONS];
+    kipp_step_item items[SESSIONS];
+    const uint32_t tokens[16] = {0};
+    for (size_t i = 0; i < SESSIONS; ++i) CHECK(kipp_session_create(model, 0, &sessions[i], &error) == 0);
+    for (size_t c = 0; c < sizeof(counts) / sizeof(counts[0]); ++c) {
+        for (uint32_t i = 0; i < counts[c]; ++i) { /* 0 to 9 tokens each: many contexts are as long as another */
+            uint32_t length = rnd(10);
+            CHECK(kipp_session_truncate(sessions[i], 0, &error) == 0);
+            kipp_step_item item = {sessions[i], tokens, length, NULL, 0};
+            if (length > 0) CHECK(kipp_step(model, &item, 1, NULL, 0, &error) == 0);
+        }
+        uint32_t single = 0;
+        for (uint32_t i = 0; i < counts[c]; ++i) {
+            size_t takes = counts[c] > 2 && rnd(4) == 0 ? 2 + rnd(3) : 1;
+            single += takes == 1;
+            items[i] = (kipp_step_item){sessions[i], tokens, takes, NULL, 0};
+        }
+        CHECK(kipp_step(model, items, counts[c], NULL, 0, &error) == 0);
+        const kipp_batch *batch = &model->batch;
+        CHECK(batch->n_decode == single);
+        for (uint32_t i = 0; i < batch->n_decode; ++i) {
+            int32_t row = batch->decode_rows[i];
+            CHECK(row >= 0 && (uint32_t)row < batch->n_tokens && batch->h_q_len[batch->seq_of_token[row]] == 1);
+            if (i == 0) continue;
+            int32_t before = batch->decode_rows[i - 1];
+            CHECK(batch->positions[before] > batch->positions[row] || (batch->positions[before] == batch->positions[row] && before < row));
+        }
+    }
+    for (size_t i = 0; i < SESSIONS; ++i) kipp_session_destroy(sessions[i]);
+    CHECK(kipp_model_close(model, &error) == 0);
+}
+
 static void test_scheduler(const char *folder) {
     kipp_model *model = NULL;
     kipp_error error;
@@ -702,6 +750,7 @@ int main(int argc, char **argv) {
     }
     for (int i = 1; i < models; ++i) test_model(argv[i]);
     for (int i = 1; i < models; ++i) test_scheduler(argv[i]);
+    if (models > 1) test_decode_order(argv[1]);
     if (failures != 0) {
         fprintf(stderr, "%d of %d checks failed\n", failures, checks);
         return 1;
