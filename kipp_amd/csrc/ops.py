@@ -1494,7 +1494,7 @@ def mixed_attention_mfma(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.
     fn = _fn("attention_mixed_mfma", "kipp_mixed_attention_mfma",
              [_c_ptr] * 5 + [_c_int, _c_int] + [_c_ptr] * 4 + [_c_int, _c_ptr, _c_int] + [_c_ptr] * 4 + [_c_int] + [_c_ptr] * 6
              + [_c_int] * 6 + [_c_float, _c_int, _c_int, _c_ptr],
-             # fewer items than compute units: the value columns are shared out over more workgroups
+             # items that leave room for it in one round of workgroups: the value columns are shared out over several
              mixed_attention_defines(n_q, n_kv, d, dv, sliced=n_items * mixed_attention_slices(n_q, dv) <= COMPUTE_UNITS))
     gate_ptr = gate.data_ptr() + 4 * gate_at if gate is not None else None
     _check(fn(_ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(out), gate_ptr, gate_stride, gate_parts,

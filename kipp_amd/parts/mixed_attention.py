@@ -134,8 +134,8 @@ class MixedHeadAttention:
 
     def _items(self, batch):
         """What the matrix-core forms work through: the space of the one for single tokens (None: there are none, or it does not
-        take them), and the item list of the other (None: every entry brings one token): every entry's rows in tiles of 16, and where
-        the tiles alone are too few workgroups to fill the GPU, each tile's keys in several runs (at least 128 keys a run, at most 16 runs).
+        take them), and the item list of the other (None: every entry brings one token): every entry's rows in tiles of 16, each
+        tile's keys in the runs (one tile of 32 keys and more, at most 16 of them) that `mixed_tile_runs` finds cheapest, the longest runs first.
         Made by the first layer of a geometry and kept while the batch object lives: a recorded step keeps its own,
         made for the longest context of its class (the kernels take the true lengths from the device)."""
         s, ops = self.spec, self.rt.ops
