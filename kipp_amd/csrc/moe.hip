@@ -258,7 +258,7 @@ __device__ __forceinline__ float sum_of_slabs(const float* __restrict__ z, int p
 // Few tokens (one workgroup's) are chosen for and sorted in one launch (`SORT`): one token's four of 32 experts 4.3 us by the sigmoid, 5.6 by the softmax.
 #define ROUTE_SORT_TOKENS 16        // a wave each
 // Choices by rank cost a step an expert (up to 64), one after the other a tree of exchanges each.  17 tokens, us, by trees / by rank: one of 32 experts 5.6 / 5.9,
-// four 7.1 / 6.0, one of 64 5.5 / 6.7, two 6.1 / 6.7, eight 9.6 / 6.9.
+// four 7.1 / 6.0, one of 64 5.5 / 6.7, two 6.1 / 6.7, eight 9.6 / 6.9.  A build each.
 #define RANK_EXPERTS 24
 // One wave a token, a lane REGS of the experts.  z: float32 [tokens][stride] (or slabs of it, added in order).
 template <int REGS, int WAVES, bool SORT>
@@ -326,7 +326,7 @@ moe_route_kernel(const float* __restrict__ z, int parts, size_t part_stride, int
 
 // One wave a token: sigmoid scores (`softmax`: a softmax over all of them), a correction for the choice alone, groups of
 // neighbouring experts of which the best stay (by the sum of their two largest, or, `by_largest`, by their largest).
-template <int REGS, int WAVES, bool SORT>
+template <int REGS, int WAVES, bool SORT, bool BY_RANK>
 __global__ void __launch_bounds__(WAVES * KIPP_WAVE)
 moe_route_grouped_kernel(const float* __restrict__ z, int parts, size_t part_stride, int stride, const float* __restrict__ correction,
                          int32_t* chosen, float* weight, int tokens, int experts, int top, float eps,
@@ -418,7 +418,8 @@ moe_route_grouped_kernel(const float* __restrict__ z, int parts, size_t part_str
     __shared__ float weight_s[WAVES * MAX_TOP];
     float picked_sum = 0.0f, mine = 0.0f;       // lane j keeps the j-th choice
     int mine_e = 0;
-    if (REGS == 1 && experts <= RANK_EXPERTS * top) {
+    if constexpr (BY_RANK) {
+        static_assert(REGS == 1, "a lane an expert");
         // a lane an expert: its place is the number of experts ahead of it (a larger score, or as large with a lower index)
         const float own = lane < experts ? c_s[wave][lane] : -INFINITY;
         int ahead = 0;
@@ -1119,19 +1120,23 @@ extern "C" int kipp_moe_route_grouped(const float* z, int parts, int stride, con
     if (tile_rows != TILE_ROWS && tile_rows != ROWS_TILE && tile_rows != MFMA_ROWS && tile_rows != MANY_ROWS) return -1;
     if (max_tiles < (pairs + tile_rows - 1) / tile_rows + (real < pairs ? real : pairs)) return -1;
     const Sort sort = {pairs, real, top, pair_token, place_of_pair, tiles, max_tiles, tile_rows, row_weight};
-#define KIPP_RG(REGS, WAVES, SORT)                                                                                                     \
-    hipLaunchKernelGGL((moe_route_grouped_kernel<REGS, WAVES, SORT>), dim3((tokens + WAVES - 1) / WAVES), dim3(WAVES * KIPP_WAVE), 0, stream, \
+#define KIPP_RG(REGS, WAVES, SORT, BY_RANK)                                                                                            \
+    hipLaunchKernelGGL((moe_route_grouped_kernel<REGS, WAVES, SORT, BY_RANK>), dim3((tokens + WAVES - 1) / WAVES), dim3(WAVES * KIPP_WAVE), 0, stream, \
                        z, parts, (size_t)tokens * stride, stride, correction, chosen, weight, tokens, experts, top, eps, group_count, group_keep, \
                        scale, renormalize, softmax, by_largest, sort)
+    const bool by_rank = experts <= KIPP_WAVE && experts <= RANK_EXPERTS * top;
     if (tokens <= ROUTE_SORT_TOKENS && experts <= 4 * KIPP_WAVE) {
-        if (tokens <= ROUTE_WAVES && experts <= KIPP_WAVE) KIPP_RG(1, ROUTE_WAVES, true);
-        else if (experts <= KIPP_WAVE) KIPP_RG(1, ROUTE_SORT_TOKENS, true);
-        else KIPP_RG(4, ROUTE_SORT_TOKENS, true);
+        if (tokens <= ROUTE_WAVES && by_rank) KIPP_RG(1, ROUTE_WAVES, true, true);
+        else if (by_rank) KIPP_RG(1, ROUTE_SORT_TOKENS, true, true);
+        else if (tokens <= ROUTE_WAVES && experts <= KIPP_WAVE) KIPP_RG(1, ROUTE_WAVES, true, false);
+        else if (experts <= KIPP_WAVE) KIPP_RG(1, ROUTE_SORT_TOKENS, true, false);
+        else KIPP_RG(4, ROUTE_SORT_TOKENS, true, false);
         return KIPP_LAUNCH_CHECK();
     }
-    if (experts <= KIPP_WAVE) KIPP_RG(1, ROUTE_WAVES, false);
-    else if (experts <= 4 * KIPP_WAVE) KIPP_RG(4, ROUTE_WAVES, false);
-    else KIPP_RG(MAX_EXPERTS / KIPP_WAVE, ROUTE_WAVES, false);
+    if (by_rank) KIPP_RG(1, ROUTE_WAVES, false, true);
+    else if (experts <= KIPP_WAVE) KIPP_RG(1, ROUTE_WAVES, false, false);
+    else if (experts <= 4 * KIPP_WAVE) KIPP_RG(4, ROUTE_WAVES, false, false);
+    else KIPP_RG(MAX_EXPERTS / KIPP_WAVE, ROUTE_WAVES, false, false);
 #undef KIPP_RG
     launch_sort(sort, chosen, weight, stream);
     return KIPP_LAUNCH_CHECK();
